@@ -198,29 +198,29 @@ def step_case(model, dtype="bfloat16", layers=8, decodes=0, low=0, high=0, porti
 def listed():
     return [
         # one user's chat with the small model: every launch counts; all 28 layers, as nothing else hides the host
-        step_case("qwen2-1.5b", layers=28, decodes=1, low=391, high=391, name="decode 1, 1.5B"),
+        step_case("qwen2-1.5b", layers=28, decodes=1, low=391, high=391, name="decode-1-qwen2-1.5b"),
         # the engine's headline: eight requests behind 4,096 tokens each
-        step_case("qwen2-7b", decodes=8, low=4096, high=4096, name="decode 8 behind 4096, 7B"),
+        step_case("qwen2-7b", decodes=8, low=4096, high=4096, name="decode-8-qwen2-7b"),
         # a busy server between prompts: an odd number of requests, each at another place of its answer
-        step_case("qwen2-7b", decodes=57, low=65, high=1500, name="decode 57 ragged, 7B"),
+        step_case("qwen2-7b", decodes=57, low=65, high=1500, name="decode-57-qwen2-7b"),
         # a busy server's usual step: decoding requests beside a 512-token portion of a longer prompt and a short new one
-        step_case("qwen2-7b", decodes=23, low=100, high=2000, portions=2, shortest=301, longest=512, name="serving step, 7B"),
+        step_case("qwen2-7b", decodes=23, low=100, high=2000, portions=2, shortest=301, longest=512, name="step-qwen2-7b"),
         # one prompt read at once (retrieval, a long question)
-        step_case("qwen2-7b", portions=1, shortest=2048, longest=2048, name="prompt 2048, 7B"),
+        step_case("qwen2-7b", portions=1, shortest=2048, longest=2048, name="prompt-qwen2-7b"),
         # the true 32-bit path: a small serving step
-        step_case("qwen2-1.5b", dtype="float32", decodes=5, low=100, high=900, portions=1, shortest=611, longest=611, name="float32 serving step, 1.5B"),
+        step_case("qwen2-1.5b", dtype="float32", decodes=5, low=100, high=900, portions=1, shortest=611, longest=611, name="float32-step-qwen2-1.5b"),
         # drawing the tokens of a busy server's step
-        dict(name="sample 48 rows", rows=48, vocab=152064, temperature=0.8, top_p=0.9, top_k=0, greedy=6),
+        dict(name="sample-48", rows=48, vocab=152064, temperature=0.8, top_p=0.9, top_k=0, greedy=6),
         # prompts through routed experts and attention over a latent
-        step_case("tiverax-4k", portions=2, shortest=1000, longest=1500, name="prompts, Tiverax 4k"),
+        step_case("tiverax-4k", portions=2, shortest=1000, longest=1500, name="prompts-tiverax-4k"),
         # prompts of unequal length through delta rules and window attention
-        step_case("gosulorn-2k", portions=3, shortest=400, longest=1300, name="prompts, Gosulorn 2k"),
+        step_case("gosulorn-2k", portions=3, shortest=400, longest=1300, name="prompts-gosulorn-2k"),
         # a serving step through the generalized delta rule, gated recurrences and experts
-        step_case("kedanex-2k", decodes=12, low=50, high=1500, portions=1, shortest=1024, longest=1024, name="serving step, Kedanex 2k"),
+        step_case("kedanex-2k", decodes=12, low=50, high=1500, portions=1, shortest=1024, longest=1024, name="step-kedanex-2k"),
         # a long prompt through state spaces, windows with kept tokens and capped attention
-        step_case("kukulorn-4k", portions=1, shortest=4001, longest=4001, name="prompt 4001, Kukulorn 4k"),
+        step_case("kukulorn-4k", portions=1, shortest=4001, longest=4001, name="prompt-kukulorn-4k"),
         # decoding through experts and latents: the weights of the experts that were hit, and many small kernels
-        step_case("tiverax-4k", decodes=16, low=100, high=3000, name="decode 16, Tiverax 4k"),
+        step_case("tiverax-4k", decodes=16, low=100, high=3000, name="decode-16-tiverax-4k"),
     ]
 
 
