@@ -1166,3 +1166,46 @@ def test_place_tokens_puts_sampled_ids_into_a_steps_rows(ops, ref):
     assert torch.equal(untouched, ids)
     with pytest.raises(KernelError):
         ops.place_tokens(got, dest, source, tokens, 7)
+
+
+# -- routed experts on the matrix cores: tiles of 128 rows x 256 rows of W, steps of 64 indices --------------------------------
+@pytest.mark.parametrize("rows, hidden, inter, top, scale_input, unit", [
+    ((65,), 64, 64, 1, False, "glu"),  # one row beyond a half tile, one step
+    ((64, 1, 0, 129, 127), 200, 136, 1, True, "glu"),  # a last step of fewer indices, columns beyond a tile, groups of every size
+    ((128, 128, 1), 256, 264, 1, True, "relu2"),
+    ((300, 70), 136, 72, 2, False, "relu2"),
+    ((40, 33, 20, 200, 90), 328, 520, 2, True, "glu"),
+])
+def test_grouped_products_at_the_edges_of_their_tiles(ops, rows, hidden, inter, top, scale_input, unit):
+    """Against float64.  Two roundings to bfloat16 (8 bits), each off by at most 2^-8 of its value: the units' middles, which the second
+    product adds up (at most 2^-8 sum |W_down| |middle|), and the result.  Float32 sums of a few hundred terms add less than
+    1e-5 of the same sums."""
+    generator = torch.Generator(device="cuda").manual_seed(sum(rows) + hidden)
+    experts, tokens = len(rows), max(sum(rows) // top, max(rows))
+    drawn = lambda *shape: torch.randn(*shape, generator=generator, device="cuda")  # noqa: E731
+    x = drawn(tokens, hidden).bfloat16()
+    branches = 2 if unit == "glu" else 1
+    first = (drawn(experts * branches * inter, hidden) * hidden ** -0.5).bfloat16()
+    down = (drawn(experts * hidden, inter) * inter ** -0.5).bfloat16()
+    weight = torch.rand(tokens, top, generator=generator, device="cuda") + 0.5
+    choice = torch.full((tokens, top), experts, dtype=torch.int32, device="cuda")  # (no expert: such a pair has no row)
+    at = [(t, k) for k in range(top) for t in range(tokens)]
+    for e, count in enumerate(rows):
+        for t, k in at[:count]:
+            choice[t, k] = e
+        at = at[count:]
+    got = ops.routed_experts(x, choice, weight, first, down, experts, scale_input, None, torch.bfloat16, identity_experts=1, **({"ungated": unit} if unit != "glu" else {}))
+    want = torch.zeros(tokens, hidden, dtype=torch.float64, device="cuda")
+    spread = torch.zeros_like(want)
+    for e in range(experts):
+        w1, w2 = first.view(experts, -1, hidden)[e].double(), down.view(experts, hidden, inter)[e].double()
+        t, k = (choice == e).nonzero(as_tuple=True)
+        share = weight[t, k].double()[:, None]
+        both = x[t].double() @ w1.T * (share if scale_input else 1.0)
+        middle = both[:, :inter] * torch.sigmoid(both[:, :inter]) * both[:, inter:] if unit == "glu" else torch.relu(both).square()
+        want.index_add_(0, t, middle @ w2.T * (1.0 if scale_input else share))
+        spread.index_add_(0, t, middle.abs() @ w2.abs().T * (1.0 if scale_input else share))
+    none = choice == experts
+    want += (x.double()[:, None, :] * (weight.double() * none)[:, :, None]).sum(1)
+    bound = (2.0 ** -8 + 2e-5) * spread + 2.0 ** -8 * 1.01 * want.abs() + 1e-6
+    assert torch.all((got.double() - want).abs() <= bound), float(((got.double() - want).abs() / bound).max())

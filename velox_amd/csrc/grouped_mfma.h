@@ -2,7 +2,7 @@
 // over its own rows, out[r, g, :] = W_g a[r, g, :].  Shared by the routed experts and by the per-head products of
 // attention over a latent.
 //
-// A workgroup of four waves owns 64 rows (128 for the large tiles of a plan) and 64 NT output columns of one group (NT = 2 or 4 tiles of W per wave; half as
+// A workgroup of four waves of the kernel without a plan owns 64 rows and 64 NT output columns of one group (NT = 2 or 4 tiles of W per wave; half as
 // many gate columns and the up columns of the same outputs with the GLU epilogue); a wave owns 16 NT of the columns and all
 // 64 rows: 4 NT 16x16 accumulators.  W comes straight from global memory in the layout of
 // v_mfma_f32_16x16x32_bf16 (lane = 16 g + i holds indices 8 g .. 8 g + 7 of row i: 16 bytes) and is the left operand, so
@@ -23,7 +23,7 @@ typedef __bf16 gm_bf16x8_t __attribute__((ext_vector_type(8)));
 #define GM_ROWS 64       // rows of a tile without a plan (a plan's tiles hold 64 or 128)
 #define GM_FEW_COLS 32   // output columns of a workgroup of the kernel for few rows (GLU: 16)
 
-enum { GM_PLAIN = 0, GM_GLU = 1, GM_GATE = 2, GM_ROW_SCALE = 3, GM_ACT = 4 };
+enum { GM_PLAIN = 0, GM_GLU = 1, GM_GATE = 2, GM_ACT = 3 };
 
 struct GroupedArgs {
   const bf16_t* a;     // element (row r, group g, k) at a[r * a_ld + g * a_group + k]
@@ -41,7 +41,8 @@ struct GroupedArgs {
   const bf16_t* gate;  // GM_GATE: times sigmoid(gate[r * gate_ld + g * gate_group + col * gate_col]); (n, 1) is a number per output, (1, 0) one per group
   long long gate_ld, gate_group, gate_col;
   int act = 0;         // GM_ACT: the result goes through ungated_act(., act)
-  const float* row_scale;  // GM_ROW_SCALE: times row_scale[order[r]]
+  const float* row_scale;  // grouped_tiles_kernel: the sums in front of a GLU or an activation are multiplied with row_scale[order[r]] (nullptr: none)
+  int gather_top = 0;      // grouped_tiles_kernel: > 0: sorted row r is row order[r] / gather_top of `a`
   GluUnit unit = {1.f, INFINITY, 0.f};  // GM_GLU: the unit's middle (see glu_middle)
 };
 
@@ -53,31 +54,12 @@ __device__ __forceinline__ gm_bf16x8_t gm_load(const bf16_t* p, bool ok) {
   return __builtin_bit_cast(gm_bf16x8_t, *reinterpret_cast<const float4_t*>(p));
 }
 
-template <int EPI, typename TO, int GM_NT, int MT>
+template <int EPI, typename TO, int GM_NT>
 __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs args) {
   constexpr int GM_COLS = 64 * GM_NT;    // output columns of the workgroup (GLU: half as many)
-  constexpr int ROWS = 16 * MT;          // rows of a tile: 64 or 128
-  constexpr int HALVES = MT == 8 ? 1 : 2;  // 32-index halves per step (the larger tile takes shorter steps: registers)
-  constexpr int STEP = 32 * HALVES;
-  constexpr int PIECES = MT / 4;         // 16-byte pieces of `a` per thread and half
-  __shared__ float4_t a_lds[2][HALVES][4 * ROWS];
-  int group, row0, rows;
-  const int* order = nullptr;
-  if (args.plan != nullptr) {
-    const int tile = blockIdx.y;
-    if (tile >= args.plan[0]) return;  // (uniform over the workgroup)
-    const int* starts = args.plan + 1;
-    order = starts + args.plan_groups + 1;
-    const int* tile_group = order + 2 * (size_t)args.plan_pairs;
-    const int* tile_row = tile_group + args.plan_max_tiles;
-    group = tile_group[tile];
-    row0 = tile_row[tile];
-    rows = min(ROWS, starts[group + 1] - row0);
-  } else {
-    group = blockIdx.z;
-    row0 = blockIdx.y * ROWS;
-    rows = min(ROWS, args.m - row0);
-  }
+  constexpr int MT = GM_ROWS / 16, HALVES = 2, STEP = 32 * HALVES;
+  __shared__ float4_t a_lds[2][HALVES][4 * GM_ROWS];
+  const int group = blockIdx.z, row0 = blockIdx.y * GM_ROWS, rows = min(GM_ROWS, args.m - row0);
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int i = lane & 15, g4 = lane >> 4;
@@ -96,17 +78,11 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
     const int col = min(col0[t] + i, n - 1);
     w_row[t] = w_base + (size_t)(EPI == GM_GLU && t >= GM_NT / 2 ? n + col : col) * k + 8 * g4;
   }
-  // this thread's pieces of the rows of `a`: piece q = tid + 256 p is row q / 4, indices 8 (q % 4) .. + 7 of a half; in LDS
-  // [part][row], so that a row tile's operand reads are 256 contiguous bytes per 16 lanes
-  const bf16_t* a_piece[PIECES];
-  int a_slot[PIECES];
-#pragma unroll
-  for (int p = 0; p < PIECES; ++p) {
-    const int q = tid + 256 * p;
-    a_piece[p] = args.a + (size_t)(row0 + min(q >> 2, rows - 1)) * args.a_ld + (size_t)group * args.a_group + 8 * (q & 3);
-    a_slot[p] = (q & 3) * ROWS + (q >> 2);
-  }
-  const int a_part = 8 * (tid & 3);  // (q % 4 is tid % 4 for every piece)
+  // this thread's piece of the rows of `a`: row tid / 4, indices 8 (tid % 4) .. + 7 of a half; in LDS [part][row], so that a
+  // row tile's operand reads are 256 contiguous bytes per 16 lanes
+  const int a_part = 8 * (tid & 3);
+  const bf16_t* a_piece = args.a + (size_t)(row0 + min(tid >> 2, rows - 1)) * args.a_ld + (size_t)group * args.a_group + a_part;
+  const int a_slot = (tid & 3) * GM_ROWS + (tid >> 2);
   float4_t acc[GM_NT][MT];
 #pragma unroll
   for (int t = 0; t < GM_NT; ++t)
@@ -118,38 +94,31 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
   for (int u = 0; u < HALVES; ++u) {
 #pragma unroll
     for (int t = 0; t < GM_NT; ++t) w_cur[u][t] = gm_load(w_row[t] + 32 * u, 32 * u + 8 * g4 < k);
-#pragma unroll
-    for (int p = 0; p < PIECES; ++p) a_lds[0][u][a_slot[p]] = __builtin_bit_cast(float4_t, gm_load(a_piece[p] + 32 * u, 32 * u + a_part < k));
+    a_lds[0][u][a_slot] = __builtin_bit_cast(float4_t, gm_load(a_piece + 32 * u, 32 * u + a_part < k));
   }
   __syncthreads();
   int buffer = 0;
   for (int k0 = 0; k0 < k; k0 += STEP) {
-    gm_bf16x8_t a_next[HALVES][PIECES];
+    gm_bf16x8_t a_next[HALVES];
 #pragma unroll
     for (int u = 0; u < HALVES; ++u) {
       const int at = k0 + STEP + 32 * u;
 #pragma unroll
       for (int t = 0; t < GM_NT; ++t) w_next[u][t] = gm_load(w_row[t] + at, at + 8 * g4 < k);
-#pragma unroll
-      for (int p = 0; p < PIECES; ++p) a_next[u][p] = gm_load(a_piece[p] + at, at + a_part < k);
+      a_next[u] = gm_load(a_piece + at, at + a_part < k);
     }
 #pragma unroll
     for (int u = 0; u < HALVES; ++u) {
+      gm_bf16x8_t a_cur[MT];
 #pragma unroll
-      for (int mh = 0; mh < MT; mh += 4) {  // four row tiles at a time: their operands live in registers together
-        gm_bf16x8_t a_cur[4];
+      for (int mt = 0; mt < MT; ++mt) a_cur[mt] = __builtin_bit_cast(gm_bf16x8_t, a_lds[buffer][u][g4 * GM_ROWS + mt * 16 + i]);
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) a_cur[mt] = __builtin_bit_cast(gm_bf16x8_t, a_lds[buffer][u][g4 * ROWS + (mh + mt) * 16 + i]);
+      for (int t = 0; t < GM_NT; ++t)
 #pragma unroll
-        for (int t = 0; t < GM_NT; ++t)
-#pragma unroll
-          for (int mt = 0; mt < 4; ++mt) acc[t][mh + mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_cur[u][t], a_cur[mt], acc[t][mh + mt], 0, 0, 0);
-      }
+        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_cur[u][t], a_cur[mt], acc[t][mt], 0, 0, 0);
     }
 #pragma unroll
-    for (int u = 0; u < HALVES; ++u)
-#pragma unroll
-      for (int p = 0; p < PIECES; ++p) a_lds[buffer ^ 1][u][a_slot[p]] = __builtin_bit_cast(float4_t, a_next[u][p]);
+    for (int u = 0; u < HALVES; ++u) a_lds[buffer ^ 1][u][a_slot] = __builtin_bit_cast(float4_t, a_next[u]);
     __syncthreads();
     buffer ^= 1;
 #pragma unroll
@@ -164,8 +133,6 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
     const int r = mt * 16 + i;
     if (r >= rows) continue;
     const size_t out_row = (size_t)(row0 + r) * args.out_ld + (size_t)group * args.out_group;
-    float scale = 1.f;
-    if (EPI == GM_ROW_SCALE) scale = args.row_scale[order[row0 + r]];
 #pragma unroll
     for (int t = 0; t < (EPI == GM_GLU ? GM_NT / 2 : GM_NT); ++t)
 #pragma unroll
@@ -178,7 +145,6 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
           const float z = to_f32(args.gate[(size_t)(row0 + r) * args.gate_ld + (size_t)group * args.gate_group + (size_t)col * args.gate_col]);
           v *= 1.f / (1.f + expf(-z));
         }
-        if (EPI == GM_ROW_SCALE) v *= scale;
         if (EPI == GM_ACT) v = ungated_act(v, args.act);
         out[out_row + col] = from_f32<TO>(v);
       }
@@ -273,8 +239,6 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
     const int r = mt * 16 + i;
     if (r >= rows) continue;
     const size_t out_row = (size_t)(row0 + r) * args.out_ld + (size_t)group * args.out_group;
-    float scale = 1.f;
-    if (EPI == GM_ROW_SCALE) scale = args.row_scale[order[row0 + r]];
 #pragma unroll
     for (int t = 0; t < (EPI == GM_GLU ? 1 : 2); ++t)
 #pragma unroll
@@ -287,35 +251,215 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
           const float z = to_f32(args.gate[(size_t)(row0 + r) * args.gate_ld + (size_t)group * args.gate_group + (size_t)col * args.gate_col]);
           v *= 1.f / (1.f + expf(-z));
         }
-        if (EPI == GM_ROW_SCALE) v *= scale;
         if (EPI == GM_ACT) v = ungated_act(v, args.act);
         out[out_row + col] = from_f32<TO>(v);
       }
   }
 }
 
-// Launches the kernel that fits: `most_rows` is the most rows any tile can have (the plan's pairs, or m), `tile_rows` the
-// rows of the plan's tiles (64 or 128; without a plan rows come in tiles of 64), `tiles_y` and `tiles_z` the launch's other
-// two dimensions.
+// Steps of many rows with a plan: tiles of 128 rows x 256 rows of W, both operands through LDS by loads that write LDS
+// directly.  What bounds it is how far ahead the loads are: a step of 64 indices is 1,024 cycles of the matrix cores and 48 KB,
+// of which the rows of W come from HBM, so three buffers (144 KB, one workgroup per compute unit) keep two steps' loads in
+// flight behind the one that is multiplied.  Eight waves of 64 x 64, two per SIMD; ONE barrier per step, between the halves
+// of a step: the second half's operands leave LDS while the first half's are multiplied, the next step's first while the
+// second's are.  A row of 64 indices is 128 bytes, eight pieces of 16; the pieces of row r are exchanged by an XOR with r's low
+// three bits, which the loads do by asking for another piece (lane l's piece always lands at base + 16 l): no bank
+// conflicts.  The rows of `a` are fetched where they are: with `gather_top` sorted row r is row order[r] / gather_top of `a`, and
+// the pair's weight, if it scales the unit's input, multiplies the float32 sums instead (W (s x) = s (W x)): no sorted copy is
+// made and nothing is rounded in between.  The tiles of one expert that read the same rows of W come one after the other on
+// the same XCD (workgroups are dealt to the eight XCDs in turn), so W leaves HBM once.
+// Measured on MI355X (both products; before: 128 rows x 256 columns with W straight from global memory into the matrix
+// instructions' layout and one step of loads in flight): 10,000 pairs over 32 experts, 4,096 -> 1,408 -> 4,096: 748 + 280 -> 294 +
+// 168 us (0.78 and 0.69 PFLOP/s; W alone at 4.5 TB/s is 164 + 82 us); 2,072 pairs over 16 experts, 2,048 -> 1,408: 153 + 71 -> 70 + 33.
+// Without its loads the first takes 255 us, without its matrix instructions 302: a tile of 256 x 256 is no faster, nor is a
+// ninth wave that reads W ahead into L2 (335).
+static __device__ __attribute__((aligned(16))) const unsigned int gm_zero_piece[4] = {0u, 0u, 0u, 0u};
+
+#define GM_TILE_ROWS 128  // rows of `a` and
+#define GM_TILE_COLS 256  // rows of W per workgroup of grouped_tiles_kernel
+#define GM_XCDS 8
+
 template <int EPI, typename TO>
-static void grouped_mfma_launch(const GroupedArgs& args, int most_rows, int tile_rows, int tiles_y, int tiles_z, hipStream_t stream) {
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) grouped_tiles_kernel(const GroupedArgs args, const int cols) {
+  constexpr int ROWS = GM_TILE_ROWS, STAGES = 3, WAVES = 8;
+  constexpr int WM = 2, WN = WAVES / WM;               // waves along the rows of `a` and along those of W
+  constexpr int RT = 4, CT = GM_TILE_COLS / WN / 16;   // 16 x 16 tiles of a wave
+  constexpr int A_LOADS = ROWS / 8 / WAVES, W_LOADS = GM_TILE_COLS / 8 / WAVES, LOADS = A_LOADS + W_LOADS;
+  constexpr int GROUP = GM_TILE_COLS / WN;             // rows of W of a wave (GLU: half gate rows, half the up rows of the same outputs)
+  __shared__ __attribute__((aligned(1024))) char smem[STAGES][(ROWS + GM_TILE_COLS) * 128];
+
+  const int total = args.plan[0] * cols;
+  const int share = (total + GM_XCDS - 1) / GM_XCDS;
+  const int mine = (int)(blockIdx.x / GM_XCDS);
+  const int work = (int)(blockIdx.x % GM_XCDS) * share + mine;
+  if (mine >= share || work >= total) return;  // (uniform over the workgroup)
+  const int* starts = args.plan + 1;
+  const int* order = starts + args.plan_groups + 1;
+  const int* tile_group = order + 2 * (size_t)args.plan_pairs;
+  const int* tile_row = tile_group + args.plan_max_tiles;
+  // (a group's tiles follow one another, so work / cols lies among the tiles of the right one)
+  const int near = work / cols, group = tile_group[near];
+  const int begin = starts[group], end = starts[group + 1];
+  const int first_tile = near - (tile_row[near] - begin) / ROWS, tiles = (end - begin + ROWS - 1) / ROWS;
+  const int at = work - first_tile * cols;
+  const int row0 = begin + (at % tiles) * ROWS, rows = min(ROWS, end - row0);
+  const int column = at / tiles;
+
+  const bool half = rows <= 64;  // (a group's last tile) the second 64 rows are neither fetched nor multiplied
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 15, g4 = lane >> 4;
+  const int n = args.n, k = args.k;
+  const int piece = 8 * ((lane & 7) ^ (lane >> 3));  // first index of the piece this lane asks for, in every load
+  const bf16_t* a_at[A_LOADS];
+  const bf16_t* w_at[W_LOADS];
+#pragma unroll
+  for (int m = 0; m < A_LOADS; ++m) {
+    int r = row0 + min(8 * (wave + WAVES * m) + (lane >> 3), rows - 1);
+    if (args.gather_top > 0) r = order[r] / args.gather_top;
+    a_at[m] = args.a + (size_t)r * args.a_ld + piece;
+  }
+  const bf16_t* w_base = args.w + (size_t)group * args.w_group;
+#pragma unroll
+  for (int m = 0; m < W_LOADS; ++m) {
+    const int r = 8 * (wave + WAVES * m) + (lane >> 3);
+    int row;
+    if (EPI == GM_GLU) {
+      const int u = r % GROUP;
+      row = min(column * (GM_TILE_COLS / 2) + r / GROUP * (GROUP / 2) + u % (GROUP / 2), n - 1) + (u >= GROUP / 2 ? n : 0);
+    } else {
+      row = min(column * GM_TILE_COLS + r, n - 1);
+    }
+    w_at[m] = w_base + (size_t)row * k + piece;
+  }
+  auto ask = [&](int k0, int buffer) {
+    const bool beyond = k0 + piece >= k;  // (only ever true in a last step of fewer than 64 indices)
+#pragma unroll
+    for (int m = 0; m < A_LOADS; ++m)
+      if (m == 0 || !half) load_to_lds_16(beyond ? reinterpret_cast<const bf16_t*>(gm_zero_piece) : a_at[m] + k0, smem[buffer] + 1024 * (wave + WAVES * m));
+#pragma unroll
+    for (int m = 0; m < W_LOADS; ++m) load_to_lds_16(beyond ? reinterpret_cast<const bf16_t*>(gm_zero_piece) : w_at[m] + k0, smem[buffer] + ROWS * 128 + 1024 * (wave + WAVES * m));
+  };
+
+  const int wm = wave / WN, wn = wave % WN;
+  const bool idle = half && wm > 0;
+  auto wait_for_one = [&] {  // the oldest of the steps that were asked for has landed; those behind it are still under way
+    if (half) wait_for_loads<(STAGES - 2) * (LOADS - 1)>();
+    else wait_for_loads<(STAGES - 2) * LOADS>();
+  };
+  float4_t acc[CT][RT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int steps = (k + 63) / 64;
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < steps) ask(64 * s, s);
+  const int swizzle = i & 7;
+  const int a_byte = (wm * 64 + i) * 128, w_byte = ROWS * 128 + (wn * GROUP + i) * 128;
+  gm_bf16x8_t a_op[2][RT], w_op[2][CT];
+  auto fetch = [&](int part, int buffer) {
+    if (idle) return;
+    const char* base = smem[buffer];
+    const int place = ((4 * part + g4) ^ swizzle) * 16;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) w_op[part][ct] = *reinterpret_cast<const gm_bf16x8_t*>(base + w_byte + ct * 2048 + place);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) a_op[part][rt] = *reinterpret_cast<const gm_bf16x8_t*>(base + a_byte + rt * 2048 + place);
+  };
+  auto multiply = [&](int part) {
+    if (idle) return;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_op[part][ct], a_op[part][rt], acc[ct][rt], 0, 0, 0);
+  };
+  // the first step's loads have landed when at most those of the later steps that were asked for are under way
+  if (steps >= STAGES - 1) wait_for_one();
+  else wait_for_loads<0>();
+  __syncthreads();
+  fetch(0, 0);
+  int buffer = 0;
+  for (int s = 0; s < steps; ++s) {
+    // operands of the second half on their way while the first half's are multiplied, and the loads of a later step into the
+    // buffer that everybody was done with at the last barrier
+    fetch(1, buffer);
+    int freed = buffer + STAGES - 1;
+    if (freed >= STAGES) freed -= STAGES;
+    if (s + STAGES - 1 < steps) ask(64 * (s + STAGES - 1), freed);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+    __builtin_amdgcn_sched_barrier(0);
+    buffer = buffer + 1 == STAGES ? 0 : buffer + 1;
+    if (s + 1 < steps) {  // the next step's loads: at most those of the steps behind it are still under way
+      if (s + STAGES <= steps) wait_for_one();
+      else wait_for_loads<0>();
+      __syncthreads();
+      fetch(0, buffer);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // lane (g4, i) holds outputs 4 g4 .. + 3 of row i of every tile: one 8- or 16-byte store each (n is a multiple of 4)
+  typedef TO Four __attribute__((ext_vector_type(4)));
+  TO* out = reinterpret_cast<TO*>(args.out);
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int r = wm * 64 + rt * 16 + i;
+    if (r >= rows) continue;
+    float scale = 1.f;
+    if (EPI != GM_PLAIN && args.row_scale != nullptr) scale = args.row_scale[order[row0 + r]];
+    TO* out_row = out + (size_t)(row0 + r) * args.out_ld;
+#pragma unroll
+    for (int ct = 0; ct < (EPI == GM_GLU ? CT / 2 : CT); ++ct) {
+      const int col = (EPI == GM_GLU ? column * (GM_TILE_COLS / 2) + wn * (GROUP / 2) : column * GM_TILE_COLS + wn * GROUP) + ct * 16 + 4 * g4;
+      if (col >= n) continue;
+      Four four;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float v = acc[ct][rt][j];
+        if (EPI == GM_GLU) v = glu_middle(v * scale, acc[ct + CT / 2][rt][j] * scale, args.unit);
+        if (EPI == GM_ACT) v = ungated_act(v * scale, args.act);
+        four[j] = from_f32<TO>(v);
+      }
+      *reinterpret_cast<Four*>(out_row + col) = four;
+    }
+  }
+}
+
+// Launches the kernel that fits: `most_rows` is the most rows any tile can have (the plan's pairs, or m), `tiles_y` the most
+// tiles there can be and `tiles_z` the groups (without a plan).  A plan's tiles hold 64 rows up to 64 pairs, GM_TILE_ROWS above;
+// without a plan rows come in tiles of GM_ROWS.  (Tiles of 64 rows were no quicker at any number of pairs above 64: 12 rows per
+// expert 66 us either way, 56: 80 / 81, 75: 100 / 83, 130: 127 / 125, 256: 187 / 155, 16 experts of 2,048 -> 1,408 -> 2,048.)
+template <int EPI, typename TO>
+static void grouped_mfma_launch(const GroupedArgs& args, int most_rows, int tiles_y, int tiles_z, hipStream_t stream) {
   const int n = args.n;
-  if (most_rows <= 64 && args.plan != nullptr) {
-    // (only with a plan: its tiles hold at most `most_rows` rows whatever their size; without one, rows come in tiles of the kernel's own size)
-    dim3 grid((n + (EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS) - 1) / (EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS), tiles_y, tiles_z);
-    if (most_rows <= 16) grouped_mfma_few_rows_kernel<EPI, TO, 1><<<grid, 256, 0, stream>>>(args);
-    else if (most_rows <= 32) grouped_mfma_few_rows_kernel<EPI, TO, 2><<<grid, 256, 0, stream>>>(args);
-    else grouped_mfma_few_rows_kernel<EPI, TO, 4><<<grid, 256, 0, stream>>>(args);
+  const int outputs = EPI == GM_GLU ? 2 * n : n;  // rows of W
+  if (args.plan != nullptr) {
+    // (its tiles hold at most `most_rows` rows whatever their size)
+    if (most_rows <= 64) {
+      constexpr int COLS = EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS;
+      dim3 grid((n + COLS - 1) / COLS, tiles_y, 1);
+      if (most_rows <= 16) grouped_mfma_few_rows_kernel<EPI, TO, 1><<<grid, 256, 0, stream>>>(args);
+      else if (most_rows <= 32) grouped_mfma_few_rows_kernel<EPI, TO, 2><<<grid, 256, 0, stream>>>(args);
+      else grouped_mfma_few_rows_kernel<EPI, TO, 4><<<grid, 256, 0, stream>>>(args);
+      return;
+    }
+    const int cols = (outputs + GM_TILE_COLS - 1) / GM_TILE_COLS;
+    const int workgroups = (tiles_y * cols + GM_XCDS - 1) / GM_XCDS * GM_XCDS;
+    grouped_tiles_kernel<EPI, TO><<<workgroups, 512, 0, stream>>>(args, cols);
     return;
   }
-  const int outputs = EPI == GM_GLU ? 2 * n : n;  // rows of W
   if (outputs <= 128) {
     const int cols = EPI == GM_GLU ? 64 : 128;
-    grouped_mfma_kernel<EPI, TO, 2, 4><<<dim3((n + cols - 1) / cols, tiles_y, tiles_z), 256, 0, stream>>>(args);
+    grouped_mfma_kernel<EPI, TO, 2><<<dim3((n + cols - 1) / cols, tiles_y, tiles_z), 256, 0, stream>>>(args);
   } else {
     const int cols = EPI == GM_GLU ? 128 : 256;
-    if (tile_rows == 128) grouped_mfma_kernel<EPI, TO, 4, 8><<<dim3((n + cols - 1) / cols, tiles_y, tiles_z), 256, 0, stream>>>(args);
-    else grouped_mfma_kernel<EPI, TO, 4, 4><<<dim3((n + cols - 1) / cols, tiles_y, tiles_z), 256, 0, stream>>>(args);
+    grouped_mfma_kernel<EPI, TO, 4><<<dim3((n + cols - 1) / cols, tiles_y, tiles_z), 256, 0, stream>>>(args);
   }
 }
 

@@ -251,8 +251,8 @@ extern "C" long long velox_routed_plan_elems(int pairs, int experts) {
 
 extern "C" int velox_routed_max_tiles(int pairs, int experts) { return (pairs + RT_BM - 1) / RT_BM + experts; }
 
-// tile_rows: 64, or 128 for the matrix-core products of a step with many rows per expert.  The plan's layout is that of
-// 64-row tiles either way (the most tiles there can be).
+// tile_rows: 64, or 128 for the matrix-core products of more than PLAN_COPY_PAIRS pairs.  The plan's layout is that of 64-row
+// tiles either way (the most tiles there can be).
 // x, sorted, pair_weight, top, hidden, scale: see routed_plan_kernel (sorted == nullptr: the plan alone).
 extern "C" int velox_routed_plan(const int* choice, int pairs, int experts, int* plan, int tile_rows, const void* x, void* sorted, const float* pair_weight,
                                  int top, int hidden, int scale, hipStream_t stream) {
@@ -433,20 +433,10 @@ extern "C" int velox_grouped_down(const void* act, const void* down, float* y, c
 }
 
 // ---------------------------------------------------------------------------------------------
-// bfloat16 on the matrix cores: the rows of x are first copied into the order of the plan (and scaled, when the pair's
-// weight scales the expert's input: float32 product, one rounding), then both grouped products read sorted rows.
+// bfloat16 on the matrix cores.  A step of few pairs reads rows that the plan's kernel has copied into its order (scaled, when
+// the pair's weight scales the expert's input: float32 product, one rounding); a larger one fetches the rows of x through the
+// plan and scales the first product's float32 sums.
 // ---------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) routed_gather_kernel(const bf16_t* __restrict__ x, const int* __restrict__ order, const float* __restrict__ pair_weight,
-                                                            bf16_t* __restrict__ sorted, int top, int hidden, int scale, const int* __restrict__ placed) {
-  const int row = blockIdx.x;
-  if (row >= *placed) return;  // (pairs whose expert the plan leaves out have no row: `order` ends at the placed ones)
-  const int pair = order[row];
-  const bf16_t* src = x + (size_t)(pair / top) * hidden;
-  bf16_t* dst = sorted + (size_t)row * hidden;
-  const float w = scale ? pair_weight[pair] : 1.f;
-  for (int i = threadIdx.x; i < hidden; i += blockDim.x) dst[i] = scale ? from_f32<bf16_t>(to_f32(src[i]) * w) : src[i];
-}
-
 static GroupedArgs routed_args(const void* a, const void* w, void* out, const int* plan, int pairs, int experts, int n, int k, int w_rows) {
   GroupedArgs args = {};
   args.a = (const bf16_t*)a;
@@ -464,32 +454,31 @@ static GroupedArgs routed_args(const void* a, const void* w, void* out, const in
   return args;
 }
 
-// x [T, hidden] -> sorted [pairs, hidden] -> act [pairs, inter] -> y [pairs, hidden] float32.  Needs hidden % 8 == 0 and
-// inter % 8 == 0 (the caller checks).
-extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, const void* down, void* sorted, void* act, float* y, const int* plan,
+// x [T, hidden] -> act [pairs, inter] -> y [pairs, hidden] float32.  Needs hidden % 8 == 0 and inter % 8 == 0 (the caller
+// checks).  `sorted` [pairs, hidden]: the rows as the plan's kernel has copied them, for up to PLAN_COPY_PAIRS pairs; more
+// pairs come with `x` and a plan of tiles of GM_TILE_ROWS rows.
+extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, const void* down, const void* sorted, void* act, float* y, const int* plan,
                                           const float* pair_weight, int pairs, int experts, int top, int inter, int hidden, int scale_input,
-                                          int tile_rows, float alpha, float limit, float shift, int ungated, hipStream_t stream) {
+                                          float alpha, float limit, float shift, int ungated, hipStream_t stream) {
   // `ungated` > 0: `gate_up` holds [experts * inter, hidden] (up rows only) and the unit is ungated_act(up, ungated)
   if (pairs <= 0) return 0;
-  if (hidden % 8 != 0 || inter % 8 != 0) return -1;
+  const void* rows = pairs <= PLAN_COPY_PAIRS ? sorted : x;
+  if (hidden % 8 != 0 || inter % 8 != 0 || top < 1 || rows == nullptr || (uintptr_t)rows % 16 != 0) return -1;
   const int max_tiles = velox_routed_max_tiles(pairs, experts);
   if (max_tiles > 65535) return -1;
-  const int* order = plan + 1 + (experts + 1);
-  if (x != nullptr)  // (nullptr: the plan kernel has copied the rows already)
-    routed_gather_kernel<<<pairs, 256, 0, stream>>>((const bf16_t*)x, order, pair_weight, (bf16_t*)sorted, top, hidden, scale_input, plan + 1 + experts);
-  if (ungated > 0) {
-    GroupedArgs first = routed_args(sorted, gate_up, act, plan, pairs, experts, inter, hidden, inter);
-    first.act = ungated;
-    grouped_mfma_launch<GM_ACT, bf16_t>(first, pairs, tile_rows, max_tiles, 1, stream);
-  } else {
-    GroupedArgs glu = routed_args(sorted, gate_up, act, plan, pairs, experts, inter, hidden, 2 * inter);
-    glu.unit = GluUnit{alpha, limit, shift};
-    grouped_mfma_launch<GM_GLU, bf16_t>(glu, pairs, tile_rows, max_tiles, 1, stream);
+  GroupedArgs first = routed_args(rows, gate_up, act, plan, pairs, experts, inter, hidden, ungated > 0 ? inter : 2 * inter);
+  if (rows == x) {
+    first.gather_top = top;
+    first.row_scale = scale_input ? pair_weight : nullptr;
   }
+  first.act = ungated;
+  first.unit = GluUnit{alpha, limit, shift};
+  if (ungated > 0) grouped_mfma_launch<GM_ACT, bf16_t>(first, pairs, max_tiles, 1, stream);
+  else grouped_mfma_launch<GM_GLU, bf16_t>(first, pairs, max_tiles, 1, stream);
   GroupedArgs last = routed_args(act, down, y, plan, pairs, experts, hidden, inter, hidden);
   // (a weight on the experts' OUTPUT is applied where the results are added up, routed_combine with scale_rows: the product
   // itself is the same kernel either way)
-  grouped_mfma_launch<GM_PLAIN, float>(last, pairs, tile_rows, max_tiles, 1, stream);
+  grouped_mfma_launch<GM_PLAIN, float>(last, pairs, max_tiles, 1, stream);
   VELOX_RETURN_LAUNCH_STATUS();
 }
 
