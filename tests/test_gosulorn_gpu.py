@@ -521,3 +521,44 @@ def test_the_replay_program_itself(tmp_path):
         assert not (out / "1.f32").exists()
         got = torch.from_numpy(np.concatenate([np.fromfile(out / "0.f32", dtype="<f4").reshape(2, -1), np.fromfile(out / "2.f32", dtype="<f4").reshape(1, -1)]))
         close(got, logits_of(config, weights, tokens)[[0, 16, 29]], dtype)
+
+
+# -- long portions in chunks of 16 tokens ------------------------------------------------------------------------------------
+@pytest.mark.parametrize("rule, per_channel, heads, kv_heads, dim, vdim", [("delta", True, 2, 2, 128, 128), ("delta", False, 4, 2, 64, 48), ("additive", True, 2, 2, 128, 80),
+                                                                           ("delta", True, 3, 3, 64, 20), ("additive", False, 1, 1, 64, 16), ("delta", True, 2, 1, 128, 33)])
+@pytest.mark.parametrize("strength", [0.01, 3.0, 200.0])
+def test_chunks_of_the_recurrences_against_a_loop_in_float64(ops, rule, per_channel, heads, kv_heads, dim, vdim, strength):
+    """Portions that end inside, at and just behind a chunk, single tokens beside them; decays near 1, ordinary and so strong that a
+    chunk's products underflow.  Every sum is float32 over at most a state's column (dim terms) and a chunk's 16 tokens, and the
+    rule contracts (decays at most 1, unit keys, gates below 1), so an error stays near its token's: 64 float32 roundings of the
+    largest value of a head's read-outs or state bound it."""
+    generator = torch.Generator(device="cuda").manual_seed(dim + vdim)
+    lengths = [33, 1, 16, 70, 17]
+    tokens = sum(lengths)
+    drawn = lambda *shape: torch.randn(*shape, generator=generator, device="cuda")  # noqa: E731
+    qk = torch.nn.functional.normalize(drawn(tokens, kv_heads, 2, dim), dim=-1)
+    v = drawn(tokens, heads * vdim + 8)
+    columns = heads * dim if per_channel else heads
+    decay = torch.exp(-strength * torch.rand(tokens, columns, generator=generator, device="cuda") ** 2)
+    beta = torch.rand(tokens, heads, generator=generator, device="cuda") if rule == "delta" else None
+    state = drawn(len(lengths) + 1, heads, dim, vdim)
+    slots = torch.tensor([4, 0, 2, 1, 5], dtype=torch.int32, device="cuda")
+    cu = torch.tensor([0] + lengths, device="cuda").cumsum(0).int()
+    mine = state.clone()
+    got = ops.linear_scan(qk, v, 8, decay, beta, mine, slots, cu, max(lengths), heads, kv_heads, dim, vdim, rule, chunked=True).view(tokens, heads, vdim)
+    want, after = torch.zeros(tokens, heads, vdim, dtype=torch.float64, device="cuda"), state.double()
+    q, k = (qk[:, :, i].double().repeat_interleave(heads // kv_heads, dim=1) for i in (0, 1))
+    values = v[:, 8:].double().view(tokens, heads, vdim)
+    g = decay.double().view(tokens, heads, -1).expand(tokens, heads, dim)
+    for b, slot in enumerate(slots.tolist()):
+        s = after[slot]
+        for t in range(int(cu[b]), int(cu[b + 1])):
+            s = s * g[t][:, :, None]
+            u = values[t] if rule == "additive" else beta[t].double()[:, None] * (values[t] - torch.einsum("hdv,hd->hv", s, k[t]))
+            s = s + k[t][:, :, None] * u[:, None, :]
+            want[t] = torch.einsum("hdv,hd->hv", s, q[t])
+        after[slot] = s
+    bound = 64 * 2.0 ** -24
+    assert float((got.double() - want).abs().max()) <= bound * float(want.abs().max())
+    assert float((mine.double() - after).abs().max()) <= bound * float(after.abs().max())
+    assert torch.equal(mine[3], state[3])  # a slot that no sequence holds

@@ -1,0 +1,377 @@
+// The gated delta rule and gated linear attention over long portions of prompts, in chunks of 16 tokens on the float32 matrix
+// instructions.
+//
+// Per head, with decays g_t (a number or one per key channel, at most 1), key k_t, query q_t, value v_t and update gate b_t:
+//     S <- diag(g_t) S;   u_t = b_t (v_t - S^T k_t)  ("delta")  or  u_t = v_t  ("additive");   S <- S + k_t u_t^T;   o_t = S^T q_t.
+// Inside a chunk let P_t = g_1 .. g_t and P(j, t) = g_(j+1) .. g_t, all per channel.  From the state Z before the chunk
+//     u_t = b_t (v_t - (k_t P_t)^T Z - sum_(j<t) M1_tj u_j),   M1_tj = sum_c k_tc k_jc P(j, t)_c,
+//     o_t = (q_t P_t)^T Z + sum_(j<=t) M3_tj u_j,              M3_tj = sum_c q_tc k_jc P(j, t)_c,
+//     S' = diag(P_16) Z + sum_j (k_j P(j, 16)) u_j^T.
+// With T = (I + diag(b) M1)^-1 diag(b) (unit lower triangular, by substitution; M1 below the diagonal, M3 with it) everything that
+// does not touch the state is worked for all chunks at the same time:
+//     U' = T (k P),  Dv = T V,  R' = q P - M3 U',  Ov = M3 Dv          (additive: Dv = V, R' = q P, Ov = M3 V)
+// and what is left of the dependent chain is, per chunk,   D = Dv - U' Z,   O = R' Z + Ov,   S' = diag(P_16) Z + K'^T D.
+// All of it is float32 and no quotient of decays is ever formed: a decay may underflow to 0 and nothing else does.  M1 and M3 are
+// built from products of rows whose factors are at most 1: at the level of blocks of 2 h tokens (h = 8, 4, 2, 1) a token t of a
+// block's second half and a token j of its first meet as k_t P(m, t) and k_j P(j, m) with m the last token of the first half, so
+// every pair below the diagonal belongs to exactly one level, and a level is one 16 x 16 product over the channels.
+//
+//   linear_chunk_prepare_kernel   a workgroup per chunk and head: a wave per level, then T and the matrices above into `scratch`
+//   linear_chunk_scan_kernel      a workgroup per 16 value columns, head and sequence; a wave holds 16 rows of the state in the
+//                                 matrix instructions' result layout, which is also their operand layout; the waves exchange
+//                                 their parts of D and O through LDS with one barrier a chunk, loads four chunks ahead
+// The first is bound by what it moves (41 KB of records a chunk and head of 128 x 128), the second by the chain: per chunk four
+// matrix instructions, a barrier, a sum over the waves' parts, four more: 0.9 us.  Measured on MI355X, three prompts of 400 to
+// 1,300 tokens (2,421 in all), 8 heads of 128 x 128: 31 + 74 us against 377 us token by token (a column of the state per wave);
+// 16 heads 52 + 80 against 447; additive, 8 heads of 128 x 256: 38 + 47 against 370.
+#include "common.h"
+
+#define CHUNK 16
+#define CHUNK_STRIDE 20  // floats between the rows of a 16 x 16 matrix in LDS (16-byte aligned, rows on different banks)
+
+struct LinearChunkArgs {
+  const float* qk;     // [T, kv_heads, 2, dim]
+  const void* v;       // values of a token's head h at v_at + h * vdim of its row
+  int v_bf16, v_ld, v_at;
+  const float* decay;  // [T, heads] or [T, heads * dim]
+  int decay_per_channel;
+  const float* beta;   // [T, heads] (delta)
+  float* scratch;
+  float* state;        // [slots, heads, dim, vdim]
+  const int* slots;
+  const int* cu_q;
+  float* out;          // [T, heads * vdim]
+  int heads, kv_heads, dim, vdim;
+};
+
+// A chunk and head in `scratch`, in floats: -U' | R' | K' (each 16 * dim), P_16 (dim), Dv | Ov (each 16 * columns).  U' and R' as
+// [dim / 16][16 tokens][16 channels], K' as [dim][16 tokens], Dv and Ov as [columns][16 tokens]: what a wave reads of one of them is
+// one contiguous kilobyte, 16 bytes a lane.
+__host__ __device__ __forceinline__ int chunk_columns(int vdim) { return (vdim + 15) / 16 * 16; }
+__host__ __device__ __forceinline__ size_t chunk_record(int dim, int vdim) { return (size_t)49 * dim + 32 * chunk_columns(vdim); }
+// the first record of a sequence: sequences' chunks never overlap, because floor((a + n) / 16) + 1 >= floor(a / 16) + ceil(n / 16)
+__device__ __forceinline__ int first_chunk(int first_token, int sequence) { return first_token / CHUNK + sequence; }
+
+__device__ __forceinline__ float4_t mfma4(float a, float b, float4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ float4_t four(const float* p) { return *reinterpret_cast<const float4_t*>(p); }
+
+template <bool DELTA>
+__global__ void __launch_bounds__(256) linear_chunk_prepare_kernel(const LinearChunkArgs a) {
+  extern __shared__ float4_t lds_pieces[];
+  float* lds = reinterpret_cast<float*>(lds_pieces);
+  const int h = blockIdx.x, b = blockIdx.z;
+  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
+  const int t0 = lo + blockIdx.y * CHUNK;
+  if (t0 >= hi) return;  // (the whole workgroup)
+  const int count = hi - t0 < CHUNK ? hi - t0 : CHUNK;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = lane & 15, g = lane >> 4;  // column and group of four rows in the matrix instructions' layouts
+  const int dim = a.dim, row = dim + 4;
+  // rows of q, k and the decays (16 x dim each), and 16 x 16 matrices: M1, M3, T, M3 T
+  float* q = lds;
+  float* k = lds + CHUNK * row;
+  float* decays = lds + 2 * CHUNK * row;
+  float* M1 = lds + 3 * CHUNK * row;
+  float* M3 = M1 + CHUNK * CHUNK_STRIDE;
+  float* T = M1 + 2 * CHUNK * CHUNK_STRIDE;
+  float* M3T = M1 + 3 * CHUNK * CHUNK_STRIDE;
+
+  // the rows, four channels a lane at a time (tokens beyond the portion: zeros, with decays of 1)
+  const int quads = dim / 4;
+  const int kv = h / (a.heads / a.kv_heads);
+  for (int at = tid; at < CHUNK * quads; at += 256) {
+    const int j = at / quads, c = 4 * (at - j * quads);
+    const bool there = j < count;
+    const size_t t = t0 + (there ? j : 0);
+    const float* qk = a.qk + (t * a.kv_heads + kv) * 2 * dim + c;
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
+    float4_t dec;
+    if (a.decay_per_channel) {
+      dec = four(a.decay + (t * a.heads + h) * dim + c);
+    } else {
+      const float d = a.decay[t * a.heads + h];
+      dec = float4_t{d, d, d, d};
+    }
+    *reinterpret_cast<float4_t*>(q + j * row + c) = there ? four(qk) : zero;
+    *reinterpret_cast<float4_t*>(k + j * row + c) = there ? four(qk + dim) : zero;
+    *reinterpret_cast<float4_t*>(decays + j * row + c) = there ? dec : one;
+  }
+  __syncthreads();
+
+  // M1 and M3 level by level, a wave each: half = 8, 4, 2, 1; lane (n, g) scales channels 4 g + 16 m .. + 3 of token n's rows
+  {
+    const int half = 8 >> wave;
+    const int middle = (n & ~(2 * half - 1)) + half - 1;  // the last token of the first half of n's block
+    const bool second = (n & half) != 0;
+    const int first = second ? middle + 1 : n + 1, last = second ? n : middle;
+    float4_t m1 = {0.f, 0.f, 0.f, 0.f}, m3 = m1, diagonal = m1;
+    for (int c = 4 * g; c < dim; c += 16) {
+      const float4_t kn = four(k + n * row + c), qn = four(q + n * row + c);
+      float4_t f = {1.f, 1.f, 1.f, 1.f};
+      for (int s = 0; s < half; ++s) {
+        const int t = first + s <= last ? first + s : last;
+        const float4_t d = four(decays + (t < 0 ? 0 : t) * row + c);
+        if (first + s <= last) f *= d;
+      }
+      const float4_t ks = kn * f, qs = qn * f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (DELTA) m1 = mfma4(ks[e], ks[e], m1);
+        m3 = mfma4(qs[e], ks[e], m3);
+      }
+      if (wave == 3) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) diagonal = mfma4(qn[e], kn[e], diagonal);
+      }
+    }
+    // lane (n, g) holds rows 4 g + i of column n; a level owns the pairs (second half, first half) of its blocks
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = 4 * g + i;
+      const bool same = (t & ~(2 * half - 1)) == (n & ~(2 * half - 1));
+      if (same && (t & half) != 0 && (n & half) == 0) {
+        if (DELTA) M1[t * CHUNK_STRIDE + n] = m1[i];
+        M3[t * CHUNK_STRIDE + n] = m3[i];
+      }
+      if (wave == 3 && t == n) M3[t * CHUNK_STRIDE + n] = diagonal[i];
+      if (wave == 2 && t < n) M3[t * CHUNK_STRIDE + n] = 0.f;
+    }
+  }
+  // the running products: a lane walks one channel forwards (k P and q P, in place behind the barrier) or backwards (K')
+  __syncthreads();
+  const int record_at = first_chunk(lo, b) + blockIdx.y;
+  float* record = a.scratch + ((size_t)record_at * a.heads + h) * chunk_record(dim, a.vdim);
+  float* record_k = record + 32 * dim;
+  float* record_p = record + 48 * dim;
+  for (int c = tid; c < dim; c += 256) {
+    float p = 1.f;
+    float4_t kept[4];
+#pragma unroll
+    for (int t = CHUNK - 1; t >= 0; --t) {
+      kept[t >> 2][t & 3] = k[t * row + c] * p;
+      p *= decays[t * row + c];
+    }
+    record_p[c] = p;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) *reinterpret_cast<float4_t*>(record_k + (size_t)c * CHUNK + 4 * s) = kept[s];
+    p = 1.f;
+#pragma unroll
+    for (int t = 0; t < CHUNK; ++t) {
+      p *= decays[t * row + c];
+      k[t * row + c] *= p;
+      q[t * row + c] *= p;
+    }
+  }
+  if (DELTA && wave == 3) {  // column n of T, by substitution (the four groups of lanes do the same)
+    float x[CHUNK];
+    const float own = n < count ? a.beta[(size_t)(t0 + n) * a.heads + h] : 0.f;
+#pragma unroll
+    for (int t = 0; t < CHUNK; ++t) {
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < t; ++j) sum += M1[t * CHUNK_STRIDE + j] * x[j];
+      const float bt = __shfl(own, t, VELOX_WAVE);
+      x[t] = (t == n ? 1.f : 0.f) - bt * sum;
+    }
+    if (g == 0) {
+#pragma unroll
+      for (int t = 0; t < CHUNK; ++t) T[t * CHUNK_STRIDE + n] = x[t] * own;
+    }
+  }
+  __syncthreads();
+  if (DELTA && wave == 0) {  // M3 T
+    const float4_t x = four(M3 + n * CHUNK_STRIDE + 4 * g);
+    float4_t m = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m = mfma4(x[e], T[(4 * g + e) * CHUNK_STRIDE + n], m);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) M3T[(4 * g + i) * CHUNK_STRIDE + n] = m[i];
+  }
+  if (DELTA) __syncthreads();
+  const float4_t t4 = DELTA ? four(T + n * CHUNK_STRIDE + 4 * g) : float4_t{}, m3t = DELTA ? four(M3T + n * CHUNK_STRIDE + 4 * g) : float4_t{};
+  for (int tile = wave; tile < dim / 16; tile += 4) {  // -U' and R', 16 channels at a time
+    float4_t up = {0.f, 0.f, 0.f, 0.f}, rp;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rp[i] = q[(4 * g + i) * row + tile * 16 + n];
+    if (DELTA) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float y = k[(4 * g + e) * row + tile * 16 + n];
+        up = mfma4(-t4[e], y, up);
+        rp = mfma4(-m3t[e], y, rp);
+      }
+    }
+    float* to = record + tile * 256 + n;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (DELTA) to[(4 * g + i) * 16] = up[i];
+      to[16 * dim + (4 * g + i) * 16] = rp[i];
+    }
+  }
+  const float4_t m3 = four(M3 + n * CHUNK_STRIDE + 4 * g);
+  const int columns = chunk_columns(a.vdim);
+  float* record_d = record + 49 * dim;
+  for (int tile = wave; tile < columns / 16; tile += 4) {  // Dv and Ov, 16 columns of values at a time
+    const int column = tile * 16 + n;
+    const size_t at = (size_t)t0 * a.v_ld + a.v_at + (size_t)h * a.vdim + (column < a.vdim ? column : a.vdim - 1);
+    float4_t v, dv = {0.f, 0.f, 0.f, 0.f}, ov = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const size_t token = at + (size_t)(4 * g + e < count ? 4 * g + e : 0) * a.v_ld;
+      const float x = a.v_bf16 ? to_f32(((const bf16_t*)a.v)[token]) : ((const float*)a.v)[token];
+      v[e] = 4 * g + e < count ? x : 0.f;
+    }
+    if (DELTA) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dv = mfma4(t4[e], v[e], dv);
+    } else {
+      dv = v;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ov = mfma4(m3[e], dv[e], ov);
+    *reinterpret_cast<float4_t*>(record_d + (size_t)column * CHUNK + 4 * g) = dv;
+    *reinterpret_cast<float4_t*>(record_d + (size_t)(columns + column) * CHUNK + 4 * g) = ov;
+  }
+}
+
+// What a wave reads of one chunk, in registers: loaded SCAN_AHEAD chunks before it is worked.
+template <int WAVES>
+struct ChunkOperands {
+  float4_t up, rp, k, p, dv;
+  float ov;  // of the read-out that the lane finishes
+};
+#define SCAN_AHEAD 4
+
+// (at most 256 registers a wave: the matrix instructions then keep the state in ordinary registers)
+template <int WAVES, bool DELTA>
+__global__ void __launch_bounds__(64 * WAVES, 2) linear_chunk_scan_kernel(const LinearChunkArgs a) {
+  __shared__ float4_t parts[2][2][WAVES][64];  // [buffer][D, O][wave][lane]
+  // (heads lie along the grid's first dimension in both kernels: with a multiple of 8 heads the workgroups that read a record run
+  // on the XCD that wrote it and share it in that XCD's L2)
+  const int h = blockIdx.x, tile = blockIdx.y, b = blockIdx.z;
+  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
+  if (hi <= lo) return;  // (the whole workgroup)
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = lane & 15, g = lane >> 4;
+  constexpr int dim = 16 * WAVES;
+  static_assert(WAVES >= 4, "a chunk's 256 read-outs are finished by the first 256 lanes");
+  const int vdim = a.vdim, columns = chunk_columns(vdim);
+  const int column = tile * 16 + n;
+  const bool live = column < vdim;
+  const int chunks = (hi - lo + CHUNK - 1) / CHUNK;
+  const size_t stride = (size_t)a.heads * chunk_record(dim, vdim);  // between a sequence's records of this head
+  // a lane's places in a record, in floats (the record's own address is the same for the whole wave and moves from chunk to chunk)
+  const uint32_t rows_at = wave * 256 + n * 16 + 4 * g, decays_at = 48 * dim + wave * 16 + 4 * g, column_at = 49 * dim + column * CHUNK + 4 * g;
+  // the read-out that a lane finishes, by its place in the order in which the parts lie in LDS
+  const int out_t = ((tid >> 6) & 3) * 4 + (tid & 3), out_e = (tid >> 2) & 15;
+  const uint32_t read_at = 49 * dim + (columns + tile * 16 + out_e) * CHUNK + out_t;
+  const float* next = a.scratch + ((size_t)first_chunk(lo, b) * a.heads + h) * chunk_record(dim, vdim);
+  int asked = 0;  // chunks asked for so far
+  auto load = [&](ChunkOperands<WAVES>& o) {
+    const float* record = next;
+    if (DELTA) o.up = four(record + rows_at);
+    o.rp = four(record + 16 * dim + rows_at);
+    o.k = four(record + 32 * dim + rows_at);
+    o.p = four(record + decays_at);
+    o.dv = four(record + column_at);
+    o.ov = record[read_at];
+    ++asked;
+    if (asked < chunks) next += stride;  // (beyond the last chunk the last one is asked for again)
+  };
+
+  float* S = a.state + (((size_t)a.slots[b] * a.heads + h) * dim + wave * 16 + 4 * g) * vdim + (live ? column : vdim - 1);
+  float4_t z;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) z[i] = S[(size_t)i * vdim];
+
+  const size_t out_row = (size_t)a.heads * vdim;
+  float* out = a.out + (size_t)lo * out_row + (size_t)h * vdim + tile * 16;
+  int left = hi - lo;  // tokens from the current chunk on
+
+  auto work = [&](int buffer, const ChunkOperands<WAVES>& o) {
+    float4_t d = {0.f, 0.f, 0.f, 0.f}, read = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (DELTA) d = mfma4(o.up[e], z[e], d);
+      read = mfma4(o.rp[e], z[e], read);
+    }
+    if (DELTA) parts[buffer][0][wave][lane] = d;
+    parts[buffer][1][wave][lane] = read;
+    z *= o.p;
+    if (!DELTA) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z = mfma4(o.k[e], o.dv[e], z);
+    }
+    __syncthreads();  // (one a chunk: a buffer is written again behind the next chunk's barrier)
+    if (DELTA) {
+      d = o.dv;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) d += parts[buffer][0][w][lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z = mfma4(o.k[e], d[e], z);
+    }
+    // the chunk's read-outs: 256 of them over the workgroup's lanes
+    const float* sums = reinterpret_cast<const float*>(parts[buffer][1]);
+    if (tid < 256) {
+      float v = o.ov;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) v += sums[w * 256 + tid];
+      if (out_t < left && tile * 16 + out_e < vdim) out[out_t * out_row + out_e] = v;
+    }
+    left -= CHUNK;
+    out += CHUNK * out_row;
+  };
+
+  // Loads are asked for whether or not there is a chunk that far ahead (then the last one's again): the same number of them lies
+  // between a chunk's loads and its work on every path, so that waiting for the one does not wait for the others.
+  ChunkOperands<WAVES> ops[SCAN_AHEAD];
+#pragma unroll
+  for (int j = 0; j < SCAN_AHEAD; ++j) load(ops[j]);
+  int c = 0;
+  for (; c + SCAN_AHEAD <= chunks; c += SCAN_AHEAD) {
+#pragma unroll
+    for (int j = 0; j < SCAN_AHEAD; ++j) {
+      work(j & 1, ops[j]);
+      load(ops[j]);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < SCAN_AHEAD - 1; ++j)
+    if (c + j < chunks) work(j & 1, ops[j]);  // (the same for the whole workgroup)
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[(size_t)i * vdim] = z[i];
+  }
+}
+
+// float32 elements of the scratch of a step; 0: these sizes are not for these kernels.  Key heads of 64 and 128 channels: the sizes
+// whose long portions ran a column of the state per wave, in an order of sums of their own.  (Other sizes are worked in one
+// order whether a portion is long or short, and larger ones would need more than a workgroup's waves for a column tile.)
+extern "C" long long velox_linear_chunk_scratch_elems(int tokens, int num_seqs, int heads, int dim, int vdim) {
+  if ((dim != 64 && dim != 128) || vdim < 1) return 0;
+  return ((long long)tokens / CHUNK + num_seqs + 1) * heads * (long long)chunk_record(dim, vdim);
+}
+
+template <bool DELTA>
+static void linear_chunk_launch(const LinearChunkArgs& a, int num_seqs, int max_q_len, hipStream_t stream) {
+  const size_t lds = (size_t)CHUNK * (3 * (a.dim + 4) + 4 * CHUNK_STRIDE) * sizeof(float);
+  linear_chunk_prepare_kernel<DELTA><<<dim3(a.heads, (max_q_len + CHUNK - 1) / CHUNK, num_seqs), 256, lds, stream>>>(a);
+  const dim3 grid(a.heads, chunk_columns(a.vdim) / 16, num_seqs);
+  if (a.dim == 64) linear_chunk_scan_kernel<4, DELTA><<<grid, 256, 0, stream>>>(a);
+  else linear_chunk_scan_kernel<8, DELTA><<<grid, 512, 0, stream>>>(a);
+}
+
+// beta: nullptr for the additive rule.  qk and a decay per channel are read in 16-byte pieces (dim is a multiple of 16; the caller
+// checks that the bases are aligned).
+extern "C" int velox_linear_chunk_scan(const float* qk, const void* v, int v_dtype, int v_ld, int v_at, const float* decay, int decay_per_channel,
+                                       const float* beta, float* scratch, float* state, const int* slots, const int* cu_q, float* out, int num_seqs,
+                                       int max_q_len, int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
+  if (num_seqs <= 0 || max_q_len <= 0) return 0;
+  if (velox_linear_chunk_scratch_elems(max_q_len, num_seqs, heads, dim, vdim) == 0 || heads < 1 || heads > 65535 || num_seqs > 65535 ||
+      max_q_len > 65535 * CHUNK || vdim > 65535 * 16 || kv_heads < 1 || heads % kv_heads != 0 || !scratch)
+    return (int)hipErrorInvalidValue;
+  LinearChunkArgs a{qk, v, v_dtype == VELOX_BF16, v_ld, v_at, decay, decay_per_channel, beta, scratch, state, slots, cu_q, out, heads, kv_heads, dim, vdim};
+  if (beta) linear_chunk_launch<true>(a, num_seqs, max_q_len, stream);
+  else linear_chunk_launch<false>(a, num_seqs, max_q_len, stream);
+  VELOX_RETURN_LAUNCH_STATUS();
+}

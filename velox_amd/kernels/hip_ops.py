@@ -187,6 +187,10 @@ class HipOps:
         c.velox_poly_norm.argtypes = [_P, _P, _P, _I, _I, _F, _I, _P]
         c.velox_removal_chunk_scan.argtypes = [_P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _P, _P, _I, _I, _P]
         c.velox_removal_chunk_scan.restype = _I
+        c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]
+        c.velox_linear_chunk_scan.restype = _I
+        c.velox_linear_chunk_scratch_elems.argtypes = [_I, _I, _I, _I, _I]
+        c.velox_linear_chunk_scratch_elems.restype = ctypes.c_longlong
         c.velox_removal_chunk_scratch_elems.argtypes = [_I, _I, _I, _I, _I, _I]
         c.velox_removal_chunk_scratch_elems.restype = ctypes.c_longlong
         for fn in (c.velox_removal_prepare, c.velox_gated_scan, c.velox_norm_add_norm, c.velox_poly_norm):
@@ -1275,11 +1279,16 @@ class HipOps:
 
     _SCAN_RULES = {"additive": 0, "delta": 1, "removal": 2}
 
-    def linear_scan(self, qk, v_source, v_at, decay, beta, state, slots, cu_q, max_q_len, heads, kv_heads, dim, vdim, rule):
+    LINEAR_CHUNK_TOKENS = 32  # portions at least this long go through the chunked kernels where the sizes are theirs
+    LINEAR_CHUNK_SCRATCH = 1 << 28  # the most float32 numbers of scratch they may ask for (1 GB: 13,000 tokens of 32 heads of 128 x 128)
+
+    def linear_scan(self, qk, v_source, v_at, decay, beta, state, slots, cu_q, max_q_len, heads, kv_heads, dim, vdim, rule, chunked: Optional[bool] = None):
         """Per sequence and head, token by token from ``state[slot, head]`` ([dim, vdim] float32), which is written back:
         ``S <- g S`` (rows); ``u = beta (v - S^T k)`` (rule ``"delta"``) or ``u = v`` (``"additive"``); ``S <- S + k u^T``; ``o = S^T q``.
         Rule ``"removal"``: ``qk`` holds a third vector ``b`` per head and token, and ``S <- g S - b (k^T S) + k (beta v)^T`` with both
-        terms on the old state.  ``decay`` is [T, heads] or [T, heads * dim].  Returns float32 [T, heads * vdim]."""
+        terms on the old state.  ``decay`` is [T, heads] or [T, heads * dim].  Returns float32 [T, heads * vdim].  Steps of the first two
+        rules with a long portion are worked in chunks of 16 tokens on the matrix cores (key heads of 64 or 128 channels), all others
+        token by token; ``chunked`` decides it for a test."""
         if rule not in self._SCAN_RULES:
             raise KernelError(f"linear_scan: rule {rule!r} is not implemented ({', '.join(self._SCAN_RULES)})")
         delta = rule != "additive"
@@ -1303,6 +1312,18 @@ class HipOps:
         self._check("cu_q", cu_q, torch.int32, (slots.shape[0] + 1,))
         self.linear_scan_supports(dim, vdim)
         out = torch.empty((tokens, heads * vdim), dtype=torch.float32, device=self.device)
+        scratch_elems = 0
+        if rule != "removal" and chunked is not False and max_q_len >= (1 if chunked else self.LINEAR_CHUNK_TOKENS):
+            scratch_elems = int(self._core.velox_linear_chunk_scratch_elems(tokens, slots.shape[0], int(heads), int(dim), int(vdim)))
+            scratch_elems = scratch_elems if scratch_elems <= self.LINEAR_CHUNK_SCRATCH else 0
+        if chunked and scratch_elems == 0:
+            raise KernelError(f"linear_scan: heads of {dim} channels (rule {rule!r}, {tokens} tokens) are not the chunked kernels'")
+        if scratch_elems:
+            scratch = torch.empty(scratch_elems, dtype=torch.float32, device=self.device)
+            self._launched(self._core.velox_linear_chunk_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
+                                                              _ptr(beta) if delta else _P(0), _ptr(scratch), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out),
+                                                              slots.shape[0], int(max_q_len), int(heads), int(kv_heads), int(dim), int(vdim), self._stream()), "linear_chunk_scan")
+            return out
         status = self._core.velox_linear_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
                                               _ptr(beta) if delta else _P(0), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out), slots.shape[0], int(max_q_len), int(heads),
                                               int(kv_heads), int(dim), int(vdim), self._SCAN_RULES[rule], self._stream())
@@ -1646,7 +1667,7 @@ class HipOps:
         # few pairs: the plan's kernel also copies the rows into its order; more of them are fetched where they are
         copied_by_plan = on_matrix_cores and pairs <= self.FEW_PAIRS
         ordered = torch.empty((pairs, hidden), dtype=x.dtype, device=self.device) if copied_by_plan else None
-        if on_matrix_cores and x.data_ptr() % 16 != 0:
+        if on_matrix_cores and not copied_by_plan and x.data_ptr() % 16 != 0:
             x = x.clone()
         self._launched(self._core.velox_routed_plan(_ptr(choice), pairs, num_experts, _ptr(plan), tile_rows, _ptr(x) if copied_by_plan else _P(0),
                                                     _ptr(ordered) if copied_by_plan else _P(0), _ptr(weight), top, hidden, int(bool(scale_input)), self._stream()),
