@@ -1209,3 +1209,17 @@ def test_grouped_products_at_the_edges_of_their_tiles(ops, rows, hidden, inter, 
     want += (x.double()[:, None, :] * (weight.double() * none)[:, :, None]).sum(1)
     bound = (2.0 ** -8 + 2e-5) * spread + 2.0 ** -8 * 1.01 * want.abs() + 1e-6
     assert torch.all((got.double() - want).abs() <= bound), float(((got.double() - want).abs() / bound).max())
+
+
+@pytest.mark.parametrize("m, n, k", [(17, 64, 4), (33, 65, 36), (64, 100, 256), (70, 333, 260), (65, 2048, 1540), (200, 2048, 516), (300, 6500, 132), (610, 1536, 288), (1025, 4100, 100)])
+def test_float32_products_on_the_matrix_instructions(ops, m, n, k):
+    """Every tile and both numbers of sets of waves, remainders in all three sizes.  A sum of at most GEMM_FOLD = 128 terms, then of as many
+    such sums, all float32: off by at most (128 + k / 128 + 2) 2^-24 of the sum of the terms' sizes.  The same row in a batch of
+    another size, which takes another tile, has the same bits."""
+    generator = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w, bias = (torch.randn(*shape, generator=generator, device="cuda") for shape in ((m, k), (n, k), (n,)))
+    got = ops.gemm_fma(a, w, bias, torch.float32)
+    want = a.double() @ w.double().T + bias.double()
+    bound = (128 + k / 128 + 2) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + bias.double().abs())
+    assert torch.all((got.double() - want).abs() <= bound)
+    assert torch.equal(ops.gemm_fma(a[-17:].contiguous(), w, bias, torch.float32), got[-17:])

@@ -1,9 +1,10 @@
 // out[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) with float32 accumulation, for gfx950.
 //
-// `gemm_fma_kernel` is the exact path: operands are widened to float32 (exactly, for bfloat16) and
-// multiplied with plain fused multiply-adds, so a float32 run never touches a reduced-precision
-// matrix mode.  It also serves operand mixes no library call covers (bfloat16 activations with
-// weights a checkpoint stores in float32).  Each output element is summed over k in one fixed
+// `gemm_fma_kernel` widens its operands to float32 (exactly, for bfloat16) and multiplies them with
+// plain fused multiply-adds.  It serves operand mixes no library call covers (bfloat16 activations with
+// weights a checkpoint stores in float32) and float32 rows that are not whole 16-byte pieces; other
+// float32 products run on the float32 matrix instructions (gemm_mfma_f32_kernel), so a float32 run
+// never touches a reduced-precision matrix mode.  Each output element is summed over k in one fixed
 // order by one thread, so a row's result does not depend on the other rows of the batch.  The sum
 // is built from sums of GEMM_FOLD consecutive terms, each started at zero: the rounding error of a
 // long sum (the down projection adds 18944 terms) then grows with the square roots of the two
@@ -81,6 +82,201 @@ __global__ void __launch_bounds__(256) gemm_fma_kernel(const TA* __restrict__ a,
       out[(size_t)row * n + col] = from_f32<TO>(v);
     }
   }
+}
+
+// The float32 product of more than 16 rows on the matrix cores (v_mfma_f32_16x16x4_f32: float32 operands, products and sums, twice
+// the rate of scalar multiply-adds).  A set of four waves owns 32 RT x 32 CT outputs, a wave 16 RT x 16 CT of them; a step is 32
+// indices, so a row of either operand is 128 bytes of LDS, eight pieces of 16, exchanged by an XOR with the row's low three
+// bits (no bank conflicts), filled by loads that write LDS directly, STAGES - 1 steps ahead, with one barrier per step.  Lane
+// (g, i) takes indices 4 g .. 4 g + 3 of every 16 of row i as one 16-byte read and feeds one of them to each of four matrix
+// instructions: both operands in the same order of k.  As in the kernel above an output is built from sums of GEMM_FOLD terms;
+// here those of either half of k are added up first.  Where a step has too few tiles to fill the card, two sets of waves take
+// the halves (SETS = 2), otherwise one set takes both in turn: an output's order of additions depends on k alone, whichever
+// kernel a batch size leads to.
+// Bound by the matrix instructions (157 TFLOP/s) where there are tiles enough, by how far ahead the loads are where there are
+// few.  Tiles follow one another along the rows of A on the same XCD, so the rows of W that they share leave its L2.
+// Measured on MI355X (us, multiply-adds -> this): 616 rows, 1,536 -> 17,920: 593 -> 360 (94 TFLOP/s); 616 rows, 8,960 -> 1,536: 590 ->
+// 182; 2,048 rows, 1,536 -> 17,920: 1,576 -> 986 (114 TFLOP/s); 64 rows, 8,960 -> 1,536: 582 -> 70; error against float64 1.5e-07 to
+// 1.7e-07 of the result's norm (before 1.5e-07 to 1.8e-07).
+static __device__ __attribute__((aligned(16))) const unsigned int gemm_zero_piece[4] = {0u, 0u, 0u, 0u};
+
+#define GEMM_XCDS 8
+
+template <int RT, int CT, int SETS, int STAGES>
+__global__ void __launch_bounds__(256 * SETS) __attribute__((amdgpu_waves_per_eu(2, 4))) gemm_mfma_f32_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                                                                              const float* __restrict__ bias, float* __restrict__ out, int m, int n, int k) {
+  constexpr int ROWS = 32 * RT, COLS = 32 * CT, WAVES = 4;
+  constexpr int A_LOADS = ROWS / 8 / WAVES, W_LOADS = COLS / 8 / WAVES, LOADS = A_LOADS + W_LOADS;
+  constexpr int BYTES = (ROWS + COLS) * 128;
+  __shared__ __attribute__((aligned(1024))) char smem_all[SETS][STAGES][BYTES];
+  const int row_tiles = (m + ROWS - 1) / ROWS, total_tiles = row_tiles * ((n + COLS - 1) / COLS);
+  const int share = (total_tiles + GEMM_XCDS - 1) / GEMM_XCDS;
+  const int mine = (int)(blockIdx.x / GEMM_XCDS), tile = (int)(blockIdx.x % GEMM_XCDS) * share + mine;
+  if (mine >= share || tile >= total_tiles) return;  // (uniform over the workgroup)
+  const int m0 = tile % row_tiles * ROWS, n0 = tile / row_tiles * COLS;
+
+  const int set = SETS == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+  char (*const smem)[BYTES] = smem_all[set];
+  const int i = lane & 15, g = lane >> 4;
+  const int piece = 4 * ((lane & 7) ^ (lane >> 3));  // first index of the piece this lane asks for, in every load
+  const float* a_at[A_LOADS];
+  const float* w_at[W_LOADS];
+#pragma unroll
+  for (int q = 0; q < A_LOADS; ++q) a_at[q] = a + (size_t)min(m0 + 8 * (wave + WAVES * q) + (lane >> 3), m - 1) * k + piece;
+#pragma unroll
+  for (int q = 0; q < W_LOADS; ++q) w_at[q] = w + (size_t)min(n0 + 8 * (wave + WAVES * q) + (lane >> 3), n - 1) * k + piece;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int a_byte = (wm * 16 * RT + i) * 128, w_byte = ROWS * 128 + (wn * 16 * CT + i) * 128;
+  // k in two halves that meet at a multiple of GEMM_FOLD: two sets of waves take one each, or one set both in turn.  (The first is
+  // the longer one, and two sets run its number of steps.)
+  const int middle = min(k, (k + 2 * GEMM_FOLD - 1) / (2 * GEMM_FOLD) * GEMM_FOLD);
+
+  float4_t sum[CT][RT], acc[CT][RT], total[CT][RT];
+  auto half_of_k = [&](int begin, int end, int steps) {
+    auto ask = [&](int s, int buffer) {
+      const int k0 = begin + 32 * s;
+      const bool beyond = k0 + piece >= end;  // (zeros behind the end of the half)
+#pragma unroll
+      for (int q = 0; q < A_LOADS; ++q) load_to_lds_16(beyond ? reinterpret_cast<const float*>(gemm_zero_piece) : a_at[q] + k0, smem[buffer] + 1024 * (wave + WAVES * q));
+#pragma unroll
+      for (int q = 0; q < W_LOADS; ++q) load_to_lds_16(beyond ? reinterpret_cast<const float*>(gemm_zero_piece) : w_at[q] + k0, smem[buffer] + ROWS * 128 + 1024 * (wave + WAVES * q));
+    };
+    float4_t a_op[2][RT], w_op[2][CT];
+    auto fetch = [&](int part, int buffer) {
+      const char* base = smem[buffer];
+      const int place = ((4 * part + g) ^ (i & 7)) * 16;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) w_op[part][ct] = *reinterpret_cast<const float4_t*>(base + w_byte + ct * 2048 + place);
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) a_op[part][rt] = *reinterpret_cast<const float4_t*>(base + a_byte + rt * 2048 + place);
+    };
+    auto multiply = [&](int part) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w_op[part][ct][e], a_op[part][rt][e], acc[ct][rt], 0, 0, 0);
+    };
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = total[ct][rt] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s)
+      if (s < steps) ask(s, s);
+    // the first step's loads have landed when at most those of the later steps that were asked for are under way
+    if (steps >= STAGES - 1) wait_for_loads<(STAGES - 2) * LOADS>();
+    else wait_for_loads<0>();
+    __syncthreads();
+    fetch(0, 0);
+    int buffer = 0;
+    for (int s = 0; s < steps; ++s) {
+      fetch(1, buffer);
+      int freed = buffer + STAGES - 1;
+      if (freed >= STAGES) freed -= STAGES;
+      if (s + STAGES - 1 < steps) ask(s + STAGES - 1, freed);  // (the buffer that everybody was done with at the last barrier)
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0);
+      __builtin_amdgcn_sched_barrier(0);
+      buffer = buffer + 1 == STAGES ? 0 : buffer + 1;
+      if (s + 1 < steps) {
+        if (s + STAGES <= steps) wait_for_loads<(STAGES - 2) * LOADS>();
+        else wait_for_loads<0>();
+        __syncthreads();
+        fetch(0, buffer);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(1);
+      if ((s + 1) % (GEMM_FOLD / 32) == 0) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) {
+            total[ct][rt] += acc[ct][rt];
+            acc[ct][rt] = float4_t{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) total[ct][rt] += acc[ct][rt];
+    __syncthreads();  // (everybody is done with the buffers)
+  };
+  if (SETS == 2) {
+    half_of_k(set == 0 ? 0 : middle, set == 0 ? middle : k, (middle + 31) / 32);
+    float4_t* joined = reinterpret_cast<float4_t*>(smem_all[0]) + (threadIdx.x & 255);
+    if (set == 1) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) joined[256 * (ct * RT + rt)] = total[ct][rt];
+    }
+    __syncthreads();
+    if (set == 1) return;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) sum[ct][rt] = total[ct][rt] + joined[256 * (ct * RT + rt)];
+  } else {
+    half_of_k(0, middle, (middle + 31) / 32);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) sum[ct][rt] = total[ct][rt];
+    if (middle < k) {
+      half_of_k(middle, k, (k - middle + 31) / 32);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) sum[ct][rt] += total[ct][rt];
+    }
+  }
+  // lane (g, i) holds outputs 4 g .. + 3 of row i of every tile
+  const bool vec = n % 4 == 0 && ((uintptr_t)out & 15) == 0;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int row = m0 + wm * 16 * RT + rt * 16 + i;
+    if (row >= m) continue;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const int col = n0 + wn * 16 * CT + ct * 16 + 4 * g;
+      float4_t v = sum[ct][rt];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (bias != nullptr && col + j < n) v[j] += bias[col + j];
+      if (vec && col < n) {
+        *reinterpret_cast<float4_t*>(out + (size_t)row * n + col) = v;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (col + j < n) out[(size_t)row * n + col + j] = v[j];
+      }
+    }
+  }
+}
+
+// Which tile, by the number of tiles.  Measured on MI355X (us; 128 x 64 and 64 x 64 by one set | 64 x 64, 32 x 64, 32 x 32 by two):
+//   4,096 rows, 2,048 -> 11,264   1588  1690 | 1900  1960  2900        2,048 rows, 8,960 -> 1,536   614  515 | 532  586  802
+//   616 rows, 1,536 -> 17,920      359   370 |  393   432   583        300 rows, 1,536 -> 17,920    242  197 | 218  212  290
+//   616 rows, 8,960 -> 1,536       329   210 |  182   214   268        616 rows, 1,536 -> 2,048      65   65 |  70   58   66
+//   300 rows, 8,960 -> 1,536       331   204 |  182   119   139        64 rows, 8,960 -> 1,536      330  200 | 178  111   70
+// so: from two workgroups per compute unit on one set, in tiles of 128 rows if few of them stay empty; with about one workgroup
+// per compute unit 64 x 64 by two sets; with fewer the largest tile that still gives most compute units a workgroup.
+static void launch_mfma_f32(const void* a, const void* w, const float* bias, void* out, int m, int n, int k, hipStream_t stream) {
+  auto tiles = [&](int rt, int ct) { return (long long)((m + 32 * rt - 1) / (32 * rt)) * ((n + 32 * ct - 1) / (32 * ct)); };
+#define MFMA(RT, CT, SETS, STAGES)                                                                                                     \
+  gemm_mfma_f32_kernel<RT, CT, SETS, STAGES><<<(unsigned)((tiles(RT, CT) + GEMM_XCDS - 1) / GEMM_XCDS * GEMM_XCDS), 256 * SETS, 0, stream>>>( \
+      (const float*)a, (const float*)w, bias, (float*)out, m, n, k)
+  if (tiles(4, 2) >= 512 && (m + 127) / 128 * 128 * 10 <= m * 11) MFMA(4, 2, 1, 2);
+  else if (tiles(2, 2) >= 512) MFMA(2, 2, 1, 3);
+  else if (tiles(2, 2) >= 200 && tiles(2, 2) <= 256) MFMA(2, 2, 2, 3);
+  else if (tiles(1, 2) >= 200) MFMA(1, 2, 2, 3);
+  else MFMA(1, 1, 2, 3);
+#undef MFMA
 }
 
 // The same product for few rows (M <= 16), where it is bound by reading W once: the decode steps of a float32 run.
@@ -163,6 +359,10 @@ extern "C" int velox_gemm_fma(const void* a, const void* w, const float* bias, v
       case 7: launch_skinny_fma<bf16_t, bf16_t, bf16_t>(a, w, bias, out, m, n, k, stream); break;
       default: return -1;
     }
+    VELOX_RETURN_LAUNCH_STATUS();
+  }
+  if (key == 0 && a_vec && w_vec) {
+    launch_mfma_f32(a, w, bias, out, m, n, k, stream);
     VELOX_RETURN_LAUNCH_STATUS();
   }
   switch (key) {
