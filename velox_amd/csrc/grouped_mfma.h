@@ -41,8 +41,8 @@ struct GroupedArgs {
   const bf16_t* gate;  // GM_GATE: times sigmoid(gate[r * gate_ld + g * gate_group + col * gate_col]); (n, 1) is a number per output, (1, 0) one per group
   long long gate_ld, gate_group, gate_col;
   int act = 0;         // GM_ACT: the result goes through ungated_act(., act)
-  const float* row_scale;  // grouped_tiles_kernel: the sums in front of a GLU or an activation are multiplied with row_scale[order[r]] (nullptr: none)
-  int gather_top = 0;      // grouped_tiles_kernel: > 0: sorted row r is row order[r] / gather_top of `a`
+  const float* row_scale;  // with a plan: the sums in front of a GLU or an activation are multiplied with row_scale[order[r]] (nullptr: none)
+  int gather_top = 0;      // with a plan: > 0: sorted row r is row order[r] / gather_top of `a`
   GluUnit unit = {1.f, INFINITY, 0.f};  // GM_GLU: the unit's middle (see glu_middle)
 };
 
@@ -151,30 +151,15 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
   }
 }
 
-// The same products when no tile has more than 16 MT rows (a decode step's pairs): then a product is bound by reading W
-// once, and what counts is how many loads are in flight.  A workgroup owns 32 output columns (GLU: 16 gate columns and
-// their up columns) of one tile; its four waves split K into quarters, each wave asks for four steps' operands at once,
-// and the waves' sums are added through LDS in the order of the waves (no atomics: the same result on every run).
+// The same products when no tile has more than 64 rows (a decode step's pairs, with a plan): then a product is bound by reading
+// W once, and what counts is how many loads are in flight.  A workgroup owns 32 output columns (GLU: 16 gate columns and
+// their up columns) of one tile; its four waves split K into quarters, each wave asks for four steps' operands at once, W's a
+// round ahead, and the waves' sums are added through LDS in the order of the waves (no atomics: the same result on every
+// run).  A tile works as many 16-row tiles as it has rows, whatever the step's number of pairs would allow.  Measured on MI355X: 64
+// pairs over 32 experts of 4,096 -> 1,408 -> 4,096 122 + 70 us (W: 650 + 325 MB; before: 143 + 82, rows copied by another kernel).
 template <int EPI, typename TO, int MT>
-__global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const GroupedArgs args) {
-  __shared__ float4_t partial[3][2 * MT][64];
-  int group, row0, rows;
-  const int* order = nullptr;
-  if (args.plan != nullptr) {
-    const int tile = blockIdx.y;
-    if (tile >= args.plan[0]) return;  // (uniform over the workgroup)
-    const int* starts = args.plan + 1;
-    order = starts + args.plan_groups + 1;
-    const int* tile_group = order + 2 * (size_t)args.plan_pairs;
-    const int* tile_row = tile_group + args.plan_max_tiles;
-    group = tile_group[tile];
-    row0 = tile_row[tile];
-    rows = min(16 * MT, starts[group + 1] - row0);
-  } else {
-    group = blockIdx.z;
-    row0 = blockIdx.y * 16 * MT;
-    rows = min(16 * MT, args.m - row0);
-  }
+__device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int group, const int row0, const int rows, const int* order,
+                                              float4_t (*partial)[8][64]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int i = lane & 15, g4 = lane >> 4;
   const int n = args.n, k = args.k;
@@ -188,26 +173,40 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
     const int col = min(col0[t] + i, n - 1);
     w_row[t] = w_base + (size_t)(EPI == GM_GLU && t == 1 ? n + col : col) * k + 8 * g4;
   }
-  const bf16_t* a_row[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) a_row[mt] = args.a + (size_t)(row0 + min(mt * 16 + i, rows - 1)) * args.a_ld + (size_t)group * args.a_group + 8 * g4;
   const int quarter = ((k + 127) / 128) * 32;  // indices per wave: a multiple of 32
   const int k_begin = wave * quarter, k_end = min(k, k_begin + quarter);
+  // W is what there is to read: its next step is asked for before the current one is multiplied, and its first before the rows of
+  // `a` have been looked up
+  gm_bf16x8_t wv[2][4], w_next[2][4];
+  auto ask = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) w_next[t][u] = gm_load(w_row[t] + k0 + 32 * u, k0 + 32 * u + 8 * g4 < k_end);
+  };
+  ask(k_begin);
+  const bf16_t* a_row[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    int r = row0 + min(mt * 16 + i, rows - 1);
+    if (args.gather_top > 0) r = order[r] / args.gather_top;
+    a_row[mt] = args.a + (size_t)r * args.a_ld + (size_t)group * args.a_group + 8 * g4;
+  }
   float4_t acc[2][MT];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[t][mt] = float4_t{0.f, 0.f, 0.f, 0.f};
   for (int k0 = k_begin; k0 < k_end; k0 += 128) {
-    gm_bf16x8_t wv[2][4], av[MT][4];
+    gm_bf16x8_t av[MT][4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const bool ok = k0 + 32 * u + 8 * g4 < k_end;
 #pragma unroll
-      for (int t = 0; t < 2; ++t) wv[t][u] = gm_load(w_row[t] + k0 + 32 * u, ok);
+      for (int t = 0; t < 2; ++t) wv[t][u] = w_next[t][u];
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) av[mt][u] = gm_load(a_row[mt] + k0 + 32 * u, ok);
+      for (int mt = 0; mt < MT; ++mt) av[mt][u] = gm_load(a_row[mt] + k0 + 32 * u, k0 + 32 * u + 8 * g4 < k_end);
     }
+    ask(k0 + 128);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -239,14 +238,16 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
     const int r = mt * 16 + i;
     if (r >= rows) continue;
     const size_t out_row = (size_t)(row0 + r) * args.out_ld + (size_t)group * args.out_group;
+    float scale = 1.f;
+    if (EPI != GM_PLAIN && args.row_scale != nullptr) scale = args.row_scale[order[row0 + r]];
 #pragma unroll
     for (int t = 0; t < (EPI == GM_GLU ? 1 : 2); ++t)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int col = col0[t] + 4 * g4 + j;
         if (col >= n) continue;
-        float v = acc[t][mt][j];
-        if (EPI == GM_GLU) v = glu_middle(v, acc[1][mt][j], args.unit);
+        float v = acc[t][mt][j] * scale;
+        if (EPI == GM_GLU) v = glu_middle(v, acc[1][mt][j] * scale, args.unit);
         if (EPI == GM_GATE) {
           const float z = to_f32(args.gate[(size_t)(row0 + r) * args.gate_ld + (size_t)group * args.gate_group + (size_t)col * args.gate_col]);
           v *= 1.f / (1.f + expf(-z));
@@ -255,6 +256,23 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
         out[out_row + col] = from_f32<TO>(v);
       }
   }
+}
+
+template <int EPI, typename TO>
+__global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const GroupedArgs args) {
+  __shared__ float4_t partial[3][8][64];
+  const int tile = blockIdx.y;
+  if (tile >= args.plan[0]) return;  // (uniform over the workgroup)
+  const int* starts = args.plan + 1;
+  const int* order = starts + args.plan_groups + 1;
+  const int* tile_group = order + 2 * (size_t)args.plan_pairs;
+  const int* tile_row = tile_group + args.plan_max_tiles;
+  const int group = tile_group[tile], row0 = tile_row[tile];
+  const int rows = min(64, starts[group + 1] - row0);
+  // (the same for the whole workgroup)
+  if (rows <= 16) few_rows_tile<EPI, TO, 1>(args, group, row0, rows, order, partial);
+  else if (rows <= 32) few_rows_tile<EPI, TO, 2>(args, group, row0, rows, order, partial);
+  else few_rows_tile<EPI, TO, 4>(args, group, row0, rows, order, partial);
 }
 
 // Steps of many rows with a plan: tiles of 128 rows x 256 rows of W, both operands through LDS by loads that write LDS
@@ -444,9 +462,7 @@ static void grouped_mfma_launch(const GroupedArgs& args, int most_rows, int tile
     if (most_rows <= 64) {
       constexpr int COLS = EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS;
       dim3 grid((n + COLS - 1) / COLS, tiles_y, 1);
-      if (most_rows <= 16) grouped_mfma_few_rows_kernel<EPI, TO, 1><<<grid, 256, 0, stream>>>(args);
-      else if (most_rows <= 32) grouped_mfma_few_rows_kernel<EPI, TO, 2><<<grid, 256, 0, stream>>>(args);
-      else grouped_mfma_few_rows_kernel<EPI, TO, 4><<<grid, 256, 0, stream>>>(args);
+      grouped_mfma_few_rows_kernel<EPI, TO><<<grid, 256, 0, stream>>>(args);
       return;
     }
     const int cols = (outputs + GM_TILE_COLS - 1) / GM_TILE_COLS;

@@ -177,70 +177,97 @@ extern "C" int velox_route_top(const float* logits, int* choice, float* weight, 
 // is up to tile_rows consecutive sorted rows of one expert.
 // ---------------------------------------------------------------------------------------------
 #define PLAN_MAX_EXPERTS 2048
-#define PLAN_COPY_PAIRS 64  // up to this many pairs the plan kernel can copy the rows itself
 
-// With `sorted` the kernel also copies the rows of x into the plan's order (scaled by the pair's weight when `scale`), what
-// routed_gather_kernel does: for steps of few pairs, which then run one kernel less.
+// One workgroup, bound by the latency of its few passes over LDS and memory: every pair takes its place among its expert's rows
+// from one LDS atomic (kept in `place` until the experts' first rows are known), and the experts' first rows and tiles come from
+// one scan over the experts, two a thread.  Measured on MI355X: 10,000 pairs over 32 experts 14.0 us, 64 pairs 4.7 (a serial walk
+// over the experts and a second round of atomics 15.2; with the rows of x copied in the same kernel, 64 pairs of 4,096, 23.8).
 __global__ void __launch_bounds__(1024) routed_plan_kernel(const int* __restrict__ choice, int pairs, int experts, int max_tiles, int tile_rows,
-                                                           int* __restrict__ plan, const bf16_t* __restrict__ x, bf16_t* __restrict__ sorted,
-                                                           const float* __restrict__ pair_weight, int top, int hidden, int scale) {
+                                                           int* __restrict__ plan) {
   __shared__ int count[PLAN_MAX_EXPERTS];
-  __shared__ int first[PLAN_MAX_EXPERTS + 1];
-  __shared__ int order_s[PLAN_COPY_PAIRS];
-  int* num_tiles = plan;
+  __shared__ int first[PLAN_MAX_EXPERTS];
+  __shared__ int wave_rows[16], wave_tiles[16];
+  constexpr int BATCH = 4;
   int* starts = plan + 1;
   int* order = starts + experts + 1;
   int* place = order + pairs;
   int* tile_expert = place + pairs;
   int* tile_row = tile_expert + max_tiles;
-  for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int e = tid; e < experts; e += 1024) count[e] = 0;
   __syncthreads();
-  for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-    const int e = choice[p];
-    if (e >= 0 && e < experts) atomicAdd(&count[e], 1);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0, tiles = 0;
-    for (int e = 0; e < experts; ++e) {
-      first[e] = at;
-      starts[e] = at;
-      for (int r = 0; r < count[e] && tiles < max_tiles; r += tile_rows) {
-        tile_expert[tiles] = e;
-        tile_row[tiles] = at + r;
-        ++tiles;
-      }
-      at += count[e];
-      count[e] = 0;  // (from here on: how many of the expert's rows are placed)
-    }
-    first[experts] = at;
-    starts[experts] = at;
-    *num_tiles = tiles;
-  }
-  __syncthreads();
-  for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-    const int e = choice[p];
-    if (e < 0 || e >= experts) { place[p] = -1; continue; }
-    const int row = first[e] + atomicAdd(&count[e], 1);
-    order[row] = p;
-    place[p] = row;
-    if (sorted != nullptr) order_s[row] = p;
-  }
-  if (sorted == nullptr) return;  // (uniform over the workgroup)
-  __syncthreads();
-  // the rows of x in the plan's order, 16 bytes per thread at a time (the caller checked hidden % 8 == 0 and pairs <= PLAN_COPY_PAIRS)
-  const int pieces = hidden / 8;
-  for (int at = threadIdx.x; at < first[experts] * pieces; at += blockDim.x) {  // (first[experts]: the pairs that were placed)
-    const int row = at / pieces, piece_at = at % pieces;
-    const int p = order_s[row];
-    float4_t piece = reinterpret_cast<const float4_t*>(x + (size_t)(p / top) * hidden)[piece_at];
-    if (scale) {
-      const float w = pair_weight[p];
-      bf16_t* e8 = reinterpret_cast<bf16_t*>(&piece);
+  for (int p0 = tid; p0 < pairs; p0 += 1024 * BATCH) {
+    int e[BATCH];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) e8[j] = from_f32<bf16_t>(to_f32(e8[j]) * w);
+    for (int j = 0; j < BATCH; ++j) e[j] = p0 + 1024 * j < pairs ? choice[p0 + 1024 * j] : -1;
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j)
+      if (p0 + 1024 * j < pairs) place[p0 + 1024 * j] = e[j] >= 0 && e[j] < experts ? atomicAdd(&count[e[j]], 1) : -1;
+  }
+  __syncthreads();
+  {
+    int rows[2], tiles[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      rows[j] = 2 * tid + j < experts ? count[2 * tid + j] : 0;
+      tiles[j] = (rows[j] + tile_rows - 1) / tile_rows;
     }
-    reinterpret_cast<float4_t*>(sorted + (size_t)row * hidden)[piece_at] = piece;
+    int row_at = rows[0] + rows[1], tile_at = tiles[0] + tiles[1];  // inclusive sums over the wave, then exclusive over the workgroup
+#pragma unroll
+    for (int offset = 1; offset < 64; offset <<= 1) {
+      const int r = __shfl_up(row_at, offset, VELOX_WAVE), t = __shfl_up(tile_at, offset, VELOX_WAVE);
+      if (lane >= offset) {
+        row_at += r;
+        tile_at += t;
+      }
+    }
+    if (lane == 63) {
+      wave_rows[wave] = row_at;
+      wave_tiles[wave] = tile_at;
+    }
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) {
+      row_at += wave_rows[w];
+      tile_at += wave_tiles[w];
+    }
+    if (tid == 1023) {
+      plan[0] = min(tile_at, max_tiles);
+      starts[experts] = row_at;
+    }
+    row_at -= rows[0] + rows[1];
+    tile_at -= tiles[0] + tiles[1];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int e = 2 * tid + j;
+      if (e < experts) {
+        first[e] = row_at;
+        starts[e] = row_at;
+        for (int t = 0; t < tiles[j] && tile_at + t < max_tiles; ++t) {
+          tile_expert[tile_at + t] = e;
+          tile_row[tile_at + t] = row_at + t * tile_rows;
+        }
+      }
+      row_at += rows[j];
+      tile_at += tiles[j];
+    }
+  }
+  __syncthreads();
+  for (int p0 = tid; p0 < pairs; p0 += 1024 * BATCH) {
+    int e[BATCH], rank[BATCH];
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+      const int p = p0 + 1024 * j < pairs ? p0 + 1024 * j : p0;
+      e[j] = choice[p];
+      rank[j] = place[p];
+    }
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+      const int p = p0 + 1024 * j;
+      if (p >= pairs || rank[j] < 0) continue;
+      const int row = first[e[j]] + rank[j];
+      order[row] = p;
+      place[p] = row;
+    }
   }
 }
 
@@ -251,16 +278,12 @@ extern "C" long long velox_routed_plan_elems(int pairs, int experts) {
 
 extern "C" int velox_routed_max_tiles(int pairs, int experts) { return (pairs + RT_BM - 1) / RT_BM + experts; }
 
-// tile_rows: 64, or 128 for the matrix-core products of more than PLAN_COPY_PAIRS pairs.  The plan's layout is that of 64-row
-// tiles either way (the most tiles there can be).
-// x, sorted, pair_weight, top, hidden, scale: see routed_plan_kernel (sorted == nullptr: the plan alone).
-extern "C" int velox_routed_plan(const int* choice, int pairs, int experts, int* plan, int tile_rows, const void* x, void* sorted, const float* pair_weight,
-                                 int top, int hidden, int scale, hipStream_t stream) {
+// tile_rows: 64, or 128 for the matrix-core products of more than 64 pairs.  The plan's layout is that of 64-row tiles either way
+// (the most tiles there can be).
+extern "C" int velox_routed_plan(const int* choice, int pairs, int experts, int* plan, int tile_rows, hipStream_t stream) {
   if (pairs <= 0) return 0;
   if (experts < 1 || experts > PLAN_MAX_EXPERTS || (tile_rows != RT_BM && tile_rows != 2 * RT_BM)) return -1;
-  if (sorted != nullptr && (x == nullptr || pairs > PLAN_COPY_PAIRS || hidden % 8 != 0 || top < 1 || (((uintptr_t)x | (uintptr_t)sorted) & 15) != 0)) return -1;
-  routed_plan_kernel<<<1, 1024, 0, stream>>>(choice, pairs, experts, velox_routed_max_tiles(pairs, experts), tile_rows, plan, (const bf16_t*)x, (bf16_t*)sorted,
-                                             pair_weight, top, hidden, scale);
+  routed_plan_kernel<<<1, 1024, 0, stream>>>(choice, pairs, experts, velox_routed_max_tiles(pairs, experts), tile_rows, plan);
   VELOX_RETURN_LAUNCH_STATUS();
 }
 
@@ -433,9 +456,8 @@ extern "C" int velox_grouped_down(const void* act, const void* down, float* y, c
 }
 
 // ---------------------------------------------------------------------------------------------
-// bfloat16 on the matrix cores.  A step of few pairs reads rows that the plan's kernel has copied into its order (scaled, when
-// the pair's weight scales the expert's input: float32 product, one rounding); a larger one fetches the rows of x through the
-// plan and scales the first product's float32 sums.
+// bfloat16 on the matrix cores: the first product fetches the rows of x through the plan and, when the pair's weight scales the
+// expert's input, scales its float32 sums; the second reads sorted rows.
 // ---------------------------------------------------------------------------------------------
 static GroupedArgs routed_args(const void* a, const void* w, void* out, const int* plan, int pairs, int experts, int n, int k, int w_rows) {
   GroupedArgs args = {};
@@ -454,23 +476,19 @@ static GroupedArgs routed_args(const void* a, const void* w, void* out, const in
   return args;
 }
 
-// x [T, hidden] -> act [pairs, inter] -> y [pairs, hidden] float32.  Needs hidden % 8 == 0 and inter % 8 == 0 (the caller
-// checks).  `sorted` [pairs, hidden]: the rows as the plan's kernel has copied them, for up to PLAN_COPY_PAIRS pairs; more
-// pairs come with `x` and a plan of tiles of GM_TILE_ROWS rows.
-extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, const void* down, const void* sorted, void* act, float* y, const int* plan,
+// x [T, hidden] -> act [pairs, inter] -> y [pairs, hidden] float32.  Needs hidden % 8 == 0, inter % 8 == 0 and x on a 16-byte
+// boundary (the caller checks).  The plan's tiles hold 64 rows for up to 64 pairs, GM_TILE_ROWS for more.
+extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, const void* down, void* act, float* y, const int* plan,
                                           const float* pair_weight, int pairs, int experts, int top, int inter, int hidden, int scale_input,
                                           float alpha, float limit, float shift, int ungated, hipStream_t stream) {
   // `ungated` > 0: `gate_up` holds [experts * inter, hidden] (up rows only) and the unit is ungated_act(up, ungated)
   if (pairs <= 0) return 0;
-  const void* rows = pairs <= PLAN_COPY_PAIRS ? sorted : x;
-  if (hidden % 8 != 0 || inter % 8 != 0 || top < 1 || rows == nullptr || (uintptr_t)rows % 16 != 0) return -1;
+  if (hidden % 8 != 0 || inter % 8 != 0 || top < 1 || (uintptr_t)x % 16 != 0) return -1;
   const int max_tiles = velox_routed_max_tiles(pairs, experts);
   if (max_tiles > 65535) return -1;
-  GroupedArgs first = routed_args(rows, gate_up, act, plan, pairs, experts, inter, hidden, ungated > 0 ? inter : 2 * inter);
-  if (rows == x) {
-    first.gather_top = top;
-    first.row_scale = scale_input ? pair_weight : nullptr;
-  }
+  GroupedArgs first = routed_args(x, gate_up, act, plan, pairs, experts, inter, hidden, ungated > 0 ? inter : 2 * inter);
+  first.gather_top = top;
+  first.row_scale = scale_input ? pair_weight : nullptr;
   first.act = ungated;
   first.unit = GluUnit{alpha, limit, shift};
   if (ungated > 0) grouped_mfma_launch<GM_ACT, bf16_t>(first, pairs, max_tiles, 1, stream);
@@ -488,86 +506,141 @@ extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, co
 // pair_weight[t * top + k] * x[t, :] in its turn.  With `scale_rows` every row of y is multiplied with its pair's weight here
 // (the products then left it out).
 // ---------------------------------------------------------------------------------------------
-template <typename T>
+// V neighbouring entries a thread (4: rows in 16-byte pieces, the choices' rows all asked for before the first is added), a
+// workgroup per token and 256 V entries.  Bound by what it moves: 2,500 tokens of 4 x 4,096 float32 and a shared row, 205 MB,
+// 34 us (one entry a thread and a workgroup per token: 100); 16 tokens 4.6 us (34).  With the norms, 1,036 tokens of 2 x 2,048: 9.8 (18.5).
+template <int V> struct Entries { float v[V]; };
+template <typename T, int V>
+__device__ __forceinline__ Entries<V> entries_of(const T* p) {
+  Entries<V> out;
+  typedef T Pieces __attribute__((ext_vector_type(V)));
+  if constexpr (V == 1) {
+    out.v[0] = to_f32(*p);
+  } else {
+    const Pieces x = *reinterpret_cast<const Pieces*>(p);
+#pragma unroll
+    for (int e = 0; e < V; ++e) out.v[e] = to_f32(x[e]);
+  }
+  return out;
+}
+template <typename T, int V>
+__device__ __forceinline__ void store_entries(T* p, const Entries<V>& in) {
+  typedef T Pieces __attribute__((ext_vector_type(V)));
+  if constexpr (V == 1) {
+    *p = from_f32<T>(in.v[0]);
+  } else {
+    Pieces x;
+#pragma unroll
+    for (int e = 0; e < V; ++e) x[e] = from_f32<T>(in.v[e]);
+    *reinterpret_cast<Pieces*>(p) = x;
+  }
+}
+
+// A token's sum at V entries from i on, in float32.
+template <typename T, int V>
+__device__ __forceinline__ Entries<V> combined(const float* __restrict__ y, const int* mine, const T* __restrict__ shared, int t, int top, int hidden,
+                                               const T* __restrict__ x, const float* __restrict__ pair_weight, int scale_rows, int i) {
+  constexpr int BATCH = 4;
+  Entries<V> sum = {};
+  for (int k0 = 0; k0 < top; k0 += BATCH) {
+    Entries<V> part[BATCH];
+    float factor[BATCH];
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+      const int row = k0 + j < top ? mine[k0 + j] : -1;
+      part[j] = Entries<V>{};
+      factor[j] = 1.f;
+      if (row >= 0) {
+        part[j] = entries_of<float, V>(y + (size_t)row * hidden + i);
+        if (scale_rows) factor[j] = pair_weight[(size_t)t * top + k0 + j];
+      } else if (x && k0 + j < top) {
+        part[j] = entries_of<T, V>(x + (size_t)t * hidden + i);
+        factor[j] = pair_weight[(size_t)t * top + k0 + j];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j)
+#pragma unroll
+      for (int e = 0; e < V; ++e) sum.v[e] += factor[j] * part[j].v[e];
+  }
+  if (shared) {
+    const Entries<V> s = entries_of<T, V>(shared + (size_t)t * hidden + i);
+#pragma unroll
+    for (int e = 0; e < V; ++e) sum.v[e] += s.v[e];
+  }
+  return sum;
+}
+
+template <typename T, int V>
 __global__ void __launch_bounds__(256) routed_combine_kernel(const float* __restrict__ y, const int* __restrict__ place, const T* __restrict__ shared,
                                                              T* __restrict__ out, int top, int hidden, const T* __restrict__ x,
                                                              const float* __restrict__ pair_weight, int scale_rows) {
-  __shared__ int rows[64];  // the token's rows of y, looked up once (up to 64 choices; more are looked up as they are added)
-  const int t = blockIdx.x;
-  const int* mine = place + (size_t)t * top;
-  if (top <= 64) {
-    if (threadIdx.x < top) rows[threadIdx.x] = mine[threadIdx.x];
-    __syncthreads();
-    mine = rows;
-  }
-  for (int i = threadIdx.x; i < hidden; i += blockDim.x) {
-    float v = 0.f;
-    for (int k = 0; k < top; ++k) {
-      const int row = mine[k];
-      if (row >= 0) v += scale_rows ? pair_weight[(size_t)t * top + k] * y[(size_t)row * hidden + i] : y[(size_t)row * hidden + i];
-      else if (x) v += pair_weight[(size_t)t * top + k] * to_f32(x[(size_t)t * hidden + i]);
-    }
-    if (shared) v += to_f32(shared[(size_t)t * hidden + i]);
-    out[(size_t)t * hidden + i] = from_f32<T>(v);
-  }
+  const int t = blockIdx.x, i = (blockIdx.y * 256 + threadIdx.x) * V;
+  if (i >= hidden) return;
+  store_entries<T, V>(out + (size_t)t * hidden + i, combined<T, V>(y, place + (size_t)t * top, shared, t, top, hidden, x, pair_weight, scale_rows, i));
 }
 
 // The same sum, handed straight to a norm on the experts' output: residual[t, :] += mult * v * rsqrt(mean(v^2) + eps) * w, with v the
 // sum above in float32 (never rounded to T), and `copy` (nullable) the updated residual in T; with `next_weight` `copy` is instead
 // what the norm that reads the residual next makes of it, r * rsqrt(mean(r^2) + next_eps) * next_weight.  One workgroup per
 // token holds the row in registers: hidden <= 16 * blockDim.x.
-template <typename T>
+template <typename T, int V>
 __global__ void routed_combine_norm_kernel(const float* __restrict__ y, const int* __restrict__ place, const T* __restrict__ shared, int top, int hidden,
                                            const T* __restrict__ x, const float* __restrict__ pair_weight, int scale_rows, float* __restrict__ residual,
                                            const float* __restrict__ norm_weight, float eps, float mult, T* __restrict__ copy,
                                            const float* __restrict__ next_weight, float next_eps) {
-  __shared__ int rows[64];
+  constexpr int HELD = 16 / V;
   __shared__ float scratch[16];
   const int t = blockIdx.x;
   const int* mine = place + (size_t)t * top;
-  if (top <= 64) {
-    if (threadIdx.x < top) rows[threadIdx.x] = mine[threadIdx.x];
-    __syncthreads();
-    mine = rows;
-  }
-  float held[16];
+  Entries<V> held[HELD];
   float sumsq = 0.f;
 #pragma unroll
-  for (int c = 0; c < 16; ++c) {
-    const int i = threadIdx.x + c * blockDim.x;
-    float v = 0.f;
-    if (i < hidden) {
-      for (int k = 0; k < top; ++k) {
-        const int row = mine[k];
-        if (row >= 0) v += scale_rows ? pair_weight[(size_t)t * top + k] * y[(size_t)row * hidden + i] : y[(size_t)row * hidden + i];
-        else if (x) v += pair_weight[(size_t)t * top + k] * to_f32(x[(size_t)t * hidden + i]);
-      }
-      if (shared) v += to_f32(shared[(size_t)t * hidden + i]);
-    }
-    held[c] = v;
-    sumsq += v * v;
+  for (int c = 0; c < HELD; ++c) {
+    const int i = (threadIdx.x + c * blockDim.x) * V;
+    held[c] = Entries<V>{};
+    if (i < hidden) held[c] = combined<T, V>(y, mine, shared, t, top, hidden, x, pair_weight, scale_rows, i);
+#pragma unroll
+    for (int e = 0; e < V; ++e) sumsq += held[c].v[e] * held[c].v[e];
   }
   const float total = block_sum(sumsq, scratch);
   const float inv = 1.f / sqrtf(total / (float)hidden + eps);
   sumsq = 0.f;
 #pragma unroll
-  for (int c = 0; c < 16; ++c) {
-    const int i = threadIdx.x + c * blockDim.x;
+  for (int c = 0; c < HELD; ++c) {
+    const int i = (threadIdx.x + c * blockDim.x) * V;
     if (i < hidden) {
-      const float r = residual[(size_t)t * hidden + i] + mult * (held[c] * inv * norm_weight[i]);
-      residual[(size_t)t * hidden + i] = r;
-      if (copy && !next_weight) copy[(size_t)t * hidden + i] = from_f32<T>(r);
+      const Entries<V> w = entries_of<float, V>(norm_weight + i);
+      Entries<V> r = entries_of<float, V>(residual + (size_t)t * hidden + i);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        r.v[e] = r.v[e] + mult * (held[c].v[e] * inv * w.v[e]);
+        sumsq += r.v[e] * r.v[e];
+      }
+      store_entries<float, V>(residual + (size_t)t * hidden + i, r);
+      if (copy && !next_weight) store_entries<T, V>(copy + (size_t)t * hidden + i, r);
       held[c] = r;
-      sumsq += r * r;
     }
   }
   if (!next_weight) return;
   const float next_inv = 1.f / sqrtf(block_sum(sumsq, scratch) / (float)hidden + next_eps);
 #pragma unroll
-  for (int c = 0; c < 16; ++c) {
-    const int i = threadIdx.x + c * blockDim.x;
-    if (i < hidden) copy[(size_t)t * hidden + i] = from_f32<T>(held[c] * next_inv * next_weight[i]);
+  for (int c = 0; c < HELD; ++c) {
+    const int i = (threadIdx.x + c * blockDim.x) * V;
+    if (i < hidden) {
+      const Entries<V> w = entries_of<float, V>(next_weight + i);
+      Entries<V> r = held[c];
+#pragma unroll
+      for (int e = 0; e < V; ++e) r.v[e] = r.v[e] * next_inv * w.v[e];
+      store_entries<T, V>(copy + (size_t)t * hidden + i, r);
+    }
   }
+}
+
+// Whether all rows start on the boundaries that four entries at a time need.
+static bool combine_in_fours(int hidden, int dtype, const void* y, const void* shared, const void* x, const void* a, const void* b, const void* c, const void* d) {
+  const uintptr_t narrow = (uintptr_t)shared | (uintptr_t)x | (uintptr_t)d, wide = (uintptr_t)y | (uintptr_t)a | (uintptr_t)b | (uintptr_t)c;
+  return hidden % 4 == 0 && wide % 16 == 0 && narrow % (dtype == VELOX_BF16 ? 8 : 16) == 0;
 }
 
 // copy: nullptr in a float32 run (the residual is its own copy).  Returns -1 when the row does not fit the registers
@@ -581,12 +654,18 @@ extern "C" int velox_routed_combine_norm(const float* y, const int* plan, const 
   const int* place = plan + 1 + (experts + 1) + (size_t)tokens * top;
   int threads = tokens <= 64 ? 512 : 256;  // (few rows: more threads each with less to do)
   while (16 * threads < hidden) threads *= 2;
-  if (dtype == VELOX_BF16)
-    routed_combine_norm_kernel<bf16_t><<<tokens, threads, 0, stream>>>(y, place, (const bf16_t*)shared, top, hidden, (const bf16_t*)x, pair_weight, scale_rows,
-                                                                       residual, norm_weight, eps, mult, (bf16_t*)copy, next_weight, next_eps);
-  else
-    routed_combine_norm_kernel<float><<<tokens, threads, 0, stream>>>(y, place, (const float*)shared, top, hidden, (const float*)x, pair_weight, scale_rows,
-                                                                      residual, norm_weight, eps, mult, (float*)copy, next_weight, next_eps);
+#define COMBINE(T, V)                                                                                                                              \
+  routed_combine_norm_kernel<T, V><<<tokens, threads, 0, stream>>>(y, place, (const T*)shared, top, hidden, (const T*)x, pair_weight, scale_rows, residual, \
+                                                                   norm_weight, eps, mult, (T*)copy, next_weight, next_eps)
+  const bool fours = combine_in_fours(hidden, dtype, y, shared, x, residual, norm_weight, next_weight, copy);
+  if (dtype == VELOX_BF16) {
+    if (fours) COMBINE(bf16_t, 4);
+    else COMBINE(bf16_t, 1);
+  } else {
+    if (fours) COMBINE(float, 4);
+    else COMBINE(float, 1);
+  }
+#undef COMBINE
   VELOX_RETURN_LAUNCH_STATUS();
 }
 
@@ -594,9 +673,17 @@ extern "C" int velox_routed_combine(const float* y, const int* plan, const void*
                                     const void* x, const float* pair_weight, int scale_rows, hipStream_t stream) {
   if (tokens <= 0) return 0;
   const int* place = plan + 1 + (experts + 1) + (size_t)tokens * top;
-  if (dtype == VELOX_BF16)
-    routed_combine_kernel<bf16_t><<<tokens, 256, 0, stream>>>(y, place, (const bf16_t*)shared, (bf16_t*)out, top, hidden, (const bf16_t*)x, pair_weight, scale_rows);
-  else
-    routed_combine_kernel<float><<<tokens, 256, 0, stream>>>(y, place, (const float*)shared, (float*)out, top, hidden, (const float*)x, pair_weight, scale_rows);
+#define COMBINE(T, V)                                                                                                                              \
+  routed_combine_kernel<T, V><<<dim3(tokens, (hidden + 256 * V - 1) / (256 * V)), 256, 0, stream>>>(y, place, (const T*)shared, (T*)out, top, hidden, (const T*)x, \
+                                                                                                    pair_weight, scale_rows)
+  const bool fours = combine_in_fours(hidden, dtype, y, shared, x, nullptr, nullptr, nullptr, out);
+  if (dtype == VELOX_BF16) {
+    if (fours) COMBINE(bf16_t, 4);
+    else COMBINE(bf16_t, 1);
+  } else {
+    if (fours) COMBINE(float, 4);
+    else COMBINE(float, 1);
+  }
+#undef COMBINE
   VELOX_RETURN_LAUNCH_STATUS();
 }

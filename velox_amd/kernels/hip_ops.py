@@ -79,7 +79,7 @@ def _weight_of(weight) -> Tuple[torch.Tensor, Optional[PreparedWeight]]:
 class HipOps:
     name = "hip-gfx950"
     MAX_TILED_HEAD_DIM = 256  # head sizes above this go to the plain attention kernel
-    FEW_PAIRS = 64  # up to this many (token, expert) pairs the experts' plan kernel copies the rows itself
+    FEW_PAIRS = 64  # up to this many (token, expert) pairs the experts' plan has tiles of 64 rows, which hold any of them whole
 
     def __init__(self, device) -> None:
         self.device = torch.device(device)
@@ -150,11 +150,11 @@ class HipOps:
         c.velox_route_top.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _I, _F, _P]
         c.velox_routed_plan_elems.argtypes = [_I, _I]
         c.velox_routed_plan_elems.restype = ctypes.c_longlong
-        c.velox_routed_plan.argtypes = [_P, _I, _I, _P, _I, _P, _P, _P, _I, _I, _I, _P]
+        c.velox_routed_plan.argtypes = [_P, _I, _I, _P, _I, _P]
         c.velox_grouped_glu.argtypes = [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _I, _P]
         c.velox_grouped_down.argtypes = [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]
         c.velox_routed_combine.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P]
-        c.velox_routed_products_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _F, _I, _P]
+        c.velox_routed_products_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _F, _I, _P]
         c.velox_routed_combine_norm.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _F, _F, _P, _P, _F, _P]
         c.velox_routed_combine_norm.restype = _I
         c.velox_add_sinusoid.argtypes = [_P, _P, _P, _I, _I, _P]
@@ -1664,19 +1664,14 @@ class HipOps:
             plan = torch.empty(elems, dtype=torch.int32, device=self.device)
         on_matrix_cores = x.dtype == torch.bfloat16 and hidden % 8 == 0 and inter % 8 == 0 and self.use_grouped_mfma
         tile_rows = 128 if on_matrix_cores and pairs > self.FEW_PAIRS else 64
-        # few pairs: the plan's kernel also copies the rows into its order; more of them are fetched where they are
-        copied_by_plan = on_matrix_cores and pairs <= self.FEW_PAIRS
-        ordered = torch.empty((pairs, hidden), dtype=x.dtype, device=self.device) if copied_by_plan else None
-        if on_matrix_cores and not copied_by_plan and x.data_ptr() % 16 != 0:
+        if on_matrix_cores and x.data_ptr() % 16 != 0:
             x = x.clone()
-        self._launched(self._core.velox_routed_plan(_ptr(choice), pairs, num_experts, _ptr(plan), tile_rows, _ptr(x) if copied_by_plan else _P(0),
-                                                    _ptr(ordered) if copied_by_plan else _P(0), _ptr(weight), top, hidden, int(bool(scale_input)), self._stream()),
-                       "routed_plan")
+        self._launched(self._core.velox_routed_plan(_ptr(choice), pairs, num_experts, _ptr(plan), tile_rows, self._stream()), "routed_plan")
         act = torch.empty((pairs, inter), dtype=x.dtype, device=self.device)
         y = torch.empty((pairs, hidden), dtype=torch.float32, device=self.device)
         if on_matrix_cores:
             # bfloat16 rows of whole 16-byte pieces: both products on the matrix cores
-            self._launched(self._core.velox_routed_products_bf16(_P(0) if copied_by_plan else _ptr(x), _ptr(gate_up_weight), _ptr(down_weight), _ptr(ordered), _ptr(act), _ptr(y), _ptr(plan),
+            self._launched(self._core.velox_routed_products_bf16(_ptr(x), _ptr(gate_up_weight), _ptr(down_weight), _ptr(act), _ptr(y), _ptr(plan),
                                                                  _ptr(weight), pairs, num_experts, top, inter, hidden, int(bool(scale_input)),
                                                                  alpha, limit, shift, act_code, self._stream()), "routed_products")
             # (a weight on the output is applied by the last kernel: the second product is the same kernel either way)
