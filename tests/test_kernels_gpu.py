@@ -1223,3 +1223,14 @@ def test_float32_products_on_the_matrix_instructions(ops, m, n, k):
     bound = (128 + k / 128 + 2) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + bias.double().abs())
     assert torch.all((got.double() - want).abs() <= bound)
     assert torch.equal(ops.gemm_fma(a[-17:].contiguous(), w, bias, torch.float32), got[-17:])
+
+
+@pytest.mark.parametrize("nh, nkv, page", [(32, 1, 16), (6, 2, 8), (65, 1, 32)])
+@pytest.mark.parametrize("window", [None, 90])
+def test_portions_of_heads_of_256_channels(ops, ref, nh, nkv, page, window):
+    """Rows and keys at the edges of the 128-row and 64-key tiles, portions behind contexts, single tokens beside them."""
+    seqs = [(1, 129), (4, 4), (64, 64), (5, 69), (43, 107), (130, 200), (2, 63), (33, 33)]
+    case = _attention_case(torch.bfloat16, nh, nkv, 256, page, seqs, seed=nh + page)
+    got = _run_attention(ops, case, nh, nkv, 256, page, window=window)
+    want = _run_attention(ref, case, nh, nkv, 256, page, window=window)
+    torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-2)  # (the tolerance of the other bfloat16 attention tests above)

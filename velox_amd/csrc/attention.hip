@@ -703,7 +703,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
 }
 
 // ---- portions of prompts, bfloat16, tiles brought into LDS by the memory system itself ---------------------------------
-// The same arithmetic as the general kernel with CT row tiles per wave, for head sizes of 64 and 128 channels and pages
+// The same arithmetic as the general kernel with CT row tiles per wave, for head sizes of 64, 128 and 256 channels and pages
 // of at least 8 tokens.  What differs is how a tile of 64 keys gets into LDS: every lane asks for 16 bytes of the
 // cache with a load that writes LDS directly (no registers, no LDS write instructions, no address arithmetic on the
 // way back), a whole tile AHEAD of the one being multiplied, into the other of two tile buffers.  One barrier per tile
@@ -737,7 +737,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
   typedef bf16_t T;
   typedef Block<T> B;
   typedef typename B::Operand Operand;
-  static_assert(CT > 0 && (D == 64 || D == 128), "head sizes whose rows are a power of two of 16-byte pieces, at least eight");
+  static_assert(CT > 0 && (D == 64 || D == 128 || D == 256), "head sizes whose rows are a power of two of 16-byte pieces, at least eight");
   constexpr int BN = 64, KB = 32, VEC = 8;
   constexpr int NT = BN / 16, NQB = D / KB, NKB = BN / KB, NC = D / 16;
   constexpr int CPR = D / 8;                        // 16-byte pieces of a K row
@@ -974,7 +974,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
     float4_t s[CT][NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      Operand kf[NQB > 0 ? NQB : 1];  // (the template is parsed for every head size, run for 64 and 128)
+      Operand kf[NQB > 0 ? NQB : 1];  // (the template is parsed for every head size, run for 64, 128 and 256)
       const int tile_bytes = (32 * (t >> 1) + 4 * (t & 1)) * (2 * D);
 #pragma unroll
       for (int cb = 0; cb < NQB; ++cb)
@@ -1072,7 +1072,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
       m_i[ct] = m_new;
     }
     // ---- O^T = O^T * alpha + V^T P^T --------------------------------------------------------
-    constexpr int AHEAD = 1;  // channel tiles whose operands are in flight ahead of the one being multiplied
+    constexpr int AHEAD = D == 256 ? 3 : 1;  // channel tiles whose operands are in flight ahead of the one being multiplied
     Operand vf[AHEAD + 1][NKB];
     auto read_values = [&](int c, Operand (&into)[NKB]) {
 #pragma unroll
@@ -1526,19 +1526,22 @@ static int launch(const void* qkv, int qkv_stride, const void* k_cache, const vo
     merge_splits_kernel<T><<<dim3(total_tokens, nh), MERGE_THREADS, 0, stream>>>(part_o, part_lse, (T*)out, nh, splits, total_tokens, 0, sinks, extras);
     return (int)hipGetLastError();
   }
-  // The kernel whose tiles reach LDS by direct loads: bfloat16, head sizes 64 and 128, pages of at least 8 tokens.
-  constexpr bool HAS_DIRECT = sizeof(T) == 2 && (D == 64 || D == 128);
+  // The kernel whose tiles reach LDS by direct loads: bfloat16, head sizes 64, 128 and 256, pages of at least 8 tokens.
+  constexpr bool HAS_DIRECT = sizeof(T) == 2 && (D == 64 || D == 128 || D == 256);
   const bool direct_ok = HAS_DIRECT && page_shift >= 3 && portion_kernel_choice != 1;
   auto launch_direct = [&](bool two_sets = false) -> int {
     if constexpr (HAS_DIRECT) {
       dim3 grid(num_seqs * splits, nkv, (max_q_len * group + 127) / 128);
       if (grid.z > 65535u) return (int)hipErrorInvalidValue;  // (more than 8 million rows in one portion)
-      if (two_sets)
-        direct_attention_kernel<2, 4, 2><<<grid, 512, 0, stream>>>(
+      // 256 channels: one set's tile buffers take 128 KB of LDS, and eight waves of one row tile keep two waves on a SIMD within
+      // its registers
+      constexpr int CT = D == 256 ? 1 : 2, WAVES = D == 256 ? 8 : 4, MOST_SETS = D == 256 ? 1 : 2;
+      if (two_sets && MOST_SETS == 2)
+        direct_attention_kernel<CT, WAVES, MOST_SETS><<<grid, 512, 0, stream>>>(
             (const bf16_t*)qkv, qkv_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, table_width, cu_q, kv_lens, (bf16_t*)out,
             part_o, part_lse, nh, nkv, page_shift, scale, window, splits, total_tokens, bias_table, bias_len, sinks, extras);
       else
-        direct_attention_kernel<2, 4><<<grid, 256, 0, stream>>>(
+        direct_attention_kernel<CT, WAVES><<<grid, 64 * WAVES, 0, stream>>>(
             (const bf16_t*)qkv, qkv_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, table_width, cu_q, kv_lens, (bf16_t*)out,
             part_o, part_lse, nh, nkv, page_shift, scale, window, splits, total_tokens, bias_table, bias_len, sinks, extras);
     }
@@ -1549,6 +1552,12 @@ static int launch(const void* qkv, int qkv_stride, const void* k_cache, const vo
     return (int)hipGetLastError();
   };
   if (direct_ok && portion_kernel_choice >= 2 && max_q_len * group > 64) return launch_direct(portion_kernel_choice == 3);
+  // 256 channels (a latent and its rotated part, all heads over one KV head): direct loads wherever there are more than 64 rows.
+  // Measured on MI355X (us, the kernels below / direct loads, 32 heads over 1): 300 tokens 24 / 21, 600 tokens 42 / 33, 1,500 tokens
+  // 164 / 70, 4,096 tokens 908 / 355, 64 tokens behind 1,000 keys 62 / 45, 12 single tokens behind 700 keys beside 300 tokens 42 /
+  // 23; 8 over 2: 600 tokens 40 / 29, 4,096 tokens 237 / 151; up to 150 tokens equal.  (With four waves of two row tiles, one wave
+  // per SIMD, 1,500 and 1,000 tokens took 180 instead of 126.)
+  if (direct_ok && D == 256 && max_q_len * group > 64) return launch_direct();
   if (direct_ok && max_q_len * group > 64) {
     // Measured on MI355X over prompts and portions of 128 to 8,192 tokens behind up to 30,000 keys, with 28 heads over 4,
     // 12 over 2 and 40 over 8 (us: the kernels below / direct loads / direct loads with two sets of waves).  Direct loads
