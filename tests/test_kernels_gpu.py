@@ -1234,3 +1234,16 @@ def test_portions_of_heads_of_256_channels(ops, ref, nh, nkv, page, window):
     got = _run_attention(ops, case, nh, nkv, 256, page, window=window)
     want = _run_attention(ref, case, nh, nkv, 256, page, window=window)
     torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-2)  # (the tolerance of the other bfloat16 attention tests above)
+
+
+@pytest.mark.parametrize("m, n, k, splits", [(65, 100, 5128, 1), (128, 256, 64, 1), (129, 260, 200, 2), (300, 516, 1096, 3), (1100, 300, 520, 5), (70, 1024, 72, 8)])
+def test_products_in_tiles_with_a_cut_sum(ops, m, n, k, splits):
+    """Against float64: remainders in all sizes, more than one block of row tiles, a last part that is short or empty.  Float32 sums of at
+    most k terms in one part (an error below k 2^-24 of the sum of the terms' sizes), one rounding to bfloat16 (2^-8) for one part."""
+    generator = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w = (torch.randn(*shape, generator=generator, device="cuda").bfloat16() for shape in ((m, k), (n, k)))
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    whole = ops.gemm_tiles(a, w)
+    assert torch.all((whole.double() - want).abs() <= k * 2.0 ** -24 * size + 2.0 ** -8 * 1.01 * want.abs() + 1e-6)
+    parts = ops.gemm_tiles(a, w, splits, torch.float32)
+    assert parts.shape == (splits, m, n) and torch.all((parts.double().sum(0) - want).abs() <= k * 2.0 ** -24 * size + 1e-6)

@@ -11,6 +11,7 @@
 // lengths and not with that of their product, which keeps the float32 path as close to the exact
 // result as a blocked library product on a CPU is.
 #include "common.h"
+#include "grouped_mfma.h"
 
 #define GEMM_BM 64
 #define GEMM_BN 64
@@ -380,5 +381,29 @@ extern "C" int velox_gemm_fma(const void* a, const void* w, const float* bias, v
     default: return -1;
   }
 #undef LAUNCH
+  VELOX_RETURN_LAUNCH_STATUS();
+}
+
+// out[M, N] (bfloat16, or float32 partial sums [splits, M, N] of `splits` parts of k) = A[M, K] * W[N, K]^T, bfloat16, in the tiles of the
+// experts' products (grouped_tiles_kernel).  Needs k % 8 == 0, n % 4 == 0 and 16-byte aligned bases.
+extern "C" int velox_gemm_tiles_bf16(const void* a, const void* w, void* out, int m, int n, int k, int splits, int out_dtype, hipStream_t stream) {
+  if (m <= 0 || n <= 0) return 0;
+  if (k < 1 || k % 8 != 0 || n % 4 != 0 || splits < 1 || (out_dtype == VELOX_BF16 && splits != 1) || (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) != 0) return -1;
+  GroupedArgs args = {};
+  args.a = (const bf16_t*)a;
+  args.a_ld = k;
+  args.w = (const bf16_t*)w;
+  args.out = out;
+  args.out_ld = n;
+  args.n = n;
+  args.k = k;
+  args.m = m;
+  args.splits = splits;
+  const int cols = (n + GM_TILE_COLS - 1) / GM_TILE_COLS;
+  const long long tiles = (long long)((m + GM_TILE_ROWS - 1) / GM_TILE_ROWS) * cols * splits;
+  if (tiles > (1 << 30)) return -1;
+  const int workgroups = (int)((tiles + GM_XCDS - 1) / GM_XCDS * GM_XCDS);
+  if (out_dtype == VELOX_BF16) grouped_tiles_kernel<GM_PLAIN, bf16_t><<<workgroups, 512, 0, stream>>>(args, cols);
+  else grouped_tiles_kernel<GM_PLAIN, float><<<workgroups, 512, 0, stream>>>(args, cols);
   VELOX_RETURN_LAUNCH_STATUS();
 }

@@ -1,6 +1,6 @@
 // Many small bfloat16 products in one launch on the matrix cores of gfx950: a product per group (an expert, a head), each
-// over its own rows, out[r, g, :] = W_g a[r, g, :].  Shared by the routed experts and by the per-head products of
-// attention over a latent.
+// over its own rows, out[r, g, :] = W_g a[r, g, :].  Shared by the routed experts, by the per-head products of
+// attention over a latent and by single products whose sum is long and whose tiles are few (velox_gemm_tiles_bf16).
 //
 // A workgroup of four waves of the kernel without a plan owns 64 rows and 64 NT output columns of one group (NT = 2 or 4 tiles of W per wave; half as
 // many gate columns and the up columns of the same outputs with the GLU epilogue); a wave owns 16 NT of the columns and all
@@ -42,6 +42,7 @@ struct GroupedArgs {
   long long gate_ld, gate_group, gate_col;
   int act = 0;         // GM_ACT: the result goes through ungated_act(., act)
   const float* row_scale;  // with a plan: the sums in front of a GLU or an activation are multiplied with row_scale[order[r]] (nullptr: none)
+  int splits = 1;          // grouped_tiles_kernel without a plan: parts of k, each with a result [m, out_ld] of its own, one after the other
   int gather_top = 0;      // with a plan: > 0: sorted row r is row order[r] / gather_top of `a`
   GluUnit unit = {1.f, INFINITY, 0.f};  // GM_GLU: the unit's middle (see glu_middle)
 };
@@ -291,11 +292,15 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
 // 168 us (0.78 and 0.69 PFLOP/s; W alone at 4.5 TB/s is 164 + 82 us); 2,072 pairs over 16 experts, 2,048 -> 1,408: 153 + 71 -> 70 + 33.
 // Without its loads the first takes 255 us, without its matrix instructions 302: a tile of 256 x 256 is no faster, nor is a
 // ninth wave that reads W ahead into L2 (335).
+// Without a plan it works ONE product, whole or in `splits` parts of k that the kernel behind it adds.  A group's tiles go in
+// blocks of GM_BLOCK_ROWS row tiles, column after column: the 32 tiles that an XCD has under way at once then read 8 row
+// tiles and 4 columns, which its L2 keeps, rather than 32 row tiles of one column (4,096 x 18,944 -> 3,584: 0.85 -> 0.90 PFLOP/s).
 static __device__ __attribute__((aligned(16))) const unsigned int gm_zero_piece[4] = {0u, 0u, 0u, 0u};
 
 #define GM_TILE_ROWS 128  // rows of `a` and
 #define GM_TILE_COLS 256  // rows of W per workgroup of grouped_tiles_kernel
 #define GM_XCDS 8
+#define GM_BLOCK_ROWS 8   // row tiles of a block (see above)
 
 template <int EPI, typename TO>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) grouped_tiles_kernel(const GroupedArgs args, const int cols) {
@@ -306,28 +311,42 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   constexpr int GROUP = GM_TILE_COLS / WN;             // rows of W of a wave (GLU: half gate rows, half the up rows of the same outputs)
   __shared__ __attribute__((aligned(1024))) char smem[STAGES][(ROWS + GM_TILE_COLS) * 128];
 
-  const int total = args.plan[0] * cols;
+  // the plan's tiles, or all rows of one product in `splits` parts of k
+  const int row_tiles = args.plan != nullptr ? args.plan[0] : (args.m + ROWS - 1) / ROWS;
+  const int total = row_tiles * cols * args.splits;
   const int share = (total + GM_XCDS - 1) / GM_XCDS;
   const int mine = (int)(blockIdx.x / GM_XCDS);
-  const int work = (int)(blockIdx.x % GM_XCDS) * share + mine;
+  int work = (int)(blockIdx.x % GM_XCDS) * share + mine;
   if (mine >= share || work >= total) return;  // (uniform over the workgroup)
-  const int* starts = args.plan + 1;
-  const int* order = starts + args.plan_groups + 1;
-  const int* tile_group = order + 2 * (size_t)args.plan_pairs;
-  const int* tile_row = tile_group + args.plan_max_tiles;
-  // (a group's tiles follow one another, so work / cols lies among the tiles of the right one)
-  const int near = work / cols, group = tile_group[near];
-  const int begin = starts[group], end = starts[group + 1];
-  const int first_tile = near - (tile_row[near] - begin) / ROWS, tiles = (end - begin + ROWS - 1) / ROWS;
-  const int at = work - first_tile * cols;
-  const int row0 = begin + (at % tiles) * ROWS, rows = min(ROWS, end - row0);
-  const int column = at / tiles;
-
+  int group = 0, begin = 0, end = args.m, first_tile = 0, split = 0;
+  const int* order = nullptr;
+  if (args.plan != nullptr) {
+    const int* starts = args.plan + 1;
+    order = starts + args.plan_groups + 1;
+    const int* tile_group = order + 2 * (size_t)args.plan_pairs;
+    const int* tile_row = tile_group + args.plan_max_tiles;
+    // (a group's tiles follow one another, so work / cols lies among the tiles of the right one)
+    const int near = work / cols;
+    group = tile_group[near];
+    begin = starts[group];
+    end = starts[group + 1];
+    first_tile = near - (tile_row[near] - begin) / ROWS;
+  } else {
+    split = work / (row_tiles * cols);
+    work -= split * row_tiles * cols;
+  }
+  // a group's tiles in blocks of GM_BLOCK_ROWS row tiles: a block's tiles of one column, then those of the next
+  const int tiles = (end - begin + ROWS - 1) / ROWS, at = work - first_tile * cols;
+  const int block = at / (GM_BLOCK_ROWS * cols), in_block = at % (GM_BLOCK_ROWS * cols), block_rows = min(GM_BLOCK_ROWS, tiles - block * GM_BLOCK_ROWS);
+  const int row0 = begin + (block * GM_BLOCK_ROWS + in_block % block_rows) * ROWS, rows = min(ROWS, end - row0);
+  const int column = in_block / block_rows;
   const bool half = rows <= 64;  // (a group's last tile) the second 64 rows are neither fetched nor multiplied
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 15, g4 = lane >> 4;
   const int n = args.n, k = args.k;
+  const int all_steps = (k + 63) / 64, split_steps = (all_steps + args.splits - 1) / args.splits;
+  const int k_begin = split * split_steps * 64, k_end = min(k, k_begin + split_steps * 64);
   const int piece = 8 * ((lane & 7) ^ (lane >> 3));  // first index of the piece this lane asks for, in every load
   const bf16_t* a_at[A_LOADS];
   const bf16_t* w_at[W_LOADS];
@@ -335,7 +354,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   for (int m = 0; m < A_LOADS; ++m) {
     int r = row0 + min(8 * (wave + WAVES * m) + (lane >> 3), rows - 1);
     if (args.gather_top > 0) r = order[r] / args.gather_top;
-    a_at[m] = args.a + (size_t)r * args.a_ld + piece;
+    a_at[m] = args.a + (size_t)r * args.a_ld + k_begin + piece;
   }
   const bf16_t* w_base = args.w + (size_t)group * args.w_group;
 #pragma unroll
@@ -348,10 +367,10 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     } else {
       row = min(column * GM_TILE_COLS + r, n - 1);
     }
-    w_at[m] = w_base + (size_t)row * k + piece;
+    w_at[m] = w_base + (size_t)row * k + k_begin + piece;
   }
   auto ask = [&](int k0, int buffer) {
-    const bool beyond = k0 + piece >= k;  // (only ever true in a last step of fewer than 64 indices)
+    const bool beyond = k_begin + k0 + piece >= k_end;  // (only ever true in a last step of fewer than 64 indices)
 #pragma unroll
     for (int m = 0; m < A_LOADS; ++m)
       if (m == 0 || !half) load_to_lds_16(beyond ? reinterpret_cast<const bf16_t*>(gm_zero_piece) : a_at[m] + k0, smem[buffer] + 1024 * (wave + WAVES * m));
@@ -371,7 +390,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int steps = (k + 63) / 64;
+  const int steps = k_end > k_begin ? (k_end - k_begin + 63) / 64 : 0;  // (a last part may be empty: zeros)
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < steps) ask(64 * s, s);
@@ -398,7 +417,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   if (steps >= STAGES - 1) wait_for_one();
   else wait_for_loads<0>();
   __syncthreads();
-  fetch(0, 0);
+  if (steps > 0) fetch(0, 0);
   int buffer = 0;
   for (int s = 0; s < steps; ++s) {
     // operands of the second half on their way while the first half's are multiplied, and the loads of a later step into the
@@ -424,7 +443,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   // lane (g4, i) holds outputs 4 g4 .. + 3 of row i of every tile: one 8- or 16-byte store each (n is a multiple of 4)
   typedef TO Four __attribute__((ext_vector_type(4)));
-  TO* out = reinterpret_cast<TO*>(args.out);
+  TO* out = reinterpret_cast<TO*>(args.out) + (size_t)split * args.m * args.out_ld;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int r = wm * 64 + rt * 16 + i;

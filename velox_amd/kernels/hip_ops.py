@@ -98,6 +98,7 @@ class HipOps:
         self.use_skinny_gemm = True
         self.pack_decode_weights = True
         self.fuse_residual_norm = True
+        self._timed_products = set()  # (m, n, k) whose library kernels have been timed (``tune_library_products``)
         self.use_grouped_mfma = True  # (False: the grouped bfloat16 products take the exact multiply-add tiles, for tests)
         self._mm_out_dtype_ok: Optional[bool] = None
         self._bias_copies: Dict[Tuple[int, int], Tuple[torch.Tensor, torch.Tensor]] = {}
@@ -187,6 +188,8 @@ class HipOps:
         c.velox_poly_norm.argtypes = [_P, _P, _P, _I, _I, _F, _I, _P]
         c.velox_removal_chunk_scan.argtypes = [_P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _P, _P, _I, _I, _P]
         c.velox_removal_chunk_scan.restype = _I
+        c.velox_gemm_tiles_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P]
+        c.velox_gemm_tiles_bf16.restype = _I
         c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]
         c.velox_linear_chunk_scan.restype = _I
         c.velox_linear_chunk_scratch_elems.argtypes = [_I, _I, _I, _I, _I]
@@ -332,6 +335,7 @@ class HipOps:
                 for m in sorted(set(token_counts)):
                     x = torch.randn((m, k), dtype=torch.float32, device=self.device).to(torch.bfloat16)
                     torch.nn.functional.linear(x, weight)
+                    self._timed_products.add((m, n, k))
                     done += 1
                 del weight
             torch.cuda.synchronize(self.device)
@@ -797,6 +801,10 @@ class HipOps:
         if (partials_ok and bias is None and self.use_skinny_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
                 and 16 < m <= 64 and k % 64 == 0 and n <= 8192 and n % 4 == 0):
             return self.skinny_gemm_splitk(x, weight, packed=packed)
+        if bias is None and out_dtype == torch.bfloat16 and self.use_library_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
+            splits = self.tile_splits(m, n, k)
+            if splits == 1 or (splits > 1 and partials_ok):
+                return self.gemm_tiles(x, weight, splits, torch.bfloat16 if splits == 1 else torch.float32)
         skinny_rows = 16 if n > 8192 else 32  # measured on MI355X: beyond this the library's kernels stream faster
         if self.use_skinny_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and m <= skinny_rows and k % 64 == 0:
             return self.skinny_gemm(x, weight, bias, out_dtype, packed=packed, x_packed=self._packed_rows_of(x, k))
@@ -1012,6 +1020,36 @@ class HipOps:
         status = self._core.velox_skinny_gemm_splitk_bf16(_ptr(x), _ptr(weight if packed is None else packed), _ptr(out), m, n, k, splits,
                                                           int(packed is not None), self._stream())
         self._launched(status, "skinny_gemm_splitk")
+        return out
+
+    def tile_splits(self, m: int, n: int, k: int) -> int:
+        """Parts of k in which ``linear`` works a product in the framework's own tiles of 128 x 256 (0: not at all, the library's).  The
+        library gives a product with few tiles and a long sum (a feed-forward's second product) too few workgroups; here
+        the sum is cut until about every compute unit has one, and the norm that follows adds the parts.  Measured on
+        MI355X, product and norm (us, library / own): 18,944 -> 3,584 at 300 tokens 103 / 61, 512: 178 / 83, 836: 188 / 146, 1,036: 209 /
+        159, 1,536: 289 / 222, 2,048: 377 / 310, 4,096: 581 / 615; 8,448 -> 2,048 at 200: 31 / 27, 836: 53 / 47, 1,536: 65 / 74; 11,008 -> 4,096 at
+        512: 69 / 59, 836: 101 / 97, 1,036: 115 / 162; 4,096 -> 4,096 at 512: 33 / 34.  So: at least three parts, or sums so long that the
+        library is far from its rate, and one workgroup per compute unit.  Sizes that ``tune_library_products`` has timed
+        stay with the library (18,944 -> 3,584 at 2,048 tokens then takes 239 us alone)."""
+        if m <= 64 or k < 5120 or k % 8 != 0 or n % 4 != 0 or (m, n, k) in self._timed_products:
+            return 0
+        tiles, steps = -(-m // 128) * -(-n // 256), -(-k // 64)
+        if 3 * tiles <= self.num_cus:
+            splits = min(8, self.num_cus // tiles)
+        elif tiles <= self.num_cus and k >= 16384:
+            splits = min((1, 2, 3, 4), key=lambda s: -(-tiles * s // self.num_cus) * -(-steps // s))
+        else:
+            return 0
+        return -(-steps // -(-steps // splits))  # (no empty part)
+
+    def gemm_tiles(self, x, weight, splits: int = 1, out_dtype=torch.bfloat16):
+        """``x @ weight^T`` in bfloat16 in tiles of 128 x 256: [M, N] in bfloat16, or float32 partial sums [splits, M, N]."""
+        self._check("x", x, torch.bfloat16, align=16)
+        self._check("weight", weight, torch.bfloat16, (weight.shape[0], x.shape[1]), align=16)
+        m, k = x.shape
+        n = weight.shape[0]
+        out = torch.empty((m, n) if out_dtype == torch.bfloat16 else (splits, m, n), dtype=out_dtype, device=self.device)
+        self._launched(self._core.velox_gemm_tiles_bf16(_ptr(x), _ptr(weight), _ptr(out), m, n, k, int(splits), _code(out_dtype), self._stream()), "gemm_tiles")
         return out
 
     def gemm_fma(self, x, weight, bias, out_dtype):
