@@ -887,6 +887,25 @@ def test_sampling_with_rows_cut_into_chunks_gives_the_same_tokens(ops, vocab, sp
     assert (broken[has_filter] == -1).all() and (broken[~has_filter] == whole[~has_filter]).all()
 
 
+@pytest.mark.parametrize("vocab", [16384, 16389, 40000])
+@pytest.mark.parametrize("top_p, top_k", [(0.9, 0), (1.0, 40), (0.8, 300)])
+def test_sampling_with_as_many_tokens_left_as_a_list_holds(ops, vocab, top_p, top_k):
+    """Two chunks of 2,048 quads and more hand the tokens that the first digit leaves over from kernel to kernel, at most 256 a wave: rows
+    that leave a wave (quads 0 .. 63, then 1,024 .. 1,087 of the first chunk) one less, as many and one more, or none.  The one-workgroup
+    kernel has no lists: the same tokens, bit for bit."""
+    wave = [i for i in range(vocab // 2 - 8) if i // 4 % 1024 < 64]
+    logits = rand((4 * 6, vocab), torch.float32, 5, 0.5) - 30.0
+    for r in range(logits.shape[0]):
+        left = wave[:(255, 256, 257, 0)[r % 4]]
+        logits[r, left] = 4.0 + 0.9 * torch.rand(len(left), generator=torch.Generator().manual_seed(r)).to(logits)
+        logits[r, vocab - 1 - r] = 4.5
+    options = np.zeros((logits.shape[0], 6), dtype=np.int32)
+    options.view(np.float32)[:, 0], options.view(np.float32)[:, 1] = 1.0, top_p
+    options[:, 2], options[:, 3] = top_k, np.arange(logits.shape[0])
+    options = torch.from_numpy(options).cuda()
+    assert torch.equal(ops.sample(logits, options, chunks=2), ops.sample(logits, options, chunks=1))
+
+
 def test_penalties_over_long_histories_and_a_large_vocabulary(ops, ref):
     vocab, rows, width = 152064, 4, 6000
     logits = rand((rows, vocab), torch.float32, 34, 2.0)

@@ -189,7 +189,7 @@ __device__ __forceinline__ uint32_t sort_key(float v) {
 // probability.  Both conditions only get harder to meet as x falls, so the kept tokens are those whose key is at least
 // some threshold.  The threshold is found digit by digit (11, 11 and 10 bits of the 32-bit key): one pass over the row
 // fills, for the tokens that match the digits found so far, a table per value of the next digit (how many tokens, how
-// much probability); a walk down the table from the largest digit finds the last digit whose largest member is still
+// much probability); a scan down the table from the largest digit finds the last digit whose largest member is still
 // kept.  Probabilities are summed as 40-bit fixed-point integers, so a sum does not depend on the order in which the
 // threads add and a row's threshold is the same in every run and every batch.
 #define SELECT_BINS 2048
@@ -228,59 +228,77 @@ template <typename F> __device__ __forceinline__ void for_each_in_quads(const fl
   for (int i = 4 * whole + threadIdx.x; i < end; i += stride) f(i, row[i]);
 }
 
-// One digit of the search.  `counts` and `masses` hold the table of this digit (SELECT_BINS entries, filled by the whole
-// workgroup, barrier behind it); `above` is what lies above every token that matches the digits found so far.  Wave 0 walks
-// the table; every thread gets the digit found, and `above` grows by what lies above that digit's tokens.
-__device__ __forceinline__ int select_digit(const unsigned int* counts, const unsigned long long* masses, int bins, int top_k, bool use_mass,
-                                            unsigned long long mass_limit, Above& above, int* found_digit, Above* found_above) {
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    const int per_lane = bins / 64;  // lane 0 holds the largest digits
-    const int hi = bins - 1 - lane * per_lane;  // this lane's digits: hi, hi - 1, ..., hi - per_lane + 1
-    unsigned int c = 0;
-    unsigned long long m = 0;
-    for (int j = 0; j < per_lane; ++j) { c += counts[hi - j]; m += masses[hi - j]; }
-    // what lies above this lane's first digit: the sums of the lanes before it
-    unsigned int c_before = c;
-    unsigned long long m_before = m;
+// One digit of the search.  Every thread brings its share of the digit's table, the largest digits in thread 0: digits
+// hi, hi - 1, .. with hi = bins - 1 - per_thread * threadIdx.x (`c`: tokens, `m`: probability); `above` is what lies above
+// every token that matches the digits found so far.  A scan over the workgroup finds what lies above each digit; every
+// thread gets the digit found, and `above` grows by what lies above that digit's tokens.  `top_p` below 1 with
+// `first`: the table holds all tokens, so its sum is the row's whole probability and gives the limit for this level and
+// (left in `mass_limit`) the next ones.
+// One wave that walked the table out of LDS, 32 entries a lane, had all 64 lanes on one bank at every step: about 6 us a
+// digit, against 1 us for the scan (MI355X, three digits a row).
+struct SelectScratch {
+  unsigned long long wave_mass[SAMPLE_THREADS / 64];
+  unsigned int wave_count[SAMPLE_THREADS / 64];
+  int digit;
+  Above above;
+};
+
+__device__ __forceinline__ int select_digit(const unsigned int (&c)[2], const unsigned long long (&m)[2], int per_thread, int bins, int top_k, bool use_mass,
+                                            bool first, float top_p, unsigned long long& mass_limit, Above& above, SelectScratch& scratch) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  unsigned int c_before = c[0] + (per_thread > 1 ? c[1] : 0u);
+  unsigned long long m_before = m[0] + (per_thread > 1 ? m[1] : 0ull);
+  const unsigned int c_own = c_before;
+  const unsigned long long m_own = m_before;
 #pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-      const unsigned int oc = __shfl_up(c_before, offset, VELOX_WAVE);
-      const unsigned long long om = __shfl_up(m_before, offset, VELOX_WAVE);
-      if (lane >= offset) { c_before += oc; m_before += om; }
-    }
-    c_before = above.count + c_before - c;
-    m_before = above.mass + m_before - m;
-    // the smallest digit of this lane whose members' top is still kept
-    int lowest = 0x7fffffff;
-    unsigned int lowest_c = 0;
-    unsigned long long lowest_m = 0;
-    for (int j = 0; j < per_lane; ++j) {
+  for (int offset = 1; offset < 64; offset <<= 1) {
+    const unsigned int oc = __shfl_up(c_before, offset, VELOX_WAVE);
+    const unsigned long long om = __shfl_up(m_before, offset, VELOX_WAVE);
+    if (lane >= offset) { c_before += oc; m_before += om; }
+  }
+  if (lane == 63) { scratch.wave_count[wave] = c_before; scratch.wave_mass[wave] = m_before; }
+  if (threadIdx.x == 0) scratch.digit = 0x7fffffff;
+  __syncthreads();
+  c_before += above.count - c_own;
+  m_before += above.mass - m_own;
+  unsigned long long total = 0ull;
+#pragma unroll
+  for (int w = 0; w < SAMPLE_THREADS / 64; ++w) {
+    const unsigned long long wave_mass = scratch.wave_mass[w];
+    total += wave_mass;
+    if (w < wave) { c_before += scratch.wave_count[w]; m_before += wave_mass; }
+  }
+  // (at least 1: the largest token is kept however small top_p is)
+  if (first) mass_limit = max(1ull, (unsigned long long)((double)top_p * (double)total));
+  // the smallest digit of this thread whose members' top is still kept
+  const int hi = bins - 1 - (int)threadIdx.x * per_thread;
+  int lowest = 0x7fffffff;
+  Above lowest_above{0u, 0ull};
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if (j < per_thread) {
       const bool kept = (top_k <= 0 || c_before < (unsigned int)top_k) && (!use_mass || m_before < mass_limit);
-      if (kept) { lowest = hi - j; lowest_c = c_before; lowest_m = m_before; }
-      c_before += counts[hi - j];
-      m_before += masses[hi - j];
-    }
-    // over the wave: kept digits form a run from the top, so the smallest one overall is the answer
-    int best = lowest;
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) {
-      const int other = __shfl_xor(best, offset, VELOX_WAVE);
-      best = other < best ? other : best;
-    }
-    if (best == lowest && lowest != 0x7fffffff) {
-      *found_digit = lowest;
-      found_above->count = lowest_c;
-      found_above->mass = lowest_m;
-    }
-    if (best == 0x7fffffff && lane == 0) {  // (cannot happen: the largest digit's top is always kept)
-      *found_digit = bins - 1;
-      *found_above = above;
+      if (kept) { lowest = hi - j; lowest_above = Above{c_before, m_before}; }
+      c_before += c[j];
+      m_before += m[j];
     }
   }
+  // over the workgroup: kept digits form a run from the top, so the smallest one overall is the answer
+  int best = lowest;
+#pragma unroll
+  for (int offset = 32; offset > 0; offset >>= 1) {
+    const int other = __shfl_xor(best, offset, VELOX_WAVE);
+    best = other < best ? other : best;
+  }
+  if (lane == 0 && best != 0x7fffffff) atomicMin(&scratch.digit, best);
   __syncthreads();
-  above = *found_above;
-  return *found_digit;
+  int digit = scratch.digit;
+  if (digit == 0x7fffffff) digit = bins - 1;  // (cannot happen: the largest digit's top is always kept)
+  else if (lowest == digit) scratch.above = lowest_above;
+  if (scratch.digit == 0x7fffffff && threadIdx.x == 0) scratch.above = above;
+  __syncthreads();
+  above = scratch.above;
+  return digit;
 }
 
 // options per row, int32[6]: temperature (float bits), top_p (float bits), top_k, seed low 31 bits, seed high 31 bits, counter
@@ -318,81 +336,153 @@ __device__ __forceinline__ RowOptions read_options(const int* __restrict__ opt, 
 __device__ __forceinline__ int level_shift(int level) { return level == 0 ? 21 : level == 1 ? 10 : 0; }
 __device__ __forceinline__ int level_bins(int level) { return level == 2 ? 1024 : 2048; }
 
+// A level's table in LDS: what it needs of counts (top-k) and probabilities (top-p) is kept, the other is neither cleared
+// nor added to.  The first digit is sign, exponent and two bits of the mantissa: the tokens of a row share a few dozen
+// values, and lanes of a wave that add to one entry wait for each other.  Its entries are therefore kept in
+// TABLE_COPIES copies next to each other (other banks), a lane's number picks the copy.
+#define TABLE_COPIES 4
+template <int COPIES> struct LevelTables {
+  unsigned long long masses[SELECT_BINS * COPIES];
+  unsigned int counts[SELECT_BINS * COPIES];
+};
+__device__ __forceinline__ int level_copies(int level) { return level == 0 ? TABLE_COPIES : 1; }
+
+template <int C> __device__ __forceinline__ void clear_tables(LevelTables<C>& t, int level, const RowOptions& o) {
+  const int entries = level_bins(level) * level_copies(level);
+  for (int b = threadIdx.x; b < entries; b += blockDim.x) {
+    if (o.top_k > 0) t.counts[b] = 0u;
+    if (o.use_mass) t.masses[b] = 0ull;
+  }
+}
+
+template <int C> __device__ __forceinline__ void add_token(LevelTables<C>& t, int entry, float x, const RowOptions& o, float mx) {
+  if (o.top_k > 0) atomicAdd(&t.counts[entry], 1u);
+  if (o.use_mass) {
+    const unsigned long long mass = fixed_point_mass(expf(x - mx));
+    if (mass != 0ull) atomicAdd(&t.masses[entry], mass);
+  }
+}
+
 // Adds the tokens of quads [q_lo, q_hi) that match the digits found so far (`prefix`) to the tables of digit `level`
-// (`counts`, `masses`: LDS, cleared by the caller, barrier behind the clearing).  At level 0 every token's mass also goes
-// into the returned sum.
-__device__ __forceinline__ unsigned long long add_to_tables(const float* __restrict__ row, int vocab, int q_lo, int q_hi, const RowOptions& o, float mx,
-                                                            int level, uint32_t prefix, unsigned int* counts, unsigned long long* masses) {
+// (cleared by the caller, barrier behind the clearing).
+template <int C>
+__device__ __forceinline__ void add_to_tables(const float* __restrict__ row, int vocab, int q_lo, int q_hi, const RowOptions& o, float mx,
+                                              int level, uint32_t prefix, LevelTables<C>& t) {
   const int shift = level_shift(level);
   const int bins = level_bins(level);
+  const int copies = level_copies(level);
+  const int copy = threadIdx.x & (copies - 1);
   const uint32_t known = level == 0 ? 0u : ~((1u << (shift + (level == 2 ? 10 : 11))) - 1u);  // mask of the digits found so far
-  unsigned long long my_total = 0ull;
-  const bool use_mass = o.use_mass;
   const float inv_t = o.inv_t;
   for_each_in_quads(row, vocab, q_lo, q_hi, [&](int, float v) {
     const float x = v * inv_t;
     const uint32_t key = sort_key(x);
-    const bool match = (key & known) == prefix;
-    if (level == 0 || match) {
-      const unsigned long long mass = use_mass ? fixed_point_mass(expf(x - mx)) : 0ull;
-      if (level == 0) my_total += mass;
-      if (match) {
-        const int digit = (int)((key >> shift) & (uint32_t)(bins - 1));
-        atomicAdd(&counts[digit], 1u);
-        if (use_mass && mass != 0ull) atomicAdd(&masses[digit], mass);
-      }
-    }
+    if ((key & known) == prefix) add_token(t, (int)((key >> shift) & (uint32_t)(bins - 1)) * copies + copy, x, o, mx);
   });
-  return my_total;
+}
+
+// the sums of digit `bin` over the copies
+template <int C> __device__ __forceinline__ void table_entry(const LevelTables<C>& t, int level, int bin, const RowOptions& o, unsigned int& c, unsigned long long& m) {
+  const int copies = level_copies(level);
+  c = 0u;
+  m = 0ull;
+  for (int e = bin * copies; e < (bin + 1) * copies; ++e) {
+    if (o.top_k > 0) c += t.counts[e];
+    if (o.use_mass) m += t.masses[e];
+  }
+}
+
+// quad q of a row; elements beyond the vocabulary: -inf
+__device__ __forceinline__ float4_t load_quad(const float* __restrict__ row, int vocab, int q, bool aligned) {
+  float4_t v;
+  if (aligned && 4 * q + 3 < vocab) {
+    v = *reinterpret_cast<const float4_t*>(row + 4 * q);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = 4 * q + e < vocab ? row[4 * q + e] : -INFINITY;
+  }
+  return v;
+}
+
+// A wave's kept quads, waiting until there are as many as lanes.
+#define DRAW_QUEUE 128
+struct DrawQueue {
+  float4_t values[SAMPLE_THREADS / 64][DRAW_QUEUE];
+  int quads[SAMPLE_THREADS / 64][DRAW_QUEUE];
+};
+
+// token i with its word of the noise
+__device__ __forceinline__ void draw_token(int i, float x, uint32_t bits, float mx, Best& best) {
+  const float u = ((float)(bits >> 8) + 0.5f) * (1.0f / 16777216.0f);
+  const float noise = fmaxf(-logf(u), 1e-10f);
+  const float score = (x - mx) - logf(noise);
+  // (a thread's tokens come in no order: equal scores go to the smaller index here too)
+  if (score > best.value || best.index == 0x7fffffff || (score == best.value && i < best.index)) best = Best{score, i};
 }
 
 // The draw among the kept tokens of quads [q_lo, q_hi): this thread's best (score, index).
-__device__ __forceinline__ Best draw_in_quads(const float* __restrict__ row, int vocab, int q_lo, int q_hi, const RowOptions& o, float mx, uint32_t threshold) {
+// Behind a filter a token or two of 256 are kept, yet nearly every wave of quads has one: the noise (ten rounds of Philox
+// and eight logarithms a quad) would be worked out by whole waves for a lane or two.  The kept quads are therefore queued
+// in LDS first and taken up 64 at a time (48 rows of 152,064, top-p 0.9: the pass with the digit before it 19.7 us
+// without the queue, 13.4 with it).
+__device__ __forceinline__ Best draw_in_quads(const float* __restrict__ row, int vocab, int q_lo, int q_hi, const RowOptions& o, float mx, uint32_t threshold,
+                                              DrawQueue& queue) {
   Best best{-INFINITY, 0x7fffffff};
   const bool aligned = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
   const bool filter = o.filter;
   const float inv_t = o.inv_t;
-  auto load_quad = [&](int q, float (&v)[4]) {
-    if (aligned && 4 * q + 3 < vocab) {
-      const float4_t loaded = *reinterpret_cast<const float4_t*>(row + 4 * q);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  auto draw_quad = [&](int q, const float4_t& v) {
+    uint32_t bits[4];
+    philox4x32((uint32_t)q, o.counter, 0u, 0u, o.seed_lo, o.seed_hi, bits);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = loaded[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = 4 * q + e < vocab ? row[4 * q + e] : -INFINITY;
+    for (int e = 0; e < 4; ++e) {
+      const int i = 4 * q + e;
+      if (i >= vocab) break;
+      const float x = v[e] * inv_t;
+      if (filter && sort_key(x) < threshold) continue;
+      draw_token(i, x, bits[e], mx, best);
     }
   };
   constexpr int AHEAD = 4;  // quads in flight per thread
-  for (int q0 = q_lo + threadIdx.x; q0 < q_hi; q0 += AHEAD * blockDim.x) {
-    float ahead[AHEAD][4];
+  int queued = 0;           // of this wave
+  for (int base = q_lo + wave * 64; base < q_hi; base += AHEAD * (int)blockDim.x) {  // (the same for all lanes of a wave)
+    float4_t ahead[AHEAD];
 #pragma unroll
     for (int a = 0; a < AHEAD; ++a) {
-      const int qa = q0 + a * blockDim.x;
-      load_quad(qa < q_hi ? qa : q0, ahead[a]);
+      const int qa = base + lane + a * (int)blockDim.x;
+      ahead[a] = load_quad(row, vocab, qa < q_hi ? qa : q_hi - 1, aligned);
     }
 #pragma unroll
     for (int a = 0; a < AHEAD; ++a) {
-      const int q = q0 + a * blockDim.x;
-      if (q >= q_hi) break;
-      float (&v)[4] = ahead[a];
+      const int q = base + lane + a * (int)blockDim.x;
+      const float4_t v = ahead[a];
+      if (!filter) {
+        if (q < q_hi) draw_quad(q, v);
+        continue;
+      }
       bool any = false;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) any = any || (4 * q + e < vocab && !(filter && sort_key(v[e] * inv_t) < threshold));
-      if (!any) continue;  // (the noise of a quad is only worked out where a token of it is kept)
-      uint32_t bits[4];
-      philox4x32((uint32_t)q, o.counter, 0u, 0u, o.seed_lo, o.seed_hi, bits);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 4 * q + e;
-        if (i >= vocab) break;
-        const float x = v[e] * inv_t;
-        if (filter && sort_key(x) < threshold) continue;
-        const float u = ((float)(bits[e] >> 8) + 0.5f) * (1.0f / 16777216.0f);
-        const float noise = fmaxf(-logf(u), 1e-10f);
-        const float score = (x - mx) - logf(noise);
-        if (score > best.value || best.index == 0x7fffffff) best = Best{score, i};
+      for (int e = 0; e < 4; ++e) any = any || (4 * q + e < vocab && sort_key(v[e] * inv_t) >= threshold);
+      any = any && q < q_hi;
+      const unsigned long long kept = __ballot(any);
+      if (any) {
+        const int at = queued + __popcll(kept & ((1ull << lane) - 1ull));  // below 63 + 64
+        queue.values[wave][at] = v;
+        queue.quads[wave][at] = q;
+      }
+      queued += __popcll(kept);
+      if (queued >= 64) {
+        queued -= 64;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        draw_quad(queue.quads[wave][queued + lane], queue.values[wave][queued + lane]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
     }
+  }
+  if (queued > 0) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < queued) draw_quad(queue.quads[wave][lane], queue.values[wave][lane]);
   }
   return best;
 }
@@ -402,11 +492,8 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_kernel(const float* __r
                                                                 int* __restrict__ out, int vocab) {
   __shared__ Best best_scratch[16];
   __shared__ float scratch[16];
-  __shared__ unsigned int counts[SELECT_BINS];
-  __shared__ unsigned long long masses[SELECT_BINS];
-  __shared__ unsigned long long total_mass;
-  __shared__ int found_digit;
-  __shared__ Above found_above;
+  __shared__ union { LevelTables<TABLE_COPIES> tables; DrawQueue queue; } shared;  // (the draw comes when the search is over)
+  __shared__ SelectScratch select;
   const float* row = logits + (size_t)blockIdx.x * vocab;
   const RowOptions o = read_options(options + (size_t)blockIdx.x * 6, vocab);
   const int tid = threadIdx.x;
@@ -431,23 +518,22 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_kernel(const float* __r
     uint32_t prefix = 0u;  // the digits found so far, in place
 #pragma unroll 1
     for (int level = 0; level < 3; ++level) {
-      const int bins = level_bins(level);
-      for (int b = tid; b < bins; b += blockDim.x) { counts[b] = 0u; masses[b] = 0ull; }
-      if (tid == 0 && level == 0) total_mass = 0ull;
+      const int bins = level_bins(level), per_thread = bins / SAMPLE_THREADS;
+      clear_tables(shared.tables, level, o);
       __syncthreads();
-      const unsigned long long my_total = add_to_tables(row, vocab, 0, quads, o, mx, level, prefix, counts, masses);
-      if (level == 0 && o.use_mass) atomicAdd(&total_mass, my_total);
+      add_to_tables(row, vocab, 0, quads, o, mx, level, prefix, shared.tables);
       __syncthreads();
-      // (at least 1: the largest token is kept however small top_p is)
-      if (level == 0) mass_limit = max(1ull, (unsigned long long)((double)o.top_p * (double)total_mass));
-      const int digit = select_digit(counts, masses, bins, o.top_k, o.use_mass, mass_limit, above, &found_digit, &found_above);
+      unsigned int c[2] = {0u, 0u};
+      unsigned long long m[2] = {0ull, 0ull};
+      for (int j = 0; j < per_thread; ++j) table_entry(shared.tables, level, bins - 1 - tid * per_thread - j, o, c[j], m[j]);
+      const int digit = select_digit(c, m, per_thread, bins, o.top_k, o.use_mass, level == 0, o.top_p, mass_limit, above, select);
       prefix |= (uint32_t)digit << level_shift(level);
-      __syncthreads();  // the tables are free again
+      __syncthreads();  // the tables and the scratch are free again
     }
     threshold = prefix;
   }
 
-  Best best = draw_in_quads(row, vocab, 0, quads, o, mx, threshold);
+  Best best = draw_in_quads(row, vocab, 0, quads, o, mx, threshold, shared.queue);
   best = block_best(best, best_scratch);
   if (tid == 0) out[blockIdx.x] = best.index;
 }
@@ -462,15 +548,25 @@ extern "C" int velox_sample(const float* logits, const int* options, int* out, i
 // What the chunks of a row share, in global memory: each chunk's maximum and best pair, the tables of the three digits
 // (cleared by the first kernel, added to with integer atomics by the kernels of the digits) and what the search has
 // found so far.  Every workgroup of a kernel reads what the kernel before left and works out the digit before its own
-// once more for itself (a walk down 2,048 entries); the workgroup of chunk 0 writes it down for the kernels after.
+// once more for itself (a scan over 2,048 entries); the workgroup of chunk 0 writes it down for the kernels after.
 struct RowSearch {
-  unsigned long long total_mass;
+  unsigned long long mass_limit;  // top_p of the row's whole probability (after level 0)
   unsigned long long above_mass[2];
   unsigned int above_count[2];
   unsigned int prefix[2];  // the digits found after level 0 and after level 1, in place
 };
 
+// The tokens that the first digit does not rule out (of a row with top-p 0.9 or top-k 50 about one in a hundred), which each
+// wave of the kernel of the second digit leaves for the kernels behind it: those need not walk the row again (48 rows of 152,064:
+// the kernels of the second and third digit and the draw 33.7 -> 28.8 us).  A wave that finds more than LIST_ENTRIES says so, and the chunk is walked as before.  Chunks of fewer than
+// LIST_QUADS quads get no lists: they would be larger than the logits.
+#define LIST_ENTRIES 256
+#define LIST_QUADS 2048
+struct Listed { float logit; int index; };
+
 struct ChunkedScratch {
+  Listed* lists;               // [rows, chunks, waves, LIST_ENTRIES], nullptr: none
+  int* list_lengths;           // [rows, chunks, waves]
   float* chunk_max;            // [rows, chunks]
   Best* chunk_best;            // [rows, chunks]
   RowSearch* search;           // [rows]
@@ -478,7 +574,7 @@ struct ChunkedScratch {
   unsigned long long* masses;  // [rows, 3, SELECT_BINS]
 };
 
-static size_t chunked_scratch_layout(int rows, int chunks, void* base, ChunkedScratch* scratch) {
+static size_t chunked_scratch_layout(int rows, int vocab, int chunks, void* base, ChunkedScratch* scratch) {
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   size_t at = 0;
   char* p = (char*)base;
@@ -489,6 +585,10 @@ static size_t chunked_scratch_layout(int rows, int chunks, void* base, ChunkedSc
   s.search = (RowSearch*)take((size_t)rows * sizeof(RowSearch));
   s.chunk_best = (Best*)take((size_t)rows * chunks * sizeof(Best));
   s.chunk_max = (float*)take((size_t)rows * chunks * sizeof(float));
+  const size_t waves = (size_t)rows * chunks * (SAMPLE_THREADS / 64);
+  const bool listed = ((vocab + 3) / 4 + chunks - 1) / chunks >= LIST_QUADS;
+  s.lists = listed ? (Listed*)take(waves * LIST_ENTRIES * sizeof(Listed)) : nullptr;
+  s.list_lengths = listed ? (int*)take(waves * sizeof(int)) : nullptr;
   if (scratch != nullptr) *scratch = s;
   return at;
 }
@@ -521,10 +621,9 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_max_kernel(const 
   if (o.filter) {
     const int entries = 3 * SELECT_BINS;
     for (int e = c * blockDim.x + threadIdx.x; e < entries; e += chunks * blockDim.x) {
-      s.counts[(size_t)r * entries + e] = 0u;
-      s.masses[(size_t)r * entries + e] = 0ull;
+      if (o.top_k > 0) s.counts[(size_t)r * entries + e] = 0u;
+      if (o.use_mass) s.masses[(size_t)r * entries + e] = 0ull;
     }
-    if (c == 0 && threadIdx.x == 0) s.search[r].total_mass = 0ull;
   }
   float mx = -INFINITY;
   for_each_in_quads(row, vocab, q_lo, q_hi, [&](int, float v) { mx = fmaxf(mx, v * o.inv_t); });
@@ -538,28 +637,95 @@ __device__ __forceinline__ float row_max_of_chunks(const float* __restrict__ chu
   return mx;
 }
 
-// The digit of `level` from the row's finished tables (global), given what was found before; `counts`, `masses`: LDS.
-__device__ __forceinline__ uint32_t finished_digit(const ChunkedScratch& s, int r, int level, const RowOptions& o, uint32_t prefix_before, Above& above,
-                                                   unsigned int* counts, unsigned long long* masses, int* found_digit, Above* found_above) {
-  const int bins = level_bins(level);
+// The digit of `level` from the row's finished tables (global), given what was found before.
+__device__ __forceinline__ uint32_t finished_digit(const ChunkedScratch& s, int r, int level, const RowOptions& o, uint32_t prefix_before,
+                                                   unsigned long long& mass_limit, Above& above, SelectScratch& select) {
+  const int bins = level_bins(level), per_thread = bins / SAMPLE_THREADS;
   const size_t base = ((size_t)r * 3 + level) * SELECT_BINS;
-  for (int b = threadIdx.x; b < bins; b += blockDim.x) { counts[b] = s.counts[base + b]; masses[b] = s.masses[base + b]; }
-  __syncthreads();
-  const unsigned long long mass_limit = max(1ull, (unsigned long long)((double)o.top_p * (double)s.search[r].total_mass));
-  const int digit = select_digit(counts, masses, bins, o.top_k, o.use_mass, mass_limit, above, found_digit, found_above);
-  __syncthreads();  // the tables are free again
+  unsigned int c[2] = {0u, 0u};
+  unsigned long long m[2] = {0ull, 0ull};
+  for (int j = 0; j < per_thread; ++j) {
+    const int bin = bins - 1 - (int)threadIdx.x * per_thread - j;
+    if (o.top_k > 0) c[j] = s.counts[base + bin];
+    if (o.use_mass) m[j] = s.masses[base + bin];
+  }
+  const int digit = select_digit(c, m, per_thread, bins, o.top_k, o.use_mass, level == 0, o.top_p, mass_limit, above, select);
   return prefix_before | ((uint32_t)digit << level_shift(level));
+}
+
+// Lists this wave's tokens of quads [q_lo, q_hi) whose key is at least `floor`: up to LIST_ENTRIES of them in `mine` (LDS).  Returns how
+// many there are (some number above LIST_ENTRIES if there are more).
+__device__ __forceinline__ int list_tokens(const float* __restrict__ row, int vocab, int q_lo, int q_hi, const RowOptions& o, uint32_t floor, Listed* mine) {
+  constexpr int AHEAD = 4;  // quads in flight per thread
+  const bool aligned = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int found = 0;
+  for (int base = q_lo + wave * 64; base < q_hi && found <= LIST_ENTRIES; base += AHEAD * (int)blockDim.x) {  // (the same for all lanes of a wave)
+    float4_t ahead[AHEAD];
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) {
+      const int qa = base + lane + a * (int)blockDim.x;
+      ahead[a] = load_quad(row, vocab, qa < q_hi ? qa : q_hi - 1, aligned);
+    }
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) {
+      if (found > LIST_ENTRIES) break;
+      const int q = base + lane + a * (int)blockDim.x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool in = q < q_hi && 4 * q + e < vocab && sort_key(ahead[a][e] * o.inv_t) >= floor;
+        const unsigned long long all = __ballot(in);
+        if (all == 0ull) continue;
+        const int at = found + __popcll(all & ((1ull << lane) - 1ull));
+        if (in && at < LIST_ENTRIES) mine[at] = Listed{ahead[a][e], 4 * q + e};
+        found += __popcll(all);
+      }
+    }
+  }
+  return found;
+}
+
+// How many tokens the waves of a chunk have listed before each wave's own (`before`, LDS), all of them in before[waves]; -1: not all are listed.
+__device__ __forceinline__ int listed_tokens(const ChunkedScratch& s, int chunk, int* before) {
+  constexpr int WAVES = SAMPLE_THREADS / 64;
+  if (s.lists == nullptr) return -1;  // (the same for all workgroups)
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    int length = lane < WAVES ? s.list_lengths[(size_t)chunk * WAVES + lane] : 0;
+    const bool whole = __ballot(length > LIST_ENTRIES) == 0ull;
+    int upto = length;
+#pragma unroll
+    for (int offset = 1; offset < 64; offset <<= 1) {
+      const int other = __shfl_up(upto, offset, VELOX_WAVE);
+      if (lane >= offset) upto += other;
+    }
+    if (lane < WAVES) before[lane] = upto - length;
+    if (lane == WAVES) before[WAVES] = whole ? upto : -1;
+  }
+  __syncthreads();
+  return before[WAVES];
+}
+
+// f(index, logit) for the chunk's `total` listed tokens, dealt to the threads one after the other
+template <typename F> __device__ __forceinline__ void for_each_listed(const ChunkedScratch& s, int chunk, const int* before, int total, F f) {
+  constexpr int WAVES = SAMPLE_THREADS / 64;
+  for (int j = threadIdx.x; j < total; j += blockDim.x) {
+    int wave = 0;
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) wave += j >= before[w] ? 1 : 0;
+    const Listed token = s.lists[((size_t)chunk * WAVES + wave) * LIST_ENTRIES + (j - before[wave])];
+    f(token.index, token.logit);
+  }
 }
 
 // passes 2..4: the tables of digit LEVEL
 template <int LEVEL>
 __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_tables_kernel(const float* __restrict__ logits, const int* __restrict__ options,
                                                                              ChunkedScratch s, int vocab) {
-  __shared__ unsigned int counts[SELECT_BINS];
-  __shared__ unsigned long long masses[SELECT_BINS];
-  __shared__ unsigned long long total_mass;
-  __shared__ int found_digit;
-  __shared__ Above found_above;
+  __shared__ LevelTables<LEVEL == 0 ? TABLE_COPIES : 1> tables;
+  __shared__ SelectScratch select;
+  __shared__ Listed listed[LEVEL == 1 ? SAMPLE_THREADS / 64 : 1][LEVEL == 1 ? LIST_ENTRIES : 1];
+  __shared__ int before[SAMPLE_THREADS / 64 + 1], overflow;
   const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
   const float* row = logits + (size_t)r * vocab;
   const RowOptions o = read_options(options + (size_t)r * 6, vocab);
@@ -567,41 +733,74 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_tables_kernel(con
   const int tid = threadIdx.x;
   int q_lo, q_hi;
   chunk_quads(vocab, q_lo, q_hi);
+  clear_tables(tables, LEVEL, o);
+  if (tid == 0) overflow = 0;
+  const int total = LEVEL == 2 ? listed_tokens(s, r * chunks + c, before) : -1;
   const float mx = row_max_of_chunks(s.chunk_max + r * chunks, chunks);
   uint32_t prefix = 0u;
   if (LEVEL >= 1) {
     Above above{0u, 0ull};
-    if (LEVEL == 2) { prefix = s.search[r].prefix[0]; above.count = s.search[r].above_count[0]; above.mass = s.search[r].above_mass[0]; }
-    prefix = finished_digit(s, r, LEVEL - 1, o, prefix, above, counts, masses, &found_digit, &found_above);
+    unsigned long long mass_limit = 0ull;
+    if (LEVEL == 2) {
+      prefix = s.search[r].prefix[0];
+      above.count = s.search[r].above_count[0];
+      above.mass = s.search[r].above_mass[0];
+      mass_limit = s.search[r].mass_limit;
+    }
+    prefix = finished_digit(s, r, LEVEL - 1, o, prefix, mass_limit, above, select);
     if (c == 0 && tid == 0) {
+      if (LEVEL == 1) s.search[r].mass_limit = mass_limit;
       s.search[r].prefix[LEVEL - 1] = prefix;
       s.search[r].above_count[LEVEL - 1] = above.count;
       s.search[r].above_mass[LEVEL - 1] = above.mass;
     }
   }
-  const int bins = level_bins(LEVEL);
-  for (int b = tid; b < bins; b += blockDim.x) { counts[b] = 0u; masses[b] = 0ull; }
-  if (tid == 0) total_mass = 0ull;
   __syncthreads();
-  const unsigned long long my_total = add_to_tables(row, vocab, q_lo, q_hi, o, mx, LEVEL, prefix, counts, masses);
-  if (LEVEL == 0 && o.use_mass && my_total != 0ull) atomicAdd(&total_mass, my_total);
+  if (LEVEL == 1 && s.lists != nullptr) {
+    const int lane = tid & 63, wave = tid >> 6;
+    const int found = list_tokens(row, vocab, q_lo, q_hi, o, prefix, listed[wave]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const size_t list = ((size_t)r * chunks + c) * (SAMPLE_THREADS / 64) + wave;
+    if (lane == 0) s.list_lengths[list] = found;
+    for (int j = lane; j < min(found, LIST_ENTRIES); j += 64) s.lists[list * LIST_ENTRIES + j] = listed[wave][j];
+    if (lane == 0 && found > LIST_ENTRIES) overflow = 1;
+    __syncthreads();
+    if (overflow == 0) {
+      for (int j = lane; j < found; j += 64) {
+        const float x = listed[wave][j].logit * o.inv_t;
+        const uint32_t key = sort_key(x);
+        if ((key >> 21) == (prefix >> 21)) add_token(tables, (int)((key >> level_shift(1)) & (uint32_t)(level_bins(1) - 1)), x, o, mx);
+      }
+    } else {
+      add_to_tables(row, vocab, q_lo, q_hi, o, mx, LEVEL, prefix, tables);
+    }
+  } else if (LEVEL == 2 && total >= 0) {
+    for_each_listed(s, r * chunks + c, before, total, [&](int, float v) {
+      const float x = v * o.inv_t;
+      const uint32_t key = sort_key(x);
+      if ((key >> 10) == (prefix >> 10)) add_token(tables, (int)(key & (uint32_t)(level_bins(2) - 1)), x, o, mx);
+    });
+  } else {
+    add_to_tables(row, vocab, q_lo, q_hi, o, mx, LEVEL, prefix, tables);
+  }
   __syncthreads();
   const size_t base = ((size_t)r * 3 + LEVEL) * SELECT_BINS;
-  for (int b = tid; b < bins; b += blockDim.x) {
-    if (counts[b] != 0u) atomicAdd(&s.counts[base + b], counts[b]);
-    if (masses[b] != 0ull) atomicAdd(&s.masses[base + b], masses[b]);
+  for (int b = tid; b < level_bins(LEVEL); b += blockDim.x) {
+    unsigned int count;
+    unsigned long long mass;
+    table_entry(tables, LEVEL, b, o, count, mass);
+    if (count != 0u) atomicAdd(&s.counts[base + b], count);
+    if (mass != 0ull) atomicAdd(&s.masses[base + b], mass);
   }
-  if (LEVEL == 0 && tid == 0 && total_mass != 0ull) atomicAdd(&s.search[r].total_mass, total_mass);
 }
 
 // pass 5: the last digit, then the draw among the chunk's kept tokens
 __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_draw_kernel(const float* __restrict__ logits, const int* __restrict__ options,
                                                                            ChunkedScratch s, int vocab, int with_filter) {
   __shared__ Best best_scratch[16];
-  __shared__ unsigned int counts[SELECT_BINS];
-  __shared__ unsigned long long masses[SELECT_BINS];
-  __shared__ int found_digit;
-  __shared__ Above found_above;
+  __shared__ DrawQueue queue;
+  __shared__ SelectScratch select;
+  __shared__ int before[SAMPLE_THREADS / 64 + 1];
   const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
   const float* row = logits + (size_t)r * vocab;
   const RowOptions o = read_options(options + (size_t)r * 6, vocab);
@@ -616,29 +815,43 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_draw_kernel(const
     if (threadIdx.x == 0) s.chunk_best[r * chunks + c] = Best{INFINITY, -1};
     return;
   }
+  int total = -1;
   if (o.filter) {
+    total = listed_tokens(s, r * chunks + c, before);
     Above above{s.search[r].above_count[1], s.search[r].above_mass[1]};
-    threshold = finished_digit(s, r, 2, o, s.search[r].prefix[1], above, counts, masses, &found_digit, &found_above);
+    unsigned long long mass_limit = s.search[r].mass_limit;
+    threshold = finished_digit(s, r, 2, o, s.search[r].prefix[1], mass_limit, above, select);
   }
-  Best best = draw_in_quads(row, vocab, q_lo, q_hi, o, mx, threshold);
+  Best best{-INFINITY, 0x7fffffff};
+  if (total >= 0) {
+    for_each_listed(s, r * chunks + c, before, total, [&](int i, float v) {
+      const float x = v * o.inv_t;
+      if (sort_key(x) < threshold) return;
+      uint32_t bits[4];
+      philox4x32((uint32_t)(i >> 2), o.counter, 0u, 0u, o.seed_lo, o.seed_hi, bits);
+      draw_token(i, x, (i & 2) ? ((i & 1) ? bits[3] : bits[2]) : ((i & 1) ? bits[1] : bits[0]), mx, best);
+    });
+  } else {
+    best = draw_in_quads(row, vocab, q_lo, q_hi, o, mx, threshold, queue);
+  }
   best = block_best(best, best_scratch);
   if (threadIdx.x == 0) s.chunk_best[r * chunks + c] = best;
 }
 
-extern "C" long long velox_sample_chunked_scratch_bytes(int rows, int chunks) {
-  if (rows < 1 || chunks < 1) return 0;
-  return (long long)chunked_scratch_layout(rows, chunks, nullptr, nullptr);
+extern "C" long long velox_sample_chunked_scratch_bytes(int rows, int vocab, int chunks) {
+  if (rows < 1 || vocab < 1 || chunks < 1) return 0;
+  return (long long)chunked_scratch_layout(rows, vocab, chunks, nullptr, nullptr);
 }
 
 // The same tokens as velox_sample, every row cut into `chunks` chunks.  scratch: velox_sample_chunked_scratch_bytes(rows,
-// chunks) bytes at a 256-byte boundary, contents arbitrary.  with_filter = 0 promises that no row has top-k or top-p (the
+// vocab, chunks) bytes at a 256-byte boundary, contents arbitrary.  with_filter = 0 promises that no row has top-k or top-p (the
 // three kernels of the digits are then left out; a row that has one all the same gets the token -1).
 extern "C" int velox_sample_chunked(const float* logits, const int* options, int* out, int rows, int vocab, int chunks, void* scratch,
                                     long long scratch_bytes, int with_filter, hipStream_t stream) {
   if (rows <= 0) return 0;
   if (chunks < 2 || chunks > 1024 || rows > 65535 || scratch == nullptr || ((uintptr_t)scratch & 255) != 0) return -1;
   ChunkedScratch s;
-  if ((long long)chunked_scratch_layout(rows, chunks, scratch, &s) > scratch_bytes) return -1;
+  if ((long long)chunked_scratch_layout(rows, vocab, chunks, scratch, &s) > scratch_bytes) return -1;
   const dim3 grid(rows, chunks);
   sample_chunk_max_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, s, vocab);
   if (with_filter) {

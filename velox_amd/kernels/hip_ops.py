@@ -135,7 +135,7 @@ class HipOps:
         c.velox_count_sampled.argtypes = [_P, _P, _P, _I, _I, _P]
         c.velox_penalties_from_counts.argtypes = [_P, _P, _P, _P, _I, _I, _I, _P]
         c.velox_sample_chunked.argtypes = [_P, _P, _P, _I, _I, _I, _P, ctypes.c_longlong, _I, _P]
-        c.velox_sample_chunked_scratch_bytes.argtypes = [_I, _I]
+        c.velox_sample_chunked_scratch_bytes.argtypes = [_I, _I, _I]
         c.velox_sample_chunked_scratch_bytes.restype = ctypes.c_longlong
         c.velox_apply_penalties.argtypes = [_P, _P, _P, _P, _I, _I, _I, _P]
         c.velox_probe_read.argtypes = [_P, ctypes.c_longlong, _P, _I, _P]
@@ -1935,12 +1935,12 @@ class HipOps:
         if chunks is None:
             # About one workgroup per compute unit: every workgroup of a pass works out the digit before its own from the
             # row's tables again, so more chunks than fill the GPU cost more than they save (64 rows of 152,064 on
-            # MI355X: 187 us whole, 86 us in 4 chunks, 148 us in 16; 8 rows: 178 us whole, 46 us in 16 chunks).
+            # MI355X: 132 us whole, 55 us in 4 chunks, 104 us in 16; 8 rows: 36 us in 16 or 32 chunks, 57 us in 2).
             chunks = max(1, min(self.num_cus // rows, vocab // 8192, 32))
         if chunks > 1:
             if chunks > 1024 or rows > 65535:
                 raise KernelError(f"sample: {rows} rows x {chunks} chunks exceed the launch grid")
-            size = int(self._core.velox_sample_chunked_scratch_bytes(rows, chunks))
+            size = int(self._core.velox_sample_chunked_scratch_bytes(rows, vocab, chunks))
             scratch = torch.empty(size, dtype=torch.uint8, device=self.device)
             status = self._core.velox_sample_chunked(_ptr(logits), _ptr(options), _ptr(out), rows, vocab, chunks, _ptr(scratch), size,
                                                      1 if with_filter else 0, self._stream())
