@@ -44,4 +44,4 @@ class SamplingParams:
 
     @property
     def has_penalties(self) -> bool:
-        return (self.repetition_penalty, self.presence_penalty, self.frequency_penalty) != (1.0, 0.0, 0.0)
+        return not (self.repetition_penalty == 1.0 and self.presence_penalty == 0.0 and self.frequency_penalty == 0.0)
