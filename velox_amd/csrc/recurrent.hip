@@ -5,7 +5,8 @@
 //   rotate_pad_write    partial rotation of q and k, q at the attention kernels' head size, k and v into the paged cache
 //   recurrence_prepare  unit q and k, decay and beta of a linear recurrence, all float32
 //   removal_prepare     the same for the generalized delta rule: unit keys and their lengths, removal vectors, the decay's map
-//   linear_scan         the recurrence itself, token by token from the state slot (portions of prompts staged through LDS)
+//   linear_scan         the recurrence itself, token by token from the state slot (portions of prompts staged through LDS; long ones of
+//                       the first two rules with key heads of 64 or 128 channels go in chunks, linear_chunk.hip)
 //   gated_head_norm     RMS norm of each head's read-out, a shared weight, a gate
 // Everything between a load and a store is float32; stores round once.  No result depends on how a sequence's tokens
 // were cut into steps or on what else is in the batch: sums run in an order that only the sizes fix.
@@ -881,7 +882,8 @@ extern "C" int velox_removal_prepare(const void* main, int dtype, int ld, int r_
 //                              columns, beta) from memory into registers before it works through the current block out of
 //                              LDS, and writes the registers to the other LDS buffer behind it: one barrier per block, the
 //                              loads' latency lies behind a block's arithmetic.
-//   linear_scan_wave_kernel    the same for dim = 64, 128, 256, 512, a column per wave (described at the kernel).
+//   linear_scan_wave_kernel    the same for dim = 64, 128, 256, 512, a column per wave (described at the kernel).  Portions of 32 tokens and
+//                              more of dim = 64 and 128 come here only with the removal rule or where the chunks' scratch would be too large.
 // The first two give the same bits: they differ in where the operands wait, not in what is done with them; the third sums in
 // another order (which, like theirs, only the sizes fix).
 // ---------------------------------------------------------------------------------------------
