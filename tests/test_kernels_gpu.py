@@ -1255,6 +1255,32 @@ def test_portions_of_heads_of_256_channels(ops, ref, nh, nkv, page, window):
     torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-2)  # (the tolerance of the other bfloat16 attention tests above)
 
 
+@pytest.mark.parametrize("n, k", [(128, 224), (100, 96), (4, 8), (260, 72)])
+@pytest.mark.parametrize("gated", [None, "output", "head"])
+def test_per_head_products_in_pieces_of_four_and_one_by_one(ops, n, k, gated):
+    """Rows laid out for 8-byte stores and gate loads, and the same rows two columns further on, which are written one by one: the same
+    bits, nothing beside them touched, and the float32 product within one rounding of the result and, with a gate, its exponential."""
+    rows, heads = 130, 5
+    x, maps = rand((rows, heads * k), torch.bfloat16, n), rand((heads, n, k), torch.bfloat16, k, k ** -0.5)
+    wide = n + 4
+    want = torch.stack([x.float()[:, h * k:(h + 1) * k] @ maps[h].float().T for h in range(heads)], 1)
+    gate = None
+    if gated is not None:
+        gate = rand((rows, 8 + (heads * n if gated == "output" else heads)), torch.bfloat16, 3)
+        z = gate[:, 4:4 + (heads * n if gated == "output" else heads)].float().reshape(rows, heads, -1)
+        want = want * torch.sigmoid(z)
+    results = []
+    for offset in (0, 2):
+        out = torch.full((rows, heads * wide), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.head_linear(x, k, 0, maps, out, wide, offset, gate, 4 if gate is not None else 0, gated == "head")
+        out = out.view(rows, heads, wide)
+        results.append(out[:, :, offset:offset + n])
+        assert torch.all(out[:, :, :offset] == 7.0) and torch.all(out[:, :, offset + n:] == 7.0)
+    assert torch.equal(results[0], results[1])
+    # bfloat16's unit roundoff is 2^-8; float32 sums of k terms of size about k^-1/2 are off by far less than 1e-4
+    assert torch.all((results[0].float() - want).abs() <= 2.0 ** -8 * 1.01 * want.abs() + 1e-4)
+
+
 @pytest.mark.parametrize("m, n, k, splits", [(65, 100, 5128, 1), (128, 256, 64, 1), (129, 260, 200, 2), (300, 516, 1096, 3), (1100, 300, 520, 5), (70, 1024, 72, 8)])
 def test_products_in_tiles_with_a_cut_sum(ops, m, n, k, splits):
     """Against float64: remainders in all sizes, more than one block of row tiles, a last part that is short or empty.  Float32 sums of at

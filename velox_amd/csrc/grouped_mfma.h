@@ -128,27 +128,57 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
       for (int t = 0; t < GM_NT; ++t) w_cur[u][t] = w_next[u][t];
   }
 
+  // A lane holds four neighbouring outputs of a row: one store, and one load of their gates, where the rows are laid out for it.
+  // (Element by element the per-head products were bound by their stores and gates, not by what they move.  Measured on
+  // MI355X, 2,500 rows, 32 heads: 224 -> 128 with a gate per output 53.5 -> 28.2 us, 96 -> 224 45.9 -> 23.7; 16 rows 7.4 -> 5.8 and
+  // 6.1 -> 4.9.)
+  typedef TO Four __attribute__((ext_vector_type(4)));
   TO* out = reinterpret_cast<TO*>(args.out);
+  const bool vec = ((n | args.out_ld | args.out_group) & 3) == 0 && ((uintptr_t)args.out & (sizeof(Four) - 1)) == 0;
+  const bool gate_vec = EPI == GM_GATE && args.gate_col == 1 && ((args.gate_ld | args.gate_group) & 3) == 0 && ((uintptr_t)args.gate & 7) == 0;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int r = mt * 16 + i;
     if (r >= rows) continue;
     const size_t out_row = (size_t)(row0 + r) * args.out_ld + (size_t)group * args.out_group;
 #pragma unroll
-    for (int t = 0; t < (EPI == GM_GLU ? GM_NT / 2 : GM_NT); ++t)
+    for (int t = 0; t < (EPI == GM_GLU ? GM_NT / 2 : GM_NT); ++t) {
+      const int col = col0[t] + 4 * g4;
+      if (col >= n) continue;
+      float v[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = col0[t] + 4 * g4 + j;
-        if (col >= n) continue;
-        float v = acc[t][mt][j];
-        if (EPI == GM_GLU) v = glu_middle(v, acc[t + GM_NT / 2][mt][j], args.unit);
-        if (EPI == GM_GATE) {
-          const float z = to_f32(args.gate[(size_t)(row0 + r) * args.gate_ld + (size_t)group * args.gate_group + (size_t)col * args.gate_col]);
-          v *= 1.f / (1.f + expf(-z));
+      for (int j = 0; j < 4; ++j) v[j] = EPI == GM_GLU ? glu_middle(acc[t][mt][j], acc[t + GM_NT / 2][mt][j], args.unit) : acc[t][mt][j];
+      if (EPI == GM_GATE) {
+        const bf16_t* gate = args.gate + (size_t)(row0 + r) * args.gate_ld + (size_t)group * args.gate_group;
+        float z[4];
+        if (gate_vec && vec) {
+          const short4_t held = *reinterpret_cast<const short4_t*>(gate + col);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) z[j] = __uint_as_float(((uint32_t)(uint16_t)held[j]) << 16);
+        } else if (args.gate_col == 0) {
+          z[0] = z[1] = z[2] = z[3] = to_f32(gate[0]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) z[j] = to_f32(gate[(size_t)min(col + j, n - 1) * args.gate_col]);
         }
-        if (EPI == GM_ACT) v = ungated_act(v, args.act);
-        out[out_row + col] = from_f32<TO>(v);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] *= 1.f / (1.f + expf(-z[j]));
       }
+      if (EPI == GM_ACT) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = ungated_act(v[j], args.act);
+      }
+      if (vec) {
+        Four four;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) four[j] = from_f32<TO>(v[j]);
+        *reinterpret_cast<Four*>(out + out_row + col) = four;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (col + j < n) out[out_row + col + j] = from_f32<TO>(v[j]);
+      }
+    }
   }
 }
 
