@@ -1281,6 +1281,23 @@ def test_per_head_products_in_pieces_of_four_and_one_by_one(ops, n, k, gated):
     assert torch.all((results[0].float() - want).abs() <= 2.0 ** -8 * 1.01 * want.abs() + 1e-4)
 
 
+@pytest.mark.parametrize("tokens", [65, 512, 513, 3072, 3073])
+@pytest.mark.parametrize("kv_heads, dim, heads, columns", [(3, 40, 6, 6), (8, 64, 8, 520)])
+def test_what_a_recurrence_reads_does_not_depend_on_how_tokens_are_spread(ops, tokens, kv_heads, dim, heads, columns):
+    """One, two and eight workgroups a token: the same bits as 40 tokens at a time."""
+    main, decay = rand((tokens, 2 * kv_heads * dim + 8), torch.bfloat16, tokens), rand((tokens, columns), torch.float32, 2)
+    rate, bias, beta = rand((heads,), torch.float32, 3).abs(), rand((columns,), torch.float32, 4), rand((tokens, heads), torch.bfloat16, 5)
+
+    def prepare(rows):
+        return ops.recurrence_prepare(main[rows].contiguous(), 0, kv_heads * dim, kv_heads, dim, True, 0.3, decay[rows].contiguous(), 0, heads, columns, rate, bias, 1.0, beta[rows].contiguous(), 0)
+
+    whole = prepare(slice(0, tokens))
+    for first in (0, tokens // 2, tokens - 40):
+        rows = slice(first, first + 40)
+        for got, want in zip(whole, prepare(rows)):
+            assert torch.equal(got[rows], want)
+
+
 @pytest.mark.parametrize("m, n, k, splits", [(65, 100, 5128, 1), (128, 256, 64, 1), (129, 260, 200, 2), (300, 516, 1096, 3), (1100, 300, 520, 5), (70, 1024, 72, 8)])
 def test_products_in_tiles_with_a_cut_sum(ops, m, n, k, splits):
     """Against float64: remainders in all sizes, more than one block of row tiles, a last part that is short or empty.  Float32 sums of at

@@ -745,7 +745,11 @@ extern "C" int velox_recurrence_prepare(const void* qkv, int qkv_dtype, int ld, 
   if (heads < 1 || columns % heads != 0) return (int)hipErrorInvalidValue;
   PrepareArgs a{qkv, qkv_dtype == VELOX_BF16, ld, q_at, k_at, kv_heads, dim, unit, q_scale, decay_src, decay_dtype == VELOX_BF16, decay_ld, decay_at, heads,
                 columns, rate, bias, sign, beta_src, beta_dtype == VELOX_BF16, beta_ld, beta_at, qk, decay, beta};
-  const int parts = tokens <= 64 ? 8 : 1;
+  // A token's work is a chain of a few trips to memory per head, so a step of few tokens spreads each over several workgroups until
+  // the card is full (2,048 of them run at a time); each number comes out the same whichever workgroup works it.  Measured on MI355X
+  // (us with 1, 2, 4, 8 workgroups a token; 8 heads of 128 with a decay per channel): 65 tokens 8.1 5.2 3.8 3.8, 300: 9.1 6.2 5.1 5.1, 1,000: 12.1
+  // 10.7 10.7 10.7, 2,421: 24.6 21.7 22.6 23.5, 4,096: 32.8 32.6 35.1 37.9; 32 heads of 64 at 300 tokens: 19.0 12.0 9.1 8.8.
+  const int parts = tokens <= 512 ? 8 : tokens <= 3072 ? 2 : 1;
   recurrence_prepare_kernel<<<dim3(tokens, parts), 256, 0, stream>>>(a);
   VELOX_RETURN_LAUNCH_STATUS();
 }
