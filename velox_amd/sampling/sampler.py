@@ -14,14 +14,18 @@ sits; unseeded requests get a seed from the sampler's own generator when first s
 """
 from __future__ import annotations
 
+import math
 import random
-from array import array
+import struct
 from typing import Dict, List, Optional, Sequence
 
 import numpy as np
 import torch
 
 from .params import SamplingParams
+
+_ROW = struct.Struct("=ffiiii")  # a row's options as the kernel reads them: temperature, top_p, top_k, the seed's two halves, the counter
+_FLOAT32_END = (2.0 - 2.0 ** -24) * 2.0 ** 127  # from here on a number rounds to infinity in float32
 
 
 class _Upload:
@@ -152,10 +156,10 @@ class Sampler:
         if all(p.is_greedy for p in sampling_params):
             tokens = self.ops.argmax(logits)
         else:
-            # (the rows' options go into two flat lists and from there into the array: an element of a numpy array set by itself
-            # costs as much as a whole row this way, and the host's share of a call was longer than the kernels' 46 us of 48 rows)
-            floats, integers, with_filter = [], [], False
-            known = self._seeds
+            # (the rows are packed into bytes: setting the elements of a numpy array one by one took the host longer than the
+            # kernels' 46 us of 48 rows; 48 rows 39 -> 23 us, one row 2.4 -> 1.6)
+            buffer, at, with_filter = bytearray(_ROW.size * rows), 0, False
+            known, put = self._seeds, _ROW.pack_into
             for p, rid, n in zip(sampling_params, request_ids, num_generated):
                 seed = known.get(rid)
                 if seed is None:
@@ -164,11 +168,9 @@ class Sampler:
                 top_k = int(top_k) if 0 < top_k < vocab else 0
                 if (top_k or top_p < 1.0) and temperature != 0.0:
                     with_filter = True
-                floats += (temperature, top_p)
-                integers += (top_k, seed & 0x7FFFFFFF, (seed >> 31) & 0x7FFFFFFF, int(n))
-            packed = np.zeros((rows, 6), dtype=np.int32)
-            packed[:len(integers) // 4, :2] = np.frombuffer(array("f", floats), dtype=np.int32).reshape(-1, 2)
-            packed[:len(integers) // 4, 2:] = np.frombuffer(array("i", integers), dtype=np.int32).reshape(-1, 4)
+                put(buffer, at, temperature if temperature < _FLOAT32_END else math.inf, top_p, top_k, seed & 0x7FFFFFFF, (seed >> 31) & 0x7FFFFFFF, int(n))
+                at += _ROW.size
+            packed = np.frombuffer(buffer, dtype=np.int32).reshape(rows, 6)
             tokens = self.ops.sample(logits, self._upload.send(packed), with_filter=with_filter)
         if row_of is not None:
             self.ops.count_sampled(self._seen.table, row_of, tokens)  # the new tokens are seen from the next step on
