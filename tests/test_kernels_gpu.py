@@ -1220,7 +1220,7 @@ def test_grouped_products_at_the_edges_of_their_tiles(ops, rows, hidden, inter, 
         w1, w2 = first.view(experts, -1, hidden)[e].double(), down.view(experts, hidden, inter)[e].double()
         t, k = (choice == e).nonzero(as_tuple=True)
         share = weight[t, k].double()[:, None]
-        both = x[t].double() @ w1.T * (share if scale_input else 1.0)
+        both = ((x[t].float() * share.float()).bfloat16() if scale_input else x[t]).double() @ w1.T  # (a scaled row is a bfloat16 row, as in the reference)
         middle = both[:, :inter] * torch.sigmoid(both[:, :inter]) * both[:, inter:] if unit == "glu" else torch.relu(both).square()
         want.index_add_(0, t, middle @ w2.T * (1.0 if scale_input else share))
         spread.index_add_(0, t, middle.abs() @ w2.abs().T * (1.0 if scale_input else share))
@@ -1228,6 +1228,26 @@ def test_grouped_products_at_the_edges_of_their_tiles(ops, rows, hidden, inter, 
     want += (x.double()[:, None, :] * (weight.double() * none)[:, :, None]).sum(1)
     bound = (2.0 ** -8 + 2e-5) * spread + 2.0 ** -8 * 1.01 * want.abs() + 1e-6
     assert torch.all((got.double() - want).abs() <= bound), float(((got.double() - want).abs() / bound).max())
+
+
+@pytest.mark.parametrize("tokens, top, hidden, inter, unit", [(1, 2, 64, 72, "glu"), (7, 3, 328, 64, "glu"), (16, 4, 200, 136, "relu2"), (21, 3, 264, 40, "glu"), (22, 3, 264, 40, "glu"),
+                                                              (90, 2, 136, 264, "relu2"), (300, 4, 520, 72, "glu")])
+def test_rows_that_their_pairs_weight_scales_are_rounded_once_on_every_path(ops, tokens, top, hidden, inter, unit):
+    """Up to 64 pairs are scaled where they are loaded, more are copied: the same bits as rows that were scaled beforehand (a float32
+    product, one rounding).  Each token has one pair with an expert, so nothing is added up behind the products."""
+    experts, branches = 6, 2 if unit == "glu" else 1
+    generator = torch.Generator().manual_seed(tokens)
+    x, weight = rand((tokens, hidden), torch.bfloat16, tokens), torch.rand(tokens, top, generator=generator).cuda() + 0.3
+    first = rand((experts * branches * inter, hidden), torch.bfloat16, 1, hidden ** -0.5)
+    down = rand((experts * hidden, inter), torch.bfloat16, 2, inter ** -0.5)
+    at = torch.arange(tokens, device="cuda")
+    choice = torch.full((tokens, top), experts, dtype=torch.int32, device="cuda")  # (no expert: such a pair has no row)
+    choice[at, at % top] = torch.randint(0, experts, (tokens,), generator=generator).to(torch.int32).cuda()
+    more = {"ungated": unit} if unit != "glu" else {}
+    got = ops.routed_experts(x, choice, weight, first, down, experts, True, None, torch.bfloat16, **more)
+    rows = (x.float() * weight[at, at % top][:, None]).bfloat16()
+    want = ops.routed_experts(rows, choice, torch.ones_like(weight), first, down, experts, False, None, torch.bfloat16, **more)
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("m, n, k", [(17, 64, 128), (33, 65, 36), (64, 100, 256), (70, 333, 260), (65, 2048, 1540), (200, 2048, 516), (300, 6500, 132), (610, 1536, 288), (1025, 4100, 196)])

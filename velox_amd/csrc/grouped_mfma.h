@@ -41,7 +41,7 @@ struct GroupedArgs {
   const bf16_t* gate;  // GM_GATE: times sigmoid(gate[r * gate_ld + g * gate_group + col * gate_col]); (n, 1) is a number per output, (1, 0) one per group
   long long gate_ld, gate_group, gate_col;
   int act = 0;         // GM_ACT: the result goes through ungated_act(., act)
-  const float* row_scale;  // with a plan: the sums in front of a GLU or an activation are multiplied with row_scale[order[r]] (nullptr: none)
+  const float* row_scale;  // grouped_mfma_few_rows_kernel: row r of `a` times row_scale[order[r]], rounded to bfloat16, takes its place (nullptr: none)
   int splits = 1;          // grouped_tiles_kernel without a plan: parts of k, each with a result [m, out_ld] of its own, one after the other
   int gather_top = 0;      // with a plan: > 0: sorted row r is row order[r] / gather_top of `a`
   GluUnit unit = {1.f, INFINITY, 0.f};  // GM_GLU: the unit's middle (see glu_middle)
@@ -186,7 +186,8 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
 // W once, and what counts is how many loads are in flight.  A workgroup owns 32 output columns (GLU: 16 gate columns and
 // their up columns) of one tile; its four waves split K into quarters, each wave asks for four steps' operands at once, W's a
 // round ahead, and the waves' sums are added through LDS in the order of the waves (no atomics: the same result on every
-// run).  A tile works as many 16-row tiles as it has rows, whatever the step's number of pairs would allow.  Measured on MI355X: 64
+// run).  A tile works as many 16-row tiles as it has rows, whatever the step's number of pairs would allow.  With `row_scale` the
+// rows are scaled in registers, behind the wait for them and before that for W: the same bits as a scaled copy.  Measured on MI355X: 64
 // pairs over 32 experts of 4,096 -> 1,408 -> 4,096 122 + 70 us (W: 650 + 325 MB; before: 143 + 82, rows copied by another kernel).
 template <int EPI, typename TO, int MT>
 __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int group, const int row0, const int rows, const int* order,
@@ -217,9 +218,12 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
   };
   ask(k_begin);
   const bf16_t* a_row[MT];
+  float factor[MT];
+  const bool scaled = EPI != GM_PLAIN && args.row_scale != nullptr;  // (uniform)
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     int r = row0 + min(mt * 16 + i, rows - 1);
+    factor[mt] = scaled ? args.row_scale[order[r]] : 1.f;
     if (args.gather_top > 0) r = order[r] / args.gather_top;
     a_row[mt] = args.a + (size_t)r * args.a_ld + (size_t)group * args.a_group + 8 * g4;
   }
@@ -238,6 +242,16 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
       for (int mt = 0; mt < MT; ++mt) av[mt][u] = gm_load(a_row[mt] + k0 + 32 * u, k0 + 32 * u + 8 * g4 < k_end);
     }
     ask(k0 + 128);
+    if (scaled) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (k0 + 32 * u + 8 * g4 >= k_end) continue;  // (zeros stay zeros, whatever the factor is)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) av[mt][u][e] = from_f32<bf16_t>(to_f32(av[mt][u][e]) * factor[mt]);
+      }
+    }
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -269,16 +283,14 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
     const int r = mt * 16 + i;
     if (r >= rows) continue;
     const size_t out_row = (size_t)(row0 + r) * args.out_ld + (size_t)group * args.out_group;
-    float scale = 1.f;
-    if (EPI != GM_PLAIN && args.row_scale != nullptr) scale = args.row_scale[order[row0 + r]];
 #pragma unroll
     for (int t = 0; t < (EPI == GM_GLU ? 1 : 2); ++t)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int col = col0[t] + 4 * g4 + j;
         if (col >= n) continue;
-        float v = acc[t][mt][j] * scale;
-        if (EPI == GM_GLU) v = glu_middle(v, acc[1][mt][j] * scale, args.unit);
+        float v = acc[t][mt][j];
+        if (EPI == GM_GLU) v = glu_middle(v, acc[1][mt][j], args.unit);
         if (EPI == GM_GATE) {
           const float z = to_f32(args.gate[(size_t)(row0 + r) * args.gate_ld + (size_t)group * args.gate_group + (size_t)col * args.gate_col]);
           v *= 1.f / (1.f + expf(-z));
@@ -314,8 +326,7 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
 // second's are.  A row of 64 indices is 128 bytes, eight pieces of 16; the pieces of row r are exchanged by an XOR with r's low
 // three bits, which the loads do by asking for another piece (lane l's piece always lands at base + 16 l): no bank
 // conflicts.  The rows of `a` are fetched where they are: with `gather_top` sorted row r is row order[r] / gather_top of `a`, and
-// the pair's weight, if it scales the unit's input, multiplies the float32 sums instead (W (s x) = s (W x)): no sorted copy is
-// made and nothing is rounded in between.  The tiles of one expert that read the same rows of W come one after the other on
+// no sorted copy is made (rows that the pair's weight scales do come as a sorted copy, routed_scale_kernel).  The tiles of one expert that read the same rows of W come one after the other on
 // the same XCD (workgroups are dealt to the eight XCDs in turn), so W leaves HBM once.
 // Measured on MI355X (both products; before: 128 rows x 256 columns with W straight from global memory into the matrix
 // instructions' layout and one step of loads in flight): 10,000 pairs over 32 experts, 4,096 -> 1,408 -> 4,096: 748 + 280 -> 294 +
@@ -478,8 +489,6 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   for (int rt = 0; rt < RT; ++rt) {
     const int r = wm * 64 + rt * 16 + i;
     if (r >= rows) continue;
-    float scale = 1.f;
-    if (EPI != GM_PLAIN && args.row_scale != nullptr) scale = args.row_scale[order[row0 + r]];
     TO* out_row = out + (size_t)(row0 + r) * args.out_ld;
 #pragma unroll
     for (int ct = 0; ct < (EPI == GM_GLU ? CT / 2 : CT); ++ct) {
@@ -489,8 +498,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         float v = acc[ct][rt][j];
-        if (EPI == GM_GLU) v = glu_middle(v * scale, acc[ct + CT / 2][rt][j] * scale, args.unit);
-        if (EPI == GM_ACT) v = ungated_act(v * scale, args.act);
+        if (EPI == GM_GLU) v = glu_middle(v, acc[ct + CT / 2][rt][j], args.unit);
+        if (EPI == GM_ACT) v = ungated_act(v, args.act);
         four[j] = from_f32<TO>(v);
       }
       *reinterpret_cast<Four*>(out_row + col) = four;

@@ -456,9 +456,29 @@ extern "C" int velox_grouped_down(const void* act, const void* down, float* y, c
 }
 
 // ---------------------------------------------------------------------------------------------
-// bfloat16 on the matrix cores: the first product fetches the rows of x through the plan and, when the pair's weight scales the
-// expert's input, scales its float32 sums; the second reads sorted rows.
+// bfloat16 on the matrix cores: the first product fetches the rows of x through the plan, the second reads sorted rows.  When the
+// pair's weight scales the expert's input, the scaled row is rounded to bfloat16 (a float32 product, one rounding) on every path:
+// a router behind it that stands near a tie then chooses alike however many pairs a step has.  Up to 64 pairs are scaled where the
+// first product loads them; more are copied into the plan's order by the kernel below, 16 bytes a thread.  Bound by what it moves: a
+// step of 2,500 tokens of 4 x 4,096 is about 28 us longer per layer with it than with unscaled rows, one of 64 pairs about 3 us.
 // ---------------------------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) routed_scale_kernel(const bf16_t* __restrict__ x, const int* __restrict__ order, const float* __restrict__ pair_weight,
+                                                           bf16_t* __restrict__ sorted, int top, int hidden, const int* __restrict__ placed) {
+  const int row = blockIdx.x;
+  if (row >= *placed) return;  // (pairs whose expert the plan leaves out have no row: `order` ends at the placed ones)
+  const int pair = order[row];
+  const float w = pair_weight[pair];
+  typedef bf16_t Pieces __attribute__((ext_vector_type(8)));
+  const Pieces* src = reinterpret_cast<const Pieces*>(x + (size_t)(pair / top) * hidden);
+  Pieces* dst = reinterpret_cast<Pieces*>(sorted + (size_t)row * hidden);
+  for (int at = threadIdx.x; at < hidden / 8; at += 256) {
+    Pieces piece = src[at];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) piece[e] = from_f32<bf16_t>(to_f32(piece[e]) * w);
+    dst[at] = piece;
+  }
+}
+
 static GroupedArgs routed_args(const void* a, const void* w, void* out, const int* plan, int pairs, int experts, int n, int k, int w_rows) {
   GroupedArgs args = {};
   args.a = (const bf16_t*)a;
@@ -476,19 +496,23 @@ static GroupedArgs routed_args(const void* a, const void* w, void* out, const in
   return args;
 }
 
-// x [T, hidden] -> act [pairs, inter] -> y [pairs, hidden] float32.  Needs hidden % 8 == 0, inter % 8 == 0 and x on a 16-byte
-// boundary (the caller checks).  The plan's tiles hold 64 rows for up to 64 pairs, GM_TILE_ROWS for more.
-extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, const void* down, void* act, float* y, const int* plan,
+// x [T, hidden] -> (`sorted` [pairs, hidden], with scale_input and more than 64 pairs) -> act [pairs, inter] -> y [pairs, hidden]
+// float32.  Needs hidden % 8 == 0, inter % 8 == 0 and x and `sorted` on 16-byte boundaries (the caller checks).  The plan's tiles hold 64 rows for up to 64 pairs, GM_TILE_ROWS for more.
+extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, const void* down, void* sorted, void* act, float* y, const int* plan,
                                           const float* pair_weight, int pairs, int experts, int top, int inter, int hidden, int scale_input,
                                           float alpha, float limit, float shift, int ungated, hipStream_t stream) {
   // `ungated` > 0: `gate_up` holds [experts * inter, hidden] (up rows only) and the unit is ungated_act(up, ungated)
   if (pairs <= 0) return 0;
-  if (hidden % 8 != 0 || inter % 8 != 0 || top < 1 || (uintptr_t)x % 16 != 0) return -1;
+  if (hidden % 8 != 0 || inter % 8 != 0 || top < 1 || ((uintptr_t)x | (uintptr_t)sorted) % 16 != 0) return -1;
+  const bool copied = scale_input && pairs > RT_BM;
+  if (copied && sorted == nullptr) return -1;
   const int max_tiles = velox_routed_max_tiles(pairs, experts);
   if (max_tiles > 65535) return -1;
-  GroupedArgs first = routed_args(x, gate_up, act, plan, pairs, experts, inter, hidden, ungated > 0 ? inter : 2 * inter);
-  first.gather_top = top;
-  first.row_scale = scale_input ? pair_weight : nullptr;
+  if (copied)
+    routed_scale_kernel<<<pairs, 256, 0, stream>>>((const bf16_t*)x, plan + 1 + (experts + 1), pair_weight, (bf16_t*)sorted, top, hidden, plan + 1 + experts);
+  GroupedArgs first = routed_args(copied ? sorted : x, gate_up, act, plan, pairs, experts, inter, hidden, ungated > 0 ? inter : 2 * inter);
+  first.gather_top = copied ? 0 : top;
+  first.row_scale = scale_input ? pair_weight : nullptr;  // (read by the kernel for few rows alone)
   first.act = ungated;
   first.unit = GluUnit{alpha, limit, shift};
   if (ungated > 0) grouped_mfma_launch<GM_ACT, bf16_t>(first, pairs, max_tiles, 1, stream);
