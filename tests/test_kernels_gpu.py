@@ -1275,6 +1275,28 @@ def test_portions_of_heads_of_256_channels(ops, ref, nh, nkv, page, window):
     torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-2)  # (the tolerance of the other bfloat16 attention tests above)
 
 
+@pytest.mark.parametrize("nh, nkv, page", [(32, 1, 16), (6, 2, 8), (65, 1, 32)])
+@pytest.mark.parametrize("window", [None, 90])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_portions_of_heads_of_256_channels_have_the_general_kernels_bits(ops, nh, nkv, page, window, splits):
+    """Direct loads change how keys and values reach LDS and not what is added in which order: a latent's outputs reach a router, and a
+    token that stands near a tie there must not go to another expert because of the kernel its step has run."""
+    from velox_amd.engine.batch import Workspace
+
+    seqs = [(1, 129), (4, 4), (64, 64), (5, 69), (43, 107), (130, 200), (2, 63), (33, 330), (300, 777)]
+    case = _attention_case(torch.bfloat16, nh, nkv, 256, page, seqs, seed=nh + page)
+    case["qkv"] *= 2  # (scores that move a row's maximum now and then)
+    lib = ops.attention_library(256)
+    try:
+        results = []
+        for choice in (1, 0):
+            lib.velox_attention_portion_kernel(choice)
+            results.append(_run_attention(ops, case, nh, nkv, 256, page, window=window, splits=splits, workspace=Workspace(torch.device("cuda"))))
+    finally:
+        lib.velox_attention_portion_kernel(0)
+    assert torch.equal(results[0], results[1])
+
+
 @pytest.mark.parametrize("n, k", [(128, 224), (100, 96), (4, 8), (260, 72)])
 @pytest.mark.parametrize("gated", [None, "output", "head"])
 def test_per_head_products_in_pieces_of_four_and_one_by_one(ops, n, k, gated):

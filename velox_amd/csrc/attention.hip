@@ -721,6 +721,11 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
 // of keys 8 g .. 8 g + 7 of the block: eight consecutive keys, which is one 16-byte piece of a V^T row in its natural
 // order.  (The general kernel reorders V^T instead, in pieces of 8 bytes; a direct load cannot.)  For such a row of K
 // f(k) is i & 7 for lane i: a constant of the lane.
+//
+// Heads of 256 channels (latents, whose outputs reach a router) keep the general kernel's order of additions, and with it its
+// bits: tile t's row i is key 16 t + i (f(k) = k & 7), a lane takes its eight values of a channel as two pieces of 8 bytes (no bank
+// conflicts either, two read instructions where one did), a row's exponents always refer to its maximum, and with split keys
+// each half of 64 rows walks the tiles that a workgroup of the general kernel would.
 __device__ __attribute__((aligned(16))) const unsigned int zero_piece[4] = {0u, 0u, 0u, 0u};
 
 // KSPLIT = 2: two sets of WAVES waves own the same rows and take the key tiles alternately, each set with tile buffers of
@@ -749,6 +754,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
   constexpr int SETW = 64 * WAVES;                  // threads of a set of waves
   constexpr int MERGE_BYTES = KSPLIT > 1 ? 4 * SETW * CT * (4 * NC + 2) : 0;  // what the second set hands over at the end
   static_assert(MERGE_BYTES <= KSPLIT * 4 * TILE_BYTES, "the hand-over fits into the tile buffers");
+  constexpr bool SAME_BITS = D == 256;              // the general kernel's order of keys and exponents (see above)
   __shared__ __attribute__((aligned(1024))) char smem_all[KSPLIT][2][2 * TILE_BYTES];
   __shared__ int page_ids[PREFILL_PAGE_IDS];
 
@@ -795,9 +801,38 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
   const int n_begin = keys.n_begin;
   const int tiles_total = keys.kept_tiles + (n_end - n_begin + BN - 1) / BN;
   const int tiles_per_split = (tiles_total + splits - 1) / splits;
-  const int tile_lo = split * tiles_per_split;
+  int tile_lo = split * tiles_per_split;
   int tile_hi = tile_lo + tiles_per_split;
   if (tile_hi > tiles_total) tile_hi = tiles_total;
+  // this wave's tiles of them: with split keys (and no kept ones) those that its 64 rows would have as a row block of their own
+  int own_lo = tile_lo, own_hi = tile_hi;
+  if constexpr (SAME_BITS && !KEEPS) {
+    if (splits > 1) {
+      static_assert(!SAME_BITS || (WAVES * CT == 8 && KSPLIT == 1), "two halves of 64 rows");
+      tile_lo = 0x7fffffff;
+      tile_hi = 0;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const int first_row = r0 + 64 * half, end_row = first_row + 63 < rows_total - 1 ? first_row + 63 : rows_total - 1;
+        if (first_row >= rows_total) continue;
+        const int begin = KeyTiles::of<BN>(ctx + first_row / group - window + 1, window, 0, page_shift).n_begin;
+        int end = ctx + end_row / group + 1;
+        if (end > kv_len) end = kv_len;
+        const int total = (end - begin + BN - 1) / BN, per_split = (total + splits - 1) / splits, before = (begin - n_begin) / BN;
+        const int lo = before + split * per_split;
+        const int hi = before + (split * per_split + per_split < total ? split * per_split + per_split : total);
+        if (hi > lo) {
+          tile_lo = lo < tile_lo ? lo : tile_lo;
+          tile_hi = hi > tile_hi ? hi : tile_hi;
+        }
+        if (wave * CT / 4 == half) {
+          own_lo = lo;
+          own_hi = hi;
+        }
+      }
+      if (tile_hi == 0) tile_lo = 0;
+    }
+  }
 
   int wave_last_pos = -1, wave_first_pos = 0x7fffffff;
 #pragma unroll
@@ -857,7 +892,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
     const int s = 64 * (wave + WAVES * m) + lane;
     const int key = s / CPR, place = s % CPR;
     k_key[m] = key;
-    k_col[m] = 8 * (place ^ ((key & 3) | (((key >> 3) & 1) << 2)));
+    k_col[m] = 8 * (place ^ (SAME_BITS ? key & 7 : (key & 3) | (((key >> 3) & 1) << 2)));
     v_chan[m] = s / 8;
   }
   v_key = 8 * ((lane & 7) ^ ((lane >> 3) & 7));  // (the channel's low bits are the lane's: 64 q is a multiple of 8 channels)
@@ -920,10 +955,17 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
   // block b), piece (4 cb + g) ^ (i & 7) = 4 (cb ^ h) + (g ^ (i & 3)) with h = (i / 4) & 1.  V^T: row i of a channel
   // tile, piece (4 kb + g) ^ (i & 7) likewise.
   const int h = (i >> 2) & 1;
-  const int k_row_bytes = (8 * (i >> 2) + (i & 3)) * (2 * D) + 16 * (g ^ (i & 3));
+  const int k_row_bytes = (SAME_BITS ? i : 8 * (i >> 2) + (i & 3)) * (2 * D) + 16 * (g ^ (i & 3));
   const int k_even = k_row_bytes + 64 * h, k_odd = k_row_bytes + 64 * (1 - h);           // cb even / odd: + 128 (cb / 2)
   const int v_row_bytes = TILE_BYTES + i * 128 + 16 * (g ^ (i & 3));
   const int v_first = v_row_bytes + 64 * h, v_second = v_row_bytes + 64 * (1 - h);       // kb = 0 / 1
+  // SAME_BITS: of row i the keys 32 kb + 16 u + 4 g .. + 3, half a piece: place (4 kb + 2 u + g / 2) ^ (i & 7)
+  int v_half[NKB][2];
+#pragma unroll
+  for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) v_half[kb][u] = TILE_BYTES + i * 128 + 16 * ((4 * kb + 2 * u + (g >> 1)) ^ (i & 7)) + 8 * (g & 1);
+  auto key_in_tile = [&](int t) { return SAME_BITS ? 16 * t + 4 * g : 32 * (t >> 1) + 8 * g + 4 * (t & 1); };  // of a lane's first score of S^T tile t
 
   // (the queries have arrived before the loop, said in a way the compiler sees: it would otherwise wait for them, and with
   // them for every load in flight, at their first use in every round of the loop)
@@ -968,6 +1010,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
     }
     if (!have_tile) continue;
     if (n0 > wave_last_pos) continue;  // nothing this wave may read
+    if (SAME_BITS && (tile < own_lo || tile >= own_hi)) continue;
     const char* const tile_base = smem[buffer];
 
     // ---- S^T = K Q^T: tile t = 2 b + u of the 64 keys ----------------------------------------
@@ -975,7 +1018,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       Operand kf[NQB > 0 ? NQB : 1];  // (the template is parsed for every head size, run for 64, 128 and 256)
-      const int tile_bytes = (32 * (t >> 1) + 4 * (t & 1)) * (2 * D);
+      const int tile_bytes = (SAME_BITS ? 16 * t : 32 * (t >> 1) + 4 * (t & 1)) * (2 * D);
 #pragma unroll
       for (int cb = 0; cb < NQB; ++cb)
         kf[cb] = __builtin_bit_cast(Operand, *reinterpret_cast<const float4_t*>(tile_base + ((cb & 1) ? k_odd : k_even) + 128 * (cb >> 1) + tile_bytes));
@@ -1012,7 +1055,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
           for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              int d = d0 - (32 * (t >> 1) + 8 * g + 4 * (t & 1) + j);
+              int d = d0 - (key_in_tile(t) + j);
               d = d < 0 ? 0 : (d > bias_len - 1 ? bias_len - 1 : d);
               s[ct][t][j] = fmaf(s[ct][t][j], CAPPED ? 1.f : scale_eff, tab[d] * Softmax<T>::SCALE);
             }
@@ -1034,7 +1077,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
         for (int t = 0; t < NT; ++t)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const int n = n0 + 32 * (t >> 1) + 8 * g + 4 * (t & 1) + j;
+            const int n = n0 + key_in_tile(t) + j;
             const bool keep = row_ok[ct] && n < kv_len && n <= pos[ct] && (window <= 0 || n > pos[ct] - window || (KEEPS && n < extras.keep_first));
             s[ct][t][j] = keep ? s[ct][t][j] : -INFINITY;
             mx = fmaxf(mx, s[ct][t][j]);
@@ -1049,8 +1092,8 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
       // formats, and after a row's first tile the rescaling is the exception.
       constexpr float REFERENCE_SLACK = 8.f;
       const float top = mx * scale_used;
-      const bool stays = top - m_i[ct] <= REFERENCE_SLACK;  // (false while the row has seen no key: -inf)
-      const float m_new = stays ? m_i[ct] : top;
+      const bool stays = SAME_BITS ? top <= m_i[ct] && m_i[ct] != -INFINITY : top - m_i[ct] <= REFERENCE_SLACK;  // (false while the row has seen no key: -inf)
+      const float m_new = stays ? m_i[ct] : (SAME_BITS ? fmaxf(m_i[ct], top) : top);
       const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
       alpha[ct] = stays ? 1.f : ((m_i[ct] == -INFINITY) ? 0.f : Softmax<T>::exp_of(m_i[ct] - m_safe));
       float psum = 0.f;
@@ -1076,7 +1119,16 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
     Operand vf[AHEAD + 1][NKB];
     auto read_values = [&](int c, Operand (&into)[NKB]) {
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) into[kb] = __builtin_bit_cast(Operand, *reinterpret_cast<const float4_t*>(tile_base + (kb ? v_second : v_first) + 2048 * c));
+      for (int kb = 0; kb < NKB; ++kb) {
+        if constexpr (SAME_BITS) {
+          typedef float float2_t __attribute__((ext_vector_type(2)));
+          const float2_t lo = *reinterpret_cast<const float2_t*>(tile_base + v_half[kb][0] + 2048 * c);
+          const float2_t hi = *reinterpret_cast<const float2_t*>(tile_base + v_half[kb][1] + 2048 * c);
+          into[kb] = __builtin_bit_cast(Operand, float4_t{lo[0], lo[1], hi[0], hi[1]});
+        } else {
+          into[kb] = __builtin_bit_cast(Operand, *reinterpret_cast<const float4_t*>(tile_base + (kb ? v_second : v_first) + 2048 * c));
+        }
+      }
     };
 #pragma unroll
     for (int a = 0; a < AHEAD; ++a) read_values(a, vf[a]);
@@ -1552,11 +1604,12 @@ static int launch(const void* qkv, int qkv_stride, const void* k_cache, const vo
     return (int)hipGetLastError();
   };
   if (direct_ok && portion_kernel_choice >= 2 && max_q_len * group > 64) return launch_direct(portion_kernel_choice == 3);
-  // 256 channels (a latent and its rotated part, all heads over one KV head): direct loads wherever there are more than 64 rows.
-  // Measured on MI355X (us, the kernels below / direct loads, 32 heads over 1): 300 tokens 24 / 21, 600 tokens 42 / 33, 1,500 tokens
-  // 164 / 70, 4,096 tokens 908 / 355, 64 tokens behind 1,000 keys 62 / 45, 12 single tokens behind 700 keys beside 300 tokens 42 /
-  // 23; 8 over 2: 600 tokens 40 / 29, 4,096 tokens 237 / 151; up to 150 tokens equal.  (With four waves of two row tiles, one wave
-  // per SIMD, 1,500 and 1,000 tokens took 180 instead of 126.)
+  // 256 channels (a latent and its rotated part, all heads over one KV head): direct loads wherever there are more than 64 rows, with
+  // the bits of the kernels below.  Measured on MI355X (us, the kernels below / direct loads, 32 heads over 1): 300 tokens 24 / 24, 600
+  // tokens 42 / 39, 1,500 tokens 163 / 83, 4,096 tokens 906 / 406, 64 tokens behind 1,000 keys 63 / 54, 300 behind 1,000 80 / 68, 12
+  // single tokens behind 700 keys beside 300 tokens 42 / 25; 8 over 2: 600 tokens 40 / 34, 4,096 tokens 234 / 182; up to 150 tokens equal.
+  // (Keys in the order of the smaller heads and references that stay take 13 to 18% less and other bits: 71, 356, 45, 56, 23.  With four
+  // waves of two row tiles, one wave per SIMD, 1,500 and 1,000 tokens took 180 then instead of 126.)
   if (direct_ok && D == 256 && max_q_len * group > 64) return launch_direct();
   if (direct_ok && max_q_len * group > 64) {
     // Measured on MI355X over prompts and portions of 128 to 8,192 tokens behind up to 30,000 keys, with 28 heads over 4,
