@@ -562,3 +562,66 @@ def test_chunks_of_the_recurrences_against_a_loop_in_float64(ops, rule, per_chan
     assert float((got.double() - want).abs().max()) <= bound * float(want.abs().max())
     assert float((mine.double() - after).abs().max()) <= bound * float(after.abs().max())
     assert torch.equal(mine[3], state[3])  # a slot that no sequence holds
+
+
+def scan_case(lengths, rule, per_channel, heads, kv_heads, dim, vdim, v_dtype, seed=1):
+    """What ``linear_scan`` takes for sequences of these lengths, and a function that runs it on some of them from the same states."""
+    generator = torch.Generator(device="cuda").manual_seed(seed)
+    drawn = lambda *shape: torch.randn(*shape, generator=generator, device="cuda")  # noqa: E731
+    tokens = sum(lengths)
+    qk = torch.nn.functional.normalize(drawn(tokens, kv_heads, 2, dim), dim=-1)
+    v = drawn(tokens, heads * vdim + 8).to(v_dtype)
+    decay = torch.exp(-torch.rand(tokens, heads * dim if per_channel else heads, generator=generator, device="cuda"))
+    beta = torch.rand(tokens, heads, generator=generator, device="cuda") if rule == "delta" else None
+    state = drawn(len(lengths), heads, dim, vdim)
+    starts = [sum(lengths[:i]) for i in range(len(lengths))]
+
+    def run(ops, which, **more):
+        rows = torch.cat([torch.arange(starts[i], starts[i] + lengths[i]) for i in which]).cuda()
+        cu = torch.tensor([0] + [lengths[i] for i in which], device="cuda").cumsum(0).int()
+        mine, slots = state.clone(), torch.tensor(which, dtype=torch.int32, device="cuda")
+        out = ops.linear_scan(qk[rows].contiguous(), v[rows].contiguous(), 8, decay[rows].contiguous(), beta[rows].contiguous() if beta is not None else None, mine, slots, cu,
+                              max(lengths[i] for i in which), heads, kv_heads, dim, vdim, rule, **more)
+        return [out[int(cu[j]):int(cu[j + 1])] for j in range(len(which))], [mine[i] for i in which]
+
+    run.state = state
+    return run
+
+
+SCAN_SHAPES = [("delta", True, 4, 2, 128, 128, torch.bfloat16), ("additive", True, 2, 2, 128, 80, torch.float32), ("delta", False, 3, 3, 64, 20, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("rule, per_channel, heads, kv_heads, dim, vdim, v_dtype", SCAN_SHAPES)
+@pytest.mark.parametrize("lengths", [(1, 70, 1, 1), (1, 40, 2, 5, 31, 1, 33, 3), (33, 64), (1,) * 70 + (32, 50)])
+def test_a_sequences_bits_beside_long_portions_are_those_it_has_alone(ops, rule, per_channel, heads, kv_heads, dim, vdim, v_dtype, lengths):
+    """Single tokens, pairs, short portions and long ones each keep the kernel of their own length; so does a long portion whose heads are
+    worked some at a time because the scratch holds no more."""
+    run = scan_case(lengths, rule, per_channel, heads, kv_heads, dim, vdim, v_dtype)
+    everything = list(range(len(lengths)))
+    outs, states = run(ops, everything)
+    for i in everything:
+        (alone,), (after,) = run(ops, [i])
+        assert torch.equal(outs[i], alone) and torch.equal(states[i], after), lengths[i]
+    held = ops.LINEAR_CHUNK_SCRATCH
+    try:
+        ops.LINEAR_CHUNK_SCRATCH = 1
+        sliced, after = run(ops, everything)
+    finally:
+        ops.LINEAR_CHUNK_SCRATCH = held
+    assert all(torch.equal(a, b) for a, b in zip(outs + states, sliced + after))
+
+
+@pytest.mark.parametrize("rule, per_channel, heads, kv_heads, dim, vdim, v_dtype", SCAN_SHAPES)
+@pytest.mark.parametrize("lengths", [(0, 40, 0, 1, 3, 0), (0, 0, 17), (0, 36, 0, 48)])
+def test_empty_sequences_beside_long_portions(ops, rule, per_channel, heads, kv_heads, dim, vdim, v_dtype, lengths):
+    """Empty ones change nothing, and what they hide from the count of tokens is worked all the same.  (Sums of at most 128 terms in
+    different orders: 64 float32 roundings of the largest value, as above.)"""
+    run = scan_case(lengths, rule, per_channel, heads, kv_heads, dim, vdim, v_dtype)
+    outs, states = run(ops, list(range(len(lengths))))
+    for i, n in enumerate(lengths):
+        if n == 0:
+            assert torch.equal(states[i], run.state[i])
+            continue
+        (want,), (after,) = run(ops, [i], chunked=False)
+        bound = 64 * 2.0 ** -24
+        assert float((outs[i] - want).abs().max()) <= bound * float(want.abs().max()) and float((states[i] - after).abs().max()) <= bound * float(after.abs().max())

@@ -16,6 +16,9 @@
 // block's second half and a token j of its first meet as k_t P(m, t) and k_j P(j, m) with m the last token of the first half, so
 // every pair below the diagonal belongs to exactly one level, and a level is one 16 x 16 product over the channels.
 //
+// Sequences of fewer than `long_from` tokens are left to the kernels that go token by token, whatever else is in the step, and a
+// step whose records would not fit the scratch is worked some heads at a time: a sequence's bits depend on its own tokens alone.
+//
 //   linear_chunk_prepare_kernel   a workgroup per chunk and head: a wave per level, then T and the matrices above into `scratch`
 //   linear_chunk_scan_kernel      a workgroup per 16 value columns, head and sequence; a wave holds 16 rows of the state in the
 //                                 matrix instructions' result layout, which is also their operand layout; the waves exchange
@@ -42,6 +45,8 @@ struct LinearChunkArgs {
   const int* cu_q;
   float* out;          // [T, heads * vdim]
   int heads, kv_heads, dim, vdim;
+  int num_seqs, long_from;      // sequences of at least long_from tokens are worked
+  int first_head, head_count;   // the heads that this launch works; their records lie side by side in `scratch`
 };
 
 // A chunk and head in `scratch`, in floats: -U' | R' | K' (each 16 * dim), P_16 (dim), Dv | Ov (each 16 * columns).  U' and R' as
@@ -55,16 +60,34 @@ __device__ __forceinline__ int first_chunk(int first_token, int sequence) { retu
 __device__ __forceinline__ float4_t mfma4(float a, float b, float4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ float4_t four(const float* p) { return *reinterpret_cast<const float4_t*>(p); }
 
+// The last sequence whose first record is not behind `record` (-1: none), the same in every lane.
+__device__ __forceinline__ int sequence_of(int record, const int* cu_q, int num_seqs, int lane) {
+  int before = 0;
+  for (int s0 = 0; s0 < num_seqs; s0 += 64) {
+    const int s = s0 + lane;
+    const int found = __popcll(__ballot(s < num_seqs && first_chunk(cu_q[s], s) <= record));  // (first records rise from sequence to sequence)
+    before += found;
+    if (found < 64) break;
+  }
+  return __builtin_amdgcn_readfirstlane(before) - 1;
+}
+
+// The grid counts records, of which there are about as many as chunks: one per longest portion's chunk and sequence would be a hundred
+// thousand workgroups that only end, for 60 single tokens beside 1,000.  Measured on MI355X (us a step with the kernels for the short ones
+// behind it; token by token / everything in chunks with such a grid / this): 60 single tokens beside 1,000, 16 heads of 128 x 128 519 / 195 /
+// 149, 32 heads 677 / 359 / 238; beside 64 131 / 141 / 87, 240 / 239 / 147; 12 beside 300 142 / 62 / 56; 1 beside 300 92 / 35 / 41.
 template <bool DELTA>
 __global__ void __launch_bounds__(256) linear_chunk_prepare_kernel(const LinearChunkArgs a) {
   extern __shared__ float4_t lds_pieces[];
   float* lds = reinterpret_cast<float*>(lds_pieces);
-  const int h = blockIdx.x, b = blockIdx.z;
-  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  const int t0 = lo + blockIdx.y * CHUNK;
-  if (t0 >= hi) return;  // (the whole workgroup)
-  const int count = hi - t0 < CHUNK ? hi - t0 : CHUNK;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int record_at = blockIdx.x / a.head_count, local_head = blockIdx.x % a.head_count, h = a.first_head + local_head;
+  const int b = sequence_of(record_at, a.cu_q, a.num_seqs, lane);
+  if (b < 0) return;  // (the whole workgroup)
+  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
+  const int t0 = lo + (record_at - first_chunk(lo, b)) * CHUNK;
+  if (t0 >= hi || hi - lo < a.long_from) return;  // (the whole workgroup)
+  const int count = hi - t0 < CHUNK ? hi - t0 : CHUNK;
   const int n = lane & 15, g = lane >> 4;  // column and group of four rows in the matrix instructions' layouts
   const int dim = a.dim, row = dim + 4;
   // rows of q, k and the decays (16 x dim each), and 16 x 16 matrices: M1, M3, T, M3 T
@@ -139,8 +162,7 @@ __global__ void __launch_bounds__(256) linear_chunk_prepare_kernel(const LinearC
   }
   // the running products: a lane walks one channel forwards (k P and q P, in place behind the barrier) or backwards (K')
   __syncthreads();
-  const int record_at = first_chunk(lo, b) + blockIdx.y;
-  float* record = a.scratch + ((size_t)record_at * a.heads + h) * chunk_record(dim, a.vdim);
+  float* record = a.scratch + ((size_t)record_at * a.head_count + local_head) * chunk_record(dim, a.vdim);
   float* record_k = record + 32 * dim;
   float* record_p = record + 48 * dim;
   for (int c = tid; c < dim; c += 256) {
@@ -248,9 +270,9 @@ __global__ void __launch_bounds__(64 * WAVES, 2) linear_chunk_scan_kernel(const 
   __shared__ float4_t parts[2][2][WAVES][64];  // [buffer][D, O][wave][lane]
   // (heads lie along the grid's first dimension in both kernels: with a multiple of 8 heads the workgroups that read a record run
   // on the XCD that wrote it and share it in that XCD's L2)
-  const int h = blockIdx.x, tile = blockIdx.y, b = blockIdx.z;
+  const int h = a.first_head + blockIdx.x, tile = blockIdx.y, b = blockIdx.z;
   const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  if (hi <= lo) return;  // (the whole workgroup)
+  if (hi - lo < a.long_from || hi <= lo) return;  // (the whole workgroup)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = lane & 15, g = lane >> 4;
   constexpr int dim = 16 * WAVES;
@@ -259,13 +281,13 @@ __global__ void __launch_bounds__(64 * WAVES, 2) linear_chunk_scan_kernel(const 
   const int column = tile * 16 + n;
   const bool live = column < vdim;
   const int chunks = (hi - lo + CHUNK - 1) / CHUNK;
-  const size_t stride = (size_t)a.heads * chunk_record(dim, vdim);  // between a sequence's records of this head
+  const size_t stride = (size_t)a.head_count * chunk_record(dim, vdim);  // between a sequence's records of this head
   // a lane's places in a record, in floats (the record's own address is the same for the whole wave and moves from chunk to chunk)
   const uint32_t rows_at = wave * 256 + n * 16 + 4 * g, decays_at = 48 * dim + wave * 16 + 4 * g, column_at = 49 * dim + column * CHUNK + 4 * g;
   // the read-out that a lane finishes, by its place in the order in which the parts lie in LDS
   const int out_t = ((tid >> 6) & 3) * 4 + (tid & 3), out_e = (tid >> 2) & 15;
   const uint32_t read_at = 49 * dim + (columns + tile * 16 + out_e) * CHUNK + out_t;
-  const float* next = a.scratch + ((size_t)first_chunk(lo, b) * a.heads + h) * chunk_record(dim, vdim);
+  const float* next = a.scratch + ((size_t)first_chunk(lo, b) * a.head_count + blockIdx.x) * chunk_record(dim, vdim);
   int asked = 0;  // chunks asked for so far
   auto load = [&](ChunkOperands<WAVES>& o) {
     const float* record = next;
@@ -344,34 +366,41 @@ __global__ void __launch_bounds__(64 * WAVES, 2) linear_chunk_scan_kernel(const 
   }
 }
 
-// float32 elements of the scratch of a step; 0: these sizes are not for these kernels.  Key heads of 64 and 128 channels: the sizes
-// whose long portions ran a column of the state per wave, in an order of sums of their own.  (Other sizes are worked in one
+static int records_of_step(int tokens, int num_seqs) { return tokens / CHUNK + num_seqs + 1; }
+
+// float32 elements of scratch that a head takes in a step; 0: these sizes are not for these kernels.  Key heads of 64 and 128 channels:
+// the sizes whose long portions ran a column of the state per wave, in an order of sums of their own.  (Other sizes are worked in one
 // order whether a portion is long or short, and larger ones would need more than a workgroup's waves for a column tile.)
-extern "C" long long velox_linear_chunk_scratch_elems(int tokens, int num_seqs, int heads, int dim, int vdim) {
+extern "C" long long velox_linear_chunk_scratch_elems(int tokens, int num_seqs, int dim, int vdim) {
   if ((dim != 64 && dim != 128) || vdim < 1) return 0;
-  return ((long long)tokens / CHUNK + num_seqs + 1) * heads * (long long)chunk_record(dim, vdim);
+  return (long long)records_of_step(tokens, num_seqs) * (long long)chunk_record(dim, vdim);
 }
 
 template <bool DELTA>
-static void linear_chunk_launch(const LinearChunkArgs& a, int num_seqs, int max_q_len, hipStream_t stream) {
+static void linear_chunk_launch(const LinearChunkArgs& a, int tokens, hipStream_t stream) {
   const size_t lds = (size_t)CHUNK * (3 * (a.dim + 4) + 4 * CHUNK_STRIDE) * sizeof(float);
-  linear_chunk_prepare_kernel<DELTA><<<dim3(a.heads, (max_q_len + CHUNK - 1) / CHUNK, num_seqs), 256, lds, stream>>>(a);
-  const dim3 grid(a.heads, chunk_columns(a.vdim) / 16, num_seqs);
+  linear_chunk_prepare_kernel<DELTA><<<(unsigned)records_of_step(tokens, a.num_seqs) * (unsigned)a.head_count, 256, lds, stream>>>(a);
+  const dim3 grid(a.head_count, chunk_columns(a.vdim) / 16, a.num_seqs);
   if (a.dim == 64) linear_chunk_scan_kernel<4, DELTA><<<grid, 256, 0, stream>>>(a);
   else linear_chunk_scan_kernel<8, DELTA><<<grid, 512, 0, stream>>>(a);
 }
 
-// beta: nullptr for the additive rule.  qk and a decay per channel are read in 16-byte pieces (dim is a multiple of 16; the caller
-// checks that the bases are aligned).
+// The sequences of at least `long_from` tokens.  beta: nullptr for the additive rule.  `scratch` holds the records of `heads_at_once`
+// heads (velox_linear_chunk_scratch_elems each), which are worked one such group after the other.  qk and a decay per channel are
+// read in 16-byte pieces (dim is a multiple of 16; the caller checks that the bases are aligned).
 extern "C" int velox_linear_chunk_scan(const float* qk, const void* v, int v_dtype, int v_ld, int v_at, const float* decay, int decay_per_channel,
                                        const float* beta, float* scratch, float* state, const int* slots, const int* cu_q, float* out, int num_seqs,
-                                       int max_q_len, int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
-  if (num_seqs <= 0 || max_q_len <= 0) return 0;
-  if (velox_linear_chunk_scratch_elems(max_q_len, num_seqs, heads, dim, vdim) == 0 || heads < 1 || heads > 65535 || num_seqs > 65535 ||
-      max_q_len > 65535 * CHUNK || vdim > 65535 * 16 || kv_heads < 1 || heads % kv_heads != 0 || !scratch)
+                                       int tokens, int long_from, int heads_at_once, int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
+  if (num_seqs <= 0 || tokens <= 0) return 0;
+  if (velox_linear_chunk_scratch_elems(tokens, num_seqs, dim, vdim) == 0 || heads < 1 || heads > 65535 || num_seqs > 65535 || heads_at_once < 1 ||
+      (long long)records_of_step(tokens, num_seqs) * (heads_at_once < heads ? heads_at_once : heads) > (1 << 23) || vdim > 65535 * 16 || kv_heads < 1 ||
+      heads % kv_heads != 0 || !scratch)
     return (int)hipErrorInvalidValue;
-  LinearChunkArgs a{qk, v, v_dtype == VELOX_BF16, v_ld, v_at, decay, decay_per_channel, beta, scratch, state, slots, cu_q, out, heads, kv_heads, dim, vdim};
-  if (beta) linear_chunk_launch<true>(a, num_seqs, max_q_len, stream);
-  else linear_chunk_launch<false>(a, num_seqs, max_q_len, stream);
+  for (int first = 0; first < heads; first += heads_at_once) {
+    LinearChunkArgs a{qk, v, v_dtype == VELOX_BF16, v_ld, v_at, decay, decay_per_channel, beta, scratch, state, slots, cu_q, out, heads, kv_heads, dim, vdim,
+                      num_seqs, long_from, first, heads - first < heads_at_once ? heads - first : heads_at_once};
+    if (beta) linear_chunk_launch<true>(a, tokens, stream);
+    else linear_chunk_launch<false>(a, tokens, stream);
+  }
   VELOX_RETURN_LAUNCH_STATUS();
 }

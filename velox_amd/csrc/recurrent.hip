@@ -8,8 +8,10 @@
 //   linear_scan         the recurrence itself, token by token from the state slot (portions of prompts staged through LDS; long ones of
 //                       the first two rules with key heads of 64 or 128 channels go in chunks, linear_chunk.hip)
 //   gated_head_norm     RMS norm of each head's read-out, a shared weight, a gate
-// Everything between a load and a store is float32; stores round once.  No result depends on how a sequence's tokens
-// were cut into steps or on what else is in the batch: sums run in an order that only the sizes fix.
+// Everything between a load and a store is float32; stores round once.  Sums run in an order that only the sizes fix, except that
+// linear_scan's depends on how many tokens a sequence has in the step (one order for single tokens and pairs, with key heads of 64,
+// 128, 256 and 512 channels another for longer portions, with 64 and 128 a third from 32 tokens on, where chunks start at the
+// portion's first token) and, beside portions of 3 to 31 tokens, that of single tokens is the portions'.  The orders differ by roundings.
 #include <type_traits>
 
 #include "common.h"
@@ -887,7 +889,8 @@ extern "C" int velox_removal_prepare(const void* main, int dtype, int ld, int r_
 //                              LDS, and writes the registers to the other LDS buffer behind it: one barrier per block, the
 //                              loads' latency lies behind a block's arithmetic.
 //   linear_scan_wave_kernel    the same for dim = 64, 128, 256, 512, a column per wave (described at the kernel).  Portions of 32 tokens and
-//                              more of dim = 64 and 128 come here only with the removal rule or where the chunks' scratch would be too large.
+//                              more of dim = 64 and 128 come here only with the removal rule; the shorter ones beside them do, single
+//                              tokens and pairs of tokens beside them go to linear_scan_kernel.
 // The first two give the same bits: they differ in where the operands wait, not in what is done with them; the third sums in
 // another order (which, like theirs, only the sizes fix).
 // ---------------------------------------------------------------------------------------------
@@ -923,6 +926,7 @@ struct ScanArgs {
   const int* cu_q;
   float* out;            // [T, heads * vdim]
   int heads, kv_heads, dim, vdim, delta;
+  int from_tokens, below_tokens;  // sequences of at least from_tokens (1 or more) and fewer than below_tokens tokens are worked
 };
 
 __device__ __forceinline__ void scan_load_rows(const float* __restrict__ p, int d0, int dim, bool vec, float fill, float (&r)[SCAN_ROWS]) {
@@ -981,7 +985,7 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(const ScanArgs a) {
   const int e = blockIdx.x * (256 / R) + threadIdx.x / R;
   const int h = blockIdx.y, b = blockIdx.z;
   const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  if (hi <= lo) return;
+  if (hi - lo < a.from_tokens || hi - lo >= a.below_tokens) return;
   const bool live = e < a.vdim;
   const int col = live ? e : a.vdim - 1;  // (lanes beyond the last column follow it and write nothing: the shuffles need every lane)
   const int dim = a.dim, vdim = a.vdim;
@@ -1041,7 +1045,7 @@ __global__ void __launch_bounds__(256) linear_scan_staged_kernel(const ScanArgs 
   const int e = blockIdx.x * COLS + c_local;
   const int h = blockIdx.y, b = blockIdx.z;
   const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  if (hi <= lo) return;  // (the whole workgroup: no barrier is left waiting)
+  if (hi - lo < a.from_tokens || hi - lo >= a.below_tokens) return;  // (the whole workgroup: no barrier is left waiting)
   const bool live = e < a.vdim;
   const int col = live ? e : a.vdim - 1;
   const int dim = a.dim, vdim = a.vdim, heads = a.heads;
@@ -1240,7 +1244,7 @@ __global__ void __launch_bounds__(512) linear_scan_wave_kernel(const ScanArgs a,
   const int e = blockIdx.x * WAVE_COLS + wave;
   const int h = blockIdx.y, b = blockIdx.z;
   const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  if (hi <= lo) return;  // (the whole workgroup)
+  if (hi - lo < a.from_tokens || hi - lo >= a.below_tokens) return;  // (the whole workgroup)
   const bool live = e < a.vdim;
   const int col = live ? e : a.vdim - 1;
   const int dim = 64 * RW, vdim = a.vdim, heads = a.heads;
@@ -1441,15 +1445,17 @@ static void linear_scan_launch(const ScanArgs& a, int lanes, int num_seqs, int m
   }
 }
 
-// rule 0: additive, 1: delta, 2: removal (three vectors per token, a decay per channel; beta holds the keys' lengths)
+// rule 0: additive, 1: delta, 2: removal (three vectors per token, a decay per channel; beta holds the keys' lengths).  Sequences of
+// fewer than from_tokens or of below_tokens tokens and more are left alone; max_q_len chooses the kernel for the others.
 extern "C" int velox_linear_scan(const float* qk, const void* v, int v_dtype, int v_ld, int v_at, const float* decay, int decay_per_channel, const float* beta,
                                  float* state, const int* slots, const int* cu_q, float* out, int num_seqs, int max_q_len, int heads, int kv_heads, int dim,
-                                 int vdim, int rule, hipStream_t stream) {
+                                 int vdim, int rule, int from_tokens, int below_tokens, hipStream_t stream) {
   if (num_seqs <= 0) return 0;
   const int lanes = velox_linear_scan_lanes(dim);
   if (lanes > 64 || heads > 65535 || num_seqs > 65535 || kv_heads < 1 || heads % kv_heads != 0 || rule < 0 || rule > 2 || (rule != 0 && !beta))
     return (int)hipErrorInvalidValue;
-  ScanArgs a{qk, v, v_dtype == VELOX_BF16, v_ld, v_at, decay, decay_per_channel, beta, state, slots, cu_q, out, heads, kv_heads, dim, vdim, rule == 1};
+  ScanArgs a{qk, v, v_dtype == VELOX_BF16, v_ld, v_at, decay, decay_per_channel, beta, state, slots, cu_q, out, heads, kv_heads, dim, vdim, rule == 1,
+             from_tokens < 1 ? 1 : from_tokens, below_tokens};
   if (rule == 2) linear_scan_launch<true>(a, lanes, num_seqs, max_q_len, stream);
   else linear_scan_launch<false>(a, lanes, num_seqs, max_q_len, stream);
   VELOX_RETURN_LAUNCH_STATUS();

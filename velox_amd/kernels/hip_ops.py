@@ -177,7 +177,7 @@ class HipOps:
             fn.restype = _I
         c.velox_rotate_pad_write.argtypes = [_P, _I, _P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P]
         c.velox_recurrence_prepare.argtypes = [_P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _I, _I, _I, _I, _I, _P, _P, _F, _P, _I, _I, _I, _P, _P, _P, _I, _P]
-        c.velox_linear_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]
+        c.velox_linear_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         c.velox_linear_scan_lanes.argtypes = [_I]
         c.velox_gated_head_norm.argtypes = [_P, _P, _F, _P, _I, _I, _I, _I, _P, _I, _I, _I, _I, _I, _P]
         c.velox_removal_prepare.argtypes = [_P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _I, _P]
@@ -190,9 +190,9 @@ class HipOps:
         c.velox_removal_chunk_scan.restype = _I
         c.velox_gemm_tiles_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P]
         c.velox_gemm_tiles_bf16.restype = _I
-        c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]
+        c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         c.velox_linear_chunk_scan.restype = _I
-        c.velox_linear_chunk_scratch_elems.argtypes = [_I, _I, _I, _I, _I]
+        c.velox_linear_chunk_scratch_elems.argtypes = [_I, _I, _I, _I]
         c.velox_linear_chunk_scratch_elems.restype = ctypes.c_longlong
         c.velox_removal_chunk_scratch_elems.argtypes = [_I, _I, _I, _I, _I, _I]
         c.velox_removal_chunk_scratch_elems.restype = ctypes.c_longlong
@@ -1317,16 +1317,20 @@ class HipOps:
 
     _SCAN_RULES = {"additive": 0, "delta": 1, "removal": 2}
 
-    LINEAR_CHUNK_TOKENS = 32  # portions at least this long go through the chunked kernels where the sizes are theirs
-    LINEAR_CHUNK_SCRATCH = 1 << 28  # the most float32 numbers of scratch they may ask for (1 GB: 13,000 tokens of 32 heads of 128 x 128)
+    # Portions at least this long go through the chunked kernels where the sizes are theirs.  Measured on MI355X (us, token by token /
+    # chunks; heads of 128 x 128 and, additive, 128 x 256): one portion of 16 tokens, 16 heads 9.9 / 15.5, 32 heads 14.0 / 15.8, additive,
+    # 8 heads 9.2 / 15.1; of 32 tokens 14.8 / 16.2, 20.1 / 16.6, 12.8 / 15.5; of 48 tokens 19.4 / 16.9, 25.6 / 17.5, 16.5 / 15.9.  (Four
+    # portions meet at about 10 tokens: 21.3 / 19.3, 32.8 / 26.3, 20.2 / 18.0 at 12.)
+    LINEAR_CHUNK_TOKENS = 32
+    LINEAR_CHUNK_SCRATCH = 1 << 28  # the most float32 numbers of scratch they ask for, if one head's fit (1 GB: 13,000 tokens of 32 heads of 128 x 128 at once)
 
     def linear_scan(self, qk, v_source, v_at, decay, beta, state, slots, cu_q, max_q_len, heads, kv_heads, dim, vdim, rule, chunked: Optional[bool] = None):
         """Per sequence and head, token by token from ``state[slot, head]`` ([dim, vdim] float32), which is written back:
         ``S <- g S`` (rows); ``u = beta (v - S^T k)`` (rule ``"delta"``) or ``u = v`` (``"additive"``); ``S <- S + k u^T``; ``o = S^T q``.
         Rule ``"removal"``: ``qk`` holds a third vector ``b`` per head and token, and ``S <- g S - b (k^T S) + k (beta v)^T`` with both
-        terms on the old state.  ``decay`` is [T, heads] or [T, heads * dim].  Returns float32 [T, heads * vdim].  Steps of the first two
-        rules with a long portion are worked in chunks of 16 tokens on the matrix cores (key heads of 64 or 128 channels), all others
-        token by token; ``chunked`` decides it for a test."""
+        terms on the old state.  ``decay`` is [T, heads] or [T, heads * dim].  Returns float32 [T, heads * vdim].  Long portions of the
+        first two rules are worked in chunks of 16 tokens on the matrix cores (key heads of 64 or 128 channels), all others, also beside
+        them, token by token; ``chunked`` decides it for a test, for all sequences."""
         if rule not in self._SCAN_RULES:
             raise KernelError(f"linear_scan: rule {rule!r} is not implemented ({', '.join(self._SCAN_RULES)})")
         delta = rule != "additive"
@@ -1350,22 +1354,37 @@ class HipOps:
         self._check("cu_q", cu_q, torch.int32, (slots.shape[0] + 1,))
         self.linear_scan_supports(dim, vdim)
         out = torch.empty((tokens, heads * vdim), dtype=torch.float32, device=self.device)
-        scratch_elems = 0
-        if rule != "removal" and chunked is not False and max_q_len >= (1 if chunked else self.LINEAR_CHUNK_TOKENS):
-            scratch_elems = int(self._core.velox_linear_chunk_scratch_elems(tokens, slots.shape[0], int(heads), int(dim), int(vdim)))
-            scratch_elems = scratch_elems if scratch_elems <= self.LINEAR_CHUNK_SCRATCH else 0
-        if chunked and scratch_elems == 0:
-            raise KernelError(f"linear_scan: heads of {dim} channels (rule {rule!r}, {tokens} tokens) are not the chunked kernels'")
-        if scratch_elems:
-            scratch = torch.empty(scratch_elems, dtype=torch.float32, device=self.device)
-            self._launched(self._core.velox_linear_chunk_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
-                                                              _ptr(beta) if delta else _P(0), _ptr(scratch), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out),
-                                                              slots.shape[0], int(max_q_len), int(heads), int(kv_heads), int(dim), int(vdim), self._stream()), "linear_chunk_scan")
+        sequences = slots.shape[0]
+
+        def token_by_token(longest, from_tokens=1, below_tokens=1 << 30):
+            status = self._core.velox_linear_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
+                                                  _ptr(beta) if delta else _P(0), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out), sequences, int(longest), int(heads),
+                                                  int(kv_heads), int(dim), int(vdim), self._SCAN_RULES[rule], from_tokens, below_tokens, self._stream())
+            self._launched(status, "linear_scan")
+
+        long_from = 1 if chunked else self.LINEAR_CHUNK_TOKENS
+        per_head = 0
+        if rule != "removal" and chunked is not False and max_q_len >= long_from:
+            per_head = int(self._core.velox_linear_chunk_scratch_elems(tokens, sequences, int(dim), int(vdim)))
+        if per_head == 0:
+            if chunked:
+                raise KernelError(f"linear_scan: heads of {dim} channels (rule {rule!r}) are not the chunked kernels'")
+            token_by_token(max_q_len)
             return out
-        status = self._core.velox_linear_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
-                                              _ptr(beta) if delta else _P(0), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out), slots.shape[0], int(max_q_len), int(heads),
-                                              int(kv_heads), int(dim), int(vdim), self._SCAN_RULES[rule], self._stream())
-        self._launched(status, "linear_scan")
+        heads_at_once = max(1, min(int(heads), self.LINEAR_CHUNK_SCRATCH // per_head))
+        scratch = torch.empty(per_head * heads_at_once, dtype=torch.float32, device=self.device)
+        self._launched(self._core.velox_linear_chunk_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
+                                                          _ptr(beta) if delta else _P(0), _ptr(scratch), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out),
+                                                          sequences, tokens, long_from, heads_at_once, int(heads), int(kv_heads), int(dim), int(vdim), self._stream()),
+                       "linear_chunk_scan")
+        if long_from > 1 and tokens != sequences * max_q_len:  # (some sequence is shorter than the longest)
+            # What is beside the long portions: single tokens and pairs, and longer ones if the number of tokens leaves room for one.  (If
+            # it leaves none, no sequence lies between, or empty ones make up for it and this kernel takes all.)
+            if tokens - max_q_len == sequences - 1:
+                token_by_token(1, below_tokens=long_from)
+            else:
+                token_by_token(1, below_tokens=3)
+                token_by_token(3, from_tokens=3, below_tokens=long_from)
         return out
 
     def gated_head_norm(self, read, weight, eps, gate_source, gate_at, gate_kind, heads, vdim, out_dtype):
