@@ -564,8 +564,9 @@ def test_chunks_of_the_recurrences_against_a_loop_in_float64(ops, rule, per_chan
     assert torch.equal(mine[3], state[3])  # a slot that no sequence holds
 
 
-def scan_case(lengths, rule, per_channel, heads, kv_heads, dim, vdim, v_dtype, seed=1):
-    """What ``linear_scan`` takes for sequences of these lengths, and a function that runs it on some of them from the same states."""
+def scan_case(lengths, rule, per_channel, heads, kv_heads, dim, vdim, v_dtype, seed=1, change=None):
+    """What ``linear_scan`` takes for sequences of these lengths, and a function that runs it on some of them from the same states.
+    ``change(qk, v, decay, beta)`` may alter the inputs first."""
     generator = torch.Generator(device="cuda").manual_seed(seed)
     drawn = lambda *shape: torch.randn(*shape, generator=generator, device="cuda")  # noqa: E731
     tokens = sum(lengths)
@@ -574,6 +575,8 @@ def scan_case(lengths, rule, per_channel, heads, kv_heads, dim, vdim, v_dtype, s
     decay = torch.exp(-torch.rand(tokens, heads * dim if per_channel else heads, generator=generator, device="cuda"))
     beta = torch.rand(tokens, heads, generator=generator, device="cuda") if rule == "delta" else None
     state = drawn(len(lengths), heads, dim, vdim)
+    if change is not None:
+        change(qk, v, decay, beta)
     starts = [sum(lengths[:i]) for i in range(len(lengths))]
 
     def run(ops, which, **more):
@@ -625,3 +628,31 @@ def test_empty_sequences_beside_long_portions(ops, rule, per_channel, heads, kv_
         (want,), (after,) = run(ops, [i], chunked=False)
         bound = 64 * 2.0 ** -24
         assert float((outs[i] - want).abs().max()) <= bound * float(want.abs().max()) and float((states[i] - after).abs().max()) <= bound * float(after.abs().max())
+
+
+@pytest.mark.parametrize("rule, per_channel, heads, kv_heads, dim, vdim, v_dtype", SCAN_SHAPES)
+@pytest.mark.parametrize("what, token", [("value", 9), ("value", 31), ("key", 1), ("query", 12), ("decay", 20), ("beta", 5), ("beta", 15)])
+@pytest.mark.parametrize("number", [float("inf"), float("nan")])
+def test_a_number_that_is_not_finite_reaches_its_own_token_and_later_ones_only(ops, rule, per_channel, heads, kv_heads, dim, vdim, v_dtype, what, token, number):
+    """The tokens before it in its chunk keep their read-outs (up to the order of sums: 64 roundings, as above), and behind it just what
+    token by token is not finite either is not: a value's column, the read-outs of a query, everything for the others."""
+    if what == "beta" and rule != "delta":
+        pytest.skip("the additive rule has no update gate")
+    shape = ((37,), rule, per_channel, heads, kv_heads, dim, vdim, v_dtype)
+
+    def change(qk, v, decay, beta):
+        if what == "value":
+            v[token, 8 + vdim // 2] = number
+        elif what in ("key", "query"):
+            qk[token, 0, 0 if what == "query" else 1, dim // 3] = number
+        elif what == "decay":
+            decay[token, 1] = number
+        else:
+            beta[token, heads - 1] = number
+
+    (got,), (state,) = scan_case(*shape, change=change)(ops, [0])
+    (want,), (after,) = scan_case(*shape, change=change)(ops, [0], chunked=False)
+    (clean,), _ = scan_case(*shape)(ops, [0])
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want)) and torch.equal(torch.isfinite(state), torch.isfinite(after))
+    assert float((got[:token] - clean[:token]).abs().max()) <= 64 * 2.0 ** -24 * float(clean.abs().max())
+    assert not torch.isfinite(want).all()

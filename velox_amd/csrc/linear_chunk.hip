@@ -15,6 +15,8 @@
 // built from products of rows whose factors are at most 1: at the level of blocks of 2 h tokens (h = 8, 4, 2, 1) a token t of a
 // block's second half and a token j of its first meet as k_t P(m, t) and k_j P(j, m) with m the last token of the first half, so
 // every pair below the diagonal belongs to exactly one level, and a level is one 16 x 16 product over the channels.
+// What T, M3 and M3 T have above the diagonal is zero, but zero times an infinity or a NaN of a later token is not: a tile that
+// holds one is multiplied without those terms (lower_times), so that such a value reaches its own token and later ones only.
 //
 // Sequences of fewer than `long_from` tokens are left to the kernels that go token by token, whatever else is in the step, and a
 // step whose records would not fit the scratch is worked some heads at a time: a sequence's bits depend on its own tokens alone.
@@ -59,6 +61,25 @@ __device__ __forceinline__ int first_chunk(int first_token, int sequence) { retu
 
 __device__ __forceinline__ float4_t mfma4(float a, float b, float4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ float4_t four(const float* p) { return *reinterpret_cast<const float4_t*>(p); }
+
+// acc + L y for a lower triangular L (16 x 16, in LDS; `l`: row n's entries 4 g .. + 3) and a tile y of which lane (n, g) holds rows
+// 4 g .. + 3 of column n; the result in the same layout.  The same for the whole wave.
+__device__ __forceinline__ float4_t lower_times(const float4_t l, const float* L, const float4_t y, float4_t acc, int n, int g) {
+  const float zero = y[0] * 0.f + y[1] * 0.f + y[2] * 0.f + y[3] * 0.f;
+  if (__ballot(!(zero == 0.f)) == 0ull) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = mfma4(l[e], y[e], acc);
+    return acc;
+  }
+#pragma unroll
+  for (int j = 0; j < CHUNK; ++j) {
+    const float yj = __shfl(y[j & 3], n + 16 * (j >> 2), VELOX_WAVE);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (j <= 4 * g + i) acc[i] += L[(4 * g + i) * CHUNK_STRIDE + j] * yj;
+  }
+  return acc;
+}
 
 // The last sequence whose first record is not behind `record` (-1: none), the same in every lane.
 __device__ __forceinline__ int sequence_of(int record, const int* cu_q, int num_seqs, int lane) {
@@ -197,15 +218,15 @@ __global__ void __launch_bounds__(256) linear_chunk_prepare_kernel(const LinearC
     }
     if (g == 0) {
 #pragma unroll
-      for (int t = 0; t < CHUNK; ++t) T[t * CHUNK_STRIDE + n] = x[t] * own;
+      for (int t = 0; t < CHUNK; ++t) T[t * CHUNK_STRIDE + n] = t < n ? 0.f : x[t] * own;
     }
   }
   __syncthreads();
   if (DELTA && wave == 0) {  // M3 T
-    const float4_t x = four(M3 + n * CHUNK_STRIDE + 4 * g);
-    float4_t m = {0.f, 0.f, 0.f, 0.f};
+    float4_t t4;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) m = mfma4(x[e], T[(4 * g + e) * CHUNK_STRIDE + n], m);
+    for (int e = 0; e < 4; ++e) t4[e] = T[(4 * g + e) * CHUNK_STRIDE + n];
+    const float4_t m = lower_times(four(M3 + n * CHUNK_STRIDE + 4 * g), M3, t4, float4_t{0.f, 0.f, 0.f, 0.f}, n, g);
 #pragma unroll
     for (int i = 0; i < 4; ++i) M3T[(4 * g + i) * CHUNK_STRIDE + n] = m[i];
   }
@@ -216,12 +237,11 @@ __global__ void __launch_bounds__(256) linear_chunk_prepare_kernel(const LinearC
 #pragma unroll
     for (int i = 0; i < 4; ++i) rp[i] = q[(4 * g + i) * row + tile * 16 + n];
     if (DELTA) {
+      float4_t minus_k;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float y = k[(4 * g + e) * row + tile * 16 + n];
-        up = mfma4(-t4[e], y, up);
-        rp = mfma4(-m3t[e], y, rp);
-      }
+      for (int e = 0; e < 4; ++e) minus_k[e] = -k[(4 * g + e) * row + tile * 16 + n];
+      up = lower_times(t4, T, minus_k, up, n, g);
+      rp = lower_times(m3t, M3T, minus_k, rp, n, g);
     }
     float* to = record + tile * 256 + n;
 #pragma unroll
@@ -243,14 +263,8 @@ __global__ void __launch_bounds__(256) linear_chunk_prepare_kernel(const LinearC
       const float x = a.v_bf16 ? to_f32(((const bf16_t*)a.v)[token]) : ((const float*)a.v)[token];
       v[e] = 4 * g + e < count ? x : 0.f;
     }
-    if (DELTA) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dv = mfma4(t4[e], v[e], dv);
-    } else {
-      dv = v;
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ov = mfma4(m3[e], dv[e], ov);
+    dv = DELTA ? lower_times(t4, T, v, dv, n, g) : v;
+    ov = lower_times(m3, M3, dv, ov, n, g);
     *reinterpret_cast<float4_t*>(record_d + (size_t)column * CHUNK + 4 * g) = dv;
     *reinterpret_cast<float4_t*>(record_d + (size_t)(columns + column) * CHUNK + 4 * g) = ov;
   }
