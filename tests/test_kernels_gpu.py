@@ -1351,3 +1351,47 @@ def test_products_in_tiles_with_a_cut_sum(ops, m, n, k, splits):
     assert torch.all((whole.double() - want).abs() <= k * 2.0 ** -24 * size + 2.0 ** -8 * 1.01 * want.abs() + 1e-6)
     parts = ops.gemm_tiles(a, w, splits, torch.float32)
     assert parts.shape == (splits, m, n) and torch.all((parts.double().sum(0) - want).abs() <= k * 2.0 ** -24 * size + 1e-6)
+
+
+@pytest.mark.parametrize("m, n, k, parts", [(65, 2560, 8192, 8), (300, 2048, 8448, 8), (700, 1024, 28672, 8), (300, 4096, 16512, 5), (129, 8192, 16384, 4)])
+def test_linear_with_parts_of_a_long_sum_into_every_consumer(ops, ref, m, n, k, parts):
+    """More than 64 rows of a long product come back as partial sums.  Each kernel that takes them gives what it gives for their float32
+    sum (a handful of float32 additions in another order), which is the product within its own float32 sums' rounding."""
+    from velox_amd.parts.norms import StreamNorm
+
+    generator = torch.Generator(device="cuda").manual_seed(m)
+    x, w = torch.randn(m, k, generator=generator, device="cuda").bfloat16(), (k ** -0.5 * torch.randn(n, k, generator=generator, device="cuda")).bfloat16()
+    assert ops.tile_splits(m, n, k) == parts
+    got = ops.linear(x, w, None, torch.bfloat16, partials_ok=True)
+    assert got.shape == (parts, m, n) and got.dtype == torch.float32
+    assert ops.linear(x, w, None, torch.bfloat16).shape == (m, n)  # (who cannot take parts gets none)
+    whole = got.double().sum(0).float()
+    for rows in (slice(0, 17), slice(m - 17, m)):
+        want = x[rows].double() @ w.double().T
+        assert float((whole[rows].double() - want).abs().max()) <= k * 2.0 ** -24 * float((x[rows].double().abs() @ w.double().abs().T).max())
+    residual, weight = rand((m, n), torch.float32, 5), 1 + rand((n,), torch.float32, 6, 0.02)
+    rows = torch.tensor([m - 1, 0, m // 2], dtype=torch.int32).cuda()
+    close = dict(rtol=2e-5, atol=2e-5)
+    calls = [lambda r, delta: ops.add_rmsnorm(r, delta, weight, 1e-5, torch.float32), lambda r, delta: ops.add_rmsnorm_rows(r, delta, rows, weight, 1e-5, torch.float32),
+             lambda r, delta: ops.norm_add(r, delta, weight, 1e-5, 0.7, torch.float32), lambda r, delta: ops.norm_add_norm(r, delta, weight, 1e-5, weight, 1e-6, torch.float32)]
+    for call in calls:
+        a, b = residual.clone(), residual.clone()
+        torch.testing.assert_close(call(a, got).float(), call(b, whole).float(), **close)
+        torch.testing.assert_close(a, b, **close)
+
+    class Context:
+        dtype = torch.float32
+
+    Context.ops = ops
+    norm = StreamNorm("", n, 1e-5, streams=2, center=False)
+    norm.weight = weight
+    wide = torch.cat([residual, -residual], 1)
+    a, b = wide.clone(), wide.clone()
+    torch.testing.assert_close(norm.forward(a, got, Context), norm.forward(b, whole, Context), **close)
+    torch.testing.assert_close(a, b, **close)
+
+
+@pytest.mark.parametrize("m, n, k", [(128, 2048, 8448), (512, 2048, 5632), (1036, 2048, 5632), (128, 1536, 8960), (256, 512, 16384), (400, 256, 12288), (700, 8192, 29568), (836, 8192, 29568),
+                                     (400, 16384, 16384), (1280, 6144, 16384), (1536, 5120, 13824), (64, 3584, 18944), (4096, 3584, 18944)])
+def test_products_that_the_library_works_faster_stay_with_it(ops, m, n, k):
+    assert ops.tile_splits(m, n, k) == 0

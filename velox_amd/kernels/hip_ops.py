@@ -802,7 +802,7 @@ class HipOps:
                 and 16 < m <= 64 and k % 64 == 0 and n <= 8192 and n % 4 == 0):
             return self.skinny_gemm_splitk(x, weight, packed=packed)
         if bias is None and out_dtype == torch.bfloat16 and self.use_library_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
-            splits = self.tile_splits(m, n, k)
+            splits = 0 if (m, n, k) in self._timed_products else self.tile_splits(m, n, k)
             if splits == 1 or (splits > 1 and partials_ok):
                 return self.gemm_tiles(x, weight, splits, torch.bfloat16 if splits == 1 else torch.float32)
         skinny_rows = 16 if n > 8192 else 32  # measured on MI355X: beyond this the library's kernels stream faster
@@ -1026,17 +1026,31 @@ class HipOps:
         """Parts of k in which ``linear`` works a product in the framework's own tiles of 128 x 256 (0: not at all, the library's).  The
         library gives a product with few tiles and a long sum (a feed-forward's second product) too few workgroups; here
         the sum is cut until about every compute unit has one, and the norm that follows adds the parts.  Measured on
-        MI355X, product and norm (us, library / own): 18,944 -> 3,584 at 300 tokens 103 / 61, 512: 178 / 83, 836: 188 / 146, 1,036: 209 /
-        159, 1,536: 289 / 222, 2,048: 377 / 310, 4,096: 581 / 615; 8,448 -> 2,048 at 200: 31 / 27, 836: 53 / 47, 1,536: 65 / 74; 11,008 -> 4,096 at
-        512: 69 / 59, 836: 101 / 97, 1,036: 115 / 162; 4,096 -> 4,096 at 512: 33 / 34.  So: at least three parts, or sums so long that the
-        library is far from its rate, and one workgroup per compute unit.  Sizes that ``tune_library_products`` has timed
-        stay with the library (18,944 -> 3,584 at 2,048 tokens then takes 239 us alone)."""
-        if m <= 64 or k < 5120 or k % 8 != 0 or n % 4 != 0 or (m, n, k) in self._timed_products:
+        MI355X, product and norm (us, library / own, n x k):
+
+        - tiles for a third of the compute units: 3,584 x 18,944 at 65 tokens 100 / 46, 300: 105 / 62, 700: 171 / 111; 1,024 x 28,672 at 150:
+          104 / 54; 4,096 x 11,008 at 65: 42 / 34, 512: 76 / 61; 2,048 x 10,944 at 65: 37 / 30; 2,560 x 10,240 at 65: 31 / 31.  Below 20 million
+          weights the library cuts the sum itself and wins up to a few hundred tokens: 2,048 x 8,448 at 65: 25 / 25, 128: 26 / 29, 300: 39 / 30,
+          1,036: 73 / 57; 1,536 x 8,960 at 128: 23 / 28, 512: 34 / 33, 1,036: 53 / 48; 2,048 x 7,168 at 256: 26 / 27, 400: 34 / 29; 1,024 x 8,192 at
+          400: 28 / 28, 640: 31 / 29; 512 x 16,384 at 256: 25 / 36, 640: 46 / 37; 256 x 12,288 at 640: 27 / 30, 1,280: 37 / 31.  Shorter sums
+          stay with it: 2,048 x 5,632 at 300: 25 / 25, 512: 26 / 29, 836: 38 / 38, 1,036: 46 / 44.
+        - more tiles, up to one per compute unit, and sums so long that the library is far from its rate: 3,584 x 18,944 at 836: 182 / 153,
+          1,536: 283 / 233, 2,048: 381 / 287; 4,096 x 16,512 at 700: 197 / 128, 2,048: 376 / 273; 5,120 x 27,648 at 836: 335 / 294, 1,536: 558 /
+          428; but 3,072 x 12,288 at 1,036: 112 / 104, 1,536: 138 / 144; 5,120 x 13,824 at 836: 156 / 158, 1,536: 211 / 227.  Wide products
+          have tiles enough for the library earlier: 8,192 x 29,568 at 512 (128 tiles): 327 / 274, 700 (192): 322 / 392; 8,192 x 16,384 at
+          512: 170 / 155, 640 (160): 192 / 203; 16,384 x 16,384 at 256 (128): 242 / 226, 400 (256): 278 / 298; 6,144 x 24,576 at 900 (192):
+          399 / 310, 6,144 x 16,384 at 1,280 (240): 245 / 268; 7,168 x 28,672 at 900 (224): 499 / 413, 1,100 (252): 426 / 466.
+
+        (Residual streams add the parts in a pass of their own: 4,096 x 11,008 at 128 rows 65 / 46, 512: 85 / 77; 2,048 x 8,448 at 300: 43 / 38,
+        836: 66 / 61; 1,536 x 8,960 at 512: 38 / 42.)"""
+        if m <= 64 or k % 8 != 0 or n % 4 != 0:
             return 0
         tiles, steps = -(-m // 128) * -(-n // 256), -(-k // 64)
         if 3 * tiles <= self.num_cus:
+            if k < 7168 or (n * k < 20_000_000 and m * n * k < 4_500_000_000):
+                return 0
             splits = min(8, self.num_cus // tiles)
-        elif tiles <= self.num_cus and k >= 16384:
+        elif k >= 16384 and tiles <= (self.num_cus if n < 6144 else 7 * self.num_cus // 8 if n < 8192 else self.num_cus // 2):
             splits = min((1, 2, 3, 4), key=lambda s: -(-tiles * s // self.num_cus) * -(-steps // s))
         else:
             return 0
