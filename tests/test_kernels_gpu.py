@@ -1395,3 +1395,40 @@ def test_linear_with_parts_of_a_long_sum_into_every_consumer(ops, ref, m, n, k, 
                                      (400, 16384, 16384), (1280, 6144, 16384), (1536, 5120, 13824), (64, 3584, 18944), (4096, 3584, 18944)])
 def test_products_that_the_library_works_faster_stay_with_it(ops, m, n, k):
     assert ops.tile_splits(m, n, k) == 0
+
+
+def test_products_whose_library_kernel_was_timed_elsewhere_stay_with_it(ops, tmp_path, monkeypatch):
+    """Timings that come from a file, and products that TunableOp is about to time, are respected like those of this object; without them
+    the same product takes the own tiles."""
+    m, n, k = 300, 2560, 8192
+    x, w = rand((m, k), torch.bfloat16, 1), rand((n, k), torch.bfloat16, 2, k ** -0.5)
+    own = []
+    monkeypatch.setattr(ops, "gemm_tiles", lambda *a, **more: own.append(a) or type(ops).gemm_tiles(ops, *a, **more))
+    tunable = torch.cuda.tunable
+    held = tunable.get_filename(), tunable.get_max_tuning_duration(), tunable.get_max_tuning_iterations()
+
+    def calls_own():
+        own.clear()
+        ops.linear(x, w, None, torch.bfloat16, partials_ok=True)
+        return len(own) == 1
+
+    assert calls_own()
+    try:
+        tunable.set_filename(str(tmp_path / "timed.csv"))
+        tunable.set_max_tuning_duration(1)
+        tunable.set_max_tuning_iterations(1)
+        tunable.enable(True)
+        tunable.tuning_enable(False)
+        assert calls_own()  # (switched on, but nothing known about this product)
+        tunable.tuning_enable(True)
+        assert not calls_own()  # (timed now, by the library's call)
+        tunable.tuning_enable(False)
+        assert not calls_own()
+        assert ops.linear(x, w, None, torch.bfloat16, partials_ok=True).shape == (m, n)
+    finally:
+        tunable.tuning_enable(False)
+        tunable.enable(False)
+        tunable.set_max_tuning_duration(held[1])
+        tunable.set_max_tuning_iterations(held[2])
+        tunable.set_filename(held[0])
+    assert calls_own()

@@ -98,7 +98,6 @@ class HipOps:
         self.use_skinny_gemm = True
         self.pack_decode_weights = True
         self.fuse_residual_norm = True
-        self._timed_products = set()  # (m, n, k) whose library kernels have been timed (``tune_library_products``)
         self.use_grouped_mfma = True  # (False: the grouped bfloat16 products take the exact multiply-add tiles, for tests)
         self._mm_out_dtype_ok: Optional[bool] = None
         self._bias_copies: Dict[Tuple[int, int], Tuple[torch.Tensor, torch.Tensor]] = {}
@@ -335,7 +334,6 @@ class HipOps:
                 for m in sorted(set(token_counts)):
                     x = torch.randn((m, k), dtype=torch.float32, device=self.device).to(torch.bfloat16)
                     torch.nn.functional.linear(x, weight)
-                    self._timed_products.add((m, n, k))
                     done += 1
                 del weight
             torch.cuda.synchronize(self.device)
@@ -802,8 +800,8 @@ class HipOps:
                 and 16 < m <= 64 and k % 64 == 0 and n <= 8192 and n % 4 == 0):
             return self.skinny_gemm_splitk(x, weight, packed=packed)
         if bias is None and out_dtype == torch.bfloat16 and self.use_library_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
-            splits = 0 if (m, n, k) in self._timed_products else self.tile_splits(m, n, k)
-            if splits == 1 or (splits > 1 and partials_ok):
+            splits = self.tile_splits(m, n, k)
+            if (splits == 1 or (splits > 1 and partials_ok)) and not self._library_has_timed(m, n, k):
                 return self.gemm_tiles(x, weight, splits, torch.bfloat16 if splits == 1 else torch.float32)
         skinny_rows = 16 if n > 8192 else 32  # measured on MI355X: beyond this the library's kernels stream faster
         if self.use_skinny_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and m <= skinny_rows and k % 64 == 0:
@@ -1055,6 +1053,18 @@ class HipOps:
         else:
             return 0
         return -(-steps // -(-steps // splits))  # (no empty part)
+
+    @staticmethod
+    def _library_has_timed(m: int, n: int, k: int) -> bool:
+        """Whether TunableOp holds a choice of its own for this product, or is about to make one: timed by this process
+        (``tune_library_products``) or read from a file, by whom ever.  Such a product stays with the library (3,584 x 18,944 at 2,048 rows,
+        with the norm behind it: the library's default 381 us, the own tiles 287; its timed kernel takes 239 alone).  What TunableOp holds can change at any time and is
+        asked for each time, 6 us for 50 results and only while it is switched on."""
+        tunable = torch.cuda.tunable
+        if not tunable.is_enabled():
+            return False
+        size = f"tn_{n}_{m}_{k}_"
+        return tunable.tuning_is_enabled() or any(r[0] == "GemmTunableOp_BFloat16_TN" and r[1].startswith(size) for r in tunable.get_results())
 
     def gemm_tiles(self, x, weight, splits: int = 1, out_dtype=torch.bfloat16):
         """``x @ weight^T`` in bfloat16 in tiles of 128 x 256: [M, N] in bfloat16, or float32 partial sums [splits, M, N]."""
