@@ -1432,3 +1432,31 @@ def test_products_whose_library_kernel_was_timed_elsewhere_stay_with_it(ops, tmp
         tunable.set_max_tuning_iterations(held[2])
         tunable.set_filename(held[0])
     assert calls_own()
+
+
+@pytest.mark.parametrize("top_p, top_k", [(1.0, 0), (0.9, 0), (1e-6, 0), (1.0, 1), (1.0, 50), (0.5, 20)])
+@pytest.mark.parametrize("temperature", [0.7, 1e-30, float("inf")])
+def test_rows_with_numbers_that_are_not_finite_get_a_token_of_the_row(ops, top_p, top_k, temperature):
+    """Whatever a row holds, the token lies in the vocabulary and does not depend on how the row is cut; a NaN is never drawn and, behind
+    top-p, does not change the draw (its probability counts as none)."""
+    vocab, inf, nan = 32773, float("inf"), float("nan")
+    logits = rand((9, vocab), torch.float32, 3, 3.0)
+    logits[0, 777] = inf
+    logits[1, [5, 9000]] = inf
+    logits[2, [333, 20000]] = nan
+    logits[3] = -inf
+    logits[4, 40:] = -inf
+    logits[5] = torch.finfo(torch.float32).min
+    logits[6] *= 1e37
+    logits[7] = nan
+    logits[8] = logits[2].nan_to_num(nan=-inf)
+    options = np.zeros((9, 6), dtype=np.int32)
+    options.view(np.float32)[:, 0], options.view(np.float32)[:, 1] = temperature, top_p
+    options[:, 2], options[:, 3] = top_k, 11
+    options = torch.from_numpy(options).cuda()
+    whole = ops.sample(logits, options, chunks=1)
+    for chunks in (2, 3, 8):
+        assert torch.equal(ops.sample(logits, options, chunks=chunks), whole)
+    assert torch.all((whole >= 0) & (whole < vocab))
+    if top_k == 0:
+        assert whole[2] == whole[8]

@@ -415,7 +415,10 @@ struct DrawQueue {
 __device__ __forceinline__ void draw_token(int i, float x, uint32_t bits, float mx, Best& best) {
   const float u = ((float)(bits >> 8) + 0.5f) * (1.0f / 16777216.0f);
   const float noise = fmaxf(-logf(u), 1e-10f);
-  const float score = (x - mx) - logf(noise);
+  const float raw = (x - mx) - logf(noise);
+  // A score that is no number (of a NaN among the logits, or where the row's largest is infinite) counts as -inf: it would otherwise
+  // win or lose by the order in which threads meet it, and could leave a row without any token.
+  const float score = raw > -INFINITY ? raw : -INFINITY;
   // (a thread's tokens come in no order: equal scores go to the smaller index here too)
   if (score > best.value || best.index == 0x7fffffff || (score == best.value && i < best.index)) best = Best{score, i};
 }
