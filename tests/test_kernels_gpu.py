@@ -1460,3 +1460,22 @@ def test_rows_with_numbers_that_are_not_finite_get_a_token_of_the_row(ops, top_p
     assert torch.all((whole >= 0) & (whole < vocab))
     if top_k == 0:
         assert whole[2] == whole[8]
+
+
+def test_experts_whose_weights_lie_off_16_byte_boundaries(ops):
+    """More than 64 pairs then take the multiply-add tiles: the same products in another order of float32 sums, the units' middles and the
+    result rounded to bfloat16 on both paths (2^-8 each, of terms that add up to a few times the result)."""
+    tokens, top, experts, hidden, inter = 60, 2, 4, 72, 40
+    x, weight = rand((tokens, hidden), torch.bfloat16, 1), rand((tokens, top), torch.float32, 2).abs()
+    choice = torch.randint(0, experts, (tokens, top), generator=torch.Generator().manual_seed(3)).to(torch.int32).cuda()
+    first, down = rand((experts * 2 * inter, hidden), torch.bfloat16, 4, hidden ** -0.5), rand((experts * hidden, inter), torch.bfloat16, 5, inter ** -0.5)
+
+    def moved(w):
+        flat = torch.empty(w.numel() + 2, dtype=w.dtype, device=w.device)
+        flat[2:] = w.reshape(-1)
+        return flat[2:].view(w.shape)
+
+    want = ops.routed_experts(x, choice, weight, first, down, experts, False, None, torch.bfloat16)
+    for a, b in ((moved(first), down), (first, moved(down))):
+        assert (a.data_ptr() | b.data_ptr()) % 16 == 4
+        torch.testing.assert_close(ops.routed_experts(x, choice, weight, a, b, experts, False, None, torch.bfloat16).float(), want.float(), rtol=2e-2, atol=2e-2)

@@ -1744,6 +1744,8 @@ class HipOps:
         else:
             plan = torch.empty(elems, dtype=torch.int32, device=self.device)
         on_matrix_cores = x.dtype == torch.bfloat16 and hidden % 8 == 0 and inter % 8 == 0 and self.use_grouped_mfma
+        if pairs > self.FEW_PAIRS and (gate_up_weight.data_ptr() | down_weight.data_ptr()) % 16 != 0:
+            on_matrix_cores = False  # (loads that write LDS directly need 16-byte boundaries; the multiply-add tiles take any)
         tile_rows = 128 if on_matrix_cores and pairs > self.FEW_PAIRS else 64
         if on_matrix_cores and x.data_ptr() % 16 != 0:
             x = x.clone()
