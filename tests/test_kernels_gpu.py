@@ -1250,11 +1250,16 @@ def test_rows_that_their_pairs_weight_scales_are_rounded_once_on_every_path(ops,
     assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("m, n, k", [(17, 64, 128), (33, 65, 36), (64, 100, 256), (70, 333, 260), (65, 2048, 1540), (200, 2048, 516), (300, 6500, 132), (610, 1536, 288), (1025, 4100, 196)])
-def test_float32_products_on_the_matrix_instructions(ops, m, n, k):
-    """Every tile and both numbers of sets of waves, remainders in all three sizes.  A sum of at most GEMM_FOLD = 128 terms, then of as many
+@pytest.mark.parametrize("m, n, k, tile", [(17, 64, 128, "32 x 32, 2"), (33, 65, 36, None), (64, 100, 256, "32 x 32, 2"), (70, 333, 260, "32 x 32, 2"), (65, 2048, 1540, "32 x 32, 2"),
+                                           (200, 2048, 516, "32 x 64, 2"), (300, 6500, 132, "32 x 64, 2"), (610, 1536, 288, "64 x 64, 2"), (1025, 4100, 196, "64 x 64, 1"),
+                                           (1020, 4100, 260, "128 x 64, 1"), (616, 7004, 1540, "128 x 64, 1"), (1024, 4096, 128, "128 x 64, 1"), (640, 6565, 132, "128 x 64, 1")])
+def test_float32_products_on_the_matrix_instructions(ops, m, n, k, tile):
+    """Every tile and both numbers of sets of waves, remainders in all three sizes (and one sum too short for them).  A sum of at most GEMM_FOLD = 128 terms, then of as many
     such sums, all float32: off by at most (128 + k / 128 + 2) 2^-24 of the sum of the terms' sizes.  The same row in a batch of
     another size, which takes another tile, has the same bits."""
+    if tile is not None:
+        code = ops._core.velox_gemm_f32_tile(m, n)
+        assert f"{code // 10000} x {code // 10 % 1000}, {code % 10}" == tile
     generator = torch.Generator(device="cuda").manual_seed(m + n + k)
     a, w, bias = (torch.randn(*shape, generator=generator, device="cuda") for shape in ((m, k), (n, k), (n,)))
     got = ops.gemm_fma(a, w, bias, torch.float32)

@@ -267,16 +267,29 @@ __global__ void __launch_bounds__(256 * SETS) __attribute__((amdgpu_waves_per_eu
 //   300 rows, 8,960 -> 1,536       331   204 |  182   119   139        64 rows, 8,960 -> 1,536      330  200 | 178  111   70
 // so: from two workgroups per compute unit on one set, in tiles of 128 rows if few of them stay empty; with about one workgroup
 // per compute unit 64 x 64 by two sets; with fewer the largest tile that still gives most compute units a workgroup.
-static void launch_mfma_f32(const void* a, const void* w, const float* bias, void* out, int m, int n, int k, hipStream_t stream) {
+// The tile as rows * 10,000 + columns * 10 + sets (an entry point so that a test can tell which one a size takes).
+extern "C" int velox_gemm_f32_tile(int m, int n) {
   auto tiles = [&](int rt, int ct) { return (long long)((m + 32 * rt - 1) / (32 * rt)) * ((n + 32 * ct - 1) / (32 * ct)); };
-#define MFMA(RT, CT, SETS, STAGES)                                                                                                     \
-  gemm_mfma_f32_kernel<RT, CT, SETS, STAGES><<<(unsigned)((tiles(RT, CT) + GEMM_XCDS - 1) / GEMM_XCDS * GEMM_XCDS), 256 * SETS, 0, stream>>>( \
-      (const float*)a, (const float*)w, bias, (float*)out, m, n, k)
-  if (tiles(4, 2) >= 512 && (m + 127) / 128 * 128 * 10 <= m * 11) MFMA(4, 2, 1, 2);
-  else if (tiles(2, 2) >= 512) MFMA(2, 2, 1, 3);
-  else if (tiles(2, 2) >= 200 && tiles(2, 2) <= 256) MFMA(2, 2, 2, 3);
-  else if (tiles(1, 2) >= 200) MFMA(1, 2, 2, 3);
-  else MFMA(1, 1, 2, 3);
+  if (tiles(4, 2) >= 512 && (m + 127) / 128 * 128 * 10 <= m * 11) return 1280641;
+  if (tiles(2, 2) >= 512) return 640641;
+  if (tiles(2, 2) >= 200 && tiles(2, 2) <= 256) return 640642;
+  return tiles(1, 2) >= 200 ? 320642 : 320322;
+}
+
+static void launch_mfma_f32(const void* a, const void* w, const float* bias, void* out, int m, int n, int k, hipStream_t stream) {
+#define MFMA(RT, CT, SETS, STAGES)                                                                                                  \
+  {                                                                                                                                 \
+    const long long tiles = (long long)((m + 32 * RT - 1) / (32 * RT)) * ((n + 32 * CT - 1) / (32 * CT));                           \
+    gemm_mfma_f32_kernel<RT, CT, SETS, STAGES><<<(unsigned)((tiles + GEMM_XCDS - 1) / GEMM_XCDS * GEMM_XCDS), 256 * SETS, 0, stream>>>( \
+        (const float*)a, (const float*)w, bias, (float*)out, m, n, k);                                                              \
+  }
+  switch (velox_gemm_f32_tile(m, n)) {
+    case 1280641: MFMA(4, 2, 1, 2) break;
+    case 640641: MFMA(2, 2, 1, 3) break;
+    case 640642: MFMA(2, 2, 2, 3) break;
+    case 320642: MFMA(1, 2, 2, 3) break;
+    default: MFMA(1, 1, 2, 3) break;
+  }
 #undef MFMA
 }
 
@@ -362,9 +375,10 @@ extern "C" int velox_gemm_fma(const void* a, const void* w, const float* bias, v
     }
     VELOX_RETURN_LAUNCH_STATUS();
   }
-  // Sums of fewer terms than one inner sum stay with the multiply-adds, whose order of additions is that of k: the maps of small
-  // models keep their bits, and what the matrix instructions would save there is small (64 terms, us, multiply-adds / matrix
-  // instructions: 417 x 256 outputs 6.4 / 3.4, 2,048 x 2,048 14.8 / 10.7; 256 terms 17.7 / 4.3 and 39.1 / 27.3).
+  // Sums of fewer terms than one inner sum stay with the multiply-adds, whose order of additions is that of k.  The matrix
+  // instructions are quicker there too (64 terms, us, multiply-adds / matrix instructions: 417 x 256 outputs 6.4 / 3.4, 2,048 x 2,048
+  // 14.8 / 10.7; 256 terms 17.7 / 4.3 and 39.1 / 27.3) and no less exact on average: the line is here because a small model with
+  // sharp weights, whose recurrences blow a rounding up a thousandfold, left its tolerance in the other order of additions.
   if (key == 0 && a_vec && w_vec && k >= GEMM_FOLD) {
     launch_mfma_f32(a, w, bias, out, m, n, k, stream);
     VELOX_RETURN_LAUNCH_STATUS();

@@ -187,6 +187,8 @@ class HipOps:
         c.velox_poly_norm.argtypes = [_P, _P, _P, _I, _I, _F, _I, _P]
         c.velox_removal_chunk_scan.argtypes = [_P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _P, _P, _I, _I, _P]
         c.velox_removal_chunk_scan.restype = _I
+        c.velox_gemm_f32_tile.argtypes = [_I, _I]
+        c.velox_gemm_f32_tile.restype = _I
         c.velox_gemm_tiles_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P]
         c.velox_gemm_tiles_bf16.restype = _I
         c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
