@@ -2,9 +2,8 @@
 // over its own rows, out[r, g, :] = W_g a[r, g, :].  Shared by the routed experts, by the per-head products of
 // attention over a latent and by single products whose sum is long and whose tiles are few (velox_gemm_tiles_bf16).
 //
-// A workgroup of four waves of the kernel without a plan owns 64 rows and 64 NT output columns of one group (NT = 2 or 4 tiles of W per wave; half as
-// many gate columns and the up columns of the same outputs with the GLU epilogue); a wave owns 16 NT of the columns and all
-// 64 rows: 4 NT 16x16 accumulators.  W comes straight from global memory in the layout of
+// A workgroup of four waves of the kernel without a plan owns 64 rows and 64 NT output columns of one group (NT = 2 or 4 tiles of W
+// per wave); a wave owns 16 NT of the columns and all 64 rows: 4 NT 16x16 accumulators.  W comes straight from global memory in the layout of
 // v_mfma_f32_16x16x32_bf16 (lane = 16 g + i holds indices 8 g .. 8 g + 7 of row i: 16 bytes) and is the left operand, so
 // acc[j] of lane (g, i) is out[row i][column 4 g + j]; no two waves read the same W.  The rows of `a`, which all four
 // waves need, pass through LDS: a step is 64 indices, 8 KB for the 64 rows, two 16-byte pieces per thread, laid out [piece][row] so
@@ -33,8 +32,8 @@ struct GroupedArgs {
   void* out;           // element (row r, group g, col) at out[r * out_ld + g * out_group + col]
   long long out_ld, out_group;
   int n, k;
-  // rows: either every group runs rows [0, m) (plan == nullptr, blockIdx.y = row tile, blockIdx.z = group), or the plan's
-  // tiles say which group runs which rows (blockIdx.y = tile)
+  // rows: either every group runs rows [0, m) (plan == nullptr; grouped_mfma_kernel: blockIdx.y = row tile, blockIdx.z = group;
+  // grouped_tiles_kernel: one group), or the plan's tiles say which group runs which rows
   int m;
   const int* plan;
   int plan_pairs, plan_groups, plan_max_tiles;
@@ -57,7 +56,8 @@ __device__ __forceinline__ gm_bf16x8_t gm_load(const bf16_t* p, bool ok) {
 
 template <int EPI, typename TO, int GM_NT>
 __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs args) {
-  constexpr int GM_COLS = 64 * GM_NT;    // output columns of the workgroup (GLU: half as many)
+  static_assert(EPI == GM_PLAIN || EPI == GM_GATE, "no other epilogue here");
+  constexpr int GM_COLS = 64 * GM_NT;    // output columns of the workgroup
   constexpr int MT = GM_ROWS / 16, HALVES = 2, STEP = 32 * HALVES;
   __shared__ float4_t a_lds[2][HALVES][4 * GM_ROWS];
   const int group = blockIdx.z, row0 = blockIdx.y * GM_ROWS, rows = min(GM_ROWS, args.m - row0);
@@ -65,19 +65,15 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
   const int lane = tid & 63, wave = tid >> 6;
   const int i = lane & 15, g4 = lane >> 4;
   const int n = args.n, k = args.k;
-  // the tiles of W this wave owns: their first output columns (GLU: the first half are gate rows, the others the up rows of the same)
-  int col0[GM_NT];
+  int col0[GM_NT];  // the first output columns of the tiles of W this wave owns
 #pragma unroll
-  for (int t = 0; t < GM_NT; ++t) {
-    if (EPI == GM_GLU) col0[t] = blockIdx.x * (GM_COLS / 2) + wave * (8 * GM_NT) + (t % (GM_NT / 2)) * 16;
-    else col0[t] = blockIdx.x * GM_COLS + wave * (16 * GM_NT) + t * 16;
-  }
+  for (int t = 0; t < GM_NT; ++t) col0[t] = blockIdx.x * GM_COLS + wave * (16 * GM_NT) + t * 16;
   const bf16_t* w_base = args.w + (size_t)group * args.w_group;
   const bf16_t* w_row[GM_NT];
 #pragma unroll
   for (int t = 0; t < GM_NT; ++t) {
     const int col = min(col0[t] + i, n - 1);
-    w_row[t] = w_base + (size_t)(EPI == GM_GLU && t >= GM_NT / 2 ? n + col : col) * k + 8 * g4;
+    w_row[t] = w_base + (size_t)col * k + 8 * g4;
   }
   // this thread's piece of the rows of `a`: row tid / 4, indices 8 (tid % 4) .. + 7 of a half; in LDS [part][row], so that a
   // row tile's operand reads are 256 contiguous bytes per 16 lanes
@@ -142,12 +138,12 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
     if (r >= rows) continue;
     const size_t out_row = (size_t)(row0 + r) * args.out_ld + (size_t)group * args.out_group;
 #pragma unroll
-    for (int t = 0; t < (EPI == GM_GLU ? GM_NT / 2 : GM_NT); ++t) {
+    for (int t = 0; t < GM_NT; ++t) {
       const int col = col0[t] + 4 * g4;
       if (col >= n) continue;
       float v[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = EPI == GM_GLU ? glu_middle(acc[t][mt][j], acc[t + GM_NT / 2][mt][j], args.unit) : acc[t][mt][j];
+      for (int j = 0; j < 4; ++j) v[j] = acc[t][mt][j];
       if (EPI == GM_GATE) {
         const bf16_t* gate = args.gate + (size_t)(row0 + r) * args.gate_ld + (size_t)group * args.gate_group;
         float z[4];
@@ -163,10 +159,6 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] *= 1.f / (1.f + expf(-z[j]));
-      }
-      if (EPI == GM_ACT) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = ungated_act(v[j], args.act);
       }
       if (vec) {
         Four four;
@@ -291,10 +283,6 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
         if (col >= n) continue;
         float v = acc[t][mt][j];
         if (EPI == GM_GLU) v = glu_middle(v, acc[1][mt][j], args.unit);
-        if (EPI == GM_GATE) {
-          const float z = to_f32(args.gate[(size_t)(row0 + r) * args.gate_ld + (size_t)group * args.gate_group + (size_t)col * args.gate_col]);
-          v *= 1.f / (1.f + expf(-z));
-        }
         if (EPI == GM_ACT) v = ungated_act(v, args.act);
         out[out_row + col] = from_f32<TO>(v);
       }
@@ -303,6 +291,7 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
 
 template <int EPI, typename TO>
 __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const GroupedArgs args) {
+  static_assert(EPI == GM_PLAIN || EPI == GM_GLU || EPI == GM_ACT, "no gate here");
   __shared__ float4_t partial[3][8][64];
   const int tile = blockIdx.y;
   if (tile >= args.plan[0]) return;  // (uniform over the workgroup)
@@ -345,6 +334,7 @@ static __device__ __attribute__((aligned(16))) const unsigned int gm_zero_piece[
 
 template <int EPI, typename TO>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) grouped_tiles_kernel(const GroupedArgs args, const int cols) {
+  static_assert(EPI == GM_PLAIN || EPI == GM_GLU || EPI == GM_ACT, "no gate here");
   constexpr int ROWS = GM_TILE_ROWS, STAGES = 3, WAVES = 8;
   constexpr int WM = 2, WN = WAVES / WM;               // waves along the rows of `a` and along those of W
   constexpr int RT = 4, CT = GM_TILE_COLS / WN / 16;   // 16 x 16 tiles of a wave
@@ -507,34 +497,27 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 }
 
-// Launches the kernel that fits: `most_rows` is the most rows any tile can have (the plan's pairs, or m), `tiles_y` the most
-// tiles there can be and `tiles_z` the groups (without a plan).  A plan's tiles hold 64 rows up to 64 pairs, GM_TILE_ROWS above;
-// without a plan rows come in tiles of GM_ROWS.  (Tiles of 64 rows were no quicker at any number of pairs above 64: 12 rows per
-// expert 66 us either way, 56: 80 / 81, 75: 100 / 83, 130: 127 / 125, 256: 187 / 155, 16 experts of 2,048 -> 1,408 -> 2,048.)
+// The products of a plan: `pairs` is the most rows a tile can have, `most_tiles` the most tiles there can be.  Tiles hold 64 rows up to 64
+// pairs, GM_TILE_ROWS above.  (Tiles of 64 rows were no quicker at any number of pairs above 64: 12 rows per expert 66 us either way,
+// 56: 80 / 81, 75: 100 / 83, 130: 127 / 125, 256: 187 / 155, 16 experts of 2,048 -> 1,408 -> 2,048.)
 template <int EPI, typename TO>
-static void grouped_mfma_launch(const GroupedArgs& args, int most_rows, int tiles_y, int tiles_z, hipStream_t stream) {
-  const int n = args.n;
-  const int outputs = EPI == GM_GLU ? 2 * n : n;  // rows of W
-  if (args.plan != nullptr) {
-    // (its tiles hold at most `most_rows` rows whatever their size)
-    if (most_rows <= 64) {
-      constexpr int COLS = EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS;
-      dim3 grid((n + COLS - 1) / COLS, tiles_y, 1);
-      grouped_mfma_few_rows_kernel<EPI, TO><<<grid, 256, 0, stream>>>(args);
-      return;
-    }
-    const int cols = (outputs + GM_TILE_COLS - 1) / GM_TILE_COLS;
-    const int workgroups = (tiles_y * cols + GM_XCDS - 1) / GM_XCDS * GM_XCDS;
-    grouped_tiles_kernel<EPI, TO><<<workgroups, 512, 0, stream>>>(args, cols);
+static void grouped_plan_launch(const GroupedArgs& args, int pairs, int most_tiles, hipStream_t stream) {
+  if (pairs <= 64) {
+    constexpr int COLS = EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS;
+    grouped_mfma_few_rows_kernel<EPI, TO><<<dim3((args.n + COLS - 1) / COLS, most_tiles), 256, 0, stream>>>(args);
     return;
   }
-  if (outputs <= 128) {
-    const int cols = EPI == GM_GLU ? 64 : 128;
-    grouped_mfma_kernel<EPI, TO, 2><<<dim3((n + cols - 1) / cols, tiles_y, tiles_z), 256, 0, stream>>>(args);
-  } else {
-    const int cols = EPI == GM_GLU ? 128 : 256;
-    grouped_mfma_kernel<EPI, TO, 4><<<dim3((n + cols - 1) / cols, tiles_y, tiles_z), 256, 0, stream>>>(args);
-  }
+  const int cols = ((EPI == GM_GLU ? 2 * args.n : args.n) + GM_TILE_COLS - 1) / GM_TILE_COLS;
+  const int workgroups = (most_tiles * cols + GM_XCDS - 1) / GM_XCDS * GM_XCDS;
+  grouped_tiles_kernel<EPI, TO><<<workgroups, 512, 0, stream>>>(args, cols);
+}
+
+// The products of `groups` groups that all run rows [0, m).
+template <int EPI, typename TO>
+static void grouped_rows_launch(const GroupedArgs& args, int groups, hipStream_t stream) {
+  const int row_tiles = (args.m + GM_ROWS - 1) / GM_ROWS;
+  if (args.n <= 128) grouped_mfma_kernel<EPI, TO, 2><<<dim3(1, row_tiles, groups), 256, 0, stream>>>(args);
+  else grouped_mfma_kernel<EPI, TO, 4><<<dim3((args.n + 255) / 256, row_tiles, groups), 256, 0, stream>>>(args);
 }
 
 // Whether the operands meet what the kernels' 16-byte loads need.

@@ -515,12 +515,12 @@ extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, co
   first.row_scale = scale_input ? pair_weight : nullptr;  // (read by the kernel for few rows alone)
   first.act = ungated;
   first.unit = GluUnit{alpha, limit, shift};
-  if (ungated > 0) grouped_mfma_launch<GM_ACT, bf16_t>(first, pairs, max_tiles, 1, stream);
-  else grouped_mfma_launch<GM_GLU, bf16_t>(first, pairs, max_tiles, 1, stream);
+  if (ungated > 0) grouped_plan_launch<GM_ACT, bf16_t>(first, pairs, max_tiles, stream);
+  else grouped_plan_launch<GM_GLU, bf16_t>(first, pairs, max_tiles, stream);
   GroupedArgs last = routed_args(act, down, y, plan, pairs, experts, hidden, inter, hidden);
   // (a weight on the experts' OUTPUT is applied where the results are added up, routed_combine with scale_rows: the product
   // itself is the same kernel either way)
-  grouped_mfma_launch<GM_PLAIN, float>(last, pairs, max_tiles, 1, stream);
+  grouped_plan_launch<GM_PLAIN, float>(last, pairs, max_tiles, stream);
   VELOX_RETURN_LAUNCH_STATUS();
 }
 
