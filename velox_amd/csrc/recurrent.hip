@@ -926,8 +926,13 @@ struct ScanArgs {
   const int* cu_q;
   float* out;            // [T, heads * vdim]
   int heads, kv_heads, dim, vdim, delta;
-  int from_tokens, below_tokens;  // sequences of at least from_tokens (1 or more) and fewer than below_tokens tokens are worked
+  int from_tokens, below_tokens;  // the kernels with SOME work sequences of at least from_tokens and fewer than below_tokens tokens
 };
+// Whether a sequence of `count` tokens is left alone (empty ones always are).  Read only where it has to be: two numbers more in front of
+// a decode step's first loads cost 0.5 us of 9.
+template <bool SOME> __device__ __forceinline__ bool scan_leaves(const ScanArgs& a, int count) {
+  return SOME ? count < a.from_tokens || count >= a.below_tokens : count <= 0;
+}
 
 __device__ __forceinline__ void scan_load_rows(const float* __restrict__ p, int d0, int dim, bool vec, float fill, float (&r)[SCAN_ROWS]) {
   if (vec && d0 + SCAN_ROWS <= dim) {
@@ -979,13 +984,13 @@ __device__ __forceinline__ float scan_token(float (&s)[SCAN_ROWS], const float (
   return sum_over_lanes<R>((p[0] + p[1]) + (p[2] + p[3]));
 }
 
-template <int R, bool REMOVAL>
+template <int R, bool REMOVAL, bool SOME = false>
 __global__ void __launch_bounds__(256) linear_scan_kernel(const ScanArgs a) {
   const int r = threadIdx.x % R;
   const int e = blockIdx.x * (256 / R) + threadIdx.x / R;
   const int h = blockIdx.y, b = blockIdx.z;
   const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  if (hi - lo < a.from_tokens || hi - lo >= a.below_tokens) return;
+  if (scan_leaves<SOME>(a, hi - lo)) return;
   const bool live = e < a.vdim;
   const int col = live ? e : a.vdim - 1;  // (lanes beyond the last column follow it and write nothing: the shuffles need every lane)
   const int dim = a.dim, vdim = a.vdim;
@@ -1045,7 +1050,7 @@ __global__ void __launch_bounds__(256) linear_scan_staged_kernel(const ScanArgs 
   const int e = blockIdx.x * COLS + c_local;
   const int h = blockIdx.y, b = blockIdx.z;
   const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  if (hi - lo < a.from_tokens || hi - lo >= a.below_tokens) return;  // (the whole workgroup: no barrier is left waiting)
+  if (hi <= lo) return;  // (the whole workgroup: no barrier is left waiting)
   const bool live = e < a.vdim;
   const int col = live ? e : a.vdim - 1;
   const int dim = a.dim, vdim = a.vdim, heads = a.heads;
@@ -1236,7 +1241,7 @@ __host__ __device__ __forceinline__ int wave_buffer_floats(int tokens, int dim, 
   return tokens * (vectors * dim + (per_channel ? dim : 0) + WAVE_COLS + 2);
 }
 
-template <int RW, bool REMOVAL>
+template <int RW, bool REMOVAL, bool SOME = false>
 __global__ void __launch_bounds__(512) linear_scan_wave_kernel(const ScanArgs a, const int block_tokens) {
   extern __shared__ float4_t stage_pieces[];
   float* stage = reinterpret_cast<float*>(stage_pieces);
@@ -1244,7 +1249,7 @@ __global__ void __launch_bounds__(512) linear_scan_wave_kernel(const ScanArgs a,
   const int e = blockIdx.x * WAVE_COLS + wave;
   const int h = blockIdx.y, b = blockIdx.z;
   const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  if (hi - lo < a.from_tokens || hi - lo >= a.below_tokens) return;  // (the whole workgroup)
+  if (scan_leaves<SOME>(a, hi - lo)) return;  // (the whole workgroup)
   const bool live = e < a.vdim;
   const int col = live ? e : a.vdim - 1;
   const int dim = 64 * RW, vdim = a.vdim, heads = a.heads;
@@ -1401,15 +1406,36 @@ static int scan_block_tokens(int dim, int lanes, int per_channel, int vectors) {
   return tokens >= 2 ? tokens : 0;
 }
 
+static size_t wave_scan_lds(const ScanArgs& a, int vectors, int& tokens) {
+  tokens = 16;
+  while (2 * wave_buffer_floats(tokens, a.dim, a.decay_per_channel, vectors) * (int)sizeof(float) > 60 * 1024) tokens >>= 1;  // (dim = 512 with a decay per channel: 4, or 2)
+  return (size_t)2 * (wave_buffer_floats(tokens, a.dim, a.decay_per_channel, vectors) + tokens * WAVE_COLS) * sizeof(float);  // (+ two blocks of read-outs)
+}
+
+// The sequences that are shorter than the chunked kernels' (key heads of 64 or 128 channels): single tokens and pairs, or longer ones.
+static void linear_scan_short_launch(const ScanArgs& a, int num_seqs, bool singles, hipStream_t stream) {
+  if (singles) {
+    const int cols = a.dim == 64 ? 32 : 16;
+    const dim3 grid((a.vdim + cols - 1) / cols, a.heads, num_seqs);
+    if (a.dim == 64) linear_scan_kernel<8, false, true><<<grid, 256, 0, stream>>>(a);
+    else linear_scan_kernel<16, false, true><<<grid, 256, 0, stream>>>(a);
+    return;
+  }
+  int tokens;
+  const size_t lds = wave_scan_lds(a, 2, tokens);
+  const dim3 grid((a.vdim + WAVE_COLS - 1) / WAVE_COLS, a.heads, num_seqs);
+  if (a.dim == 64) linear_scan_wave_kernel<1, false, true><<<grid, 512, lds, stream>>>(a, tokens);
+  else linear_scan_wave_kernel<2, false, true><<<grid, 512, lds, stream>>>(a, tokens);
+}
+
 template <bool REMOVAL>
 static void linear_scan_launch(const ScanArgs& a, int lanes, int num_seqs, int max_q_len, hipStream_t stream) {
   const int dim = a.dim, vectors = REMOVAL ? 3 : 2;
   const int cols = 256 / lanes;
   const dim3 grid((a.vdim + cols - 1) / cols, a.heads, num_seqs);
   if (max_q_len > 2 && (dim == 64 || dim == 128 || dim == 256 || dim == 512)) {
-    int tokens = 16;
-    while (2 * wave_buffer_floats(tokens, dim, a.decay_per_channel, vectors) * (int)sizeof(float) > 60 * 1024) tokens >>= 1;  // (dim = 512 with a decay per channel: 4, or 2)
-    const size_t lds = (size_t)2 * (wave_buffer_floats(tokens, dim, a.decay_per_channel, vectors) + tokens * WAVE_COLS) * sizeof(float);  // (+ two blocks of read-outs)
+    int tokens;
+    const size_t lds = wave_scan_lds(a, vectors, tokens);
     const dim3 wave_grid((a.vdim + WAVE_COLS - 1) / WAVE_COLS, a.heads, num_seqs);
     switch (dim) {
       case 64: linear_scan_wave_kernel<1, REMOVAL><<<wave_grid, 512, lds, stream>>>(a, tokens); break;
@@ -1445,18 +1471,21 @@ static void linear_scan_launch(const ScanArgs& a, int lanes, int num_seqs, int m
   }
 }
 
-// rule 0: additive, 1: delta, 2: removal (three vectors per token, a decay per channel; beta holds the keys' lengths).  Sequences of
-// fewer than from_tokens or of below_tokens tokens and more are left alone; max_q_len chooses the kernel for the others.
+// rule 0: additive, 1: delta, 2: removal (three vectors per token, a decay per channel; beta holds the keys' lengths).  With
+// below_tokens > 0 only sequences of at least from_tokens (1 or more) and fewer than below_tokens tokens are worked (the first two rules,
+// key heads of 64 or 128 channels).
 extern "C" int velox_linear_scan(const float* qk, const void* v, int v_dtype, int v_ld, int v_at, const float* decay, int decay_per_channel, const float* beta,
                                  float* state, const int* slots, const int* cu_q, float* out, int num_seqs, int max_q_len, int heads, int kv_heads, int dim,
                                  int vdim, int rule, int from_tokens, int below_tokens, hipStream_t stream) {
   if (num_seqs <= 0) return 0;
   const int lanes = velox_linear_scan_lanes(dim);
-  if (lanes > 64 || heads > 65535 || num_seqs > 65535 || kv_heads < 1 || heads % kv_heads != 0 || rule < 0 || rule > 2 || (rule != 0 && !beta))
+  if (lanes > 64 || heads > 65535 || num_seqs > 65535 || kv_heads < 1 || heads % kv_heads != 0 || rule < 0 || rule > 2 || (rule != 0 && !beta) ||
+      (below_tokens > 0 && (rule == 2 || (dim != 64 && dim != 128) || from_tokens < 1)))
     return (int)hipErrorInvalidValue;
   ScanArgs a{qk, v, v_dtype == VELOX_BF16, v_ld, v_at, decay, decay_per_channel, beta, state, slots, cu_q, out, heads, kv_heads, dim, vdim, rule == 1,
-             from_tokens < 1 ? 1 : from_tokens, below_tokens};
-  if (rule == 2) linear_scan_launch<true>(a, lanes, num_seqs, max_q_len, stream);
+             from_tokens, below_tokens};
+  if (below_tokens > 0) linear_scan_short_launch(a, num_seqs, max_q_len <= 2, stream);
+  else if (rule == 2) linear_scan_launch<true>(a, lanes, num_seqs, max_q_len, stream);
   else linear_scan_launch<false>(a, lanes, num_seqs, max_q_len, stream);
   VELOX_RETURN_LAUNCH_STATUS();
 }

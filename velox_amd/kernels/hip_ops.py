@@ -1382,7 +1382,7 @@ class HipOps:
         out = torch.empty((tokens, heads * vdim), dtype=torch.float32, device=self.device)
         sequences = slots.shape[0]
 
-        def token_by_token(longest, from_tokens=1, below_tokens=1 << 30):
+        def token_by_token(longest, from_tokens=1, below_tokens=0):
             status = self._core.velox_linear_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
                                                   _ptr(beta) if delta else _P(0), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out), sequences, int(longest), int(heads),
                                                   int(kv_heads), int(dim), int(vdim), self._SCAN_RULES[rule], from_tokens, below_tokens, self._stream())
