@@ -115,6 +115,24 @@ def test_stream_update_and_norm(ops, ref, dtype, hidden, streams):
     near(a_res, b_res, 2e-6, "unweighted streams")
 
 
+@pytest.mark.parametrize("hidden,streams,parts", [(96, 4, 2), (70, 1, 3), (2048, 3, 8), (5000, 2, 5), (321, 8, 4)])
+def test_stream_update_with_a_term_in_parts(ops, hidden, streams, parts):
+    """A first term that comes as partial sums gives what their sum gives, added first to last (whole rows and chosen ones, both widths of loads)."""
+    g = torch.Generator().manual_seed(hidden)
+    tokens = 70
+    residual, term, other = rnd(g, tokens, streams * hidden), rnd(g, parts, tokens, hidden), rnd(g, tokens, hidden, dtype=torch.bfloat16)
+    mix, ow, iw, w = rnd(g, streams, streams), rnd(g, streams), rnd(g, streams), rnd(g, hidden)
+    whole = term[0].clone()
+    for part in term[1:]:
+        whole += part
+    for rows in (None, torch.tensor([5, 69, 0], dtype=torch.int32).cuda()):
+        for more, scales in ((), (0.8,)), ((other,), (0.8, 1.1)):
+            a_res, b_res = residual.clone(), residual.clone()
+            a = ops.stream_norm(a_res, (term, *more), scales, mix, ow, iw, w, 1e-6, streams, True, torch.float32, rows=rows)
+            b = ops.stream_norm(b_res, (whole, *more), scales, mix, ow, iw, w, 1e-6, streams, True, torch.float32, rows=rows)
+            near(a, b, 1e-6), near(a_res, b_res, 1e-6)  # (a product and a sum may be contracted in one build and not in the other)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_embedding_copies_and_gated_activation(ops, ref, dtype):
     g, dt = torch.Generator().manual_seed(3), DTYPES[dtype]

@@ -33,11 +33,14 @@ __device__ __forceinline__ float softplus_f32(float z) { return z > 20.f ? z : l
 //   u is kept in LDS between the passes (H floats).
 // ---------------------------------------------------------------------------------------------
 #define STREAMS_MAX 8
+#define STREAM_PARTS 8  // the most partial sums a term may come in
 struct StreamNormArgs {
   float* residual;
   const void* term0;
   const void* term1;
   int term0_bf16, term1_bf16, num_terms;
+  int parts;            // term0 is the sum of so many float32 parts, part_stride elements apart, added first to last
+  size_t part_stride;
   float scale0, scale1;
   const float* mix;
   const float* out_w;
@@ -78,7 +81,9 @@ __global__ void __launch_bounds__(256) stream_norm_kernel(const StreamNormArgs a
     for (int s = 0; s < STREAMS_MAX; ++s) x[s] = s < S ? res[(size_t)s * H + i] : 0.f;
     float u = 0.f;
     if (update) {
-      float y = a.scale0 * load_as_f32(a.term0, a.term0_bf16, src * H + i);
+      float y = load_as_f32(a.term0, a.term0_bf16, src * H + i);
+      for (int p = 1; p < a.parts; ++p) y += ((const float*)a.term0)[p * a.part_stride + src * H + i];
+      y *= a.scale0;
       if (a.num_terms > 1) y += a.scale1 * load_as_f32(a.term1, a.term1_bf16, src * H + i);
 #pragma unroll
       for (int t = 0; t < STREAMS_MAX; ++t) {
@@ -131,7 +136,7 @@ __device__ __forceinline__ void store4_from_f32(void* p, int is_bf16, size_t i, 
   *reinterpret_cast<short4_t*>((bf16_t*)p + i) = raw;
 }
 
-template <int PIECES>
+template <int PIECES, bool IN_PARTS = false>
 __global__ void __launch_bounds__(1024) stream_norm_vec_kernel(const StreamNormArgs a) {
   __shared__ float scratch[16];
   __shared__ float coef[STREAMS_MAX * STREAMS_MAX + 2 * STREAMS_MAX];
@@ -166,7 +171,17 @@ __global__ void __launch_bounds__(1024) stream_norm_vec_kernel(const StreamNormA
     for (int s = 0; s < STREAMS_MAX; ++s)
       if (s < S) x[s] = *reinterpret_cast<const float4_t*>(res + (size_t)s * H + i);
     if (update) {
-      float4_t y = a.scale0 * load4_as_f32(a.term0, a.term0_bf16, src * H + i);
+      float4_t y = load4_as_f32(a.term0, a.term0_bf16, src * H + i);
+      if (IN_PARTS) {  // the parts' loads all under way before the first is added
+        float4_t part[STREAM_PARTS - 1];
+#pragma unroll
+        for (int q = 1; q < STREAM_PARTS; ++q)
+          if (q < a.parts) part[q - 1] = *reinterpret_cast<const float4_t*>((const float*)a.term0 + q * a.part_stride + src * H + i);
+#pragma unroll
+        for (int q = 1; q < STREAM_PARTS; ++q)
+          if (q < a.parts) y += part[q - 1];
+      }
+      y *= a.scale0;
       if (a.num_terms > 1) y += a.scale1 * load4_as_f32(a.term1, a.term1_bf16, src * H + i);
 #pragma unroll
       for (int t = 0; t < STREAMS_MAX; ++t) {
@@ -208,12 +223,15 @@ __global__ void __launch_bounds__(1024) stream_norm_vec_kernel(const StreamNormA
   }
 }
 
-extern "C" int velox_stream_norm(float* residual, const void* term0, int term0_dtype, float scale0, const void* term1, int term1_dtype, float scale1,
+// term0_parts > 1: term0 holds so many float32 partial sums [term0_parts, tokens, hidden], part_stride = tokens * hidden.
+extern "C" int velox_stream_norm(float* residual, const void* term0, int term0_dtype, int term0_parts, long long part_stride, float scale0, const void* term1, int term1_dtype, float scale1,
                                  int num_terms, const float* mix, const float* out_w, const float* in_w, const float* weight, const int* rows,
                                  void* out, int out_dtype, int count, int hidden, int streams, int center, float eps, hipStream_t stream) {
   if (count <= 0) return 0;
-  if (streams < 1 || streams > STREAMS_MAX || hidden < 1 || hidden > 16384 || num_terms < 0 || num_terms > 2) return (int)hipErrorInvalidValue;
-  StreamNormArgs a{residual, term0, term1, term0_dtype == VELOX_BF16, term1_dtype == VELOX_BF16, num_terms, scale0, scale1, mix, out_w, in_w, weight,
+  if (streams < 1 || streams > STREAMS_MAX || hidden < 1 || hidden > 16384 || num_terms < 0 || num_terms > 2 || term0_parts < 1 || term0_parts > STREAM_PARTS ||
+      (term0_parts > 1 && term0_dtype != VELOX_F32))
+    return (int)hipErrorInvalidValue;
+  StreamNormArgs a{residual, term0, term1, term0_dtype == VELOX_BF16, term1_dtype == VELOX_BF16, num_terms, term0_parts, (size_t)part_stride, scale0, scale1, mix, out_w, in_w, weight,
                    rows, out, out_dtype == VELOX_BF16, hidden, streams, center, eps};
   const uintptr_t addresses = (uintptr_t)residual | (uintptr_t)weight | (uintptr_t)out | (uintptr_t)term0 | (uintptr_t)term1;
   if (hidden % 4 == 0 && addresses % 16 == 0) {  // (rows are a multiple of four elements, so their pieces are as aligned as the tensors)
@@ -221,7 +239,11 @@ extern "C" int velox_stream_norm(float* residual, const void* term0, int term0_d
     int lanes = (pieces + 63) / 64 * 64;
     if (lanes > 1024) lanes = 1024;
     const int per_lane = (pieces + lanes - 1) / lanes;
-    if (per_lane == 1) stream_norm_vec_kernel<1><<<count, lanes, 0, stream>>>(a);
+    if (a.parts > 1) {
+      if (per_lane == 1) stream_norm_vec_kernel<1, true><<<count, lanes, 0, stream>>>(a);
+      else if (per_lane == 2) stream_norm_vec_kernel<2, true><<<count, lanes, 0, stream>>>(a);
+      else stream_norm_vec_kernel<4, true><<<count, lanes, 0, stream>>>(a);
+    } else if (per_lane == 1) stream_norm_vec_kernel<1><<<count, lanes, 0, stream>>>(a);
     else if (per_lane == 2) stream_norm_vec_kernel<2><<<count, lanes, 0, stream>>>(a);
     else stream_norm_vec_kernel<4><<<count, lanes, 0, stream>>>(a);
     VELOX_RETURN_LAUNCH_STATUS();

@@ -161,7 +161,7 @@ class HipOps:
         c.velox_add_cast.argtypes = [_P, _P, _I, _P, ctypes.c_longlong, _P]
         c.velox_norm_add.argtypes = [_P, _P, _I, _P, _P, _I, _I, _F, _F, _I, ctypes.c_longlong, _P]
         c.velox_qk_norm_write.argtypes = [_P, _I, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _I, _I, _P]
-        c.velox_stream_norm.argtypes = [_P, _P, _I, _F, _P, _I, _F, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P]
+        c.velox_stream_norm.argtypes = [_P, _P, _I, _I, ctypes.c_longlong, _F, _P, _I, _F, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P]
         c.velox_embed_copies.argtypes = [_P, _P, _I, _P, _I, _I, _I, _F, _I, _P]
         c.velox_gated_act_mul.argtypes = [_P, _P, _I, _I, _I, _I, _P]
         c.velox_short_conv.argtypes = [_P, _I, _I, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P]
@@ -1098,11 +1098,12 @@ class HipOps:
 
     # -- residual streams, short convolution, linear recurrences ------------------------------------
     MAX_STREAMS = 8
+    MAX_STREAM_PARTS = 8  # partial sums that a term may come in
     MAX_STREAM_WIDTH = 16384
     MAX_CONV_TAPS = 8
 
     def stream_norm(self, residual, terms, scales, mix, out_weights, in_weights, weight, eps, streams, center, out_dtype, rows=None):
-        """``residual`` float32 ``[T, streams * H]``.  With ``terms`` (one or two ``[T, H]`` tensors, ``y = sum_i scales[i] terms[i]``):
+        """``residual`` float32 ``[T, streams * H]``.  With ``terms`` (one or two ``[T, H]`` tensors, the first also as float32 partial sums ``[S, T, H]``, ``y = sum_i scales[i] terms[i]``):
         ``x_t <- sum_s mix[s, t] x_s + out_weights[t] y`` for all streams at once (``mix`` None: the identity, ``out_weights``
         None: ones), in place unless ``rows`` picks rows.  Returns ``norm(sum_s in_weights[s] x_s) * weight`` in
         ``out_dtype``, for all rows or for ``rows``; ``center``: a layer norm without bias, else an RMS norm."""
@@ -1115,8 +1116,15 @@ class HipOps:
         self._check("weight", weight, torch.float32, (hidden,))
         if len(terms) > 2 or len(terms) != len(scales):
             raise KernelError("stream_norm: one or two terms, each with its scale")
+        parts = 1
         for i, term in enumerate(terms):
-            self._check(f"term {i}", term, None, (tokens, hidden))
+            if i == 0 and term.dim() == 3:
+                parts = term.shape[0]
+                if not 1 <= parts <= self.MAX_STREAM_PARTS:
+                    raise KernelError(f"stream_norm: a term in {parts} parts, at most {self.MAX_STREAM_PARTS}")
+                self._check("term 0", term, torch.float32, (parts, tokens, hidden))
+            else:
+                self._check(f"term {i}", term, None, (tokens, hidden))
         for name, t, shape in (("mix", mix, (streams, streams)), ("out_weights", out_weights, (streams,)), ("in_weights", in_weights, (streams,))):
             if t is not None:
                 self._check(name, t, torch.float32, shape)
@@ -1127,7 +1135,7 @@ class HipOps:
         t0 = terms[0] if len(terms) > 0 else None
         t1 = terms[1] if len(terms) > 1 else None
         status = self._core.velox_stream_norm(
-            _ptr(residual), _ptr(t0), _code(t0.dtype) if t0 is not None else 0, float(scales[0]) if t0 is not None else 0.0,
+            _ptr(residual), _ptr(t0), _code(t0.dtype) if t0 is not None else 0, parts, tokens * hidden, float(scales[0]) if t0 is not None else 0.0,
             _ptr(t1), _code(t1.dtype) if t1 is not None else 0, float(scales[1]) if t1 is not None else 0.0, len(terms),
             _ptr(mix), _ptr(out_weights), _ptr(in_weights), _ptr(weight), _ptr(rows), _ptr(out), _code(out_dtype), count, hidden, int(streams),
             int(bool(center)), float(eps), self._stream())

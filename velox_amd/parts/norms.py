@@ -97,8 +97,8 @@ class StreamNorm(Norm):
             if isinstance(y, ScaledSum):
                 terms, scales = tuple(y.terms), tuple(float(s) for s in y.scales)
             else:
-                if y.dim() == 3:
-                    y = y.sum(0)  # (float32 partial sums of a product)
+                if y.dim() == 3 and y.shape[1] <= 64:
+                    y = y.sum(0)  # (float32 partial sums of a product; those of more rows are added by the norm's kernel)
                 terms, scales = (y,), (1.0,)
         return ctx.ops.stream_norm(residual, terms, scales, update.mix if update is not None else None, update.out if update is not None else None,
                                    in_weights, self.weight, self.eps, self.streams, self.center, ctx.dtype, rows=rows)
