@@ -1029,11 +1029,14 @@ class HipOps:
         MI355X, product and norm (us, library / own, n x k):
 
         - tiles for a third of the compute units: 3,584 x 18,944 at 65 tokens 100 / 46, 300: 105 / 62, 700: 171 / 111; 1,024 x 28,672 at 150:
-          104 / 54; 4,096 x 11,008 at 65: 42 / 34, 512: 76 / 61; 2,048 x 10,944 at 65: 37 / 30; 2,560 x 10,240 at 65: 31 / 31.  Below 20 million
-          weights the library cuts the sum itself and wins up to a few hundred tokens: 2,048 x 8,448 at 65: 25 / 25, 128: 26 / 29, 300: 39 / 30,
-          1,036: 73 / 57; 1,536 x 8,960 at 128: 23 / 28, 512: 34 / 33, 1,036: 53 / 48; 2,048 x 7,168 at 256: 26 / 27, 400: 34 / 29; 1,024 x 8,192 at
-          400: 28 / 28, 640: 31 / 29; 512 x 16,384 at 256: 25 / 36, 640: 46 / 37; 256 x 12,288 at 640: 27 / 30, 1,280: 37 / 31.  Shorter sums
-          stay with it: 2,048 x 5,632 at 300: 25 / 25, 512: 26 / 29, 836: 38 / 38, 1,036: 46 / 44.
+          104 / 54; 4,096 x 11,008 at 65: 42 / 34, 512: 76 / 61; 2,048 x 10,944 at 65: 37 / 30; 2,560 x 10,240 at 65: 31 / 31; 4,096 x 5,120 at
+          100: 25 / 25, 512: 45 / 41.  Below 20 million weights the library cuts the sum itself and is 2 to 5 us quicker with few rows:
+          2,048 x 8,448 at 128: 26 / 29, 150: 32 / 27, 1,036: 73 / 57; 1,536 x 8,960 at 128: 23 / 28, 150: 23 / 28, 200: 30 / 28, 1,036: 53 / 48;
+          2,048 x 7,168 at 150: 25 / 24, 400: 28 / 30, 700: 43 / 39; 2,048 x 5,632 at 128: 18 / 22, 150: 21 / 23, 300: 24 / 25, 512: 26 / 29, 700: 34 /
+          34, 1,280: 47 / 47; 1,024 x 8,192 at 200: 21 / 26, 300: 27 / 27, 1,000: 34 / 33.  Its call costs the host 19 us, though, and the own one
+          8, and a step of portions through a model of that size waits for the host up to some 500 rows (width 2,048, ff 5,632, 140 tokens:
+          2,260 to 2,390 us a step by the library, 2,190 to 2,360 with the own tiles, four runs each).  So: the own ones above 128 rows, where steps are not captured.  Smaller
+          still: 1,024 x 5,632 at 512: 22 / 27; 512 x 16,384 at 400: 33 / 36; 256 x 12,288 at 640: 27 / 30.
         - more tiles, up to one per compute unit, and sums so long that the library is far from its rate: 3,584 x 18,944 at 836: 182 / 153,
           1,536: 283 / 233, 2,048: 381 / 287; 4,096 x 16,512 at 700: 197 / 128, 2,048: 376 / 273; 5,120 x 27,648 at 836: 335 / 294, 1,536: 558 /
           428; but 3,072 x 12,288 at 1,036: 112 / 104, 1,536: 138 / 144; 5,120 x 13,824 at 836: 156 / 158, 1,536: 211 / 227.  Wide products
@@ -1041,13 +1044,13 @@ class HipOps:
           512: 170 / 155, 640 (160): 192 / 203; 16,384 x 16,384 at 256 (128): 242 / 226, 400 (256): 278 / 298; 6,144 x 24,576 at 900 (192):
           399 / 310, 6,144 x 16,384 at 1,280 (240): 245 / 268; 7,168 x 28,672 at 900 (224): 499 / 413, 1,100 (252): 426 / 466.
 
-        (Residual streams add the parts in a pass of their own: 4,096 x 11,008 at 128 rows 65 / 46, 512: 85 / 77; 2,048 x 8,448 at 300: 43 / 38,
-        836: 66 / 61; 1,536 x 8,960 at 512: 38 / 42.)"""
-        if m <= 64 or k % 8 != 0 or n % 4 != 0:
+        (With residual streams, whose norm adds the parts too: 4,096 x 11,008 at 100 rows 45 / 39, 512: 87 / 72; 2,048 x 8,448 at 300: 43 / 34;
+        2,048 x 5,632 at 300: 28 / 29, 512: 32 / 34, 1,280: 63 / 58.)"""
+        if m <= 64 or k < 5120 or k % 8 != 0 or n % 4 != 0:
             return 0
         tiles, steps = -(-m // 128) * -(-n // 256), -(-k // 64)
         if 3 * tiles <= self.num_cus:
-            if k < 7168 or (n * k < 20_000_000 and m * n * k < 4_500_000_000):
+            if n * k < 20_000_000 and (n < 1024 or n * k < 8_000_000 or m <= 128):
                 return 0
             splits = min(8, self.num_cus // tiles)
         elif k >= 16384 and tiles <= (self.num_cus if n < 6144 else 7 * self.num_cus // 8 if n < 8192 else self.num_cus // 2):
