@@ -399,12 +399,18 @@ static void linear_chunk_launch(const LinearChunkArgs& a, int tokens, hipStream_
   else linear_chunk_scan_kernel<8, DELTA><<<grid, 512, 0, stream>>>(a);
 }
 
-// The sequences of at least `long_from` tokens.  beta: nullptr for the additive rule.  `scratch` holds the records of `heads_at_once`
+extern "C" int velox_linear_scan(const float* qk, const void* v, int v_dtype, int v_ld, int v_at, const float* decay, int decay_per_channel, const float* beta,
+                                 float* state, const int* slots, const int* cu_q, float* out, int num_seqs, int max_q_len, int heads, int kv_heads, int dim,
+                                 int vdim, int rule, int from_tokens, int below_tokens, hipStream_t stream);
+
+// The sequences of at least `long_from` tokens, then the shorter ones token by token: `shorter` says which kernels they may need (0: there
+// are none, 1: single tokens and pairs, 2: longer ones too).  Launched from here, since a call costs the host more than a launch.
+// beta: nullptr for the additive rule.  `scratch` holds the records of `heads_at_once`
 // heads (velox_linear_chunk_scratch_elems each), which are worked one such group after the other.  qk and a decay per channel are
 // read in 16-byte pieces (dim is a multiple of 16; the caller checks that the bases are aligned).
 extern "C" int velox_linear_chunk_scan(const float* qk, const void* v, int v_dtype, int v_ld, int v_at, const float* decay, int decay_per_channel,
                                        const float* beta, float* scratch, float* state, const int* slots, const int* cu_q, float* out, int num_seqs,
-                                       int tokens, int long_from, int heads_at_once, int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
+                                       int tokens, int long_from, int shorter, int heads_at_once, int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
   if (num_seqs <= 0 || tokens <= 0) return 0;
   if (velox_linear_chunk_scratch_elems(tokens, num_seqs, dim, vdim) == 0 || heads < 1 || heads > 65535 || num_seqs > 65535 || heads_at_once < 1 ||
       (long long)records_of_step(tokens, num_seqs) * (heads_at_once < heads ? heads_at_once : heads) > (1 << 23) || vdim > 65535 * 16 || kv_heads < 1 ||
@@ -416,5 +422,13 @@ extern "C" int velox_linear_chunk_scan(const float* qk, const void* v, int v_dty
     if (beta) linear_chunk_launch<true>(a, tokens, stream);
     else linear_chunk_launch<false>(a, tokens, stream);
   }
-  VELOX_RETURN_LAUNCH_STATUS();
+  const int status = (int)hipGetLastError();
+  if (status != 0 || shorter == 0) return status;
+  auto token_by_token = [&](int longest, int from, int below) {
+    return velox_linear_scan(qk, v, v_dtype, v_ld, v_at, decay, decay_per_channel, beta, state, slots, cu_q, out, num_seqs, longest, heads, kv_heads, dim, vdim, beta ? 1 : 0, from,
+                             below, stream);
+  };
+  // (1: what is neither long nor a single token or a pair can only be there beside empty sequences, and this kernel takes it too)
+  const int singles = token_by_token(1, 1, shorter == 1 ? long_from : 3);
+  return singles != 0 || shorter == 1 ? singles : token_by_token(3, 3, long_from);
 }

@@ -191,7 +191,7 @@ class HipOps:
         c.velox_gemm_f32_tile.restype = _I
         c.velox_gemm_tiles_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P]
         c.velox_gemm_tiles_bf16.restype = _I
-        c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
+        c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         c.velox_linear_chunk_scan.restype = _I
         c.velox_linear_chunk_scratch_elems.argtypes = [_I, _I, _I, _I]
         c.velox_linear_chunk_scratch_elems.restype = ctypes.c_longlong
@@ -1392,13 +1392,6 @@ class HipOps:
         self.linear_scan_supports(dim, vdim)
         out = torch.empty((tokens, heads * vdim), dtype=torch.float32, device=self.device)
         sequences = slots.shape[0]
-
-        def token_by_token(longest, from_tokens=1, below_tokens=0):
-            status = self._core.velox_linear_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
-                                                  _ptr(beta) if delta else _P(0), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out), sequences, int(longest), int(heads),
-                                                  int(kv_heads), int(dim), int(vdim), self._SCAN_RULES[rule], from_tokens, below_tokens, self._stream())
-            self._launched(status, "linear_scan")
-
         long_from = 1 if chunked else self.LINEAR_CHUNK_TOKENS
         per_head = 0
         if rule != "removal" and chunked is not False and max_q_len >= long_from:
@@ -1406,22 +1399,19 @@ class HipOps:
         if per_head == 0:
             if chunked:
                 raise KernelError(f"linear_scan: heads of {dim} channels (rule {rule!r}) are not the chunked kernels'")
-            token_by_token(max_q_len)
+            status = self._core.velox_linear_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
+                                                  _ptr(beta) if delta else _P(0), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out), sequences, int(max_q_len), int(heads),
+                                                  int(kv_heads), int(dim), int(vdim), self._SCAN_RULES[rule], 1, 0, self._stream())
+            self._launched(status, "linear_scan")
             return out
+        # What may be beside the long portions: nothing if all are as long as the longest; single tokens and pairs; longer ones too if the
+        # number of tokens leaves room for one.
+        shorter = 0 if long_from == 1 or tokens == sequences * max_q_len else 1 if tokens - max_q_len == sequences - 1 else 2
         heads_at_once = max(1, min(int(heads), self.LINEAR_CHUNK_SCRATCH // per_head))
         scratch = torch.empty(per_head * heads_at_once, dtype=torch.float32, device=self.device)
         self._launched(self._core.velox_linear_chunk_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
-                                                          _ptr(beta) if delta else _P(0), _ptr(scratch), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out),
-                                                          sequences, tokens, long_from, heads_at_once, int(heads), int(kv_heads), int(dim), int(vdim), self._stream()),
-                       "linear_chunk_scan")
-        if long_from > 1 and tokens != sequences * max_q_len:  # (some sequence is shorter than the longest)
-            # What is beside the long portions: single tokens and pairs, and longer ones if the number of tokens leaves room for one.  (If
-            # it leaves none, no sequence lies between, or empty ones make up for it and this kernel takes all.)
-            if tokens - max_q_len == sequences - 1:
-                token_by_token(1, below_tokens=long_from)
-            else:
-                token_by_token(1, below_tokens=3)
-                token_by_token(3, from_tokens=3, below_tokens=long_from)
+                                                          _ptr(beta) if delta else _P(0), _ptr(scratch), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out), sequences, tokens,
+                                                          long_from, shorter, heads_at_once, int(heads), int(kv_heads), int(dim), int(vdim), self._stream()), "linear_chunk_scan")
         return out
 
     def gated_head_norm(self, read, weight, eps, gate_source, gate_at, gate_kind, heads, vdim, out_dtype):
