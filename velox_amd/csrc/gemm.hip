@@ -5,7 +5,8 @@
 // weights a checkpoint stores in float32), float32 rows that are not whole 16-byte pieces and sums of
 // fewer than GEMM_FOLD terms; other float32 products run on the float32 matrix instructions (gemm_mfma_f32_kernel), so a float32 run
 // never touches a reduced-precision matrix mode.  Each output element is summed over k in one fixed
-// order by one thread, so a row's result does not depend on the other rows of the batch.  The sum
+// order by one thread, so a row's result does not depend on what the other rows of the batch hold (their number chooses the
+// kernel: up to 16 rows have one of their own, with an order of its own).  The sum
 // is built from sums of GEMM_FOLD consecutive terms, each started at zero: the rounding error of a
 // long sum (the down projection adds 18944 terms) then grows with the square roots of the two
 // lengths and not with that of their product, which keeps the float32 path as close to the exact
