@@ -33,6 +33,20 @@ def test_whole_then_decode_matches_plain(tmp_path, ops, name, dtype):
     torch.testing.assert_close(got, expected, **TOL[dtype])
 
 
+def test_a_float32_model_whose_products_all_run_on_the_matrix_instructions(tmp_path, ops):
+    """Sums of 128 terms and more in portions of more than 16 tokens: every product of a width of 160 takes the float32 matrix
+    instructions, which the widths above reach in an output or second feed-forward product at most.  Single tokens behind the
+    portions take the kernel for few rows, on the same cache."""
+    from velox_amd.weights import write_random_model
+
+    folder = write_random_model({**CONFIGS["B"], "hidden_size": 160, "num_attention_heads": 5, "intermediate_size": 388}, str(tmp_path / "wide"), 4, dtype="float32")
+    config, weights = read_model_folder(folder)
+    tokens = random_tokens(config["vocab_size"], 150, seed=9)
+    h = Harness(folder, ops, torch.float32, "cuda", PAGE_SIZE["B"], num_pages=64)
+    got = [h.feed([("a", tokens[lo:hi], list(range(hi - lo)))]) for lo, hi in ((0, 17), (17, 146), (146, 147), (147, 148), (148, 150))]
+    torch.testing.assert_close(torch.cat(got), qwen2_logits(config, weights, tokens), **TOL[torch.float32])
+
+
 @pytest.mark.parametrize("name", ["A", "B", "C"])
 def test_the_cache_holds_the_first_layers_rotated_keys_and_values(tmp_path, ops, name):
     """What the pages hold, read back in sequence order (``CacheManager.gather_sequence``): layer 0's keys with bias and
