@@ -1358,6 +1358,66 @@ def test_products_in_tiles_with_a_cut_sum(ops, m, n, k, splits):
     assert parts.shape == (splits, m, n) and torch.all((parts.double().sum(0) - want).abs() <= k * 2.0 ** -24 * size + 1e-6)
 
 
+TILES = (128128, 128192, 128256, 192192, 192256, 256192, 256256)
+
+
+@pytest.mark.parametrize("m, n, k", [(1, 8, 8), (129, 260, 200), (65, 64, 64), (193, 264, 128), (257, 520, 192), (1030, 1544, 448), (3000, 6152, 320)])
+def test_products_in_every_tile(ops, m, n, k):
+    """Remainders in all sizes, odd numbers of steps, sums shorter than the loads are ahead, more tiles than workgroups.  Against float64 as
+    above, the bias one more float32 addition; every tile has the same bits and writes nothing else."""
+    generator = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w, bias = (torch.randn(*shape, generator=generator, device="cuda") for shape in ((m, k), (n, k), (n,)))
+    a, w = a.bfloat16(), w.bfloat16()
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    first = None
+    for tile in TILES if k % 64 == 0 else (128256, 0):
+        plain = ops.gemm_tiles(a, w, tile=tile)
+        biased = ops.gemm_tiles(a, w, bias=bias, tile=tile)
+        parts = ops.gemm_tiles(a, w, 3, torch.float32, tile=tile)
+        assert torch.all((plain.double() - want).abs() <= k * 2.0 ** -24 * size + 2.0 ** -8 * 1.01 * want.abs() + 1e-6)
+        exact = want + bias.double()
+        assert torch.all((biased.double() - exact).abs() <= (k + 2) * 2.0 ** -24 * (size + bias.double().abs()) + 2.0 ** -8 * 1.01 * exact.abs() + 1e-6)
+        assert torch.all((parts.double().sum(0) - want).abs() <= k * 2.0 ** -24 * size + 1e-6)
+        first = first or (plain, biased, parts)
+        assert all(torch.equal(x, y) for x, y in zip(first, (plain, biased, parts)))
+        held = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device="cuda")
+        assert ops._core.velox_tiles_bf16(a.data_ptr(), w.data_ptr(), None, held.data_ptr(), m, n, k, 1, 1, tile, ops._stream()) == 0
+        assert torch.equal(held[:m], plain) and torch.all(held[m] == 7.0)
+
+
+@pytest.mark.parametrize("activation", ["silu", "relu"])
+@pytest.mark.parametrize("m, n, k", [(65, 8, 64), (129, 132, 200), (193, 136, 128), (257, 264, 192), (1030, 776, 448), (2100, 3080, 320)])
+def test_gated_products_in_every_tile(ops, m, n, k, activation):
+    """The product's own bits, then the activation in float32 (an exponential and a reciprocal, each within 2^-23) and one rounding; rows with
+    infinities and NaN give what the kernel behind a product gives."""
+    a, w = rand((m, k), torch.bfloat16, m), rand((2 * n, k), torch.bfloat16, n, 3 * k ** -0.5)
+    a[m // 2, 3] = float("inf")
+    a[m - 1, 5] = float("nan")
+    product = ops.gemm_tiles(a, w)
+    g, u = product[:, :n].double(), product[:, n:].double()
+    want = (g * torch.sigmoid(g) if activation == "silu" else g.clamp(min=0)) * u
+    behind = ops.silu_mul(product) if activation == "silu" else ops.gated_act_mul(product, activation)
+    for tile in TILES if k % 64 == 0 else (128256, 0):
+        got = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device="cuda")
+        assert ops._core.velox_tiles_glu_bf16(a.data_ptr(), w.data_ptr(), got.data_ptr(), m, n, k, 0 if activation == "silu" else 2, tile, ops._stream()) == 0
+        finite = torch.isfinite(want)
+        assert torch.all(got[m] == 7.0) and torch.equal(torch.isnan(got[:m]), torch.isnan(behind)) and torch.equal(torch.isinf(got[:m]), torch.isinf(behind))
+        error = (got[:m].double() - want).abs() - (2.0 ** -8 * 1.01 + g.abs() * 2.0 ** -22) * want.abs() - 1e-30
+        assert torch.all(error[finite] <= 0)
+
+
+@pytest.mark.parametrize("m, n, k, own", [(64, 4096, 2048, False), (65, 4096, 2048, True), (300, 4608, 3584, False), (836, 37888, 3584, True), (836, 4608, 3584, True), (1036, 64, 2048, True),
+                                          (1036, 56, 2048, False), (1036, 4100, 2048, False), (1036, 4096, 2056, False), (1036, 4096, 192, False)])
+def test_which_products_run_in_the_own_tiles(ops, monkeypatch, m, n, k, own):
+    calls = []
+    monkeypatch.setattr(ops, "gemm_tiles", lambda *a, **more: calls.append(a) or type(ops).gemm_tiles(ops, *a, **more))
+    x, w, bias = rand((m, k), torch.bfloat16, 1), rand((n, k), torch.bfloat16, 2, k ** -0.5), rand((n,), torch.float32, 3)
+    got = ops.linear(x, w, bias, torch.bfloat16)
+    assert ops.tiles_serve(m, n, k) == own and len(calls) == int(own) and ops.library_serves(m, n, k) == (m > 64 and not own)
+    want = x.double() @ w.double().T + bias.double()
+    assert torch.all((got.double() - want).abs() <= 2.0 ** -7 * (want.abs() + bias.double().abs()) + k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T))
+
+
 @pytest.mark.parametrize("m, n, k, parts", [(65, 2560, 8192, 8), (300, 2048, 8448, 8), (700, 2048, 5632, 5), (700, 1024, 28672, 8), (300, 4096, 16512, 5), (129, 8192, 16384, 4)])
 def test_linear_with_parts_of_a_long_sum_into_every_consumer(ops, ref, m, n, k, parts):
     """More than 64 rows of a long product come back as partial sums.  Each kernel that takes them gives what it gives for their float32

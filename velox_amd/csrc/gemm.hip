@@ -12,7 +12,7 @@
 // lengths and not with that of their product, which keeps the float32 path as close to the exact
 // result as a blocked library product on a CPU is.
 #include "common.h"
-#include "grouped_mfma.h"
+#include "tiles_mfma.h"
 
 #define GEMM_BM 64
 #define GEMM_BN 64
@@ -399,26 +399,47 @@ extern "C" int velox_gemm_fma(const void* a, const void* w, const float* bias, v
   VELOX_RETURN_LAUNCH_STATUS();
 }
 
-// out[M, N] (bfloat16, or float32 partial sums [splits, M, N] of `splits` parts of k) = A[M, K] * W[N, K]^T, bfloat16, in the tiles of the
-// experts' products (grouped_tiles_kernel).  Needs k % 8 == 0, n % 4 == 0 and 16-byte aligned bases.
-extern "C" int velox_gemm_tiles_bf16(const void* a, const void* w, void* out, int m, int n, int k, int splits, int out_dtype, hipStream_t stream) {
+// out[M, N] (bfloat16, + bias; or float32 partial sums [splits, M, N] of `splits` parts of k) = A[M, K] * W[N, K]^T, bfloat16, in tiles_mfma.h's tiles of
+// `tile` = rows * 1,000 + columns (0: the one that tiles_pick takes).  Needs k % 8 == 0, n % 4 == 0 and 16-byte aligned bases; k % 64 != 0 has 128 x 256 alone.
+extern "C" int velox_tiles_bf16(const void* a, const void* w, const float* bias, void* out, int m, int n, int k, int splits, int out_dtype, int tile, hipStream_t stream) {
   if (m <= 0 || n <= 0) return 0;
-  if (k < 1 || k % 8 != 0 || n % 4 != 0 || splits < 1 || (out_dtype == VELOX_BF16 && splits != 1) || (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) != 0) return -1;
-  GroupedArgs args = {};
+  if (k < 1 || k % 8 != 0 || n % 4 != 0 || splits < 1 || (splits != 1 && (out_dtype == VELOX_BF16 || bias != nullptr)) ||
+      (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) != 0 || !tiles_fit(256, k, 256, k))
+    return -1;
+  TileArgs args = {};
+  args.a = (const bf16_t*)a;
+  args.a_ld = k;
+  args.w = (const bf16_t*)w;
+  args.bias = bias;
+  args.out = out;
+  args.m = m;
+  args.n = n;
+  args.k = k;
+  args.splits = splits;
+  if (tile == 0) tile = tiles_pick(m, n, k, splits);
+  if (k % 64 == 0) return out_dtype == VELOX_BF16 ? tiles_launch<TL_PLAIN, bf16_t, false>(args, tile, stream) : tiles_launch<TL_PLAIN, float, false>(args, tile, stream);
+  return out_dtype == VELOX_BF16 ? tiles_launch<TL_PLAIN, bf16_t, true>(args, tile, stream) : tiles_launch<TL_PLAIN, float, true>(args, tile, stream);
+}
+
+// out[M, N] = act(A Wgate^T) * (A Wup^T) in bfloat16 for W = [Wgate; Wup] [2 N, K], both sums rounded to bfloat16 in front of it; act 0: SiLU, 2: the
+// rectifier (the tanh form of GELU stays a kernel of its own: its tangent costs more than the pass).
+extern "C" int velox_tiles_glu_bf16(const void* a, const void* w, void* out, int m, int n, int k, int act, int tile, hipStream_t stream) {
+  if (m <= 0 || n <= 0) return 0;
+  if (k < 1 || k % 8 != 0 || n % 4 != 0 || (act != 0 && act != 2) || (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) != 0 || !tiles_fit(256, k, n + 256LL, k)) return -1;
+  TileArgs args = {};
   args.a = (const bf16_t*)a;
   args.a_ld = k;
   args.w = (const bf16_t*)w;
   args.out = out;
-  args.out_ld = n;
+  args.m = m;
   args.n = n;
   args.k = k;
-  args.m = m;
-  args.splits = splits;
-  const int cols = (n + GM_TILE_COLS - 1) / GM_TILE_COLS;
-  const long long tiles = (long long)((m + GM_TILE_ROWS - 1) / GM_TILE_ROWS) * cols * splits;
-  if (tiles > (1 << 30)) return -1;
-  const int workgroups = (int)((tiles + GM_XCDS - 1) / GM_XCDS * GM_XCDS);
-  if (out_dtype == VELOX_BF16) grouped_tiles_kernel<GM_PLAIN, bf16_t><<<workgroups, 512, 0, stream>>>(args, cols);
-  else grouped_tiles_kernel<GM_PLAIN, float><<<workgroups, 512, 0, stream>>>(args, cols);
-  VELOX_RETURN_LAUNCH_STATUS();
+  args.splits = 1;
+  if (tile == 0) tile = tiles_pick(m, 2LL * n, k, 1);
+  if (act == 0) return k % 64 == 0 ? tiles_launch<TL_SILU, bf16_t, false>(args, tile, stream) : tiles_launch<TL_SILU, bf16_t, true>(args, tile, stream);
+  return k % 64 == 0 ? tiles_launch<TL_RELU, bf16_t, false>(args, tile, stream) : tiles_launch<TL_RELU, bf16_t, true>(args, tile, stream);
 }
+
+// The tile that a product of m rows with w_rows x k takes, as rows * 1,000 + columns (an entry point so that a test can tell).
+extern "C" int velox_tiles_pick(int m, int w_rows, int k, int splits) { return tiles_pick(m, w_rows, k, splits); }
+extern "C" int velox_tiles_splits(int m, int n, int k, int most) { return tiles_splits(m, n, k, most); }

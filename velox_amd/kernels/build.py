@@ -25,7 +25,7 @@ ARCH = "gfx950"
 FLAGS = ["-O3", f"--offload-arch={ARCH}", "-shared", "-fPIC", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 CORE_SOURCES = ["elementwise.hip", "gemm.hip", "skinny_gemm.hip", "latent.hip", "routed.hip", "normed.hip", "recurrent.hip", "removal.hip", "linear_chunk.hip", "state_space.hip", "gated.hip", "sampling.hip", "probe.hip"]
 ATTENTION_SOURCES = ["attention.hip"]
-HEADERS = ["common.h", "no_alloc.h", "grouped_mfma.h"]
+HEADERS = ["common.h", "no_alloc.h", "grouped_mfma.h", "tiles_mfma.h"]
 # head sizes built ahead of time by build_all(); any other multiple of 16 up to 256 is built at first use
 DEFAULT_HEAD_DIMS = (16, 32, 48, 64, 80, 96, 128, 192, 256)
 # the same kernels with a bias by distance on the scores (``attnbias_d<N>``), built ahead of time for these head sizes

@@ -189,8 +189,11 @@ class HipOps:
         c.velox_removal_chunk_scan.restype = _I
         c.velox_gemm_f32_tile.argtypes = [_I, _I]
         c.velox_gemm_f32_tile.restype = _I
-        c.velox_gemm_tiles_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P]
-        c.velox_gemm_tiles_bf16.restype = _I
+        c.velox_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]
+        c.velox_tiles_glu_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P]
+        c.velox_tiles_pick.argtypes = c.velox_tiles_splits.argtypes = [_I, _I, _I, _I]
+        for fn in (c.velox_tiles_bf16, c.velox_tiles_glu_bf16, c.velox_tiles_pick, c.velox_tiles_splits):
+            fn.restype = _I
         c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         c.velox_linear_chunk_scan.restype = _I
         c.velox_linear_chunk_scratch_elems.argtypes = [_I, _I, _I, _I]
@@ -291,7 +294,7 @@ class HipOps:
         if not self.use_library_gemm:
             return False
         if m > 64:
-            return True
+            return not self.tiles_serve(m, n, k) and self.tile_splits(m, n, k) == 0
         return m > 16 and n > 8192 and n * k >= (32 << 20)
 
     def tuning_file(self) -> Optional[str]:
@@ -805,6 +808,9 @@ class HipOps:
             splits = self.tile_splits(m, n, k)
             if (splits == 1 or (splits > 1 and partials_ok)) and not self._library_has_timed(m, n, k):
                 return self.gemm_tiles(x, weight, splits, torch.bfloat16 if splits == 1 else torch.float32)
+        if (out_dtype == torch.bfloat16 and self.use_library_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+                and self.tiles_serve(m, n, k) and not self._library_has_timed(m, n, k)):
+            return self.gemm_tiles(x, weight, bias=bias)
         skinny_rows = 16 if n > 8192 else 32  # measured on MI355X: beyond this the library's kernels stream faster
         if self.use_skinny_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and m <= skinny_rows and k % 64 == 0:
             return self.skinny_gemm(x, weight, bias, out_dtype, packed=packed, x_packed=self._packed_rows_of(x, k))
@@ -976,6 +982,16 @@ class HipOps:
             self._launched(self._core.velox_skinny_glu_rows_bf16(_ptr(x), _ptr(packed), _ptr(out), m, n, k, per_group if pairs is None else int(pairs), self._stream()),
                            "skinny_glu_rows")
             return out
+        if (not fused and activation != "gelu_tanh" and deferred is None and self.use_library_gemm and x.dim() == 2 and gate_up_weight.dim() == 2 and two_n % 16 == 0
+                and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16 and out_dtype == torch.bfloat16 and gate_up_weight.shape[1] == k
+                and (two_n // 2 + 256) * k < 1 << 30 and self.tiles_serve(m, two_n, k) and not self._library_has_timed(m, two_n, k)):
+            # many rows: the activation where the tiles' sums are finished.  Both sums are rounded to bfloat16 in front of it, as a
+            # product of its own leaves them
+            self._check("x", x, align=16)
+            self._check("gate_up_weight", gate_up_weight, align=16)
+            out = torch.empty((m, two_n // 2), dtype=torch.bfloat16, device=self.device)
+            self._launched(self._core.velox_tiles_glu_bf16(_ptr(x), _ptr(gate_up_weight), _ptr(out), m, two_n // 2, k, self._GATED_ACTIVATIONS[activation], 0, self._stream()), "tiles_glu")
+            return out
         if not fused:
             product = self.linear(deferred if deferred is not None else x, operand, None, out_dtype)
             return self.silu_mul(product) if activation == "silu" else self.gated_act_mul(product, activation)
@@ -1054,10 +1070,22 @@ class HipOps:
                 return 0
             splits = min(8, self.num_cus // tiles)
         elif k >= 16384 and tiles <= (self.num_cus if n < 6144 else 7 * self.num_cus // 8 if n < 8192 else self.num_cus // 2):
-            splits = min((1, 2, 3, 4), key=lambda s: -(-tiles * s // self.num_cus) * -(-steps // s))
+            splits = self._core.velox_tiles_splits(m, n, k, 4)
         else:
             return 0
         return -(-steps // -(-steps // splits))  # (no empty part)
+
+    def tiles_serve(self, m: int, n: int, k: int) -> bool:
+        """Whether a whole bfloat16 product of more than 64 rows runs in the framework's own tiles (``gemm_tiles``; the tile is picked in
+        tiles_mfma.h).  The library is left what has few tiles of 128 x 128 and a sum of more than 2,048 terms, where it cuts the
+        sum: 300 rows of 4,608 x 3,584 (108 tiles) 22 us by the library and 25 here, 512 of 4,096 x 4,096 (128) 30 / 33, 836 of 2,048 x
+        5,632 (112) 34 / 41.  Elsewhere, of 27 shapes from 1,536 x 1,536 to 37,888 x 3,584 at 16 numbers of rows, the own tiles took
+        0.90 of the library's time on average and 1.17 at worst, and their call costs the host 8 us instead of 19: 836 rows of 37,888 x
+        3,584 268 / 198, 2,048 535 / 409; 4,001 of 22,016 x 4,096 640 / 530, of 4,096 x 4,096 90 / 91; 1,036 of 10,368 x 2,048 49 / 38; 2,048 of
+        4,608 x 3,584 56 / 56."""
+        if m <= 64 or n % 8 != 0 or n < 64 or k % 64 != 0 or k < 256:
+            return False
+        return k <= 2048 or -(-m // 128) * -(-n // 128) * 4 >= 3 * self.num_cus
 
     @staticmethod
     def _library_has_timed(m: int, n: int, k: int) -> bool:
@@ -1071,14 +1099,17 @@ class HipOps:
         size = f"tn_{n}_{m}_{k}_"
         return tunable.tuning_is_enabled() or any(r[0] == "GemmTunableOp_BFloat16_TN" and r[1].startswith(size) for r in tunable.get_results())
 
-    def gemm_tiles(self, x, weight, splits: int = 1, out_dtype=torch.bfloat16):
-        """``x @ weight^T`` in bfloat16 in tiles of 128 x 256: [M, N] in bfloat16, or float32 partial sums [splits, M, N]."""
+    def gemm_tiles(self, x, weight, splits: int = 1, out_dtype=torch.bfloat16, bias: Optional[torch.Tensor] = None, tile: int = 0):
+        """``x @ weight^T (+ bias)`` in bfloat16 in large tiles: [M, N] in bfloat16, or float32 partial sums [splits, M, N].  ``tile``: rows * 1,000 +
+        columns of a tile (0: the one that suits the sizes)."""
         self._check("x", x, torch.bfloat16, align=16)
         self._check("weight", weight, torch.bfloat16, (weight.shape[0], x.shape[1]), align=16)
         m, k = x.shape
         n = weight.shape[0]
+        if bias is not None:
+            self._check("bias", bias, torch.float32, (n,))
         out = torch.empty((m, n) if out_dtype == torch.bfloat16 else (splits, m, n), dtype=out_dtype, device=self.device)
-        self._launched(self._core.velox_gemm_tiles_bf16(_ptr(x), _ptr(weight), _ptr(out), m, n, k, int(splits), _code(out_dtype), self._stream()), "gemm_tiles")
+        self._launched(self._core.velox_tiles_bf16(_ptr(x), _ptr(weight), _ptr(bias), _ptr(out), m, n, k, int(splits), _code(out_dtype), int(tile), self._stream()), "gemm_tiles")
         return out
 
     def gemm_fma(self, x, weight, bias, out_dtype):
