@@ -8,7 +8,7 @@ import pytest
 from velox_amd.kernels import build
 
 
-@pytest.mark.parametrize("source", ["gemm.hip"])
+@pytest.mark.parametrize("source", ["gemm.hip", "routed.hip"])
 def test_nothing_moves_an_accumulator_between_matrix_instructions(source, tmp_path):
     """The matrix instructions are assembly to the compiler, so it does not wait for one before it moves the register that the instruction
     still writes: between the first and the last of a kernel there must be no such move, no spilled register and no branch target but the loop's."""

@@ -1,6 +1,6 @@
 // Many small bfloat16 products in one launch on the matrix cores of gfx950: a product per group (an expert, a head), each
-// over its own rows, out[r, g, :] = W_g a[r, g, :].  Shared by the routed experts, by the per-head products of
-// attention over a latent and by single products whose sum is long and whose tiles are few (velox_gemm_tiles_bf16).
+// over its own rows, out[r, g, :] = W_g a[r, g, :].  Shared by the routed experts and the per-head products of
+// attention over a latent.
 //
 // A workgroup of four waves of the kernel without a plan owns 64 rows and 64 NT output columns of one group (NT = 2 or 4 tiles of W
 // per wave); a wave owns 16 NT of the columns and all 64 rows: 4 NT 16x16 accumulators.  W comes straight from global memory in the layout of
@@ -16,6 +16,7 @@
 // aligned bases.
 #pragma once
 #include "common.h"
+#include "tiles_mfma.h"
 
 typedef __bf16 gm_bf16x8_t __attribute__((ext_vector_type(8)));
 
@@ -32,8 +33,8 @@ struct GroupedArgs {
   void* out;           // element (row r, group g, col) at out[r * out_ld + g * out_group + col]
   long long out_ld, out_group;
   int n, k;
-  // rows: either every group runs rows [0, m) (plan == nullptr; grouped_mfma_kernel: blockIdx.y = row tile, blockIdx.z = group;
-  // grouped_tiles_kernel: one group), or the plan's tiles say which group runs which rows
+  // rows: either every group runs rows [0, m) (plan == nullptr: blockIdx.y = row tile, blockIdx.z = group), or the plan's tiles say
+  // which group runs which rows
   int m;
   const int* plan;
   int plan_pairs, plan_groups, plan_max_tiles;
@@ -41,7 +42,6 @@ struct GroupedArgs {
   long long gate_ld, gate_group, gate_col;
   int act = 0;         // GM_ACT: the result goes through ungated_act(., act)
   const float* row_scale;  // grouped_mfma_few_rows_kernel: row r of `a` times row_scale[order[r]], rounded to bfloat16, takes its place (nullptr: none)
-  int splits = 1;          // grouped_tiles_kernel without a plan: parts of k, each with a result [m, out_ld] of its own, one after the other
   int gather_top = 0;      // with a plan: > 0: sorted row r is row order[r] / gather_top of `a`
   GluUnit unit = {1.f, INFINITY, 0.f};  // GM_GLU: the unit's middle (see glu_middle)
 };
@@ -307,209 +307,64 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
   else few_rows_tile<EPI, TO, 4>(args, group, row0, rows, order, partial);
 }
 
-// Steps of many rows with a plan: tiles of 128 rows x 256 rows of W, both operands through LDS by loads that write LDS
-// directly.  What bounds it is how far ahead the loads are: a step of 64 indices is 1,024 cycles of the matrix cores and 48 KB,
-// of which the rows of W come from HBM, so three buffers (144 KB, one workgroup per compute unit) keep two steps' loads in
-// flight behind the one that is multiplied.  Eight waves of 64 x 64, two per SIMD; ONE barrier per step, between the halves
-// of a step: the second half's operands leave LDS while the first half's are multiplied, the next step's first while the
-// second's are.  A row of 64 indices is 128 bytes, eight pieces of 16; the pieces of row r are exchanged by an XOR with r's low
-// three bits, which the loads do by asking for another piece (lane l's piece always lands at base + 16 l): no bank
-// conflicts.  The rows of `a` are fetched where they are: with `gather_top` sorted row r is row order[r] / gather_top of `a`, and
-// no sorted copy is made (rows that the pair's weight scales do come as a sorted copy, routed_scale_kernel).  The tiles of one expert that read the same rows of W come one after the other on
-// the same XCD (workgroups are dealt to the eight XCDs in turn), so W leaves HBM once.
-// Measured on MI355X (both products; before: 128 rows x 256 columns with W straight from global memory into the matrix
-// instructions' layout and one step of loads in flight): 10,000 pairs over 32 experts, 4,096 -> 1,408 -> 4,096: 748 + 280 -> 294 +
-// 168 us (0.78 and 0.69 PFLOP/s; W alone at 4.5 TB/s is 164 + 82 us); 2,072 pairs over 16 experts, 2,048 -> 1,408: 153 + 71 -> 70 + 33.
-// Without its loads the first takes 255 us, without its matrix instructions 302: a tile of 256 x 256 is no faster, nor is a
-// ninth wave that reads W ahead into L2 (335).
-// Without a plan it works ONE product, whole or in `splits` parts of k that the kernel behind it adds.  A group's tiles go in
-// blocks of GM_BLOCK_ROWS row tiles, column after column: the 32 tiles that an XCD has under way at once then read 8 row
-// tiles and 4 columns, which its L2 keeps, rather than 32 row tiles of one column (4,096 x 18,944 -> 3,584: 0.85 -> 0.90 PFLOP/s).
-static __device__ __attribute__((aligned(16))) const unsigned int gm_zero_piece[4] = {0u, 0u, 0u, 0u};
-
-#define GM_TILE_ROWS 128  // rows of `a` and
-#define GM_TILE_COLS 256  // rows of W per workgroup of grouped_tiles_kernel
-#define GM_XCDS 8
-#define GM_BLOCK_ROWS 8   // row tiles of a block (see above)
-
-template <int EPI, typename TO>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) grouped_tiles_kernel(const GroupedArgs args, const int cols) {
-  static_assert(EPI == GM_PLAIN || EPI == GM_GLU || EPI == GM_ACT, "no gate here");
-  constexpr int ROWS = GM_TILE_ROWS, STAGES = 3, WAVES = 8;
-  constexpr int WM = 2, WN = WAVES / WM;               // waves along the rows of `a` and along those of W
-  constexpr int RT = 4, CT = GM_TILE_COLS / WN / 16;   // 16 x 16 tiles of a wave
-  constexpr int A_LOADS = ROWS / 8 / WAVES, W_LOADS = GM_TILE_COLS / 8 / WAVES, LOADS = A_LOADS + W_LOADS;
-  constexpr int GROUP = GM_TILE_COLS / WN;             // rows of W of a wave (GLU: half gate rows, half the up rows of the same outputs)
-  __shared__ __attribute__((aligned(1024))) char smem[STAGES][(ROWS + GM_TILE_COLS) * 128];
-
-  // the plan's tiles, or all rows of one product in `splits` parts of k
-  const int row_tiles = args.plan != nullptr ? args.plan[0] : (args.m + ROWS - 1) / ROWS;
-  const int total = row_tiles * cols * args.splits;
-  const int share = (total + GM_XCDS - 1) / GM_XCDS;
-  const int mine = (int)(blockIdx.x / GM_XCDS);
-  int work = (int)(blockIdx.x % GM_XCDS) * share + mine;
-  if (mine >= share || work >= total) return;  // (uniform over the workgroup)
-  int group = 0, begin = 0, end = args.m, first_tile = 0, split = 0;
-  const int* order = nullptr;
-  if (args.plan != nullptr) {
-    const int* starts = args.plan + 1;
-    order = starts + args.plan_groups + 1;
-    const int* tile_group = order + 2 * (size_t)args.plan_pairs;
-    const int* tile_row = tile_group + args.plan_max_tiles;
-    // (a group's tiles follow one another, so work / cols lies among the tiles of the right one)
-    const int near = work / cols;
-    group = tile_group[near];
-    begin = starts[group];
-    end = starts[group + 1];
-    first_tile = near - (tile_row[near] - begin) / ROWS;
-  } else {
-    split = work / (row_tiles * cols);
-    work -= split * row_tiles * cols;
+// The rows of a tile of the plan's products: 64 up to 64 pairs, above 128 or 192 (tiles_mfma.h's kernel, 256 rows of W), whichever is likely to
+// cost less: an expert's last tile is half empty on average, and all tiles take whole rounds over the compute units.  k % 64 != 0 is
+// built for 128.  (Tiles of 64 rows were no quicker at any number of pairs above 64: 12 rows per expert 66 us either way, 56: 80 /
+// 81, 75: 100 / 83, 130: 127 / 125, 256: 187 / 155, 16 experts of 2,048 -> 1,408 -> 2,048.)
+static inline int grouped_tile_rows(int pairs, int experts, int inter, int hidden, int branches) {
+  if (pairs <= 64) return 64;
+  if (inter % 64 != 0 || hidden % 64 != 0) return 128;
+  float cost[2];
+  for (int rt = 2; rt <= 3; ++rt) {
+    const TileCost* t = TILE_COSTS;
+    while (t->rt != rt || t->ct != 4) ++t;
+    const long long rows = (long long)(experts * ((float)pairs / (experts * 64 * rt) + 0.5f)) * 64 * rt;
+    cost[rt - 2] = tiles_cost(*t, rows, (long long)branches * inter, hidden, 1) + tiles_cost(*t, rows, hidden, inter, 1);
   }
-  // a group's tiles in blocks of GM_BLOCK_ROWS row tiles: a block's tiles of one column, then those of the next
-  const int tiles = (end - begin + ROWS - 1) / ROWS, at = work - first_tile * cols;
-  const int block = at / (GM_BLOCK_ROWS * cols), in_block = at % (GM_BLOCK_ROWS * cols), block_rows = min(GM_BLOCK_ROWS, tiles - block * GM_BLOCK_ROWS);
-  const int row0 = begin + (block * GM_BLOCK_ROWS + in_block % block_rows) * ROWS, rows = min(ROWS, end - row0);
-  const int column = in_block / block_rows;
-  const bool half = rows <= 64;  // (a group's last tile) the second 64 rows are neither fetched nor multiplied
-
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int i = lane & 15, g4 = lane >> 4;
-  const int n = args.n, k = args.k;
-  const int all_steps = (k + 63) / 64, split_steps = (all_steps + args.splits - 1) / args.splits;
-  const int k_begin = split * split_steps * 64, k_end = min(k, k_begin + split_steps * 64);
-  const int piece = 8 * ((lane & 7) ^ (lane >> 3));  // first index of the piece this lane asks for, in every load
-  const bf16_t* a_at[A_LOADS];
-  const bf16_t* w_at[W_LOADS];
-#pragma unroll
-  for (int m = 0; m < A_LOADS; ++m) {
-    int r = row0 + min(8 * (wave + WAVES * m) + (lane >> 3), rows - 1);
-    if (args.gather_top > 0) r = order[r] / args.gather_top;
-    a_at[m] = args.a + (size_t)r * args.a_ld + k_begin + piece;
-  }
-  const bf16_t* w_base = args.w + (size_t)group * args.w_group;
-#pragma unroll
-  for (int m = 0; m < W_LOADS; ++m) {
-    const int r = 8 * (wave + WAVES * m) + (lane >> 3);
-    int row;
-    if (EPI == GM_GLU) {
-      const int u = r % GROUP;
-      row = min(column * (GM_TILE_COLS / 2) + r / GROUP * (GROUP / 2) + u % (GROUP / 2), n - 1) + (u >= GROUP / 2 ? n : 0);
-    } else {
-      row = min(column * GM_TILE_COLS + r, n - 1);
-    }
-    w_at[m] = w_base + (size_t)row * k + k_begin + piece;
-  }
-  auto ask = [&](int k0, int buffer) {
-    const bool beyond = k_begin + k0 + piece >= k_end;  // (only ever true in a last step of fewer than 64 indices)
-#pragma unroll
-    for (int m = 0; m < A_LOADS; ++m)
-      if (m == 0 || !half) load_to_lds_16(beyond ? reinterpret_cast<const bf16_t*>(gm_zero_piece) : a_at[m] + k0, smem[buffer] + 1024 * (wave + WAVES * m));
-#pragma unroll
-    for (int m = 0; m < W_LOADS; ++m) load_to_lds_16(beyond ? reinterpret_cast<const bf16_t*>(gm_zero_piece) : w_at[m] + k0, smem[buffer] + ROWS * 128 + 1024 * (wave + WAVES * m));
-  };
-
-  const int wm = wave / WN, wn = wave % WN;
-  const bool idle = half && wm > 0;
-  auto wait_for_one = [&] {  // the oldest of the steps that were asked for has landed; those behind it are still under way
-    if (half) wait_for_loads<(STAGES - 2) * (LOADS - 1)>();
-    else wait_for_loads<(STAGES - 2) * LOADS>();
-  };
-  float4_t acc[CT][RT];
-#pragma unroll
-  for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-  const int steps = k_end > k_begin ? (k_end - k_begin + 63) / 64 : 0;  // (a last part may be empty: zeros)
-#pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s)
-    if (s < steps) ask(64 * s, s);
-  const int swizzle = i & 7;
-  const int a_byte = (wm * 64 + i) * 128, w_byte = ROWS * 128 + (wn * GROUP + i) * 128;
-  gm_bf16x8_t a_op[2][RT], w_op[2][CT];
-  auto fetch = [&](int part, int buffer) {
-    if (idle) return;
-    const char* base = smem[buffer];
-    const int place = ((4 * part + g4) ^ swizzle) * 16;
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) w_op[part][ct] = *reinterpret_cast<const gm_bf16x8_t*>(base + w_byte + ct * 2048 + place);
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) a_op[part][rt] = *reinterpret_cast<const gm_bf16x8_t*>(base + a_byte + rt * 2048 + place);
-  };
-  auto multiply = [&](int part) {
-    if (idle) return;
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_op[part][ct], a_op[part][rt], acc[ct][rt], 0, 0, 0);
-  };
-  // the first step's loads have landed when at most those of the later steps that were asked for are under way
-  if (steps >= STAGES - 1) wait_for_one();
-  else wait_for_loads<0>();
-  __syncthreads();
-  if (steps > 0) fetch(0, 0);
-  int buffer = 0;
-  for (int s = 0; s < steps; ++s) {
-    // operands of the second half on their way while the first half's are multiplied, and the loads of a later step into the
-    // buffer that everybody was done with at the last barrier
-    fetch(1, buffer);
-    int freed = buffer + STAGES - 1;
-    if (freed >= STAGES) freed -= STAGES;
-    if (s + STAGES - 1 < steps) ask(64 * (s + STAGES - 1), freed);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(0);
-    __builtin_amdgcn_sched_barrier(0);
-    buffer = buffer + 1 == STAGES ? 0 : buffer + 1;
-    if (s + 1 < steps) {  // the next step's loads: at most those of the steps behind it are still under way
-      if (s + STAGES <= steps) wait_for_one();
-      else wait_for_loads<0>();
-      __syncthreads();
-      fetch(0, buffer);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(1);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-
-  // lane (g4, i) holds outputs 4 g4 .. + 3 of row i of every tile: one 8- or 16-byte store each (n is a multiple of 4)
-  typedef TO Four __attribute__((ext_vector_type(4)));
-  TO* out = reinterpret_cast<TO*>(args.out) + (size_t)split * args.m * args.out_ld;
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int r = wm * 64 + rt * 16 + i;
-    if (r >= rows) continue;
-    TO* out_row = out + (size_t)(row0 + r) * args.out_ld;
-#pragma unroll
-    for (int ct = 0; ct < (EPI == GM_GLU ? CT / 2 : CT); ++ct) {
-      const int col = (EPI == GM_GLU ? column * (GM_TILE_COLS / 2) + wn * (GROUP / 2) : column * GM_TILE_COLS + wn * GROUP) + ct * 16 + 4 * g4;
-      if (col >= n) continue;
-      Four four;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float v = acc[ct][rt][j];
-        if (EPI == GM_GLU) v = glu_middle(v, acc[ct + CT / 2][rt][j], args.unit);
-        if (EPI == GM_ACT) v = ungated_act(v, args.act);
-        four[j] = from_f32<TO>(v);
-      }
-      *reinterpret_cast<Four*>(out_row + col) = four;
-    }
-  }
+  return cost[1] < cost[0] ? 192 : 128;
 }
 
-// The products of a plan: `pairs` is the most rows a tile can have, `most_tiles` the most tiles there can be.  Tiles hold 64 rows up to 64
-// pairs, GM_TILE_ROWS above.  (Tiles of 64 rows were no quicker at any number of pairs above 64: 12 rows per expert 66 us either way,
-// 56: 80 / 81, 75: 100 / 83, 130: 127 / 125, 256: 187 / 155, 16 experts of 2,048 -> 1,408 -> 2,048.)
 template <int EPI, typename TO>
-static void grouped_plan_launch(const GroupedArgs& args, int pairs, int most_tiles, hipStream_t stream) {
-  if (pairs <= 64) {
+static int grouped_plan_launch(const GroupedArgs& args, int tile_rows, int most_tiles, hipStream_t stream) {
+  if (tile_rows == 64) {
     constexpr int COLS = EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS;
     grouped_mfma_few_rows_kernel<EPI, TO><<<dim3((args.n + COLS - 1) / COLS, most_tiles), 256, 0, stream>>>(args);
-    return;
+    return (int)hipGetLastError();
   }
-  const int cols = ((EPI == GM_GLU ? 2 * args.n : args.n) + GM_TILE_COLS - 1) / GM_TILE_COLS;
-  const int workgroups = (most_tiles * cols + GM_XCDS - 1) / GM_XCDS * GM_XCDS;
-  grouped_tiles_kernel<EPI, TO><<<workgroups, 512, 0, stream>>>(args, cols);
+  constexpr int TILES_EPI = EPI == GM_GLU ? TL_UNIT : EPI == GM_ACT ? TL_ACT : TL_PLAIN;
+  TileArgs tiles = {};
+  tiles.a = args.a;
+  tiles.a_ld = args.a_ld;
+  tiles.w = args.w;
+  tiles.w_group = args.w_group;
+  tiles.out = args.out;
+  tiles.n = args.n;
+  tiles.k = args.k;
+  tiles.splits = 1;
+  tiles.plan = args.plan;
+  tiles.plan_pairs = args.plan_pairs;
+  tiles.plan_groups = args.plan_groups;
+  tiles.plan_max_tiles = args.plan_max_tiles;
+  tiles.gather_top = args.gather_top;
+  tiles.act = args.act;
+  tiles.unit = args.unit;
+  if (!tiles_fit(args.gather_top > 0 ? args.plan_pairs / args.gather_top : 256, args.a_ld, EPI == GM_GLU ? args.n + 256LL : 256, args.k)) return -1;
+  const long long most = (long long)most_tiles * (((EPI == GM_GLU ? 2LL : 1LL) * args.n + 255) / 256);
+  const int workgroups = (int)(most < TL_WORKGROUPS ? (most + TL_XCDS - 1) / TL_XCDS * TL_XCDS : TL_WORKGROUPS);
+#define TILES(RT, S, GATHER, TAIL) tiles_kernel<RT, 4, S, TILES_EPI, TO, true, GATHER, TAIL><<<workgroups, 256, 0, stream>>>(tiles)
+  if constexpr (EPI != GM_PLAIN) {
+    if (args.gather_top > 0) {
+      if (tile_rows == 192) TILES(3, 2, true, false);
+      else if (args.k % 64 == 0) TILES(2, 3, true, false);
+      else TILES(2, 3, true, true);
+      return (int)hipGetLastError();
+    }
+  }
+  if (tile_rows == 192) TILES(3, 2, false, false);
+  else if (args.k % 64 == 0) TILES(2, 3, false, false);
+  else TILES(2, 3, false, true);
+#undef TILES
+  return (int)hipGetLastError();
 }
 
 // The products of `groups` groups that all run rows [0, m).

@@ -278,11 +278,11 @@ extern "C" long long velox_routed_plan_elems(int pairs, int experts) {
 
 extern "C" int velox_routed_max_tiles(int pairs, int experts) { return (pairs + RT_BM - 1) / RT_BM + experts; }
 
-// tile_rows: 64, or 128 for the matrix-core products of more than 64 pairs.  The plan's layout is that of 64-row tiles either way
+// tile_rows: 64, or what velox_routed_tile_rows says for the matrix-core products.  The plan's layout is that of 64-row tiles either way
 // (the most tiles there can be).
 extern "C" int velox_routed_plan(const int* choice, int pairs, int experts, int* plan, int tile_rows, hipStream_t stream) {
   if (pairs <= 0) return 0;
-  if (experts < 1 || experts > PLAN_MAX_EXPERTS || (tile_rows != RT_BM && tile_rows != 2 * RT_BM)) return -1;
+  if (experts < 1 || experts > PLAN_MAX_EXPERTS || (tile_rows != RT_BM && tile_rows != 2 * RT_BM && tile_rows != 3 * RT_BM)) return -1;
   routed_plan_kernel<<<1, 1024, 0, stream>>>(choice, pairs, experts, velox_routed_max_tiles(pairs, experts), tile_rows, plan);
   VELOX_RETURN_LAUNCH_STATUS();
 }
@@ -497,7 +497,9 @@ static GroupedArgs routed_args(const void* a, const void* w, void* out, const in
 }
 
 // x [T, hidden] -> (`sorted` [pairs, hidden], with scale_input and more than 64 pairs) -> act [pairs, inter] -> y [pairs, hidden]
-// float32.  Needs hidden % 8 == 0, inter % 8 == 0 and x and `sorted` on 16-byte boundaries (the caller checks).  The plan's tiles hold 64 rows for up to 64 pairs, GM_TILE_ROWS for more.
+// float32.  Needs hidden % 8 == 0, inter % 8 == 0 and x and `sorted` on 16-byte boundaries (the caller checks).  The plan's tiles hold velox_routed_tile_rows rows.
+extern "C" int velox_routed_tile_rows(int pairs, int experts, int inter, int hidden, int branches) { return grouped_tile_rows(pairs, experts, inter, hidden, branches); }
+
 extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, const void* down, void* sorted, void* act, float* y, const int* plan,
                                           const float* pair_weight, int pairs, int experts, int top, int inter, int hidden, int scale_input,
                                           float alpha, float limit, float shift, int ungated, hipStream_t stream) {
@@ -506,7 +508,7 @@ extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, co
   if (hidden % 8 != 0 || inter % 8 != 0 || top < 1 || ((uintptr_t)x | (uintptr_t)sorted) % 16 != 0) return -1;
   const bool copied = scale_input && pairs > RT_BM;
   if (copied && sorted == nullptr) return -1;
-  const int max_tiles = velox_routed_max_tiles(pairs, experts);
+  const int max_tiles = velox_routed_max_tiles(pairs, experts), tile_rows = grouped_tile_rows(pairs, experts, inter, hidden, ungated > 0 ? 1 : 2);
   if (max_tiles > 65535) return -1;
   if (copied)
     routed_scale_kernel<<<pairs, 256, 0, stream>>>((const bf16_t*)x, plan + 1 + (experts + 1), pair_weight, (bf16_t*)sorted, top, hidden, plan + 1 + experts);
@@ -515,13 +517,12 @@ extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, co
   first.row_scale = scale_input ? pair_weight : nullptr;  // (read by the kernel for few rows alone)
   first.act = ungated;
   first.unit = GluUnit{alpha, limit, shift};
-  if (ungated > 0) grouped_plan_launch<GM_ACT, bf16_t>(first, pairs, max_tiles, stream);
-  else grouped_plan_launch<GM_GLU, bf16_t>(first, pairs, max_tiles, stream);
+  const int status = ungated > 0 ? grouped_plan_launch<GM_ACT, bf16_t>(first, tile_rows, max_tiles, stream) : grouped_plan_launch<GM_GLU, bf16_t>(first, tile_rows, max_tiles, stream);
+  if (status != 0) return status;
   GroupedArgs last = routed_args(act, down, y, plan, pairs, experts, hidden, inter, hidden);
   // (a weight on the experts' OUTPUT is applied where the results are added up, routed_combine with scale_rows: the product
   // itself is the same kernel either way)
-  grouped_plan_launch<GM_PLAIN, float>(last, pairs, max_tiles, stream);
-  VELOX_RETURN_LAUNCH_STATUS();
+  return grouped_plan_launch<GM_PLAIN, float>(last, tile_rows, max_tiles, stream);
 }
 
 // ---------------------------------------------------------------------------------------------
