@@ -325,13 +325,30 @@ static inline int grouped_tile_rows(int pairs, int experts, int inter, int hidde
 }
 
 template <int EPI, typename TO>
+static void grouped_tiles_launch(const TileArgs& tiles, int tile_rows, int workgroups, hipStream_t stream) {
+#define TILES(RT, S, GATHER, TAIL) tiles_kernel<RT, 4, S, EPI, TO, true, GATHER, TAIL><<<workgroups, 256, 0, stream>>>(tiles)
+  const bool tail = tiles.k % 64 != 0;
+  if constexpr (EPI != TL_PLAIN) {
+    if (tiles.gather_top > 0) {
+      if (tile_rows == 192) TILES(3, 2, true, false);
+      else if (!tail) TILES(2, 3, true, false);
+      else TILES(2, 3, true, true);
+      return;
+    }
+  }
+  if (tile_rows == 192) TILES(3, 2, false, false);
+  else if (!tail) TILES(2, 3, false, false);
+  else TILES(2, 3, false, true);
+#undef TILES
+}
+
+template <int EPI, typename TO>
 static int grouped_plan_launch(const GroupedArgs& args, int tile_rows, int most_tiles, hipStream_t stream) {
   if (tile_rows == 64) {
     constexpr int COLS = EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS;
     grouped_mfma_few_rows_kernel<EPI, TO><<<dim3((args.n + COLS - 1) / COLS, most_tiles), 256, 0, stream>>>(args);
     return (int)hipGetLastError();
   }
-  constexpr int TILES_EPI = EPI == GM_GLU ? TL_UNIT : EPI == GM_ACT ? TL_ACT : TL_PLAIN;
   TileArgs tiles = {};
   tiles.a = args.a;
   tiles.a_ld = args.a_ld;
@@ -351,19 +368,12 @@ static int grouped_plan_launch(const GroupedArgs& args, int tile_rows, int most_
   if (!tiles_fit(args.gather_top > 0 ? args.plan_pairs / args.gather_top : 256, args.a_ld, EPI == GM_GLU ? args.n + 256LL : 256, args.k)) return -1;
   const long long most = (long long)most_tiles * (((EPI == GM_GLU ? 2LL : 1LL) * args.n + 255) / 256);
   const int workgroups = (int)(most < TL_WORKGROUPS ? (most + TL_XCDS - 1) / TL_XCDS * TL_XCDS : TL_WORKGROUPS);
-#define TILES(RT, S, GATHER, TAIL) tiles_kernel<RT, 4, S, TILES_EPI, TO, true, GATHER, TAIL><<<workgroups, 256, 0, stream>>>(tiles)
-  if constexpr (EPI != GM_PLAIN) {
-    if (args.gather_top > 0) {
-      if (tile_rows == 192) TILES(3, 2, true, false);
-      else if (args.k % 64 == 0) TILES(2, 3, true, false);
-      else TILES(2, 3, true, true);
-      return (int)hipGetLastError();
-    }
+  if constexpr (EPI == GM_GLU) {
+    if (args.unit.alpha == 1.f && args.unit.limit == INFINITY && args.unit.shift == 0.f) grouped_tiles_launch<TL_SILU_UNIT, TO>(tiles, tile_rows, workgroups, stream);
+    else grouped_tiles_launch<TL_UNIT, TO>(tiles, tile_rows, workgroups, stream);
+  } else {
+    grouped_tiles_launch<EPI == GM_ACT ? TL_ACT : TL_PLAIN, TO>(tiles, tile_rows, workgroups, stream);
   }
-  if (tile_rows == 192) TILES(3, 2, false, false);
-  else if (args.k % 64 == 0) TILES(2, 3, false, false);
-  else TILES(2, 3, false, true);
-#undef TILES
   return (int)hipGetLastError();
 }
 

@@ -35,8 +35,8 @@ typedef unsigned int tl_uint2_t __attribute__((ext_vector_type(2)));
 typedef unsigned int tl_uint4_t __attribute__((ext_vector_type(4)));
 
 // what becomes of the sums: nothing; silu(gate) * up and max(gate, 0) * up of sums that are rounded to bfloat16 first, as a product of its
-// own would leave them; an expert's gated middle; a unit without a gate branch
-enum { TL_PLAIN = 0, TL_SILU = 1, TL_RELU = 2, TL_UNIT = 3, TL_ACT = 4 };
+// own would leave them; an expert's gated middle, silu(gate) * up or any other; a unit without a gate branch
+enum { TL_PLAIN = 0, TL_SILU = 1, TL_RELU = 2, TL_SILU_UNIT = 3, TL_UNIT = 4, TL_ACT = 5 };
 
 #define TL_XCDS 8
 #define TL_WORKGROUPS 256  // one per compute unit
@@ -93,8 +93,10 @@ __device__ __forceinline__ uint32_t tl_pack(float x, float y) {
 template <int EPI>
 __device__ __forceinline__ float tl_middle(float gate, float up, const TileArgs& args) {
   if (EPI == TL_UNIT) return glu_middle(gate, up, args.unit);
-  gate = to_f32(from_f32<bf16_t>(gate));
-  up = to_f32(from_f32<bf16_t>(up));
+  if (EPI != TL_SILU_UNIT) {
+    gate = to_f32(from_f32<bf16_t>(gate));
+    up = to_f32(from_f32<bf16_t>(up));
+  }
   if (EPI == TL_RELU) return fmaxf(gate, 0.f) * up;
   return gate * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gate * -1.44269504f)) * up;
 }
@@ -107,7 +109,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
   static_assert(S * STAGE <= 160 * 1024, "LDS of a compute unit");
   constexpr int RH0 = (RT + 1) / 2, RH1 = RT - RH0, CH0 = (CT + 1) / 2, CH1 = CT - CH0;  // halves of a wave's tiles
   constexpr int LA0 = 2 * RH0, LC0 = 2 * CH0, LC1 = 2 * CH1, LA1 = 2 * RH1, LOADS = LA0 + LC0 + LC1 + LA1;  // loads of a wave in a step, in this order
-  constexpr bool GLU = EPI == TL_SILU || EPI == TL_RELU || EPI == TL_UNIT;
+  constexpr bool GLU = EPI == TL_SILU || EPI == TL_RELU || EPI == TL_SILU_UNIT || EPI == TL_UNIT;
   constexpr int OUT_COLS = GLU ? TN / 2 : TN;  // output columns of the tile
   constexpr int BLOCK_ROWS = 1024 / TM;        // row tiles of a block
   __shared__ __attribute__((aligned(1024))) char smem[S * STAGE];
@@ -466,7 +468,7 @@ static inline int tiles_splits(long long m, long long n, int k, int most) {
 // One product in tiles of `tile`.
 template <int EPI, typename TO, bool TAIL>
 static int tiles_launch(const TileArgs& args, int tile, hipStream_t stream) {
-  constexpr int BRANCHES = EPI == TL_SILU || EPI == TL_RELU || EPI == TL_UNIT ? 2 : 1;
+  constexpr int BRANCHES = EPI == TL_SILU || EPI == TL_RELU ? 2 : 1;
 #define TILES(RT, CT, S)                                                                                                              \
   case 64 * RT * 1000 + 64 * CT: {                                                                                                    \
     const long long cols = (args.n + 64 * CT / BRANCHES - 1) / (64 * CT / BRANCHES);                                                  \
