@@ -1413,7 +1413,7 @@ def test_which_products_run_in_the_own_tiles(ops, monkeypatch, m, n, k, own):
     monkeypatch.setattr(ops, "gemm_tiles", lambda *a, **more: calls.append(a) or type(ops).gemm_tiles(ops, *a, **more))
     x, w, bias = rand((m, k), torch.bfloat16, 1), rand((n, k), torch.bfloat16, 2, k ** -0.5), rand((n,), torch.float32, 3)
     got = ops.linear(x, w, bias, torch.bfloat16)
-    assert ops.tiles_serve(m, n, k) == own and len(calls) == int(own) and ops.library_serves(m, n, k) == (m > 64 and not own)
+    assert ops.tiles_serve(m, n, k) == own and len(calls) == int(own) and type(ops).library_serves(ops, m, n, k) == (m > 64 and not own)
     want = x.double() @ w.double().T + bias.double()
     assert torch.all((got.double() - want).abs() <= 2.0 ** -7 * (want.abs() + bias.double().abs()) + k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T))
 
@@ -1544,3 +1544,42 @@ def test_experts_whose_weights_lie_off_16_byte_boundaries(ops):
     for a, b in ((moved(first), down), (first, moved(down))):
         assert (a.data_ptr() | b.data_ptr()) % 16 == 4
         torch.testing.assert_close(ops.routed_experts(x, choice, weight, a, b, experts, False, None, torch.bfloat16).float(), want.float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("tile", [128256, 128192, 96192, 64256, 64128, 64064, 32128, 0])
+@pytest.mark.parametrize("m, n, k, splits", [(17, 64, 32, 1), (129, 260, 160, 1), (97, 388, 672, 3), (300, 132, 4096, 8), (65, 4100, 128, 1), (33, 132, 2080, 1), (70, 64, 6176, 1)])
+def test_float32_products_of_split_operands(ops, tile, m, n, k, splits):
+    """Every tile, remainders of rows and columns, last sums of fewer than 128 terms, sums of more than one level.  A term's left-out products are below 2^-24 of it;
+    an instruction is off by at most 2^-22 of the sizes it adds (24 of them in a sum of 128 terms, on average over half of these); each sum of
+    128 terms, of 2,048, part and bias is added with a rounding: (24 + min(k / 128, 16) + k / 2048 + splits + 3) 2^-23 of the sum of the terms' sizes."""
+    generator = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w, bias = (torch.randn(*shape, generator=generator, device="cuda") for shape in ((m, k), (n, k), (n,)))
+    a *= 10.0 ** torch.randint(-6, 7, (m, 1), generator=generator, device="cuda")
+    got = ops.split_f32(a, w, None if splits > 1 else bias, splits, tile)
+    want, sizes = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    if splits > 1:
+        got = got.sum(0)
+    else:
+        want, sizes = want + bias.double(), sizes + bias.double().abs()
+    assert torch.all((got.double() - want).abs() <= (24 + min(k / 128, 16) + k / 2048 + splits + 3) * 2.0 ** -23 * sizes)
+
+
+@pytest.mark.parametrize("tile", [128256, 128192, 64064])
+def test_float32_products_of_numbers_that_do_not_split(ops, tile):
+    """Infinities, NaN, numbers that round to an infinity and numbers without lower parts: as the float32 instructions have them.  Those add
+    in another order, so finite outcomes differ by their two roundings."""
+    m, n, k = 150, 324, 288
+    generator = torch.Generator(device="cuda").manual_seed(5)
+    a, w = (torch.randn(*shape, generator=generator, device="cuda") for shape in ((m, k), (n, k)))
+    a[3, 7], a[40, 100], a[77, 30], a[78, 31] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    w[100, 5], w[200, 287] = float("inf"), 0.0
+    w[:, 31] *= 0.01
+    a[120:130] *= 1e-36
+    a[131] = 0.0
+    got, want = ops.split_f32(a, w, tile=tile), ops.gemm_fma(a, w, None, torch.float32)
+    assert torch.equal(got.isnan(), want.isnan())
+    whole = want.isfinite()
+    assert torch.equal(got[~whole & ~want.isnan()], want[~whole & ~want.isnan()])
+    sizes = torch.where(a.isfinite(), a, 0).double().abs() @ torch.where(w.isfinite(), w, 0).double().abs().T
+    assert torch.all(((got.double() - want.double()).abs() <= 160 * 2.0 ** -23 * sizes)[whole])
+    assert torch.all(got[131][want[131].isfinite()] == 0)

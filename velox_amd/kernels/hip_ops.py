@@ -189,6 +189,10 @@ class HipOps:
         c.velox_removal_chunk_scan.restype = _I
         c.velox_gemm_f32_tile.argtypes = [_I, _I]
         c.velox_gemm_f32_tile.restype = _I
+        c.velox_split_f32.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P]
+        c.velox_split_f32_tile.argtypes = c.velox_split_f32_parts.argtypes = [_I, _I, _I, _I]
+        for fn in (c.velox_split_f32, c.velox_split_f32_tile, c.velox_split_f32_parts):
+            fn.restype = _I
         c.velox_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]
         c.velox_tiles_glu_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P]
         c.velox_tiles_pick.argtypes = c.velox_tiles_splits.argtypes = [_I, _I, _I, _I]
@@ -825,6 +829,10 @@ class HipOps:
                 if self._mm_out_dtype_ok is None:
                     self._decide_float32_out_route()
                 return torch.mm(x, weight.t(), out_dtype=torch.float32)
+        if x.dtype == torch.float32 and weight.dtype == torch.float32 and out_dtype == torch.float32:
+            splits = self.split_f32_parts(m, n, k, partials_ok and bias is None)
+            if splits > 0:
+                return self.split_f32(x, weight, bias, splits)
         return self.gemm_fma(x, weight, bias, out_dtype)
 
     def _bias_in_bfloat16(self, bias: torch.Tensor) -> torch.Tensor:
@@ -1099,6 +1107,28 @@ class HipOps:
             return False
         size = f"tn_{n}_{m}_{k}_"
         return tunable.tuning_is_enabled() or any(r[0] == "GemmTunableOp_BFloat16_TN" and r[1].startswith(size) for r in tunable.get_results())
+
+    def split_f32_parts(self, m: int, n: int, k: int, partials_ok: bool) -> int:
+        """Parts of k in which ``linear`` works a float32 product of more than 16 rows as products of bfloat16 parts (split_f32.hip; 0: not
+        at all, ``gemm_fma``'s kernels).  In parts it is the quicker one throughout (129 products, 0.62 of the time on average, 0.92 at
+        worst).  Whole it needs tiles for the card, which ``gemm_fma`` gives two sets of waves (us, ``gemm_fma`` / this): 330 rows of 2,048 x 1,536 (192
+        tiles of 64 x 64) 38 / 29, 150 of 17,920 x 1,536 120 / 67, 616 of 17,920 x 1,536 322 / 187, but 256 of 2,048 x 1,536 (128) 23 / 29, 100 of 11,264 x
+        2,048 (352) 71 / 71, and with up to 64 rows 17 of 17,920 x 1,536 44 / 57.  Sums of fewer than 512 terms are quicker and no less exact here too
+        (616 rows of 2,048 x 256 12.6 / 10.6, of 8,192 x 256 39 / 23) and stay away all the same: a small model with sharp weights, whose recurrences
+        blow a rounding up a thousandfold, left its tolerance of 3e-5 by a fifth in another order of additions."""
+        if m <= 16 or k < 512 or k % 32 != 0 or n % 4 != 0:
+            return 0
+        splits = self._core.velox_split_f32_parts(m, n, k, 8) if partials_ok else 1
+        return splits if splits > 1 or (m > 64 and -(-m // 64) * -(-n // 64) > 160) else 0
+
+    def split_f32(self, x, weight, bias: Optional[torch.Tensor] = None, splits: int = 1, tile: int = 0):
+        """``x @ weight^T (+ bias)`` of float32 operands: [M, N], or with ``splits`` > 1 partial sums [splits, M, N].  ``tile``: rows * 1,000 +
+        columns (0: picked by the product's size)."""
+        m, k = x.shape
+        n = weight.shape[0]
+        out = torch.empty((m, n) if splits == 1 else (splits, m, n), dtype=torch.float32, device=self.device)
+        self._launched(self._core.velox_split_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(out), m, n, k, int(splits), int(tile), self._stream()), "split_f32")
+        return out
 
     def gemm_tiles(self, x, weight, splits: int = 1, out_dtype=torch.bfloat16, bias: Optional[torch.Tensor] = None, tile: int = 0):
         """``x @ weight^T (+ bias)`` in bfloat16 in large tiles: [M, N] in bfloat16, or float32 partial sums [splits, M, N].  ``tile``: rows * 1,000 +
