@@ -169,6 +169,31 @@ def test_chunks_of_tokens_equal_the_token_by_token_kernels(ops, dtype, heads, di
     assert float((run((n,), quiet)[0][-1] - whole[-1]).abs().max()) > 0.2 * float(whole[-1].abs().max())
 
 
+@pytest.mark.parametrize("lengths", [[1] * 63 + [40], [1] * 64 + [33], [17] + [1] * 70 + [100, 1, 16, 31, 32, 2], [3] * 130 + [65]])
+def test_pieces_and_chunks_among_many_sequences(ops, lengths):
+    """Sequences beyond the 64 that a wave looks through at a time, at the edges of that number, with chunks and pieces at their borders."""
+    ref, count, tokens = TorchOps(), len(lengths), sum(lengths)
+    heads, dim, vdim, rank, width = 2, 16, 16, 4, 40
+    cu, slot = ints([0] + list(np.cumsum(lengths))), ints(list(np.random.RandomState(count).permutation(count)))
+    ks, vs = heads * dim, heads * vdim
+    at = (0, ks, 2 * ks, 2 * ks + vs, 3 * ks + 2 * vs)
+    main = torch.randn(tokens, 3 * ks + 2 * vs + rank).cuda()
+    w2, a_bias, w0 = torch.randn(ks, rank).cuda(), torch.randn(ks).cuda(), torch.randn(ks).cuda()
+    states = [torch.randn(count, heads, dim, vdim).cuda() * 0.3]
+    states.append(states[0].clone())
+    got = ops.removal_scan(main, *at, rank, heads, dim, vdim, a_bias, w2, w0, math.exp(-0.5), states[0], slot, cu, max(lengths), chunked=True)
+    want = ref.removal_scan(main, *at, rank, heads, dim, vdim, a_bias, w2, w0, math.exp(-0.5), states[1], slot, cu, max(lengths))
+    near(got, want, 3e-5, "read-out")  # (as above)
+    near(states[0], states[1], 3e-5, "state")
+    rows, zb, xb = torch.randn(tokens, 3 * width).cuda(), torch.randn(width).cuda(), torch.randn(width).cuda()
+    states = [torch.randn(count, width).cuda()]
+    states.append(states[0].clone())
+    got = ops.gated_scan(rows, width, zb, xb, 0.5, states[0], slot, cu, max(lengths))
+    want = ref.gated_scan(rows, width, zb, xb, 0.5, states[1], slot, cu, max(lengths))
+    close(got, want, "float32")
+    torch.testing.assert_close(states[0], states[1], rtol=2e-5, atol=2e-6)
+
+
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 64), (1, 128, 128), (3, 32, 48), (2, 12, 12), (1, 256, 16), (1, 72, 40)])
 def test_a_long_portion_equals_its_pieces_and_its_first_token_is_kept(ops, heads, dim, vdim):
     """600 tokens in one step, in pieces (one of a single token, one of two) and against the plain loop; with decays close

@@ -72,6 +72,28 @@ template <int N> __device__ __forceinline__ void wait_for_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
+// Work item `item` of a step whose sequence b has items of `size` tokens from item cu_q[b] / size + b on: those of two sequences never overlap,
+// floor((a + n) / size) + 1 >= floor(a / size) + ceil(n / size), so `step_items` of them hold all.  Gives the sequence with its tokens [lo, hi)
+// and the item's place in it (sequence -1: none, and lo == hi; pieces behind a sequence's end are the caller's to skip).  The whole wave
+// takes part.  For a grid of one workgroup per item and not of the longest sequence's items for each: 12 single tokens beside 1,024 are
+// 77 chunks of 16 and not 832, of which the empty ones held compute units while they read their sequence's ends.
+struct StepItem { int sequence, lo, hi, piece; };
+__host__ __device__ __forceinline__ long long step_items(int tokens, int num_seqs, int size) { return (long long)(tokens / size) + num_seqs; }
+__device__ __forceinline__ StepItem step_item(const int* cu_q, int num_seqs, int size, int item) {
+  const int lane = threadIdx.x & (VELOX_WAVE - 1);
+  StepItem found = {-1, 0, 0, 0};
+  for (int base = 0; base < num_seqs; base += VELOX_WAVE) {
+    const int b = base + lane;
+    const int lo = b < num_seqs ? cu_q[b] : 0, hi = b < num_seqs ? cu_q[b + 1] : 0;
+    const int first = lo / size + b, here = __popcll(__ballot(b < num_seqs && first <= item));
+    if (here == 0) break;
+    const int last = here - 1;  // (first items rise with the sequence)
+    found = {base + last, __builtin_amdgcn_readlane(lo, last), __builtin_amdgcn_readlane(hi, last), item - __builtin_amdgcn_readlane(first, last)};
+    if (here < VELOX_WAVE) break;
+  }
+  return found;
+}
+
 // Four consecutive elements of a row, widened to float32: one 8- or 16-byte access when `vec_ok` (the row starts on such a
 // boundary and k is a multiple of 4) and all four lie below k_limit, else element by element with zeros beyond k_limit.
 template <typename T>

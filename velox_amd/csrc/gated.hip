@@ -10,6 +10,8 @@
 //     [sequence][1 + pieces][2][width]; the first entry is (0, the slot's state), which only this pass reads;
 //   gated_scan_kernel: every piece folds the entries before it into the state it starts from, walks its tokens and writes
 //     the outputs; a sequence's last piece writes the slot's state.
+// A workgroup per piece that there is, not per piece of the longest portion for every sequence: 1,024 tokens beside 12 single ones of
+// 3,072 channels 10.1 + 20.1 -> 9.3 + 17.8 us.
 // (A lane with two neighbouring channels reads wider but leaves half the waves: 53 us for 2,048 tokens of 3,072 channels where
 // one channel a lane takes 48.)
 #include "common.h"
@@ -29,6 +31,7 @@ struct GatedArgs {
   void* out;
   float* scratch;  // nullptr: portions of one piece
   int entries;     // 1 + the pieces of the longest portion
+  int num_seqs, column_blocks;
 };
 
 // sigmoid(x) and 1 - sigmoid(x) = sigmoid(-x) (taken so, nothing is lost near 0) from one exponential and one reciprocal of a
@@ -50,10 +53,10 @@ __device__ __forceinline__ void gated_token(float xz, float xu, float shift, flo
 
 template <typename T>
 __global__ void __launch_bounds__(128) gated_pieces_kernel(const GatedArgs a) {
-  const int c = blockIdx.x * 128 + threadIdx.x;
-  const int b = blockIdx.z, piece = blockIdx.y, W = a.width;
-  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  const int first = lo + piece * GATED_PIECE;
+  const int c = blockIdx.x % a.column_blocks * 128 + threadIdx.x;
+  const StepItem item = step_item(a.cu_q, a.num_seqs, GATED_PIECE, blockIdx.x / a.column_blocks);
+  const int b = item.sequence, piece = item.piece, hi = item.hi, W = a.width;
+  const int first = item.lo + piece * GATED_PIECE;
   if (c >= W || first >= hi) return;
   float* entry = a.scratch + (size_t)b * a.entries * 2 * W + c;
   if (piece == 0) {
@@ -86,10 +89,10 @@ __global__ void __launch_bounds__(128) gated_pieces_kernel(const GatedArgs a) {
 
 template <typename T>
 __global__ void __launch_bounds__(128) gated_scan_kernel(const GatedArgs a) {
-  const int c = blockIdx.x * 128 + threadIdx.x;
-  const int b = blockIdx.z, piece = blockIdx.y, W = a.width;
-  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  const int first = lo + piece * GATED_PIECE;
+  const int c = blockIdx.x % a.column_blocks * 128 + threadIdx.x;
+  const StepItem item = step_item(a.cu_q, a.num_seqs, GATED_PIECE, blockIdx.x / a.column_blocks);
+  const int b = item.sequence, piece = item.piece, hi = item.hi, W = a.width;
+  const int first = item.lo + piece * GATED_PIECE;
   if (c >= W || first >= hi) return;
   const int last = first + GATED_PIECE < hi ? first + GATED_PIECE : hi;
   float* my_state = a.state + (size_t)a.slots[b] * W + c;
@@ -134,19 +137,19 @@ extern "C" long long velox_gated_scan_scratch_elems(int num_seqs, int max_q_len,
 }
 
 template <typename T>
-static void gated_scan_launch(const GatedArgs& a, int pieces, int num_seqs, hipStream_t stream) {
-  const dim3 grid((a.width + 127) / 128, pieces, num_seqs);
+static void gated_scan_launch(const GatedArgs& a, int tokens, hipStream_t stream) {
+  const unsigned grid = (unsigned)(a.column_blocks * step_items(tokens, a.num_seqs, GATED_PIECE));
   if (a.scratch) gated_pieces_kernel<T><<<grid, 128, 0, stream>>>(a);
   gated_scan_kernel<T><<<grid, 128, 0, stream>>>(a);
 }
 
 extern "C" int velox_gated_scan(const void* proj, int dtype, int width, const float* bias_z, const float* bias_u, float shift, float* state, const int* slots,
-                                const int* cu_q, void* out, float* scratch, int num_seqs, int max_q_len, hipStream_t stream) {
+                                const int* cu_q, void* out, float* scratch, int tokens, int num_seqs, int max_q_len, hipStream_t stream) {
   if (num_seqs <= 0 || max_q_len <= 0) return 0;
   const int pieces = (max_q_len + GATED_PIECE - 1) / GATED_PIECE;
-  if (width < 1 || num_seqs > 65535 || pieces > 65535 || (pieces > 1 && !scratch)) return (int)hipErrorInvalidValue;
-  GatedArgs a{proj, width, bias_z, bias_u, shift, state, slots, cu_q, out, pieces > 1 ? scratch : nullptr, 1 + pieces};
-  if (dtype == VELOX_BF16) gated_scan_launch<bf16_t>(a, pieces, num_seqs, stream);
-  else gated_scan_launch<float>(a, pieces, num_seqs, stream);
+  if (width < 1 || tokens < max_q_len || (width + 127) / 128 * step_items(tokens, num_seqs, GATED_PIECE) > 0x7fffffff || (pieces > 1 && !scratch)) return (int)hipErrorInvalidValue;
+  GatedArgs a{proj, width, bias_z, bias_u, shift, state, slots, cu_q, out, pieces > 1 ? scratch : nullptr, 1 + pieces, num_seqs, (width + 127) / 128};
+  if (dtype == VELOX_BF16) gated_scan_launch<bf16_t>(a, tokens, stream);
+  else gated_scan_launch<float>(a, tokens, stream);
   VELOX_RETURN_LAUNCH_STATUS();
 }

@@ -42,7 +42,7 @@ struct RemovalChunkArgs {
 // of them is one contiguous kilobyte, 16 bytes a lane.
 __host__ __device__ __forceinline__ int removal_columns(int vdim) { return (vdim + 15) / 16 * 16; }
 __host__ __device__ __forceinline__ size_t removal_record(int dim, int vdim) { return (size_t)65 * dim + 48 * removal_columns(vdim); }
-// the first record of a sequence: sequences' chunks never overlap, because floor((a + n) / 16) + 1 >= floor(a / 16) + ceil(n / 16)
+// the first record of a sequence (chunks are a step's items, see step_item)
 __device__ __forceinline__ int removal_first_chunk(int first_token, int sequence) { return first_token / CHUNK + sequence; }
 
 __device__ __forceinline__ float removal_sigmoid(float z) { return 1.f / (1.f + expf(-z)); }
@@ -50,12 +50,12 @@ __device__ __forceinline__ float4_t mfma4(float a, float b, float4_t c) { return
 __device__ __forceinline__ float4_t four(const float* p) { return *reinterpret_cast<const float4_t*>(p); }
 
 template <typename T>
-__global__ void __launch_bounds__(256) removal_chunk_prepare_kernel(const RemovalChunkArgs a) {
+__global__ void __launch_bounds__(256) removal_chunk_prepare_kernel(const RemovalChunkArgs a, int num_seqs) {
   extern __shared__ float4_t lds_pieces[];
   float* lds = reinterpret_cast<float*>(lds_pieces);
-  const int h = blockIdx.x, b = blockIdx.z;
-  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  const int t0 = lo + blockIdx.y * CHUNK;
+  const int h = blockIdx.x % a.heads, record_at = blockIdx.x / a.heads;
+  const StepItem item = step_item(a.cu_q, num_seqs, CHUNK, record_at);
+  const int hi = item.hi, t0 = item.lo + item.piece * CHUNK;
   if (t0 >= hi) return;  // (the whole workgroup)
   const int count = hi - t0 < CHUNK ? hi - t0 : CHUNK;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -137,7 +137,6 @@ __global__ void __launch_bounds__(256) removal_chunk_prepare_kernel(const Remova
   }
   __syncthreads();
   // the running products and the scaled rows; a lane walks one channel of one of the four matrices
-  const int record_at = removal_first_chunk(lo, b) + blockIdx.y;
   float* record = a.scratch + ((size_t)record_at * a.heads + h) * removal_record(dim, a.vdim);
   float* record_b = record + 32 * dim;
   float* record_k = record + 48 * dim;
@@ -272,7 +271,7 @@ struct RemovalOperands {
 template <int WAVES>
 __global__ void __launch_bounds__(64 * WAVES, 2) removal_chunk_scan_kernel(const RemovalChunkArgs a) {
   __shared__ float4_t parts[2][2][WAVES][64];  // [buffer][D, O][wave][lane]
-  // (heads lie along the grid's first dimension in both kernels: with a multiple of 8 heads the workgroups that read a record run
+  // (heads lie along the grid fastest in both kernels: with a multiple of 8 heads the workgroups that read a record run
   // on the XCD that wrote it and share it in that XCD's L2)
   const int h = blockIdx.x, tile = blockIdx.y, b = blockIdx.z;
   const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
@@ -385,13 +384,13 @@ static size_t removal_prepare_lds(int dim, int rank) {
 // float32 elements of the scratch of a step; 0: these sizes are not for these kernels
 extern "C" long long velox_removal_chunk_scratch_elems(int tokens, int num_seqs, int heads, int dim, int vdim, int rank) {
   if (dim % 16 != 0 || dim < 16 || dim > 128 || vdim < 1 || rank < 1 || removal_prepare_lds(dim, rank) > 64 * 1024) return 0;
-  return ((long long)tokens / CHUNK + num_seqs + 1) * heads * (long long)removal_record(dim, vdim);
+  return (step_items(tokens, num_seqs, CHUNK) + 1) * heads * (long long)removal_record(dim, vdim);
 }
 
 template <typename T>
-static void removal_chunk_launch(const RemovalChunkArgs& a, int num_seqs, int max_q_len, hipStream_t stream) {
-  const int chunks = (max_q_len + CHUNK - 1) / CHUNK;
-  removal_chunk_prepare_kernel<T><<<dim3(a.heads, chunks, num_seqs), 256, removal_prepare_lds(a.dim, a.rank), stream>>>(a);
+static void removal_chunk_launch(const RemovalChunkArgs& a, int tokens, int num_seqs, hipStream_t stream) {
+  // (1,024 tokens beside 12 single ones, 32 heads of 64 x 64, us: with the longest portion's chunks for every sequence 55.4, so 51.0)
+  removal_chunk_prepare_kernel<T><<<(unsigned)(a.heads * step_items(tokens, num_seqs, CHUNK)), 256, removal_prepare_lds(a.dim, a.rank), stream>>>(a, num_seqs);
   const dim3 grid(a.heads, removal_columns(a.vdim) / 16, num_seqs);
   switch (a.dim / 16) {
     case 1: removal_chunk_scan_kernel<1><<<grid, 64, 0, stream>>>(a); break;
@@ -407,13 +406,13 @@ static void removal_chunk_launch(const RemovalChunkArgs& a, int num_seqs, int ma
 
 extern "C" int velox_removal_chunk_scan(const void* main, int dtype, int ld, int r_at, int k_at, int v_at, int a_at, int low_at, int rank, int heads, int dim,
                                         int vdim, const float* a_bias, const void* w2, const float* w0, float scale, float* scratch, float* state,
-                                        const int* slots, const int* cu_q, float* out, int num_seqs, int max_q_len, hipStream_t stream) {
-  if (num_seqs <= 0 || max_q_len <= 0) return 0;
-  if (velox_removal_chunk_scratch_elems(max_q_len, num_seqs, heads, dim, vdim, rank) == 0 || heads < 1 || heads > 65535 || num_seqs > 65535 ||
-      max_q_len > 65535 * CHUNK || !scratch || !(scale * CHUNK < 13.f))
+                                        const int* slots, const int* cu_q, float* out, int tokens, int num_seqs, hipStream_t stream) {
+  if (num_seqs <= 0 || tokens <= 0) return 0;
+  if (velox_removal_chunk_scratch_elems(tokens, num_seqs, heads, dim, vdim, rank) == 0 || heads < 1 || heads > 65535 || num_seqs > 65535 ||
+      heads * step_items(tokens, num_seqs, CHUNK) > 0x7fffffff || !scratch || !(scale * CHUNK < 13.f))
     return (int)hipErrorInvalidValue;
   RemovalChunkArgs a{main, ld, r_at, k_at, v_at, a_at, low_at, rank, heads, dim, vdim, a_bias, w2, w0, scale, scratch, state, slots, cu_q, out};
-  if (dtype == VELOX_BF16) removal_chunk_launch<bf16_t>(a, num_seqs, max_q_len, stream);
-  else removal_chunk_launch<float>(a, num_seqs, max_q_len, stream);
+  if (dtype == VELOX_BF16) removal_chunk_launch<bf16_t>(a, tokens, num_seqs, stream);
+  else removal_chunk_launch<float>(a, tokens, num_seqs, stream);
   VELOX_RETURN_LAUNCH_STATUS();
 }

@@ -180,7 +180,7 @@ class HipOps:
         c.velox_linear_scan_lanes.argtypes = [_I]
         c.velox_gated_head_norm.argtypes = [_P, _P, _F, _P, _I, _I, _I, _I, _P, _I, _I, _I, _I, _I, _P]
         c.velox_removal_prepare.argtypes = [_P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _I, _P]
-        c.velox_gated_scan.argtypes = [_P, _I, _I, _P, _P, _F, _P, _P, _P, _P, _P, _I, _I, _P]
+        c.velox_gated_scan.argtypes = [_P, _I, _I, _P, _P, _F, _P, _P, _P, _P, _P, _I, _I, _I, _P]
         c.velox_gated_scan_scratch_elems.argtypes = [_I, _I, _I]
         c.velox_gated_scan_scratch_elems.restype = ctypes.c_longlong
         c.velox_norm_add_norm.argtypes = [_P, _P, _I, _P, _F, _P, _F, _P, _P, _I, _I, _I, _I, ctypes.c_longlong, _P]
@@ -1382,7 +1382,7 @@ class HipOps:
         scratch = torch.empty(scratch_elems, dtype=torch.float32, device=self.device)
         self._launched(self._core.velox_removal_chunk_scan(_ptr(main), _code(main.dtype), main.shape[1], int(r_at), int(k_at), int(v_at), int(a_at), int(low_at), int(rank),
                                                            int(heads), int(dim), int(vdim), _ptr(a_bias), _ptr(w2), _ptr(w0), float(decay_scale), _ptr(scratch), _ptr(state),
-                                                           _ptr(slots), _ptr(cu_q), _ptr(out), slots.shape[0], int(max_q_len), self._stream()), "removal_scan")
+                                                           _ptr(slots), _ptr(cu_q), _ptr(out), tokens, slots.shape[0], self._stream()), "removal_scan")
         return out
 
     def gated_scan(self, projected, width, gate_bias, input_bias, shift, state, slots, cu_q, max_q_len):
@@ -1406,7 +1406,7 @@ class HipOps:
         elems = int(self._core.velox_gated_scan_scratch_elems(slots.shape[0], int(max_q_len), int(width)))
         scratch = torch.empty(elems, dtype=torch.float32, device=self.device) if elems else None
         self._launched(self._core.velox_gated_scan(_ptr(projected), _code(projected.dtype), int(width), _ptr(gate_bias), _ptr(input_bias), float(shift), _ptr(state),
-                                                   _ptr(slots), _ptr(cu_q), _ptr(out), _ptr(scratch), slots.shape[0], int(max_q_len), self._stream()), "gated_scan")
+                                                   _ptr(slots), _ptr(cu_q), _ptr(out), _ptr(scratch), tokens, slots.shape[0], int(max_q_len), self._stream()), "gated_scan")
         return out
 
     def linear_scan_supports(self, dim: int, vdim: int) -> None:
