@@ -1328,6 +1328,25 @@ def test_per_head_products_in_pieces_of_four_and_one_by_one(ops, n, k, gated):
     assert torch.all((results[0].float() - want).abs() <= 2.0 ** -8 * 1.01 * want.abs() + 1e-4)
 
 
+@pytest.mark.parametrize("rows, heads, n, k", [(2049, 8, 224, 96), (513, 32, 132, 72), (130, 128, 512, 128), (8193, 2, 260, 104)])
+@pytest.mark.parametrize("gated", [None, "output", "head"])
+def test_per_head_products_whose_maps_stay_in_registers(ops, rows, heads, n, k, gated):
+    """Remainders of the 16 rows, of a workgroup's rows, of 64 columns a wave and 32 indices: the bits of the same products in two launches of
+    half of the rows and fewer, which the kernel with the rows in LDS takes."""
+    x, maps = rand((rows, heads * k), torch.bfloat16, n), rand((heads, n, k), torch.bfloat16, k, k ** -0.5)
+    gate = None if gated is None else rand((rows, 8 + (heads * n if gated == "output" else heads)), torch.bfloat16, 3)
+    wide, few = n + 4, 16383 // heads
+
+    def run(first, last):
+        out = torch.full((last - first, heads * wide), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.head_linear(x[first:last], k, 0, maps, out, wide, 0, gate[first:last] if gate is not None else None, 4 if gate is not None else 0, gated == "head")
+        return out
+
+    whole = run(0, rows)
+    assert torch.all(whole.view(rows, heads, wide)[:, :, n:] == 7.0)
+    assert torch.equal(whole, torch.cat([run(at, min(rows, at + few)) for at in range(0, rows, few)]))
+
+
 @pytest.mark.parametrize("tokens", [65, 512, 513, 3072, 3073])
 @pytest.mark.parametrize("kv_heads, dim, heads, columns", [(3, 40, 6, 6), (8, 64, 8, 520)])
 def test_what_a_recurrence_reads_does_not_depend_on_how_tokens_are_spread(ops, tokens, kv_heads, dim, heads, columns):

@@ -377,9 +377,95 @@ static int grouped_plan_launch(const GroupedArgs& args, int tile_rows, int most_
   return (int)hipGetLastError();
 }
 
+// The products of `groups` groups that all run the same rows, where a group's matrix fits the registers of four waves: a wave keeps its 16 NT
+// rows of W whole (up to 32 KC indices, asked for once) and walks 16 rows of `a` at a time, straight from memory into matrix operands, the
+// next rows and their gates asked for before this step's products; no LDS and no barrier.  Bound by what it reads and writes and by the
+// loads in flight: rows are dealt out so that a compute unit has about two workgroups, which reads W rarely and leaves each several
+// steps.  The order of additions is that of grouped_mfma_kernel (indices beyond k are zeros).
+// Measured on MI355X, 2,500 rows, 32 heads of 224 x 96: 24.2 -> 17.9 us (51 MB: 2.1 -> 2.9 TB/s).
+// Needs k <= 32 KC and four outputs of a row and of its gates on 8-byte boundaries (GM_GATE with gate_col == 0: any).
+template <int EPI>
+__global__ void __launch_bounds__(256) head_rows_kernel(const GroupedArgs args, int rows_each) {
+  static_assert(EPI == GM_PLAIN || EPI == GM_GATE, "no other epilogue here");
+  constexpr int NT = 4, KC = 4;
+  const int group = blockIdx.z, first = blockIdx.y * rows_each, last = min(args.m, first + rows_each);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g4 = lane >> 4;
+  const int n = args.n, k = args.k, col0 = (blockIdx.x * 4 + wave) * (16 * NT);
+  if (col0 >= n) return;  // (the whole wave)
+  const bf16_t* w = args.w + (size_t)group * args.w_group + 8 * g4;
+  const bf16_t* a = args.a + (size_t)group * args.a_group + 8 * g4;
+  const bf16_t* gate = EPI == GM_GATE ? args.gate + (size_t)group * args.gate_group : nullptr;
+  bf16_t* out = reinterpret_cast<bf16_t*>(args.out) + (size_t)group * args.out_group;
+  gm_bf16x8_t w_op[NT][KC], a_next[KC], a_op[KC];
+  short4_t gate_next[NT], gate_now[NT];
+  auto ask = [&](int row0) {
+    const size_t row = min(row0 + i, last - 1);
+#pragma unroll
+    for (int c = 0; c < KC; ++c) a_next[c] = gm_load(a + row * args.a_ld + 32 * c, 32 * c + 8 * g4 < k);
+    if constexpr (EPI == GM_GATE) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const bf16_t* from = gate + row * args.gate_ld + (args.gate_col == 0 ? 0 : min(col0 + 16 * t + 4 * g4, n - 4));
+        if (args.gate_col == 0) gate_next[t][0] = __builtin_bit_cast(short, *from);
+        else gate_next[t] = *reinterpret_cast<const short4_t*>(from);
+      }
+    }
+  };
+  ask(first);
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int c = 0; c < KC; ++c) w_op[t][c] = gm_load(w + (size_t)min(col0 + 16 * t + i, n - 1) * k + 32 * c, 32 * c + 8 * g4 < k);
+  for (int row0 = first; row0 < last; row0 += 16) {
+#pragma unroll
+    for (int c = 0; c < KC; ++c) a_op[c] = a_next[c];
+    if constexpr (EPI == GM_GATE) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) gate_now[t] = gate_next[t];
+    }
+    if (row0 + 16 < last) ask(row0 + 16);
+    float4_t acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_op[t][c], a_op[c], acc[t], 0, 0, 0);
+    if (row0 + i >= last) continue;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int col = col0 + 16 * t + 4 * g4;
+      if (col >= n) continue;
+      typedef bf16_t Four __attribute__((ext_vector_type(4)));
+      Four four;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float v = acc[t][j];
+        if (EPI == GM_GATE) {
+          const float z = __uint_as_float(((uint32_t)(uint16_t)gate_now[t][args.gate_col == 0 ? 0 : j]) << 16);
+          v *= 1.f / (1.f + expf(-z));
+        }
+        four[j] = from_f32<bf16_t>(v);
+      }
+      *reinterpret_cast<Four*>(out + (size_t)(row0 + i) * args.out_ld + col) = four;
+    }
+  }
+}
+
 // The products of `groups` groups that all run rows [0, m).
 template <int EPI, typename TO>
 static void grouped_rows_launch(const GroupedArgs& args, int groups, hipStream_t stream) {
+  const bool fours = ((args.n | args.out_ld | args.out_group) & 3) == 0 && ((uintptr_t)args.out & 7) == 0;
+  const bool gates = EPI != GM_GATE || args.gate_col == 0 || (args.gate_col == 1 && ((args.gate_ld | args.gate_group) & 3) == 0 && ((uintptr_t)args.gate & 7) == 0);
+  // wide outputs of short sums, with rows enough for several steps of 16 a workgroup (us, grouped_mfma_kernel / head_rows_kernel: 32 heads of
+  // 224 x 96: 200 rows 7.6 / 8.1, 1,000 10.6 / 10.1, 2,500 24.2 / 17.9, 4,096 33.4 / 25.6; 128 of 512 x 128: 64 rows 9.9 / 11.2, 200 27.2 / 20.5, 1,000 75 /
+  // 62, 4,096 382 / 315.  Longer sums or up to 128 outputs were not quicker in it: 32 of 128 x 224 with gates, 2,500 rows 28.0 / 30.4, 16 of 256 x 256
+  // 24.7 / 27.0, 64 of 128 x 64 with gates 32.2 / 32.8)
+  if (sizeof(TO) == 2 && fours && gates && args.n > 128 && args.k > 64 && args.k <= 128 && (long long)args.m * groups >= 16384) {
+    const int columns = (args.n + 255) / 256, parts = max(1, 2 * TL_WORKGROUPS / (columns * groups)), rows_each = ((args.m + parts - 1) / parts + 15) / 16 * 16;
+    head_rows_kernel<EPI><<<dim3(columns, (args.m + rows_each - 1) / rows_each, groups), 256, 0, stream>>>(args, rows_each);
+    return;
+  }
   const int row_tiles = (args.m + GM_ROWS - 1) / GM_ROWS;
   if (args.n <= 128) grouped_mfma_kernel<EPI, TO, 2><<<dim3(1, row_tiles, groups), 256, 0, stream>>>(args);
   else grouped_mfma_kernel<EPI, TO, 4><<<dim3((args.n + 255) / 256, row_tiles, groups), 256, 0, stream>>>(args);
