@@ -81,18 +81,6 @@ __device__ __forceinline__ float4_t lower_times(const float4_t l, const float* L
   return acc;
 }
 
-// The last sequence whose first record is not behind `record` (-1: none), the same in every lane.
-__device__ __forceinline__ int sequence_of(int record, const int* cu_q, int num_seqs, int lane) {
-  int before = 0;
-  for (int s0 = 0; s0 < num_seqs; s0 += 64) {
-    const int s = s0 + lane;
-    const int found = __popcll(__ballot(s < num_seqs && first_chunk(cu_q[s], s) <= record));  // (first records rise from sequence to sequence)
-    before += found;
-    if (found < 64) break;
-  }
-  return __builtin_amdgcn_readfirstlane(before) - 1;
-}
-
 // The grid counts records, of which there are about as many as chunks: one per longest portion's chunk and sequence would be a hundred
 // thousand workgroups that only end, for 60 single tokens beside 1,000.  Measured on MI355X (us a step with the kernels for the short ones
 // behind it; token by token / everything in chunks with such a grid / this): 60 single tokens beside 1,000, 16 heads of 128 x 128 519 / 195 /
@@ -103,10 +91,8 @@ __global__ void __launch_bounds__(256) linear_chunk_prepare_kernel(const LinearC
   float* lds = reinterpret_cast<float*>(lds_pieces);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int record_at = blockIdx.x / a.head_count, local_head = blockIdx.x % a.head_count, h = a.first_head + local_head;
-  const int b = sequence_of(record_at, a.cu_q, a.num_seqs, lane);
-  if (b < 0) return;  // (the whole workgroup)
-  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
-  const int t0 = lo + (record_at - first_chunk(lo, b)) * CHUNK;
+  const StepItem item = step_item(a.cu_q, a.num_seqs, CHUNK, record_at);
+  const int lo = item.lo, hi = item.hi, t0 = lo + item.piece * CHUNK;
   if (t0 >= hi || hi - lo < a.long_from) return;  // (the whole workgroup)
   const int count = hi - t0 < CHUNK ? hi - t0 : CHUNK;
   const int n = lane & 15, g = lane >> 4;  // column and group of four rows in the matrix instructions' layouts

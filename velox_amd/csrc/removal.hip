@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(256) removal_chunk_prepare_kernel(const Remova
   float* matrix[4] = {lds, lds + CHUNK * row, lds + 2 * CHUNK * row, lds + 3 * CHUNK * row};
   float* decays = lds + 4 * CHUNK * row;
   float* inner = decays + CHUNK * row;
-  float* small = inner + CHUNK * inner_row;
+  float* small = decays;  // (the decays and the inner rows are of no use behind the running products)
   const T* rows = (const T*)a.main + (size_t)t0 * a.ld;
 
   // a wave takes four tokens and a lane two channels of each (dim <= 128): all of a wave's loads are asked for before the first
@@ -376,20 +376,23 @@ __global__ void __launch_bounds__(64 * WAVES, 2) removal_chunk_scan_kernel(const
   }
 }
 
+// LDS of removal_chunk_prepare_kernel.  Its time is that of its dependent steps, so workgroups per compute unit count: with the small
+// matrices where the decays were six instead of four of them hold 64 channels and an inner size of 64 (26 KB, not 35).
 static size_t removal_prepare_lds(int dim, int rank) {
-  const int padded_rank = (rank + 15) / 16 * 16;
-  return (size_t)CHUNK * (5 * (dim + 4) + padded_rank + 4 + 7 * CHUNK_STRIDE) * sizeof(float);
+  const int row = dim + 4, inner_row = (rank + 15) / 16 * 16 + 4;
+  return (size_t)CHUNK * (4 * row + (row + inner_row > 7 * CHUNK_STRIDE ? row + inner_row : 7 * CHUNK_STRIDE)) * sizeof(float);
 }
 
 // float32 elements of the scratch of a step; 0: these sizes are not for these kernels
 extern "C" long long velox_removal_chunk_scratch_elems(int tokens, int num_seqs, int heads, int dim, int vdim, int rank) {
-  if (dim % 16 != 0 || dim < 16 || dim > 128 || vdim < 1 || rank < 1 || removal_prepare_lds(dim, rank) > 64 * 1024) return 0;
+  if (dim % 16 != 0 || dim < 16 || dim > 128 || vdim < 1 || rank < 1 || removal_prepare_lds(dim, rank) > 55 * 1024) return 0;
   return (step_items(tokens, num_seqs, CHUNK) + 1) * heads * (long long)removal_record(dim, vdim);
 }
 
 template <typename T>
 static void removal_chunk_launch(const RemovalChunkArgs& a, int tokens, int num_seqs, hipStream_t stream) {
-  // (1,024 tokens beside 12 single ones, 32 heads of 64 x 64, us: with the longest portion's chunks for every sequence 55.4, so 51.0)
+  // (1,024 tokens beside 12 single ones, 32 heads of 64 x 64, us: with the longest portion's chunks for every sequence 55.4, so 51.0, and six workgroups per
+  // compute unit 44.4)
   removal_chunk_prepare_kernel<T><<<(unsigned)(a.heads * step_items(tokens, num_seqs, CHUNK)), 256, removal_prepare_lds(a.dim, a.rank), stream>>>(a, num_seqs);
   const dim3 grid(a.heads, removal_columns(a.vdim) / 16, num_seqs);
   switch (a.dim / 16) {
