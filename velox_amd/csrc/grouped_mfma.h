@@ -308,7 +308,8 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
 }
 
 // The rows of a tile of the plan's products: 64 up to 64 pairs, above 128 or 192 (tiles_mfma.h's kernel, 256 rows of W), whichever is likely to
-// cost less: an expert's last tile is half empty on average, and all tiles take whole rounds over the compute units.  k % 64 != 0 is
+// cost less: an expert's last tile is half empty on average, none has less than one (1,340 pairs over 32 experts of 4,096 -> 1,408 read W, us of
+// the two products in tiles of 192 rows 177 + 76, of 128, whose loads are further ahead, 169 + 72), and all tiles take whole rounds over the compute units.  k % 64 != 0 is
 // built for 128.  (Tiles of 64 rows were no quicker at any number of pairs above 64: 12 rows per expert 66 us either way, 56: 80 /
 // 81, 75: 100 / 83, 130: 127 / 125, 256: 187 / 155, 16 experts of 2,048 -> 1,408 -> 2,048.)
 static inline int grouped_tile_rows(int pairs, int experts, int inter, int hidden, int branches) {
@@ -318,7 +319,7 @@ static inline int grouped_tile_rows(int pairs, int experts, int inter, int hidde
   for (int rt = 2; rt <= 3; ++rt) {
     const TileCost* t = TILE_COSTS;
     while (t->rt != rt || t->ct != 4) ++t;
-    const long long rows = (long long)(experts * ((float)pairs / (experts * 64 * rt) + 0.5f)) * 64 * rt;
+    const long long rows = (long long)(experts * fmaxf(1.f, (float)pairs / (experts * 64 * rt) + 0.5f)) * 64 * rt;
     cost[rt - 2] = tiles_cost(*t, rows, (long long)branches * inter, hidden, 1) + tiles_cost(*t, rows, hidden, inter, 1);
   }
   return cost[1] < cost[0] ? 192 : 128;
