@@ -1602,3 +1602,16 @@ def test_float32_products_of_numbers_that_do_not_split(ops, tile):
     sizes = torch.where(a.isfinite(), a, 0).double().abs() @ torch.where(w.isfinite(), w, 0).double().abs().T
     assert torch.all(((got.double() - want.double()).abs() <= 160 * 2.0 ** -23 * sizes)[whole])
     assert torch.all(got[131][want[131].isfinite()] == 0)
+
+
+@pytest.mark.parametrize("tile", [128256, 96192, 64064])
+@pytest.mark.parametrize("exponent", [-44, -40, -38, -36, -34, -30])
+def test_float32_products_of_tiny_and_huge_numbers(ops, tile, exponent):
+    """Operands whose lower parts are far below bfloat16's smallest numbers, times large ones: as exact as any.  The sums of 512 terms of random signs
+    show 1.6e-7 of their norm."""
+    generator = torch.Generator(device="cuda").manual_seed(-exponent)
+    tiny, huge = (torch.randn(132, 512, generator=generator, device="cuda").double() * s for s in (10.0 ** exponent, 1e20))
+    tiny, huge = tiny.float(), huge.float()
+    for a, w in ((tiny, huge), (huge, tiny)):
+        want = a.double() @ w.double().T
+        assert float((ops.split_f32(a, w, tile=tile).double() - want).norm() / want.norm()) <= 3e-7

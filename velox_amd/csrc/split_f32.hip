@@ -1,6 +1,7 @@
 // out[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) of float32 operands on the bfloat16 matrix instructions of gfx950, which multiply 16 times as
-// fast as the float32 ones, with no bit of an operand left out: a float32 number is the sum of three bfloat16 ones (x = hi + mid +
-// lo, each the nearest to what is left: 8 + 8 + 8 significant bits), their products are exact in float32, and of the nine products
+// fast as the float32 ones, with no bit of an operand left out: a float32 number, times 2^24, is the sum of three bfloat16 ones (hi + mid +
+// lo, each the nearest to what is left: 8 + 8 + 8 significant bits; without the factor, parts of a number below 2^-109 are beyond bfloat16's
+// smallest ones, and 1e-36 times 1e20 came out with an error of 3e-5, 1e-38 with 3e-3; the multiplication costs no time), their products are exact in float32, and of the nine products
 // of parts six count, hi hi + hi mid + mid hi + hi lo + mid mid + lo hi (the other three are 2^-26 of a term; the method is that of
 // Henry, Tang, Heinecke: Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations, 2019).
 //
@@ -12,7 +13,7 @@
 // sums of 1,024 in the result's place: 190 instead of 180 us where 1,536 terms are added, for the passes over the result.)
 //
 // What bounds it: the matrix cores (six instructions of 16 cycles for 16 x 16 x 32 terms: at most 2,500 / 6 = 417 TFLOP/s of float32
-// products, 250 at the rate that power leaves them), and beside them the splitting: 44 vector instructions for eight numbers.
+// products, 250 at the rate that power leaves them), and beside them the splitting: 52 vector instructions for eight numbers.
 //   - Eight waves own 32 RT x 64 CT outputs.  A step is 32 indices: operands come into registers a step ahead, are split ONCE per
 //     workgroup on their way into LDS (not by each wave that reads them: half of the vector work) and lie there as three planes, two buffers.
 //   - Half of the waves split before they multiply and half behind it, so that the vector units and the matrix cores have work at the
@@ -30,6 +31,7 @@ typedef float sp_float8_t __attribute__((ext_vector_type(8)));
 
 #define SPLIT_FOLD 4    // steps of 32 terms per inner sum
 #define SPLIT_LEVEL 64  // steps whose inner sums are added up in registers, at most
+#define SPLIT_SCALE 0x1p24f  // of either operand
 #define SPLIT_XCDS 8
 #define SPLIT_CUS 256
 
@@ -43,8 +45,8 @@ struct SplitArgs {
 };
 
 // The same outputs with the float32 matrix instruction, from memory, for the rows and columns of one wave.  It is taken where a sum is no
-// finite number (an infinity, a number that rounds to one, NaN: their parts are not what they should be) or is so small, below 2^-80
-// but not zero, that an operand's lower parts may be beyond bfloat16's smallest numbers.  Slow and seldom.
+// finite number: an operand is an infinity, NaN or beyond 2^104, or the sum is beyond 2^80, where the factors leave float32's range.  Slow
+// and seldom.
 template <int RT, int CT>
 __device__ __forceinline__ void split_outputs_in_float32(const SplitArgs& args, int row0, int col0, int part) {
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
@@ -112,7 +114,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int j = 0; j < J; ++j)
       if ((j + 1) * 512 <= PIECES || wave * 64 + 512 * j < PIECES) {
-        sp_float8_t x = __builtin_shufflevector(raw[j][0], raw[j][1], 0, 1, 2, 3, 4, 5, 6, 7);
+        sp_float8_t x = __builtin_shufflevector(raw[j][0], raw[j][1], 0, 1, 2, 3, 4, 5, 6, 7) * SPLIT_SCALE;
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
           sp_uint4_t bits;
@@ -218,7 +220,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       if (begun) v += *p;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        beyond |= !(fabsf(v[u]) < INFINITY) || (v[u] != 0.f && fabsf(v[u]) < 0x1p-80f);
+        beyond |= !(fabsf(v[u]) < INFINITY);
+        v[u] *= 1.f / (SPLIT_SCALE * SPLIT_SCALE);
         if (args.bias != nullptr) v[u] += args.bias[col0 + 16 * c + 4 * h + u];
       }
       *p = v;
