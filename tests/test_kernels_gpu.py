@@ -2,6 +2,7 @@
 bfloat16, at sizes other than the engine's tiny models: widths and vocabularies that are no power
 of two, head sizes 16 .. 256, groups of 1, 3, 7, page sizes 4 .. 64."""
 import math
+import threading
 
 import numpy as np
 import pytest
@@ -1425,8 +1426,8 @@ def test_gated_products_in_every_tile(ops, m, n, k, activation):
         assert torch.all(error[finite] <= 0)
 
 
-@pytest.mark.parametrize("m, n, k, own", [(64, 4096, 2048, False), (65, 4096, 2048, True), (300, 4608, 3584, False), (836, 37888, 3584, True), (836, 4608, 3584, True), (1036, 64, 2048, True),
-                                          (1036, 56, 2048, False), (1036, 4100, 2048, False), (1036, 4096, 2056, False), (1036, 4096, 192, False)])
+@pytest.mark.parametrize("m, n, k, own", [(64, 4096, 2048, False), (65, 4096, 2048, True), (300, 4608, 3584, False), (836, 37888, 3584, True), (836, 4608, 3584, True), (1036, 64, 2048, False),
+                                          (768, 64, 2048, True), (769, 64, 2048, False), (2421, 128, 2048, False), (1408, 1536, 1024, False), (1409, 1536, 1024, True), (1036, 56, 2048, False), (1036, 4100, 2048, False), (1036, 4096, 2056, False), (1036, 4096, 192, False)])
 def test_which_products_run_in_the_own_tiles(ops, monkeypatch, m, n, k, own):
     calls = []
     monkeypatch.setattr(ops, "gemm_tiles", lambda *a, **more: calls.append(a) or type(ops).gemm_tiles(ops, *a, **more))
@@ -1435,6 +1436,38 @@ def test_which_products_run_in_the_own_tiles(ops, monkeypatch, m, n, k, own):
     assert ops.tiles_serve(m, n, k) == own and len(calls) == int(own) and type(ops).library_serves(ops, m, n, k) == (m > 64 and not own)
     want = x.double() @ w.double().T + bias.double()
     assert torch.all((got.double() - want).abs() <= 2.0 ** -7 * (want.abs() + bias.double().abs()) + k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T))
+
+
+@pytest.mark.parametrize("m, n, k, own", [(128, 64, 2048, False), (100, 2048, 2048, False), (200, 1536, 1024, False), (256, 768, 256, False), (128, 18432, 256, True)])
+def test_products_of_recorded_steps(ops, monkeypatch, m, n, k, own):
+    """What is recorded takes the library where tiles are few, and another thread's products do not.  Replays on other rows, with eager work between
+    them, against float64 within a rounding of the result and the additions' own."""
+    calls = []
+    monkeypatch.setattr(ops, "gemm_tiles", lambda *a, **more: calls.append(a) or type(ops).gemm_tiles(ops, *a, **more))
+    x, w = rand((m, k), torch.bfloat16, 1), rand((n, k), torch.bfloat16, 2, k ** -0.5)
+    elsewhere = []
+    with ops.recording():
+        thread = threading.Thread(target=lambda: elsewhere.append(ops.tiles_serve(m, n, k)))
+        thread.start()
+        thread.join()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            ops.linear(x, w, None, torch.bfloat16)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = ops.linear(x, w, None, torch.bfloat16)
+    assert elsewhere == [True] and len(calls) == 2 * int(own)
+    for seed in range(4):
+        x.copy_(rand((m, k), torch.bfloat16, 10 + seed))
+        graph.replay()
+        torch.cuda.synchronize()
+        want = x.double() @ w.double().T
+        assert torch.all((out.double() - want).abs() <= 2.0 ** -8 * 1.01 * want.abs() + k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T))
+        ops.linear(x, w, None, torch.bfloat16)
+    assert len(calls) == 4 + 2 * int(own)
 
 
 @pytest.mark.parametrize("m, n, k, parts", [(65, 2560, 8192, 8), (300, 2048, 8448, 8), (700, 2048, 5632, 5), (700, 1024, 28672, 8), (300, 4096, 16512, 5), (129, 8192, 16384, 4)])

@@ -22,6 +22,7 @@ scratch are the runner's own buffers.
 """
 from __future__ import annotations
 
+import contextlib
 import time
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -168,14 +169,15 @@ class ModelRunner:
     def _capture(self, ctx: StepContext, warmup_iters: int):
         stream = torch.cuda.Stream(device=self.device)
         stream.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(stream):
-            for _ in range(warmup_iters):
-                self._forward(ctx)
-        torch.cuda.current_stream().wait_stream(stream)
-        torch.cuda.synchronize()
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, pool=self._graph_pool):
-            logits = self._forward(ctx)
+        with getattr(self.ops, "recording", contextlib.nullcontext)():
+            with torch.cuda.stream(stream):
+                for _ in range(warmup_iters):
+                    self._forward(ctx)
+            torch.cuda.current_stream().wait_stream(stream)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, pool=self._graph_pool):
+                logits = self._forward(ctx)
         return graph, logits, ctx
 
     def _graph_context(self, bucket: int, max_kv_len: int) -> StepContext:

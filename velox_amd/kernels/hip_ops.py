@@ -12,10 +12,12 @@ a library has no call for.  bfloat16 x bfloat16 products go to the library behin
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import logging
 import os
 import tempfile
+import threading
 from typing import Tuple, Dict, Optional
 
 import torch
@@ -76,6 +78,10 @@ def _weight_of(weight) -> Tuple[torch.Tensor, Optional[PreparedWeight]]:
     return weight, None
 
 
+class _Recording(threading.local):
+    on = False
+
+
 class HipOps:
     name = "hip-gfx950"
     MAX_TILED_HEAD_DIM = 256  # head sizes above this go to the plain attention kernel
@@ -101,6 +107,7 @@ class HipOps:
         self.use_grouped_mfma = True  # (False: the grouped bfloat16 products take the exact multiply-add tiles, for tests)
         self._mm_out_dtype_ok: Optional[bool] = None
         self._bias_copies: Dict[Tuple[int, int], Tuple[torch.Tensor, torch.Tensor]] = {}
+        self._recording = _Recording()
         self._raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
     # -- loading --------------------------------------------------------------------------------
@@ -993,7 +1000,7 @@ class HipOps:
             return out
         if (not fused and activation != "gelu_tanh" and deferred is None and self.use_library_gemm and x.dim() == 2 and gate_up_weight.dim() == 2 and two_n % 16 == 0
                 and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16 and out_dtype == torch.bfloat16 and gate_up_weight.shape[1] == k
-                and (two_n // 2 + 256) * k < 1 << 30 and self.tiles_serve(m, two_n, k) and not self._library_has_timed(m, two_n, k)):
+                and (two_n // 2 + 256) * k < 1 << 30 and self.tiles_serve(m, two_n, k, gated=True) and not self._library_has_timed(m, two_n, k)):
             # many rows: the activation where the tiles' sums are finished.  Both sums are rounded to bfloat16 in front of it, as a
             # product of its own leaves them
             self._check("x", x, align=16)
@@ -1071,7 +1078,7 @@ class HipOps:
 
         (With residual streams, whose norm adds the parts too: 4,096 x 11,008 at 100 rows 45 / 39, 512: 87 / 72; 2,048 x 8,448 at 300: 43 / 34;
         2,048 x 5,632 at 300: 28 / 29, 512: 32 / 34, 1,280: 63 / 58.)"""
-        if m <= 64 or k < 5120 or k % 8 != 0 or n % 4 != 0:
+        if m <= 64 or not 5120 <= k < 1 << 21 or k % 8 != 0 or n % 4 != 0:
             return 0
         tiles, steps = -(-m // 128) * -(-n // 256), -(-k // 64)
         if 3 * tiles <= self.num_cus:
@@ -1084,17 +1091,38 @@ class HipOps:
             return 0
         return -(-steps // -(-steps // splits))  # (no empty part)
 
-    def tiles_serve(self, m: int, n: int, k: int) -> bool:
+    def tiles_serve(self, m: int, n: int, k: int, gated: bool = False, recorded: Optional[bool] = None) -> bool:
         """Whether a whole bfloat16 product of more than 64 rows runs in the framework's own tiles (``gemm_tiles``; the tile is picked in
-        tiles_mfma.h).  The library is left what has few tiles of 128 x 128 and a sum of more than 2,048 terms, where it cuts the
-        sum: 300 rows of 4,608 x 3,584 (108 tiles) 22 us by the library and 25 here, 512 of 4,096 x 4,096 (128) 30 / 33, 836 of 2,048 x
-        5,632 (112) 34 / 41.  Elsewhere, of 27 shapes from 1,536 x 1,536 to 37,888 x 3,584 at 16 numbers of rows, the own tiles took
-        0.90 of the library's time on average and 1.17 at worst, and their call costs the host 8 us instead of 19: 836 rows of 37,888 x
-        3,584 268 / 198, 2,048 535 / 409; 4,001 of 22,016 x 4,096 640 / 530, of 4,096 x 4,096 90 / 91; 1,036 of 10,368 x 2,048 49 / 38; 2,048 of
-        4,608 x 3,584 56 / 56."""
-        if m <= 64 or n % 8 != 0 or n < 64 or k % 64 != 0 or k < 256:
+        tiles_mfma.h).  ``gated``: with the activation where its sums end, which spares a pass.  ``recorded``: whether it goes into a graph
+        (default: as ``recording`` says).  The library is left what has few tiles of 128 x 128: it cuts its sum or has smaller tiles for it.  The
+        lines, of 16 shapes from 4,096 x 2,048 to 57,344 x 8,192 and 60 from 64 x 256 to 2,048 x 2,048 at 10 numbers of rows (us of the GPU, weights from memory, the
+        library / own):
+
+        - sums of more than 2,048 terms: from 3/4 of a tile per compute unit on (4,608 x 3,584 at 512 rows, 144 tiles, 32 / 37, at 700, 216, 36 / 32; 4,096 x 4,096 at 512
+          29 / 37; 12,288 x 4,096 at 200, 192, 40 / 38; 37,888 x 3,584 at 1,000 295 / 241; at worst 81 / 69 the other way, 27,648 x 5,120 at 160).
+        - shorter ones: from 9/16 on (6,144 x 2,048 at 200, 96 tiles, 16 / 19, at 384, 144, 24 / 22; 2,048 x 2,048 at 700 13 / 17, at 1,036, 144, 20 / 18; 1,536 x 1,024 at 1,036,
+          108, 9.6 / 10.9, at 1,536, 144, 11.7 / 11.4; 17,920 x 1,536 at 100, 140, 23 / 21; 128 x 2,048 at 2,421, 19, 10.7 / 16.0), with the activation from 3/8 on (128 rows and eight
+          layers of width 1,536, a step 898 / 854).
+        - and up to 768 rows below that where nothing is recorded: the library's call costs the host 19 us, the own one 8, and a step of
+          so few rows waits for the host (a step of eight layers, us, the library for these / own tiles: width 1,536 at 150 tokens 1,220 / 957, at 600 1,218 / 1,196, at
+          1,000 1,517 / 1,536; 2,048, with products of 64 to 512 columns, at 300 2,384 / 1,974, at 600 2,386 / 2,107, at 1,000 2,557 / 2,615).  A recorded step waits for nothing (128
+          rows: 898 / 1,016 and 2,098 / 2,348)."""
+        if m <= 64 or n % 8 != 0 or n < 64 or k % 64 != 0 or not 256 <= k < 1 << 21:
             return False
-        return k <= 2048 or -(-m // 128) * -(-n // 128) * 4 >= 3 * self.num_cus
+        tiles = -(-m // 128) * -(-n // 128)
+        if k > 2048:
+            return 4 * tiles >= 3 * self.num_cus
+        return 16 * tiles >= (6 if gated else 9) * self.num_cus or (m <= 768 and not (self._recording.on if recorded is None else recorded))
+
+    @contextlib.contextmanager
+    def recording(self):
+        """Around the passes that are recorded into a graph and those that warm up for them: of two kernels the one is taken that the GPU is through
+        with sooner, whatever its call costs the host.  Holds for the calling thread."""
+        before, self._recording.on = self._recording.on, True
+        try:
+            yield
+        finally:
+            self._recording.on = before
 
     @staticmethod
     def _library_has_timed(m: int, n: int, k: int) -> bool:
