@@ -249,6 +249,23 @@ def test_library_tuning_recaptures_the_decode_graphs_and_keeps_the_logits(tmp_pa
             assert logits[step][token] >= logits[step].max() - 0.05  # the chosen token is the best one up to rounding
 
 
+def test_products_that_are_taken_in_parts_are_not_timed(tmp_path, monkeypatch):
+    """A long sum whose parts the next norm adds runs in the own tiles and is not timed; the same product with a bias, or wanted whole, is the library's."""
+    engine = engine_for(make_folder(tmp_path, "A", "bfloat16"), "A", "bfloat16", max_num_seqs=4, max_num_batched_tokens=64)
+    timed = []
+    monkeypatch.setattr(engine.ops, "tune_library_products", lambda shapes, counts, results_file=None: timed.extend(shapes) or len(shapes))
+    mixer, feed_forward = engine.model.blocks[0].mixer, engine.model.blocks[0].feed_forward
+    wanted = {tuple(w.shape) for w in (mixer.qkv_weight, feed_forward.gate_up_weight)}
+    in_parts = {tuple(w.shape) for w in (mixer.o_weight, feed_forward.down_weight)}
+    assert wanted.isdisjoint(in_parts)
+    engine.tune_matrix_products([128])
+    assert wanted | in_parts <= set(timed)  # (short sums: no parts)
+    timed.clear()
+    monkeypatch.setattr(engine.ops, "tile_splits", lambda m, n, k: 2)
+    engine.tune_matrix_products([129])
+    assert wanted <= set(timed) and in_parts.isdisjoint(timed)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_requests_that_take_over_a_published_prefix(tmp_path, dtype):
     """Prefix caching on the GPU, with captured decode steps: a request whose prompt begins like an earlier one computes

@@ -1470,6 +1470,21 @@ def test_products_of_recorded_steps(ops, monkeypatch, m, n, k, own):
     assert len(calls) == 4 + 2 * int(own)
 
 
+@pytest.mark.parametrize("m, n, k, in_parts", [(128, 10240, 8192, 6), (128, 7168, 5120, 8), (700, 7168, 5120, 1), (300, 4608, 3584, 0), (836, 4608, 3584, 1), (70, 2048, 2048, 1)])
+def test_the_library_is_said_to_serve_what_linear_hands_to_it(ops, monkeypatch, m, n, k, in_parts):
+    """With a bias, whole and in parts: a long sum over few tiles runs in the own tiles where its parts are wanted and in the library where not."""
+    calls = []
+    monkeypatch.setattr(ops, "gemm_tiles", lambda *a, **more: calls.append(a) or type(ops).gemm_tiles(ops, *a, **more))
+    x, w, bias = rand((m, k), torch.bfloat16, 1), rand((n, k), torch.bfloat16, 2, k ** -0.5), rand((n,), torch.float32, 3)
+    for given in (bias, None):
+        calls.clear()
+        assert ops.linear(x, w, given, torch.bfloat16).shape == (m, n)
+        assert ops.library_serves(m, n, k) == (not calls) == (in_parts != 1)
+    calls.clear()
+    got = ops.linear(x, w, None, torch.bfloat16, partials_ok=True)
+    assert ops.own_tile_parts(m, n, k, True) == in_parts and len(calls) == (in_parts > 0) and (got.shape == (in_parts, m, n) if in_parts > 1 else got.shape == (m, n))
+
+
 @pytest.mark.parametrize("m, n, k, parts", [(65, 2560, 8192, 8), (300, 2048, 8448, 8), (700, 2048, 5632, 5), (700, 1024, 28672, 8), (300, 4096, 16512, 5), (129, 8192, 16384, 4)])
 def test_linear_with_parts_of_a_long_sum_into_every_consumer(ops, ref, m, n, k, parts):
     """More than 64 rows of a long product come back as partial sums.  Each kernel that takes them gives what it gives for their float32

@@ -171,23 +171,27 @@ class Engine:
         the given numbers of tokens per step (typically the prefill chunk size and the larger decode batch sizes) and
         keep the fastest.  Takes seconds per shape.  A step of prompt portions with a few rows less than one of these
         counts is padded up to it from then on (``ModelRunner.tuned_row_counts``); other steps are unaffected.  Only products that
-        the engine hands to the library are timed (``ops.library_serves``); captured decode steps are captured again
+        the engine hands to the library are timed (``ops.library_serves``, and not what it takes in parts from the own tiles); captured decode steps are captured again
         if one of them holds such a product.  ``progress(text)``, if given, is told after every count (a ladder of
         counts takes minutes)."""
         if self.dtype != torch.bfloat16 or self.device.type != "cuda" or not hasattr(self.ops, "tune_library_products"):
             return 0
-        shapes = set()
+        shapes = {}  # (N, K) -> whether some part takes its products in parts alone
         for part in self.model.all_parts():
             for attr, param in part.params().items():
                 tensor = getattr(part, attr, None)
                 if param.role == "matrix" and param.product and tensor is not None and tensor.dim() == 2 and tensor.dtype == torch.bfloat16:
-                    shapes.add(tuple(tensor.shape))
+                    shape = tuple(tensor.shape)
+                    shapes[shape] = shapes.get(shape, True) and attr in part.products_in_parts
         done = 0
         recapture = False
         results_file = self.ops.tuning_file() if self.config.library_tuning_file == "auto" else self.config.library_tuning_file
         counts = sorted(set(int(m) for m in token_counts))
         for index, count in enumerate(counts):
-            served = [shape for shape in shapes if self.ops.library_serves(count, *shape)]
+            recorded = self.runner.uses_graphs and count <= self.config.max_num_seqs
+            served = [shape for shape, in_parts in shapes.items()
+                      if (self.ops.library_serves(count, *shape) or (recorded and self.ops.library_serves(count, *shape, recorded=True)))
+                      and not (in_parts and self.ops.tile_splits(count, *shape) > 0)]
             if served:
                 done += self.ops.tune_library_products(served, [count], results_file=results_file)
                 if progress is not None:

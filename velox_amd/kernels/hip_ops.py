@@ -299,14 +299,14 @@ class HipOps:
         values = torch.arange((heads + kv_heads) * head_dim, (heads + 2 * kv_heads) * head_dim, device=device)
         return torch.cat([rotary, values])
 
-    def library_serves(self, m: int, n: int, k: int) -> bool:
-        """Whether ``linear`` hands ``x[m, k] @ w[n, k]^T`` in bfloat16 to the matrix library, and the product is large
+    def library_serves(self, m: int, n: int, k: int, recorded: Optional[bool] = None) -> bool:
+        """Whether ``linear`` hands ``x[m, k] @ w[n, k]^T`` in bfloat16, with a bias or wanted whole, to the matrix library, and the product is large
         enough for the library's timing of its candidates to mean something (a weight of a few megabytes is timed
-        from the caches, which says little about a step that streams it from memory)."""
+        from the caches, which says little about a step that streams it from memory).  ``recorded``: as for ``tiles_serve``."""
         if not self.use_library_gemm:
             return False
         if m > 64:
-            return not self.tiles_serve(m, n, k) and self.tile_splits(m, n, k) == 0
+            return self.own_tile_parts(m, n, k, False, recorded) == 0
         return m > 16 and n > 8192 and n * k >= (32 << 20)
 
     def tuning_file(self) -> Optional[str]:
@@ -816,13 +816,10 @@ class HipOps:
         if (partials_ok and bias is None and self.use_skinny_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
                 and 16 < m <= 64 and k % 64 == 0 and n <= 8192 and n % 4 == 0):
             return self.skinny_gemm_splitk(x, weight, packed=packed)
-        if bias is None and out_dtype == torch.bfloat16 and self.use_library_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
-            splits = self.tile_splits(m, n, k)
-            if (splits == 1 or (splits > 1 and partials_ok)) and not self._library_has_timed(m, n, k):
-                return self.gemm_tiles(x, weight, splits, torch.bfloat16 if splits == 1 else torch.float32)
-        if (out_dtype == torch.bfloat16 and self.use_library_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
-                and self.tiles_serve(m, n, k) and not self._library_has_timed(m, n, k)):
-            return self.gemm_tiles(x, weight, bias=bias)
+        if out_dtype == torch.bfloat16 and self.use_library_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
+            parts = self.own_tile_parts(m, n, k, partials_ok and bias is None)
+            if parts > 0 and not self._library_has_timed(m, n, k):
+                return self.gemm_tiles(x, weight, parts, torch.bfloat16 if parts == 1 else torch.float32, bias)
         skinny_rows = 16 if n > 8192 else 32  # measured on MI355X: beyond this the library's kernels stream faster
         if self.use_skinny_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and m <= skinny_rows and k % 64 == 0:
             return self.skinny_gemm(x, weight, bias, out_dtype, packed=packed, x_packed=self._packed_rows_of(x, k))
@@ -1054,6 +1051,14 @@ class HipOps:
         self._launched(status, "skinny_gemm_splitk")
         return out
 
+    def own_tile_parts(self, m: int, n: int, k: int, in_parts: bool, recorded: Optional[bool] = None) -> int:
+        """Parts of k in which ``linear`` works a bfloat16 product of more than 64 rows in the own tiles: 0, it goes to the library; 1, a whole
+        result; more, with ``in_parts`` (float32 partial sums are wanted) alone.  ``recorded``: as for ``tiles_serve``."""
+        splits = self.tile_splits(m, n, k)
+        if splits == 1 or (splits > 1 and in_parts):
+            return splits
+        return int(self.tiles_serve(m, n, k, recorded=recorded))
+
     def tile_splits(self, m: int, n: int, k: int) -> int:
         """Parts of k in which ``linear`` works a product in the framework's own tiles of 128 x 256 (0: not at all, the library's).  The
         library gives a product with few tiles and a long sum (a feed-forward's second product) too few workgroups; here
@@ -1127,9 +1132,9 @@ class HipOps:
     @staticmethod
     def _library_has_timed(m: int, n: int, k: int) -> bool:
         """Whether TunableOp holds a choice of its own for this product, or is about to make one: timed by this process
-        (``tune_library_products``) or read from a file, by whom ever.  Such a product stays with the library (3,584 x 18,944 at 2,048 rows,
-        with the norm behind it: the library's default 381 us, the own tiles 287; its timed kernel takes 239 alone).  What TunableOp holds can change at any time and is
-        asked for each time, 6 us for 50 results and only while it is switched on."""
+        (``tune_library_products``) or read from a file, by whom ever.  Such a product stays with the library.  ``Engine.tune_matrix_products`` has
+        only timed what ``library_serves``: for a product that the own tiles take, a choice comes from another caller or from a file.  What TunableOp holds can change
+        at any time and is asked for each time, 6 us for 50 results and only while it is switched on."""
         tunable = torch.cuda.tunable
         if not tunable.is_enabled():
             return False

@@ -112,6 +112,7 @@ class AttentionMixer(Mixer):
         partial_out, partial_lse = sizes(self.num_heads, self.num_kv_heads, self.head_dim, limits.max_num_tokens, limits.max_num_seqs, limits.max_model_len)
         return {"attention_partial_out": partial_out, "attention_partial_lse": partial_lse}
 
+    products_in_parts = ("o_weight",)
     accepts_sink = True  # its last product may add itself to the residual (ResidualSink)
     accepts_deferred = True  # its first product can read a DeferredNorm
 

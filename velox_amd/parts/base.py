@@ -80,6 +80,10 @@ class Part:
     # on the same addresses every time.  One part that says False keeps the whole model's decode steps uncaptured.
     graph_safe = True
 
+    # The matrices (attribute names) whose products ``forward`` asks for without a bias and takes in parts
+    # (``ops.linear(..., partials_ok=True)``).
+    products_in_parts: Tuple[str, ...] = ()
+
     def __init__(self, prefix: str = "") -> None:
         self.prefix = prefix
         self._prepared: Dict[str, object] = {}

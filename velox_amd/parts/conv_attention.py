@@ -77,6 +77,7 @@ class ConvAttentionMixer(Mixer):
         self.conv_taps = int(conv_taps)
         self.qkv_bias = bool(qkv_bias)
         self.out_bias = bool(out_bias)
+        self.products_in_parts = ("o_weight",) if gate is not None and not out_bias else ()
         self.position = position
         if position is not None and getattr(position, "rotary_dim", 0) > self.dim:
             raise ValueError(f"the rotation spans {position.rotary_dim} channels but a query head has {self.dim}")

@@ -51,6 +51,7 @@ class GatedMLP(FeedForward):
         self.prepare_weight(ops, "gate_up_weight", stacked=2)
         self.prepare_weight(ops, "down_weight")
 
+    products_in_parts = ("down_weight",)
     accepts_sink = True  # its last product may add itself to the residual (ResidualSink)
     accepts_deferred = True  # its first product can read a DeferredNorm
 
@@ -103,6 +104,8 @@ class PlainMLP(FeedForward):
     def prepare_kernels(self, ops) -> None:
         self.prepare_weight(ops, "up_weight")
         self.prepare_weight(ops, "down_weight")
+
+    products_in_parts = ("down_weight",)
 
     def forward(self, x, ctx, sink=None):
         ops = ctx.ops
@@ -192,6 +195,7 @@ class RoutedExperts(FeedForward):
         self.shared = None
         if shared_intermediate_size:
             self.shared = GatedMLP(prefix + shared_prefix, hidden_size, int(shared_intermediate_size), names=shared_names)
+            self.shared.products_in_parts = ()  # (the experts' results are added to its whole output)
         self.router_weight: Optional[torch.Tensor] = None
         self.gate_up_weight: Optional[torch.Tensor] = None
         self.down_weight: Optional[torch.Tensor] = None

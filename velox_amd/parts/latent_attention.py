@@ -42,6 +42,8 @@ _NAMES = {"q": "q.weight", "down": "down.weight", "down_norm": "down_norm.weight
 
 
 class LatentAttentionMixer(Mixer):
+    products_in_parts = ("out_weight",)
+
     def __init__(self, prefix: str, hidden_size: int, num_heads: int, dim: int, rot_dim: int, vdim: int, kv_rank: int, scale: float,
                  norm_eps: float, position: Optional[PositionEncoding] = None, gate=True, own_latent: bool = True,
                  names: Tuple[Tuple[str, str], ...] = (), q_rank: Optional[int] = None, sink: bool = False) -> None:

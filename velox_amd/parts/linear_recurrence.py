@@ -230,6 +230,8 @@ register_part("mixer", "linear_recurrence", LinearRecurrenceMixer)
 
 
 class GeneralDeltaMixer(Mixer):
+    products_in_parts = ("o_weight",)
+
     def __init__(self, prefix: str, hidden_size: int, num_heads: int, dim: int, vdim: int, norm_eps: float, decay_rank: int, decay_scale: float = math.exp(-0.5),
                  names: Tuple[Tuple[str, str], ...] = ()) -> None:
         """``decay_rank``: the inner size of the decay's low-rank map (rows of ``w1``); ``decay_scale``: the constant ``c``;

@@ -128,6 +128,7 @@ class NormedAttentionMixer(Mixer):
         self.window = int(window) if window is not None else None
         self.keep_first = int(keep_first) if window is not None else 0
         self.gate = gate
+        self.products_in_parts = ("o_weight",) if gate is not None and not out_bias else ()
         self.names = {"gate": "gate_proj.weight", "q": "q_proj.weight", "k": "k_proj.weight", "v": "v_proj.weight", "o": "o_proj.weight", "q_norm": "q_norm.weight",
                       "k_norm": "k_norm.weight", "rel": "distance_bias", "mix": "value_mix"}
         self.names.update(dict(names))

@@ -26,6 +26,8 @@ from .base import Mixer, Param, StateNeed, register_part, single
 
 
 class StateSpaceMixer(Mixer):
+    products_in_parts = ("o_weight",)
+
     def __init__(self, prefix: str, hidden_size: int, num_heads: int, groups: int, state: int, vdim: int, conv_taps: int, norm_groups: int,
                  norm_eps: float, names: Tuple[Tuple[str, str], ...] = ()) -> None:
         """``names``: pairs (tensor, name below the prefix) that replace the default names ``in``, ``conv``, ``conv.b``,
