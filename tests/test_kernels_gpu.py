@@ -1663,3 +1663,18 @@ def test_float32_products_of_tiny_and_huge_numbers(ops, tile, exponent):
     for a, w in ((tiny, huge), (huge, tiny)):
         want = a.double() @ w.double().T
         assert float((ops.split_f32(a, w, tile=tile).double() - want).norm() / want.norm()) <= 3e-7
+
+
+@pytest.mark.parametrize("m, n, k, splits, tile", [(150, 324, 288, 1, 128256), (150, 324, 288, 1, 96192), (97, 132, 4192, 1, 64064), (97, 132, 2080, 3, 0)])
+def test_rows_beside_numbers_that_do_not_split_keep_their_bits(ops, m, n, k, splits, tile):
+    """A row with an infinity, NaN, a number near float32's end or tiny ones changes no other row."""
+    a, w = rand((m, k), torch.float32, m), rand((n, k), torch.float32, n)
+    strange = a.clone()
+    strange[3, 7], strange[20, k - 1], strange[37, 30], strange[m - 1] = float("inf"), float("nan"), 3e38, a[m - 1] * 1e-37
+    plain, got = ops.split_f32(a, w, None, splits, tile), ops.split_f32(strange, w, None, splits, tile)
+    same = [r for r in range(m) if r not in (3, 20, 37, m - 1)]
+    assert torch.equal(got[..., same, :], plain[..., same, :])
+    last = a[m - 1:].double() * 1e-37 @ w.double().T
+    whole = got.double().sum(0) if splits > 1 else got.double()
+    assert float((whole[m - 1] - last[0]).norm() / last.norm()) <= 1e-6  # (the row itself, its numbers rounded once more)
+    assert whole[3].isinf().any() and whole[20].isnan().all() and not whole[37].isnan().any()

@@ -44,15 +44,18 @@ struct SplitArgs {
   int splits, split_steps;  // parts of k and steps of 32 of each (a multiple of SPLIT_FOLD)
 };
 
-// The same outputs with the float32 matrix instruction, from memory, for the rows and columns of one wave.  It is taken where a sum is no
-// finite number: an operand is an infinity, NaN or beyond 2^104, or the sum is beyond 2^80, where the factors leave float32's range.  Slow
-// and seldom.
+// Outputs of one wave with the float32 matrix instruction, from memory: those four of a lane's row in tile t that bit t of its `wanted` asks for, so
+// that no row's bits depend on another's numbers.  It is taken where a sum is no finite number: an operand is an infinity, NaN or
+// beyond 2^104, or the sum is beyond 2^80, where the factors leave float32's range.  Slow and
+// seldom: a row of NaN among 616 takes 17,920 x 1,536 from 213 to 510 us, 8,960 -> 1,536 in eight parts from 95 to 331.
 template <int RT, int CT>
-__device__ __forceinline__ void split_outputs_in_float32(const SplitArgs& args, int row0, int col0, int part) {
+__device__ __forceinline__ void split_outputs_in_float32(const SplitArgs& args, int row0, int col0, int part, uint32_t wanted) {
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int begin = part * args.split_steps * 32, end = min(args.k, begin + args.split_steps * 32);
   float* out = args.out + (size_t)part * args.m * args.n;
   for (int t = 0; t < RT * CT; ++t) {
+    const bool mine = (wanted >> t & 1) != 0;
+    if (!__any(mine)) continue;  // (the whole wave)
     const int row = row0 + t / CT * 16 + i, col = col0 + t % CT * 16;
     const float* a_row = args.a + (size_t)min(row, args.m - 1) * args.k + g;
     const float* w_row = args.w + (size_t)min(col + i, args.n - 1) * args.k + g;
@@ -66,7 +69,7 @@ __device__ __forceinline__ void split_outputs_in_float32(const SplitArgs& args, 
       }
       total += acc;
     }
-    if (row >= args.m || col + 4 * g >= args.n) continue;
+    if (!mine) continue;
     if (args.bias != nullptr) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) total[u] += args.bias[col + 4 * g + u];
@@ -209,7 +212,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     begun = true;
   }
 
-  bool beyond = false;
+  uint32_t beyond = 0;  // bit r CT + c
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -220,13 +223,13 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       if (begun) v += *p;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        beyond |= !(fabsf(v[u]) < INFINITY);
+        if (!(fabsf(v[u]) < INFINITY)) beyond |= 1u << (r * CT + c);
         v[u] *= 1.f / (SPLIT_SCALE * SPLIT_SCALE);
         if (args.bias != nullptr) v[u] += args.bias[col0 + 16 * c + 4 * h + u];
       }
       *p = v;
     }
-  if (__any(beyond)) split_outputs_in_float32<RT, CT>(args, row0, col0, part);
+  if (__any(beyond != 0)) split_outputs_in_float32<RT, CT>(args, row0, col0, part, beyond);
 }
 
 // The tile of a product as rows * 1,000 + columns, by what it costs, fitted to 129 products of 512 to 37,888 columns, 1,024 to 8,960 terms and 17 to
