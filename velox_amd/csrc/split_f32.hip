@@ -5,9 +5,12 @@
 // of parts six count, hi hi + hi mid + mid hi + hi lo + mid mid + lo hi (the other three are 2^-26 of a term; the method is that of
 // Henry, Tang, Heinecke: Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations, 2019).
 //
-// Precision: the instruction truncates where it adds 32 products to the sum so far, which one long chain would show (1,536 terms: 6e-7
+// Precision: the instruction rounds down where it adds 32 products to the sum so far, which one long chain would show (1,536 terms: 6e-7
 // of the result's norm; 8,960: 1.5e-6).  So an output is built from sums of 128 terms (24 instructions from zero), added in float32
-// with rounding to sums of up to 2,048, which are added up in the result's place.  Error against float64, float32 matrix
+// with rounding to sums of up to 2,048, which are added up in the result's place.  Every other one of them is of the negative terms (the rows
+// times -2^24) and subtracted: rounded down throughout, all of a layer's outputs were too small by the same 3e-8 (1,536 terms) or 8e-8 (8,960) of
+// their norm, which added up from layer to layer, and a model's logits were 3% further from 64 bits than with the float32 instructions,
+// although each product was closer (eight layers of width 1,536, six seeds: 1.64 to 1.94e-06, 1.68 to 2.00e-06; so 1.59 to 1.90e-06).  Error against float64, float32 matrix
 // instructions / this: 512 terms 2.1e-07 / 1.6e-07, 1,536 2.1e-07 / 1.7e-07, 8,960 2.3e-07 / 1.9e-07, 18,944 2.6e-07 / 2.1e-07; of terms of one
 // sign 9.5e-08 / 7.4e-08, 6.2e-08 / 6.2e-08, 7.5e-08 / 5.3e-08, 9.8e-08 / 5.8e-08.  (Inner sums of 64 terms: 1.3e-07 at 1,536 terms, 2% slower;
 // sums of 1,024 in the result's place: 190 instead of 180 us where 1,536 terms are added, for the passes over the result.)
@@ -83,7 +86,7 @@ template <int RT, int CT>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) split_f32_kernel(const SplitArgs args) {
   constexpr int TM = 32 * RT, TN = 64 * CT, BLOCKS = (TM + TN) / 16, PLANE = BLOCKS * 1024, STAGE = 3 * PLANE;
   constexpr int PIECES = (TM + TN) * 4, J = (PIECES + 511) / 512;
-  static_assert(2 * STAGE <= 160 * 1024 && PIECES % 64 == 0, "LDS of a compute unit; whole waves of pieces");
+  static_assert(2 * STAGE <= 160 * 1024 && PIECES % 64 == 0 && TM * 4 % 64 == 0, "LDS of a compute unit; whole waves of pieces, of rows or columns");
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
   const int m = args.m, n = args.n, k = args.k;
   const int row_tiles = (m + TM - 1) / TM, tiles = row_tiles * ((n + TN - 1) / TN), total_tiles = tiles * args.splits;
@@ -113,11 +116,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         raw[j][1] = *reinterpret_cast<const float4_t*>(from[j] + 32 * s + 4);
       }
   };
-  auto put = [&](char* stage) {
+  auto put = [&](char* stage, int s) {
+    const float row_scale = s / SPLIT_FOLD % 2 != 0 ? -SPLIT_SCALE : SPLIT_SCALE;
 #pragma unroll
     for (int j = 0; j < J; ++j)
       if ((j + 1) * 512 <= PIECES || wave * 64 + 512 * j < PIECES) {
-        sp_float8_t x = __builtin_shufflevector(raw[j][0], raw[j][1], 0, 1, 2, 3, 4, 5, 6, 7) * SPLIT_SCALE;
+        sp_float8_t x = __builtin_shufflevector(raw[j][0], raw[j][1], 0, 1, 2, 3, 4, 5, 6, 7) * (wave * 64 + 512 * j < 4 * TM ? row_scale : SPLIT_SCALE);
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
           sp_uint4_t bits;
@@ -140,12 +144,14 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   for (int c = 0; c < CT; ++c)
 #pragma unroll
     for (int r = 0; r < RT; ++r) acc[c][r] = total[c][r] = float4_t{0.f, 0.f, 0.f, 0.f};
-  auto fold = [&] {
+  auto fold = [&](int s) {  // the inner sum that step s belongs to
+    const float sign = s / SPLIT_FOLD % 2 != 0 ? -1.f : 1.f;
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
       for (int r = 0; r < RT; ++r) {
-        total[c][r] += acc[c][r];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) total[c][r][u] = fmaf(acc[c][r][u], sign, total[c][r][u]);
         acc[c][r] = float4_t{0.f, 0.f, 0.f, 0.f};
       }
   };
@@ -171,7 +177,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   };
 
   ask(0);
-  put(smem);
+  put(smem, 0);
   if (steps > 1) ask(1);
   // lane (h, i) holds outputs 4 h .. + 3 of row i of every tile
   float* out = args.out + (size_t)part * m * n;
@@ -191,16 +197,16 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       __builtin_amdgcn_s_barrier();
       asm volatile("" : : : "memory");
       auto next = [&] {
-        if (s + 1 < steps) put(then);
+        if (s + 1 < steps) put(then, s + 1);
         if (s + 2 < steps) ask(s + 2);
         __builtin_amdgcn_sched_barrier(0);
       };
       if (splits_first) next();
       multiply(now);
       if (!splits_first) next();
-      if (s % SPLIT_FOLD == SPLIT_FOLD - 1) fold();
+      if (s % SPLIT_FOLD == SPLIT_FOLD - 1) fold(s);
     }
-    fold();  // (a last inner sum of fewer terms, or zeros)
+    fold(s);  // (a last inner sum of fewer terms, or zeros)
     if (s >= steps) break;
 #pragma unroll
     for (int r = 0; r < RT; ++r)
