@@ -1689,3 +1689,39 @@ def test_float32_products_of_split_operands_are_off_to_either_side(ops, m, n, k,
     error = (got.double().sum(0) if splits > 1 else got.double()) - want
     assert abs(float(error.mean())) * error.numel() ** 0.5 <= 5e-9 * float(want.norm())
     assert float(error.norm()) <= 2.1e-7 * float(want.norm())
+
+
+@pytest.mark.parametrize("up", [1.0, -3.0, 1e30])
+def test_gated_products_of_every_gate_have_the_bits_of_the_kernel_behind_a_product(ops, up):
+    """All finite bfloat16 gates, down to those whose result only a large factor shows: the activation where the sums end, and the kernel with the
+    library's exponential and division."""
+    bits = torch.arange(65536, dtype=torch.int32, device="cuda")
+    gates = torch.where(bits >= 32768, bits - 65536, bits).to(torch.int16).view(torch.bfloat16)
+    gates = gates[gates.isfinite()]
+    a, w = torch.zeros((gates.numel(), 64), dtype=torch.bfloat16, device="cuda"), torch.zeros((16, 64), dtype=torch.bfloat16, device="cuda")
+    a[:, 0], a[:, 1], w[:8, 0], w[8:, 1] = gates, up, 1.0, 1.0
+    product = ops.gemm_tiles(a, w)
+    assert torch.equal(product[:, :8], gates[:, None].expand(-1, 8))
+    want = ops.silu_mul(product)
+    for tile in (128128, 256256):
+        got = torch.empty_like(want)
+        assert ops._core.velox_tiles_glu_bf16(a.data_ptr(), w.data_ptr(), got.data_ptr(), gates.numel(), 8, 64, 0, tile, ops._stream()) == 0
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_an_experts_silu_does_not_depend_on_the_number_of_pairs(ops):
+    """Sums of one term, so that the kernels for few pairs and for many differ in nothing but the unit's middle: the same bits, for gates
+    down to the last one with a result."""
+    gates = torch.cat([torch.linspace(-89, -86, 60), torch.linspace(-30, 30, 200)]).cuda()
+    x = torch.zeros((gates.numel(), 64), dtype=torch.bfloat16, device="cuda")
+    x[:, 0], x[:, 1] = gates.bfloat16(), 1e30
+    first, down = torch.zeros((2, 128, 64), dtype=torch.bfloat16, device="cuda"), torch.eye(64, dtype=torch.bfloat16, device="cuda").repeat(2, 1)
+    first[:, :64, 0], first[:, 64:, 1] = 1.0, 1.0
+    choice, weight = (torch.arange(gates.numel(), device="cuda") % 2).int()[:, None], torch.ones((gates.numel(), 1), device="cuda")
+
+    def run(lo, hi):
+        return ops.routed_experts(x[lo:hi], choice[lo:hi].contiguous(), weight[lo:hi], first.view(256, 64), down, 2, False, None, torch.bfloat16)
+
+    whole = run(0, gates.numel())
+    assert torch.equal(whole, torch.cat([run(at, min(at + 40, gates.numel())) for at in range(0, gates.numel(), 40)]))
+    assert int((whole[:60] != 0).all(1).sum()) >= 50  # (all but those below -88.72)

@@ -88,8 +88,26 @@ __device__ __forceinline__ uint32_t tl_pack(float x, float y) {
   return (uint32_t)(uint16_t)bf16_bits(x) | ((uint32_t)(uint16_t)bf16_bits(y) << 16);
 }
 
-// A gated unit's middle.  SiLU with the exponential and the reciprocal of the instruction set (1 ulp each in float32): with the
-// library's, whose some forty instructions per output nothing hides, 2,048 x 37,888 x 3,584 took 479 us, a product and a kernel behind it 446.
+// g / (1 + e^-g), as close to it as the library's exponential and division come, in half of their some forty instructions per output, which nothing
+// hides here.  e^-g is 2^whole 2^rest; the rest has what the product with log2 e is rounded by, or, of a bfloat16 g (SHORT), that product with 16
+// bits of log2 e is exact.  The quotient by the instruction set's reciprocal is corrected once.  Below -64, where the denominator nears float32's
+// end and its reciprocal the end of what that instruction returns, both sides are 2^-8 of themselves; beyond +-88.7 the correction would
+// multiply an infinity.  Every bfloat16 g has the library's bits; of 2e8 float32 ones from 0.01 to 20 and from -20 to -0.01 five have not, and either is
+// 3.6e-08 and 4.4e-08 off 64 bits (the exponential and the reciprocal of the instruction set alone 4.6e-08 and 2.4e-07, and 0 below -87.3).  2,048 x 37,888 x
+// 3,584: 428 us, with those two 417, with the library's 479, a product and a kernel behind it 446.
+template <bool SHORT>
+__device__ __forceinline__ float tl_silu(float g) {
+#pragma clang fp contract(off)  // (what `power` is rounded by is added back)
+  const float z = __builtin_amdgcn_fmed3f(g, -104.f, 104.f);
+  const float power = z * (SHORT ? -1.44268799f : -1.44269502f), whole = rintf(power);
+  const float rest = SHORT ? fmaf(z, -7.05260771e-06f, power - whole) : power - whole + fmaf(z, -1.92596303e-08f, fmaf(z, -1.44269502f, -power));
+  const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(rest), (int)whole);
+  const float part = g < -64.f ? 0x1p-8f : 1.f;
+  const float below = fmaf(e, part, part), above = g * part, inverse = __builtin_amdgcn_rcpf(below), near = above * inverse;
+  return fabsf(g) <= 88.7f ? fmaf(-fmaf(near, below, -above), inverse, near) : near;
+}
+
+// A gated unit's middle.
 template <int EPI>
 __device__ __forceinline__ float tl_middle(float gate, float up, const TileArgs& args) {
   if (EPI == TL_UNIT) return glu_middle(gate, up, args.unit);
@@ -98,7 +116,7 @@ __device__ __forceinline__ float tl_middle(float gate, float up, const TileArgs&
     up = to_f32(from_f32<bf16_t>(up));
   }
   if (EPI == TL_RELU) return fmaxf(gate, 0.f) * up;
-  return gate * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gate * -1.44269504f)) * up;
+  return tl_silu<EPI == TL_SILU>(gate) * up;
 }
 
 // RT, CT: tiles of 32 rows and 32 columns per wave; S: buffers.  GATHER: rows through the plan's order.  TAIL: k % 64 != 0.
