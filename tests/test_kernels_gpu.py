@@ -1725,3 +1725,35 @@ def test_an_experts_silu_does_not_depend_on_the_number_of_pairs(ops):
     whole = run(0, gates.numel())
     assert torch.equal(whole, torch.cat([run(at, min(at + 40, gates.numel())) for at in range(0, gates.numel(), 40)]))
     assert int((whole[:60] != 0).all(1).sum()) >= 50  # (all but those below -88.72)
+
+
+@pytest.mark.parametrize("scale_input", [False, True])
+def test_experts_of_rows_further_apart_than_the_tiles_loads_reach(ops, monkeypatch, scale_input):
+    """131,080 rows of 8,192 channels, more than 2 GiB: on the matrix cores, with the bits that the same rows have in a small step (each output is one
+    chain of sums whatever else is in its tile)."""
+    monkeypatch.setattr(ops._core, "velox_grouped_glu", None)  # (the multiply-adds)
+    tokens, hidden, inter, experts = 131080, 8192, 64, 2
+    x = torch.empty((tokens, hidden), dtype=torch.bfloat16, device="cuda").normal_(generator=torch.Generator(device="cuda").manual_seed(1))
+    first, down = rand((experts * 2 * inter, hidden), torch.bfloat16, 2, hidden ** -0.5), rand((experts * hidden, inter), torch.bfloat16, 3, inter ** -0.5)
+    choice, weight = (torch.arange(tokens, device="cuda") // 3 % experts).int()[:, None].contiguous(), torch.rand((tokens, 1), device="cuda")
+
+    def run(rows):
+        return ops.routed_experts(x[rows], choice[rows], weight[rows], first, down, experts, scale_input, None, torch.bfloat16)
+
+    whole = run(slice(0, tokens))
+    for rows in (slice(0, 150), slice(65500, 65640), slice(tokens - 300, tokens)):
+        assert torch.equal(whole[rows], run(rows))
+
+
+def test_experts_whose_gate_and_up_rows_are_further_apart_than_the_tiles_loads_reach(ops, monkeypatch):
+    """One expert of 65,536 x 16,384, 2 GiB a branch: on the matrix cores, in tiles of 64 rows and so with the bits of steps of at most 64 pairs."""
+    monkeypatch.setattr(ops._core, "velox_grouped_glu", None)
+    tokens, hidden, inter = 150, 16384, 65536
+    generator = torch.Generator(device="cuda").manual_seed(1)
+    first, down = (torch.empty(shape, dtype=torch.bfloat16, device="cuda").normal_(std=0.01, generator=generator) for shape in ((2 * inter, hidden), (hidden, inter)))
+    x, choice, weight = rand((tokens, hidden), torch.bfloat16, 4), torch.zeros((tokens, 1), dtype=torch.int32, device="cuda"), torch.rand((tokens, 1), device="cuda")
+    for scale_input in (False, True):
+        whole = ops.routed_experts(x, choice, weight, first, down, 1, scale_input, None, torch.bfloat16)
+        for at in (0, 64, 86):
+            rows = slice(at, at + 64)
+            assert torch.equal(whole[rows], ops.routed_experts(x[rows], choice[rows], weight[rows], first, down, 1, scale_input, None, torch.bfloat16))

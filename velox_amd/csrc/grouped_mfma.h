@@ -310,10 +310,10 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
 // The rows of a tile of the plan's products: 64 up to 64 pairs, above 128 or 192 (tiles_mfma.h's kernel, 256 rows of W), whichever is likely to
 // cost less: an expert's last tile is half empty on average, none has less than one (1,340 pairs over 32 experts of 4,096 -> 1,408 read W, us of
 // the two products in tiles of 192 rows 177 + 76, of 128, whose loads are further ahead, 169 + 72), and all tiles take whole rounds over the compute units.  k % 64 != 0 is
-// built for 128.  (Tiles of 64 rows were no quicker at any number of pairs above 64: 12 rows per expert 66 us either way, 56: 80 /
+// built for 128.  Experts with 2 GiB or more from a gate row to its up row, which the large tiles' loads do not reach, stay with 64 rows at any number of pairs.  (Tiles of 64 rows were no quicker at any number of pairs above 64: 12 rows per expert 66 us either way, 56: 80 /
 // 81, 75: 100 / 83, 130: 127 / 125, 256: 187 / 155, 16 experts of 2,048 -> 1,408 -> 2,048.)
 static inline int grouped_tile_rows(int pairs, int experts, int inter, int hidden, int branches) {
-  if (pairs <= 64) return 64;
+  if (pairs <= 64 || !tiles_fit(256, hidden, branches == 2 ? inter + 256LL : 256, hidden) || !tiles_fit(256, inter, 256, inter)) return 64;
   if (inter % 64 != 0 || hidden % 64 != 0) return 128;
   float cost[2];
   for (int rt = 2; rt <= 3; ++rt) {

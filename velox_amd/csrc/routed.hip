@@ -467,7 +467,7 @@ __global__ void __launch_bounds__(256) routed_scale_kernel(const bf16_t* __restr
   const int row = blockIdx.x;
   if (row >= *placed) return;  // (pairs whose expert the plan leaves out have no row: `order` ends at the placed ones)
   const int pair = order[row];
-  const float w = pair_weight[pair];
+  const float w = pair_weight != nullptr ? pair_weight[pair] : 1.f;
   typedef bf16_t Pieces __attribute__((ext_vector_type(8)));
   const Pieces* src = reinterpret_cast<const Pieces*>(x + (size_t)(pair / top) * hidden);
   Pieces* dst = reinterpret_cast<Pieces*>(sorted + (size_t)row * hidden);
@@ -496,9 +496,15 @@ static GroupedArgs routed_args(const void* a, const void* w, void* out, const in
   return args;
 }
 
-// x [T, hidden] -> (`sorted` [pairs, hidden], with scale_input and more than 64 pairs) -> act [pairs, inter] -> y [pairs, hidden]
+// x [T, hidden] -> (`sorted` [pairs, hidden], where velox_routed_copies_rows says so) -> act [pairs, inter] -> y [pairs, hidden]
 // float32.  Needs hidden % 8 == 0, inter % 8 == 0 and x and `sorted` on 16-byte boundaries (the caller checks).  The plan's tiles hold velox_routed_tile_rows rows.
 extern "C" int velox_routed_tile_rows(int pairs, int experts, int inter, int hidden, int branches) { return grouped_tile_rows(pairs, experts, inter, hidden, branches); }
+
+// Whether the products read sorted copies of the rows: rows that their pair's weight scales (tiles of 64 rows do that themselves), and rows further
+// apart than the large tiles' loads reach through the plan (2 GiB: from 131,072 tokens of 8,192 channels on).
+extern "C" int velox_routed_copies_rows(int pairs, int top, int hidden, int tile_rows, int scale_input) {
+  return tile_rows != RT_BM && (scale_input || !tiles_fit(pairs / top, hidden, 256, hidden));
+}
 
 extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, const void* down, void* sorted, void* act, float* y, const int* plan,
                                           const float* pair_weight, int pairs, int experts, int top, int inter, int hidden, int scale_input,
@@ -506,15 +512,15 @@ extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, co
   // `ungated` > 0: `gate_up` holds [experts * inter, hidden] (up rows only) and the unit is ungated_act(up, ungated)
   if (pairs <= 0) return 0;
   if (hidden % 8 != 0 || inter % 8 != 0 || top < 1 || ((uintptr_t)x | (uintptr_t)sorted) % 16 != 0) return -1;
-  const bool copied = scale_input && pairs > RT_BM;
-  if (copied && sorted == nullptr) return -1;
   const int max_tiles = velox_routed_max_tiles(pairs, experts), tile_rows = grouped_tile_rows(pairs, experts, inter, hidden, ungated > 0 ? 1 : 2);
+  const bool copied = velox_routed_copies_rows(pairs, top, hidden, tile_rows, scale_input);
+  if (copied && sorted == nullptr) return -1;
   if (max_tiles > 65535) return -1;
   if (copied)
-    routed_scale_kernel<<<pairs, 256, 0, stream>>>((const bf16_t*)x, plan + 1 + (experts + 1), pair_weight, (bf16_t*)sorted, top, hidden, plan + 1 + experts);
+    routed_scale_kernel<<<pairs, 256, 0, stream>>>((const bf16_t*)x, plan + 1 + (experts + 1), scale_input ? pair_weight : nullptr, (bf16_t*)sorted, top, hidden, plan + 1 + experts);
   GroupedArgs first = routed_args(copied ? sorted : x, gate_up, act, plan, pairs, experts, inter, hidden, ungated > 0 ? inter : 2 * inter);
   first.gather_top = copied ? 0 : top;
-  first.row_scale = scale_input ? pair_weight : nullptr;  // (read by the kernel for few rows alone)
+  first.row_scale = scale_input && !copied ? pair_weight : nullptr;  // (read by the kernel for tiles of 64 rows alone)
   first.act = ungated;
   first.unit = GluUnit{alpha, limit, shift};
   const int status = ungated > 0 ? grouped_plan_launch<GM_ACT, bf16_t>(first, tile_rows, max_tiles, stream) : grouped_plan_launch<GM_GLU, bf16_t>(first, tile_rows, max_tiles, stream);

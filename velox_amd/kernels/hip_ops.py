@@ -223,7 +223,8 @@ class HipOps:
                    c.velox_linear_scan, c.velox_linear_scan_lanes, c.velox_gated_head_norm):
             fn.restype = _I
         c.velox_routed_products_bf16.restype = _I
-        c.velox_routed_tile_rows.argtypes, c.velox_routed_tile_rows.restype = [_I, _I, _I, _I, _I], _I
+        for fn in (c.velox_routed_tile_rows, c.velox_routed_copies_rows):
+            fn.argtypes, fn.restype = [_I, _I, _I, _I, _I], _I
         for fn in (c.velox_latent_rotate_write, c.velox_head_linear, c.velox_route_top, c.velox_routed_plan, c.velox_grouped_glu, c.velox_grouped_down,
                    c.velox_routed_combine, c.velox_add_sinusoid, c.velox_add_cast, c.velox_norm_add, c.velox_qk_norm_write):
             fn.restype = _I
@@ -1844,8 +1845,6 @@ class HipOps:
         on_matrix_cores = x.dtype == torch.bfloat16 and hidden % 8 == 0 and inter % 8 == 0 and self.use_grouped_mfma
         if pairs > self.FEW_PAIRS and (gate_up_weight.data_ptr() | down_weight.data_ptr()) % 16 != 0:
             on_matrix_cores = False  # (loads that write LDS directly need 16-byte boundaries; the multiply-add tiles take any)
-        if pairs > self.FEW_PAIRS and max(tokens, inter + 256) * hidden >= 1 << 30:
-            on_matrix_cores = False  # (nor do those loads reach further than 2 GiB)
         tile_rows = self._core.velox_routed_tile_rows(pairs, num_experts, inter, hidden, branches) if on_matrix_cores else 64
         if on_matrix_cores and x.data_ptr() % 16 != 0:
             x = x.clone()
@@ -1854,7 +1853,8 @@ class HipOps:
         y = torch.empty((pairs, hidden), dtype=torch.float32, device=self.device)
         if on_matrix_cores:
             # bfloat16 rows of whole 16-byte pieces: both products on the matrix cores
-            scaled = torch.empty((pairs, hidden), dtype=x.dtype, device=self.device) if scale_input and pairs > self.FEW_PAIRS else None
+            copied = self._core.velox_routed_copies_rows(pairs, top, hidden, tile_rows, int(bool(scale_input)))
+            scaled = torch.empty((pairs, hidden), dtype=x.dtype, device=self.device) if copied else None
             self._launched(self._core.velox_routed_products_bf16(_ptr(x), _ptr(gate_up_weight), _ptr(down_weight), _ptr(scaled), _ptr(act), _ptr(y), _ptr(plan),
                                                                  _ptr(weight), pairs, num_experts, top, inter, hidden, int(bool(scale_input)),
                                                                  alpha, limit, shift, act_code, self._stream()), "routed_products")
