@@ -1188,7 +1188,7 @@ def test_place_tokens_puts_sampled_ids_into_a_steps_rows(ops, ref):
         ops.place_tokens(got, dest, source, tokens, 7)
 
 
-# -- routed experts on the matrix cores: tiles of 128 rows x 256 rows of W, steps of 64 indices --------------------------------
+# -- routed experts on the matrix cores: tiles of 128 or 192 rows x 256 rows of W, steps of 64 indices -------------------------
 @pytest.mark.parametrize("rows, hidden, inter, top, scale_input, unit", [
     ((65,), 64, 64, 1, False, "glu"),  # one row beyond a half tile, one step
     ((64, 1, 0, 129, 127), 200, 136, 1, True, "glu"),  # a last step of fewer indices, columns beyond a tile, groups of every size
@@ -1197,6 +1197,22 @@ def test_place_tokens_puts_sampled_ids_into_a_steps_rows(ops, ref):
     ((40, 33, 20, 200, 90), 328, 520, 2, True, "glu"),
 ])
 def test_grouped_products_at_the_edges_of_their_tiles(ops, rows, hidden, inter, top, scale_input, unit):
+    experts_against_float64(ops, rows, hidden, inter, top, scale_input, unit)
+
+
+@pytest.mark.parametrize("rows, hidden, inter, top", [((700, 0, 1, 193, 192, 1153), 64, 128, 1), ((191, 2100, 385), 192, 320, 2), ((97,), 128, 64, 1)])
+@pytest.mark.parametrize("scale_input", [False, True])
+@pytest.mark.parametrize("unit", ["glu", "clamped", "relu2"])
+def test_grouped_products_in_tiles_of_128_and_192_rows(ops, monkeypatch, rows, hidden, inter, top, scale_input, unit):
+    """Empty experts, last tiles of one row and of all, more than the five tiles that are dealt out together; rows gathered through the plan and
+    copied.  Each output is one chain of sums: the same bits either way."""
+    monkeypatch.setattr(ops._core, "velox_routed_tile_rows", lambda *sizes: 128)
+    first = experts_against_float64(ops, rows, hidden, inter, top, scale_input, unit)
+    monkeypatch.setattr(ops._core, "velox_routed_tile_rows", lambda *sizes: 192)
+    assert torch.equal(experts_against_float64(ops, rows, hidden, inter, top, scale_input, unit), first)
+
+
+def experts_against_float64(ops, rows, hidden, inter, top, scale_input, unit):
     """Against float64.  Two roundings to bfloat16 (8 bits), each off by at most 2^-8 of its value: the units' middles, which the second
     product adds up (at most 2^-8 sum |W_down| |middle|), and the result.  Float32 sums of a few hundred terms add less than
     1e-5 of the same sums."""
@@ -1204,7 +1220,8 @@ def test_grouped_products_at_the_edges_of_their_tiles(ops, rows, hidden, inter, 
     experts, tokens = len(rows), max(sum(rows) // top, max(rows))
     drawn = lambda *shape: torch.randn(*shape, generator=generator, device="cuda")  # noqa: E731
     x = drawn(tokens, hidden).bfloat16()
-    branches = 2 if unit == "glu" else 1
+    branches = 1 if unit == "relu2" else 2
+    alpha, limit, shift = (1.702, 2.0, 1.0) if unit == "clamped" else (1.0, float("inf"), 0.0)
     first = (drawn(experts * branches * inter, hidden) * hidden ** -0.5).bfloat16()
     down = (drawn(experts * hidden, inter) * inter ** -0.5).bfloat16()
     weight = torch.rand(tokens, top, generator=generator, device="cuda") + 0.5
@@ -1214,7 +1231,7 @@ def test_grouped_products_at_the_edges_of_their_tiles(ops, rows, hidden, inter, 
         for t, k in at[:count]:
             choice[t, k] = e
         at = at[count:]
-    got = ops.routed_experts(x, choice, weight, first, down, experts, scale_input, None, torch.bfloat16, identity_experts=1, **({"ungated": unit} if unit != "glu" else {}))
+    got = ops.routed_experts(x, choice, weight, first, down, experts, scale_input, None, torch.bfloat16, identity_experts=1, **({"ungated": unit} if unit == "relu2" else {"unit": (alpha, limit, shift)}))
     want = torch.zeros(tokens, hidden, dtype=torch.float64, device="cuda")
     spread = torch.zeros_like(want)
     for e in range(experts):
@@ -1222,13 +1239,18 @@ def test_grouped_products_at_the_edges_of_their_tiles(ops, rows, hidden, inter, 
         t, k = (choice == e).nonzero(as_tuple=True)
         share = weight[t, k].double()[:, None]
         both = ((x[t].float() * share.float()).bfloat16() if scale_input else x[t]).double() @ w1.T  # (a scaled row is a bfloat16 row, as in the reference)
-        middle = both[:, :inter] * torch.sigmoid(both[:, :inter]) * both[:, inter:] if unit == "glu" else torch.relu(both).square()
+        if unit == "relu2":
+            middle = torch.relu(both).square()
+        else:
+            gate, up = both[:, :inter].clamp(max=limit), both[:, inter:].clamp(-limit, limit)
+            middle = gate * torch.sigmoid(alpha * gate) * (up + shift)
         want.index_add_(0, t, middle @ w2.T * (1.0 if scale_input else share))
         spread.index_add_(0, t, middle.abs() @ w2.abs().T * (1.0 if scale_input else share))
     none = choice == experts
     want += (x.double()[:, None, :] * (weight.double() * none)[:, :, None]).sum(1)
     bound = (2.0 ** -8 + 2e-5) * spread + 2.0 ** -8 * 1.01 * want.abs() + 1e-6
     assert torch.all((got.double() - want).abs() <= bound), float(((got.double() - want).abs() / bound).max())
+    return got
 
 
 @pytest.mark.parametrize("tokens, top, hidden, inter, unit", [(1, 2, 64, 72, "glu"), (7, 3, 328, 64, "glu"), (16, 4, 200, 136, "relu2"), (21, 3, 264, 40, "glu"), (22, 3, 264, 40, "glu"),

@@ -497,7 +497,8 @@ static GroupedArgs routed_args(const void* a, const void* w, void* out, const in
 }
 
 // x [T, hidden] -> (`sorted` [pairs, hidden], where velox_routed_copies_rows says so) -> act [pairs, inter] -> y [pairs, hidden]
-// float32.  Needs hidden % 8 == 0, inter % 8 == 0 and x and `sorted` on 16-byte boundaries (the caller checks).  The plan's tiles hold velox_routed_tile_rows rows.
+// float32.  Needs hidden % 8 == 0, inter % 8 == 0 and x and `sorted` on 16-byte boundaries (the caller checks).  The plan's tiles hold `tile_rows` rows: 64, 128 or, of
+// sizes that are multiples of 64, 192 (velox_routed_tile_rows says which is likely to be the quickest).
 extern "C" int velox_routed_tile_rows(int pairs, int experts, int inter, int hidden, int branches) { return grouped_tile_rows(pairs, experts, inter, hidden, branches); }
 
 // Whether the products read sorted copies of the rows: rows that their pair's weight scales (tiles of 64 rows do that themselves), and rows further
@@ -508,11 +509,12 @@ extern "C" int velox_routed_copies_rows(int pairs, int top, int hidden, int tile
 
 extern "C" int velox_routed_products_bf16(const void* x, const void* gate_up, const void* down, void* sorted, void* act, float* y, const int* plan,
                                           const float* pair_weight, int pairs, int experts, int top, int inter, int hidden, int scale_input,
-                                          float alpha, float limit, float shift, int ungated, hipStream_t stream) {
+                                          float alpha, float limit, float shift, int ungated, int tile_rows, hipStream_t stream) {
   // `ungated` > 0: `gate_up` holds [experts * inter, hidden] (up rows only) and the unit is ungated_act(up, ungated)
   if (pairs <= 0) return 0;
+  if (tile_rows != RT_BM && tile_rows != 2 * RT_BM && (tile_rows != 3 * RT_BM || hidden % 64 != 0 || inter % 64 != 0)) return -1;
   if (hidden % 8 != 0 || inter % 8 != 0 || top < 1 || ((uintptr_t)x | (uintptr_t)sorted) % 16 != 0) return -1;
-  const int max_tiles = velox_routed_max_tiles(pairs, experts), tile_rows = grouped_tile_rows(pairs, experts, inter, hidden, ungated > 0 ? 1 : 2);
+  const int max_tiles = velox_routed_max_tiles(pairs, experts);
   const bool copied = velox_routed_copies_rows(pairs, top, hidden, tile_rows, scale_input);
   if (copied && sorted == nullptr) return -1;
   if (max_tiles > 65535) return -1;

@@ -161,7 +161,7 @@ class HipOps:
         c.velox_grouped_glu.argtypes = [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _I, _P]
         c.velox_grouped_down.argtypes = [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]
         c.velox_routed_combine.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P]
-        c.velox_routed_products_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _F, _I, _P]
+        c.velox_routed_products_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _F, _I, _I, _P]
         c.velox_routed_combine_norm.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _F, _F, _P, _P, _F, _P]
         c.velox_routed_combine_norm.restype = _I
         c.velox_add_sinusoid.argtypes = [_P, _P, _P, _I, _I, _P]
@@ -1857,7 +1857,7 @@ class HipOps:
             scaled = torch.empty((pairs, hidden), dtype=x.dtype, device=self.device) if copied else None
             self._launched(self._core.velox_routed_products_bf16(_ptr(x), _ptr(gate_up_weight), _ptr(down_weight), _ptr(scaled), _ptr(act), _ptr(y), _ptr(plan),
                                                                  _ptr(weight), pairs, num_experts, top, inter, hidden, int(bool(scale_input)),
-                                                                 alpha, limit, shift, act_code, self._stream()), "routed_products")
+                                                                 alpha, limit, shift, act_code, tile_rows, self._stream()), "routed_products")
             # (a weight on the output is applied by the last kernel: the second product is the same kernel either way)
             return self._routed_combine(y, plan, shared, tokens, top, num_experts, hidden, out_dtype, x if identity_experts else None, weight,
                                         scale_rows=not scale_input, output_norm=output_norm)
