@@ -124,8 +124,6 @@ __device__ __forceinline__ float glu_middle(float gate, float up, const GluUnit&
   return g / (1.f + expf(-unit.alpha * g)) * (u + unit.shift);
 }
 
-__device__ __forceinline__ float gelu_tanh_f32(float z) { return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))); }
-
 // The middle of a unit without a gate branch, act(up): kind 1 is relu(up)^2 (any other kind passes the value).
 #define VELOX_ACT_RELU2 1
 __device__ __forceinline__ float ungated_act(float v, int kind) {

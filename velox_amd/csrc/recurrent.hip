@@ -277,6 +277,8 @@ extern "C" int velox_embed_copies(const int* ids, const void* table, int table_d
 // ---------------------------------------------------------------------------------------------
 // gated_act_mul: out[t, i] = act(gate_up[t, i]) * gate_up[t, I + i]; kind 0: SiLU, 1: the tanh form of GELU, 2: max(z, 0).
 // ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ float gelu_tanh_f32(float z) { return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))); }
+
 __device__ __forceinline__ float gate_act(float g, int kind) { return kind == 1 ? gelu_tanh_f32(g) : kind == 2 ? fmaxf(g, 0.f) : g * sigmoid_f32(g); }
 
 // 16-byte accesses; needs inter % (16 / sizeof(T)) == 0 and aligned rows

@@ -202,8 +202,8 @@ class HipOps:
             fn.restype = _I
         c.velox_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]
         c.velox_tiles_glu_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _P]
-        c.velox_tiles_pick.argtypes = c.velox_tiles_splits.argtypes = [_I, _I, _I, _I]
-        for fn in (c.velox_tiles_bf16, c.velox_tiles_glu_bf16, c.velox_tiles_pick, c.velox_tiles_splits):
+        c.velox_tiles_splits.argtypes = [_I, _I, _I, _I]
+        for fn in (c.velox_tiles_bf16, c.velox_tiles_glu_bf16, c.velox_tiles_splits):
             fn.restype = _I
         c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         c.velox_linear_chunk_scan.restype = _I
