@@ -47,6 +47,22 @@ def test_a_float32_model_whose_products_all_run_on_the_matrix_instructions(tmp_p
     torch.testing.assert_close(torch.cat(got), qwen2_logits(config, weights, tokens), **TOL[torch.float32])
 
 
+def test_a_float32_model_whose_products_are_worked_on_split_operands(tmp_path, ops, monkeypatch):
+    """Sums of 512 terms and more: portions of more than 16 tokens have all products but the head's worked as products of bfloat16 parts, whole and in
+    parts that the norms add."""
+    from velox_amd.weights import write_random_model
+
+    folder = write_random_model({**CONFIGS["B"], "hidden_size": 512, "num_attention_heads": 16, "intermediate_size": 2048}, str(tmp_path / "wide"), 4, dtype="float32")
+    config, weights = read_model_folder(folder)
+    tokens = random_tokens(config["vocab_size"], 420, seed=9)
+    calls = []
+    monkeypatch.setattr(ops, "split_f32", lambda x, w, bias=None, splits=1, tile=0: calls.append((x.shape[0], w.shape[0], splits)) or type(ops).split_f32(ops, x, w, bias, splits, tile))
+    h = Harness(folder, ops, torch.float32, "cuda", PAGE_SIZE["B"], num_pages=128)
+    got = [h.feed([("a", tokens[lo:hi], list(range(hi - lo)))]) for lo, hi in ((0, 17), (17, 398), (398, 399), (399, 420))]
+    assert {m for m, _n, _s in calls} == {17, 381, 21} and any(s > 1 for _m, _n, s in calls) and any(s == 1 for _m, _n, s in calls)
+    torch.testing.assert_close(torch.cat(got), qwen2_logits(config, weights, tokens), **TOL[torch.float32])
+
+
 @pytest.mark.parametrize("name", ["A", "B", "C"])
 def test_the_cache_holds_the_first_layers_rotated_keys_and_values(tmp_path, ops, name):
     """What the pages hold, read back in sequence order (``CacheManager.gather_sequence``): layer 0's keys with bias and

@@ -1511,14 +1511,42 @@ def test_the_library_is_said_to_serve_what_linear_hands_to_it(ops, monkeypatch, 
 def test_linear_with_parts_of_a_long_sum_into_every_consumer(ops, ref, m, n, k, parts):
     """More than 64 rows of a long product come back as partial sums.  Each kernel that takes them gives what it gives for their float32
     sum (a handful of float32 additions in another order), which is the product within its own float32 sums' rounding."""
+    assert ops.tile_splits(m, n, k) == parts
+    parts_into_every_consumer(ops, m, n, k, parts, torch.bfloat16)
+
+
+@pytest.mark.parametrize("m, n, k", [(17, 256, 512), (64, 1536, 1536), (65, 1536, 8960), (300, 2048, 1536), (616, 1536, 8960), (2400, 1024, 2048)])
+def test_float32_linear_with_parts_into_every_consumer(ops, m, n, k):
+    """The same in float32, where sums of 512 terms and more are cut."""
+    parts = ops.split_f32_parts(m, n, k, True)
+    assert parts > 1
+    parts_into_every_consumer(ops, m, n, k, parts, torch.float32)
+
+
+@pytest.mark.parametrize("m, n, k, whole, most", [(16, 2048, 2048, 0, 0), (17, 2048, 480, 0, 0), (17, 2048, 528, 0, 0), (17, 2046, 2048, 0, 0), (64, 17920, 1536, 0, 8), (100, 11264, 2048, 1, 8), (256, 2048, 1536, 0, 8),
+                                                  (330, 2048, 1536, 1, 8), (4000, 11264, 2048, 1, 8), (33, 512, 512, 0, 8), (5000, 4096, 512, 1, 8)])
+def test_float32_products_in_parts_and_whole(ops, m, n, k, whole, most):
+    """Which products are worked as products of bfloat16 parts, and that no part of a sum is empty: each has whole inner sums of 128 terms but the last."""
+    assert ops.split_f32_parts(m, n, k, False) == whole
+    parts = ops.split_f32_parts(m, n, k, True)
+    assert whole <= parts <= max(whole, most)
+    if parts > 1:
+        each = -(-(-(-k // 128)) // parts) * 128
+        assert (parts - 1) * each < k
+    x, w = rand((m, k), torch.float32, 1), rand((n, k), torch.float32, 2, k ** -0.5)
+    assert ops.linear(x, w, None, torch.float32, partials_ok=True).shape == ((parts, m, n) if parts > 1 else (m, n))
+    assert ops.linear(x, w, rand((n,), torch.float32, 3), torch.float32, partials_ok=True).shape == (m, n)  # (a bias belongs to a whole sum)
+
+
+def parts_into_every_consumer(ops, m, n, k, parts, dtype):
+    from velox_amd.parts.base import NormedSum, SumOf
     from velox_amd.parts.norms import StreamNorm
 
     generator = torch.Generator(device="cuda").manual_seed(m)
-    x, w = torch.randn(m, k, generator=generator, device="cuda").bfloat16(), (k ** -0.5 * torch.randn(n, k, generator=generator, device="cuda")).bfloat16()
-    assert ops.tile_splits(m, n, k) == parts
-    got = ops.linear(x, w, None, torch.bfloat16, partials_ok=True)
+    x, w = torch.randn(m, k, generator=generator, device="cuda").to(dtype), (k ** -0.5 * torch.randn(n, k, generator=generator, device="cuda")).to(dtype)
+    got = ops.linear(x, w, None, dtype, partials_ok=True)
     assert got.shape == (parts, m, n) and got.dtype == torch.float32
-    assert ops.linear(x, w, None, torch.bfloat16).shape == (m, n)  # (who cannot take parts gets none)
+    assert ops.linear(x, w, None, dtype).shape == (m, n)  # (who cannot take parts gets none)
     whole = got.double().sum(0).float()
     for rows in (slice(0, 17), slice(m - 17, m)):
         want = x[rows].double() @ w.double().T
@@ -1527,7 +1555,11 @@ def test_linear_with_parts_of_a_long_sum_into_every_consumer(ops, ref, m, n, k, 
     rows = torch.tensor([m - 1, 0, m // 2], dtype=torch.int32).cuda()
     close = dict(rtol=2e-5, atol=2e-5)
     calls = [lambda r, delta: ops.add_rmsnorm(r, delta, weight, 1e-5, torch.float32), lambda r, delta: ops.add_rmsnorm_rows(r, delta, rows, weight, 1e-5, torch.float32),
-             lambda r, delta: ops.norm_add(r, delta, weight, 1e-5, 0.7, torch.float32), lambda r, delta: ops.norm_add_norm(r, delta, weight, 1e-5, weight, 1e-6, torch.float32)]
+             lambda r, delta: ops.norm_add(r, delta, weight, 1e-5, 0.7, torch.float32), lambda r, delta: ops.norm_add_norm(r, delta, weight, 1e-5, weight, 1e-6, torch.float32),
+             lambda r, delta: ops.add_dynamic_tanh(r, delta, weight, weight, weight[:1], torch.float32), lambda r, delta: ops.join_rows(r, delta, residual, torch.float32),
+             lambda r, delta: ops.normed_sum_norm(r, NormedSum((delta, delta), (weight, weight), (0.5, 2.0), 1e-5), weight, 1e-5, torch.float32),
+             lambda r, delta: ops.normed_sum_norm(r, NormedSum((delta,), (weight,), (0.5,), 1e-5, delta), weight, 1e-5, torch.float32),
+             lambda r, delta: ops.add_rmsnorm(r, SumOf(delta, residual), weight, 1e-5, torch.float32)]
     for call in calls:
         a, b = residual.clone(), residual.clone()
         torch.testing.assert_close(call(a, got).float(), call(b, whole).float(), **close)
@@ -1545,10 +1577,12 @@ def test_linear_with_parts_of_a_long_sum_into_every_consumer(ops, ref, m, n, k, 
     torch.testing.assert_close(a, b, **close)
 
 
+# (what is cut into no parts; which of these the library gets and which the own tiles take whole is tiles_serve's to say)
 @pytest.mark.parametrize("m, n, k", [(128, 2048, 8448), (128, 2048, 5632), (512, 1024, 5632), (128, 1536, 8960), (128, 1024, 8192), (300, 2048, 5112), (256, 512, 16384), (400, 256, 12288), (700, 8192, 29568), (836, 8192, 29568),
                                      (400, 16384, 16384), (1280, 6144, 16384), (1536, 5120, 13824), (64, 3584, 18944), (4096, 3584, 18944)])
-def test_products_that_the_library_works_faster_stay_with_it(ops, m, n, k):
+def test_products_whose_sum_is_not_cut(ops, m, n, k):
     assert ops.tile_splits(m, n, k) == 0
+    assert ops.library_serves(m, n, k) == (m > 64 and not ops.tiles_serve(m, n, k)) and ops.tiles_serve(m, n, k) == (-(-m // 128) * -(-n // 128) >= 192 and k % 64 == 0)
 
 
 def test_products_whose_library_kernel_was_timed_elsewhere_stay_with_it(ops, tmp_path, monkeypatch):
@@ -1651,6 +1685,43 @@ def test_float32_products_of_split_operands(ops, tile, m, n, k, splits):
     else:
         want, sizes = want + bias.double(), sizes + bias.double().abs()
     assert torch.all((got.double() - want).abs() <= (24 + min(k / 128, 16) + k / 2048 + splits + 3) * 2.0 ** -23 * sizes)
+    # errors of random signs: 1.6e-7 to 1.9e-7 of a row's norm; without one of the three smallest products of parts it is 1.7e-6 at least, worked in
+    # float64
+    if splits > 1 or k >= 512:
+        assert torch.all((got.double() - want).norm(dim=1) <= 4e-7 * want.norm(dim=1))
+
+
+@pytest.mark.parametrize("tile", [128256, 128192, 96192, 64256, 64128, 64064, 32128])
+@pytest.mark.parametrize("k", [128, 480])
+def test_every_product_of_parts_is_there(ops, tile, k):
+    """Sums in which all products of parts but one cancel exactly.  1 + 2^-9 + 2^-20 has the parts 1, 2^-9 and 2^-20; the results are exact: the rest of
+    a sum is zeros."""
+    from velox_amd.kernels.hip_ops import KernelError
+
+    m, n, u, v, low = 130, 260, 2.0 ** -9, 2.0 ** -10, 2.0 ** -20
+    at = 4 * torch.randint(0, k // 4, (m,), generator=torch.Generator().manual_seed(k)).cuda()
+    rows = torch.arange(m, device="cuda")
+
+    def a_of(*values):
+        a = torch.zeros(m, k, device="cuda")
+        for i, value in enumerate(values):
+            a[rows, at + i] = value
+        return a
+
+    def w_of(*values):
+        return torch.tensor(values, dtype=torch.float32, device="cuda").repeat(n, k // 4)
+
+    with pytest.raises(KernelError):
+        ops.split_f32(a_of(1, 0, 0, 0), w_of(1, 0, 0, 0).double(), tile=tile)
+    cases = [(a_of(1, 0, 0, 0), w_of(1, 0, 0, 0), 1.0),  # hi hi
+             (a_of(1 + u, -1, 0, 0), w_of(1, 1, 0, 0), u),  # mid hi
+             (a_of(1, -1, 0, 0), w_of(1 + u, 1, 0, 0), u),  # hi mid
+             (a_of(1 + u + low, -(1 + u), 0, 0), w_of(1, 1, 0, 0), low),  # lo hi
+             (a_of(1, -1, 0, 0), w_of(1 + u + low, 1 + u, 0, 0), low),  # hi lo
+             (a_of(1 + u, -(1 + u), -1, 1), w_of(1 + v, 1, 1 + v, 1), u * v)]  # mid mid
+    for which, (a, w, want) in enumerate(cases):
+        got = ops.split_f32(a, w, tile=tile)
+        assert torch.all(got == want), (which, float(got.min()), float(got.max()), want)
 
 
 @pytest.mark.parametrize("tile", [128256, 128192, 64064])

@@ -1158,8 +1158,12 @@ class HipOps:
     def split_f32(self, x, weight, bias: Optional[torch.Tensor] = None, splits: int = 1, tile: int = 0):
         """``x @ weight^T (+ bias)`` of float32 operands: [M, N], or with ``splits`` > 1 partial sums [splits, M, N].  ``tile``: rows * 1,000 +
         columns (0: picked by the product's size)."""
+        self._check("x", x, torch.float32, align=16)
+        self._check("weight", weight, torch.float32, (weight.shape[0], x.shape[1]), align=16)
         m, k = x.shape
         n = weight.shape[0]
+        if bias is not None:
+            self._check("bias", bias, torch.float32, (n,))
         out = torch.empty((m, n) if splits == 1 else (splits, m, n), dtype=torch.float32, device=self.device)
         self._launched(self._core.velox_split_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(out), m, n, k, int(splits), int(tile), self._stream()), "split_f32")
         return out
