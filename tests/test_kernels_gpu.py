@@ -1449,7 +1449,7 @@ def test_gated_products_in_every_tile(ops, m, n, k, activation):
 
 
 @pytest.mark.parametrize("m, n, k, own", [(64, 4096, 2048, False), (65, 4096, 2048, True), (300, 4608, 3584, False), (836, 37888, 3584, True), (836, 4608, 3584, True), (1036, 64, 2048, False),
-                                          (768, 64, 2048, True), (769, 64, 2048, False), (2421, 128, 2048, False), (1408, 1536, 1024, False), (1409, 1536, 1024, True), (1036, 56, 2048, False), (1036, 4100, 2048, False), (1036, 4096, 2056, False), (1036, 4096, 192, False)])
+                                          (768, 64, 2048, True), (769, 64, 2048, False), (2421, 128, 2048, False), (1408, 1536, 1024, False), (1409, 1536, 1024, True), (1536, 2048, 8192, False), (1793, 2048, 8192, True), (1536, 2048, 8128, True), (1036, 56, 2048, False), (1036, 4100, 2048, False), (1036, 4096, 2056, False), (1036, 4096, 192, False)])
 def test_which_products_run_in_the_own_tiles(ops, monkeypatch, m, n, k, own):
     calls = []
     monkeypatch.setattr(ops, "gemm_tiles", lambda *a, **more: calls.append(a) or type(ops).gemm_tiles(ops, *a, **more))
@@ -1582,7 +1582,7 @@ def parts_into_every_consumer(ops, m, n, k, parts, dtype):
                                      (400, 16384, 16384), (1280, 6144, 16384), (1536, 5120, 13824), (64, 3584, 18944), (4096, 3584, 18944)])
 def test_products_whose_sum_is_not_cut(ops, m, n, k):
     assert ops.tile_splits(m, n, k) == 0
-    assert ops.library_serves(m, n, k) == (m > 64 and not ops.tiles_serve(m, n, k)) and ops.tiles_serve(m, n, k) == (-(-m // 128) * -(-n // 128) >= 192 and k % 64 == 0)
+    assert ops.library_serves(m, n, k) == (m > 64 and not ops.tiles_serve(m, n, k)) and ops.tiles_serve(m, n, k) == (-(-m // 128) * -(-n // 128) >= (224 if k >= 8192 else 192) and k % 64 == 0)
 
 
 def test_products_whose_library_kernel_was_timed_elsewhere_stay_with_it(ops, tmp_path, monkeypatch):
