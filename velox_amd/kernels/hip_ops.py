@@ -1061,29 +1061,21 @@ class HipOps:
         return int(self.tiles_serve(m, n, k, recorded=recorded))
 
     def tile_splits(self, m: int, n: int, k: int) -> int:
-        """Parts of k in which ``linear`` works a product in the framework's own tiles of 128 x 256 (0: not at all, the library's).  The
+        """Parts of k in which ``linear`` works a long sum over few tiles in the own tiles (0: it is not cut and ``tiles_serve`` decides).  The
         library gives a product with few tiles and a long sum (a feed-forward's second product) too few workgroups; here
-        the sum is cut until about every compute unit has one, and the norm that follows adds the parts.  Measured on
-        MI355X, product and norm (us, library / own, n x k):
+        the sum is cut until about every compute unit has one, and the norm that follows adds the parts.  Counted in tiles of 128 x 256.  Measured on
+        MI355X, product and norm (us of the GPU, library / own, n x k, weights from memory):
 
-        - tiles for a third of the compute units: 3,584 x 18,944 at 65 tokens 100 / 46, 300: 105 / 62, 700: 171 / 111; 1,024 x 28,672 at 150:
-          104 / 54; 4,096 x 11,008 at 65: 42 / 34, 512: 76 / 61; 2,048 x 10,944 at 65: 37 / 30; 2,560 x 10,240 at 65: 31 / 31; 4,096 x 5,120 at
-          100: 25 / 25, 512: 45 / 41.  Below 20 million weights the library cuts the sum itself and is 2 to 5 us quicker with few rows:
-          2,048 x 8,448 at 128: 26 / 29, 150: 32 / 27, 1,036: 73 / 57; 1,536 x 8,960 at 128: 23 / 28, 150: 23 / 28, 200: 30 / 28, 1,036: 53 / 48;
-          2,048 x 7,168 at 150: 25 / 24, 400: 28 / 30, 700: 43 / 39; 2,048 x 5,632 at 128: 18 / 22, 150: 21 / 23, 300: 24 / 25, 512: 26 / 29, 700: 34 /
-          34, 1,280: 47 / 47; 1,024 x 8,192 at 200: 21 / 26, 300: 27 / 27, 1,000: 34 / 33.  Its call costs the host 19 us, though, and the own one
-          8, and a step of portions through a model of that size waits for the host up to some 500 rows (width 2,048, ff 5,632, 140 tokens:
-          2,260 to 2,390 us a step by the library, 2,190 to 2,360 with the own tiles, four runs each).  So: the own ones above 128 rows, where steps are not captured.  Smaller
-          still: 1,024 x 5,632 at 512: 22 / 27; 512 x 16,384 at 400: 33 / 36; 256 x 12,288 at 640: 27 / 30.
-        - more tiles, up to one per compute unit, and sums so long that the library is far from its rate: 3,584 x 18,944 at 836: 182 / 153,
-          1,536: 283 / 233, 2,048: 381 / 287; 4,096 x 16,512 at 700: 197 / 128, 2,048: 376 / 273; 5,120 x 27,648 at 836: 335 / 294, 1,536: 558 /
-          428; but 3,072 x 12,288 at 1,036: 112 / 104, 1,536: 138 / 144; 5,120 x 13,824 at 836: 156 / 158, 1,536: 211 / 227.  Wide products
-          have tiles enough for the library earlier: 8,192 x 29,568 at 512 (128 tiles): 327 / 274, 700 (192): 322 / 392; 8,192 x 16,384 at
-          512: 170 / 155, 640 (160): 192 / 203; 16,384 x 16,384 at 256 (128): 242 / 226, 400 (256): 278 / 298; 6,144 x 24,576 at 900 (192):
-          399 / 310, 6,144 x 16,384 at 1,280 (240): 245 / 268; 7,168 x 28,672 at 900 (224): 499 / 413, 1,100 (252): 426 / 466.
-
-        (With residual streams, whose norm adds the parts too: 4,096 x 11,008 at 100 rows 45 / 39, 512: 87 / 72; 2,048 x 8,448 at 300: 43 / 34;
-        2,048 x 5,632 at 300: 28 / 29, 512: 32 / 34, 1,280: 63 / 58.)"""
+        - tiles for a third of the compute units: 3,584 x 18,944 at 65 rows 100 / 34, 300: 106 / 60, 700: 170 / 100; 1,024 x 28,672 at 150:
+          103 / 34; 4,096 x 11,008 at 65: 44 / 29, 512: 82 / 61; 2,048 x 10,944 at 65: 38 / 21; 2,560 x 10,240 at 65: 31 / 23; 4,096 x 5,120 at
+          100: 25 / 21, 512: 45 / 40; 2,048 x 8,448 at 150: 33 / 20, 1,036: 74 / 54; 1,536 x 8,960 at 200: 35 / 22, 1,036: 57 / 46; 2,048 x 7,168 at 150: 29 / 18,
+          700: 46 / 38; 2,048 x 5,632 at 150: 24 / 18, 512: 31 / 30, 1,280: 56 / 47; 1,024 x 8,192 at 200: 24 / 19, 1,000: 40 / 32.  Below 20 million weights only above
+          128 rows, and not below 8 million or 1,024 columns: those lines were drawn with a slower kernel and have not been measured again.
+        - more tiles, up to one per compute unit, and sums of 16,384 terms and more: 3,584 x 18,944 at 836: 185 / 119, 2,048: 375 / 225; 4,096 x 16,512 at 700:
+          196 / 93, 2,048: 376 / 220; 5,120 x 27,648 at 1,536: 553 / 339; 6,144 x 24,576 at 900: 400 / 248; 7,168 x 28,672 at 900: 497 / 336; 8,192 x 29,568 at 512: 331 / 207,
+          640: 301 / 279, 700: 319 / 277 (whole in the own tiles 402), 836: 368 / 356, 1,000 (256 tiles): 384 / 373; 12,288 x 29,568 at 400: 328 / 316; 16,384 x 29,568 at 512 (256):
+          446 / 416; 16,384 x 16,384 at 512: 284 / 262; 6,144 x 24,576 at 1,280 (240): 401 / 325; but 6,144 x 16,384 at 1,280: 235 / 260.  Above that a cut
+          is no gain: 8,192 x 29,568 at 1,536 (384): 589, whole 579, in two parts 611."""
         if m <= 64 or not 5120 <= k < 1 << 21 or k % 8 != 0 or n % 4 != 0:
             return 0
         tiles, steps = -(-m // 128) * -(-n // 256), -(-k // 64)
@@ -1091,7 +1083,7 @@ class HipOps:
             if n * k < 20_000_000 and (n < 1024 or n * k < 8_000_000 or m <= 128):
                 return 0
             splits = min(8, self.num_cus // tiles)
-        elif k >= 16384 and tiles <= (self.num_cus if n < 6144 else 7 * self.num_cus // 8 if n < 8192 else self.num_cus // 2):
+        elif k >= 16384 and tiles <= self.num_cus:
             splits = self._core.velox_tiles_splits(m, n, k, 4)
         else:
             return 0
