@@ -253,6 +253,7 @@ def test_products_that_are_taken_in_parts_are_not_timed(tmp_path, monkeypatch):
     """A long sum whose parts the next norm adds runs in the own tiles and is not timed; the same product with a bias, or wanted whole, is the library's."""
     engine = engine_for(make_folder(tmp_path, "A", "bfloat16"), "A", "bfloat16", max_num_seqs=4, max_num_batched_tokens=64)
     timed = []
+    monkeypatch.setattr(engine.ops, "library_serves", lambda *sizes, **how: type(engine.ops).library_serves(engine.ops, *sizes, **how))
     monkeypatch.setattr(engine.ops, "tune_library_products", lambda shapes, counts, results_file=None: timed.extend(shapes) or len(shapes))
     mixer, feed_forward = engine.model.blocks[0].mixer, engine.model.blocks[0].feed_forward
     wanted = {tuple(w.shape) for w in (mixer.qkv_weight, feed_forward.gate_up_weight)}

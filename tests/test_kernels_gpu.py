@@ -1501,7 +1501,7 @@ def test_the_library_is_said_to_serve_what_linear_hands_to_it(ops, monkeypatch, 
     for given in (bias, None):
         calls.clear()
         assert ops.linear(x, w, given, torch.bfloat16).shape == (m, n)
-        assert ops.library_serves(m, n, k) == (not calls) == (in_parts != 1)
+        assert type(ops).library_serves(ops, m, n, k) == (not calls) == (in_parts != 1)
     calls.clear()
     got = ops.linear(x, w, None, torch.bfloat16, partials_ok=True)
     assert ops.own_tile_parts(m, n, k, True) == in_parts and len(calls) == (in_parts > 0) and (got.shape == (in_parts, m, n) if in_parts > 1 else got.shape == (m, n))
@@ -1582,7 +1582,7 @@ def parts_into_every_consumer(ops, m, n, k, parts, dtype):
                                      (513, 16384, 16384), (1536, 5120, 13824), (64, 3584, 18944), (4096, 3584, 18944)])
 def test_products_whose_sum_is_not_cut(ops, m, n, k):
     assert ops.tile_splits(m, n, k) == 0
-    assert ops.library_serves(m, n, k) == (m > 64 and not ops.tiles_serve(m, n, k)) and ops.tiles_serve(m, n, k) == (-(-m // 128) * -(-n // 128) >= (224 if k >= 8192 else 192) and k % 64 == 0)
+    assert type(ops).library_serves(ops, m, n, k) == (m > 64 and not ops.tiles_serve(m, n, k)) and ops.tiles_serve(m, n, k) == (-(-m // 128) * -(-n // 128) >= (224 if k >= 8192 else 192) and k % 64 == 0)
 
 
 def test_products_whose_library_kernel_was_timed_elsewhere_stay_with_it(ops, tmp_path, monkeypatch):
