@@ -4,7 +4,7 @@
 // plain fused multiply-adds.  It serves operand mixes no library call covers (bfloat16 activations with
 // weights a checkpoint stores in float32), float32 rows that are not whole 16-byte pieces and sums of
 // fewer than GEMM_FOLD terms; other float32 products run on the float32 matrix instructions (gemm_mfma_f32_kernel) or, larger ones,
-// on exactly split operands (split_f32.hip), so a float32 run nowhere has less than float32's precision.  Each output element is summed over k in one fixed
+// on exactly split operands (split_f32.hip), whose error against 64 bits is below the float32 instructions' for operands of any size.  Each output element is summed over k in one fixed
 // order by one thread, so a row's result does not depend on what the other rows of the batch hold (their number chooses the
 // kernel: up to 16 rows have one of their own, with an order of its own).  The sum
 // is built from sums of GEMM_FOLD consecutive terms, each started at zero: the rounding error of a

@@ -20,7 +20,7 @@
 
 typedef __bf16 gm_bf16x8_t __attribute__((ext_vector_type(8)));
 
-#define GM_ROWS 64       // rows of a tile without a plan (a plan's tiles hold 64 or 128)
+#define GM_ROWS 64       // rows of a tile without a plan (a plan's tiles hold 64, 128 or 192)
 #define GM_FEW_COLS 32   // output columns of a workgroup of the kernel for few rows (GLU: 16)
 
 enum { GM_PLAIN = 0, GM_GLU = 1, GM_GATE = 2, GM_ACT = 3 };

@@ -11,8 +11,8 @@
 // times -2^24) and subtracted: rounded down throughout, all of a layer's outputs were too small by the same 3e-8 (1,536 terms) or 8e-8 (8,960) of
 // their norm, which added up from layer to layer, and a model's logits were 3% further from 64 bits than with the float32 instructions,
 // although each product was closer (eight layers of width 1,536, six seeds: 1.64 to 1.94e-06, 1.68 to 2.00e-06; so 1.59 to 1.90e-06).  Error against float64, float32 matrix
-// instructions / this: 512 terms 2.1e-07 / 1.6e-07, 1,536 2.1e-07 / 1.7e-07, 8,960 2.3e-07 / 1.9e-07, 18,944 2.6e-07 / 2.1e-07; of terms of one
-// sign 9.5e-08 / 7.4e-08, 6.2e-08 / 6.2e-08, 7.5e-08 / 5.3e-08, 9.8e-08 / 5.8e-08.  (Inner sums of 64 terms: 1.3e-07 at 1,536 terms, 2% slower;
+// instructions / this: 512 terms 2.1e-07 / 1.6e-07, 1,536 2.1e-07 / 1.7e-07, 8,960 2.3e-07 / 1.7e-07, 18,944 2.6e-07 / 1.8e-07; of terms of one
+// sign 9.5e-08 / 7.3e-08, 6.2e-08 / 6.2e-08, 7.5e-08 / 5.3e-08, 9.8e-08 / 5.8e-08.  (Inner sums of 64 terms: 1.3e-07 at 1,536 terms, 2% slower;
 // sums of 1,024 in the result's place: 190 instead of 180 us where 1,536 terms are added, for the passes over the result.)
 //
 // What bounds it: the matrix cores (six instructions of 16 cycles for 16 x 16 x 32 terms: at most 2,500 / 6 = 417 TFLOP/s of float32
@@ -23,8 +23,8 @@
 //     same time.  (All of them first: 4% slower.  The two waves of a SIMD at different times is better with two tiles of rows,
 //     both at one time with four.)
 //   - One barrier a step; a wave's operands leave LDS once per step, those of a column of tiles behind the products of the one before.
-// Measured on MI355X (us, float32 matrix instructions / this): 616 rows, 1,536 -> 17,920: 322 / 190 (178 TFLOP/s); 8,960 -> 1,536 in parts 201 /
-// 96; 4,000 rows, 2,048 -> 11,264: 1,570 / 950 (194); 64 rows, 8,960 -> 1,536 in eight parts 72 / 25.  Without the splitting (stale operands)
+// Measured on MI355X (us, float32 matrix instructions / this): 616 rows, 1,536 -> 17,920: 330 / 203 (167 TFLOP/s); 8,960 -> 1,536 in parts 206 /
+// 94; 4,000 rows, 2,048 -> 11,264: 1,560 / 970 (191); 64 rows, 8,960 -> 1,536 in eight parts 69 / 25.  Without the splitting (stale operands)
 // 4,000 rows take 0.74 of the time: what is left to gain.
 #include "common.h"
 

@@ -18,7 +18,7 @@
 //   - Workgroups stay and take tile after tile; a tile's last steps already load the next one's first.
 //   - Tiles are dealt to the eight XCDs in contiguous runs, in blocks of 1,024 rows, column after column, so that the 32 tiles that an
 //     XCD has under way share a few rows of either operand in its L2 (2,048 rows instead: 4% slower at 4,001 x 22,016 x 4,096).
-// Measured on MI355X (us, the matrix library / this): 2,048 x 37,888 x 3,584 535 / 409 and with SiLU behind it 572 / 416; 836 rows 268 / 198;
+// Measured on MI355X (us, the matrix library / this): 2,048 x 37,888 x 3,584 535 / 409 and with SiLU behind it 572 / 428; 836 rows 268 / 198;
 // 4,001 x 22,016 x 4,096 640 / 530; 4,001 x 4,096 x 11,008 228 / 232; 1,036 x 10,368 x 2,048 49 / 38.
 // An output is summed over k in one chain of 32-index instructions from zero: every tile gives the same bits.
 //

@@ -5,10 +5,10 @@ what the kernels and their launch grids assume (devices, dtypes, contiguity, ali
 before launching, because a kernel that reads out of bounds takes the whole GPU down.  There
 is no fallback: without a GPU, without hipcc or without the libraries, loading fails.
 
-Matrix products: a float32 run uses the exact FMA kernel (``gemm.hip``); so does any operand mix
-a library has no call for.  bfloat16 x bfloat16 products go to the library behind
-``torch.nn.functional.linear`` (hipBLASLt), as the reference uses cuBLAS through ``nn.Linear``
-(reference ``src/self_attention.py:48,90``, ``src/mlp.py:13,15``).
+Matrix products (the reference's go to cuBLAS through ``nn.Linear``, ``src/self_attention.py:48,90``, ``src/mlp.py:13,15``): a float32 run's are
+multiply-adds, float32 matrix instructions or exactly split operands (``gemm.hip``, ``split_f32.hip``), as is any operand mix a library has
+no call for; bfloat16 ones run in the skinny kernels up to 64 rows, above that in large tiles of the framework's own, and in the library
+behind ``torch.nn.functional.linear`` (hipBLASLt) where ``HipOps.linear`` says so.
 """
 from __future__ import annotations
 
