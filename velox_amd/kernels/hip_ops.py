@@ -1055,7 +1055,9 @@ class HipOps:
     def own_tile_parts(self, m: int, n: int, k: int, in_parts: bool, recorded: Optional[bool] = None) -> int:
         """Parts of k in which ``linear`` works a bfloat16 product of more than 64 rows in the own tiles: 0, it goes to the library; 1, a whole
         result; more, with ``in_parts`` (float32 partial sums are wanted) alone.  ``recorded``: as for ``tiles_serve``."""
-        splits = self.tile_splits(m, n, k)
+        if m <= 64:
+            return 0
+        splits = self.tile_splits(m, n, k) if k >= 5120 else 0
         if splits == 1 or (splits > 1 and in_parts):
             return splits
         return int(self.tiles_serve(m, n, k, recorded=recorded))
