@@ -543,6 +543,30 @@ def test_paged_attention_long_portions(ops, ref, dtype, nh, nkv, d, page, window
     torch.testing.assert_close(_run_attention(ops, alone, nh, nkv, d, page, window=window), got[first:first + 300], **same)
 
 
+@pytest.mark.parametrize("nh,nkv,d,page", [(4, 2, 16, 4), (6, 2, 48, 16), (5, 1, 80, 8), (7, 1, 96, 32), (28, 4, 128, 16), (40, 8, 128, 2)])
+@pytest.mark.parametrize("window,splits", [(None, None), (90, None), (None, 3)])
+def test_float32_row_tiles_that_waves_share_keep_their_bits(ops, ref, nh, nkv, d, page, window, splits):
+    """Float32 portions of few rows: waves that share a row tile (each a part of the keys, then a part of the channels) give the
+    bits of one wave per row tile, in workgroups of 16, 32 and 64 rows (1 row, one short of a row tile, one beyond it, several
+    workgroups; key tiles that only some of a workgroup's rows read), and with them whatever the launcher picks."""
+    from velox_amd.engine.batch import Workspace
+
+    seqs = [(1, 97), (15, 15), (17, 145), (64, 64), (65, 193), (130, 130), (2, 66)]
+    case = _attention_case(torch.float32, nh, nkv, d, page, seqs, seed=d + nh + 4)
+    workspace = Workspace(torch.device("cuda"))
+    lib = ops.attention_library(d)
+    got = {}
+    try:
+        for choice in (1, 2, 3, 4, 0):
+            lib.velox_attention_portion_kernel(choice)
+            got[choice] = _run_attention(ops, case, nh, nkv, d, page, window=window, splits=splits, workspace=workspace)
+    finally:
+        lib.velox_attention_portion_kernel(0)
+    torch.testing.assert_close(got[1], _run_attention(ref, case, nh, nkv, d, page, window=window), rtol=1e-4, atol=1e-5)
+    for choice in (2, 3, 4, 0):
+        assert torch.equal(got[choice], got[1]), choice
+
+
 @pytest.mark.parametrize("dtype,nh,nkv,d,page,long_context,choices", [
     (torch.bfloat16, 14, 2, 128, 8, 17000, (1, 2, 3)), (torch.bfloat16, 6, 3, 64, 8, 16500, (2, 3)), (torch.float32, 4, 2, 32, 4, 9000, (0,))])
 @pytest.mark.parametrize("window", [None, 5000])

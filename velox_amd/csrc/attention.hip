@@ -253,7 +253,11 @@ constexpr int GENERAL_MIN_WAVES = D <= 128 ? 2 : 1;
 // KSPLIT = 2: the workgroup has two sets of 4 waves that own the same rows and take the key tiles alternately, each
 // set staging its own tiles; at the end the second set hands its running (maximum, sum, output) to the first
 // through LDS.  The longest workgroups of a causal step, which decide how long the step takes, finish in half the time.
-template <typename T, int BN, int CT, int KSPLIT, int WAVES = 4>
+//
+// SHARE > 1 (float32): so many waves share a row tile.  Each takes its part of a tile's keys for the scores and its part of the
+// channels for the output; the maxima and then the probabilities go through LDS, behind a barrier each.  Every score, every
+// channel and every sum is added up in the order of SHARE = 1, with its bits.
+template <typename T, int BN, int CT, int KSPLIT, int WAVES = 4, int SHARE = 1>
 __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_waves_per_eu(GENERAL_MIN_WAVES, WAVES > 4 ? 4 : 2))) paged_attention_kernel(
     const T* __restrict__ qkv, int qkv_stride, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
     const int* __restrict__ block_tables, int table_width, const int* __restrict__ cu_q, const int* __restrict__ kv_lens,
@@ -273,21 +277,27 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
   constexpr int NKB = BN / KB;                  // contraction blocks of P V
   constexpr int TPB = KB / 16;                  // S^T tiles per key block
   constexpr int NC = D / 16;                    // 16-channel tiles of the output
+  constexpr int NTP = NT / SHARE, NCP = (NC + SHARE - 1) / SHARE;  // a wave's part of the key tiles, of the channel tiles
+  static_assert(SHARE == 1 || (sizeof(T) == 4 && CT == 1 && KSPLIT == 1 && NT % SHARE == 0 && WAVES % SHARE == 0 && DP == D), "how row tiles are shared");
   constexpr int SETW = 64 * WAVES;              // threads of a set of waves
   static_assert(KSPLIT == 1 || WAVES == 4, "two sets of waves are sets of four");
-  constexpr int ROWS_PER_BLOCK = 16 * WAVES * CT;
+  constexpr int ROWS_PER_BLOCK = 16 * WAVES * CT / SHARE;
   constexpr int TILE_ELEMS = BN * KS + D * VS;                      // one set's K tile and V^T tile
   constexpr int MERGE_FLOATS = KSPLIT > 1 ? 256 * CT * (4 * NC + 2) : 0;  // what the second set hands over at the end
   constexpr int TILE_BYTES = KSPLIT * TILE_ELEMS * (int)sizeof(T);
   constexpr int SMEM_BYTES = TILE_BYTES > 4 * MERGE_FLOATS ? TILE_BYTES : 4 * MERGE_FLOATS;
   __shared__ __attribute__((aligned(16))) char smem[SMEM_BYTES];
   __shared__ int page_ids[PREFILL_PAGE_IDS];
+  __shared__ float4_t shared_probs[SHARE > 1 ? WAVES / SHARE * NT * 64 : 1];  // [row tile][key tile][lane]
+  __shared__ float shared_max[SHARE > 1 ? WAVES * 16 : 1];                    // [row tile][part][row]
 
   const int set = KSPLIT > 1 ? threadIdx.x / 256 : 0;  // which set of 4 waves
   const int tid = KSPLIT > 1 ? threadIdx.x % 256 : threadIdx.x;  // thread within the set
   T* const k_tile = reinterpret_cast<T*>(smem) + set * TILE_ELEMS;
   T* const v_tile = k_tile + BN * KS;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = (tid >> 6) / SHARE;  // (which row tile)
+  const int part = (tid >> 6) % SHARE;                   // which part of it
+  const int t_own = part * NTP, c_own = part * NCP;
   const int g = lane >> 4, i = lane & 15;
   const int group = nh / nkv;
   // The grid is (sequence and split, KV head, row block), and blockIdx.z counts a sequence's row blocks from its LAST
@@ -372,7 +382,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
 
   Operand qf[CT][NQB];
   float m_i[CT], l_i[CT];
-  float4_t acc_o[CT][NC];
+  float4_t acc_o[CT][NCP];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const T* qp = qkv + (size_t)(q_start + tok[ct]) * qkv_stride + (size_t)head[ct] * D + VEC * g;
@@ -384,7 +394,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
     m_i[ct] = -INFINITY;
     l_i[ct] = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc_o[ct][c] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < NCP; ++c) acc_o[ct][c] = float4_t{0.f, 0.f, 0.f, 0.f};
   }
   const float scale_eff = scale * Softmax<T>::SCALE;
   const float scale_used = BIASED || CAPPED ? 1.f : scale_eff;  // (with a cap or a bias the scores are scaled where it is applied)
@@ -503,7 +513,13 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
       }
       if (tile + KSPLIT < tile_hi) fetch(keys.first_key<BN>(tile + KSPLIT));  // in flight while this tile is computed
     }
-    if (!have_tile || n0 > wave_last_pos) continue;  // nothing this wave may read; it still took part in the staging
+    if (!have_tile || n0 > wave_last_pos) {  // nothing this wave may read; it still took part in the staging
+      if constexpr (SHARE > 1) {
+        __syncthreads();
+        __syncthreads();
+      }
+      continue;
+    }
 
     // ---- S^T = K Q^T ----------------------------------------------------------------------
     // bfloat16: the operands of the next 16 keys are asked for before this 16 keys' matrix instructions are issued, and
@@ -511,14 +527,14 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
     // matrix instructions it feeds: 2,048 to 8,192 tokens 2-4% faster).  float32 operands and heads beyond 128 channels
     // are too many registers for it.
     constexpr int KEYS_AHEAD = (sizeof(T) == 2 && D <= 128) ? 1 : 0;
-    float4_t s[CT][NT];
+    float4_t s[CT][NTP];
     Operand kf[KEYS_AHEAD + 1][NQB];
     if constexpr (KEYS_AHEAD > 0) {
 #pragma unroll
       for (int cb = 0; cb < NQB; ++cb) kf[0][cb] = load_operand<T>(k_tile + i * KS + KB * cb + VEC * g);
     }
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
+    for (int t = 0; t < NTP; ++t) {
       if constexpr (KEYS_AHEAD > 0) {
         if (t + 1 < NT) {
 #pragma unroll
@@ -530,7 +546,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
       for (int ct = 0; ct < CT; ++ct) s[ct][t] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int cb = 0; cb < NQB; ++cb) {
-        if constexpr (KEYS_AHEAD == 0) kf[0][cb] = load_operand<T>(k_tile + (16 * t + i) * KS + KB * cb + VEC * g);
+        if constexpr (KEYS_AHEAD == 0) kf[0][cb] = load_operand<T>(k_tile + (16 * (t_own + t) + i) * KS + KB * cb + VEC * g);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) s[ct][t] = B::mma(kf[t & KEYS_AHEAD][cb], qf[ct][cb], s[ct][t]);
       }
@@ -541,7 +557,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < NTP; ++t)
 #pragma unroll
           for (int j = 0; j < 4; ++j) s[ct][t][j] = cap(s[ct][t][j]);
     }
@@ -555,15 +571,15 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
         if (d0 - (BN - 1) >= bias_len - 1) {
           const float c = tab[bias_len - 1] * Softmax<T>::SCALE;
 #pragma unroll
-          for (int t = 0; t < NT; ++t)
+          for (int t = 0; t < NTP; ++t)
 #pragma unroll
             for (int j = 0; j < 4; ++j) s[ct][t][j] = fmaf(s[ct][t][j], CAPPED ? 1.f : scale_eff, c);
         } else {
 #pragma unroll
-          for (int t = 0; t < NT; ++t)
+          for (int t = 0; t < NTP; ++t)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              int d = d0 - (16 * t + 4 * g + j);
+              int d = d0 - (16 * (t_own + t) + 4 * g + j);
               d = d < 0 ? 0 : (d > bias_len - 1 ? bias_len - 1 : d);
               s[ct][t][j] = fmaf(s[ct][t][j], CAPPED ? 1.f : scale_eff, tab[d] * Softmax<T>::SCALE);
             }
@@ -578,15 +594,15 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
       float mx = -INFINITY;
       if (whole) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < NTP; ++t)
 #pragma unroll
           for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[ct][t][j]);
       } else {
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < NTP; ++t)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const int n = n0 + 16 * t + 4 * g + j;
+            const int n = n0 + 16 * (t_own + t) + 4 * g + j;
             const bool keep = row_ok[ct] && n < kv_len && n <= pos[ct] && (window <= 0 || n > pos[ct] - window || (KEEPS && n < extras.keep_first));
             s[ct][t][j] = keep ? s[ct][t][j] : -INFINITY;
             mx = fmaxf(mx, s[ct][t][j]);
@@ -594,24 +610,48 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
       }
       mx = fmaxf(mx, __shfl_xor(mx, 16, VELOX_WAVE));
       mx = fmaxf(mx, __shfl_xor(mx, 32, VELOX_WAVE));
+      if constexpr (SHARE > 1) {
+        if (g == 0) shared_max[(wave * SHARE + part) * 16 + i] = mx;
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < SHARE; ++p) mx = fmaxf(mx, shared_max[(wave * SHARE + p) * 16 + i]);
+      }
       const float m_new = fmaxf(m_i[ct], mx * scale_used);
       const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
       alpha[ct] = (m_i[ct] == -INFINITY) ? 0.f : Softmax<T>::exp_of(m_i[ct] - m_safe);
       float psum = 0.f;
+      if constexpr (SHARE > 1) {
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-        Vec16<T> packed;
-        T* e = reinterpret_cast<T*>(&packed.v);
+        for (int t = 0; t < NTP; ++t) {
+          float4_t p;
 #pragma unroll
-        for (int u = 0; u < TPB; ++u)
+          for (int j = 0; j < 4; ++j) p[j] = Softmax<T>::exp_of(fmaf(s[ct][t][j], scale_used, -m_safe));
+          shared_probs[(wave * NT + t_own + t) * 64 + lane] = p;
+        }
+        __syncthreads();
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            // a masked score is -inf and gives exp(-inf) = 0; m_safe is finite
-            const float p = Softmax<T>::exp_of(fmaf(s[ct][kb * TPB + u][j], scale_used, -m_safe));
-            psum += p;
-            e[4 * u + j] = from_f32<T>(p);
-          }
-        pf[ct][kb] = __builtin_bit_cast(Operand, packed.v);
+        for (int kb = 0; kb < NKB; ++kb) {
+          const float4_t p = shared_probs[(wave * NT + kb) * 64 + lane];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) psum += p[j];
+          pf[ct][kb] = __builtin_bit_cast(Operand, p);
+        }
+      } else {
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) {
+          Vec16<T> packed;
+          T* e = reinterpret_cast<T*>(&packed.v);
+#pragma unroll
+          for (int u = 0; u < TPB; ++u)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              // a masked score is -inf and gives exp(-inf) = 0; m_safe is finite
+              const float p = Softmax<T>::exp_of(fmaf(s[ct][kb * TPB + u][j], scale_used, -m_safe));
+              psum += p;
+              e[4 * u + j] = from_f32<T>(p);
+            }
+          pf[ct][kb] = __builtin_bit_cast(Operand, packed.v);
+        }
       }
       l_i[ct] = l_i[ct] * alpha[ct] + psum;  // partial over this lane's keys; the four lane groups are summed at the end
       m_i[ct] = m_new;
@@ -624,7 +664,8 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb) vf[a][kb] = load_operand<T>(v_tile + (16 * a + i) * VS + KB * kb + VEC * g);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
+    for (int c = 0; c < NCP; ++c) {
+      if (NC % SHARE != 0 && c_own + c >= NC) break;
       if constexpr (TILES_AHEAD > 0) {
         if (c + TILES_AHEAD < NC) {
 #pragma unroll
@@ -636,7 +677,7 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
       for (int ct = 0; ct < CT; ++ct) acc_o[ct][c] = acc_o[ct][c] * alpha[ct];
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb) {
-        if constexpr (TILES_AHEAD == 0) vf[0][kb] = load_operand<T>(v_tile + (16 * c + i) * VS + KB * kb + VEC * g);
+        if constexpr (TILES_AHEAD == 0) vf[0][kb] = load_operand<T>(v_tile + (16 * (c_own + c) + i) * VS + KB * kb + VEC * g);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) acc_o[ct][c] = B::mma(vf[c % (TILES_AHEAD + 1)][kb], pf[ct][kb], acc_o[ct][c]);
       }
@@ -684,20 +725,22 @@ __global__ void __launch_bounds__(64 * WAVES * KSPLIT) __attribute__((amdgpu_wav
     const float inv = l > 0.f ? 1.f / l : 1.f;
     const size_t token = (size_t)(q_start + tok[ct]);
     if (splits == 1) {
-      T* dst = out + (token * nh + head[ct]) * D + 4 * g;
+      T* dst = out + (token * nh + head[ct]) * D + 16 * c_own + 4 * g;
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
+      for (int c = 0; c < NCP; ++c) {
+        if (NC % SHARE != 0 && c_own + c >= NC) break;
         float4_t o = acc_o[ct][c] * inv;
-        if constexpr (GATED) o = o * gate_of<T>(extras, token, head[ct], 16 * c + 4 * g);
+        if constexpr (GATED) o = o * gate_of<T>(extras, token, head[ct], 16 * (c_own + c) + 4 * g);
 #pragma unroll
         for (int j = 0; j < 4; ++j) dst[16 * c + j] = from_f32<T>(o[j]);
       }
     } else {
       const size_t slot = ((size_t)split * total_tokens + token) * nh + head[ct];
-      float* dst = part_o + slot * D + 4 * g;
+      float* dst = part_o + slot * D + 16 * c_own + 4 * g;
 #pragma unroll
-      for (int c = 0; c < NC; ++c) *reinterpret_cast<float4_t*>(dst + 16 * c) = acc_o[ct][c] * inv;
-      if (g == 0) part_lse[slot] = l > 0.f ? m_i[ct] * Softmax<T>::LN_UNIT + logf(l) : -INFINITY;
+      for (int c = 0; c < NCP; ++c)
+        if (NC % SHARE == 0 || c_own + c < NC) *reinterpret_cast<float4_t*>(dst + 16 * c) = acc_o[ct][c] * inv;
+      if (part == 0 && g == 0) part_lse[slot] = l > 0.f ? m_i[ct] * Softmax<T>::LN_UNIT + logf(l) : -INFINITY;
     }
   }
 }
@@ -1538,7 +1581,8 @@ __global__ void __launch_bounds__(MERGE_THREADS) merge_splits_kernel(const float
 }
 
 // Which kernel portions of prompts take: 0 = chosen by shape; 1 = never the kernel with direct loads; 2 = that kernel
-// wherever it can run, 3 = the same with two sets of waves (for tests and measurements).
+// wherever it can run, 3 = the same with two sets of waves (for tests and measurements).  In float32 up to 128 channels: 1 = a row
+// tile per wave, 2, 3, 4 = 16, 32, 64 rows whose tiles waves share.
 static int portion_kernel_choice = 0;
 extern "C" void velox_attention_portion_kernel(int choice) { portion_kernel_choice = choice; }
 
@@ -1647,7 +1691,39 @@ static int launch(const void* qkv, int qkv_stride, const void* k_cache, const vo
   constexpr int WIDE = (sizeof(T) == 2 && D <= 128) ? 2 : 1;
   const int rows = max_q_len * group;
   if ((rows + 63) / 64 > 65535) return (int)hipErrorInvalidValue;  // (row blocks are the grid's third dimension)
-  if (WIDE == 2 && rows > 64 && (long long)total_tokens * group / 128 * nkv * splits >= compute_units()) {
+  // float32: a tile of 64 keys under a row tile is 8,192 cycles of matrix instructions on one SIMD, so a step of few workgroups is
+  // as long as its longest wave's walk, most of it on compute units whose other waves are done or on none at all.  Waves that share
+  // row tiles shorten that walk, with the same bits, and smaller workgroups spread it: 16 rows by four waves while those are no more
+  // than the compute units, 32 rows by eight waves up to the same count (up to 2 1/4 for one prompt from an empty cache, whose
+  // workgroups get shorter and shorter), 64 rows by eight waves up to two per compute unit.  Measured on MI355X (us, four waves
+  // of a row tile each / 64 rows by eight / 32 rows by eight / 16 rows by four; heads of 128 channels): 12 over 2, 64 tokens 12.4 / 12.1 /
+  // 9.4 / 8.1, 611 tokens 70 / 64 / 44 / 42, 1,024 tokens 108 / 99 / 67 / 68, 64 tokens behind 2,936 keys 305 / 277 / 184 / 159; 28 over 4, 300 tokens 38 /
+  // 36 / 25 / 25, 611 tokens 74 / 65 / 58 / 63, 1,024 tokens 131 / 105 / 135 / 149, 300 tokens behind 1,700 keys 211 / 192 / 218 / 216, 4 x 128
+  // tokens 19.7 / 18.9 / 21.2 / 23.1; 16 over 4, 2,048 tokens 260 / 209 / 269 / 309; 28 over 4, 2 x 600 tokens behind 1,000 keys (2.06 workgroups of 64
+  // rows per compute unit) 311 / 352 / 397 / 427.
+  int shared_rows = 0;
+  if constexpr (sizeof(T) == 4 && D <= 128) {
+    const long long units = compute_units(), per_block = (long long)nkv * num_seqs * splits;
+    const bool one_prompt = num_seqs == 1 && max_kv_len <= max_q_len;
+    const long long by_16 = (rows + 15) / 16 * per_block, by_32 = (rows + 31) / 32 * per_block, by_64 = (rows + 63) / 64 * per_block;
+    if (by_16 <= units) shared_rows = 16;
+    else if (by_32 <= units || (one_prompt && 4 * by_32 <= 9 * units)) shared_rows = 32;
+    else if (by_64 <= 2 * units) shared_rows = 64;
+    if (portion_kernel_choice > 0) shared_rows = portion_kernel_choice == 1 ? 0 : portion_kernel_choice == 2 ? 16 : portion_kernel_choice == 3 ? 32 : 64;
+    if (shared_rows > 0) {
+      const dim3 grid(num_seqs * splits, nkv, (rows + shared_rows - 1) / shared_rows);
+      if (grid.z > 65535u) return (int)hipErrorInvalidValue;
+      const auto kernel = shared_rows == 16   ? paged_attention_kernel<T, BN, 1, 1, 4, 4>
+                          : shared_rows == 32 ? paged_attention_kernel<T, BN, 1, 1, 8, 4>
+                                              : paged_attention_kernel<T, BN, 1, 1, 8, 2>;
+      kernel<<<grid, shared_rows == 16 ? 256 : 512, 0, stream>>>((const T*)qkv, qkv_stride, (const T*)k_cache, (const T*)v_cache, block_tables, table_width,
+                                                                 cu_q, kv_lens, (T*)out, part_o, part_lse, nh, nkv, page_shift, scale, window, splits, total_tokens,
+                                                                 bias_table, bias_len, sinks, extras);
+    }
+  }
+  if (shared_rows > 0) {
+    // launched above
+  } else if (WIDE == 2 && rows > 64 && (long long)total_tokens * group / 128 * nkv * splits >= compute_units()) {
     if (max_kv_len - max_q_len / 2 <= 1280 || rows < 192) {  // (keys an average row reads)
       dim3 grid(num_seqs * splits, nkv, (rows + 127) / 128);
       // With enough workgroups to keep two on every compute unit, the 128 rows go to four waves of two row tiles: half
