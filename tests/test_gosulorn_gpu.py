@@ -133,6 +133,45 @@ def test_stream_update_with_a_term_in_parts(ops, hidden, streams, parts):
             near(a, b, 1e-6), near(a_res, b_res, 1e-6)  # (a product and a sum may be contracted in one build and not in the other)
 
 
+@pytest.mark.parametrize("streams,hidden,center", [(4, 2048, True), (3, 68, False), (1, 1000, True), (4, 4100, True), (2, 12, False), (1, 16384, False)])
+def test_streams_that_stay_unwritten_give_the_bits_of_one_pass_each(ops, streams, hidden, center):
+    """Seven updates (one and two terms, float32, bfloat16 and parts; with and without weights) over rows that all streams begin with, written back
+    every fourth time, the third time and the second, and not at all: every norm and what is written in the end have the bits of a pass per update."""
+    g, tokens = torch.Generator().manual_seed(hidden + streams), 37
+    base = rnd(g, tokens, hidden)
+    updates = []
+    for q in range(7):
+        terms = [rnd(g, tokens, hidden, dtype=torch.bfloat16 if q % 2 else torch.float32)]
+        if q == 3:
+            terms[0] = rnd(g, 4, tokens, hidden)
+        if q % 3 == 1:
+            terms.append(rnd(g, tokens, hidden, dtype=torch.bfloat16))
+        plain = q == 5
+        updates.append((tuple(terms), (1.0, 1.1)[:len(terms)] if q != 4 else (0.8, 1.1), None if plain else rnd(g, streams, streams), None if plain else rnd(g, streams), rnd(g, streams)))
+    w = rnd(g, hidden)
+
+    def norm(residual, terms, scales, mix, out_w, in_w, rows=None, **more):
+        return ops.stream_norm(residual, terms, scales, mix, out_w, in_w, w, 1e-5, streams, center, torch.bfloat16, rows=rows, **more)
+
+    rows = torch.tensor([5, tokens - 1, 0], dtype=torch.int32).cuda()
+    want_streams = base.repeat(1, streams)
+    want = [norm(want_streams, (), (), None, None, updates[0][4])] + [norm(want_streams, *u[:4], u[4]) for u in updates]
+    chosen = norm(want_streams, (), (), None, None, None, rows=rows)
+    for most in (0, 1, 2, 3):
+        residual, held, unwritten = torch.full((tokens, streams * hidden), float("nan"), device="cuda"), [], base
+        got = [norm(residual, (), (), None, None, updates[0][4], base=base, settle=False)]
+        for u in updates:
+            wait = len(held) < most and u[0][0].dim() == 2
+            got.append(norm(residual, *u[:4], u[4], earlier=tuple(held), base=unwritten, settle=not wait))
+            held, unwritten = (held + [u[:4]], unwritten) if wait else ([], None)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), most
+        if held:
+            last = held.pop()
+            assert torch.equal(norm(residual, *last, None, rows=rows, earlier=tuple(held), base=unwritten), chosen)
+        else:
+            assert torch.equal(residual, want_streams) and torch.equal(norm(residual, (), (), None, None, None, rows=rows), chosen)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_embedding_copies_and_gated_activation(ops, ref, dtype):
     g, dt = torch.Generator().manual_seed(3), DTYPES[dtype]
@@ -407,6 +446,22 @@ def test_all_ways_of_cutting_on_the_gpu(tmp_path, name, dtype):
         for label in ("tail", "portions", "mixed", "recompute"):  # the ways of cutting agree with each other at least as closely
             for rid in requests:
                 torch.testing.assert_close(results[label][rid], results["whole"][rid], rtol=1e-4, atol=3e-5 * max(1.0, float(expected[rid].abs().max())))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", ["A", "B", "C", "D", "E"])
+def test_whole_models_whose_streams_stay_unwritten(tmp_path, ops, monkeypatch, name, dtype):
+    """Every model with its streams written every fourth time (where rows are a multiple of four channels) and once per sub-layer: the same bits, in whole
+    prompts, portions, and decoded tokens from captured steps."""
+    folder = write_folder(tmp_path / name, CONFIGS[name], seed=2, dtype=dtype)
+    requests = prompts(CONFIGS[name]["vocab"], [141, 1, 37, 98], seed=11)
+    trace, results = rc.mixed(requests, seed=5), []
+    for from_bytes in (1, 1 << 60):
+        monkeypatch.setattr(type(ops), "STREAMS_WAIT_FROM_BYTES", from_bytes)
+        replayer = Replayer(folder, dtype, rc.tokens_needed(trace, PAGE_SIZE[name]), block_size=PAGE_SIZE[name], max_live=4, enable_graphs=True)
+        results.append(rc.collect(trace, rc.run_trace(replayer, trace), requests))
+    for rid in requests:
+        assert torch.equal(results[0][rid], results[1][rid]), rid
 
 
 @pytest.mark.parametrize("name,cuts", [("E", (700,)), ("E", (3, 1, 690, 2, 1, 1, 1, 1)), ("C", (16, 15, 1, 400, 2) + (1,) * 10), ("A", (4, 4, 248) + (1,) * 4)])

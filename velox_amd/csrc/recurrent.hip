@@ -136,6 +136,31 @@ __device__ __forceinline__ void store4_from_f32(void* p, int is_bf16, size_t i, 
   *reinterpret_cast<short4_t*>((bf16_t*)p + i) = raw;
 }
 
+// The norm of a row of which a lane holds PIECES pieces `u`, whose sum over the lane is `sum`.
+template <int PIECES>
+__device__ __forceinline__ void norm_of_pieces(const StreamNormArgs& a, const float4_t (&u)[PIECES], float sum, int row, float* scratch) {
+  const int H = a.hidden, pieces = H / 4;
+  float mean = 0.f;
+  if (a.center) mean = block_sum(sum, scratch) / (float)H;
+  float sq = 0.f;
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    if (threadIdx.x + p * blockDim.x < pieces) {
+      const float4_t d = u[p] - mean;
+      sq += (d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]);
+    }
+  }
+  const float inv = 1.f / sqrtf(block_sum(sq, scratch) / (float)H + a.eps);
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int piece = threadIdx.x + p * blockDim.x;
+    if (piece < pieces) {
+      const float4_t w = *reinterpret_cast<const float4_t*>(a.weight + piece * 4);
+      store4_from_f32(a.out, a.out_bf16, (size_t)row * H + piece * 4, (u[p] - mean) * inv * w);
+    }
+  }
+}
+
 template <int PIECES, bool IN_PARTS = false>
 __global__ void __launch_bounds__(1024) stream_norm_vec_kernel(const StreamNormArgs a) {
   __shared__ float scratch[16];
@@ -202,25 +227,113 @@ __global__ void __launch_bounds__(1024) stream_norm_vec_kernel(const StreamNormA
     }
     sum += (u[p][0] + u[p][1]) + (u[p][2] + u[p][3]);
   }
-  float mean = 0.f;
-  if (a.center) mean = block_sum(sum, scratch) / (float)H;
-  float sq = 0.f;
-#pragma unroll
-  for (int p = 0; p < PIECES; ++p) {
-    if (threadIdx.x + p * blockDim.x < pieces) {
-      const float4_t d = u[p] - mean;
-      sq += (d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]);
-    }
-  }
-  const float inv = 1.f / sqrtf(block_sum(sq, scratch) / (float)H + a.eps);
+  norm_of_pieces<PIECES>(a, u, sum, row, scratch);
+}
+
+// Streams that have not taken in what earlier sub-layers produced.  A pass over four float32 streams reads and writes them whole for a
+// term of an eighth of their bytes: 2,421 rows of 4 x 2,048 31.6 us at 5.1 TB/s.  So the norm's kernel may leave the streams as they
+// are and only read what they would be: the terms since they were last written (`earlier`, oldest first) are worked in again, in
+// registers and in the order and with the bits of one pass each, and every fourth term is written back with those before it
+// (STREAM_EARLIER: a further one saves a write of four rows less often and is read more often).  `base` [T, H]: rows that every stream
+// begins with, read in the streams' place until they are written for the first time (the embeddings, once and not once a stream).
+// The same rows by themselves, us: reading alone with 1, 2, 3 terms 18 / 20 / 22 (from `base` 8 / 10 / 12), the writing one 36 (27); within
+// a step, whose products take the cache between two norms, sixteen sub-layers 504 -> 446, the embeddings 28 -> 9, the step 4,487 -> 4,290.
+#define STREAM_EARLIER 3
+struct StreamTerms {
+  const void* term0;
+  const void* term1;
+  const float* mix;
+  const float* out_w;
+  float scale0, scale1;
+  int term0_bf16, term1_bf16, num_terms, unused;
+};
+struct StreamBehindArgs {
+  StreamNormArgs now;
+  StreamTerms earlier[STREAM_EARLIER];
+  int count;          // of them
+  int settle;         // the streams are written
+  const float* base;  // nullptr: the streams
+};
+
+// (the streams' weights are the same for every lane: read as constants, into scalar registers)
+typedef const __attribute__((address_space(4))) float* stream_weights_t;
+
+template <int PIECES, int S>
+__global__ void __launch_bounds__(1024) stream_norm_behind_kernel(const StreamBehindArgs args) {
+  const StreamNormArgs& a = args.now;
+  __shared__ float scratch[16];
+  const int H = a.hidden, pieces = H / 4;
+  const int row = blockIdx.x;
+  const size_t src = a.rows ? (size_t)a.rows[row] : (size_t)row;
+  float* res = a.residual + src * (size_t)S * H;
+  const bool update = a.num_terms > 0;
+  const bool write_back = args.settle && update && a.rows == nullptr;
+  const stream_weights_t in_w = (stream_weights_t)(uintptr_t)a.in_w;
+  float4_t u[PIECES];
+  float sum = 0.f;
 #pragma unroll
   for (int p = 0; p < PIECES; ++p) {
     const int piece = threadIdx.x + p * blockDim.x;
-    if (piece < pieces) {
-      const float4_t w = *reinterpret_cast<const float4_t*>(a.weight + piece * 4);
-      store4_from_f32(a.out, a.out_bf16, (size_t)row * H + piece * 4, (u[p] - mean) * inv * w);
+    u[p] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (piece >= pieces) continue;
+    const int i = piece * 4;
+    float4_t x[S], terms[STREAM_EARLIER + 1];
+    if (args.base != nullptr) {
+      x[0] = *reinterpret_cast<const float4_t*>(args.base + src * H + i);
+#pragma unroll
+      for (int s = 1; s < S; ++s) x[s] = x[0];
+    } else {
+#pragma unroll
+      for (int s = 0; s < S; ++s) x[s] = *reinterpret_cast<const float4_t*>(res + (size_t)s * H + i);
     }
+    auto term_of = [&](const void* term0, int term0_bf16, float scale0, const void* term1, int term1_bf16, float scale1, int num_terms, int parts) {
+      float4_t y = load4_as_f32(term0, term0_bf16, src * H + i);
+      for (int q = 1; q < parts; ++q) y += *reinterpret_cast<const float4_t*>((const float*)term0 + q * a.part_stride + src * H + i);
+      y *= scale0;
+      if (num_terms > 1) y += scale1 * load4_as_f32(term1, term1_bf16, src * H + i);
+      return y;
+    };
+#pragma unroll
+    for (int l = 0; l < STREAM_EARLIER; ++l) {
+      const StreamTerms& e = args.earlier[l];
+      if (l < args.count) terms[l] = term_of(e.term0, e.term0_bf16, e.scale0, e.term1, e.term1_bf16, e.scale1, e.num_terms, 1);
+    }
+    if (update) terms[STREAM_EARLIER] = term_of(a.term0, a.term0_bf16, a.scale0, a.term1, a.term1_bf16, a.scale1, a.num_terms, a.parts);
+    auto work_in = [&](const float* mix_of, const float* out_of, const float4_t y) {
+      const stream_weights_t mix = (stream_weights_t)(uintptr_t)mix_of, out_w = (stream_weights_t)(uintptr_t)out_of;
+      float4_t n[S];
+#pragma unroll
+      for (int t = 0; t < S; ++t) {
+        n[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < S; ++s) n[t] += (mix_of ? mix[s * S + t] : (s == t ? 1.f : 0.f)) * x[s];
+        n[t] += (out_of ? out_w[t] : 1.f) * y;
+      }
+#pragma unroll
+      for (int t = 0; t < S; ++t) x[t] = n[t];
+    };
+#pragma unroll
+    for (int l = 0; l < STREAM_EARLIER; ++l)
+      if (l < args.count) work_in(args.earlier[l].mix, args.earlier[l].out_w, terms[l]);
+    if (update) work_in(a.mix, a.out_w, terms[STREAM_EARLIER]);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      if (write_back) *reinterpret_cast<float4_t*>(res + (size_t)s * H + i) = x[s];
+      u[p] += (a.in_w ? in_w[s] : 1.f) * x[s];
+    }
+    sum += (u[p][0] + u[p][1]) + (u[p][2] + u[p][3]);
   }
+  norm_of_pieces<PIECES>(a, u, sum, row, scratch);
+}
+
+template <int S>
+static void stream_norm_behind_launch(const StreamBehindArgs& a, int count, hipStream_t stream) {
+  int lanes = (a.now.hidden / 4 + 63) / 64 * 64;
+  if (lanes > 1024) lanes = 1024;
+  const int per_lane = (a.now.hidden / 4 + lanes - 1) / lanes;
+  if (per_lane == 1) stream_norm_behind_kernel<1, S><<<count, lanes, 0, stream>>>(a);
+  else if (per_lane == 2) stream_norm_behind_kernel<2, S><<<count, lanes, 0, stream>>>(a);
+  else stream_norm_behind_kernel<4, S><<<count, lanes, 0, stream>>>(a);
 }
 
 // term0_parts > 1: term0 holds so many float32 partial sums [term0_parts, tokens, hidden], part_stride = tokens * hidden.
@@ -249,6 +362,31 @@ extern "C" int velox_stream_norm(float* residual, const void* term0, int term0_d
     VELOX_RETURN_LAUNCH_STATUS();
   }
   stream_norm_kernel<<<count, 256, (size_t)hidden * sizeof(float), stream>>>(a);
+  VELOX_RETURN_LAUNCH_STATUS();
+}
+
+// velox_stream_norm behind `count_earlier` terms that the streams have not taken in, and `base` (see stream_norm_behind_kernel).  Rows of a
+// multiple of four channels on 16-byte boundaries, up to 4 streams (the caller checks).  settle == 0: the streams stay as they are.
+extern "C" int velox_stream_norm_behind(float* residual, const void* term0, int term0_dtype, int term0_parts, long long part_stride, float scale0, const void* term1, int term1_dtype, float scale1,
+                                        int num_terms, const float* mix, const float* out_w, const float* in_w, const float* weight, const int* rows,
+                                        void* out, int out_dtype, int count, int hidden, int streams, int center, float eps, const StreamTerms* earlier, int count_earlier,
+                                        int settle, const float* base, hipStream_t stream) {
+  if (count <= 0) return 0;
+  if (streams < 1 || streams > 4 || hidden < 4 || hidden > 16384 || hidden % 4 != 0 || num_terms < 0 || num_terms > 2 || term0_parts < 1 || term0_parts > STREAM_PARTS ||
+      (term0_parts > 1 && term0_dtype != VELOX_F32) || count_earlier < 0 || count_earlier > STREAM_EARLIER || (num_terms == 0 && count_earlier > 0) || (settle != 0 && num_terms == 0))
+    return (int)hipErrorInvalidValue;
+  StreamBehindArgs a{{residual, term0, term1, term0_dtype == VELOX_BF16, term1_dtype == VELOX_BF16, num_terms, term0_parts, (size_t)part_stride, scale0, scale1, mix, out_w, in_w, weight,
+                      rows, out, out_dtype == VELOX_BF16, hidden, streams, center, eps}, {}, count_earlier, settle, base};
+  uintptr_t addresses = (uintptr_t)residual | (uintptr_t)weight | (uintptr_t)out | (uintptr_t)term0 | (uintptr_t)term1 | (uintptr_t)base;
+  for (int l = 0; l < count_earlier; ++l) {
+    a.earlier[l] = earlier[l];
+    addresses |= (uintptr_t)earlier[l].term0 | (uintptr_t)earlier[l].term1;
+  }
+  if (addresses % 16 != 0) return (int)hipErrorInvalidValue;
+  if (streams == 1) stream_norm_behind_launch<1>(a, count, stream);
+  else if (streams == 2) stream_norm_behind_launch<2>(a, count, stream);
+  else if (streams == 3) stream_norm_behind_launch<3>(a, count, stream);
+  else stream_norm_behind_launch<4>(a, count, stream);
   VELOX_RETURN_LAUNCH_STATUS();
 }
 

@@ -33,6 +33,13 @@ _I = ctypes.c_int
 _F = ctypes.c_float
 
 
+class _StreamTerms(ctypes.Structure):
+    """``StreamTerms`` in recurrent.hip."""
+
+    _fields_ = [("term0", _P), ("term1", _P), ("mix", _P), ("out_w", _P), ("scale0", ctypes.c_float), ("scale1", ctypes.c_float),
+                ("term0_bf16", ctypes.c_int), ("term1_bf16", ctypes.c_int), ("num_terms", ctypes.c_int), ("unused", ctypes.c_int)]
+
+
 class KernelError(RuntimeError):
     pass
 
@@ -219,6 +226,8 @@ class HipOps:
         c.velox_activation.argtypes = [_P, _P, ctypes.c_longlong, _I, _I, _P]
         for fn in (c.velox_embed_bigram, c.velox_add_dynamic_tanh, c.velox_scale, c.velox_activation):
             fn.restype = _I
+        c.velox_stream_norm_behind.argtypes = [*c.velox_stream_norm.argtypes[:-1], ctypes.POINTER(_StreamTerms), _I, _I, _P, _P]
+        c.velox_stream_norm_behind.restype = _I
         for fn in (c.velox_stream_norm, c.velox_embed_copies, c.velox_gated_act_mul, c.velox_short_conv, c.velox_rotate_pad_write, c.velox_recurrence_prepare,
                    c.velox_linear_scan, c.velox_linear_scan_lanes, c.velox_gated_head_norm):
             fn.restype = _I
@@ -1198,14 +1207,28 @@ class HipOps:
     # -- residual streams, short convolution, linear recurrences ------------------------------------
     MAX_STREAMS = 8
     MAX_STREAM_PARTS = 8  # partial sums that a term may come in
+    MAX_UNWRITTEN_STREAMS = 4
+    MAX_STREAMS_BEHIND = 3  # updates that the streams may be behind when a norm reads them
     MAX_STREAM_WIDTH = 16384
     MAX_CONV_TAPS = 8
 
-    def stream_norm(self, residual, terms, scales, mix, out_weights, in_weights, weight, eps, streams, center, out_dtype, rows=None):
+    STREAMS_WAIT_FROM_BYTES = 4 << 20  # of streams: below that a pass over them is a kernel's own beginning and end (128 rows of 4 x 2,048)
+
+    def streams_may_wait(self, residual, terms, weight, streams: int, held: int) -> bool:
+        """Whether ``stream_norm`` should leave the streams unwritten (``settle=False``) with ``held`` updates unwritten already."""
+        return (held < self.MAX_STREAMS_BEHIND and streams <= self.MAX_UNWRITTEN_STREAMS and residual.numel() * 4 >= self.STREAMS_WAIT_FROM_BYTES and residual.shape[1] % 4 == 0
+                and terms[0].dim() == 2 and terms[0].shape[1] % 4 == 0 and all(t.data_ptr() % 16 == 0 for t in (residual, weight, *terms)))
+
+    def streams_may_begin_unwritten(self, tokens: int, streams: int, hidden: int) -> bool:
+        return hidden % 4 == 0 and tokens * streams * hidden * 4 >= self.STREAMS_WAIT_FROM_BYTES and streams <= self.MAX_UNWRITTEN_STREAMS and hidden <= self.MAX_STREAM_WIDTH
+
+    def stream_norm(self, residual, terms, scales, mix, out_weights, in_weights, weight, eps, streams, center, out_dtype, rows=None, earlier=(), base=None, settle=True):
         """``residual`` float32 ``[T, streams * H]``.  With ``terms`` (one or two ``[T, H]`` tensors, the first also as float32 partial sums ``[S, T, H]``, ``y = sum_i scales[i] terms[i]``):
         ``x_t <- sum_s mix[s, t] x_s + out_weights[t] y`` for all streams at once (``mix`` None: the identity, ``out_weights``
         None: ones), in place unless ``rows`` picks rows.  Returns ``norm(sum_s in_weights[s] x_s) * weight`` in
-        ``out_dtype``, for all rows or for ``rows``; ``center``: a layer norm without bias, else an RMS norm."""
+        ``out_dtype``, for all rows or for ``rows``; ``center``: a layer norm without bias, else an RMS norm.
+        ``earlier``: up to ``MAX_STREAMS_BEHIND`` updates ``(terms, scales, mix, out_weights)`` that are worked in before it, oldest first, ``base`` float32
+        ``[T, H]``: what every stream is taken to be before them, in place of ``residual``'s rows; ``settle=False``: ``residual`` stays as it is (rows of a multiple of four channels)."""
         self._check("residual", residual, torch.float32)
         if residual.dim() != 2 or streams < 1 or residual.shape[1] % streams != 0:
             raise KernelError(f"stream_norm: residual must be [T, streams * H], got {tuple(residual.shape)} for {streams} streams")
@@ -1231,9 +1254,37 @@ class HipOps:
             self._check("rows", rows, torch.int32)
         count = tokens if rows is None else rows.shape[0]
         out = torch.empty((count, hidden), dtype=out_dtype, device=self.device)
+        unwritten = bool(earlier) or base is not None or not settle
+        if unwritten and (hidden % 4 != 0 or streams > self.MAX_UNWRITTEN_STREAMS):
+            raise KernelError(f"stream_norm: {streams} streams of {hidden} channels cannot stay unwritten (at most {self.MAX_UNWRITTEN_STREAMS}, of a multiple of four)")
+        if unwritten:  # (16-byte accesses alone; what is held back was checked when it was)
+            terms = tuple(t if t.data_ptr() % 16 == 0 else t.clone() for t in terms)
+            weight = weight if weight.data_ptr() % 16 == 0 else weight.clone()
         t0 = terms[0] if len(terms) > 0 else None
         t1 = terms[1] if len(terms) > 1 else None
-        status = self._core.velox_stream_norm(
+        if unwritten:
+            if len(earlier) > self.MAX_STREAMS_BEHIND or (not terms and earlier):
+                raise KernelError(f"stream_norm: {len(earlier)} earlier updates, at most {self.MAX_STREAMS_BEHIND} and in front of a term")
+            if base is not None:
+                self._check("base", base, torch.float32, (tokens, hidden), align=16)
+            held = (_StreamTerms * self.MAX_STREAMS_BEHIND)()
+            for entry, (e_terms, e_scales, e_mix, e_out) in zip(held, earlier):
+                if not 1 <= len(e_terms) <= 2 or len(e_terms) != len(e_scales):
+                    raise KernelError("stream_norm: one or two terms, each with its scale")
+                for t in e_terms:
+                    self._check("earlier term", t, None, (tokens, hidden), align=16)
+                for name, t, shape in (("mix", e_mix, (streams, streams)), ("out_weights", e_out, (streams,))):
+                    if t is not None:
+                        self._check(name, t, torch.float32, shape)
+                second = e_terms[1] if len(e_terms) > 1 else None
+                entry.term0, entry.term0_bf16, entry.scale0 = e_terms[0].data_ptr(), e_terms[0].dtype == torch.bfloat16, float(e_scales[0])
+                entry.term1, entry.term1_bf16, entry.scale1 = (second.data_ptr(), second.dtype == torch.bfloat16, float(e_scales[1])) if second is not None else (None, 0, 0.0)
+                entry.mix, entry.out_w, entry.num_terms = e_mix.data_ptr() if e_mix is not None else None, e_out.data_ptr() if e_out is not None else None, len(e_terms)
+        status = self._core.velox_stream_norm_behind(
+            _ptr(residual), _ptr(t0), _code(t0.dtype) if t0 is not None else 0, parts, tokens * hidden, float(scales[0]) if t0 is not None else 0.0,
+            _ptr(t1), _code(t1.dtype) if t1 is not None else 0, float(scales[1]) if t1 is not None else 0.0, len(terms),
+            _ptr(mix), _ptr(out_weights), _ptr(in_weights), _ptr(weight), _ptr(rows), _ptr(out), _code(out_dtype), count, hidden, int(streams),
+            int(bool(center)), float(eps), held, len(earlier), int(bool(settle) and len(terms) > 0), _ptr(base), self._stream()) if unwritten else self._core.velox_stream_norm(
             _ptr(residual), _ptr(t0), _code(t0.dtype) if t0 is not None else 0, parts, tokens * hidden, float(scales[0]) if t0 is not None else 0.0,
             _ptr(t1), _code(t1.dtype) if t1 is not None else 0, float(scales[1]) if t1 is not None else 0.0, len(terms),
             _ptr(mix), _ptr(out_weights), _ptr(in_weights), _ptr(weight), _ptr(rows), _ptr(out), _code(out_dtype), count, hidden, int(streams),

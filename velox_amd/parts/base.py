@@ -212,11 +212,22 @@ class StreamUpdate:
     """A sub-layer's output that the residual STREAMS have not taken in yet: ``x_t <- sum_s mix[s, t] x_s + out[t] * y``
     for all streams at once.  ``y`` is ``[T, H]`` or a ``ScaledSum``; ``mix`` float32 ``[S, S]`` indexed [from, to],
     ``out`` float32 ``[S]`` (None: the identity and ones, which is the plain residual sum).  The norm that reads the
-    streams next applies it inside its own kernel."""
+    streams next applies it inside its own kernel.  ``behind``: what the streams have not taken in before it."""
 
     y: object
     mix: Optional[torch.Tensor] = None
     out: Optional[torch.Tensor] = None
+    behind: "UnwrittenStreams" = None
+
+
+@dataclass(frozen=True)
+class UnwrittenStreams:
+    """What has to be worked into the residual streams before they are what they should be: ``updates`` (``StreamUpdate`` of whole
+    terms, oldest first), after ``base`` float32 ``[T, H]``, the row that every stream begins with, if they were never written.
+    Norms leave streams unwritten only behind one of these: the model begins with it if all that reads the streams takes it."""
+
+    updates: Tuple[StreamUpdate, ...] = ()
+    base: Optional[torch.Tensor] = None
 
 
 @dataclass

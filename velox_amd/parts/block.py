@@ -28,7 +28,7 @@ from typing import Optional, Tuple
 import torch
 
 from .base import (
-    Block, FeedForward, Mixer, Norm, NormedDelta, NormedSum, OutputNormSink, Part, PartSpec, ResidualCopy, ResidualSink, StreamUpdate, SumOf, make_part, register_arrangement,
+    Block, FeedForward, Mixer, Norm, NormedDelta, NormedSum, OutputNormSink, Part, PartSpec, ResidualCopy, ResidualSink, StreamUpdate, SumOf, UnwrittenStreams, make_part, register_arrangement,
 )
 
 
@@ -204,7 +204,8 @@ class HyperConnectionBlock(Block):
 
     The residual is float32 ``[T, S * H]``.  A sub-layer's output is not worked into the streams by a pass of its own:
     it is handed on as a ``StreamUpdate`` and the next norm's kernel (``StreamNorm``) applies it before it reads the
-    streams, as the plain residual sum is folded into the next norm for the other arrangements.  The block's own tensors
+    streams, as the plain residual sum is folded into the next norm for the other arrangements.  In a pass that begins with
+    ``UnwrittenStreams`` that kernel may also leave the streams unwritten (the update carries on what they lack).  The block's own tensors
     are ``<prefix>hc1.{in,out,mix}`` and ``<prefix>hc2.{in,out,mix}`` (``names`` replaces the two prefixes)."""
 
     def __init__(self, prefix: str, mixer: Mixer, feed_forward: FeedForward, mixer_norm: Norm, ff_norm: Norm, streams: int = 1,
@@ -248,14 +249,20 @@ class HyperConnectionBlock(Block):
     def input_norm(self) -> Optional[Norm]:
         return self.mixer_norm
 
+    @staticmethod
+    def _read(norm, residual, pending, in_weights, ctx):
+        if isinstance(pending, UnwrittenStreams) or getattr(pending, "behind", None) is not None:
+            return norm.read_streams(residual, pending, in_weights, ctx)
+        return norm.forward_streams(residual, pending, in_weights, ctx), None
+
     def forward(self, residual: torch.Tensor, pending, ctx, cache, owns_cache: bool, next_norm: Optional[Norm] = None):
-        normed = self.mixer_norm.forward_streams(residual, pending, self.in1, ctx)
+        normed, left = self._read(self.mixer_norm, residual, pending, self.in1, ctx)
         mixed = self.mixer.forward(normed, ctx, cache, owns_cache)
-        update = StreamUpdate(mixed, self.mix1, self.out1)
+        update = StreamUpdate(mixed, self.mix1, self.out1, left)
         if not self.has_feed_forward:
             return update
-        normed = self.ff_norm.forward_streams(residual, update, self.in2, ctx)
-        return StreamUpdate(self.feed_forward.forward(normed, ctx), self.mix2, self.out2)
+        normed, left = self._read(self.ff_norm, residual, update, self.in2, ctx)
+        return StreamUpdate(self.feed_forward.forward(normed, ctx), self.mix2, self.out2, left)
 
 
 register_arrangement("hyper_connection", HyperConnectionBlock)

@@ -21,7 +21,8 @@ from typing import Dict, List, Optional, Tuple
 import torch
 
 from . import block as _block  # noqa: F401  (registers the built-in arrangement)
-from .base import Embedding, OutputHead, Param, Part, PartSpec, PassInput, StateNeed, make_part, register_part, single
+from .base import Embedding, OutputHead, Param, Part, PartSpec, PassInput, StateNeed, UnwrittenStreams, make_part, register_part, single
+from .norms import StreamNorm
 
 
 @dataclass(frozen=True)
@@ -237,6 +238,8 @@ class DecoderModel(Part):
                               tied_to=spec.embed_name if spec.tie_head else None, **head.kwargs())
         self.pass_input = make_part("pass_input", spec.pass_input.kind, hidden_size=spec.hidden_size, **spec.pass_input.kwargs()) if spec.pass_input is not None else None
         self.schedule = list(spec.schedule)
+        readers = [n for block in self.blocks for n in ((block.mixer_norm, block.ff_norm) if type(block) is _block.HyperConnectionBlock else (None,))] + [self.final_norm]
+        self.streams_can_wait = self.pass_input is None and all(type(n) is StreamNorm for n in readers)  # (nothing reads the residual but these)
 
     # -- structure ----------------------------------------------------------------------
     def children(self) -> Tuple[Part, ...]:
@@ -311,8 +314,21 @@ class DecoderModel(Part):
 
     def forward(self, token_ids: torch.Tensor, ctx):
         """Runs every block; returns ``(residual float32 [T, H], pending [T, H])``."""
-        residual = self.begin(token_ids, ctx)
-        return residual, self.run_schedule(residual, None, ctx)
+        residual, pending = self.begin_unwritten(token_ids, ctx) or (self.begin(token_ids, ctx), None)
+        return residual, self.run_schedule(residual, pending, ctx)
+
+    def begin_unwritten(self, token_ids: torch.Tensor, ctx):
+        """Streams that are not written yet and the row that all of them begin with (``begin`` writes it once per stream); None where
+        the kernels gain nothing by it or something else reads the streams."""
+        streams, hidden = self.spec.residual_streams, self.spec.hidden_size
+        may_begin = getattr(ctx.ops, "streams_may_begin_unwritten", None)
+        if (streams == 1 or may_begin is None or not may_begin(token_ids.shape[0], streams, hidden) or self.embedding.cache_need() is not None
+                or not self.streams_can_wait):
+            return None
+        base = self.embedding.forward(token_ids, ctx)
+        if self.spec.embedding_position is not None:
+            base = self.positions[self.spec.embedding_position].on_embeddings(base, ctx)
+        return torch.empty((token_ids.shape[0], streams * hidden), dtype=torch.float32, device=base.device), UnwrittenStreams((), base)
 
     def logits(self, residual: torch.Tensor, pending, rows: torch.Tensor, ctx) -> torch.Tensor:
         """Final norm and output head on ``rows`` (int32 [R]) only: float32 [R, vocab]."""

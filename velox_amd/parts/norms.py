@@ -13,7 +13,7 @@ from typing import Dict, Optional
 
 import torch
 
-from .base import DeferredNorm, Norm, NormedDelta, NormedSum, Param, ReadyInput, ResidualCopy, ScaledSum, StreamUpdate, register_part, single
+from .base import DeferredNorm, Norm, NormedDelta, NormedSum, Param, ReadyInput, ResidualCopy, ScaledSum, StreamUpdate, UnwrittenStreams, register_part, single
 
 
 class RMSNorm(Norm):
@@ -85,23 +85,44 @@ class StreamNorm(Norm):
     def params(self) -> Dict[str, Param]:
         return {"weight": single(self.weight_name, (self.hidden_size,), role="vector", init="one_plus_normal")}
 
+    @staticmethod
+    def _terms(y):
+        if isinstance(y, ScaledSum):
+            return tuple(y.terms), tuple(float(s) for s in y.scales)
+        if y.dim() == 3 and y.shape[1] <= 64:
+            y = y.sum(0)  # (float32 partial sums of a product; those of more rows are added by the norm's kernel)
+        return (y,), (1.0,)
+
     def forward_streams(self, residual, update, in_weights, ctx, rows=None):
-        """``update``: a ``StreamUpdate``, a plain delta (tensor or ``ScaledSum``: every stream takes it as it is) or None."""
+        """``update``: a ``StreamUpdate``, a plain delta (tensor or ``ScaledSum``: every stream takes it as it is), ``UnwrittenStreams`` or None."""
+        return self._read(residual, update, in_weights, ctx, rows, False)[0]
+
+    def read_streams(self, residual, update, in_weights, ctx):
+        """``forward_streams`` behind ``UnwrittenStreams`` (alone or carried by an update), and what the streams have not taken in after it: where
+        that spares passes over them, the kernel reads what they would be and leaves them as they are."""
+        return self._read(residual, update, in_weights, ctx, None, True)
+
+    def _read(self, residual, update, in_weights, ctx, rows, may_wait):
         if isinstance(update, ResidualCopy):
             update = None
-        if update is not None and not isinstance(update, StreamUpdate):
+        behind = None
+        if isinstance(update, UnwrittenStreams):
+            behind, update = update, None
+        elif isinstance(update, StreamUpdate):
+            behind = update.behind
+        elif update is not None:
             update = StreamUpdate(update)
-        terms, scales = (), ()
-        if update is not None:
-            y = update.y
-            if isinstance(y, ScaledSum):
-                terms, scales = tuple(y.terms), tuple(float(s) for s in y.scales)
-            else:
-                if y.dim() == 3 and y.shape[1] <= 64:
-                    y = y.sum(0)  # (float32 partial sums of a product; those of more rows are added by the norm's kernel)
-                terms, scales = (y,), (1.0,)
-        return ctx.ops.stream_norm(residual, terms, scales, update.mix if update is not None else None, update.out if update is not None else None,
-                                   in_weights, self.weight, self.eps, self.streams, self.center, ctx.dtype, rows=rows)
+        terms, scales = self._terms(update.y) if update is not None else ((), ())
+        more, left = {}, behind if update is None else UnwrittenStreams()
+        if behind is not None:
+            more = dict(earlier=tuple((*self._terms(u.y), u.mix, u.out) for u in behind.updates), base=behind.base)
+        held = behind.updates if behind is not None else ()
+        if may_wait and update is not None and getattr(ctx.ops, "streams_may_wait", None) is not None and ctx.ops.streams_may_wait(residual, terms, self.weight, self.streams, len(held)):
+            more["settle"] = False
+            left = UnwrittenStreams((*held, StreamUpdate(update.y, update.mix, update.out)), behind.base if behind is not None else None)
+        normed = ctx.ops.stream_norm(residual, terms, scales, update.mix if update is not None else None, update.out if update is not None else None,
+                                     in_weights, self.weight, self.eps, self.streams, self.center, ctx.dtype, rows=rows, **more)
+        return normed, left
 
     def forward(self, residual, delta, ctx, rows=None):
         if isinstance(delta, DeferredNorm):
