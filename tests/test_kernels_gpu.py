@@ -931,6 +931,31 @@ def test_sampling_with_as_many_tokens_left_as_a_list_holds(ops, vocab, top_p, to
     assert torch.equal(ops.sample(logits, options, chunks=2), ops.sample(logits, options, chunks=1))
 
 
+@pytest.mark.parametrize("vocab, chunks", [(40000, 3), (152064, 4), (9001, 32)])
+@pytest.mark.parametrize("top_p, top_k", [(0.9, 0), (1.0, 900), (0.3, 0), (1.0, 15000)])
+def test_sampling_with_lists_and_open_tokens_beyond_their_room(ops, vocab, chunks, top_p, top_k):
+    """Rows with more listed tokens (6,144) and more kept ones (3,072) than LDS holds, rows of which only some chunks are listed, and, in rows
+    that are not listed, 1,023 to 1,025 and far more equal logits around the threshold: the tokens of the one-workgroup kernel, bit for bit."""
+    g = torch.Generator().manual_seed(9)
+    logits = torch.full((8, vocab), -30.0) - torch.rand((8, vocab), generator=g)
+    logits[0, torch.randperm(vocab, generator=g)[:vocab // 10]] = 4.2
+    spread = torch.randperm(vocab, generator=g)[:vocab // 10]
+    logits[1, spread] = 4.0 + 0.9 * torch.rand(len(spread), generator=g)
+    for r, equal in enumerate((1023, 1024, 1025, 16000, vocab), start=2):
+        if r < 6:
+            logits[r, :vocab // 2] = 3.6 + 0.3 * torch.rand(vocab // 2, generator=g)  # (the other half's chunks are listed)
+        logits[r, torch.randperm(vocab, generator=g)[:equal]] = 3.75
+    logits[7] = 1.0 + 0.2 * torch.rand(vocab, generator=g)
+    logits = logits.repeat_interleave(3, 0).cuda()
+    options = np.zeros((logits.shape[0], 6), dtype=np.int32)
+    options.view(np.float32)[:, 0], options.view(np.float32)[:, 1] = 1.0, top_p
+    options[:, 2], options[:, 3] = top_k if top_k < vocab else 0, np.arange(logits.shape[0])
+    options = torch.from_numpy(options).cuda()
+    whole = ops.sample(logits, options, chunks=1)
+    for _ in range(2):
+        assert torch.equal(ops.sample(logits, options, chunks=chunks), whole)
+
+
 def test_penalties_over_long_histories_and_a_large_vocabulary(ops, ref):
     vocab, rows, width = 152064, 4, 6000
     logits = rand((rows, vocab), torch.float32, 34, 2.0)

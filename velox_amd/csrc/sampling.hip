@@ -428,8 +428,10 @@ __device__ __forceinline__ void draw_token(int i, float x, uint32_t bits, float 
 // and eight logarithms a quad) would be worked out by whole waves for a lane or two.  The kept quads are therefore queued
 // in LDS first and taken up 64 at a time (48 rows of 152,064, top-p 0.9: the pass with the digit before it 19.7 us
 // without the queue, 13.4 with it).
+// left_out(i, logit, key): a token at or above the threshold that is not drawn from.
+template <typename F>
 __device__ __forceinline__ Best draw_in_quads(const float* __restrict__ row, int vocab, int q_lo, int q_hi, const RowOptions& o, float mx, uint32_t threshold,
-                                              DrawQueue& queue) {
+                                              DrawQueue& queue, F left_out) {
   Best best{-INFINITY, 0x7fffffff};
   const bool aligned = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
   const bool filter = o.filter;
@@ -443,7 +445,7 @@ __device__ __forceinline__ Best draw_in_quads(const float* __restrict__ row, int
       const int i = 4 * q + e;
       if (i >= vocab) break;
       const float x = v[e] * inv_t;
-      if (filter && sort_key(x) < threshold) continue;
+      if (filter && (sort_key(x) < threshold || left_out(i, v[e], sort_key(x)))) continue;
       draw_token(i, x, bits[e], mx, best);
     }
   };
@@ -536,7 +538,7 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_kernel(const float* __r
     threshold = prefix;
   }
 
-  Best best = draw_in_quads(row, vocab, 0, quads, o, mx, threshold, shared.queue);
+  Best best = draw_in_quads(row, vocab, 0, quads, o, mx, threshold, shared.queue, [](int, float, uint32_t) { return false; });
   best = block_best(best, best_scratch);
   if (tid == 0) out[blockIdx.x] = best.index;
 }
@@ -547,34 +549,40 @@ extern "C" int velox_sample(const float* logits, const int* options, int* out, i
   VELOX_RETURN_LAUNCH_STATUS();
 }
 
-// ---- a row cut into chunks: one kernel per pass ---------------------------------------------------------------------
-// What the chunks of a row share, in global memory: each chunk's maximum and best pair, the tables of the three digits
-// (cleared by the first kernel, added to with integer atomics by the kernels of the digits) and what the search has
-// found so far.  Every workgroup of a kernel reads what the kernel before left and works out the digit before its own
-// once more for itself (a scan over 2,048 entries); the workgroup of chunk 0 writes it down for the kernels after.
+// ---- a row cut into chunks ------------------------------------------------------------------------------------------
+// What the chunks of a row share, in global memory: each chunk's maximum and best pair, the tables of the first two digits
+// (cleared by the first kernel, added to with integer atomics) and what the search has found so far.  A row with a filter goes
+// through four kernels: its maximum; the tables of the first digit; the tokens that this digit does not rule out, as a list per
+// chunk (of a row with top-p 0.9 or top-k 50 about one token in a hundred); and from the lists, in one workgroup, the other digits,
+// the draw and the token.  What bounds a pass is its few dependent steps (a launch, two trips to memory, a scan over the table), not
+// the row: with a kernel per digit, one for the draw and one to merge the chunks, 48 rows of 152,064 took 55 us; see
+// sample_finish_kernel.  Where a wave finds more than LIST_ENTRIES tokens the chunk is not listed: it adds its tokens to the tables
+// of the second digit instead, and the row's chunks are drawn from by a workgroup each.
 struct RowSearch {
-  unsigned long long mass_limit;  // top_p of the row's whole probability (after level 0)
-  unsigned long long above_mass[2];
-  unsigned int above_count[2];
-  unsigned int prefix[2];  // the digits found after level 0 and after level 1, in place
+  unsigned long long mass_limit;  // top_p of the row's whole probability
+  unsigned long long above_mass;  // what lies above the first digit's tokens
+  unsigned int above_count;
+  unsigned int prefix;            // the first digit, in place
+  int unlisted;                   // some chunk is not listed
+  unsigned int drawn;             // chunks of such a row that have drawn
+  unsigned int open;              // its open tokens: see sample_finish_kernel
+  unsigned int unused;
 };
+#define OPEN_TOKENS 1024
 
-// The tokens that the first digit does not rule out (of a row with top-p 0.9 or top-k 50 about one in a hundred), which each
-// wave of the kernel of the second digit leaves for the kernels behind it: those need not walk the row again (48 rows of 152,064:
-// the kernels of the second and third digit and the draw 33.7 -> 28.8 us).  A wave that finds more than LIST_ENTRIES says so, and the chunk is walked as before.  Chunks of fewer than
-// LIST_QUADS quads get no lists: they would be larger than the logits.
 #define LIST_ENTRIES 256
-#define LIST_QUADS 2048
 struct Listed { float logit; int index; };
 
 struct ChunkedScratch {
-  Listed* lists;               // [rows, chunks, waves, LIST_ENTRIES], nullptr: none
-  int* list_lengths;           // [rows, chunks, waves]
+  Listed* lists;               // [rows, chunks, list_room]
+  int* list_lengths;           // [rows, chunks]; -1: not listed
+  Listed* open;                // [rows, OPEN_TOKENS]
   float* chunk_max;            // [rows, chunks]
   Best* chunk_best;            // [rows, chunks]
   RowSearch* search;           // [rows]
-  unsigned int* counts;        // [rows, 3, SELECT_BINS]
-  unsigned long long* masses;  // [rows, 3, SELECT_BINS]
+  unsigned int* counts;        // [rows, 2, SELECT_BINS]
+  unsigned long long* masses;  // [rows, 2, SELECT_BINS]
+  int list_room;
 };
 
 static size_t chunked_scratch_layout(int rows, int vocab, int chunks, void* base, ChunkedScratch* scratch) {
@@ -583,23 +591,24 @@ static size_t chunked_scratch_layout(int rows, int vocab, int chunks, void* base
   char* p = (char*)base;
   auto take = [&](size_t bytes) { char* here = p + at; at += up(bytes); return here; };
   ChunkedScratch s;
-  s.masses = (unsigned long long*)take((size_t)rows * 3 * SELECT_BINS * sizeof(unsigned long long));
-  s.counts = (unsigned int*)take((size_t)rows * 3 * SELECT_BINS * sizeof(unsigned int));
+  s.masses = (unsigned long long*)take((size_t)rows * 2 * SELECT_BINS * sizeof(unsigned long long));
+  s.counts = (unsigned int*)take((size_t)rows * 2 * SELECT_BINS * sizeof(unsigned int));
   s.search = (RowSearch*)take((size_t)rows * sizeof(RowSearch));
   s.chunk_best = (Best*)take((size_t)rows * chunks * sizeof(Best));
   s.chunk_max = (float*)take((size_t)rows * chunks * sizeof(float));
-  const size_t waves = (size_t)rows * chunks * (SAMPLE_THREADS / 64);
-  const bool listed = ((vocab + 3) / 4 + chunks - 1) / chunks >= LIST_QUADS;
-  s.lists = listed ? (Listed*)take(waves * LIST_ENTRIES * sizeof(Listed)) : nullptr;
-  s.list_lengths = listed ? (int*)take(waves * sizeof(int)) : nullptr;
+  const int chunk_tokens = 4 * (((vocab + 3) / 4 + chunks - 1) / chunks);
+  s.list_room = chunk_tokens < LIST_ENTRIES * (SAMPLE_THREADS / 64) ? chunk_tokens : LIST_ENTRIES * (SAMPLE_THREADS / 64);
+  s.lists = (Listed*)take((size_t)rows * chunks * s.list_room * sizeof(Listed));
+  s.list_lengths = (int*)take((size_t)rows * chunks * sizeof(int));
+  s.open = (Listed*)take((size_t)rows * OPEN_TOKENS * sizeof(Listed));
   if (scratch != nullptr) *scratch = s;
   return at;
 }
 
-__device__ __forceinline__ void chunk_quads(int vocab, int& q_lo, int& q_hi) {
+__device__ __forceinline__ void chunk_quads(int vocab, int chunk, int& q_lo, int& q_hi) {
   const int quads = (vocab + 3) / 4;
   const int per_chunk = (quads + gridDim.y - 1) / gridDim.y;
-  q_lo = blockIdx.y * per_chunk;
+  q_lo = chunk * per_chunk;
   q_hi = q_lo + per_chunk < quads ? q_lo + per_chunk : quads;
   if (q_lo > quads) q_lo = quads;
 }
@@ -613,7 +622,7 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_max_kernel(const 
   const float* row = logits + (size_t)r * vocab;
   const RowOptions o = read_options(options + (size_t)r * 6, vocab);
   int q_lo, q_hi;
-  chunk_quads(vocab, q_lo, q_hi);
+  chunk_quads(vocab, c, q_lo, q_hi);
   if (o.temperature == 0.f) {
     Best best{-INFINITY, 0x7fffffff};
     for_each_in_quads(row, vocab, q_lo, q_hi, [&](int i, float v) { best = better(best, Best{v, i}); });
@@ -622,7 +631,8 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_max_kernel(const 
     return;
   }
   if (o.filter) {
-    const int entries = 3 * SELECT_BINS;
+    if (c == 0 && threadIdx.x == 0) s.search[r].unlisted = 0, s.search[r].drawn = 0u, s.search[r].open = 0u;
+    const int entries = 2 * SELECT_BINS;
     for (int e = c * blockDim.x + threadIdx.x; e < entries; e += chunks * blockDim.x) {
       if (o.top_k > 0) s.counts[(size_t)r * entries + e] = 0u;
       if (o.use_mass) s.masses[(size_t)r * entries + e] = 0ull;
@@ -636,24 +646,31 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_max_kernel(const 
 
 __device__ __forceinline__ float row_max_of_chunks(const float* __restrict__ chunk_max, int chunks) {
   float mx = -INFINITY;
-  for (int c = 0; c < chunks; ++c) mx = fmaxf(mx, chunk_max[c]);
-  return mx;
+  for (int c = threadIdx.x & 63; c < chunks; c += 64) mx = fmaxf(mx, chunk_max[c]);
+  return wave_max(mx);
 }
 
-// The digit of `level` from the row's finished tables (global), given what was found before.
-__device__ __forceinline__ uint32_t finished_digit(const ChunkedScratch& s, int r, int level, const RowOptions& o, uint32_t prefix_before,
-                                                   unsigned long long& mass_limit, Above& above, SelectScratch& select) {
+// The digit of `level`, in place behind `prefix`, from table_of(bin, count, mass).
+template <typename F>
+__device__ __forceinline__ uint32_t digit_of_table(int level, const RowOptions& o, uint32_t prefix, unsigned long long& mass_limit, Above& above, SelectScratch& select,
+                                                   F table_of) {
   const int bins = level_bins(level), per_thread = bins / SAMPLE_THREADS;
-  const size_t base = ((size_t)r * 3 + level) * SELECT_BINS;
   unsigned int c[2] = {0u, 0u};
   unsigned long long m[2] = {0ull, 0ull};
-  for (int j = 0; j < per_thread; ++j) {
-    const int bin = bins - 1 - (int)threadIdx.x * per_thread - j;
-    if (o.top_k > 0) c[j] = s.counts[base + bin];
-    if (o.use_mass) m[j] = s.masses[base + bin];
+  for (int j = 0; j < per_thread; ++j) table_of(bins - 1 - (int)threadIdx.x * per_thread - j, c[j], m[j]);
+  return prefix | ((uint32_t)select_digit(c, m, per_thread, bins, o.top_k, o.use_mass, level == 0, o.top_p, mass_limit, above, select) << level_shift(level));
+}
+
+// adds a workgroup's tables of `level` (0 or 1) to the row's
+template <int C> __device__ __forceinline__ void add_to_row_tables(const ChunkedScratch& s, int r, int level, const LevelTables<C>& tables, const RowOptions& o) {
+  const size_t base = ((size_t)r * 2 + level) * SELECT_BINS;
+  for (int b = threadIdx.x; b < level_bins(level); b += blockDim.x) {
+    unsigned int count;
+    unsigned long long mass;
+    table_entry(tables, level, b, o, count, mass);
+    if (count != 0u) atomicAdd(&s.counts[base + b], count);
+    if (mass != 0ull) atomicAdd(&s.masses[base + b], mass);
   }
-  const int digit = select_digit(c, m, per_thread, bins, o.top_k, o.use_mass, level == 0, o.top_p, mass_limit, above, select);
-  return prefix_before | ((uint32_t)digit << level_shift(level));
 }
 
 // Lists this wave's tokens of quads [q_lo, q_hi) whose key is at least `floor`: up to LIST_ENTRIES of them in `mine` (LDS).  Returns how
@@ -688,156 +705,291 @@ __device__ __forceinline__ int list_tokens(const float* __restrict__ row, int vo
   return found;
 }
 
-// How many tokens the waves of a chunk have listed before each wave's own (`before`, LDS), all of them in before[waves]; -1: not all are listed.
-__device__ __forceinline__ int listed_tokens(const ChunkedScratch& s, int chunk, int* before) {
-  constexpr int WAVES = SAMPLE_THREADS / 64;
-  if (s.lists == nullptr) return -1;  // (the same for all workgroups)
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    int length = lane < WAVES ? s.list_lengths[(size_t)chunk * WAVES + lane] : 0;
-    const bool whole = __ballot(length > LIST_ENTRIES) == 0ull;
-    int upto = length;
-#pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-      const int other = __shfl_up(upto, offset, VELOX_WAVE);
-      if (lane >= offset) upto += other;
-    }
-    if (lane < WAVES) before[lane] = upto - length;
-    if (lane == WAVES) before[WAVES] = whole ? upto : -1;
-  }
-  __syncthreads();
-  return before[WAVES];
-}
-
-// f(index, logit) for the chunk's `total` listed tokens, dealt to the threads one after the other
-template <typename F> __device__ __forceinline__ void for_each_listed(const ChunkedScratch& s, int chunk, const int* before, int total, F f) {
-  constexpr int WAVES = SAMPLE_THREADS / 64;
-  for (int j = threadIdx.x; j < total; j += blockDim.x) {
-    int wave = 0;
-#pragma unroll
-    for (int w = 1; w < WAVES; ++w) wave += j >= before[w] ? 1 : 0;
-    const Listed token = s.lists[((size_t)chunk * WAVES + wave) * LIST_ENTRIES + (j - before[wave])];
-    f(token.index, token.logit);
-  }
-}
-
-// passes 2..4: the tables of digit LEVEL
-template <int LEVEL>
+// pass 2 of a row with a filter: the tables of the first digit
 __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_tables_kernel(const float* __restrict__ logits, const int* __restrict__ options,
                                                                              ChunkedScratch s, int vocab) {
-  __shared__ LevelTables<LEVEL == 0 ? TABLE_COPIES : 1> tables;
-  __shared__ SelectScratch select;
-  __shared__ Listed listed[LEVEL == 1 ? SAMPLE_THREADS / 64 : 1][LEVEL == 1 ? LIST_ENTRIES : 1];
-  __shared__ int before[SAMPLE_THREADS / 64 + 1], overflow;
+  __shared__ LevelTables<TABLE_COPIES> tables;
   const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
   const float* row = logits + (size_t)r * vocab;
   const RowOptions o = read_options(options + (size_t)r * 6, vocab);
   if (o.temperature == 0.f || !o.filter) return;
-  const int tid = threadIdx.x;
   int q_lo, q_hi;
-  chunk_quads(vocab, q_lo, q_hi);
-  clear_tables(tables, LEVEL, o);
-  if (tid == 0) overflow = 0;
-  const int total = LEVEL == 2 ? listed_tokens(s, r * chunks + c, before) : -1;
+  chunk_quads(vocab, c, q_lo, q_hi);
+  clear_tables(tables, 0, o);
   const float mx = row_max_of_chunks(s.chunk_max + r * chunks, chunks);
-  uint32_t prefix = 0u;
-  if (LEVEL >= 1) {
-    Above above{0u, 0ull};
-    unsigned long long mass_limit = 0ull;
-    if (LEVEL == 2) {
-      prefix = s.search[r].prefix[0];
-      above.count = s.search[r].above_count[0];
-      above.mass = s.search[r].above_mass[0];
-      mass_limit = s.search[r].mass_limit;
-    }
-    prefix = finished_digit(s, r, LEVEL - 1, o, prefix, mass_limit, above, select);
-    if (c == 0 && tid == 0) {
-      if (LEVEL == 1) s.search[r].mass_limit = mass_limit;
-      s.search[r].prefix[LEVEL - 1] = prefix;
-      s.search[r].above_count[LEVEL - 1] = above.count;
-      s.search[r].above_mass[LEVEL - 1] = above.mass;
-    }
-  }
   __syncthreads();
-  if (LEVEL == 1 && s.lists != nullptr) {
-    const int lane = tid & 63, wave = tid >> 6;
-    const int found = list_tokens(row, vocab, q_lo, q_hi, o, prefix, listed[wave]);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    const size_t list = ((size_t)r * chunks + c) * (SAMPLE_THREADS / 64) + wave;
-    if (lane == 0) s.list_lengths[list] = found;
-    for (int j = lane; j < min(found, LIST_ENTRIES); j += 64) s.lists[list * LIST_ENTRIES + j] = listed[wave][j];
-    if (lane == 0 && found > LIST_ENTRIES) overflow = 1;
-    __syncthreads();
-    if (overflow == 0) {
-      for (int j = lane; j < found; j += 64) {
-        const float x = listed[wave][j].logit * o.inv_t;
-        const uint32_t key = sort_key(x);
-        if ((key >> 21) == (prefix >> 21)) add_token(tables, (int)((key >> level_shift(1)) & (uint32_t)(level_bins(1) - 1)), x, o, mx);
-      }
-    } else {
-      add_to_tables(row, vocab, q_lo, q_hi, o, mx, LEVEL, prefix, tables);
-    }
-  } else if (LEVEL == 2 && total >= 0) {
-    for_each_listed(s, r * chunks + c, before, total, [&](int, float v) {
-      const float x = v * o.inv_t;
-      const uint32_t key = sort_key(x);
-      if ((key >> 10) == (prefix >> 10)) add_token(tables, (int)(key & (uint32_t)(level_bins(2) - 1)), x, o, mx);
-    });
-  } else {
-    add_to_tables(row, vocab, q_lo, q_hi, o, mx, LEVEL, prefix, tables);
-  }
+  add_to_tables(row, vocab, q_lo, q_hi, o, mx, 0, 0u, tables);
   __syncthreads();
-  const size_t base = ((size_t)r * 3 + LEVEL) * SELECT_BINS;
-  for (int b = tid; b < level_bins(LEVEL); b += blockDim.x) {
-    unsigned int count;
-    unsigned long long mass;
-    table_entry(tables, LEVEL, b, o, count, mass);
-    if (count != 0u) atomicAdd(&s.counts[base + b], count);
-    if (mass != 0ull) atomicAdd(&s.masses[base + b], mass);
-  }
+  add_to_row_tables(s, r, 0, tables, o);
 }
 
-// pass 5: the last digit, then the draw among the chunk's kept tokens
-__global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_draw_kernel(const float* __restrict__ logits, const int* __restrict__ options,
-                                                                           ChunkedScratch s, int vocab, int with_filter) {
-  __shared__ Best best_scratch[16];
-  __shared__ DrawQueue queue;
+// pass 3: the first digit, and the chunk's tokens that it does not rule out (a row without a filter: the chunk's draw)
+__global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_list_kernel(const float* __restrict__ logits, const int* __restrict__ options,
+                                                                           ChunkedScratch s, int vocab) {
+  constexpr int WAVES = SAMPLE_THREADS / 64;
+  __shared__ union { Listed listed[WAVES][LIST_ENTRIES]; LevelTables<1> tables; DrawQueue queue; } shared;
   __shared__ SelectScratch select;
-  __shared__ int before[SAMPLE_THREADS / 64 + 1];
+  __shared__ Best best_scratch[16];
+  __shared__ int found_of_wave[WAVES];
   const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
   const float* row = logits + (size_t)r * vocab;
   const RowOptions o = read_options(options + (size_t)r * 6, vocab);
   if (o.temperature == 0.f) return;  // (its chunks' best pairs are there since the first pass)
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int q_lo, q_hi;
-  chunk_quads(vocab, q_lo, q_hi);
+  chunk_quads(vocab, c, q_lo, q_hi);
   const float mx = row_max_of_chunks(s.chunk_max + r * chunks, chunks);
-  uint32_t threshold = 0u;
-  if (o.filter && !with_filter) {
+  if (!o.filter) {
+    const Best best = block_best(draw_in_quads(row, vocab, q_lo, q_hi, o, mx, 0u, shared.queue, [](int, float, uint32_t) { return false; }), best_scratch);
+    if (tid == 0) s.chunk_best[r * chunks + c] = best;
+    return;
+  }
+  Above above{0u, 0ull};
+  unsigned long long mass_limit = 0ull;
+  const size_t base = (size_t)r * 2 * SELECT_BINS;
+  const uint32_t prefix = digit_of_table(0, o, 0u, mass_limit, above, select, [&](int bin, unsigned int& count, unsigned long long& mass) {
+    if (o.top_k > 0) count = s.counts[base + bin];
+    if (o.use_mass) mass = s.masses[base + bin];
+  });
+  if (c == 0 && tid == 0) {
+    s.search[r].mass_limit = mass_limit;
+    s.search[r].above_mass = above.mass;
+    s.search[r].above_count = above.count;
+    s.search[r].prefix = prefix;
+  }
+  const int found = list_tokens(row, vocab, q_lo, q_hi, o, prefix, shared.listed[wave]);
+  if (lane == 0) found_of_wave[wave] = found;
+  __syncthreads();
+  int before = 0, total = 0;
+  bool whole = true;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    const int of_wave = found_of_wave[w];
+    before += w < wave ? of_wave : 0;
+    total += of_wave;
+    whole = whole && of_wave <= LIST_ENTRIES;
+  }
+  if (tid == 0) s.list_lengths[r * chunks + c] = whole ? total : -1;
+  if (whole) {
+    Listed* mine = s.lists + ((size_t)r * chunks + c) * s.list_room + before;
+    for (int j = lane; j < found; j += 64) mine[j] = shared.listed[wave][j];
+    return;
+  }
+  if (tid == 0) s.search[r].unlisted = 1;
+  __syncthreads();
+  clear_tables(shared.tables, 1, o);
+  __syncthreads();
+  add_to_tables(row, vocab, q_lo, q_hi, o, mx, 1, prefix, shared.tables);
+  __syncthreads();
+  add_to_row_tables(s, r, 1, shared.tables, o);
+}
+
+// A pair that another workgroup of the same kernel reads or has written: past the caches that only some of the card's compute units share.
+__device__ __forceinline__ void store_shared_pair(void* p, unsigned long long pair) {
+  __hip_atomic_store((unsigned long long*)p, pair, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long load_shared_pair(const void* p) {
+  return __hip_atomic_load((unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T> __device__ __forceinline__ unsigned long long pair_bits(const T& pair) {
+  static_assert(sizeof(T) == 8 && alignof(T) <= 8, "two words");
+  unsigned long long bits;
+  __builtin_memcpy(&bits, &pair, 8);
+  return bits;
+}
+template <typename T> __device__ __forceinline__ T pair_of_bits(unsigned long long bits) {
+  T pair;
+  __builtin_memcpy(&pair, &bits, 8);
+  return pair;
+}
+// this wave's stores have arrived
+__device__ __forceinline__ void wait_for_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// The best pair of a row's chunks.
+__device__ __forceinline__ Best best_of_chunks(const Best* chunk_best, int chunks, Best* scratch) {
+  Best best{-INFINITY, 0x7fffffff};
+  for (int c = threadIdx.x; c < chunks; c += blockDim.x) best = better(best, pair_of_bits<Best>(load_shared_pair(chunk_best + c)));
+  return block_best(best, scratch);
+}
+
+// pass 4 of a row with a filter: the other digits, the draw and the token.  All chunks listed: the workgroup of chunk 0 does it alone.
+// Otherwise each chunk's workgroup finds the second digit, draws among its tokens above that digit's, and lists those that share
+// it, which the third digit still decides over ("open": a few, unless logits are equal); the last of the row's workgroups to come
+// that far finds the third digit, draws among the open ones and merges the chunks.
+// The sampler's kernels before (one for the third digit, one for the draw, one to merge the chunks) and now, us: 48 rows of 152,064
+// with top-p 0.9 44.8 -> 41.4, top-k 50 38.3 -> 32.6; one row 35.1 -> 29.0 and 33.6 -> 26.9; eight rows of 32,000 34.0 -> 29.6.  Flat
+// rows (standard deviation 0.4, top-p 0.95; no chunk listed): 48 and one of 152,064 66.4 -> 67.7 and 42.5 -> 42.5, of 32,000 43.6 -> 45.7.
+#define FINISH_TOKENS 6144
+__global__ void __launch_bounds__(SAMPLE_THREADS) sample_finish_kernel(const float* __restrict__ logits, const int* __restrict__ options, int* __restrict__ out,
+                                                                       ChunkedScratch s, int vocab) {
+  __shared__ union { Listed tokens[FINISH_TOKENS]; DrawQueue queue; } shared;
+  __shared__ LevelTables<1> tables;
+  __shared__ SelectScratch select;
+  __shared__ Best best_scratch[16];
+  __shared__ int before[1024 + 1], sum_of_wave[SAMPLE_THREADS / 64], kept_count, last;
+  const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
+  const float* row = logits + (size_t)r * vocab;
+  const RowOptions o = read_options(options + (size_t)r * 6, vocab);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool filtered = o.temperature != 0.f && o.filter;
+  // (asked for together: the kernel's time is that of its trips to memory)
+  const RowSearch search = s.search[r];
+  const int length = tid < chunks ? s.list_lengths[r * chunks + tid] : 0;
+  const float mx = row_max_of_chunks(s.chunk_max + r * chunks, chunks);
+  const bool unlisted = filtered && search.unlisted != 0;
+  if (c != 0 && !unlisted) return;
+  if (!filtered) {
+    const Best best = best_of_chunks(s.chunk_best + r * chunks, chunks, best_scratch);
+    if (tid == 0) out[r] = best.index;
+    return;
+  }
+  Above above{search.above_count, search.above_mass};
+  unsigned long long mass_limit = search.mass_limit;
+  uint32_t prefix = search.prefix;
+  const Listed* lists = s.lists + (size_t)r * chunks * s.list_room;
+  auto listed_at = [&](int j) {  // the row's listed token j
+    int lo = 0, hi = chunks;     // before[lo] <= j < before[hi]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (before[mid] <= j) lo = mid;
+      else hi = mid;
+    }
+    return lists + (size_t)lo * s.list_room + (j - before[lo]);
+  };
+  auto draw_one = [&](int i, float x, Best& best) {
+    uint32_t bits[4];
+    philox4x32((uint32_t)(i >> 2), o.counter, 0u, 0u, o.seed_lo, o.seed_hi, bits);
+    draw_token(i, x, (i & 2) ? ((i & 1) ? bits[3] : bits[2]) : ((i & 1) ? bits[1] : bits[0]), mx, best);
+  };
+  if (tid == 0) kept_count = 0;
+  // where each chunk's list begins among the row's
+  const int own_tokens = max(length, 0);
+  int upto = own_tokens;
+#pragma unroll
+  for (int offset = 1; offset < 64; offset <<= 1) {
+    const int other = __shfl_up(upto, offset, VELOX_WAVE);
+    if (lane >= offset) upto += other;
+  }
+  if (lane == 63) sum_of_wave[wave] = upto;
+  __syncthreads();
+  int total = 0;
+  for (int w = 0; w < SAMPLE_THREADS / 64; ++w) {
+    const int of_wave = sum_of_wave[w];
+    upto += w < wave ? of_wave : 0;
+    total += of_wave;
+  }
+  if (tid < chunks) before[tid] = upto - own_tokens;
+  __syncthreads();
+  const bool held = total <= FINISH_TOKENS;  // (each thread reads back what it wrote itself)
+  if (held)
+    for (int j = tid; j < total; j += SAMPLE_THREADS) shared.tokens[j] = *listed_at(j);
+  Best best{-INFINITY, 0x7fffffff};
+#pragma unroll 1
+  for (int level = 1; level <= (unlisted ? 1 : 2); ++level) {  // (one loop: code that runs once is fetched while it runs)
+    clear_tables(tables, level, o);
+    __syncthreads();
+    const int known = level_shift(level - 1), shift = level_shift(level);
+    for (int j = tid; j < total; j += SAMPLE_THREADS) {
+      const float x = (held ? shared.tokens[j] : *listed_at(j)).logit * o.inv_t;
+      const uint32_t key = sort_key(x);
+      if ((key >> known) == (prefix >> known)) add_token(tables, (int)((key >> shift) & (uint32_t)(level_bins(level) - 1)), x, o, mx);
+    }
+    __syncthreads();
+    const size_t base = ((size_t)r * 2 + 1) * SELECT_BINS;
+    prefix = digit_of_table(level, o, prefix, mass_limit, above, select, [&](int bin, unsigned int& count, unsigned long long& mass) {
+      table_entry(tables, level, bin, o, count, mass);
+      if (unlisted && o.top_k > 0) count += s.counts[base + bin];
+      if (unlisted && o.use_mass) mass += s.masses[base + bin];
+    });
+    __syncthreads();
+  }
+  if (!unlisted) {
+    // The kept tokens are a part of the listed ones, in no order: gathered in the tables' place, so that few waves work out noise.
+    constexpr int ROOM = (int)(sizeof(tables) / sizeof(Listed));
+    Listed* kept = reinterpret_cast<Listed*>(&tables);
+    for (int j = tid; j < total; j += SAMPLE_THREADS) {
+      const Listed token = held ? shared.tokens[j] : *listed_at(j);
+      const float x = token.logit * o.inv_t;
+      if (sort_key(x) >= prefix) {
+        const int at = atomicAdd(&kept_count, 1);
+        if (at < ROOM) kept[at] = token;
+      }
+    }
+    __syncthreads();
+    const bool all = kept_count <= ROOM;
+    for (int j = tid; j < (all ? kept_count : total); j += SAMPLE_THREADS) {
+      const Listed token = all ? kept[j] : held ? shared.tokens[j] : *listed_at(j);
+      const float x = token.logit * o.inv_t;
+      if (sort_key(x) >= prefix) draw_one(token.index, x, best);
+    }
+    best = block_best(best, best_scratch);
+    if (tid == 0) out[r] = best.index;
+    return;
+  }
+  int q_lo, q_hi;
+  chunk_quads(vocab, c, q_lo, q_hi);
+  Listed* open = s.open + (size_t)r * OPEN_TOKENS;
+  best = draw_in_quads(row, vocab, q_lo, q_hi, o, mx, prefix, shared.queue, [&](int i, float v, uint32_t key) {
+    if ((key >> 10) != (prefix >> 10)) return false;
+    const unsigned int at = __hip_atomic_fetch_add(&s.search[r].open, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (at < OPEN_TOKENS) store_shared_pair(open + at, pair_bits(Listed{v, i}));
+    return true;
+  });
+  best = block_best(best, best_scratch);
+  // (fences that write back and drop whole caches, in every wave, took 40 to 70 us here: what the last workgroup reads goes past them)
+  wait_for_stores();
+  __syncthreads();
+  if (tid == 0) {
+    store_shared_pair(s.chunk_best + r * chunks + c, pair_bits(best));
+    wait_for_stores();
+    last = __hip_atomic_fetch_add(&s.search[r].drawn, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == (unsigned int)chunks ? 1 : 0;
+  }
+  __syncthreads();
+  if (last == 0) return;
+  // The open tokens, a thread each; where there are more than their list holds they are found again in the row, for each of the two uses.
+  const unsigned int found = __hip_atomic_load(&s.search[r].open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  static_assert(OPEN_TOKENS <= SAMPLE_THREADS, "a thread each");
+  const Listed mine = pair_of_bits<Listed>(tid < min(found, (unsigned int)OPEN_TOKENS) ? load_shared_pair(open + tid) : 0ull);
+  clear_tables(tables, 2, o);
+  __syncthreads();
+  auto for_each_open = [&](auto f) {
+    if (found <= OPEN_TOKENS) {
+      if (tid < found) f(mine.index, mine.logit * o.inv_t);
+    } else {
+      for_each_in_quads(row, vocab, 0, (vocab + 3) / 4, [&](int i, float v) {
+        if ((sort_key(v * o.inv_t) >> 10) == (prefix >> 10)) f(i, v * o.inv_t);
+      });
+    }
+  };
+  for_each_open([&](int, float x) { add_token(tables, (int)(sort_key(x) & (uint32_t)(level_bins(2) - 1)), x, o, mx); });
+  __syncthreads();
+  prefix = digit_of_table(2, o, prefix, mass_limit, above, select, [&](int bin, unsigned int& count, unsigned long long& mass) { table_entry(tables, 2, bin, o, count, mass); });
+  best = Best{-INFINITY, 0x7fffffff};
+  for_each_open([&](int i, float x) {
+    if (sort_key(x) >= prefix) draw_one(i, x, best);
+  });
+  best = better(block_best(best, best_scratch), best_of_chunks(s.chunk_best + r * chunks, chunks, best_scratch));
+  if (tid == 0) out[r] = best.index;
+}
+
+// Rows of a batch without any filter: the draw behind the maximum, among all of a chunk's tokens.
+__global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_draw_kernel(const float* __restrict__ logits, const int* __restrict__ options,
+                                                                           ChunkedScratch s, int vocab) {
+  __shared__ Best best_scratch[16];
+  __shared__ DrawQueue queue;
+  const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
+  const RowOptions o = read_options(options + (size_t)r * 6, vocab);
+  if (o.temperature == 0.f) return;  // (its chunks' best pairs are there since the first pass)
+  if (o.filter) {
     // the caller promised that no row has a filter, and this one has: the kernels of the digits did not run.  No token
     // rather than one drawn from the wrong set: the row's result is -1.
     if (threadIdx.x == 0) s.chunk_best[r * chunks + c] = Best{INFINITY, -1};
     return;
   }
-  int total = -1;
-  if (o.filter) {
-    total = listed_tokens(s, r * chunks + c, before);
-    Above above{s.search[r].above_count[1], s.search[r].above_mass[1]};
-    unsigned long long mass_limit = s.search[r].mass_limit;
-    threshold = finished_digit(s, r, 2, o, s.search[r].prefix[1], mass_limit, above, select);
-  }
-  Best best{-INFINITY, 0x7fffffff};
-  if (total >= 0) {
-    for_each_listed(s, r * chunks + c, before, total, [&](int i, float v) {
-      const float x = v * o.inv_t;
-      if (sort_key(x) < threshold) return;
-      uint32_t bits[4];
-      philox4x32((uint32_t)(i >> 2), o.counter, 0u, 0u, o.seed_lo, o.seed_hi, bits);
-      draw_token(i, x, (i & 2) ? ((i & 1) ? bits[3] : bits[2]) : ((i & 1) ? bits[1] : bits[0]), mx, best);
-    });
-  } else {
-    best = draw_in_quads(row, vocab, q_lo, q_hi, o, mx, threshold, queue);
-  }
-  best = block_best(best, best_scratch);
+  int q_lo, q_hi;
+  chunk_quads(vocab, c, q_lo, q_hi);
+  const float mx = row_max_of_chunks(s.chunk_max + r * chunks, chunks);
+  const Best best = block_best(draw_in_quads(logits + (size_t)r * vocab, vocab, q_lo, q_hi, o, mx, 0u, queue, [](int, float, uint32_t) { return false; }), best_scratch);
   if (threadIdx.x == 0) s.chunk_best[r * chunks + c] = best;
 }
 
@@ -848,7 +1000,7 @@ extern "C" long long velox_sample_chunked_scratch_bytes(int rows, int vocab, int
 
 // The same tokens as velox_sample, every row cut into `chunks` chunks.  scratch: velox_sample_chunked_scratch_bytes(rows,
 // vocab, chunks) bytes at a 256-byte boundary, contents arbitrary.  with_filter = 0 promises that no row has top-k or top-p (the
-// three kernels of the digits are then left out; a row that has one all the same gets the token -1).
+// kernels of the digits are then left out; a row that has one all the same gets the token -1).
 extern "C" int velox_sample_chunked(const float* logits, const int* options, int* out, int rows, int vocab, int chunks, void* scratch,
                                     long long scratch_bytes, int with_filter, hipStream_t stream) {
   if (rows <= 0) return 0;
@@ -858,12 +1010,13 @@ extern "C" int velox_sample_chunked(const float* logits, const int* options, int
   const dim3 grid(rows, chunks);
   sample_chunk_max_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, s, vocab);
   if (with_filter) {
-    sample_chunk_tables_kernel<0><<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, s, vocab);
-    sample_chunk_tables_kernel<1><<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, s, vocab);
-    sample_chunk_tables_kernel<2><<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, s, vocab);
+    sample_chunk_tables_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, s, vocab);
+    sample_chunk_list_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, s, vocab);
+    sample_finish_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, out, s, vocab);
+  } else {
+    sample_chunk_draw_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, s, vocab);
+    argmax_merge_kernel<<<rows, 64, 0, stream>>>(s.chunk_best, out, chunks);
   }
-  sample_chunk_draw_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, options, s, vocab, with_filter);
-  argmax_merge_kernel<<<rows, 64, 0, stream>>>(s.chunk_best, out, chunks);
   VELOX_RETURN_LAUNCH_STATUS();
 }
 
