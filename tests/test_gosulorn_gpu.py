@@ -309,6 +309,23 @@ def test_recurrence_prepare_scan_and_head_norm(ops, ref, dtype, heads, kv_heads,
         near(ops.gated_head_norm(b, weight, 1e-6, low, cols, kind, heads, vdim, dt), ref.gated_head_norm(b, weight, 1e-6, low, cols, kind, heads, vdim, dt), REL[dtype], kind)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,dim,shift", [(8, 128, 0), (8, 128, 1), (3, 4, 0), (4, 20, 0), (4, 64, 2), (2, 256, 0), (2, 260, 0), (5, 100, 4)])
+def test_head_norms_of_four_channels_at_a_time_and_of_one(ops, ref, dtype, heads, dim, shift):
+    """Heads of one to 64 lanes with and without lanes to spare, wider ones, and gates off a boundary of four: against the plain reference,
+    and a token by itself, or a gate moved off a boundary of four, has the bits of the whole step."""
+    g, dt = torch.Generator().manual_seed(dim + shift), DTYPES[dtype]
+    size, tokens = heads * dim, 133
+    read, gates = rnd(g, tokens, size), rnd(g, tokens, 2 * size + 4 + shift, dtype=dt)
+    moved = torch.cat([gates[:, :1], gates], 1)
+    for weight in (rnd(g, dim), rnd(g, size)):
+        for kind in ("silu", "sigmoid"):
+            got = ops.gated_head_norm(read, weight, 1e-6, gates, size + shift, kind, heads, dim, dt)
+            near(got, ref.gated_head_norm(read, weight, 1e-6, gates, size + shift, kind, heads, dim, dt), REL[dtype], kind)
+            assert torch.equal(got, ops.gated_head_norm(read, weight, 1e-6, moved, size + shift + 1, kind, heads, dim, dt))
+            assert torch.equal(got[77:78], ops.gated_head_norm(read[77:78].clone(), weight, 1e-6, gates[77:78].clone(), size + shift, kind, heads, dim, dt))
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,per_channel,delta_rule", [(4, 2, 64, 64, True, True), (2, 2, 128, 128, False, True), (3, 3, 32, 48, True, False), (2, 1, 256, 20, True, True),
                                                                             (1, 1, 128, 9, True, False), (2, 2, 72, 40, False, True), (1, 1, 512, 16, True, True)])
 def test_a_long_portion_equals_its_pieces_and_its_first_token_is_kept(ops, ref, heads, kv_heads, dim, vdim, per_channel, delta_rule):
