@@ -1212,7 +1212,9 @@ class HipOps:
     MAX_STREAM_WIDTH = 16384
     MAX_CONV_TAPS = 8
 
-    STREAMS_WAIT_FROM_BYTES = 4 << 20  # of streams: below that a pass over them is a kernel's own beginning and end (128 rows of 4 x 2,048)
+    # Of streams: from 1,024 rows of 4 x 2,048 on.  Keeping the terms costs the host 4 us a sub-layer, and steps of fewer rows wait for the host (eight
+    # layers: 350 rows 1,974 us written every time, 2,043 not, though the kernels take 80 us less; 2,421 rows 4,487 and 4,290).
+    STREAMS_WAIT_FROM_BYTES = 32 << 20
 
     def streams_may_wait(self, residual, terms, weight, streams: int, held: int) -> bool:
         """Whether ``stream_norm`` should leave the streams unwritten (``settle=False``) with ``held`` updates unwritten already."""
