@@ -421,11 +421,11 @@ extern "C" int velox_tiles_bf16(const void* a, const void* w, const float* bias,
   return out_dtype == VELOX_BF16 ? tiles_launch<TL_PLAIN, bf16_t, true>(args, tile, stream) : tiles_launch<TL_PLAIN, float, true>(args, tile, stream);
 }
 
-// out[M, N] = act(A Wgate^T) * (A Wup^T) in bfloat16 for W = [Wgate; Wup] [2 N, K], both sums rounded to bfloat16 in front of it; act 0: SiLU, 1: the tanh form
-// of GELU, 2: the rectifier.  Needs k % 64 == 0, n % 4 == 0 and 16-byte aligned bases.
+// out[M, N] = act(A Wgate^T) * (A Wup^T) in bfloat16 for W = [Wgate; Wup] [2 N, K], both sums rounded to bfloat16 in front of it; act 0: SiLU, 2: the
+// rectifier (the tanh form of GELU stays a kernel of its own: its tangent costs more than the pass).  Needs k % 64 == 0, n % 4 == 0 and 16-byte aligned bases.
 extern "C" int velox_tiles_glu_bf16(const void* a, const void* w, void* out, int m, int n, int k, int act, int tile, hipStream_t stream) {
   if (m <= 0 || n <= 0) return 0;
-  if (k < 1 || k % 64 != 0 || n % 4 != 0 || act < 0 || act > 2 || (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) != 0 || !tiles_fit(256, k, n + 256LL, k)) return -1;
+  if (k < 1 || k % 64 != 0 || n % 4 != 0 || (act != 0 && act != 2) || (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) != 0 || !tiles_fit(256, k, n + 256LL, k)) return -1;
   TileArgs args = {};
   args.a = (const bf16_t*)a;
   args.a_ld = k;
@@ -436,7 +436,6 @@ extern "C" int velox_tiles_glu_bf16(const void* a, const void* w, void* out, int
   args.k = k;
   args.splits = 1;
   if (tile == 0) tile = tiles_pick(m, 2LL * n, k, 1);
-  if (act == 1) return tiles_launch<TL_GELU, bf16_t, false>(args, tile, stream);
   return act == 0 ? tiles_launch<TL_SILU, bf16_t, false>(args, tile, stream) : tiles_launch<TL_RELU, bf16_t, false>(args, tile, stream);
 }
 

@@ -36,7 +36,7 @@ typedef unsigned int tl_uint4_t __attribute__((ext_vector_type(4)));
 
 // what becomes of the sums: nothing; silu(gate) * up and max(gate, 0) * up of sums that are rounded to bfloat16 first, as a product of its
 // own would leave them; an expert's gated middle, silu(gate) * up or any other; a unit without a gate branch
-enum { TL_PLAIN = 0, TL_SILU = 1, TL_RELU = 2, TL_SILU_UNIT = 3, TL_UNIT = 4, TL_ACT = 5, TL_GELU = 6 };
+enum { TL_PLAIN = 0, TL_SILU = 1, TL_RELU = 2, TL_SILU_UNIT = 3, TL_UNIT = 4, TL_ACT = 5 };
 
 #define TL_XCDS 8
 #define TL_WORKGROUPS 256  // one per compute unit
@@ -107,14 +107,6 @@ __device__ __forceinline__ float tl_silu(float g) {
   return fabsf(g) <= 88.7f ? fmaf(-fmaf(near, below, -above), inverse, near) : near;
 }
 
-// The tanh form of GELU of a bfloat16 g, g (1 + tanh(y)) / 2 with y = sqrt(2 / pi) (g + 0.044715 g^3).  1 + tanh(y) is 2 / (1 + e^-2y), which a tangent
-// subtracts from 1 for g < 0 (1e-05 of the result off at -3, all of it at -6): this is g / (1 + 2^(-2 y log2 e)) by the instruction set's exponential and
-// reciprocal, within 1.4e-06 of the result for |g| <= 6 where the bfloat16 that is stored is within 3.9e-03, in 8 instructions where SiLU's way above takes some
-// twenty (2,421 x 11,264 x 2,048, us: 101; with SiLU's way 110; a product and the tangent's kernel behind it 124).
-__device__ __forceinline__ float tl_gelu(float g) {
-  return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-2.30220819f * fmaf(0.044715f * g * g, g, g)));
-}
-
 // A gated unit's middle.
 template <int EPI>
 __device__ __forceinline__ float tl_middle(float gate, float up, const TileArgs& args) {
@@ -124,7 +116,6 @@ __device__ __forceinline__ float tl_middle(float gate, float up, const TileArgs&
     up = to_f32(from_f32<bf16_t>(up));
   }
   if (EPI == TL_RELU) return fmaxf(gate, 0.f) * up;
-  if (EPI == TL_GELU) return tl_gelu(gate) * up;
   return tl_silu<EPI == TL_SILU>(gate) * up;
 }
 
@@ -136,7 +127,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
   static_assert(S * STAGE <= 160 * 1024, "LDS of a compute unit");
   constexpr int RH0 = (RT + 1) / 2, RH1 = RT - RH0, CH0 = (CT + 1) / 2, CH1 = CT - CH0;  // halves of a wave's tiles
   constexpr int LA0 = 2 * RH0, LC0 = 2 * CH0, LC1 = 2 * CH1, LA1 = 2 * RH1, LOADS = LA0 + LC0 + LC1 + LA1;  // loads of a wave in a step, in this order
-  constexpr bool GLU = EPI == TL_SILU || EPI == TL_RELU || EPI == TL_GELU || EPI == TL_SILU_UNIT || EPI == TL_UNIT;
+  constexpr bool GLU = EPI == TL_SILU || EPI == TL_RELU || EPI == TL_SILU_UNIT || EPI == TL_UNIT;
   constexpr int OUT_COLS = GLU ? TN / 2 : TN;  // output columns of the tile
   constexpr int BLOCK_ROWS = 1024 / TM;        // row tiles of a block
   __shared__ __attribute__((aligned(1024))) char smem[S * STAGE];
@@ -495,7 +486,7 @@ static inline int tiles_splits(long long m, long long n, int k, int most) {
 // One product in tiles of `tile`.
 template <int EPI, typename TO, bool TAIL>
 static int tiles_launch(const TileArgs& args, int tile, hipStream_t stream) {
-  constexpr int BRANCHES = EPI == TL_SILU || EPI == TL_RELU || EPI == TL_GELU ? 2 : 1;
+  constexpr int BRANCHES = EPI == TL_SILU || EPI == TL_RELU ? 2 : 1;
 #define TILES(RT, CT, S)                                                                                                              \
   case 64 * RT * 1000 + 64 * CT: {                                                                                                    \
     const long long cols = (args.n + 64 * CT / BRANCHES - 1) / (64 * CT / BRANCHES);                                                  \

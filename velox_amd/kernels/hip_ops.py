@@ -1005,7 +1005,7 @@ class HipOps:
             self._launched(self._core.velox_skinny_glu_rows_bf16(_ptr(x), _ptr(packed), _ptr(out), m, n, k, per_group if pairs is None else int(pairs), self._stream()),
                            "skinny_glu_rows")
             return out
-        if (not fused and deferred is None and self.use_library_gemm and x.dim() == 2 and gate_up_weight.dim() == 2 and two_n % 16 == 0
+        if (not fused and activation != "gelu_tanh" and deferred is None and self.use_library_gemm and x.dim() == 2 and gate_up_weight.dim() == 2 and two_n % 16 == 0
                 and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16 and out_dtype == torch.bfloat16 and gate_up_weight.shape[1] == k
                 and (two_n // 2 + 256) * k < 1 << 30 and self.tiles_serve(m, two_n, k, gated=True) and not self._library_has_timed(m, two_n, k)):
             # many rows: the activation where the tiles' sums are finished.  Both sums are rounded to bfloat16 in front of it, as a
