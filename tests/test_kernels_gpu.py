@@ -1,6 +1,7 @@
 """Each HIP kernel alone against its plain PyTorch reference (tests/torch_ops.py), in float32 and
 bfloat16, at sizes other than the engine's tiny models: widths and vocabularies that are no power
 of two, head sizes 16 .. 256, groups of 1, 3, 7, page sizes 4 .. 64."""
+import itertools
 import math
 import threading
 
@@ -954,6 +955,50 @@ def test_sampling_with_lists_and_open_tokens_beyond_their_room(ops, vocab, chunk
     whole = ops.sample(logits, options, chunks=1)
     for _ in range(2):
         assert torch.equal(ops.sample(logits, options, chunks=chunks), whole)
+
+
+@pytest.mark.parametrize("vocab, chunks", [(40000, 2), (40000, 3), (152064, 18), (9001, 32)])
+@pytest.mark.parametrize("top_p, top_k", [(0.9, 0), (1.0, 40), (1.0, 6000)])
+def test_sampling_with_as_many_tokens_left_as_one_workgroup_takes(ops, vocab, chunks, top_p, top_k):
+    """A chunk's share of the 6,144 tokens that one workgroup finishes a row with: chunks that leave one less, as many and one more, in one chunk of
+    the row and in all; spread over a chunk's waves, or in one wave's quads alone; scores of zero with either sign.  The tokens of the
+    one-workgroup kernel, bit for bit."""
+    g = torch.Generator().manual_seed(vocab + chunks)
+    share, per_chunk = 6144 // chunks, 4 * (((vocab + 3) // 4 + chunks - 1) // chunks)
+    logits = torch.full((16, vocab), -30.0) - torch.rand((16, vocab), generator=g)
+    for r, (more, everywhere) in enumerate(itertools.product((-1, 0, 1, 40, 4000), (False, True))):
+        for c in range(chunks if everywhere else 1):
+            room = torch.arange(c * per_chunk, min((c + 1) * per_chunk, vocab))
+            left = room[torch.randperm(len(room), generator=g)[:share + more]] if r % 4 else room[:share + more]
+            logits[r, left] = 4.0 + 0.9 * torch.rand(len(left), generator=g)
+    logits[10], logits[11], logits[12] = 0.0, -0.0, torch.where(torch.rand(vocab, generator=g) < 0.5, 0.0, -0.0)
+    logits[13, ::2], logits[14], logits[15] = float("-inf"), 1.2 * torch.randn(vocab, generator=g), 0.3 * torch.randn(vocab, generator=g).bfloat16().float()
+    logits = logits.repeat_interleave(2, 0).cuda()
+    options = np.zeros((logits.shape[0], 6), dtype=np.int32)
+    options.view(np.float32)[:, 0], options.view(np.float32)[:, 1] = 1.0, top_p
+    options[:, 2], options[:, 3] = top_k, np.arange(logits.shape[0])
+    options = torch.from_numpy(options).cuda()
+    assert torch.equal(ops.sample(logits, options, chunks=chunks), ops.sample(logits, options, chunks=1))
+
+
+@pytest.mark.parametrize("kind, top_p, top_k", [("equal", 1.0, 2000), ("masked", 1.0, 2000), ("wide", 0.9, 0), ("wide", 1.0, 20000)])
+def test_rows_in_chunks_are_worked_on_by_all_of_their_workgroups(ops, kind, top_p, top_k):
+    """Eight rows of 152,064 whose threshold many tokens share (equal logits; all but 100 masked to -inf and a larger top-k) or that leave tens of thousands
+    over: 18 workgroups a row take well below half of one workgroup's time (a tenth to a third; one of the 18 alone would take two thirds and more)."""
+    from velox_amd.kernels.measure import time_in_graph
+
+    g = torch.Generator().manual_seed(2)
+    rows, vocab = 8, 152064
+    logits = {"equal": torch.ones((rows, vocab)), "wide": 1.5 * torch.randn((rows, vocab), generator=g), "masked": torch.full((rows, vocab), float("-inf"))}[kind]
+    if kind == "masked":
+        logits[:, torch.randperm(vocab, generator=g)[:100]] = torch.randn((rows, 100), generator=g)
+    logits = logits.cuda()
+    options = np.zeros((rows, 6), dtype=np.int32)
+    options.view(np.float32)[:, 0], options.view(np.float32)[:, 1] = 0.8, top_p
+    options[:, 2], options[:, 3] = top_k, np.arange(rows)
+    options = torch.from_numpy(options).cuda()
+    one, many = (time_in_graph(lambda: ops.sample(logits, options, chunks=chunks)) for chunks in (1, 18))
+    assert many < 0.5 * one, (many, one)
 
 
 def test_penalties_over_long_histories_and_a_large_vocabulary(ops, ref):

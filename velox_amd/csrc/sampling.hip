@@ -308,8 +308,8 @@ __device__ __forceinline__ int select_digit(const unsigned int (&c)[2], const un
 //   draw is argmax(x - max - log(e)), e = max(-log(u), 1e-10), u uniform from Philox(key = seed, counter = (i / 4, counter)).
 // Passes over the row (from the caches: a row is a few hundred kilobytes): the maximum; with a filter, the sum and three
 // digits of the threshold; the draw.  Either one workgroup walks the whole row (sample_kernel), or, when the rows are
-// too few to fill the GPU that way, the row is cut into chunks of quads with a workgroup each and every pass is a
-// kernel (the sample_chunk_* kernels): the same functions over a range of quads, the tables added up in global memory
+// too few to fill the GPU that way, the row is cut into chunks of quads with a workgroup each (the sample_chunk_* kernels
+// and sample_finish_kernel): the same functions over a range of quads, the tables added up in global memory
 // as integers, so both ways give the same token.
 struct RowOptions {
   float temperature, top_p, inv_t;
@@ -411,14 +411,19 @@ struct DrawQueue {
   int quads[SAMPLE_THREADS / 64][DRAW_QUEUE];
 };
 
-// token i with its word of the noise
-__device__ __forceinline__ void draw_token(int i, float x, uint32_t bits, float mx, Best& best) {
+// what a token's word of the noise makes of it
+__device__ __forceinline__ float token_score(float x, uint32_t bits, float mx) {
   const float u = ((float)(bits >> 8) + 0.5f) * (1.0f / 16777216.0f);
   const float noise = fmaxf(-logf(u), 1e-10f);
   const float raw = (x - mx) - logf(noise);
   // A score that is no number (of a NaN among the logits, or where the row's largest is infinite) counts as -inf: it would otherwise
   // win or lose by the order in which threads meet it, and could leave a row without any token.
-  const float score = raw > -INFINITY ? raw : -INFINITY;
+  return raw > -INFINITY ? raw : -INFINITY;
+}
+
+// token i with its word of the noise
+__device__ __forceinline__ void draw_token(int i, float x, uint32_t bits, float mx, Best& best) {
+  const float score = token_score(x, bits, mx);
   // (a thread's tokens come in no order: equal scores go to the smaller index here too)
   if (score > best.value || best.index == 0x7fffffff || (score == best.value && i < best.index)) best = Best{score, i};
 }
@@ -428,10 +433,10 @@ __device__ __forceinline__ void draw_token(int i, float x, uint32_t bits, float 
 // and eight logarithms a quad) would be worked out by whole waves for a lane or two.  The kept quads are therefore queued
 // in LDS first and taken up 64 at a time (48 rows of 152,064, top-p 0.9: the pass with the digit before it 19.7 us
 // without the queue, 13.4 with it).
-// left_out(i, logit, key): a token at or above the threshold that is not drawn from.
+// open(i, x, bits): whether a token at or above the threshold is taken care of elsewhere.
 template <typename F>
 __device__ __forceinline__ Best draw_in_quads(const float* __restrict__ row, int vocab, int q_lo, int q_hi, const RowOptions& o, float mx, uint32_t threshold,
-                                              DrawQueue& queue, F left_out) {
+                                              DrawQueue& queue, F open) {
   Best best{-INFINITY, 0x7fffffff};
   const bool aligned = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
   const bool filter = o.filter;
@@ -445,7 +450,7 @@ __device__ __forceinline__ Best draw_in_quads(const float* __restrict__ row, int
       const int i = 4 * q + e;
       if (i >= vocab) break;
       const float x = v[e] * inv_t;
-      if (filter && (sort_key(x) < threshold || left_out(i, v[e], sort_key(x)))) continue;
+      if (filter && (sort_key(x) < threshold || open(i, x, bits[e]))) continue;
       draw_token(i, x, bits[e], mx, best);
     }
   };
@@ -556,33 +561,36 @@ extern "C" int velox_sample(const float* logits, const int* options, int* out, i
 // chunk (of a row with top-p 0.9 or top-k 50 about one token in a hundred); and from the lists, in one workgroup, the other digits,
 // the draw and the token.  What bounds a pass is its few dependent steps (a launch, two trips to memory, a scan over the table), not
 // the row: with a kernel per digit, one for the draw and one to merge the chunks, 48 rows of 152,064 took 55 us; see
-// sample_finish_kernel.  Where a wave finds more than LIST_ENTRIES tokens the chunk is not listed: it adds its tokens to the tables
-// of the second digit instead, and the row's chunks are drawn from by a workgroup each.
+// sample_finish_kernel.  A chunk with more such tokens than its share of FINISH_TOKENS, which is what one workgroup is quick with, adds
+// them to the tables of the second digit instead, and the row's chunks are drawn from by a workgroup each: from its list, or from
+// the row where a wave has found more than LIST_ENTRIES.
 struct RowSearch {
   unsigned long long mass_limit;  // top_p of the row's whole probability
   unsigned long long above_mass;  // what lies above the first digit's tokens
   unsigned int above_count;
   unsigned int prefix;            // the first digit, in place
-  int unlisted;                   // some chunk is not listed
+  unsigned long long best;        // of a row that is shared out, above the second digit's tokens (in_order of the pair)
+  int shared_out;                 // some chunk has more than its share of tokens
   unsigned int drawn;             // chunks of such a row that have drawn
-  unsigned int open;              // its open tokens: see sample_finish_kernel
-  unsigned int unused;
 };
-#define OPEN_TOKENS 1024
 
 #define LIST_ENTRIES 256
+#define FINISH_TOKENS 6144
+#define NOT_LISTED ((int)0x80000000)
+#define OPEN_BINS 1024  // values of the third digit
 struct Listed { float logit; int index; };
 
 struct ChunkedScratch {
   Listed* lists;               // [rows, chunks, list_room]
-  int* list_lengths;           // [rows, chunks]; -1: not listed
-  Listed* open;                // [rows, OPEN_TOKENS]
+  int* list_lengths;           // [rows, chunks]; ~length: more than the chunk's share; NOT_LISTED
   float* chunk_max;            // [rows, chunks]
   Best* chunk_best;            // [rows, chunks]
   RowSearch* search;           // [rows]
   unsigned int* counts;        // [rows, 2, SELECT_BINS]
   unsigned long long* masses;  // [rows, 2, SELECT_BINS]
-  int list_room;
+  unsigned int* open_counts;       // [rows, OPEN_BINS]: see sample_finish_kernel
+  unsigned long long* open_best;   // [rows, OPEN_BINS]
+  int list_room, share;        // tokens that a chunk has room for; that it may have for one workgroup to finish its row
 };
 
 static size_t chunked_scratch_layout(int rows, int vocab, int chunks, void* base, ChunkedScratch* scratch) {
@@ -598,9 +606,11 @@ static size_t chunked_scratch_layout(int rows, int vocab, int chunks, void* base
   s.chunk_max = (float*)take((size_t)rows * chunks * sizeof(float));
   const int chunk_tokens = 4 * (((vocab + 3) / 4 + chunks - 1) / chunks);
   s.list_room = chunk_tokens < LIST_ENTRIES * (SAMPLE_THREADS / 64) ? chunk_tokens : LIST_ENTRIES * (SAMPLE_THREADS / 64);
+  s.share = FINISH_TOKENS / chunks;
   s.lists = (Listed*)take((size_t)rows * chunks * s.list_room * sizeof(Listed));
   s.list_lengths = (int*)take((size_t)rows * chunks * sizeof(int));
-  s.open = (Listed*)take((size_t)rows * OPEN_TOKENS * sizeof(Listed));
+  s.open_best = (unsigned long long*)take((size_t)rows * OPEN_BINS * sizeof(unsigned long long));
+  s.open_counts = (unsigned int*)take((size_t)rows * OPEN_BINS * sizeof(unsigned int));
   if (scratch != nullptr) *scratch = s;
   return at;
 }
@@ -631,7 +641,11 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_max_kernel(const 
     return;
   }
   if (o.filter) {
-    if (c == 0 && threadIdx.x == 0) s.search[r].unlisted = 0, s.search[r].drawn = 0u, s.search[r].open = 0u;
+    if (c == 0 && threadIdx.x == 0) s.search[r].best = 0ull, s.search[r].shared_out = 0, s.search[r].drawn = 0u;
+    for (int e = c * blockDim.x + threadIdx.x; e < OPEN_BINS; e += chunks * blockDim.x) {
+      s.open_counts[(size_t)r * OPEN_BINS + e] = 0u;
+      s.open_best[(size_t)r * OPEN_BINS + e] = 0ull;
+    }
     const int entries = 2 * SELECT_BINS;
     for (int e = c * blockDim.x + threadIdx.x; e < entries; e += chunks * blockDim.x) {
       if (o.top_k > 0) s.counts[(size_t)r * entries + e] = 0u;
@@ -723,11 +737,19 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_tables_kernel(con
   add_to_row_tables(s, r, 0, tables, o);
 }
 
+// a chunk's draw where the row has no filter
+__device__ __forceinline__ void draw_among_all(const float* __restrict__ row, int vocab, int q_lo, int q_hi, const RowOptions& o, float mx, DrawQueue& queue,
+                                               Best* best_scratch, Best* chunk_best) {
+  const Best best = block_best(draw_in_quads(row, vocab, q_lo, q_hi, o, mx, 0u, queue, [](int, float, uint32_t) { return false; }), best_scratch);
+  if (threadIdx.x == 0) *chunk_best = best;
+}
+
 // pass 3: the first digit, and the chunk's tokens that it does not rule out (a row without a filter: the chunk's draw)
 __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_list_kernel(const float* __restrict__ logits, const int* __restrict__ options,
                                                                            ChunkedScratch s, int vocab) {
   constexpr int WAVES = SAMPLE_THREADS / 64;
-  __shared__ union { Listed listed[WAVES][LIST_ENTRIES]; LevelTables<1> tables; DrawQueue queue; } shared;
+  __shared__ union { Listed listed[WAVES][LIST_ENTRIES]; DrawQueue queue; } shared;
+  __shared__ LevelTables<1> tables;
   __shared__ SelectScratch select;
   __shared__ Best best_scratch[16];
   __shared__ int found_of_wave[WAVES];
@@ -740,8 +762,7 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_list_kernel(const
   chunk_quads(vocab, c, q_lo, q_hi);
   const float mx = row_max_of_chunks(s.chunk_max + r * chunks, chunks);
   if (!o.filter) {
-    const Best best = block_best(draw_in_quads(row, vocab, q_lo, q_hi, o, mx, 0u, shared.queue, [](int, float, uint32_t) { return false; }), best_scratch);
-    if (tid == 0) s.chunk_best[r * chunks + c] = best;
+    draw_among_all(row, vocab, q_lo, q_hi, o, mx, shared.queue, best_scratch, s.chunk_best + r * chunks + c);
     return;
   }
   Above above{0u, 0ull};
@@ -769,57 +790,72 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_list_kernel(const
     total += of_wave;
     whole = whole && of_wave <= LIST_ENTRIES;
   }
-  if (tid == 0) s.list_lengths[r * chunks + c] = whole ? total : -1;
+  const bool own_share = whole && total <= s.share;
+  if (tid == 0) s.list_lengths[r * chunks + c] = own_share ? total : whole ? ~total : NOT_LISTED;
   if (whole) {
     Listed* mine = s.lists + ((size_t)r * chunks + c) * s.list_room + before;
     for (int j = lane; j < found; j += 64) mine[j] = shared.listed[wave][j];
-    return;
   }
-  if (tid == 0) s.search[r].unlisted = 1;
+  if (own_share) return;
+  if (tid == 0) s.search[r].shared_out = 1;
+  clear_tables(tables, 1, o);
   __syncthreads();
-  clear_tables(shared.tables, 1, o);
+  if (whole) {
+    for (int j = lane; j < found; j += 64) {
+      const float x = shared.listed[wave][j].logit * o.inv_t;
+      const uint32_t key = sort_key(x);
+      if ((key >> level_shift(0)) == (prefix >> level_shift(0))) add_token(tables, (int)((key >> level_shift(1)) & (uint32_t)(level_bins(1) - 1)), x, o, mx);
+    }
+  } else {
+    add_to_tables(row, vocab, q_lo, q_hi, o, mx, 1, prefix, tables);
+  }
   __syncthreads();
-  add_to_tables(row, vocab, q_lo, q_hi, o, mx, 1, prefix, shared.tables);
-  __syncthreads();
-  add_to_row_tables(s, r, 1, shared.tables, o);
+  add_to_row_tables(s, r, 1, tables, o);
 }
 
-// A pair that another workgroup of the same kernel reads or has written: past the caches that only some of the card's compute units share.
-__device__ __forceinline__ void store_shared_pair(void* p, unsigned long long pair) {
-  __hip_atomic_store((unsigned long long*)p, pair, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// A (score, index) as one number, in the order of `better`; never 0.
+__device__ __forceinline__ unsigned long long in_order(const Best& v) {
+  return ((unsigned long long)sort_key(v.value + 0.f) << 32) | (unsigned int)~v.index;  // (a score of -0 is as good as one of 0)
 }
-__device__ __forceinline__ unsigned long long load_shared_pair(const void* p) {
-  return __hip_atomic_load((unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ float value_of_key(uint32_t key) { return __uint_as_float((key & 0x80000000u) ? key ^ 0x80000000u : ~key); }
+__device__ __forceinline__ Best of_order(unsigned long long v) {
+  return v == 0ull ? Best{-INFINITY, 0x7fffffff} : Best{value_of_key((uint32_t)(v >> 32)), (int)~(unsigned int)v};
 }
-template <typename T> __device__ __forceinline__ unsigned long long pair_bits(const T& pair) {
-  static_assert(sizeof(T) == 8 && alignof(T) <= 8, "two words");
-  unsigned long long bits;
-  __builtin_memcpy(&bits, &pair, 8);
-  return bits;
-}
-template <typename T> __device__ __forceinline__ T pair_of_bits(unsigned long long bits) {
-  T pair;
-  __builtin_memcpy(&pair, &bits, 8);
-  return pair;
-}
-// this wave's stores have arrived
+// What other workgroups of the same kernel have left by atomics: past the caches that only some of the card's compute units share.
+template <typename T> __device__ __forceinline__ T load_shared(const T* p) { return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T> __device__ __forceinline__ void add_shared(T* p, T v) { __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T> __device__ __forceinline__ void max_shared(T* p, T v) { __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// this wave's stores and atomics have arrived
 __device__ __forceinline__ void wait_for_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// The best pair of a row's chunks.
-__device__ __forceinline__ Best best_of_chunks(const Best* chunk_best, int chunks, Best* scratch) {
-  Best best{-INFINITY, 0x7fffffff};
-  for (int c = threadIdx.x; c < chunks; c += blockDim.x) best = better(best, pair_of_bits<Best>(load_shared_pair(chunk_best + c)));
-  return block_best(best, scratch);
+// a token's word of the noise
+__device__ __forceinline__ uint32_t token_bits(int i, const RowOptions& o) {
+  uint32_t bits[4];
+  philox4x32((uint32_t)(i >> 2), o.counter, 0u, 0u, o.seed_lo, o.seed_hi, bits);
+  return (i & 2) ? ((i & 1) ? bits[3] : bits[2]) : ((i & 1) ? bits[1] : bits[0]);
 }
 
-// pass 4 of a row with a filter: the other digits, the draw and the token.  All chunks listed: the workgroup of chunk 0 does it alone.
-// Otherwise each chunk's workgroup finds the second digit, draws among its tokens above that digit's, and lists those that share
-// it, which the third digit still decides over ("open": a few, unless logits are equal); the last of the row's workgroups to come
-// that far finds the third digit, draws among the open ones and merges the chunks.
-// The sampler's kernels before (one for the third digit, one for the draw, one to merge the chunks) and now, us: 48 rows of 152,064
-// with top-p 0.9 44.8 -> 41.4, top-k 50 38.3 -> 32.6; one row 35.1 -> 29.0 and 33.6 -> 26.9; eight rows of 32,000 34.0 -> 29.6.  Flat
-// rows (standard deviation 0.4, top-p 0.95; no chunk listed): 48 and one of 152,064 66.4 -> 67.7 and 42.5 -> 42.5, of 32,000 43.6 -> 45.7.
-#define FINISH_TOKENS 6144
+// A thread's open tokens of one value of the third digit, added to the workgroup's table when another value turns up: a row of equal logits
+// would otherwise queue up at one entry, token by token.
+struct OpenRun {
+  unsigned long long best;
+  unsigned int count, bin;
+};
+__device__ __forceinline__ void settle(const OpenRun& run, unsigned int* counts, unsigned long long* best) {
+  if (run.count == 0u) return;
+  atomicAdd(&counts[run.bin], run.count);
+  atomicMax(&best[run.bin], run.best);
+}
+
+// pass 4 of a row with a filter: the other digits, the draw and the token.  No chunk beyond its share: the workgroup of chunk 0 does it alone.
+// Otherwise each chunk's workgroup finds the second digit and draws among its tokens above that digit's.  Which of those that share
+// it ("open") are kept the third digit still decides: they are counted, and the best of them kept, per value of that digit, and the
+// last of the row's workgroups to come that far finds the digit in these tables and with it the token, without another look at the
+// row.  (A table of the 1,024 values and not a list: logits that are equal, or masked to -inf, may all be open.)
+// The six kernels before (one for each digit, one for the draw, one to merge the chunks) and these four, us: 48 rows of 152,064 with
+// top-p 0.9 46.3 -> 42.1, top-k 50 37.8 -> 32.6; one row 35.0 -> 32.3 and 33.3 -> 26.7; 48 rows of 32,000 34.7 -> 30.4.  Shared out, 8 rows of
+// 152,064: standard deviation 0.4 and top-p 0.9 44.9 -> 40.6, 1.5 44.0 -> 40.4, top-k 20,000 36.8 -> 33.5, equal logits 55.7 -> 45.2 (one
+// workgroup for all listed tokens took 164 us for the second, a list of the open tokens 325 for the last).
 __global__ void __launch_bounds__(SAMPLE_THREADS) sample_finish_kernel(const float* __restrict__ logits, const int* __restrict__ options, int* __restrict__ out,
                                                                        ChunkedScratch s, int vocab) {
   __shared__ union { Listed tokens[FINISH_TOKENS]; DrawQueue queue; } shared;
@@ -834,12 +870,14 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_finish_kernel(const flo
   const bool filtered = o.temperature != 0.f && o.filter;
   // (asked for together: the kernel's time is that of its trips to memory)
   const RowSearch search = s.search[r];
-  const int length = tid < chunks ? s.list_lengths[r * chunks + tid] : 0;
+  const int length = tid < chunks ? s.list_lengths[r * chunks + tid] : 0, listed = s.list_lengths[r * chunks + c];
   const float mx = row_max_of_chunks(s.chunk_max + r * chunks, chunks);
-  const bool unlisted = filtered && search.unlisted != 0;
-  if (c != 0 && !unlisted) return;
+  const bool shared_out = filtered && search.shared_out != 0;
+  if (c != 0 && !shared_out) return;
   if (!filtered) {
-    const Best best = best_of_chunks(s.chunk_best + r * chunks, chunks, best_scratch);
+    Best best{-INFINITY, 0x7fffffff};
+    for (int q = tid; q < chunks; q += SAMPLE_THREADS) best = better(best, s.chunk_best[r * chunks + q]);
+    best = block_best(best, best_scratch);
     if (tid == 0) out[r] = best.index;
     return;
   }
@@ -856,11 +894,6 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_finish_kernel(const flo
     }
     return lists + (size_t)lo * s.list_room + (j - before[lo]);
   };
-  auto draw_one = [&](int i, float x, Best& best) {
-    uint32_t bits[4];
-    philox4x32((uint32_t)(i >> 2), o.counter, 0u, 0u, o.seed_lo, o.seed_hi, bits);
-    draw_token(i, x, (i & 2) ? ((i & 1) ? bits[3] : bits[2]) : ((i & 1) ? bits[1] : bits[0]), mx, best);
-  };
   if (tid == 0) kept_count = 0;
   // where each chunk's list begins among the row's
   const int own_tokens = max(length, 0);
@@ -872,7 +905,7 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_finish_kernel(const flo
   }
   if (lane == 63) sum_of_wave[wave] = upto;
   __syncthreads();
-  int total = 0;
+  int total = 0;  // at most FINISH_TOKENS
   for (int w = 0; w < SAMPLE_THREADS / 64; ++w) {
     const int of_wave = sum_of_wave[w];
     upto += w < wave ? of_wave : 0;
@@ -880,35 +913,34 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_finish_kernel(const flo
   }
   if (tid < chunks) before[tid] = upto - own_tokens;
   __syncthreads();
-  const bool held = total <= FINISH_TOKENS;  // (each thread reads back what it wrote itself)
-  if (held)
-    for (int j = tid; j < total; j += SAMPLE_THREADS) shared.tokens[j] = *listed_at(j);
-  Best best{-INFINITY, 0x7fffffff};
+  for (int j = tid; j < total; j += SAMPLE_THREADS) shared.tokens[j] = *listed_at(j);  // (each thread reads back what it wrote itself)
 #pragma unroll 1
-  for (int level = 1; level <= (unlisted ? 1 : 2); ++level) {  // (one loop: code that runs once is fetched while it runs)
-    clear_tables(tables, level, o);
-    __syncthreads();
-    const int known = level_shift(level - 1), shift = level_shift(level);
-    for (int j = tid; j < total; j += SAMPLE_THREADS) {
-      const float x = (held ? shared.tokens[j] : *listed_at(j)).logit * o.inv_t;
-      const uint32_t key = sort_key(x);
-      if ((key >> known) == (prefix >> known)) add_token(tables, (int)((key >> shift) & (uint32_t)(level_bins(level) - 1)), x, o, mx);
+  for (int level = 1; level <= (shared_out ? 1 : 2); ++level) {  // (one loop: code that runs once is fetched while it runs)
+    if (total > 0) {
+      clear_tables(tables, level, o);
+      __syncthreads();
+      const int known = level_shift(level - 1), shift = level_shift(level);
+      for (int j = tid; j < total; j += SAMPLE_THREADS) {
+        const float x = shared.tokens[j].logit * o.inv_t;
+        const uint32_t key = sort_key(x);
+        if ((key >> known) == (prefix >> known)) add_token(tables, (int)((key >> shift) & (uint32_t)(level_bins(level) - 1)), x, o, mx);
+      }
+      __syncthreads();
     }
-    __syncthreads();
     const size_t base = ((size_t)r * 2 + 1) * SELECT_BINS;
     prefix = digit_of_table(level, o, prefix, mass_limit, above, select, [&](int bin, unsigned int& count, unsigned long long& mass) {
-      table_entry(tables, level, bin, o, count, mass);
-      if (unlisted && o.top_k > 0) count += s.counts[base + bin];
-      if (unlisted && o.use_mass) mass += s.masses[base + bin];
+      if (total > 0) table_entry(tables, level, bin, o, count, mass);
+      if (shared_out && o.top_k > 0) count += s.counts[base + bin];
+      if (shared_out && o.use_mass) mass += s.masses[base + bin];
     });
     __syncthreads();
   }
-  if (!unlisted) {
+  if (!shared_out) {
     // The kept tokens are a part of the listed ones, in no order: gathered in the tables' place, so that few waves work out noise.
     constexpr int ROOM = (int)(sizeof(tables) / sizeof(Listed));
     Listed* kept = reinterpret_cast<Listed*>(&tables);
     for (int j = tid; j < total; j += SAMPLE_THREADS) {
-      const Listed token = held ? shared.tokens[j] : *listed_at(j);
+      const Listed token = shared.tokens[j];
       const float x = token.logit * o.inv_t;
       if (sort_key(x) >= prefix) {
         const int at = atomicAdd(&kept_count, 1);
@@ -917,58 +949,77 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_finish_kernel(const flo
     }
     __syncthreads();
     const bool all = kept_count <= ROOM;
+    Best best{-INFINITY, 0x7fffffff};
     for (int j = tid; j < (all ? kept_count : total); j += SAMPLE_THREADS) {
-      const Listed token = all ? kept[j] : held ? shared.tokens[j] : *listed_at(j);
+      const Listed token = all ? kept[j] : shared.tokens[j];
       const float x = token.logit * o.inv_t;
-      if (sort_key(x) >= prefix) draw_one(token.index, x, best);
+      if (sort_key(x) >= prefix) draw_token(token.index, x, token_bits(token.index, o), mx, best);
     }
     best = block_best(best, best_scratch);
     if (tid == 0) out[r] = best.index;
     return;
   }
-  int q_lo, q_hi;
-  chunk_quads(vocab, c, q_lo, q_hi);
-  Listed* open = s.open + (size_t)r * OPEN_TOKENS;
-  best = draw_in_quads(row, vocab, q_lo, q_hi, o, mx, prefix, shared.queue, [&](int i, float v, uint32_t key) {
+  unsigned int* open_counts = tables.counts;
+  unsigned long long* open_best = tables.masses;
+  static_assert(OPEN_BINS == SAMPLE_THREADS && OPEN_BINS <= SELECT_BINS, "an entry each, in the tables' place");
+  open_counts[tid] = 0u;
+  open_best[tid] = 0ull;
+  __syncthreads();
+  OpenRun run{0ull, 0u, 0u};
+  auto take_open = [&](int i, float x, uint32_t bits) {
+    const uint32_t key = sort_key(x);
     if ((key >> 10) != (prefix >> 10)) return false;
-    const unsigned int at = __hip_atomic_fetch_add(&s.search[r].open, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (at < OPEN_TOKENS) store_shared_pair(open + at, pair_bits(Listed{v, i}));
+    const unsigned int bin = key & (OPEN_BINS - 1);
+    const unsigned long long score = in_order(Best{token_score(x, bits, mx), i});
+    if (bin != run.bin) {
+      settle(run, open_counts, open_best);
+      run = OpenRun{0ull, 0u, bin};
+    }
+    run.best = max(run.best, score);
+    ++run.count;
     return true;
-  });
-  best = block_best(best, best_scratch);
+  };
+  Best best{-INFINITY, 0x7fffffff};
+  if (listed != NOT_LISTED) {
+    const Listed* own = lists + (size_t)c * s.list_room;
+    for (int j = tid; j < (listed >= 0 ? listed : ~listed); j += SAMPLE_THREADS) {
+      const Listed token = own[j];
+      const float x = token.logit * o.inv_t;
+      if (sort_key(x) < prefix) continue;
+      const uint32_t bits = token_bits(token.index, o);
+      if (!take_open(token.index, x, bits)) draw_token(token.index, x, bits, mx, best);
+    }
+  } else {
+    int q_lo, q_hi;
+    chunk_quads(vocab, c, q_lo, q_hi);
+    best = draw_in_quads(row, vocab, q_lo, q_hi, o, mx, prefix, shared.queue, take_open);
+  }
+  settle(run, open_counts, open_best);
+  best = block_best(best, best_scratch);  // (and a barrier behind the tables)
   // (fences that write back and drop whole caches, in every wave, took 40 to 70 us here: what the last workgroup reads goes past them)
+  const size_t own_bin = (size_t)r * OPEN_BINS + tid;
+  const unsigned int own_count = open_counts[tid];
+  if (own_count != 0u) {
+    add_shared(s.open_counts + own_bin, own_count);
+    max_shared(s.open_best + own_bin, open_best[tid]);
+  }
+  if (tid == 0 && best.index != 0x7fffffff) max_shared(&s.search[r].best, in_order(best));
   wait_for_stores();
   __syncthreads();
-  if (tid == 0) {
-    store_shared_pair(s.chunk_best + r * chunks + c, pair_bits(best));
-    wait_for_stores();
-    last = __hip_atomic_fetch_add(&s.search[r].drawn, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == (unsigned int)chunks ? 1 : 0;
-  }
+  if (tid == 0) last = __hip_atomic_fetch_add(&s.search[r].drawn, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == (unsigned int)chunks ? 1 : 0;
   __syncthreads();
   if (last == 0) return;
-  // The open tokens, a thread each; where there are more than their list holds they are found again in the row, for each of the two uses.
-  const unsigned int found = __hip_atomic_load(&s.search[r].open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  static_assert(OPEN_TOKENS <= SAMPLE_THREADS, "a thread each");
-  const Listed mine = pair_of_bits<Listed>(tid < min(found, (unsigned int)OPEN_TOKENS) ? load_shared_pair(open + tid) : 0ull);
-  clear_tables(tables, 2, o);
-  __syncthreads();
-  auto for_each_open = [&](auto f) {
-    if (found <= OPEN_TOKENS) {
-      if (tid < found) f(mine.index, mine.logit * o.inv_t);
-    } else {
-      for_each_in_quads(row, vocab, 0, (vocab + 3) / 4, [&](int i, float v) {
-        if ((sort_key(v * o.inv_t) >> 10) == (prefix >> 10)) f(i, v * o.inv_t);
-      });
-    }
-  };
-  for_each_open([&](int, float x) { add_token(tables, (int)(sort_key(x) & (uint32_t)(level_bins(2) - 1)), x, o, mx); });
-  __syncthreads();
-  prefix = digit_of_table(2, o, prefix, mass_limit, above, select, [&](int bin, unsigned int& count, unsigned long long& mass) { table_entry(tables, 2, bin, o, count, mass); });
-  best = Best{-INFINITY, 0x7fffffff};
-  for_each_open([&](int i, float x) {
-    if (sort_key(x) >= prefix) draw_one(i, x, best);
+  const size_t bin_of_thread = (size_t)r * OPEN_BINS + (OPEN_BINS - 1 - tid);
+  const unsigned int open_count = load_shared(s.open_counts + bin_of_thread);
+  const Best of_bin = of_order(load_shared(s.open_best + bin_of_thread));
+  best = of_order(tid == 0 ? load_shared(&s.search[r].best) : 0ull);
+  const uint32_t own_key = prefix | (uint32_t)(OPEN_BINS - 1 - tid);
+  prefix = digit_of_table(2, o, prefix, mass_limit, above, select, [&](int, unsigned int& count, unsigned long long& mass) {
+    count = open_count;
+    if (o.use_mass && open_count != 0u) mass = open_count * fixed_point_mass(expf(value_of_key(own_key) - mx));  // (the entry's tokens are all alike)
   });
-  best = better(block_best(best, best_scratch), best_of_chunks(s.chunk_best + r * chunks, chunks, best_scratch));
+  if (own_key >= prefix) best = better(best, of_bin);
+  best = block_best(best, best_scratch);
   if (tid == 0) out[r] = best.index;
 }
 
@@ -989,8 +1040,7 @@ __global__ void __launch_bounds__(SAMPLE_THREADS) sample_chunk_draw_kernel(const
   int q_lo, q_hi;
   chunk_quads(vocab, c, q_lo, q_hi);
   const float mx = row_max_of_chunks(s.chunk_max + r * chunks, chunks);
-  const Best best = block_best(draw_in_quads(logits + (size_t)r * vocab, vocab, q_lo, q_hi, o, mx, 0u, queue, [](int, float, uint32_t) { return false; }), best_scratch);
-  if (threadIdx.x == 0) s.chunk_best[r * chunks + c] = best;
+  draw_among_all(logits + (size_t)r * vocab, vocab, q_lo, q_hi, o, mx, queue, best_scratch, s.chunk_best + r * chunks + c);
 }
 
 extern "C" long long velox_sample_chunked_scratch_bytes(int rows, int vocab, int chunks) {
