@@ -1582,7 +1582,7 @@ __global__ void __launch_bounds__(MERGE_THREADS) merge_splits_kernel(const float
 
 // Which kernel portions of prompts take: 0 = chosen by shape; 1 = never the kernel with direct loads; 2 = that kernel
 // wherever it can run, 3 = the same with two sets of waves (for tests and measurements).  In float32 up to 128 channels: 1 = a row
-// tile per wave, 2, 3, 4 = 16, 32, 64 rows whose tiles waves share.
+// tile per wave, 2, 3, 4 = 16, 32, 64 rows whose tiles waves share (heads of 16 channels: 16, of 48: at most 32).
 static int portion_kernel_choice = 0;
 extern "C" void velox_attention_portion_kernel(int choice) { portion_kernel_choice = choice; }
 
@@ -1693,29 +1693,41 @@ static int launch(const void* qkv, int qkv_stride, const void* k_cache, const vo
   if ((rows + 63) / 64 > 65535) return (int)hipErrorInvalidValue;  // (row blocks are the grid's third dimension)
   // float32: a tile of 64 keys under a row tile is 8,192 cycles of matrix instructions on one SIMD, so a step of few workgroups is
   // as long as its longest wave's walk, most of it on compute units whose other waves are done or on none at all.  Waves that share
-  // row tiles shorten that walk, with the same bits, and smaller workgroups spread it: 16 rows by four waves while those are no more
-  // than the compute units, 32 rows by eight waves up to the same count (up to 2 1/4 for one prompt from an empty cache, whose
-  // workgroups get shorter and shorter), 64 rows by eight waves up to two per compute unit.  Measured on MI355X (us, four waves
-  // of a row tile each / 64 rows by eight / 32 rows by eight / 16 rows by four; heads of 128 channels): 12 over 2, 64 tokens 12.4 / 12.1 /
-  // 9.4 / 8.1, 611 tokens 70 / 64 / 44 / 42, 1,024 tokens 108 / 99 / 67 / 68, 64 tokens behind 2,936 keys 305 / 277 / 184 / 159; 28 over 4, 300 tokens 38 /
-  // 36 / 25 / 25, 611 tokens 74 / 65 / 58 / 63, 1,024 tokens 131 / 105 / 135 / 149, 300 tokens behind 1,700 keys 211 / 192 / 218 / 216, 4 x 128
-  // tokens 19.7 / 18.9 / 21.2 / 23.1; 16 over 4, 2,048 tokens 260 / 209 / 269 / 309; 28 over 4, 2 x 600 tokens behind 1,000 keys (2.06 workgroups of 64
-  // rows per compute unit) 311 / 352 / 397 / 427.
+  // row tiles shorten that walk, with the same bits, and smaller workgroups spread it.  What the sharing costs (the barriers of every
+  // key tile, more staging per row, LDS of which fewer workgroups fit on a compute unit) is won back
+  //   by 16 rows and four waves while those workgroups are no more than the compute units (heads of 16 channels: twice as many, and
+  //   nothing else, since their tiles are hardly any work);
+  //   by 32 rows and eight waves up to the same count; for one prompt from an empty cache, whose workgroups get shorter and shorter,
+  //   up to 2 1/4, up to 1 1/4 behind a window of three key tiles and more;
+  //   by 64 rows and eight waves up to one per compute unit (not where two waves cannot halve the channel tiles), for prompts from an
+  //   empty cache up to two (1 5/8 below 512 tokens; no window, or one of three quarters of the keys).
+  // Measured on MI355X, us, a row tile per wave / 16 / 32 / 64 rows.  12 heads of 128 over 2: 64 tokens 12.4 / 8.2 / 9.4 / 12.2, 611 69.8 / 41.8 /
+  // 43.9 / 64, 1,024 108 / 67 / 67 / 99, with a window of 256 39 / 45 / 48 / 37, 64 behind 2,936 keys 305 / 158 / 184 / 277, 2,048 with a window of
+  // 256 62 / 80 / 72 / 70.  28 over 4: 611 73.5 / 63 / 59 / 65, 1,024 131 / 149 / 135 / 105, 300 behind 1,700 keys 210 / 216 / 216 / 191, 16 x 64 19.6 / 30 / 32 /
+  // 23.4.  Heads of 64, 14 over 2: 1,024 64 / 49 / 47 / 61; 32 over 8, 16 x 64 12.5 / 23 / 17 / 13.  Of 48, 12: 1,024 53 / 37 / 45 / 57.  Of 16, 8 over 2: 611
+  // 20.5 / 17.2 / 21.4 / 24.7, 2,048 56 / 58 / 64 / 70.  Over some 600 such steps (heads of 16 to 128 channels, one to sixteen sequences,
+  // windows) none is more than 2% slower than with a row tile per wave.
   int shared_rows = 0;
   if constexpr (sizeof(T) == 4 && D <= 128) {
+    constexpr bool HALVES = D % 32 == 0;  // (two waves have as many channel tiles each)
     const long long units = compute_units(), per_block = (long long)nkv * num_seqs * splits;
-    const bool one_prompt = num_seqs == 1 && max_kv_len <= max_q_len;
     const long long by_16 = (rows + 15) / 16 * per_block, by_32 = (rows + 31) / 32 * per_block, by_64 = (rows + 63) / 64 * per_block;
-    if (by_16 <= units) shared_rows = 16;
-    else if (by_32 <= units || (one_prompt && 4 * by_32 <= 9 * units)) shared_rows = 32;
-    else if (by_64 <= 2 * units) shared_rows = 64;
-    if (portion_kernel_choice > 0) shared_rows = portion_kernel_choice == 1 ? 0 : portion_kernel_choice == 2 ? 16 : portion_kernel_choice == 3 ? 32 : 64;
+    const bool from_empty = max_kv_len <= max_q_len, open = window <= 0 || window >= max_kv_len;
+    const bool triangles = from_empty && max_q_len >= 192 && (open || 4LL * window >= 3LL * max_kv_len);
+    if (by_16 <= (D == 16 ? 2 : 1) * units) shared_rows = 16;
+    else if (D > 16 && (by_32 <= units || (from_empty && num_seqs == 1 && (open || window >= 192) && 4 * by_32 <= (open ? 9 : 5) * units))) shared_rows = 32;
+    else if (D > 16 && D != 48 && 8 * by_64 <= (triangles ? (max_q_len >= 512 ? 16 : 13) : HALVES ? 8 : 0) * units) shared_rows = 64;
+    if (portion_kernel_choice > 0) shared_rows = portion_kernel_choice == 1 ? 0 : portion_kernel_choice == 2 || D == 16 ? 16 : portion_kernel_choice == 3 || D == 48 ? 32 : 64;
     if (shared_rows > 0) {
       const dim3 grid(num_seqs * splits, nkv, (rows + shared_rows - 1) / shared_rows);
       if (grid.z > 65535u) return (int)hipErrorInvalidValue;
-      const auto kernel = shared_rows == 16   ? paged_attention_kernel<T, BN, 1, 1, 4, 4>
-                          : shared_rows == 32 ? paged_attention_kernel<T, BN, 1, 1, 8, 4>
-                                              : paged_attention_kernel<T, BN, 1, 1, 8, 2>;
+      auto kernel = paged_attention_kernel<T, BN, 1, 1, 4, 4>;
+      if constexpr (D > 16) {
+        if (shared_rows == 32) kernel = paged_attention_kernel<T, BN, 1, 1, 8, 4>;
+      }
+      if constexpr (D > 16 && D != 48) {
+        if (shared_rows == 64) kernel = paged_attention_kernel<T, BN, 1, 1, 8, 2>;
+      }
       kernel<<<grid, shared_rows == 16 ? 256 : 512, 0, stream>>>((const T*)qkv, qkv_stride, (const T*)k_cache, (const T*)v_cache, block_tables, table_width,
                                                                  cu_q, kv_lens, (T*)out, part_o, part_lse, nh, nkv, page_shift, scale, window, splits, total_tokens,
                                                                  bias_table, bias_len, sinks, extras);
