@@ -181,6 +181,73 @@ def test_streams_are_mixed_from_to_and_the_norm_reads_their_weighted_sum(streams
         assert float((plain.layer_norm(wrong, norm.weight.double(), 1e-5) - plain.layer_norm(u, norm.weight.double(), 1e-5)).abs().max()) > 0.1
 
 
+class WaitingOps(TorchOps):
+    """Leaves streams unwritten wherever the model lets it, and takes what the kernels take."""
+
+    MAX_STREAMS_BEHIND = 3
+    waited = 0
+
+    def streams_may_begin_unwritten(self, tokens, streams, hidden):
+        return True
+
+    def streams_may_wait(self, residual, terms, weight, streams, held):
+        return held < self.MAX_STREAMS_BEHIND
+
+    def stream_norm(self, residual, terms, scales, mix, out_weights, in_weights, weight, eps, streams, center, out_dtype, rows=None, earlier=(), base=None, settle=True):
+        assert base is None or (base.is_contiguous() and base.data_ptr() % 16 == 0)
+        self.waited += not settle
+        streams_now = residual.clone() if base is None else base.repeat(1, streams)
+        for e_terms, e_scales, e_mix, e_out in earlier:
+            super().stream_norm(streams_now, e_terms, e_scales, e_mix, e_out, None, weight, eps, streams, center, out_dtype)
+        normed = super().stream_norm(streams_now, terms, scales, mix, out_weights, in_weights, weight, eps, streams, center, out_dtype, rows=rows)
+        if settle and len(terms) and rows is None:
+            residual.copy_(streams_now)
+        return normed
+
+
+def _logits_with(tmp_path, ops):
+    folder = write_folder(tmp_path / "A", CONFIGS["A"], seed=2)
+    harness = Harness(folder, ops, torch.float32, "cpu", PAGE_SIZE["A"], 64, max_num_seqs=3, max_num_tokens=128)
+    tokens = prompts(CONFIGS["A"]["vocab"], [23], seed=8)["r0"]
+    return harness, lambda: harness.feed([("r0", tokens, list(range(len(tokens))))], end=["r0"])
+
+
+def test_streams_stay_unwritten_only_behind_parts_whose_outputs_stay(tmp_path, monkeypatch):
+    """A feed-forward and a mixer of a user's own that hand back one buffer again and again: the model writes its streams every
+    time.  A class inherits no answer from one that it extends; the built-in parts' streams wait."""
+    from velox_amd.parts import base
+    from velox_amd.parts.feed_forward import GatedMLP
+    from velox_amd.parts.parallel_mixer import ParallelMixer
+
+    ops = WaitingOps()
+    _, run = _logits_with(tmp_path / "built in", ops)
+    want = run()
+    assert ops.waited > 0
+    buffers = {}
+
+    def in_a_buffer(y):
+        buffer = buffers.setdefault(tuple(y.shape), torch.empty_like(y))
+        return buffer.copy_(y)
+
+    class OneBuffer(GatedMLP):
+        def forward(self, x, ctx, sink=None):
+            return in_a_buffer(super().forward(x, ctx))
+
+    class OneBufferMixer(ParallelMixer):
+        def forward(self, x, ctx, cache, owns_cache=True):
+            y = super().forward(x, ctx, cache, owns_cache)
+            return ScaledSum(tuple(in_a_buffer(t) for t in y.terms[:1]) + y.terms[1:], y.scales)
+
+    for family, kind, part in (("feed_forward", "gated_mlp", OneBuffer), ("mixer", "parallel_mixers", OneBufferMixer)):
+        with monkeypatch.context() as patch:
+            patch.setitem(base._TABLES[family], kind, part)
+            ops = WaitingOps()
+            harness, run = _logits_with(tmp_path / kind, ops)
+            assert any(type(p) is part for p in harness.model.all_parts())
+            torch.testing.assert_close(run(), want, rtol=1e-5, atol=1e-5)
+            assert ops.waited == 0
+
+
 def test_layer_outputs_one_by_one(tmp_path):
     """The sum of the streams after every layer run, from the framework's blocks run one at a time, against the plain model's."""
     harness, config, weights = _harness(tmp_path, "A", seed=5)

@@ -33,6 +33,8 @@ def kv_pages(num_kv_heads: int, head_dim: int, window: Optional[int] = None, kee
 
 
 class AttentionMixer(Mixer):
+    output_stays = True
+
     def __init__(
         self,
         prefix: str,

@@ -330,7 +330,17 @@ class OutputNormSink:
     following: Optional["Norm"] = None
 
 
+def output_stays(part: "Part") -> bool:
+    """Whether what ``part.forward`` returns stays as it is: the part's own class says so, and so do the mixers and feed-forwards inside it."""
+    return bool(type(part).__dict__.get("output_stays", False)) and all(output_stays(c) for c in part.children() if isinstance(c, (Mixer, FeedForward)))
+
+
 class Mixer(Part):
+    # Whether what ``forward`` returns is the caller's for good: no later call writes to it.  Without it the next norm is the last to read it.
+    # Residual streams stay unwritten, and sub-layers' outputs are read again, only in models whose mixers and feed-forwards all say True.
+    # A subclass does not inherit the answer (its ``forward`` may be another one).
+    output_stays = False
+
     def cache_need(self):
         """``PagedNeed``, ``StateNeed`` or None."""
         return None
@@ -346,6 +356,8 @@ class Mixer(Part):
 
 
 class FeedForward(Part):
+    output_stays = False  # (see ``Mixer``)
+
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         """[T, H] -> [T, H], or float32 partial sums [S, T, H] (see ``Mixer.forward``)."""
         raise NotImplementedError

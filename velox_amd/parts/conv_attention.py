@@ -35,6 +35,8 @@ from .base import CompositeNeed, Mixer, Param, PositionEncoding, StateNeed, fuse
 
 
 class ConvAttentionMixer(Mixer):
+    output_stays = True
+
     def __init__(self, prefix: str, hidden_size: int, num_heads: int, num_kv_heads: int, dim: int, vdim: int, scale: float,
                  window: Optional[int] = None, conv_taps: int = 0, qkv_bias: bool = True, out_bias: bool = True,
                  position: Optional[PositionEncoding] = None, names: Tuple[Tuple[str, str], ...] = (), post_norm_eps: Optional[float] = None,

@@ -27,6 +27,8 @@ UNGATED_ACTIVATIONS = ("relu2",)  # activations of a unit without a gate branch
 
 
 class GatedMLP(FeedForward):
+    output_stays = True
+
     def __init__(self, prefix: str, hidden_size: int, intermediate_size: int, activation: str = "silu",
                  names: Tuple[str, str, str] = ("gate_proj.weight", "up_proj.weight", "down_proj.weight")) -> None:
         """``names``: the gate, up and down tensors below the prefix."""
@@ -78,6 +80,8 @@ class PlainMLP(FeedForward):
     by element and ``N(y) = y / sqrt(mean(y^2) + norm_eps)`` over a token's whole row (so it needs the whole row and is a
     kernel of its own between the products).  The activation is float32 with one rounding at the store."""
 
+    output_stays = True
+
     def __init__(self, prefix: str, hidden_size: int, intermediate_size: int, activation: str = "relu2",
                  names: Tuple[str, str] = ("up_proj.weight", "down_proj.weight"), norm_eps: float = 1e-6, coefficients_name: str = "act") -> None:
         """``norm_eps``, ``coefficients_name`` (of the tensor of four numbers): for ``poly_norm`` only."""
@@ -122,6 +126,8 @@ register_part("feed_forward", "plain_mlp", PlainMLP)
 class NoFeedForward(FeedForward):
     """A layer without a feed-forward: ``forward`` gives None and the block adds nothing."""
 
+    output_stays = True
+
     def __init__(self, prefix: str = "") -> None:
         super().__init__(prefix)
 
@@ -141,6 +147,8 @@ class RoutedExperts(FeedForward):
     Tensors: the experts' gate and up matrices are held as one ``[E * 2 F, H]`` tensor (expert after expert, each gate
     rows then up rows), the down matrices as ``[E * H, F]``; ``expert_names(e)`` gives the three names of expert ``e``
     below the prefix."""
+
+    output_stays = True
 
     def __init__(self, prefix: str, hidden_size: int, intermediate_size: int, num_experts: int, top: int, score: str = "sigmoid",
                  renormalize: bool = False, scale_input: bool = True, shared_intermediate_size: Optional[int] = None,

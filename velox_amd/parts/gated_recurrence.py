@@ -21,6 +21,8 @@ from .base import Mixer, Param, StateNeed, fused_rows, register_part, single
 
 
 class GatedRecurrenceMixer(Mixer):
+    output_stays = True
+
     products_in_parts = ("o_weight",)
 
     def __init__(self, prefix: str, hidden_size: int, width: int, shift: float = 0.5, names: Tuple[Tuple[str, str], ...] = ()) -> None:

@@ -42,6 +42,8 @@ _NAMES = {"q": "q.weight", "down": "down.weight", "down_norm": "down_norm.weight
 
 
 class LatentAttentionMixer(Mixer):
+    output_stays = True
+
     products_in_parts = ("out_weight",)
 
     def __init__(self, prefix: str, hidden_size: int, num_heads: int, dim: int, rot_dim: int, vdim: int, kv_rank: int, scale: float,

@@ -62,6 +62,8 @@ _DEFAULT_NAMES = {"q": "q", "k": "k", "v": "v", "o": "o", "beta": "b", "A_log": 
 
 
 class LinearRecurrenceMixer(Mixer):
+    output_stays = True
+
     def __init__(self, prefix: str, hidden_size: int, num_heads: int, num_kv_heads: int, dim: int, vdim: int, norm_eps: float,
                  rule: str = "delta", decay: str = "head", gate: str = "silu", conv_taps: int = 0, unit_qk: bool = False, qkv_silu: bool = False,
                  decay_rank: Optional[int] = None, gate_rank: Optional[int] = None, tau: float = 1.0,
@@ -230,6 +232,8 @@ register_part("mixer", "linear_recurrence", LinearRecurrenceMixer)
 
 
 class GeneralDeltaMixer(Mixer):
+    output_stays = True
+
     products_in_parts = ("o_weight",)
 
     def __init__(self, prefix: str, hidden_size: int, num_heads: int, dim: int, vdim: int, norm_eps: float, decay_rank: int, decay_scale: float = math.exp(-0.5),

@@ -21,7 +21,7 @@ from typing import Dict, List, Optional, Tuple
 import torch
 
 from . import block as _block  # noqa: F401  (registers the built-in arrangement)
-from .base import Embedding, OutputHead, Param, Part, PartSpec, PassInput, StateNeed, UnwrittenStreams, make_part, register_part, single
+from .base import Embedding, OutputHead, Param, Part, PartSpec, PassInput, StateNeed, UnwrittenStreams, make_part, output_stays, register_part, single
 from .norms import StreamNorm
 
 
@@ -239,7 +239,9 @@ class DecoderModel(Part):
         self.pass_input = make_part("pass_input", spec.pass_input.kind, hidden_size=spec.hidden_size, **spec.pass_input.kwargs()) if spec.pass_input is not None else None
         self.schedule = list(spec.schedule)
         readers = [n for block in self.blocks for n in ((block.mixer_norm, block.ff_norm) if type(block) is _block.HyperConnectionBlock else (None,))] + [self.final_norm]
-        self.streams_can_wait = self.pass_input is None and all(type(n) is StreamNorm for n in readers)  # (nothing reads the residual but these)
+        # (nothing reads the residual but these norms, and what they hold on to stays as it is)
+        self.streams_can_wait = (self.pass_input is None and all(type(n) is StreamNorm for n in readers)
+                                 and all(output_stays(part) for block in self.blocks for part in (block.mixer, *((block.feed_forward,) if block.has_feed_forward else ()))))
 
     # -- structure ----------------------------------------------------------------------
     def children(self) -> Tuple[Part, ...]:

@@ -65,6 +65,8 @@ def bias_by_distance(rel: torch.Tensor, far: float) -> torch.Tensor:
 
 
 class NormedAttentionMixer(Mixer):
+    output_stays = True
+
     def __init__(
         self,
         prefix: str,

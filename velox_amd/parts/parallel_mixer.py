@@ -14,6 +14,8 @@ from .base import CompositeNeed, Mixer, NormedSum, Part, PartSpec, ScaledSum, ma
 
 
 class ParallelMixer(Mixer):
+    output_stays = True
+
     def __init__(self, prefix: str, left: PartSpec, right: PartSpec, left_scale: float = 1.0, right_scale: float = 1.0,
                  left_prefix: str = "left.", right_prefix: str = "right.", position=None, position_to: Tuple[bool, bool] = (True, False),
                  output_norm: Optional[PartSpec] = None, output_norm_prefixes: Tuple[str, str] = ("left.out", "right.out")) -> None:

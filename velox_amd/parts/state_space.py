@@ -26,6 +26,8 @@ from .base import Mixer, Param, StateNeed, register_part, single
 
 
 class StateSpaceMixer(Mixer):
+    output_stays = True
+
     products_in_parts = ("o_weight",)
 
     def __init__(self, prefix: str, hidden_size: int, num_heads: int, groups: int, state: int, vdim: int, conv_taps: int, norm_groups: int,
