@@ -2,6 +2,7 @@
 the loader, the cache manager with its state slots, the step function, replay, the scheduler and the entry point are the
 product's.  The yardstick is ``plain_gosulorn`` (whole sequences, no cache, float64)."""
 import copy
+import dataclasses
 import math
 
 import pytest
@@ -246,6 +247,22 @@ def test_streams_stay_unwritten_only_behind_parts_whose_outputs_stay(tmp_path, m
             assert any(type(p) is part for p in harness.model.all_parts())
             torch.testing.assert_close(run(), want, rtol=1e-5, atol=1e-5)
             assert ops.waited == 0
+
+
+def test_streams_begin_unwritten_with_rows_of_any_strides(tmp_path):
+    """What a position encoding makes of the embeddings may be a view: the streams begin with a copy of it that the kernels take."""
+    from velox_amd.parts import PositionEncoding
+
+    class Strided(PositionEncoding):
+        def on_embeddings(self, hidden, ctx):
+            return torch.stack((hidden, hidden), -1)[..., 1]
+
+    ops = WaitingOps()
+    harness, run = _logits_with(tmp_path, ops)
+    want = run()
+    harness.model.positions["strided"] = Strided()
+    harness.model.spec = dataclasses.replace(harness.model.spec, embedding_position="strided")
+    assert torch.equal(run(), want) and ops.waited > 0
 
 
 def test_layer_outputs_one_by_one(tmp_path):

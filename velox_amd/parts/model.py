@@ -330,6 +330,8 @@ class DecoderModel(Part):
         base = self.embedding.forward(token_ids, ctx)
         if self.spec.embedding_position is not None:
             base = self.positions[self.spec.embedding_position].on_embeddings(base, ctx)
+            if not base.is_contiguous() or base.data_ptr() % 16 != 0:
+                base = base.clone(memory_format=torch.contiguous_format)  # (the kernel reads whole rows, 16 bytes at a time)
         return torch.empty((token_ids.shape[0], streams * hidden), dtype=torch.float32, device=base.device), UnwrittenStreams((), base)
 
     def logits(self, residual: torch.Tensor, pending, rows: torch.Tensor, ctx) -> torch.Tensor:
