@@ -265,6 +265,24 @@ def test_streams_begin_unwritten_with_rows_of_any_strides(tmp_path):
     assert torch.equal(run(), want) and ops.waited > 0
 
 
+def test_what_unwritten_streams_hold_is_counted_for_the_pool(tmp_path):
+    """A step's outputs that are read again later: no more of them live at once than the bytes that are kept out of the cache's pool."""
+    ops, live = WaitingOps(), []
+
+    def stream_norm(*args, earlier=(), base=None, **kwargs):
+        held = {t.data_ptr(): t for e in earlier for t in e[0]}
+        live.append(sum(t.numel() * t.element_size() for t in held.values()) + (base.numel() * 4 if base is not None else 0))
+        return WaitingOps.stream_norm(ops, *args, earlier=earlier, base=base, **kwargs)
+
+    ops.stream_norm = stream_norm
+    harness, run = _logits_with(tmp_path, ops)
+    run()
+    assert 23 * 64 * 4 < max(live) <= harness.model.bytes_held(23, torch.float32, ops) == 23 * 64 * (4 + 6 * 4)
+    assert harness.model.bytes_held(23, torch.bfloat16, ops) == 23 * 64 * (4 + 6 * 2) and harness.model.bytes_held(23, torch.float32, TorchOps()) == 0
+    harness.model.streams_can_wait = False
+    assert harness.model.bytes_held(23, torch.float32, ops) == 0
+
+
 def test_layer_outputs_one_by_one(tmp_path):
     """The sum of the streams after every layer run, from the framework's blocks run one at a time, against the plain model's."""
     harness, config, weights = _harness(tmp_path, "A", seed=5)

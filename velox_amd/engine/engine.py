@@ -147,7 +147,8 @@ class Engine:
             probe = CacheManager(needs, config.block_size, 2, config.max_num_seqs, dtype, device, allocate_tensors=False)
             free_bytes, _ = torch.cuda.mem_get_info(device)
             free_bytes += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
-            num_pages = pages_that_fit(probe.bytes_per_page(), free_bytes, config.gpu_memory_utilization, config.kv_cache_reserve_mb * 1024 * 1024)
+            reserve = config.kv_cache_reserve_mb * 1024 * 1024 + model.bytes_held(config.max_num_batched_tokens, dtype, ops)
+            num_pages = pages_that_fit(probe.bytes_per_page(), free_bytes, config.gpu_memory_utilization, reserve)
             wanted = (config.max_num_seqs * max_model_len + config.block_size - 1) // config.block_size + 1
             num_pages = min(num_pages, max(2, wanted))
         cache = CacheManager(needs, config.block_size, num_pages, config.max_num_seqs, dtype, device, max_model_len=max_model_len,

@@ -323,9 +323,7 @@ class DecoderModel(Part):
         """Streams that are not written yet and the row that all of them begin with (``begin`` writes it once per stream); None where
         the kernels gain nothing by it or something else reads the streams."""
         streams, hidden = self.spec.residual_streams, self.spec.hidden_size
-        may_begin = getattr(ctx.ops, "streams_may_begin_unwritten", None)
-        if (streams == 1 or may_begin is None or not may_begin(token_ids.shape[0], streams, hidden) or self.embedding.cache_need() is not None
-                or not self.streams_can_wait):
+        if not self.begins_unwritten(token_ids.shape[0], ctx.ops):
             return None
         base = self.embedding.forward(token_ids, ctx)
         if self.spec.embedding_position is not None:
@@ -333,6 +331,18 @@ class DecoderModel(Part):
             if not base.is_contiguous() or base.data_ptr() % 16 != 0:
                 base = base.clone(memory_format=torch.contiguous_format)  # (the kernel reads whole rows, 16 bytes at a time)
         return torch.empty((token_ids.shape[0], streams * hidden), dtype=torch.float32, device=base.device), UnwrittenStreams((), base)
+
+    def begins_unwritten(self, tokens: int, ops) -> bool:
+        may_begin = getattr(ops, "streams_may_begin_unwritten", None)
+        return (self.spec.residual_streams > 1 and may_begin is not None and may_begin(tokens, self.spec.residual_streams, self.spec.hidden_size)
+                and self.embedding.cache_need() is None and self.streams_can_wait)
+
+    def bytes_held(self, tokens: int, dtype: torch.dtype, ops) -> int:
+        """The most that a step of ``tokens`` tokens holds on to for streams that are not written: the float32 row that they begin with and
+        up to two terms of each sub-layer that they are behind."""
+        if not self.begins_unwritten(tokens, ops):
+            return 0
+        return tokens * self.spec.hidden_size * (4 + 2 * ops.MAX_STREAMS_BEHIND * dtype.itemsize)
 
     def logits(self, residual: torch.Tensor, pending, rows: torch.Tensor, ctx) -> torch.Tensor:
         """Final norm and output head on ``rows`` (int32 [R]) only: float32 [R, vocab]."""
