@@ -468,15 +468,24 @@ def test_all_ways_of_cutting_on_the_gpu(tmp_path, name, dtype):
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["A", "B", "C", "D", "E"])
 def test_whole_models_whose_streams_stay_unwritten(tmp_path, ops, monkeypatch, name, dtype):
-    """Every model with its streams written every fourth time (where rows are a multiple of four channels) and once per sub-layer: the same bits, in whole
-    prompts, portions, and decoded tokens from captured steps."""
+    """Models of several streams (A, C, E) with their streams written every fourth time and once per sub-layer: the same bits, in whole
+    prompts, portions, and decoded tokens from captured steps.  The others (B: no streams, D: one) have nothing that could wait."""
     folder = write_folder(tmp_path / name, CONFIGS[name], seed=2, dtype=dtype)
     requests = prompts(CONFIGS[name]["vocab"], [141, 1, 37, 98], seed=11)
-    trace, results = rc.mixed(requests, seed=5), []
+    trace, results, behind = rc.mixed(requests, seed=5), [], []
+    norm = type(ops).stream_norm
+
+    def counted(self, *args, earlier=(), **kwargs):
+        behind[-1] = max(behind[-1], len(earlier))
+        return norm(self, *args, earlier=earlier, **kwargs)
+
+    monkeypatch.setattr(type(ops), "stream_norm", counted)
     for from_bytes in (1, 1 << 60):
         monkeypatch.setattr(type(ops), "STREAMS_WAIT_FROM_BYTES", from_bytes)
+        behind.append(0)
         replayer = Replayer(folder, dtype, rc.tokens_needed(trace, PAGE_SIZE[name]), block_size=PAGE_SIZE[name], max_live=4, enable_graphs=True)
         results.append(rc.collect(trace, rc.run_trace(replayer, trace), requests))
+    assert behind == [3 if CONFIGS[name].get("streams", 1) > 1 else 0, 0]
     for rid in requests:
         assert torch.equal(results[0][rid], results[1][rid]), rid
 

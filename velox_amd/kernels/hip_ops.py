@@ -1212,8 +1212,9 @@ class HipOps:
     MAX_STREAM_WIDTH = 16384
     MAX_CONV_TAPS = 8
 
-    # Of streams: from 1,024 rows of 4 x 2,048 on.  Keeping the terms costs the host 4 us a sub-layer, and steps of fewer rows wait for the host (eight
-    # layers: 350 rows 1,974 us written every time, 2,043 not, though the kernels take 80 us less; 2,421 rows 4,487 and 4,290).
+    # Of streams: from 1,024 rows of 4 x 2,048 on.  Keeping the terms costs the host 4 us a sub-layer, and steps of fewer rows wait for the host, the
+    # more so the narrower they are.  Eight layers, us, written every time / not: 4 x 2,048, 512 rows 2,060 / 2,213, 850 2,373 / 2,515, 1,000 2,523 / 2,543,
+    # 1,200 2,841 / 2,757, 2,421 4,741 / 4,643; 4 x 4,096, 128 rows 2,559 / 2,702, 256 2,585 / 2,567, 512 3,216 / 3,133, 1,200 5,831 / 5,710.
     STREAMS_WAIT_FROM_BYTES = 32 << 20
 
     def streams_may_wait(self, residual, terms, weight, streams: int, held: int) -> bool:
@@ -2132,9 +2133,9 @@ class HipOps:
         self._check("options", options, torch.int32, (rows, 6))
         out = torch.empty(rows, dtype=torch.int32, device=self.device)
         if chunks is None:
-            # About one workgroup per compute unit: every workgroup of a pass works out the digit before its own from the
-            # row's tables again, so more chunks than fill the GPU cost more than they save (64 rows of 152,064 on
-            # MI355X: 132 us whole, 55 us in 4 chunks, 104 us in 16; 8 rows: 36 us in 16 or 32 chunks, 57 us in 2).
+            # At most one workgroup per compute unit, which holds one at a time; each reads the row's tables for itself, so a second round of
+            # them costs more than the shorter chunks save (152,064 tokens, deviation 3 and top-p 0.9 / 0.4 and 0.95, us on MI355X: 64 rows
+            # 115 / 179 whole, 52 / 82 in 4 chunks, 63 / 112 in 6, 77 / 136 in 16; 8 rows 55 / 106 in 2, 34 / 42 in 18, 33 / 41 in 32).
             chunks = max(1, min(self.num_cus // rows, vocab // 8192, 32))
         if chunks > 1:
             if chunks > 1024 or rows > 65535:
