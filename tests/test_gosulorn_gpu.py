@@ -465,11 +465,45 @@ def test_all_ways_of_cutting_on_the_gpu(tmp_path, name, dtype):
                 torch.testing.assert_close(results[label][rid], results["whole"][rid], rtol=1e-4, atol=3e-5 * max(1.0, float(expected[rid].abs().max())))
 
 
+@pytest.mark.parametrize("streams,dtype,two", [(2, torch.float32, True), (2, torch.float32, False), (2, torch.bfloat16, True), (3, torch.float32, True), (4, torch.bfloat16, False)])
+def test_streams_stay_unwritten_only_where_that_is_no_slower(ops, streams, dtype, two):
+    """Sixteen sub-layers' norms over 4,096 rows of 4,096 (every second output a sum of two): as the norms choose, within 6% of writing the streams
+    every time, what two timings of the same kernels may differ by.  The same bits in the end."""
+    from velox_amd.kernels.measure import time_in_graph
+    from velox_amd.parts import ScaledSum, StreamUpdate, make_part
+    from velox_amd.parts.base import UnwrittenStreams
+
+    class Ctx:
+        pass
+
+    Ctx.ops, Ctx.dtype = ops, dtype
+    tokens, hidden = 4096, 4096
+    draw = lambda *shape: torch.randn(shape, device="cuda")  # noqa: E731
+    norm = make_part("norm", "stream_norm", prefix="n", hidden_size=hidden, eps=1e-5, weight_name="", streams=streams, center=True)
+    norm.weight = 1 + 0.1 * draw(hidden)
+    base, residual = draw(tokens, hidden), torch.empty((tokens, streams * hidden), device="cuda")
+    mix, out, into = torch.eye(streams, device="cuda") + 0.02 * draw(streams, streams), 1 + 0.02 * draw(streams), 1 / streams + 0.02 * draw(streams)
+    ys = [tuple((0.1 * draw(tokens, hidden)).to(dtype) for _ in range(2 if two and q % 2 == 0 else 1)) for q in range(16)]
+
+    def walk(waits):
+        pending = UnwrittenStreams((), base) if waits else None
+        for y in ys:
+            normed, left = norm.read_streams(residual, pending, into, Ctx) if waits else (norm.forward_streams(residual, pending, into, Ctx), None)
+            pending = StreamUpdate(ScaledSum(y, (0.8, 1.1)) if len(y) > 1 else y[0], mix, out, left)
+        return normed
+
+    residual.copy_(base.repeat(1, streams))
+    want = walk(False)
+    assert torch.equal(walk(True), want)
+    times = {waits: time_in_graph(lambda: walk(waits), launches=1) for waits in (False, True)}
+    assert times[True] <= 1.06 * times[False], times
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["A", "B", "C", "D", "E"])
 def test_whole_models_whose_streams_stay_unwritten(tmp_path, ops, monkeypatch, name, dtype):
-    """Models of several streams (A, C, E) with their streams written every fourth time and once per sub-layer: the same bits, in whole
-    prompts, portions, and decoded tokens from captured steps.  The others (B: no streams, D: one) have nothing that could wait."""
+    """Models of several streams (A: three; C and E: two, which wait behind bfloat16 terms alone) with their streams written every fourth time and once per
+    sub-layer: the same bits, in whole prompts, portions, and decoded tokens from captured steps.  B (no streams) and D (one) have nothing that could wait."""
     folder = write_folder(tmp_path / name, CONFIGS[name], seed=2, dtype=dtype)
     requests = prompts(CONFIGS[name]["vocab"], [141, 1, 37, 98], seed=11)
     trace, results, behind = rc.mixed(requests, seed=5), [], []
@@ -485,7 +519,8 @@ def test_whole_models_whose_streams_stay_unwritten(tmp_path, ops, monkeypatch, n
         behind.append(0)
         replayer = Replayer(folder, dtype, rc.tokens_needed(trace, PAGE_SIZE[name]), block_size=PAGE_SIZE[name], max_live=4, enable_graphs=True)
         results.append(rc.collect(trace, rc.run_trace(replayer, trace), requests))
-    assert behind == [3 if CONFIGS[name].get("streams", 1) > 1 else 0, 0]
+    streams = CONFIGS[name].get("streams", 1)
+    assert behind == [3 if streams > 2 or (streams == 2 and dtype == "bfloat16") else 0, 0]
     for rid in requests:
         assert torch.equal(results[0][rid], results[1][rid]), rid
 

@@ -1218,8 +1218,11 @@ class HipOps:
     STREAMS_WAIT_FROM_BYTES = 32 << 20
 
     def streams_may_wait(self, residual, terms, weight, streams: int, held: int) -> bool:
-        """Whether ``stream_norm`` should leave the streams unwritten (``settle=False``) with ``held`` updates unwritten already."""
-        return (held < self.MAX_STREAMS_BEHIND and streams <= self.MAX_UNWRITTEN_STREAMS and residual.numel() * 4 >= self.STREAMS_WAIT_FROM_BYTES and residual.shape[1] % 4 == 0
+        """Whether ``stream_norm`` should leave the streams unwritten (``settle=False``) with ``held`` updates unwritten already.  Two streams of float32
+        terms are written every time: their terms, read again by the next norms, are as many bytes as the streams are (4,096 rows of 4,096, sixteen
+        sub-layers, us, written every time / not: one term 992 / 1,061, every second a sum of two 1,094 / 1,357; bfloat16 terms 918 / 832 and 971 /
+        972; three streams of float32 terms 1,341 / 1,274 and 1,557 / 1,536, four 1,985 / 1,516 and 2,124 / 1,753)."""
+        return (held < self.MAX_STREAMS_BEHIND and (streams > 2 or all(t.dtype == torch.bfloat16 for t in terms)) and streams <= self.MAX_UNWRITTEN_STREAMS and residual.numel() * 4 >= self.STREAMS_WAIT_FROM_BYTES and residual.shape[1] % 4 == 0
                 and terms[0].dim() == 2 and terms[0].shape[1] % 4 == 0 and all(t.data_ptr() % 16 == 0 for t in (residual, weight, *terms)))
 
     def streams_may_begin_unwritten(self, tokens: int, streams: int, hidden: int) -> bool:
