@@ -789,6 +789,40 @@ def test_decode_behind_more_pages_than_the_streaming_kernel_keeps_ids_of(ops, re
         torch.testing.assert_close(got, want, **t)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nh,nkv,d,page,lens,window", [
+    (28, 4, 128, 16, [1500, 65, 130, 300, 1, 700, 16, 17], None),  # some in several parts, some in one
+    (28, 4, 128, 16, [3000] + [20] * 70, None),  # more sequences than a wave has lanes, one far longer
+    (6, 2, 64, 4, [9000, 77, 8300, 5, 500, 31, 32, 33], None),  # more page ids than a part has room for
+    (4, 2, 16, 4, [900, 1, 1, 1, 250, 128, 129, 127], 200),  # a window bounds what a sequence's share is
+    (32, 8, 64, 64, [640] * 9, None),  # all alike
+    (3, 1, 256, 8, [2000 - 120 * b for b in range(16)], None),
+])
+def test_decoded_tokens_whose_keys_are_shared_out(ops, ref, dtype, nh, nkv, d, page, lens, window):
+    """Single tokens behind unequal contexts, their keys shared out over the workgroups by how many each sequence has: the
+    reference's results, the same bits again (the counters of arrivals are left at zero), and those of the sequences in another
+    order as far as the parts they are cut in are the same."""
+    from velox_amd.engine.batch import Workspace
+
+    assert d * (4 if dtype == torch.float32 else 2) > 512 or ops.shares_keys(len(lens), nkv)
+    case = _attention_case(dtype, nh, nkv, d, page, [(1, n) for n in lens], seed=d + len(lens))
+    workspace = Workspace(torch.device("cuda"))
+
+    def run(case, **more):
+        return ops.paged_attention(case["qkv"], nh, nkv, d, case["k_cache"], case["v_cache"], page, case["tables"], case["cu"], case["kv"], 1, case["max_kv"],
+                                   1.0 / math.sqrt(d), window, True, workspace, uneven=True, **more).float()
+
+    got = run(case)
+    want = _run_attention(ref, case, nh, nkv, d, page, window=window)
+    torch.testing.assert_close(got, want, **(dict(rtol=1e-4, atol=1e-5) if dtype == torch.float32 else dict(rtol=2e-2, atol=2e-2)))
+    if "attention_arrivals" in workspace.addresses():
+        assert not workspace.get("attention_arrivals", len(lens) * nkv).any()
+    assert torch.equal(run(case), got)
+    order = torch.randperm(len(lens), generator=torch.Generator().manual_seed(1)).cuda()
+    moved = dict(case, qkv=case["qkv"][order].contiguous(), tables=case["tables"][order].contiguous(), kv=case["kv"][order].contiguous())
+    assert torch.equal(run(moved), got[order])
+
+
 def test_far_key_among_hundreds_is_found(ops):
     # one key far back matches the query strongly: the output must be (nearly) that key's value
     nh, nkv, d, page = 4, 2, 64, 16

@@ -1296,13 +1296,89 @@ template <> struct KeyOps<bf16_t, true> {
   }
 };
 
-template <typename T, int DEPTH, int WAVES>
+// How a decode step's keys are shared out by their number (UNEVEN below).  A workgroup gets some 40 GB/s from memory and no more, so a step
+// whose sequences are of unequal length is as long as its longest workgroup's walk.  A sequence therefore takes as many workgroups per KV head
+// as its part of the step's key tiles is of `share` (the compute units over the KV heads), with at least SHARE_TILES tiles each: what a
+// workgroup costs before its first tile is in is as long as eight tiles take.  From SHARE_UP on it is one more: with more than one workgroup on
+// some compute units those decide (57 sequences of 65 to 1,500 keys, 28 heads over 4: in equal numbers of splits 24.2 us, shared out with
+// 0.75 to 2 workgroups per compute unit 20.7, 19.1, 21.6, 20.4, 19.1; 23 of 100 to 2,000: 20.0 and 13.2, 12.7, 17.3, 16.3, 16.3; 8 of 4,096
+// 19.0 and 18.1, 18.4, 24.4, 22.8, 21.9).  Sequences of less than half a share come last, beside the workgroups that are there
+// (in the order of the sequences 57: 23.7, 48: 21.1 instead of 17.7).
+// Item `item` of the step (uniform over the workgroup; the whole wave takes part) is split `split` of `used` of sequence `b`, which has `kv_len` keys;
+// b < 0: there are not that many.  There are at most num_seqs * most + share items, `most` being what the room for page ids asks of the
+// longest sequence.
+constexpr bool SHARES_KEYS = !BIASED && !KEEPS && !CAPPED && !GATED;
+constexpr int SHARE_TILES = 8, SHARE_MOST = 32;
+constexpr float SHARE_UP = 0.75f, SHARE_SMALL = 0.5f;
+struct SharedItem { int b, split, used, kv_len; };
+
+// v plus those of the lanes before (__shfl goes through LDS: with it the search below took 1.0 us of a launch, not 0.3)
+__device__ __forceinline__ int sum_up_to_lane(int v) {
+#define VELOX_ADD_SHIFTED(CONTROL, ROWS) v += __builtin_amdgcn_update_dpp(0, v, CONTROL, ROWS, 0xf, false)
+  VELOX_ADD_SHIFTED(0x111, 0xf);  // from 1, 2, 4 and 8 lanes down in a row of 16,
+  VELOX_ADD_SHIFTED(0x112, 0xf);
+  VELOX_ADD_SHIFTED(0x114, 0xf);
+  VELOX_ADD_SHIFTED(0x118, 0xf);
+  VELOX_ADD_SHIFTED(0x142, 0xa);  // from the end of the row before, into the second and the fourth,
+  VELOX_ADD_SHIFTED(0x143, 0xc);  // from the middle, into the upper half
+#undef VELOX_ADD_SHIFTED
+  return v;
+}
+
+template <typename TilesOf>
+__device__ __forceinline__ SharedItem shared_item(const int* kv_lens, int num_seqs, int share, int tiles_room, int item, TilesOf tiles_of) {
+  const int lane = threadIdx.x & 63;
+  auto len_at = [&](int b) { return kv_lens[min(b, num_seqs - 1)]; };
+  auto tiles_at = [&](int b, int len) { return b < num_seqs ? max(1, tiles_of(len)) : 0; };
+  const int len0 = len_at(lane), tiles0 = tiles_at(lane, len0);
+  int total = tiles0;
+  for (int b = 64 + lane; b - lane < num_seqs; b += 64) total += tiles_at(b, len_at(b));
+  total = __builtin_amdgcn_readlane(sum_up_to_lane(total), 63);
+  const float per_tile = (float)share / (float)total, per_room = 1.f / (float)tiles_room;
+  int before = 0;
+  for (int small = 0; small < 2; ++small)
+    for (int base = 0; base < num_seqs; base += 64) {
+      const int len = base == 0 ? len0 : len_at(base + lane), tiles = base == 0 ? tiles0 : tiles_at(base + lane, len);
+      const float part = (float)tiles * per_tile;
+      const int fair = min(min((int)(part + (1.f - SHARE_UP)), tiles / SHARE_TILES), SHARE_MOST);
+      const int used = tiles == 0 || (part < SHARE_SMALL) != (small != 0) ? 0 : max(max(1, fair), (int)((float)(tiles - 1) * per_room) + 1);
+      const int upto = sum_up_to_lane(used);
+      const uint64_t holds = __ballot(before + upto > item);
+      if (holds != 0) {
+        const int at = __ffsll((unsigned long long)holds) - 1;
+        const int own = __builtin_amdgcn_readlane(used, at);
+        return SharedItem{base + at, item - (before + __builtin_amdgcn_readlane(upto, at) - own), own, __builtin_amdgcn_readlane(len, at)};
+      }
+      before += __builtin_amdgcn_readlane(upto, 63);
+    }
+  return SharedItem{-1, 0, 0, 0};
+}
+
+// What other workgroups of the same kernel read or have left: past the caches that only some of the card's compute units share.
+__device__ __forceinline__ void store_shared(float* p, const float4_t& v) {
+  typedef unsigned long long pair_t;
+  typedef pair_t two_t __attribute__((ext_vector_type(2)));
+  const two_t bits = __builtin_bit_cast(two_t, v);
+  __hip_atomic_store(reinterpret_cast<pair_t*>(p), bits[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(reinterpret_cast<pair_t*>(p) + 1, bits[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float4_t load_shared_four(const float* p) {
+  typedef unsigned long long pair_t;
+  typedef pair_t two_t __attribute__((ext_vector_type(2)));
+  pair_t* q = reinterpret_cast<pair_t*>(const_cast<float*>(p));
+  const two_t bits = {__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
+  return __builtin_bit_cast(float4_t, bits);
+}
+
+// UNEVEN: see shared_item; the grid is (items, kv heads), `splits` is the share, part_o and part_lse have a row per item, and the last
+// workgroup of a (sequence, KV head) to arrive merges them (arrivals: [sequence][kv head], zero before and after the launch).
+template <typename T, int DEPTH, int WAVES, bool UNEVEN = false>
 __global__ void __launch_bounds__(64 * WAVES) decode_attention_kernel(
     const T* __restrict__ qkv, int qkv_stride, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
     const int* __restrict__ block_tables, int table_width, const int* __restrict__ kv_lens,
     T* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_lse,
     int nh, int nkv, int page_shift, float scale, int window, int splits, int total_tokens, const float* __restrict__ bias_table, int bias_len,
-    const float* __restrict__ sinks, const Extras extras) {
+    const float* __restrict__ sinks, const Extras extras, int* __restrict__ arrivals) {
   constexpr int NC = D / 16;
   constexpr int NCW = (NC + WAVES - 1) / WAVES;
   typedef KeyOps<T, sizeof(T) == 2 && D % 32 == 0> KO;
@@ -1315,9 +1391,21 @@ __global__ void __launch_bounds__(64 * WAVES) decode_attention_kernel(
   const int lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, i = lane & 15;
   const int group = nh / nkv;
-  const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  const int kvh = UNEVEN ? blockIdx.x : blockIdx.y;
+  int split = blockIdx.x, b = blockIdx.z, kv_len;
   const int page_size = 1 << page_shift;
-  const int kv_len = kv_lens[b];
+  if constexpr (UNEVEN) {
+    const SharedItem found = shared_item(kv_lens, total_tokens, splits, ((DECODE_PAGE_IDS - 2) << page_shift) / 16, blockIdx.y, [&](int len) {
+      return (len - KeyTiles::of<16>(len - window, window, 0, page_shift).n_begin + 15) / 16;
+    });
+    if (found.b < 0) return;  // (uniform over the workgroup)
+    b = found.b;
+    split = found.split;
+    splits = found.used;
+    kv_len = found.kv_len;
+  } else {
+    kv_len = kv_lens[b];
+  }
   const int pos = kv_len - 1;
   const bool row_ok = i < group;
   const int head = kvh * group + (row_ok ? i : 0);
@@ -1508,14 +1596,14 @@ __global__ void __launch_bounds__(64 * WAVES) decode_attention_kernel(
     weight[w] = (mw == -INFINITY) ? 0.f : softmax_exp<T>(mw - m_ref);
     l_tot += weight[w] * l_all[w * 16 + i];
   }
-  if (!row_ok) return;
+  if (!UNEVEN && !row_ok) return;  // (UNEVEN: all threads meet again below)
   if (sinks != nullptr && splits == 1 && l_tot > 0.f) l_tot += softmax_exp<T>(sinks[head] - m_ref);  // (see the general kernel)
   const float inv = l_tot > 0.f ? 1.f / l_tot : 1.f;
-  const size_t slot = ((size_t)split * total_tokens + b) * nh + head;
+  const size_t slot = (UNEVEN ? (size_t)blockIdx.y : (size_t)split * total_tokens + b) * nh + head;
 #pragma unroll
   for (int cc = 0; cc < NCW; ++cc) {
     const int c = wave + WAVES * cc;  // this wave writes channel blocks wave, wave + WAVES, ...
-    if (c >= NC) break;
+    if (c >= NC || (UNEVEN && !row_ok)) break;
     float4_t sum = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) sum += acc_all[(w * NC + c) * 64 + lane] * weight[w];
@@ -1525,11 +1613,64 @@ __global__ void __launch_bounds__(64 * WAVES) decode_attention_kernel(
       if constexpr (GATED) sum = sum * gate_of<T>(extras, (size_t)b, head, 16 * c + 4 * g);
 #pragma unroll
       for (int j = 0; j < 4; ++j) dst[j] = from_f32<T>(sum[j]);
+    } else if constexpr (UNEVEN) {
+      store_shared(part_o + slot * D + 16 * c + 4 * g, sum);
     } else {
       *reinterpret_cast<float4_t*>(part_o + slot * D + 16 * c + 4 * g) = sum;
     }
   }
-  if (splits > 1 && wave == 0 && g == 0) part_lse[slot] = l_tot > 0.f ? m_tot + logf(l_tot) : -INFINITY;
+  const float lse = l_tot > 0.f ? m_tot + logf(l_tot) : -INFINITY;
+  if constexpr (!UNEVEN) {
+    if (splits > 1 && wave == 0 && g == 0) part_lse[slot] = lse;
+  } else {
+    if (splits == 1) return;
+    if (wave == 0 && g == 0 && row_ok) __hip_atomic_store(part_lse + slot, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have arrived
+    __syncthreads();
+    int* here = arrivals + b * nkv + kvh;
+    if (tid == 0) page_ids[0] = __hip_atomic_fetch_add(here, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (page_ids[0] != splits - 1) return;
+    if (tid == 0) __hip_atomic_store(here, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // The merge, a thread per head and four channels: up to MERGE_ROUND splits' log-sums and outputs are asked for together.
+    constexpr int QUADS = D / 4, MERGE_ROUND = 8;
+    const size_t first = (size_t)blockIdx.y - split;
+    for (int at = tid; at < group * QUADS; at += 64 * WAVES) {
+      const int h = kvh * group + at / QUADS, channel = at % QUADS * 4;
+      const float* parts = part_o + (first * nh + h) * D + channel;
+      const float* sums = part_lse + first * nh + h;
+      float mx = -INFINITY, denom = 0.f;
+      float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
+      for (int s0 = 0; s0 < splits; s0 += MERGE_ROUND) {
+        float logs[MERGE_ROUND];
+        float4_t o[MERGE_ROUND];
+#pragma unroll
+        for (int j = 0; j < MERGE_ROUND; ++j) {
+          const int s = min(s0 + j, splits - 1);
+          logs[j] = __hip_atomic_load(const_cast<float*>(sums + (size_t)s * nh), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          o[j] = load_shared_four(parts + (size_t)s * nh * D);
+        }
+        float top = mx;
+#pragma unroll
+        for (int j = 0; j < MERGE_ROUND; ++j) top = s0 + j < splits ? fmaxf(top, logs[j]) : top;
+        const float safe = top == -INFINITY ? 0.f : top, old = mx == -INFINITY ? 0.f : expf(mx - safe);
+        denom *= old;
+        acc = acc * old;
+        mx = top;
+#pragma unroll
+        for (int j = 0; j < MERGE_ROUND; ++j) {
+          const float weight = s0 + j < splits && logs[j] != -INFINITY ? expf(logs[j] - safe) : 0.f;
+          denom += weight;
+          acc += o[j] * weight;
+        }
+      }
+      if (sinks != nullptr && mx != -INFINITY) denom += expf(sinks[h] - mx);
+      const float4_t result = acc * (1.f / (denom > 0.f ? denom : 1.f));
+      T* dst = out + ((size_t)b * nh + h) * D + channel;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dst[j] = from_f32<T>(result[j]);
+    }
+  }
 }
 
 // out[token, head, :] = sum_s w_s * o_s / sum_s w_s,  w_s = exp(lse_s - max_s lse_s); a sink adds exp(sink - max_s lse_s)
@@ -1603,9 +1744,23 @@ template <typename T>
 static int launch(const void* qkv, int qkv_stride, const void* k_cache, const void* v_cache, const int* block_tables, int table_width,
                   const int* cu_q, const int* kv_lens, void* out, float* part_o, float* part_lse, int num_seqs, int total_tokens,
                   int max_q_len, int max_kv_len, int nh, int nkv, int page_shift, float scale, int window, int splits, int first_token,
-                  const float* bias_table, int bias_len, const float* sinks, const Extras& extras, hipStream_t stream) {
+                  const float* bias_table, int bias_len, const float* sinks, const Extras& extras, int* arrivals, int share, hipStream_t stream) {
   constexpr int BN = tile_keys<T>();
   const int group = nh / nkv;
+  if (arrivals != nullptr) {  // (asked for only where the streaming kernel takes the step; items: see shared_item)
+    if constexpr (SHARES_KEYS && sizeof(T) * D <= 512) {
+      if (max_q_len != 1 || total_tokens != num_seqs || first_token != 0 || group > 16 || page_shift < 2 || share < 1) return -1;
+      const int room = ((DECODE_PAGE_IDS - 2) << page_shift) / 16, tiles = (max_kv_len + 15) / 16;
+      const long long items = (long long)num_seqs * ((tiles + room - 1) / room) + share;
+      if (items > 65535) return -1;
+      constexpr int DEPTH = sizeof(T) * D <= 256 ? 3 : 2;
+      decode_attention_kernel<T, DEPTH, 4, true><<<dim3(nkv, (unsigned)items), 256, 0, stream>>>(
+          (const T*)qkv, qkv_stride, (const T*)k_cache, (const T*)v_cache, block_tables, table_width, kv_lens, (T*)out, part_o, part_lse,
+          nh, nkv, page_shift, scale, window, share, total_tokens, bias_table, bias_len, sinks, extras, arrivals);
+      return (int)hipGetLastError();
+    }
+    return -1;
+  }
   // the streaming kernel keeps the page ids of a split's keys in LDS: they have to fit
   const int keys_per_split = (((max_kv_len + 15) / 16 + splits - 1) / splits) * 16;
   const bool ids_fit = (keys_per_split >> page_shift) + 2 + (KEEPS ? ((extras.keep_first + 15) / 16 * 16 >> page_shift) + 1 : 0) <= DECODE_PAGE_IDS;
@@ -1616,7 +1771,7 @@ static int launch(const void* qkv, int qkv_stride, const void* k_cache, const vo
     constexpr int DEPTH = sizeof(T) * D <= 256 ? 3 : 2;
     decode_attention_kernel<T, DEPTH, 4><<<dim3(splits, nkv, num_seqs), 256, 0, stream>>>(
         (const T*)qkv, qkv_stride, (const T*)k_cache, (const T*)v_cache, block_tables, table_width, kv_lens, (T*)out, part_o, part_lse,
-        nh, nkv, page_shift, scale, window, splits, total_tokens, bias_table, bias_len, sinks, extras);
+        nh, nkv, page_shift, scale, window, splits, total_tokens, bias_table, bias_len, sinks, extras, nullptr);
     int status = (int)hipGetLastError();
     if (status != 0 || splits == 1) return status;
     merge_splits_kernel<T><<<dim3(total_tokens, nh), MERGE_THREADS, 0, stream>>>(part_o, part_lse, (T*)out, nh, splits, total_tokens, 0, sinks, extras);
@@ -1787,12 +1942,14 @@ extern "C" int velox_attention_options() { return (BIASED ? 1 : 0) | (KEEPS ? 2 
 // part_o: float32 [splits, total_tokens, nh, D]; part_lse: float32 [splits, total_tokens, nh]; both unused when splits == 1.
 // first_token: the sequences given (cu_q holds rows of qkv and out) cover rows [first_token, total_tokens); a launch for
 // the later sequences of a step passes its first row here so that only those rows are merged.
+// arrivals (int32 [num_seqs, nkv], zero before and after; or nullptr): a decode step whose keys are shared out by their number, see
+// shared_item; `share`: workgroups per KV head, `splits` is not read; part_o and part_lse have a row of nh heads per item.
 extern "C" int velox_paged_attention(const void* qkv, int qkv_stride, const void* k_cache, const void* v_cache,
                                      const int* block_tables, int table_width, const int* cu_q, const int* kv_lens, void* out,
                                      float* part_o, float* part_lse, int num_seqs, int total_tokens, int max_q_len, int max_kv_len,
                                      int nh, int nkv, int page_shift, float scale, int window, int splits, int first_token, int dtype,
                                      const float* bias_table, int bias_len, const float* sinks, int keep_first, float softcap, const void* gate,
-                                     int gate_stride, int gate_channels, hipStream_t stream) {
+                                     int gate_stride, int gate_channels, int* arrivals, int share, hipStream_t stream) {
   // keep_first: read by a build for kept keys; softcap: by one for capped scores; gate (rows of the queries' type), its stride and
   // channels per head (0: one number per head): by one for gated outputs; each must be given exactly to the build that reads it.
   // sinks: float32 [nh] or nullptr; exp(sinks[h]) joins the softmax's denominator of every row of head h (no key, no value, not scaled)
@@ -1808,7 +1965,7 @@ extern "C" int velox_paged_attention(const void* qkv, int qkv_stride, const void
   if (nh % nkv != 0 || splits < 1 || page_shift < 0 || max_kv_len < 1 || first_token < 0 || first_token >= total_tokens) return -1;
   if (dtype == VELOX_BF16)
     return launch<bf16_t>(qkv, qkv_stride, k_cache, v_cache, block_tables, table_width, cu_q, kv_lens, out, part_o, part_lse, num_seqs,
-                          total_tokens, max_q_len, max_kv_len, nh, nkv, page_shift, scale, window, splits, first_token, bias_table, bias_len, sinks, extras, stream);
+                          total_tokens, max_q_len, max_kv_len, nh, nkv, page_shift, scale, window, splits, first_token, bias_table, bias_len, sinks, extras, arrivals, share, stream);
   return launch<float>(qkv, qkv_stride, k_cache, v_cache, block_tables, table_width, cu_q, kv_lens, out, part_o, part_lse, num_seqs,
-                       total_tokens, max_q_len, max_kv_len, nh, nkv, page_shift, scale, window, splits, first_token, bias_table, bias_len, sinks, extras, stream);
+                       total_tokens, max_q_len, max_kv_len, nh, nkv, page_shift, scale, window, splits, first_token, bias_table, bias_len, sinks, extras, arrivals, share, stream);
 }

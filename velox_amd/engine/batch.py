@@ -43,7 +43,8 @@ class WorkspaceError(RuntimeError):
 
 
 class Workspace:
-    """Scratch tensors by name, kept across steps so their addresses are stable.
+    """Scratch tensors by name, kept across steps so their addresses are stable.  A buffer begins as zeros (counters that their kernels
+    leave at zero need it).
 
     A captured step holds the addresses of the buffers it was captured with, so a buffer must never be replaced once a
     capture may exist.  The runner therefore asks every part what it can need at most (``Part.workspace_needs``),
@@ -65,7 +66,7 @@ class Workspace:
             have = "nothing" if buf is None else f"{buf.numel()} x {buf.dtype}"
             raise WorkspaceError(f"workspace buffer {name!r} holds {have} but {numel} x {dtype} are asked for; captured steps hold its "
                                  "address, so it cannot be replaced (the part that uses it must state this size in workspace_needs)")
-        self._buffers[name] = torch.empty(max(int(numel), 1), dtype=dtype, device=self.device)
+        self._buffers[name] = torch.zeros(max(int(numel), 1), dtype=dtype, device=self.device)
 
     def fix(self) -> None:
         self.fixed = True

@@ -250,7 +250,7 @@ class HipOps:
         if lib is None:
             lib = ctypes.CDLL(build.ensure_attention(head_dim, biased=bool(biased), kept=bool(kept), capped=bool(capped), gated=bool(gated)))
             lib.velox_paged_attention.argtypes = [_P, _I, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _I, _P, _I, _P,
-                                                  _I, _F, _P, _I, _I, _P]
+                                                  _I, _F, _P, _I, _I, _P, _I, _P]
             lib.velox_attention_options.restype = _I
             lib.velox_paged_attention.restype = _I
             lib.velox_attention_head_dim.restype = _I
@@ -1999,12 +1999,28 @@ class HipOps:
         for portion in range(1, max_num_tokens + 1):  # portions of prompts, behind up to max_num_seqs - 1 single tokens
             whole = min(max_num_tokens, portion + max_num_seqs - 1)
             rows = max(rows, whole * self.choose_portion_splits(portion, group, num_kv_heads, max_model_len))
+        for count in range(1, max_num_seqs + 1):  # single tokens whose keys are shared out by their number
+            if self.shares_keys(count, num_kv_heads):
+                rows = max(rows, self._shared_items(count, num_kv_heads, max_model_len, 4))
         return rows * num_heads * head_dim, rows * num_heads
+
+    def shares_keys(self, num_seqs: int, num_kv_heads: int) -> bool:
+        """Whether a decode step's keys are shared out over the workgroups by how many each sequence has (``uneven``), and not each
+        sequence's in equally many splits.  Measured on MI355X (us, equal splits / shared out): 57 sequences of 65 to 1,500 keys, 28 heads over
+        4 24.2 / 19.1, 23 of 100 to 2,000 20.0 / 12.7, one of 30,000 beside 63 of 200 337 / 29, 64 of 4,096 91.7 / 88.5, 64 of 512 16.1 / 16.0;
+        a few sequences have nothing to share and are slowed down by the merge at the kernel's end: 12 heads over 2, one of 60 keys 5.1 /
+        5.4, of 4,096 10.9 / 12.2."""
+        return 16 * num_seqs * num_kv_heads >= self.num_cus
+
+    def _shared_items(self, num_seqs: int, num_kv_heads: int, max_kv_len: int, block_size: int) -> int:
+        """The most workgroups per KV head among which such a step's keys are shared out (a split's page ids fit the kernel's 2,046)."""
+        most = -(-(-(-max_kv_len // 16)) // (2046 * block_size // 16))
+        return num_seqs * most + max(1, self.num_cus // num_kv_heads)
 
     def paged_attention(self, qkv, num_heads, num_kv_heads, head_dim, k_cache, v_cache, block_size, block_tables, cu_q, kv_lens,
                         max_q_len, max_kv_len, scale, window, all_decode, workspace, splits: Optional[int] = None, decode_prefix: int = 0,
                         portions_max_kv_len: Optional[int] = None, distance_bias: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None,
-                        keep_first: int = 0, softcap: Optional[float] = None, gate: Optional[Tuple[torch.Tensor, int, int]] = None):
+                        keep_first: int = 0, softcap: Optional[float] = None, gate: Optional[Tuple[torch.Tensor, int, int]] = None, uneven: bool = False):
         """Attention of every token of the step over its sequence's keys in the cache.  ``decode_prefix``: how many of the
         first sequences bring exactly one token (the engine puts decoded tokens before portions of prompts).  In a mixed
         step those run through the streaming kernel with their keys split over workgroups, the others through the
@@ -2016,7 +2032,8 @@ class HipOps:
         and no value and is not scaled).  ``keep_first`` beside a window: so many first tokens of a sequence are seen whatever the
         window.  ``softcap``: a scaled score ``s`` becomes ``softcap * tanh(s / softcap)`` (before the bias).  ``gate = (source, first column, channels)``:
         head ``h``'s output times ``sigmoid`` of the source's columns, ``channels`` per head (channels beyond are left alone) or one per head
-        with ``channels`` = 0.  (Each of the three has a build of the kernels: ``attention_library``.)"""
+        with ``channels`` = 0.  (Each of the three has a build of the kernels: ``attention_library``.)  ``uneven``: single tokens' keys may be
+        shared out over the workgroups by their number (``shares_keys``); a token's order of additions then depends on the lengths of the others."""
         tokens = qkv.shape[0]
         keep_first = int(keep_first) if window else 0
         gate_at, gate_stride, gate_channels = 0, 0, 0
@@ -2083,7 +2100,18 @@ class HipOps:
             # and out.  cu_q holds absolute rows, so the general kernel takes qkv and out whole; the streaming kernel
             # counts rows from its first sequence and takes the slices.
             row_tiles = (longest * group + 63) // 64
-            if splits is None:
+            part_o = part_lse = arrivals = None
+            share = 0
+            if (uneven and splits is None and decode_only and workspace is not None and distance_bias is None and softcap is None and gate is None
+                    and not keep_first and block_size >= 4 and group <= 16 and qkv.element_size() * head_dim <= 512 and self.shares_keys(count, num_kv_heads)):
+                share, splits = max(1, self.num_cus // num_kv_heads), 1
+                items = self._shared_items(count, num_kv_heads, int(max_kv_len), block_size)
+                if items > 65535:
+                    raise KernelError(f"{count} sequences exceed the launch grid")
+                part_o = workspace.get("attention_partial_out", items * num_heads * head_dim)
+                part_lse = workspace.get("attention_partial_lse", items * num_heads)
+                arrivals = workspace.get("attention_arrivals", count * num_kv_heads)
+            elif splits is None:
                 # (a window bounds the keys a row block walks, however long the sequence)
                 seen = window + keep_first + longest if window else max_kv_len
                 splits = self.choose_splits(count, num_kv_heads, row_tiles, min(max_kv_len, seen), decode_only)
@@ -2091,7 +2119,6 @@ class HipOps:
                     splits = self.choose_portion_splits(num_tokens, group, num_kv_heads, min(max_kv_len, portions_max_kv_len or max_kv_len, seen))
             if count * splits > 65535:
                 raise KernelError(f"{count} sequences x {splits} splits exceed the launch grid")
-            part_o = part_lse = None
             if splits > 1:
                 if workspace is None:
                     raise KernelError("split attention needs a workspace")
@@ -2105,7 +2132,7 @@ class HipOps:
                 num_tokens if decode_only else tokens, longest, int(max_kv_len), num_heads, num_kv_heads,
                 block_size.bit_length() - 1, float(scale), int(window or 0), splits, 0 if decode_only else first_token, _code(qkv.dtype),
                 _ptr(distance_bias), bias_len, _ptr(sinks), keep_first, float(softcap or 0.0), gate_rows(first_token if decode_only else 0), gate_stride,
-                int(gate_channels), self._stream())
+                int(gate_channels), _ptr(arrivals), share, self._stream())
             self._launched(status, "paged_attention")
 
         if not all_decode and splits is None and 0 < decode_prefix < num_seqs and group <= 16:

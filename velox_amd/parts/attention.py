@@ -112,7 +112,7 @@ class AttentionMixer(Mixer):
         if sizes is None:
             return {}
         partial_out, partial_lse = sizes(self.num_heads, self.num_kv_heads, self.head_dim, limits.max_num_tokens, limits.max_num_seqs, limits.max_model_len)
-        return {"attention_partial_out": partial_out, "attention_partial_lse": partial_lse}
+        return {"attention_partial_out": partial_out, "attention_partial_lse": partial_lse, "attention_arrivals": limits.max_num_seqs * self.num_kv_heads}
 
     products_in_parts = ("o_weight",)
     accepts_sink = True  # its last product may add itself to the residual (ResidualSink)
@@ -137,6 +137,7 @@ class AttentionMixer(Mixer):
             ctx.max_q_len, meta.max_kv_len, self.scale, self.window,
             ctx.all_decode, ctx.workspace,
             decode_prefix=getattr(ctx, "decode_prefix", 0), portions_max_kv_len=getattr(meta, "max_kv_len_of_portions", 0) or None,
+            uneven=True,
         )
         return ops.linear(attn, self.operand("o_weight"), None, ctx.dtype, partials_ok=True, residual_norm=sink)
 
