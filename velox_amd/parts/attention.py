@@ -137,7 +137,7 @@ class AttentionMixer(Mixer):
             ctx.max_q_len, meta.max_kv_len, self.scale, self.window,
             ctx.all_decode, ctx.workspace,
             decode_prefix=getattr(ctx, "decode_prefix", 0), portions_max_kv_len=getattr(meta, "max_kv_len_of_portions", 0) or None,
-            uneven=True,
+            **({"uneven": True} if hasattr(ops, "shares_keys") else {}),
         )
         return ops.linear(attn, self.operand("o_weight"), None, ctx.dtype, partials_ok=True, residual_norm=sink)
 
