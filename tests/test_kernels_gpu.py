@@ -823,6 +823,62 @@ def test_decoded_tokens_whose_keys_are_shared_out(ops, ref, dtype, nh, nkv, d, p
     assert torch.equal(run(moved), got[order])
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 512, 64), (1, 520, 8960), (4, 1536, 1536), (2, 1540, 8960), (3, 2048, 192), (1, 2048, 20480), (4, 512, 5120), (1, 768, 11008)])
+def test_a_few_rows_into_the_residual(ops, ref, m, n, k):
+    """The product of up to four rows with a narrow weight: the smallest and longest sums it takes, odd numbers of blocks of 64 indices, waves
+    without any, outputs that end inside a tile."""
+    from velox_amd.parts.base import ResidualSink
+    from velox_amd.parts.norms import RMSNorm
+
+    assert ops._few_rows_pieces(m, k) <= 10
+    x, w = rand((m, k), torch.bfloat16, 40), rand((n, k), torch.bfloat16, 41, 0.05)
+    norm = RMSNorm("", n, 1e-5)
+    norm.weight = 1.0 + rand((n,), torch.float32, 42, 0.1)
+    residual0 = rand((m, n), torch.float32, 43)
+    residual, other = residual0.clone(), residual0.clone()
+    deferred = ops.linear(x, ops.prepare_weight(w), None, torch.bfloat16, partials_ok=True, residual_norm=ResidualSink(residual, norm))
+    assert deferred.sums.shape == (16, 2 * ((n + 15) // 16))
+    want = residual0.double() + x.double() @ w.double().T
+    # products of bfloat16 numbers are exact in float32; k additions, rounded down or to nearest
+    assert torch.all((residual.double() - want).abs() <= k * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T + residual0.abs()))
+    assert torch.equal(deferred.x, (residual * norm.weight).to(torch.bfloat16))
+    torch.testing.assert_close(deferred.sums[:m].sum(1), (residual * residual).sum(1), rtol=1e-5, atol=0)
+    ops._linear_into_residual(x, ops.prepare_weight(w), ResidualSink(other, norm), row_tiles=1)
+    torch.testing.assert_close(residual, other, rtol=1e-5, atol=1e-5 * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("nh,nkv,d,n,lens", [(12, 2, 128, 1536, [391]), (12, 2, 128, 1536, [1000, 3]), (28, 4, 128, 3584, [2048]), (14, 2, 64, 896, [100, 70, 128, 1]), (12, 2, 48, 512, [65])])
+def test_parts_of_an_attention_that_the_output_product_merges(ops, ref, nh, nkv, d, n, lens):
+    from velox_amd.engine.batch import Workspace
+    from velox_amd.kernels.hip_ops import KernelError
+    from velox_amd.parts.base import AttentionParts, ResidualSink
+    from velox_amd.parts.norms import RMSNorm
+
+    case = _attention_case(torch.bfloat16, nh, nkv, d, 16, [(1, length) for length in lens], seed=3)
+    weight = ops.prepare_weight(rand((n, nh * d), torch.bfloat16, 44, 0.05))
+    norm = RMSNorm("", n, 1e-5)
+    norm.weight = torch.ones(n, device="cuda")
+    workspace, m = Workspace(torch.device("cuda")), len(lens)
+
+    def product(**more):
+        residual = torch.zeros((m, n), device="cuda")
+        sink = ResidualSink(residual, norm)
+        parts = ops.attention_parts(m, nh, nkv, d, weight, sink, max(lens))
+        attention = ops.paged_attention(case["qkv"], nh, nkv, d, case["k_cache"], case["v_cache"], 16, case["tables"], case["cu"], case["kv"], 1, max(lens),
+                                        1.0 / math.sqrt(d), None, True, workspace, **(more or {"parts": parts}))
+        assert parts in (2, 4, 8) and isinstance(attention, AttentionParts) == (not more)
+        ops.linear(attention, weight, None, torch.bfloat16, residual_norm=sink)
+        return residual
+
+    got, whole = product(), product(splits=1)
+    # (either rounds the attention's output to bfloat16 once; a wave's running maximum takes other steps)
+    assert float((got - whole).norm() / whole.norm()) < 2.0 ** -8
+    case["kv"].fill_(1)  # behind one key the other parts are empty
+    assert float((product() - product(splits=1)).norm()) <= 1e-4 * float(whole.norm())
+    with pytest.raises(KernelError):
+        ops.linear(AttentionParts(torch.zeros(8, device="cuda"), torch.zeros(8, device="cuda"), 1, m, nh, d), weight, None, torch.bfloat16)
+
+
 def test_far_key_among_hundreds_is_found(ops):
     # one key far back matches the query strongly: the output must be (nearly) that key's value
     nh, nkv, d, page = 4, 2, 64, 16

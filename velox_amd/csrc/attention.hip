@@ -1747,6 +1747,7 @@ static int launch(const void* qkv, int qkv_stride, const void* k_cache, const vo
                   const float* bias_table, int bias_len, const float* sinks, const Extras& extras, int* arrivals, int share, hipStream_t stream) {
   constexpr int BN = tile_keys<T>();
   const int group = nh / nkv;
+  if (arrivals != nullptr && out == nullptr) return -1;
   if (arrivals != nullptr) {  // (asked for only where the streaming kernel takes the step; items: see shared_item)
     if constexpr (SHARES_KEYS && sizeof(T) * D <= 512) {
       if (max_q_len != 1 || total_tokens != num_seqs || first_token != 0 || group > 16 || page_shift < 2 || share < 1) return -1;
@@ -1769,14 +1770,16 @@ static int launch(const void* qkv, int qkv_stride, const void* k_cache, const vo
     // in flight.  (For steps with one workgroup per compute unit, twice as many sets and eight waves per workgroup
     // were both measured slower on MI355X.)
     constexpr int DEPTH = sizeof(T) * D <= 256 ? 3 : 2;
+    if (out == nullptr && splits == 1) return -1;
     decode_attention_kernel<T, DEPTH, 4><<<dim3(splits, nkv, num_seqs), 256, 0, stream>>>(
         (const T*)qkv, qkv_stride, (const T*)k_cache, (const T*)v_cache, block_tables, table_width, kv_lens, (T*)out, part_o, part_lse,
         nh, nkv, page_shift, scale, window, splits, total_tokens, bias_table, bias_len, sinks, extras, nullptr);
     int status = (int)hipGetLastError();
-    if (status != 0 || splits == 1) return status;
+    if (status != 0 || splits == 1 || out == nullptr) return status;
     merge_splits_kernel<T><<<dim3(total_tokens, nh), MERGE_THREADS, 0, stream>>>(part_o, part_lse, (T*)out, nh, splits, total_tokens, 0, sinks, extras);
     return (int)hipGetLastError();
   }
+  if (out == nullptr) return -1;
   // The kernel whose tiles reach LDS by direct loads: bfloat16, head sizes 64, 128 and 256, pages of at least 8 tokens.
   constexpr bool HAS_DIRECT = sizeof(T) == 2 && (D == 64 || D == 128 || D == 256);
   const bool direct_ok = HAS_DIRECT && page_shift >= 3 && portion_kernel_choice != 1;
@@ -1942,6 +1945,7 @@ extern "C" int velox_attention_options() { return (BIASED ? 1 : 0) | (KEEPS ? 2 
 // part_o: float32 [splits, total_tokens, nh, D]; part_lse: float32 [splits, total_tokens, nh]; both unused when splits == 1.
 // first_token: the sequences given (cu_q holds rows of qkv and out) cover rows [first_token, total_tokens); a launch for
 // the later sequences of a step passes its first row here so that only those rows are merged.
+// out == nullptr: a decode step's splits are left in part_o and part_lse (what reads them merges).
 // arrivals (int32 [num_seqs, nkv], zero before and after; or nullptr): a decode step whose keys are shared out by their number, see
 // shared_item; `share`: workgroups per KV head, `splits` is not read; part_o and part_lse have a row of nh heads per item.
 extern "C" int velox_paged_attention(const void* qkv, int qkv_stride, const void* k_cache, const void* v_cache,

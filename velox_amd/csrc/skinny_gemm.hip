@@ -573,6 +573,181 @@ __global__ void __launch_bounds__(WAVES * 64) skinny_residual_norm_kernel(const 
   }
 }
 
+// The same for few rows and a narrow W (half a tile per workgroup): what bounded the kernel above there was not W's bytes (1 row,
+// 8,960 -> 1,536: 27.5 MB in 9.6 us, and in 9.6 when W was in the caches) but its loads: half of every wave's lanes asked for nothing, the
+// activations took as many load instructions as W, and a wave waited for each of its rounds.  Here a load of W brings eight rows of TWO
+// blocks of 64 indices, multiplied with the activations of the one and of the other (the accumulator's other half is not used), four waves keep
+// a second group of loads under way, and the activations of a wave's share of K come once, in whole lines, and stay in LDS: 9.6 -> 7.1 us,
+// 1,536 -> 1,536 3.9 -> 3.6.  Eight waves: 7.3 and 4.0; groups of two, three and four pairs of blocks: 7.1, 7.1, 7.1.
+// STAGED: pieces of 16 bytes per lane that hold a wave's activations.  PARTS > 0: the activations are an attention's output whose keys were split
+// over up to PARTS workgroups, merged here as they are staged; every workgroup reads all of it, which costs 0.2 us with four parts and
+// one piece, 1.2 with eight or with two pieces (1,536 -> 1,536: 3.4, 3.7, 4.7, 4.9), where a merge in a kernel of its own costs 3.3.
+struct AttentionParts {
+  const float* out;  // [splits][M][heads][dim], every split's output over its own sum
+  const float* lse;  // [splits][M][heads]
+  int splits, heads, dim;
+};
+constexpr int FEW_WAVES = 4, FEW_PAIRS = 4;
+template <int STAGED, int PARTS>
+__global__ void __launch_bounds__(FEW_WAVES * 64) skinny_few_rows_residual_kernel(const bf16_t* __restrict__ a, const AttentionParts parts, const bf16_t* __restrict__ w,
+                                                                                  float* __restrict__ residual, const float* __restrict__ norm_weight,
+                                                                                  bf16_t* __restrict__ next, float* __restrict__ sums, int m, int n, int k) {
+  __shared__ float4_t partial[FEW_WAVES][64];
+  __shared__ __attribute__((aligned(16))) bf16_t staged[FEW_WAVES][STAGED * 512];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, i = lane & 15;
+  const int tile = blockIdx.x >> 1, half = blockIdx.x & 1;
+  const int col = tile * 16 + 8 * half + 4 * g;  // (epilogue, lanes 0 .. 31 of the first wave: row i's columns col .. + 3)
+  const bool finishes = threadIdx.x < 32 && i < m;
+  float old_residual[4], weight[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const bool inside = finishes && col + j < n;
+    old_residual[j] = inside ? residual[(size_t)i * n + col + j] : 0.f;
+    weight[j] = inside ? norm_weight[col + j] : 0.f;
+  }
+  // this wave's share of K, in pairs of blocks of 64 (the last pair's second block may not be there)
+  const int blocks = k / 64, pairs = (blocks + 1) / 2, per_wave = (pairs + FEW_WAVES - 1) / FEW_WAVES;
+  const int lo = min(wave * per_wave, pairs), hi = min(lo + per_wave, pairs);
+  const int slice = 64 * (min(2 * hi, blocks) - min(2 * lo, blocks));
+  const bf16_t* w_lane = w + (size_t)tile * blocks * 1024 + (16 * g + 8 * half + (i & 7)) * 8;
+  float4_t even = {0.f, 0.f, 0.f, 0.f}, odd = {0.f, 0.f, 0.f, 0.f};
+  if (lo < hi) {
+    float4_t piece[STAGED], merged[PARTS ? STAGED : 1][PARTS ? 2 * PARTS : 1];
+    float logs[PARTS ? STAGED : 1][PARTS ? PARTS : 1];
+#pragma unroll
+    for (int t = 0; t < STAGED; ++t) {
+      const int e = min(t * 512 + lane * 8, m * slice - 8), row = m == 1 ? 0 : e / slice, c = 128 * lo + e - row * slice;
+      if constexpr (PARTS > 0) {
+        const int head = c / parts.dim;
+        const size_t slot = (size_t)row * parts.heads + head, stride = (size_t)m * parts.heads;
+#pragma unroll
+        for (int s = 0; s < PARTS; ++s) {
+          const size_t at = slot + stride * min(s, parts.splits - 1);
+          logs[t][s] = parts.lse[at];
+          const float4_t* o = reinterpret_cast<const float4_t*>(parts.out + at * parts.dim + (c - head * parts.dim));
+          merged[t][2 * s] = o[0];
+          merged[t][2 * s + 1] = o[1];
+        }
+      } else {
+        piece[t] = *reinterpret_cast<const float4_t*>(a + (size_t)row * k + c);
+      }
+    }
+    struct Group { Run16 w[FEW_PAIRS]; } x, y;
+    auto load = [&](Group& q, int p0) {
+#pragma unroll
+      for (int u = 0; u < FEW_PAIRS; ++u) {
+        const int p = min(p0 + u, hi - 1);
+        q.w[u] = load_run_packed(w_lane + (size_t)(i < 8 ? 2 * p : min(2 * p + 1, blocks - 1)) * 1024);
+      }
+    };
+    load(x, lo);
+#pragma unroll
+    for (int t = 0; t < STAGED; ++t) {
+      if constexpr (PARTS > 0) {
+        float top = -INFINITY, total = 0.f;
+#pragma unroll
+        for (int s = 0; s < PARTS; ++s) top = s < parts.splits ? fmaxf(top, logs[t][s]) : top;
+        const float safe = top == -INFINITY ? 0.f : top;
+        float4_t low = {0.f, 0.f, 0.f, 0.f}, high = low;
+#pragma unroll
+        for (int s = 0; s < PARTS; ++s) {
+          const float share = s < parts.splits && logs[t][s] != -INFINITY ? expf(logs[t][s] - safe) : 0.f;
+          total += share;
+          low += merged[t][2 * s] * share;
+          high += merged[t][2 * s + 1] * share;
+        }
+        const float over = total > 0.f ? total : 1.f;
+        bf16x8_t eight;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          eight[j] = from_f32<bf16_t>(low[j] / over);
+          eight[4 + j] = from_f32<bf16_t>(high[j] / over);
+        }
+        piece[t] = __builtin_bit_cast(float4_t, eight);
+      }
+      *reinterpret_cast<float4_t*>(&staged[wave][t * 512 + lane * 8]) = piece[t];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const bf16_t* row = &staged[wave][(i < m ? i : 0) * slice + 16 * g];
+    auto use = [&](const Group& q, int p0) {
+#pragma unroll
+      for (int u = 0; u < FEW_PAIRS; ++u) {
+        if (p0 + u >= hi) break;  // (uniform over the wave)
+        const bf16x8_t* first = reinterpret_cast<const bf16x8_t*>(row + (p0 + u - lo) * 128);
+        even = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u].lo, first[0], even, 0, 0, 0);
+        even = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u].hi, first[1], even, 0, 0, 0);
+        if (2 * (p0 + u) + 1 < blocks) {
+          odd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u].lo, first[8], odd, 0, 0, 0);
+          odd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u].hi, first[9], odd, 0, 0, 0);
+        }
+      }
+    };
+    for (int p = lo;;) {
+      if (p + FEW_PAIRS >= hi) { use(x, p); break; }
+      load(y, p + FEW_PAIRS);
+      __builtin_amdgcn_sched_barrier(0);
+      use(x, p);
+      p += FEW_PAIRS;
+      if (p + FEW_PAIRS >= hi) { use(y, p); break; }
+      load(x, p + FEW_PAIRS);
+      __builtin_amdgcn_sched_barrier(0);
+      use(y, p);
+      p += FEW_PAIRS;
+    }
+  }
+  partial[wave][lane] = lane < 32 ? even : odd;  // (rows 0 .. 7 of the one, 8 .. 15 of the other)
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  float squares = 0.f;
+  if (finishes) {
+    float4_t sum = partial[0][lane] + partial[0][lane + 32];
+#pragma unroll
+    for (int wv = 1; wv < FEW_WAVES; ++wv) sum += partial[wv][lane] + partial[wv][lane + 32];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (col + j >= n) break;
+      const size_t at = (size_t)i * n + col + j;
+      const float r = old_residual[j] + sum[j];
+      residual[at] = r;
+      next[at] = from_f32<bf16_t>(r * weight[j]);
+      squares += r * r;
+    }
+  }
+  squares += __shfl_xor(squares, 16, VELOX_WAVE);
+  if (lane < 16) sums[(size_t)lane * gridDim.x + blockIdx.x] = squares;
+}
+
+// a [M, K] bfloat16, or (parts_out != nullptr) an attention's output in `splits` parts, see AttentionParts; the others as below, with row_tiles
+// = 0.  -1: more activations than the pieces hold.
+extern "C" int velox_skinny_few_rows_residual_bf16(const void* a, const void* w, float* residual, const float* norm_weight, void* next, float* sums, int m, int n, int k,
+                                                   const float* parts_out, const float* parts_lse, int splits, int heads, int dim, hipStream_t stream) {
+  if (m <= 0 || n <= 0) return 0;
+  if (m > 16 || k % 64 != 0) return -1;
+  const int pairs = (k / 64 + 1) / 2, pieces = (m * ((pairs + FEW_WAVES - 1) / FEW_WAVES) * 128 + 511) / 512;
+  const AttentionParts parts{parts_out, parts_lse, splits, heads, dim};
+  const int grid = 2 * ((n + 15) / 16);
+#define FEW_ROWS(STAGED, PARTS) \
+  skinny_few_rows_residual_kernel<STAGED, PARTS><<<grid, FEW_WAVES * 64, 0, stream>>>((const bf16_t*)a, parts, (const bf16_t*)w, residual, norm_weight, (bf16_t*)next, sums, m, n, k)
+  if (parts_out != nullptr) {
+    if (splits < 1 || splits > 8 || dim % 8 != 0 || heads * dim != k || pieces > 2) return -1;
+    if (pieces <= 1 && splits <= 2) FEW_ROWS(1, 2);
+    else if (pieces <= 1 && splits <= 4) FEW_ROWS(1, 4);
+    else if (pieces <= 1) FEW_ROWS(1, 8);
+    else if (splits <= 4) FEW_ROWS(2, 4);
+    else FEW_ROWS(2, 8);
+  } else {
+    if (pieces <= 1) FEW_ROWS(1, 0);
+    else if (pieces <= 2) FEW_ROWS(2, 0);
+    else if (pieces <= 5) FEW_ROWS(5, 0);
+    else if (pieces <= 10) FEW_ROWS(10, 0);
+    else return -1;
+  }
+#undef FEW_ROWS
+  return (int)hipGetLastError();
+}
+
 // a [M, K] bfloat16 (M <= 16; a_packed != 0: in the lanes' order, see packed_row_offset), w packed [N, K]; sums: float32
 // [16][blocks], blocks = ceil(N / 16), or twice that with row_tiles = 0.  next_packed (or null; needs N % 64 == 0): room
 // for N / 64 * 1024 elements, `next` once more in the lanes' order.  waves: 4, 8 or 16.  row_tiles: 16-row tiles of W per

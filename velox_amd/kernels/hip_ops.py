@@ -22,10 +22,11 @@ from typing import Tuple, Dict, Optional
 
 import torch
 
-from ..parts.base import DeferredNorm, NormedSum, ReadyInput, ResidualCopy, ResidualSink, SumOf
+from ..parts.base import AttentionParts, DeferredNorm, NormedSum, ReadyInput, ResidualCopy, ResidualSink, SumOf
 from . import build
 
 logger = logging.getLogger(__name__)
+
 
 _DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}
 _P = ctypes.c_void_p
@@ -132,6 +133,8 @@ class HipOps:
         c.velox_skinny_gemm_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _F, _F, _I, _I, _P]
         c.velox_skinny_residual_norm_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P]
         c.velox_skinny_residual_norm_bf16.restype = _I
+        c.velox_skinny_few_rows_residual_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P, _P, _I, _I, _I, _P]
+        c.velox_skinny_few_rows_residual_bf16.restype = _I
         c.velox_row_scale_apply.argtypes = [_P, _P, _I, _F, _F, _P, _I, _I, _P]
         c.velox_skinny_gemm_bf16.restype = _I
         c.velox_skinny_gemm_glu_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _F, _F, _I, _P, _P]
@@ -801,7 +804,12 @@ class HipOps:
         float32 partial sums ``[S, M, N]`` that the consumer adds (``add_rmsnorm`` does).  With ``residual_norm`` it may
         come back as a ``DeferredNorm``: the product has then been added to ``residual_norm.residual`` and multiplied
         with the weight of ``residual_norm.norm`` (decode-sized bfloat16 products whose weight is registered).  ``x`` may
-        be a ``DeferredNorm``."""
+        be a ``DeferredNorm``, or the ``AttentionParts`` that ``attention_parts`` has announced for this product."""
+        if isinstance(x, AttentionParts):
+            fused = self._linear_into_residual(x, weight, residual_norm) if residual_norm is not None and bias is None else None
+            if fused is None:
+                raise KernelError("linear: this product does not merge an attention's parts (attention_parts says which does)")
+            return fused
         weight, prepared = _weight_of(weight)
         packed = prepared.copy(1) if prepared is not None else None
         deferred = x if isinstance(x, DeferredNorm) else None
@@ -873,7 +881,36 @@ class HipOps:
             raise KernelError("this PyTorch's matrix library has no bfloat16 product with a float32 result (torch.mm(..., out_dtype=)); "
                               f"logits of many rows at once need it in a bfloat16 run: {err}") from err
 
-    def _linear_into_residual(self, x: torch.Tensor, weight: torch.Tensor, sink: ResidualSink, waves: Optional[int] = None, row_tiles: Optional[int] = None,
+    def _few_rows_pieces(self, m: int, k: int) -> int:
+        """Pieces of 16 bytes per lane that hold a wave's activations in the product of few rows (skinny_few_rows_residual_kernel)."""
+        pairs = (k // 64 + 1) // 2
+        return -(-m * (-(-pairs // 4)) * 128 // 512)
+
+    # Behind up to so many keys a few decoded tokens' output product merges the splits of their attention (``attention_parts``); behind more they
+    # take more splits than are worth reading in each of its workgroups.
+    attention_parts_keys = 2048
+
+    def attention_parts(self, tokens: int, num_heads: int, num_kv_heads: int, head_dim: int, weight, sink: Optional[ResidualSink], max_kv_len: int) -> int:
+        """In how many splits of the keys the attention of ``tokens`` single tokens may leave its output (``paged_attention(parts=)``) for the
+        product with ``weight`` that adds it to ``sink`` to merge; 0: it merges them itself.  What this saves is the merge's kernel (3.3 us, and
+        about as long when the last workgroup merges), what it costs is that each of the product's workgroups reads all parts: 0.2 us at up
+        to four of them and one piece, 1.2 beyond.  Measured on MI355X, attention and product of a token (us, one pass / splits and
+        merge / parts): 12 heads over 2, 1,536 wide, 60 keys 8.6 / - / 8.8, 391 13.3 / 12.7 / 9.2, 1,000 20 / 12.8 / 10.6, 4,000 53 / 14.8 /
+        15.1; 28 over 4, 3,584 wide, 391 keys 16.6 / 15.5 / 14.3."""
+        if sink is None or sink.norm.deferred_form() is None or not 64 < max_kv_len <= self.attention_parts_keys or not self.merges_attention_parts(tokens, num_heads, num_kv_heads, head_dim, weight):
+            return 0
+        return 2 if max_kv_len <= 128 else 4 if max_kv_len <= 1024 else 8
+
+    def merges_attention_parts(self, tokens: int, num_heads: int, num_kv_heads: int, head_dim: int, weight) -> bool:
+        """Whether the product of so many rows with ``weight`` can merge an attention's splits, for some number of keys."""
+        weight, prepared = _weight_of(weight)
+        packed = prepared.copy(1) if prepared is not None else None
+        n, k = weight.shape
+        return (packed is not None and weight.dtype == torch.bfloat16 and k == num_heads * head_dim and head_dim % 8 == 0 and k % 64 == 0 and 512 <= n <= 16 * self.num_cus
+                and self.use_skinny_gemm and self.fuse_residual_norm and head_dim <= self.MAX_TILED_HEAD_DIM and tokens <= 4 and self._few_rows_pieces(tokens, k) <= 2
+                and not self.shares_keys(tokens, num_kv_heads))
+
+    def _linear_into_residual(self, x, weight: torch.Tensor, sink: ResidualSink, waves: Optional[int] = None, row_tiles: Optional[int] = None,
                               packed: Optional[torch.Tensor] = None) -> Optional[DeferredNorm]:
         """``sink.residual += x @ weight^T`` with the first half of ``sink.norm`` in the same kernel, if this product
         qualifies (bfloat16, at most 16 rows, registered weight, a norm that can be split); None otherwise."""
@@ -881,25 +918,35 @@ class HipOps:
         weight, prepared = _weight_of(weight)
         if prepared is not None and packed is None:
             packed = prepared.copy(1)
-        m, k = x.shape
+        parts = x if isinstance(x, AttentionParts) else None
+        m, k = (parts.tokens, parts.heads * parts.dim) if parts is not None else x.shape
         n = weight.shape[0]
         residual = sink.residual
         if (not self.use_skinny_gemm or not self.fuse_residual_norm or form is None or packed is None or m > 16 or k % 64 != 0 or n > 16 * 512
-                or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16):
+                or (parts is None and x.dtype != torch.bfloat16) or weight.dtype != torch.bfloat16 or weight.shape[1] != k):
             return None
         norm_weight, eps = form
         self._check("residual", residual, torch.float32, (m, n), align=16)
         self._check("norm weight", norm_weight, torch.float32, (n,))
         blocks = (n + 15) // 16
+        # up to four rows of a narrow weight have a kernel of their own (see there); measured on MI355X, us, that one / half tiles below: 1,536 x
+        # 8,960 with 1, 2 rows 7.6 / 9.6, 8.1 / 9.8, 1,536 x 1,536 with 1, 2, 4, 8 3.4 / 3.9, 3.5 / 3.9, 3.9 / 4.1, 4.2 / 4.1, 2,048 x 5,632 6.6 / 7.1
+        few = parts is not None or (row_tiles is None and waves is None and m <= 4 and n >= 512 and 2 * blocks <= self.num_cus and self._few_rows_pieces(m, k) <= 10)
         if row_tiles is None:
             # one 16-row tile of the weight per workgroup while that is at most one workgroup per compute unit; a wider
             # weight takes two (measured on MI355X at 8 rows: 5120 x 27648 65.8 -> 58.5 us, 3584 x 18944 27.8 -> 41.4)
             # and a narrow one half a tile, which gives every compute unit a workgroup (1536 x 8960: 13.0 -> 10.8 us)
             row_tiles = 2 if blocks > self.num_cus else 0 if 2 * blocks <= self.num_cus else 1
-        if row_tiles == 0:
+        if row_tiles == 0 or few:
             blocks *= 2  # (half a tile per workgroup: sums of squares per 8 columns)
         out = torch.empty((m, n), dtype=torch.bfloat16, device=self.device)
         sums = torch.empty((16, blocks), dtype=torch.float32, device=self.device)
+        if few:
+            status = self._core.velox_skinny_few_rows_residual_bf16(
+                _P(0) if parts is not None else _ptr(x), _ptr(packed), _ptr(residual), _ptr(norm_weight), _ptr(out), _ptr(sums), m, n, k,
+                *((_ptr(parts.out), _ptr(parts.lse), parts.splits, parts.heads, parts.dim) if parts is not None else (_P(0), _P(0), 0, 0, 0)), self._stream())
+            self._launched(status, "skinny_few_rows_residual")
+            return DeferredNorm(out, sums, n, float(eps), sink.norm)
         x_packed = self._packed_rows_of(x, k)
         out_packed = self._room_for_packed_rows(m, n)
         status = self._core.velox_skinny_residual_norm_bf16(_ptr(x if x_packed is None else x_packed), _ptr(packed), _ptr(residual), _ptr(norm_weight),
@@ -1999,6 +2046,7 @@ class HipOps:
         for portion in range(1, max_num_tokens + 1):  # portions of prompts, behind up to max_num_seqs - 1 single tokens
             whole = min(max_num_tokens, portion + max_num_seqs - 1)
             rows = max(rows, whole * self.choose_portion_splits(portion, group, num_kv_heads, max_model_len))
+        rows = max(rows, 8 * min(4, max_num_seqs))  # a few single tokens whose output product merges up to eight splits
         for count in range(1, max_num_seqs + 1):  # single tokens whose keys are shared out by their number
             if self.shares_keys(count, num_kv_heads):
                 rows = max(rows, self._shared_items(count, num_kv_heads, max_model_len, 4))
@@ -2020,7 +2068,8 @@ class HipOps:
     def paged_attention(self, qkv, num_heads, num_kv_heads, head_dim, k_cache, v_cache, block_size, block_tables, cu_q, kv_lens,
                         max_q_len, max_kv_len, scale, window, all_decode, workspace, splits: Optional[int] = None, decode_prefix: int = 0,
                         portions_max_kv_len: Optional[int] = None, distance_bias: Optional[torch.Tensor] = None, sinks: Optional[torch.Tensor] = None,
-                        keep_first: int = 0, softcap: Optional[float] = None, gate: Optional[Tuple[torch.Tensor, int, int]] = None, uneven: bool = False):
+                        keep_first: int = 0, softcap: Optional[float] = None, gate: Optional[Tuple[torch.Tensor, int, int]] = None, uneven: bool = False,
+                        parts: int = 0):
         """Attention of every token of the step over its sequence's keys in the cache.  ``decode_prefix``: how many of the
         first sequences bring exactly one token (the engine puts decoded tokens before portions of prompts).  In a mixed
         step those run through the streaming kernel with their keys split over workgroups, the others through the
@@ -2033,7 +2082,8 @@ class HipOps:
         window.  ``softcap``: a scaled score ``s`` becomes ``softcap * tanh(s / softcap)`` (before the bias).  ``gate = (source, first column, channels)``:
         head ``h``'s output times ``sigmoid`` of the source's columns, ``channels`` per head (channels beyond are left alone) or one per head
         with ``channels`` = 0.  (Each of the three has a build of the kernels: ``attention_library``.)  ``uneven``: single tokens' keys may be
-        shared out over the workgroups by their number (``shares_keys``); a token's order of additions then depends on the lengths of the others."""
+        shared out over the workgroups by their number (``shares_keys``); a token's order of additions then depends on the lengths of the others.
+        ``parts`` (of an all-decode step without sinks and gate): the keys are split in so many and come back as ``AttentionParts``."""
         tokens = qkv.shape[0]
         keep_first = int(keep_first) if window else 0
         gate_at, gate_stride, gate_channels = 0, 0, 0
@@ -2075,7 +2125,9 @@ class HipOps:
             raise KernelError(f"max_q_len={max_q_len} outside [1, {tokens}]")
         if not 0 <= decode_prefix <= num_seqs or num_seqs > tokens:
             raise KernelError(f"decode_prefix={decode_prefix} does not fit {num_seqs} sequences with {tokens} tokens")
-        out = torch.empty((tokens, num_heads * head_dim), dtype=qkv.dtype, device=self.device)
+        if parts and (not all_decode or tokens != num_seqs or sinks is not None or gate is not None or splits is not None or workspace is None or head_dim > self.MAX_TILED_HEAD_DIM):
+            raise KernelError("paged_attention: only an all-decode step's plain attention with a workspace is left in parts")
+        out = torch.empty((0 if parts else tokens, num_heads * head_dim), dtype=qkv.dtype, device=self.device)
         bias_len = 0
         if distance_bias is not None:
             self._check("distance_bias", distance_bias, torch.float32)
@@ -2095,7 +2147,7 @@ class HipOps:
         lib = self.attention_library(head_dim, distance_bias is not None, kept=keep_first > 0, capped=softcap is not None, gated=gate is not None)
         group = num_heads // num_kv_heads
 
-        def launch(first_seq: int, count: int, first_token: int, num_tokens: int, longest: int, decode_only: bool, splits: Optional[int]) -> None:
+        def launch(first_seq: int, count: int, first_token: int, num_tokens: int, longest: int, decode_only: bool, splits: Optional[int]):
             # sequences [first_seq, first_seq + count); their tokens are rows [first_token, first_token + num_tokens) of qkv
             # and out.  cu_q holds absolute rows, so the general kernel takes qkv and out whole; the streaming kernel
             # counts rows from its first sequence and takes the slices.
@@ -2128,13 +2180,16 @@ class HipOps:
             rows_in, rows_out = (qkv[first_token:first_token + num_tokens], out[first_token:first_token + num_tokens]) if decode_only else (qkv, out)
             status = lib.velox_paged_attention(
                 _ptr(rows_in), width, _ptr(k_cache), _ptr(v_cache), _ptr(block_tables[first_seq:]), block_tables.shape[1],
-                _ptr(cu_q[first_seq:]), _ptr(kv_lens[first_seq:]), _ptr(rows_out), _ptr(part_o), _ptr(part_lse), count,
+                _ptr(cu_q[first_seq:]), _ptr(kv_lens[first_seq:]), _P(0) if parts else _ptr(rows_out), _ptr(part_o), _ptr(part_lse), count,
                 num_tokens if decode_only else tokens, longest, int(max_kv_len), num_heads, num_kv_heads,
                 block_size.bit_length() - 1, float(scale), int(window or 0), splits, 0 if decode_only else first_token, _code(qkv.dtype),
                 _ptr(distance_bias), bias_len, _ptr(sinks), keep_first, float(softcap or 0.0), gate_rows(first_token if decode_only else 0), gate_stride,
                 int(gate_channels), _ptr(arrivals), share, self._stream())
             self._launched(status, "paged_attention")
+            return part_o, part_lse
 
+        if parts:
+            return AttentionParts(*launch(0, num_seqs, 0, tokens, 1, True, int(parts)), int(parts), tokens, num_heads, head_dim)
         if not all_decode and splits is None and 0 < decode_prefix < num_seqs and group <= 16:
             launch(0, decode_prefix, 0, decode_prefix, 1, True, None)
             launch(decode_prefix, num_seqs - decode_prefix, decode_prefix, tokens - decode_prefix, max_q_len, False, None)

@@ -105,7 +105,11 @@ class AttentionMixer(Mixer):
         if choose is None or max_model_len <= SHORT_CONTEXT_KEYS:
             return ()
         differs = choose(batch, self.num_kv_heads, 1, max_model_len, True) != choose(batch, self.num_kv_heads, 1, SHORT_CONTEXT_KEYS, True)
-        return (SHORT_CONTEXT_KEYS,) if differs else ()
+        bounds = (SHORT_CONTEXT_KEYS,) if differs else ()
+        merges = getattr(ops, "merges_attention_parts", None)  # (a few tokens' output product merges the splits behind up to so many keys)
+        if merges is not None and merges(batch, self.num_heads, self.num_kv_heads, self.head_dim, self.operand("o_weight")):
+            bounds += (ops.attention_parts_keys,)
+        return bounds
 
     def workspace_needs(self, ops, limits):
         sizes = getattr(ops, "attention_scratch_elems", None)
@@ -130,6 +134,9 @@ class AttentionMixer(Mixer):
             meta.slot_mapping, cache.tensors["k"], cache.tensors["v"], cache.block_size,
             write_kv=owns_cache,
         )
+        # a few decoded tokens: the output product may merge the splits of their keys
+        announced = getattr(ops, "attention_parts", None) if ctx.all_decode and sink is not None else None
+        parts = announced(q.shape[0], self.num_heads, self.num_kv_heads, self.head_dim, self.operand("o_weight"), sink, meta.max_kv_len) if announced is not None else 0
         attn = ops.paged_attention(
             q, self.num_heads, self.num_kv_heads, self.head_dim,
             cache.tensors["k"], cache.tensors["v"], cache.block_size,
@@ -137,7 +144,7 @@ class AttentionMixer(Mixer):
             ctx.max_q_len, meta.max_kv_len, self.scale, self.window,
             ctx.all_decode, ctx.workspace,
             decode_prefix=getattr(ctx, "decode_prefix", 0), portions_max_kv_len=getattr(meta, "max_kv_len_of_portions", 0) or None,
-            **({"uneven": True} if hasattr(ops, "shares_keys") else {}),
+            **({"parts": parts} if parts else {"uneven": True} if hasattr(ops, "shares_keys") else {}),
         )
         return ops.linear(attn, self.operand("o_weight"), None, ctx.dtype, partials_ok=True, residual_norm=sink)
 

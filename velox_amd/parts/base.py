@@ -276,6 +276,19 @@ class DeferredNorm:
 
 
 @dataclass
+class AttentionParts:
+    """A few tokens' attention whose keys were split over workgroups and not put together yet: the product that reads it
+    (``ops.linear`` with the sink that ``ops.attention_parts`` was asked about) merges the splits as it reads them."""
+
+    out: torch.Tensor  # float32 [splits, T, heads, dim]: every split's output over its own sum
+    lse: torch.Tensor  # float32 [splits, T, heads]: the logarithms of those sums
+    splits: int
+    tokens: int
+    heads: int
+    dim: int
+
+
+@dataclass
 class ResidualCopy:
     """What a block hands on when it has added everything to the residual itself and holds the updated residual in the
     run dtype already (``copy``, [T, H]; in a float32 run the residual itself): a norm that gets it as its delta adds
