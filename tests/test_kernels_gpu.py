@@ -1414,6 +1414,18 @@ def test_grouped_products_in_tiles_of_128_and_192_rows(ops, monkeypatch, rows, h
     assert torch.equal(experts_against_float64(ops, rows, hidden, inter, top, scale_input, unit), first)
 
 
+@pytest.mark.parametrize("hidden, inter", [(64, 2432), (64, 3200), (64, 5120), (4864, 64), (6400, 64), (10240, 64)])
+@pytest.mark.parametrize("scale_input, unit", [(False, "glu"), (True, "relu2")])
+def test_grouped_products_in_tiles_of_192_and_256_columns(ops, monkeypatch, hidden, inter, scale_input, unit):
+    """As many tiles as make 192 or 256 columns take fewer rounds than narrower ones, in the one product or in the other (the sizes
+    above all have 128); outputs that end inside a tile, the same bits with tiles of 128 rows, which are other widths."""
+    rows = (150, 200, 90, 130, 170, 100)
+    monkeypatch.setattr(ops._core, "velox_routed_tile_rows", lambda *sizes: 128)
+    first = experts_against_float64(ops, rows, hidden, inter, 1, scale_input, unit)
+    monkeypatch.setattr(ops._core, "velox_routed_tile_rows", lambda *sizes: 192)
+    assert torch.equal(experts_against_float64(ops, rows, hidden, inter, 1, scale_input, unit), first)
+
+
 def experts_against_float64(ops, rows, hidden, inter, top, scale_input, unit):
     """Against float64.  Two roundings to bfloat16 (8 bits), each off by at most 2^-8 of its value: the units' middles, which the second
     product adds up (at most 2^-8 sum |W_down| |middle|), and the result.  Float32 sums of a few hundred terms add less than

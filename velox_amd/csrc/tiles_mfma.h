@@ -448,11 +448,15 @@ struct TileCost { int rt, ct; float launch, round, step, step_alone; };
 static constexpr TileCost TILE_COSTS[] = {{2, 2, 3.2f, 0.9f, 0.492f, 0.347f}, {2, 3, 2.8f, 2.2f, 0.639f, 0.461f}, {2, 4, 2.0f, 3.9f, 0.776f, 0.576f}, {3, 3, 1.9f, 4.7f, 0.814f, 0.613f},
                                           {3, 4, 0.4f, 6.7f, 0.990f, 0.745f}, {4, 3, 0.0f, 7.0f, 0.985f, 0.737f}, {4, 4, -0.2f, 8.6f, 1.253f, 0.943f}};
 
-static inline float tiles_cost(const TileCost& t, long long m, long long w_rows, int k, int splits) {
+static inline float tiles_cost_of(const TileCost& t, float tiles, int k, int splits) {
   const int steps = (((k + 63) / 64 + splits - 1) / splits + 1) / 2 * 2;
-  const long long tiles = (m + 64 * t.rt - 1) / (64 * t.rt) * ((w_rows + 64 * t.ct - 1) / (64 * t.ct)) * splits;
-  const float full = (float)(tiles / TL_WORKGROUPS), rest = (float)(tiles % TL_WORKGROUPS) / TL_WORKGROUPS;
+  const float full = floorf(tiles / TL_WORKGROUPS), rest = tiles / TL_WORKGROUPS - full;
   return t.launch + full * (t.round + steps * t.step) + (rest > 0.f ? t.round + steps * (t.step_alone + (t.step - t.step_alone) * rest) : 0.f);
+}
+
+static inline float tiles_cost(const TileCost& t, long long m, long long w_rows, int k, int splits) {
+  const long long tiles = (m + 64 * t.rt - 1) / (64 * t.rt) * ((w_rows + 64 * t.ct - 1) / (64 * t.ct)) * splits;
+  return tiles_cost_of(t, (float)tiles, k, splits);
 }
 
 static inline const TileCost& tiles_best(long long m, long long w_rows, int k, int splits) {
