@@ -18,6 +18,8 @@
 //   removal_chunk_scan_kernel      a workgroup per 16 value columns, head and sequence; a wave holds 16 rows of the state in the
 //                                  matrix instructions' result layout, which is also their operand layout, so that the state
 //                                  never leaves the registers; the waves exchange their parts of D and O through LDS
+#include <type_traits>
+
 #include "common.h"
 
 #define CHUNK 16
@@ -259,121 +261,189 @@ __global__ void __launch_bounds__(256) removal_chunk_prepare_kernel(const Remova
 }
 
 // What a wave reads of one chunk, in registers: loaded SCAN_AHEAD chunks before it is worked.
+struct RemovalOperands { float4_t up, nb, k, p, dv, v; };
+// Up to 64 channels the read-outs have waves of their own.
+__host__ __device__ constexpr bool removal_readers(int waves) { return waves <= 4; }
 template <int WAVES>
-struct RemovalOperands {
-  static constexpr int READS = WAVES >= 4 ? 1 : (4 + WAVES - 1) / WAVES;  // read-outs of a chunk that a lane finishes
-  float4_t up, rp, nb, k, p, dv, v;
-  float ov[READS];
+struct RemovalReads {
+  static constexpr int EACH = WAVES >= 4 ? 1 : (4 + WAVES - 1) / WAVES;  // read-outs of a chunk that a lane finishes
+  float4_t rp;
+  float before[EACH];  // of the chunk before, whose read-outs are finished one chunk later
 };
 #define SCAN_AHEAD 4
 
-// (at most 256 registers a wave: the matrix instructions then keep the state in ordinary registers)
+// Bound by the chain of chunks on the few compute units that have a workgroup: per chunk the four dependent products that make a wave's part of D,
+// its way through LDS and a barrier, and the four that take it from the state.  So nothing else is in that chain's way: with READERS a second
+// set of waves, on the same SIMDs, gets the state in front of every chunk through LDS, makes O of it and finishes the read-outs a chunk
+// later (without, the chain's waves do so while D's parts are under way), and buffer loads and stores leave the vector unit no addresses
+// to add up.  One barrier a chunk: a buffer of `removed` or `states` is written again behind the next chunk's barrier, one of `reads` behind the
+// one that follows its readers'.  Measured on MI355X, 64 chunks, 32 heads of 64 x 64: 41.0 us with everything in one chain, 35.8 with the read-outs
+// a chunk later and buffer operations, 31.0 with waves of their own for them.
+// (At most 256 registers a wave: the matrix instructions then keep the state in ordinary registers.)
 template <int WAVES>
-__global__ void __launch_bounds__(64 * WAVES, 2) removal_chunk_scan_kernel(const RemovalChunkArgs a) {
-  __shared__ float4_t parts[2][2][WAVES][64];  // [buffer][D, O][wave][lane]
+__global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1)) __attribute__((amdgpu_waves_per_eu(2, 2))) removal_chunk_scan_kernel(const RemovalChunkArgs a) {
+  constexpr bool READERS = removal_readers(WAVES);
+  __shared__ float4_t removed[2][WAVES][64], reads[2][WAVES][64], states[READERS ? 2 : 1][READERS ? WAVES : 1][64];  // the waves' parts of D and O, [buffer][wave][lane]
   // (heads lie along the grid fastest in both kernels: with a multiple of 8 heads the workgroups that read a record run
   // on the XCD that wrote it and share it in that XCD's L2)
-  const int h = blockIdx.x, tile = blockIdx.y, b = blockIdx.z;
-  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
+  // (a step's single tokens come before its portions of prompts: from the back, so that the long chains do not begin when everything else is
+  // done: 12 single tokens beside 1,024, 32 heads of 64 x 64, 49 -> 38 us)
+  const int h = blockIdx.x, tile = blockIdx.y, b = (int)(gridDim.z - 1 - blockIdx.z);
+  const int lo = __builtin_amdgcn_readfirstlane(a.cu_q[b]), hi = __builtin_amdgcn_readfirstlane(a.cu_q[b + 1]);
   if (hi <= lo) return;  // (the whole workgroup)
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63, any_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = any_wave % WAVES, tid = wave * 64 + lane;
   const int n = lane & 15, g = lane >> 4;
   constexpr int dim = 16 * WAVES;
-  constexpr int READS = RemovalOperands<WAVES>::READS;
+  constexpr int EACH = RemovalReads<WAVES>::EACH;
   const int vdim = a.vdim, columns = removal_columns(vdim);
   const int column = tile * 16 + n;
   const bool live = column < vdim;
   const int chunks = (hi - lo + CHUNK - 1) / CHUNK;
   const size_t stride = (size_t)a.heads * removal_record(dim, vdim);  // between a sequence's records of this head
-  // a lane's places in a record, in floats (the record's own address is the same for the whole wave and moves from chunk to chunk)
-  const uint32_t rows_at = wave * 256 + n * 16 + 4 * g, decays_at = 64 * dim + wave * 16 + 4 * g, column_at = 65 * dim + column * CHUNK + 4 * g;
-  uint32_t reads_at[READS];
+  // a lane's places in a record, in bytes (the record's own address is the same for the whole wave and moves from chunk to chunk)
+  const uint32_t rows_at = 4 * (wave * 256 + n * 16 + 4 * g), decays_at = 4 * (64 * dim + wave * 16 + 4 * g), column_at = 4 * (65 * dim + column * CHUNK + 4 * g);
+  uint32_t reads_at[EACH], out_at[EACH];
 #pragma unroll
-  for (int q = 0; q < READS; ++q) {
-    const int i = (tid + q * 64 * WAVES) & 255;  // a read-out's place in the order in which the parts lie in LDS
-    reads_at[q] = 65 * dim + (columns + tile * 16 + ((i >> 2) & 15)) * CHUNK + (i >> 6) * 4 + (i & 3);
+  for (int q = 0; q < EACH; ++q) {
+    const int i = tid + q * 64 * WAVES, t = ((i >> 6) & 3) * 4 + (i & 3), e = (i >> 2) & 15;  // a read-out's place in the order in which the parts lie in LDS
+    reads_at[q] = 4 * (65 * dim + (columns + tile * 16 + e) * CHUNK + t);
+    out_at[q] = i < 256 && tile * 16 + e < vdim ? 4u * (t * (uint32_t)a.heads * vdim + e) : 0x80000000u;  // (behind any row: not stored)
   }
   const float* next = a.scratch + ((size_t)removal_first_chunk(lo, b) * a.heads + h) * removal_record(dim, vdim);
-  int asked = 0;  // chunks asked for so far
-  auto load = [&](RemovalOperands<WAVES>& o) {
-    const float* record = next;
-    o.up = four(record + rows_at);
-    o.rp = four(record + 16 * dim + rows_at);
-    o.nb = four(record + 32 * dim + rows_at);
-    o.k = four(record + 48 * dim + rows_at);
-    o.p = four(record + decays_at);
-    o.dv = four(record + column_at);
-    o.v = four(record + 32 * columns + column_at);
+  const float* before = next;
+  const int record_bytes = 4 * (int)removal_record(dim, vdim);
+  auto record_of = [&](const float* at) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(at), 0, record_bytes, 0x00020000); };
+  auto load_reads = [&](float (&ov)[EACH], const float* at) {
+    const auto record = record_of(at);
 #pragma unroll
-    for (int q = 0; q < READS; ++q) o.ov[q] = record[reads_at[q]];
-    ++asked;
-    if (asked < chunks) next += stride;  // (beyond the last chunk the last one is asked for again)
+    for (int q = 0; q < EACH; ++q) ov[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(record, reads_at[q], 0, 0));
   };
-
   float* S = a.state + (((size_t)a.slots[b] * a.heads + h) * dim + wave * 16 + 4 * g) * vdim + (live ? column : vdim - 1);
-  float4_t z;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) z[i] = S[(size_t)i * vdim];
-
   const size_t out_row = (size_t)a.heads * vdim;
   float* out = a.out + (size_t)lo * out_row + (size_t)h * vdim + tile * 16;
-  int left = hi - lo;  // tokens from the current chunk on
+  const int row_bytes = 4 * (int)out_row;
+  int pending = 0, left = hi - lo;  // tokens whose parts of O lie in LDS, tokens behind them
 
-  auto work = [&](int buffer, const RemovalOperands<WAVES>& o) {
-    float4_t d = {0.f, 0.f, 0.f, 0.f}, read = {0.f, 0.f, 0.f, 0.f};
+  // What a wave does: CHAINS the chain, READS the read-outs.  (A loop each, so that no load sits behind a branch.)
+  auto run = [&](auto chains_too, auto reads_too) {
+    constexpr bool CHAINS = decltype(chains_too)::value, READS = decltype(reads_too)::value;
+    float last_reads[EACH];
+    if constexpr (READS) load_reads(last_reads, next + (size_t)(chunks - 1) * stride);
+    int asked = 0;  // chunks asked for so far
+    auto load = [&](RemovalOperands& o, RemovalReads<WAVES>& r) {
+      __builtin_amdgcn_sched_barrier(0);  // (in this order on every path: a wait counts the loads that are younger)
+      const auto record = record_of(next);
+      auto piece = [&](uint32_t at, int from) { return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(record, at, 4 * from, 0)); };
+      if constexpr (CHAINS) {
+        o.up = piece(rows_at, 0);
+        o.nb = piece(rows_at, 32 * dim);
+        o.k = piece(rows_at, 48 * dim);
+        o.p = piece(decays_at, 0);
+        o.dv = piece(column_at, 0);
+        o.v = piece(column_at, 32 * columns);
+      }
+      if constexpr (READS) {
+        r.rp = piece(rows_at, 16 * dim);
+        load_reads(r.before, before);
+        before = next;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      ++asked;
+      if (asked < chunks) next += stride;  // (beyond the last chunk the last one is asked for again)
+    };
+    // The read-outs of a chunk, 256 over the readers' lanes, behind the barrier that follows their parts.
+    auto read_out = [&](int buffer, const float (&ov)[EACH]) {
+      const float* sums = reinterpret_cast<const float*>(reads[buffer]);
+      const auto rows = __builtin_amdgcn_make_buffer_rsrc(out, 0, pending * row_bytes, 0x00020000);  // (what lies behind the last token is not stored)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      d = mfma4(o.up[e], z[e], d);
-      read = mfma4(o.rp[e], z[e], read);
+      for (int q = 0; q < EACH; ++q) {
+        float v = ov[q];
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) v += sums[w * 256 + ((tid + q * 64 * WAVES) & 255)];
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rows, out_at[q], 0, 0);
+      }
+      out += pending * out_row;
+      pending = left < CHUNK ? left : CHUNK;
+      left -= pending;
+    };
+    auto meet = [&] {  // (what every wave has written to LDS is there; each loop comes here as often)
+      asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" : : : "memory");
+    };
+    float4_t z = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (CHAINS) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) z[i] = S[(size_t)i * vdim];
     }
-    parts[buffer][0][wave][lane] = d;
-    parts[buffer][1][wave][lane] = read;
+    auto work = [&](int buffer, const RemovalOperands& o, const RemovalReads<WAVES>& r) {
+      float4_t d = {0.f, 0.f, 0.f, 0.f}, read = d, kept = z;
+      if constexpr (CHAINS) {
+        if constexpr (!READS) states[buffer][wave][lane] = z;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) z = mfma4(o.k[e], o.v[e], z);
-    __syncthreads();  // (one a chunk: a buffer is written again behind the next chunk's barrier)
-    d = o.dv;
+        for (int e = 0; e < 4; ++e) d = mfma4(o.up[e], z[e], d);
+        __builtin_amdgcn_sched_barrier(0);
+        removed[buffer][wave][lane] = d;
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) d += parts[buffer][0][w][lane];
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (READS) read = mfma4(r.rp[e], z[e], read);
+          else kept = mfma4(o.k[e], o.v[e], kept);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      meet();
+      if constexpr (CHAINS) {
+        d = o.dv;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) z = mfma4(o.nb[e], d[e], z);
-    z *= o.p;
-    // the chunk's read-outs: 256 of them over the workgroup's lanes
-    const float* sums = reinterpret_cast<const float*>(parts[buffer][1]);
+        for (int w = 0; w < WAVES; ++w) d += removed[buffer][w][lane];
+        if constexpr (READS) {
+          reads[buffer][wave][lane] = read;
 #pragma unroll
-    for (int q = 0; q < READS; ++q) {
-      const int i = tid + q * 64 * WAVES;
-      if (i < 256) {
-        const int t = (i >> 6) * 4 + (i & 3), e = (i >> 2) & 15;
-        float v = o.ov[q];
+          for (int e = 0; e < 4; ++e) kept = mfma4(o.k[e], o.v[e], kept);
+        }
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) v += sums[w * 256 + i];
-        if (t < left && tile * 16 + e < vdim) out[t * out_row + e] = v;
+        for (int e = 0; e < 4; ++e) kept = mfma4(o.nb[e], d[e], kept);
+        if constexpr (READS) read_out(1 - buffer, r.before);
+        z = kept * o.p;
+      } else {
+        const float4_t state = states[buffer][wave][lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) read = mfma4(r.rp[e], state[e], read);
+        read_out(1 - buffer, r.before);
+        reads[buffer][wave][lane] = read;
+      }
+    };
+    // Loads are asked for whether or not there is a chunk that far ahead (then the last one's again): the same number of them lies
+    // between a chunk's loads and its work on every path, so that waiting for the one does not wait for the others.
+    RemovalOperands ops[SCAN_AHEAD];
+    RemovalReads<WAVES> of_reads[SCAN_AHEAD];
+#pragma unroll
+    for (int j = 0; j < SCAN_AHEAD; ++j) load(ops[j], of_reads[j]);
+    int c = 0;
+    for (; c + SCAN_AHEAD <= chunks; c += SCAN_AHEAD) {
+#pragma unroll
+      for (int j = 0; j < SCAN_AHEAD; ++j) {
+        work(j & 1, ops[j], of_reads[j]);
+        load(ops[j], of_reads[j]);
       }
     }
-    left -= CHUNK;
-    out += CHUNK * out_row;
-  };
-
-  // Loads are asked for whether or not there is a chunk that far ahead (then the last one's again): the same number of them lies
-  // between a chunk's loads and its work on every path, so that waiting for the one does not wait for the others.
-  RemovalOperands<WAVES> ops[SCAN_AHEAD];
 #pragma unroll
-  for (int j = 0; j < SCAN_AHEAD; ++j) load(ops[j]);
-  int c = 0;
-  for (; c + SCAN_AHEAD <= chunks; c += SCAN_AHEAD) {
+    for (int j = 0; j < SCAN_AHEAD - 1; ++j)
+      if (c + j < chunks) work(j & 1, ops[j], of_reads[j]);  // (the same for the whole workgroup)
+    meet();
+    if constexpr (READS) read_out((chunks - 1) & 1, last_reads);
+    if constexpr (CHAINS) {
+      if (live) {
 #pragma unroll
-    for (int j = 0; j < SCAN_AHEAD; ++j) {
-      work(j & 1, ops[j]);
-      load(ops[j]);
+        for (int i = 0; i < 4; ++i) S[(size_t)i * vdim] = z[i];
+      }
     }
-  }
-#pragma unroll
-  for (int j = 0; j < SCAN_AHEAD - 1; ++j)
-    if (c + j < chunks) work(j & 1, ops[j]);  // (the same for the whole workgroup)
-  if (live) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) S[(size_t)i * vdim] = z[i];
-  }
+  };
+  if constexpr (!READERS) run(std::true_type{}, std::true_type{});
+  else if (any_wave < WAVES) run(std::true_type{}, std::false_type{});
+  else run(std::false_type{}, std::true_type{});
 }
 
 // LDS of removal_chunk_prepare_kernel.  Its time is that of its dependent steps, so workgroups per compute unit count: with the small
@@ -396,10 +466,10 @@ static void removal_chunk_launch(const RemovalChunkArgs& a, int tokens, int num_
   removal_chunk_prepare_kernel<T><<<(unsigned)(a.heads * step_items(tokens, num_seqs, CHUNK)), 256, removal_prepare_lds(a.dim, a.rank), stream>>>(a, num_seqs);
   const dim3 grid(a.heads, removal_columns(a.vdim) / 16, num_seqs);
   switch (a.dim / 16) {
-    case 1: removal_chunk_scan_kernel<1><<<grid, 64, 0, stream>>>(a); break;
-    case 2: removal_chunk_scan_kernel<2><<<grid, 128, 0, stream>>>(a); break;
-    case 3: removal_chunk_scan_kernel<3><<<grid, 192, 0, stream>>>(a); break;
-    case 4: removal_chunk_scan_kernel<4><<<grid, 256, 0, stream>>>(a); break;
+    case 1: removal_chunk_scan_kernel<1><<<grid, 128, 0, stream>>>(a); break;
+    case 2: removal_chunk_scan_kernel<2><<<grid, 256, 0, stream>>>(a); break;
+    case 3: removal_chunk_scan_kernel<3><<<grid, 384, 0, stream>>>(a); break;
+    case 4: removal_chunk_scan_kernel<4><<<grid, 512, 0, stream>>>(a); break;
     case 5: removal_chunk_scan_kernel<5><<<grid, 320, 0, stream>>>(a); break;
     case 6: removal_chunk_scan_kernel<6><<<grid, 384, 0, stream>>>(a); break;
     case 7: removal_chunk_scan_kernel<7><<<grid, 448, 0, stream>>>(a); break;
