@@ -94,6 +94,21 @@ __device__ __forceinline__ StepItem step_item(const int* cu_q, int num_seqs, int
   return found;
 }
 
+// The sequence with the `rank`-th most tokens, ties in their order (beyond 64 sequences: from the back, since a step's single tokens come before
+// its portions of prompts).  The whole wave takes part.  For grids of a workgroup per sequence whose time is the longest chain's: it
+// has to begin with the first workgroups.
+__device__ __forceinline__ int sequence_by_length(const int* cu_q, int num_seqs, int rank) {
+  if (num_seqs > VELOX_WAVE) return num_seqs - 1 - rank;
+  const int lane = threadIdx.x & (VELOX_WAVE - 1), at = lane < num_seqs ? lane : 0;
+  const int mine = lane < num_seqs ? cu_q[at + 1] - cu_q[at] : -1;
+  int before = 0;
+  for (int b = 0; b < num_seqs; ++b) {
+    const int other = __builtin_amdgcn_readlane(mine, b);
+    before += other > mine || (other == mine && b < lane) ? 1 : 0;
+  }
+  return __ffsll((unsigned long long)__ballot(lane < num_seqs && before == rank)) - 1;
+}
+
 // Four consecutive elements of a row, widened to float32: one 8- or 16-byte access when `vec_ok` (the row starts on such a
 // boundary and k is a multiple of 4) and all four lie below k_limit, else element by element with zeros beyond k_limit.
 template <typename T>

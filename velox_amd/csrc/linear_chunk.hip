@@ -24,11 +24,11 @@
 //   linear_chunk_prepare_kernel   a workgroup per chunk and head: a wave per level, then T and the matrices above into `scratch`
 //   linear_chunk_scan_kernel      a workgroup per 16 value columns, head and sequence; a wave holds 16 rows of the state in the
 //                                 matrix instructions' result layout, which is also their operand layout; the waves exchange
-//                                 their parts of D and O through LDS with one barrier a chunk, loads four chunks ahead
+//                                 their parts of D through LDS with one barrier a chunk, others make O, loads four chunks ahead
 // The first is bound by what it moves (41 KB of records a chunk and head of 128 x 128), the second by the chain: per chunk four
-// matrix instructions, a barrier, a sum over the waves' parts, four more: 0.9 us.  Measured on MI355X, three prompts of 400 to
-// 1,300 tokens (2,421 in all), 8 heads of 128 x 128: 31 + 74 us against 377 us token by token (a column of the state per wave);
-// 16 heads 52 + 80 against 447; additive, 8 heads of 128 x 256: 38 + 47 against 370.
+// matrix instructions, a barrier, a sum over the waves' parts, four more: 0.67 us.  Measured on MI355X, three prompts of 400 to
+// 1,300 tokens (2,421 in all), 8 heads of 128 x 128: 31 + 55 us against 377 us token by token (a column of the state per wave);
+// 16 heads 52 + 58 against 447; additive, 8 heads of 128 x 256: 35 + 41 against 370.
 #include "common.h"
 
 #define CHUNK 16
@@ -257,112 +257,149 @@ __global__ void __launch_bounds__(256) linear_chunk_prepare_kernel(const LinearC
 }
 
 // What a wave reads of one chunk, in registers: loaded SCAN_AHEAD chunks before it is worked.
-template <int WAVES>
-struct ChunkOperands {
-  float4_t up, rp, k, p, dv;
-  float ov;  // of the read-out that the lane finishes
+struct ChunkOperands { float4_t up, k, p, dv; };
+struct ChunkReads {
+  float4_t rp;
+  float before;  // of the chunk before, whose read-outs are finished one chunk later
 };
 #define SCAN_AHEAD 4
 
-// (at most 256 registers a wave: the matrix instructions then keep the state in ordinary registers)
+// Bound by the chain of chunks on the few compute units that have a workgroup: per chunk the four dependent products that make a wave's part of D,
+// its way through LDS and a barrier, and the four that add it to the state.  Nothing else is in that chain's way: the first WAVES waves
+// work it, and as many others, on the same SIMDs, get the state in front of every chunk through LDS, make O of it and finish the
+// read-outs a chunk later; buffer loads and stores leave the vector unit no addresses to add up.  One barrier a chunk: a buffer of `removed`
+// or `states` is written again behind the next chunk's barrier, one of `reads` behind the one that follows its readers'.  Measured on MI355X,
+// 82 chunks of the longest of three sequences, us, with everything in one chain / this: 8 heads of 128 x 128 72 / 55, 16 heads 77 / 58, additive, 8
+// heads of 128 x 256, 46 / 41.
 template <int WAVES, bool DELTA>
-__global__ void __launch_bounds__(64 * WAVES, 2) linear_chunk_scan_kernel(const LinearChunkArgs a) {
-  __shared__ float4_t parts[2][2][WAVES][64];  // [buffer][D, O][wave][lane]
+__global__ void __launch_bounds__(128 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES / 2, WAVES / 2))) linear_chunk_scan_kernel(const LinearChunkArgs a) {
+  static_assert(WAVES == 4 || WAVES == 8, "a chunk's 256 read-outs are finished by 256 lanes of the readers");
+  __shared__ float4_t removed[2][DELTA ? WAVES : 1][64], reads[2][WAVES][64], states[2][WAVES][64];  // [buffer][wave][lane]
   // (heads lie along the grid's first dimension in both kernels: with a multiple of 8 heads the workgroups that read a record run
   // on the XCD that wrote it and share it in that XCD's L2)
-  const int h = a.first_head + blockIdx.x, tile = blockIdx.y, b = blockIdx.z;
-  const int lo = a.cu_q[b], hi = a.cu_q[b + 1];
+  const int h = a.first_head + blockIdx.x, tile = blockIdx.y, b = __builtin_amdgcn_readfirstlane(sequence_by_length(a.cu_q, a.num_seqs, blockIdx.z));
+  const int lo = __builtin_amdgcn_readfirstlane(a.cu_q[b]), hi = __builtin_amdgcn_readfirstlane(a.cu_q[b + 1]);
   if (hi - lo < a.long_from || hi <= lo) return;  // (the whole workgroup)
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63, any_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = any_wave % WAVES, tid = wave * 64 + lane;
   const int n = lane & 15, g = lane >> 4;
   constexpr int dim = 16 * WAVES;
-  static_assert(WAVES >= 4, "a chunk's 256 read-outs are finished by the first 256 lanes");
   const int vdim = a.vdim, columns = chunk_columns(vdim);
   const int column = tile * 16 + n;
   const bool live = column < vdim;
   const int chunks = (hi - lo + CHUNK - 1) / CHUNK;
   const size_t stride = (size_t)a.head_count * chunk_record(dim, vdim);  // between a sequence's records of this head
-  // a lane's places in a record, in floats (the record's own address is the same for the whole wave and moves from chunk to chunk)
-  const uint32_t rows_at = wave * 256 + n * 16 + 4 * g, decays_at = 48 * dim + wave * 16 + 4 * g, column_at = 49 * dim + column * CHUNK + 4 * g;
-  // the read-out that a lane finishes, by its place in the order in which the parts lie in LDS
-  const int out_t = ((tid >> 6) & 3) * 4 + (tid & 3), out_e = (tid >> 2) & 15;
-  const uint32_t read_at = 49 * dim + (columns + tile * 16 + out_e) * CHUNK + out_t;
-  const float* next = a.scratch + ((size_t)first_chunk(lo, b) * a.head_count + blockIdx.x) * chunk_record(dim, vdim);
-  int asked = 0;  // chunks asked for so far
-  auto load = [&](ChunkOperands<WAVES>& o) {
-    const float* record = next;
-    if (DELTA) o.up = four(record + rows_at);
-    o.rp = four(record + 16 * dim + rows_at);
-    o.k = four(record + 32 * dim + rows_at);
-    o.p = four(record + decays_at);
-    o.dv = four(record + column_at);
-    o.ov = record[read_at];
-    ++asked;
-    if (asked < chunks) next += stride;  // (beyond the last chunk the last one is asked for again)
-  };
-
-  float* S = a.state + (((size_t)a.slots[b] * a.heads + h) * dim + wave * 16 + 4 * g) * vdim + (live ? column : vdim - 1);
-  float4_t z;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) z[i] = S[(size_t)i * vdim];
-
   const size_t out_row = (size_t)a.heads * vdim;
-  float* out = a.out + (size_t)lo * out_row + (size_t)h * vdim + tile * 16;
-  int left = hi - lo;  // tokens from the current chunk on
-
-  auto work = [&](int buffer, const ChunkOperands<WAVES>& o) {
-    float4_t d = {0.f, 0.f, 0.f, 0.f}, read = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (DELTA) d = mfma4(o.up[e], z[e], d);
-      read = mfma4(o.rp[e], z[e], read);
-    }
-    if (DELTA) parts[buffer][0][wave][lane] = d;
-    parts[buffer][1][wave][lane] = read;
-    z *= o.p;
-    if (!DELTA) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) z = mfma4(o.k[e], o.dv[e], z);
-    }
-    __syncthreads();  // (one a chunk: a buffer is written again behind the next chunk's barrier)
-    if (DELTA) {
-      d = o.dv;
-#pragma unroll
-      for (int w = 0; w < WAVES; ++w) d += parts[buffer][0][w][lane];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) z = mfma4(o.k[e], d[e], z);
-    }
-    // the chunk's read-outs: 256 of them over the workgroup's lanes
-    const float* sums = reinterpret_cast<const float*>(parts[buffer][1]);
-    if (tid < 256) {
-      float v = o.ov;
-#pragma unroll
-      for (int w = 0; w < WAVES; ++w) v += sums[w * 256 + tid];
-      if (out_t < left && tile * 16 + out_e < vdim) out[out_t * out_row + out_e] = v;
-    }
-    left -= CHUNK;
-    out += CHUNK * out_row;
+  const float* next = a.scratch + ((size_t)first_chunk(lo, b) * a.head_count + blockIdx.x) * chunk_record(dim, vdim);
+  const int record_bytes = 4 * (int)chunk_record(dim, vdim);
+  // a lane's places in a record, in bytes (the record's own address is the same for the whole wave and moves from chunk to chunk)
+  const uint32_t rows_at = 4 * (wave * 256 + n * 16 + 4 * g);
+  auto record_of = [&](const float* at) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(at), 0, record_bytes, 0x00020000); };
+  auto piece = [&](const __amdgpu_buffer_rsrc_t& record, uint32_t at, int from) { return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(record, at, 4 * from, 0)); };
+  auto meet = [&] {  // (what every wave has written to LDS is there; both loops come here as often)
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
   };
-
-  // Loads are asked for whether or not there is a chunk that far ahead (then the last one's again): the same number of them lies
-  // between a chunk's loads and its work on every path, so that waiting for the one does not wait for the others.
-  ChunkOperands<WAVES> ops[SCAN_AHEAD];
-#pragma unroll
-  for (int j = 0; j < SCAN_AHEAD; ++j) load(ops[j]);
-  int c = 0;
-  for (; c + SCAN_AHEAD <= chunks; c += SCAN_AHEAD) {
+  // Loads are asked for whether or not there is a chunk that far ahead (then the last one's again), in this order on every path: a wait
+  // counts the loads that are younger.  A loop per set of waves, so that none sits behind a branch.
+  auto walk = [&](auto& ops, auto load, auto work) {
 #pragma unroll
     for (int j = 0; j < SCAN_AHEAD; ++j) {
-      work(j & 1, ops[j]);
       load(ops[j]);
+      if (j + 1 < chunks) next += stride;
+      __builtin_amdgcn_sched_barrier(0);
     }
-  }
+    int c = 0;
+    for (; c + SCAN_AHEAD <= chunks; c += SCAN_AHEAD) {
 #pragma unroll
-  for (int j = 0; j < SCAN_AHEAD - 1; ++j)
-    if (c + j < chunks) work(j & 1, ops[j]);  // (the same for the whole workgroup)
-  if (live) {
+      for (int j = 0; j < SCAN_AHEAD; ++j) {
+        work(j & 1, ops[j]);
+        __builtin_amdgcn_sched_barrier(0);
+        load(ops[j]);
+        if (c + j + SCAN_AHEAD + 1 < chunks) next += stride;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) S[(size_t)i * vdim] = z[i];
+    for (int j = 0; j < SCAN_AHEAD - 1; ++j)
+      if (c + j < chunks) work(j & 1, ops[j]);  // (the same for the whole workgroup)
+    meet();
+  };
+
+  if (any_wave < WAVES) {
+    const uint32_t decays_at = 4 * (48 * dim + wave * 16 + 4 * g), column_at = 4 * (49 * dim + column * CHUNK + 4 * g);
+    float* S = a.state + (((size_t)a.slots[b] * a.heads + h) * dim + wave * 16 + 4 * g) * vdim + (live ? column : vdim - 1);
+    float4_t z;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z[i] = S[(size_t)i * vdim];
+    ChunkOperands ops[SCAN_AHEAD];
+    walk(ops, [&](ChunkOperands& o) {
+      const auto record = record_of(next);
+      if (DELTA) o.up = piece(record, rows_at, 0);
+      o.k = piece(record, rows_at, 32 * dim);
+      o.p = piece(record, decays_at, 0);
+      o.dv = piece(record, column_at, 0);
+    }, [&](int buffer, const ChunkOperands& o) {
+      states[buffer][wave][lane] = z;
+      float4_t d = o.dv;
+      if constexpr (DELTA) {
+        d = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d = mfma4(o.up[e], z[e], d);
+        removed[buffer][wave][lane] = d;
+      }
+      z *= o.p;
+      if constexpr (DELTA) {
+        meet();
+        d = o.dv;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) d += removed[buffer][w][lane];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z = mfma4(o.k[e], d[e], z);
+      if constexpr (!DELTA) meet();
+    });
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[(size_t)i * vdim] = z[i];
+    }
+  } else {
+    // the read-out that a lane finishes, by its place in the order in which the parts lie in LDS
+    const int out_t = ((tid >> 6) & 3) * 4 + (tid & 3), out_e = (tid >> 2) & 15;
+    const uint32_t read_at = 4 * (49 * dim + (columns + tile * 16 + out_e) * CHUNK + out_t);
+    const uint32_t out_at = tid < 256 && tile * 16 + out_e < vdim ? 4u * (out_t * (uint32_t)out_row + out_e) : 0x80000000u;  // (behind any row: not stored)
+    float* out = a.out + (size_t)lo * out_row + (size_t)h * vdim + tile * 16;
+    const int row_bytes = 4 * (int)out_row;
+    int pending = 0, left = hi - lo;  // tokens whose parts of O lie in LDS, tokens behind them
+    auto read_of = [&](const float* at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(record_of(at), read_at, 0, 0)); };
+    const float last_read = read_of(next + (size_t)(chunks - 1) * stride);
+    const float* before = next;
+    auto read_out = [&](int buffer, float v) {
+      const auto rows = __builtin_amdgcn_make_buffer_rsrc(out, 0, pending * row_bytes, 0x00020000);  // (what lies behind the last token is not stored)
+      const float* sums = reinterpret_cast<const float*>(reads[buffer]);
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) v += sums[w * 256 + (tid & 255)];
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rows, out_at, 0, 0);
+      out += pending * out_row;
+      pending = left < CHUNK ? left : CHUNK;
+      left -= pending;
+    };
+    ChunkReads ops[SCAN_AHEAD];
+    walk(ops, [&](ChunkReads& o) {
+      o.rp = piece(record_of(next), rows_at, 16 * dim);
+      o.before = read_of(before);
+      before = next;
+    }, [&](int buffer, const ChunkReads& o) {
+      meet();
+      const float4_t z = states[buffer][wave][lane];
+      float4_t read = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) read = mfma4(o.rp[e], z[e], read);
+      if (WAVES == 4 || wave < 4) read_out(1 - buffer, o.before);  // (uniform over the wave)
+      reads[buffer][wave][lane] = read;
+    });
+    if (WAVES == 4 || wave < 4) read_out((chunks - 1) & 1, last_read);
   }
 }
 
@@ -381,8 +418,8 @@ static void linear_chunk_launch(const LinearChunkArgs& a, int tokens, hipStream_
   const size_t lds = (size_t)CHUNK * (3 * (a.dim + 4) + 4 * CHUNK_STRIDE) * sizeof(float);
   linear_chunk_prepare_kernel<DELTA><<<(unsigned)records_of_step(tokens, a.num_seqs) * (unsigned)a.head_count, 256, lds, stream>>>(a);
   const dim3 grid(a.head_count, chunk_columns(a.vdim) / 16, a.num_seqs);
-  if (a.dim == 64) linear_chunk_scan_kernel<4, DELTA><<<grid, 256, 0, stream>>>(a);
-  else linear_chunk_scan_kernel<8, DELTA><<<grid, 512, 0, stream>>>(a);
+  if (a.dim == 64) linear_chunk_scan_kernel<4, DELTA><<<grid, 512, 0, stream>>>(a);
+  else linear_chunk_scan_kernel<8, DELTA><<<grid, 1024, 0, stream>>>(a);
 }
 
 extern "C" int velox_linear_scan(const float* qk, const void* v, int v_dtype, int v_ld, int v_at, const float* decay, int decay_per_channel, const float* beta,

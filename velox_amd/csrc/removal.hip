@@ -286,9 +286,8 @@ __global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1))
   __shared__ float4_t removed[2][WAVES][64], reads[2][WAVES][64], states[READERS ? 2 : 1][READERS ? WAVES : 1][64];  // the waves' parts of D and O, [buffer][wave][lane]
   // (heads lie along the grid fastest in both kernels: with a multiple of 8 heads the workgroups that read a record run
   // on the XCD that wrote it and share it in that XCD's L2)
-  // (a step's single tokens come before its portions of prompts: from the back, so that the long chains do not begin when everything else is
-  // done: 12 single tokens beside 1,024, 32 heads of 64 x 64, 49 -> 38 us)
-  const int h = blockIdx.x, tile = blockIdx.y, b = (int)(gridDim.z - 1 - blockIdx.z);
+  // (the long chains begin first, not when the single tokens in front of them are done: 12 beside 1,024, 32 heads of 64 x 64, 49 -> 38 us)
+  const int h = blockIdx.x, tile = blockIdx.y, b = __builtin_amdgcn_readfirstlane(sequence_by_length(a.cu_q, gridDim.z, blockIdx.z));
   const int lo = __builtin_amdgcn_readfirstlane(a.cu_q[b]), hi = __builtin_amdgcn_readfirstlane(a.cu_q[b + 1]);
   if (hi <= lo) return;  // (the whole workgroup)
   const int lane = threadIdx.x & 63, any_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
