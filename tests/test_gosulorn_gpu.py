@@ -4,6 +4,7 @@ made to stand out just inside and just outside the window, at page borders and b
 recurrences over long portions; the whole model in float32 and bfloat16 through replay (every way of cutting, pages and
 slots used again), far memory, long decoding, batches against each request alone, the entry point with captured decode
 steps, and the replay program itself."""
+import itertools
 import json
 import os
 import subprocess
@@ -790,3 +791,23 @@ def test_a_number_that_is_not_finite_reaches_its_own_token_and_later_ones_only(o
     assert torch.equal(torch.isfinite(got), torch.isfinite(want)) and torch.equal(torch.isfinite(state), torch.isfinite(after))
     assert float((got[:token] - clean[:token]).abs().max()) <= 64 * 2.0 ** -24 * float(clean.abs().max())
     assert not torch.isfinite(want).all()
+
+
+@pytest.mark.parametrize("lengths", [[300, 40, 700], [33, 1, 2, 64], [200, 3, 1, 31], [90], [64, 64], [50, 0, 1]])
+def test_lengths_say_which_kernels_the_shorter_portions_need(ops, lengths):
+    """With the sequences' lengths at hand only the kernels that have work are launched; the bits are those of the guess from their sum."""
+    heads, dim, vdim, tokens = 8, 64, 32, sum(lengths)
+    rng = torch.Generator(device="cuda").manual_seed(len(lengths) + tokens)
+    rand = lambda *shape: torch.randn(shape, generator=rng, device="cuda")
+    qk, v = rand(tokens, heads, 2, dim) / 8, rand(tokens, heads * vdim).to(torch.bfloat16)
+    decay, beta = torch.sigmoid(rand(tokens, heads) + 3), torch.sigmoid(rand(tokens, heads))
+    cu = torch.tensor([0] + list(itertools.accumulate(lengths)), dtype=torch.int32, device="cuda")
+    slots = torch.arange(len(lengths), dtype=torch.int32, device="cuda")
+    start = rand(len(lengths), heads, dim, vdim)
+    results = []
+    for q_lens in (None, lengths):
+        state = start.clone()
+        results.append((ops.linear_scan(qk, v, 0, decay, beta, state, slots, cu, max(lengths), heads, heads, dim, vdim, "delta", q_lens=q_lens), state))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    want = 0 if all(n == 0 or n >= ops.LINEAR_CHUNK_TOKENS for n in lengths) else 1 if all(n <= 2 or n >= ops.LINEAR_CHUNK_TOKENS for n in lengths) else 2
+    assert ops.shorter_portions(tokens, len(lengths), max(lengths), ops.LINEAR_CHUNK_TOKENS, lengths) == want

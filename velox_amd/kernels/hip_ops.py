@@ -18,7 +18,7 @@ import logging
 import os
 import tempfile
 import threading
-from typing import Tuple, Dict, Optional
+from typing import Tuple, Dict, Optional, Sequence
 
 import torch
 
@@ -1561,13 +1561,25 @@ class HipOps:
     LINEAR_CHUNK_TOKENS = 32
     LINEAR_CHUNK_SCRATCH = 1 << 28  # the most float32 numbers of scratch they ask for, if one head's fit (1 GB: 13,000 tokens of 32 heads of 128 x 128 at once)
 
-    def linear_scan(self, qk, v_source, v_at, decay, beta, state, slots, cu_q, max_q_len, heads, kv_heads, dim, vdim, rule, chunked: Optional[bool] = None):
+    @staticmethod
+    def shorter_portions(tokens: int, sequences: int, max_q_len: int, long_from: int, q_lens: Optional[Sequence[int]] = None) -> int:
+        """What is beside the portions of at least ``long_from`` tokens: 0 nothing, 1 single tokens and pairs, 2 longer ones too.  Without the
+        lengths: nothing if all are as long as the longest; longer ones if the number of tokens leaves room for one.  (Each of the two
+        launches that are spared found nothing to do in 4.6 us: three prompts of 400 to 1,300 tokens took both in every layer.)"""
+        if q_lens is None:
+            return 0 if tokens == sequences * max_q_len else 1 if tokens - max_q_len == sequences - 1 else 2
+        most = max((n for n in q_lens if n < long_from), default=0)
+        return 0 if most == 0 else 1 if most <= 2 else 2
+
+    def linear_scan(self, qk, v_source, v_at, decay, beta, state, slots, cu_q, max_q_len, heads, kv_heads, dim, vdim, rule, chunked: Optional[bool] = None,
+                    q_lens: Optional[Sequence[int]] = None):
         """Per sequence and head, token by token from ``state[slot, head]`` ([dim, vdim] float32), which is written back:
         ``S <- g S`` (rows); ``u = beta (v - S^T k)`` (rule ``"delta"``) or ``u = v`` (``"additive"``); ``S <- S + k u^T``; ``o = S^T q``.
         Rule ``"removal"``: ``qk`` holds a third vector ``b`` per head and token, and ``S <- g S - b (k^T S) + k (beta v)^T`` with both
         terms on the old state.  ``decay`` is [T, heads] or [T, heads * dim].  Returns float32 [T, heads * vdim].  Long portions of the
         first two rules are worked in chunks of 16 tokens on the matrix cores (key heads of 64 or 128 channels), all others, also beside
-        them, token by token; ``chunked`` decides it for a test, for all sequences."""
+        them, token by token; ``chunked`` decides it for a test, for all sequences.  ``q_lens``: the sequences' numbers of tokens, where the
+        caller knows them (which kernels the shorter ones need is otherwise guessed from their sum)."""
         if rule not in self._SCAN_RULES:
             raise KernelError(f"linear_scan: rule {rule!r} is not implemented ({', '.join(self._SCAN_RULES)})")
         delta = rule != "additive"
@@ -1604,9 +1616,7 @@ class HipOps:
                                                   int(kv_heads), int(dim), int(vdim), self._SCAN_RULES[rule], 1, 0, self._stream())
             self._launched(status, "linear_scan")
             return out
-        # What may be beside the long portions: nothing if all are as long as the longest; single tokens and pairs; longer ones too if the
-        # number of tokens leaves room for one.
-        shorter = 0 if long_from == 1 or tokens == sequences * max_q_len else 1 if tokens - max_q_len == sequences - 1 else 2
+        shorter = 0 if long_from == 1 else self.shorter_portions(tokens, sequences, max_q_len, long_from, q_lens)
         heads_at_once = max(1, min(int(heads), self.LINEAR_CHUNK_SCRATCH // per_head))
         scratch = torch.empty(per_head * heads_at_once, dtype=torch.float32, device=self.device)
         self._launched(self._core.velox_linear_chunk_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),

@@ -219,7 +219,7 @@ class LinearRecurrenceMixer(Mixer):
             main if self.rule == "delta" else None, self.beta_at or 0,
         )
         read = ops.linear_scan(qk, qkv, v_at, decay, beta, cache.tensors["state"], ctx.slots, ctx.cu_q, ctx.max_q_len,
-                               heads, kv_heads, dim, vdim, self.rule)
+                               heads, kv_heads, dim, vdim, self.rule, **({"q_lens": ctx.q_lens} if hasattr(ops, "shorter_portions") else {}))
         if self.gate == "silu":
             gate_source, gate_at, gate_kind = main, self.g_at, "silu"
         else:
