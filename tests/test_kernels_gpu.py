@@ -823,6 +823,18 @@ def test_decoded_tokens_whose_keys_are_shared_out(ops, ref, dtype, nh, nkv, d, p
     assert torch.equal(run(moved), got[order])
 
 
+@pytest.mark.parametrize("n,k", [(7, 260), (4094, 36), (4099, 512), (120001, 8), (30002, 300)])
+def test_gemm_fma_of_few_rows_in_every_shape(ops, n, k):
+    """Two, four and eight rows of W a wave, numbers of rows of A between those that are built: a product's bits are those of each of its rows
+    alone, whose sums are k products and additions in float32."""
+    x, w, bias = rand((16, k), torch.float32, 60), rand((n, k), torch.float32, 61), rand((n,), torch.float32, 62)
+    whole = ops.gemm_fma(x, w, bias, torch.float32)
+    bound = (k + 8) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + bias.double().abs())
+    assert torch.all((whole.double() - (x.double() @ w.double().T + bias.double())).abs() <= bound)
+    for m in (1, 2, 3, 4, 5, 7, 8, 9, 12, 13):
+        assert torch.equal(ops.gemm_fma(x[:m].contiguous(), w, bias, torch.float32), whole[:m])
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 512, 64), (1, 520, 8960), (4, 1536, 1536), (2, 1540, 8960), (3, 2048, 192), (1, 2048, 20480), (4, 512, 5120), (1, 768, 11008)])
 def test_a_few_rows_into_the_residual(ops, ref, m, n, k):
     """The product of up to four rows with a narrow weight: the smallest and longest sums it takes, odd numbers of blocks of 64 indices, waves

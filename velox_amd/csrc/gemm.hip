@@ -295,61 +295,131 @@ static void launch_mfma_f32(const void* a, const void* w, const float* bias, voi
 }
 
 // The same product for few rows (M <= 16), where it is bound by reading W once: the decode steps of a float32 run.
-// A wave owns SKINNY_ROWS consecutive rows of W and all of K; lane l takes indices 4 l .. 4 l + 3 of every block of
+// A wave owns ROWS consecutive rows of W and all of K; lane l takes indices 4 l .. 4 l + 3 of every block of
 // 256, so a wave's load of a row's block is one contiguous kilobyte (float32) and the activations (from L2) are used
-// for SKINNY_ROWS rows of W at once.  A lane adds its terms in the order of k, the 64 lanes' sums are added in a fixed
-// tree: an element's sum depends on nothing but its own row of A and row of W.
-#define SKINNY_ROWS 4
+// for ROWS rows of W at once.  A lane adds its terms in the order of k, the 64 lanes' sums are added in a fixed
+// tree: an element's sum depends on nothing but its own row of A and row of W, whatever ROWS is.
+// Measured on MI355X, us, with four rows, a tree through LDS for every sum, ordinary loads and 8 or 16 rows of A where there are 5 or more / like this:
+// 1,536 -> 151,936, 1 row 153 / 133, 6 rows 225 / 143, 16 391 / 207; 1,536 -> 17,920, 1, 6 and 16 rows 22 / 19, 38 / 23, 59 / 35; 1,536 -> 2,048 7.6 /
+// 5.8, 15.2 / 7.3, 24.7 / 10.1; 8,960 -> 1,536 31 / 26, 50 / 33, 71 / 47.
+// (All of W is read once and in whole lines: non-temporal.)
+template <typename T>
+__device__ __forceinline__ void load4_once(const T* __restrict__ p, float (&v)[4]) {
+  if constexpr (sizeof(T) == 4) {
+    const float4_t x = __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(p));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = x[i];
+  } else {
+    const short4_t x = __builtin_nontemporal_load(reinterpret_cast<const short4_t*>(p));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(((uint32_t)(uint16_t)x[i]) << 16);
+  }
+}
 
-template <typename TA, typename TW, typename TO, int MT>
+// The wave's sums of COUNT values, in the tree of wave_sum (lanes 32 apart first, then 16, 8, ..), to its bits: at every level half of the values
+// are finished in one half of the lanes and half in the other, so that a level moves half as many as the one before.  Value i's sum lies
+// in the lanes whose bit 5 is i's bit 0, bit 4 its bit 1 and so on.  32 values: 32 moves, 24 of them between registers, instead of 192 through LDS.
+template <int COUNT>
+__device__ __forceinline__ float wave_sums(float (&v)[COUNT]) {
+  const int lane = threadIdx.x & 63;
+  int left = COUNT;
+#pragma unroll
+  for (int offset = 32; offset > 0; offset >>= 1) {
+    const bool upper = (lane & offset) != 0;
+    if (left == 1) {
+      v[0] += __shfl_xor(v[0], offset, VELOX_WAVE);
+      continue;
+    }
+#pragma unroll
+    for (int i = 0; i < left / 2; ++i) {
+      const float low = v[2 * i], high = v[2 * i + 1];
+      if (offset >= 16) {  // (the two registers' halves, or their rows of 16 lanes, change places: both then hold one value's two parts)
+        typedef unsigned int Two __attribute__((ext_vector_type(2)));
+        const Two both = offset == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(low), __float_as_uint(high), false, false)
+                                      : __builtin_amdgcn_permlane16_swap(__float_as_uint(low), __float_as_uint(high), false, false);
+        v[i] = __uint_as_float(both[0]) + __uint_as_float(both[1]);
+      } else {
+        const float mine = upper ? high : low, other = upper ? low : high;
+        v[i] = mine + __shfl_xor(other, offset, VELOX_WAVE);
+      }
+    }
+    left /= 2;
+  }
+  return v[0];
+}
+
+template <typename TA, typename TW, typename TO, int MT, int ROWS>
 __global__ void __launch_bounds__(256) skinny_fma_kernel(const TA* __restrict__ a, const TW* __restrict__ w, const float* __restrict__ bias,
                                                          TO* __restrict__ out, int m, int n, int k) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n0 = (blockIdx.x * 4 + wave) * SKINNY_ROWS;
+  const int n0 = (blockIdx.x * 4 + wave) * ROWS;
   if (n0 >= n) return;
-  float acc[SKINNY_ROWS][MT];
+  float acc[ROWS][MT];
 #pragma unroll
-  for (int r = 0; r < SKINNY_ROWS; ++r)
+  for (int r = 0; r < ROWS; ++r)
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[r][i] = 0.f;
-  size_t w_off[SKINNY_ROWS], a_off[MT];
+  size_t w_off[ROWS], a_off[MT];
 #pragma unroll
-  for (int r = 0; r < SKINNY_ROWS; ++r) w_off[r] = (size_t)(n0 + r < n ? n0 + r : n0) * k;  // (a row beyond N: row n0 again, never stored)
+  for (int r = 0; r < ROWS; ++r) w_off[r] = (size_t)(n0 + r < n ? n0 + r : n0) * k;  // (a row beyond N: row n0 again, never stored)
 #pragma unroll
   for (int i = 0; i < MT; ++i) a_off[i] = (size_t)(i < m ? i : 0) * k;
   for (int k0 = 4 * lane; k0 < k; k0 += 256) {
-    float wv[SKINNY_ROWS][4], av[MT][4];
+    float wv[ROWS][4], av[MT][4];
 #pragma unroll
-    for (int r = 0; r < SKINNY_ROWS; ++r) load4<TW>(w, w_off[r], k0, k, true, true, wv[r]);
+    for (int r = 0; r < ROWS; ++r) load4_once<TW>(w + w_off[r] + k0, wv[r]);
 #pragma unroll
     for (int i = 0; i < MT; ++i) load4<TA>(a, a_off[i], k0, k, true, true, av[i]);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int r = 0; r < SKINNY_ROWS; ++r)
+      for (int r = 0; r < ROWS; ++r)
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[r][i] = fmaf(av[i][e], wv[r][e], acc[r][i]);
   }
+  // 64 values at a time and what is left, filled up to a power of two with zeros
+  constexpr int BATCH = 64 / ROWS;  // rows of A
+  const int mine = (int)(__brev((unsigned)lane << 26) & 63u);  // the lane's six bits the other way round: which value it holds
 #pragma unroll
-  for (int r = 0; r < SKINNY_ROWS; ++r)
+  for (int i0 = 0; i0 < MT; i0 += BATCH) {
+    constexpr int LEFT = MT < BATCH ? MT : BATCH;
+    constexpr int COUNT = LEFT * ROWS <= 4 ? 4 : LEFT * ROWS <= 8 ? 8 : LEFT * ROWS <= 16 ? 16 : LEFT * ROWS <= 32 ? 32 : 64;
+    float values[COUNT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const float total = wave_sum(acc[r][i]);
-      if (lane == 0 && i < m && n0 + r < n) out[(size_t)i * n + n0 + r] = from_f32<TO>(total + (bias ? bias[n0 + r] : 0.f));
-    }
+    for (int v = 0; v < COUNT; ++v) values[v] = i0 + v / ROWS < MT ? acc[v % ROWS][i0 + v / ROWS < MT ? i0 + v / ROWS : 0] : 0.f;
+    const float total = wave_sums<COUNT>(values);
+    const int row = i0 + mine / ROWS, col = n0 + mine % ROWS;
+    if (mine < COUNT && row < m && col < n) out[(size_t)row * n + col] = from_f32<TO>(total + (bias ? bias[col] : 0.f));
+  }
 }
 
+// Rows of W per wave.  Eight, which halve the loads of A, where so many outputs leave enough waves (us, four / eight rows: 1,536 -> 151,936, 2 rows 134 / 136,
+// 3 137 / 136, 6 161 / 143; 2,048 -> 32,000, 8 rows 53 / 55, 12 64 / 60; 1,536 -> 17,920, 16 rows 35 / 37); two where four leave compute units without a
+// workgroup (four / two rows: 1,536 -> 2,048, 6 rows 8.5 / 7.3, 8,960 -> 1,536 39 / 33).  (Other types than float32 alone: four.)
 template <typename TA, typename TW, typename TO>
 static void launch_skinny_fma(const void* a, const void* w, const float* bias, void* out, int m, int n, int k, hipStream_t stream) {
-  const int waves = (n + SKINNY_ROWS - 1) / SKINNY_ROWS;
-  dim3 grid((waves + 3) / 4);
-#define SKINNY(MT) skinny_fma_kernel<TA, TW, TO, MT><<<grid, 256, 0, stream>>>((const TA*)a, (const TW*)w, bias, (TO*)out, m, n, k)
-  if (m <= 1) SKINNY(1);
-  else if (m <= 2) SKINNY(2);
-  else if (m <= 4) SKINNY(4);
-  else if (m <= 8) SKINNY(8);
-  else SKINNY(16);
+#define SKINNY_ROWS(MT, ROWS) \
+  skinny_fma_kernel<TA, TW, TO, MT, ROWS><<<(n + 4 * ROWS - 1) / (4 * ROWS), 256, 0, stream>>>((const TA*)a, (const TW*)w, bias, (TO*)out, m, n, k)
+#define SKINNY(MT)                                                              \
+  {                                                                             \
+    if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4 && sizeof(TO) == 4) {      \
+      if (MT >= 3 && (long long)n * m >= 360000) SKINNY_ROWS(MT, (MT >= 3 ? 8 : 4)); \
+      else if (n < 16 * 256) SKINNY_ROWS(MT, 2);                                \
+      else SKINNY_ROWS(MT, 4);                                                  \
+    } else {                                                                    \
+      SKINNY_ROWS(MT, 4);                                                       \
+    }                                                                           \
+  }
+  if (m <= 1) SKINNY(1)
+  else if (m <= 2) SKINNY(2)
+  else if (m <= 3) SKINNY(3)
+  else if (m <= 4) SKINNY(4)
+  else if (m <= 6) SKINNY(6)
+  else if (m <= 8) SKINNY(8)
+  else if (m <= 12) SKINNY(12)
+  else SKINNY(16)
 #undef SKINNY
+#undef SKINNY_ROWS
 }
 
 extern "C" int velox_gemm_fma(const void* a, const void* w, const float* bias, void* out, int m, int n, int k,
