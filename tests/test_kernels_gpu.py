@@ -1426,6 +1426,15 @@ def test_grouped_products_in_tiles_of_128_and_192_rows(ops, monkeypatch, rows, h
     assert torch.equal(experts_against_float64(ops, rows, hidden, inter, top, scale_input, unit), first)
 
 
+@pytest.mark.parametrize("hidden, inter", [(64, 64), (128, 24), (192, 136), (320, 64), (1088, 200)])
+@pytest.mark.parametrize("scale_input, unit", [(False, "glu"), (True, "relu2")])
+def test_grouped_products_of_few_rows_that_read_whole_lines(ops, hidden, inter, scale_input, unit):
+    """At most 64 pairs: sums that are a multiple of 64 terms read W in whole lines, in quarters that end inside a round and with waves without
+    any; outputs that end among the first or the second eight rows of a tile; one, two and four tiles of rows."""
+    for rows in ((1, 0, 16), (30, 2, 1), (40, 24)):
+        experts_against_float64(ops, rows, hidden, inter, 1, scale_input, unit)
+
+
 @pytest.mark.parametrize("hidden, inter", [(64, 2432), (64, 3200), (64, 5120), (4864, 64), (6400, 64), (10240, 64)])
 @pytest.mark.parametrize("scale_input, unit", [(False, "glu"), (True, "relu2")])
 def test_grouped_products_in_tiles_of_192_and_256_columns(ops, monkeypatch, hidden, inter, scale_input, unit):

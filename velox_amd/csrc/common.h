@@ -94,6 +94,19 @@ __device__ __forceinline__ StepItem step_item(const int* cu_q, int num_seqs, int
   return found;
 }
 
+// Rows of a matrix as the left operand of v_mfma_f32_16x16x32_bf16 want them, lane (g, i) two pieces of 16 bytes of row i, from loads of whole
+// cache lines: what a lane asks for is `first` of row i & 7 and `second` of row 8 + (i & 7), the lanes with i >= 8 the other of the two
+// pieces, so that a load covers eight rows of 128 bytes and not sixteen of 64.  Lanes eight apart then change places.  (Read once and
+// in whole lines W streams at up to 7 TB/s past the caches; sixteen half lines a load, at 5.3 to 6.3, and the hint costs speed there.)
+__device__ __forceinline__ void rows_from_lines(float4_t& first, float4_t& second) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int a = __float_as_int(first[d]), b = __float_as_int(second[d]);
+    first[d] = __int_as_float(__builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0xc, false));   // lanes 8 .. 15 of 16 from eight lanes down,
+    second[d] = __int_as_float(__builtin_amdgcn_update_dpp(b, a, 0x128, 0xf, 0x3, false));  // lanes 0 .. 7 from eight lanes up
+  }
+}
+
 // The sequence with the `rank`-th most tokens, ties in their order (beyond 64 sequences: from the back, since a step's single tokens come before
 // its portions of prompts).  The whole wave takes part.  For grids of a workgroup per sequence whose time is the longest chain's: it
 // has to begin with the first workgroups.

@@ -180,8 +180,9 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
 // round ahead, and the waves' sums are added through LDS in the order of the waves (no atomics: the same result on every
 // run).  A tile works as many 16-row tiles as it has rows, whatever the step's number of pairs would allow.  With `row_scale` the
 // rows are scaled in registers, behind the wait for them and before that for W: the same bits as a scaled copy.  Measured on MI355X: 64
-// pairs over 32 experts of 4,096 -> 1,408 -> 4,096 122 + 70 us (W: 650 + 325 MB; before: 143 + 82, rows copied by another kernel).
-template <int EPI, typename TO, int MT>
+// pairs over 32 experts of 4,096 -> 1,408 -> 4,096 193 us both products, 180 with W in whole lines past the caches (W: 650 + 325 MB), in a step 121 +
+// 66 and 107 + 67; 24 pairs over 16 experts of 2,048 -> 1,408 -> 2,048 61.6 and 56.5.
+template <int EPI, typename TO, int MT, bool LINES>
 __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int group, const int row0, const int rows, const int* order,
                                               float4_t (*partial)[8][64]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -191,12 +192,16 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
   col0[0] = blockIdx.x * (EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS);
   col0[1] = EPI == GM_GLU ? col0[0] : col0[0] + 16;
   const bf16_t* w_base = args.w + (size_t)group * args.w_group;
-  const bf16_t* w_row[2];
+  // LINES (k % 64 == 0): W in whole cache lines, see rows_from_lines; a pair of loads is two steps of 32 indices
+  const int piece = LINES ? 8 * (g4 + 4 * (i >> 3)) : 8 * g4;
+  const bf16_t* w_row[2][LINES ? 2 : 1];
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int col = min(col0[t] + i, n - 1);
-    w_row[t] = w_base + (size_t)(EPI == GM_GLU && t == 1 ? n + col : col) * k + 8 * g4;
-  }
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int half = 0; half < (LINES ? 2 : 1); ++half) {
+      const int col = min(col0[t] + (LINES ? 8 * half + (i & 7) : i), n - 1);
+      w_row[t][half] = w_base + (size_t)(EPI == GM_GLU && t == 1 ? n + col : col) * k + piece;
+    }
   const int quarter = ((k + 127) / 128) * 32;  // indices per wave: a multiple of 32
   const int k_begin = wave * quarter, k_end = min(k, k_begin + quarter);
   // W is what there is to read: its next step is asked for before the current one is multiplied, and its first before the rows of
@@ -206,7 +211,26 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) w_next[t][u] = gm_load(w_row[t] + k0 + 32 * u, k0 + 32 * u + 8 * g4 < k_end);
+      for (int t = 0; t < 2; ++t) {
+        if constexpr (LINES) {
+          const int at = k0 + 64 * (u / 2);
+          w_next[t][u] = at + piece < k_end ? __builtin_bit_cast(gm_bf16x8_t, __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(w_row[t][u % 2] + at)))
+                                            : __builtin_bit_cast(gm_bf16x8_t, float4_t{0.f, 0.f, 0.f, 0.f});
+        } else {
+          w_next[t][u] = gm_load(w_row[t][0] + k0 + 32 * u, k0 + 32 * u + 8 * g4 < k_end);
+        }
+      }
+  };
+  auto take = [&](int t, int u) {  // steps u and u + 1
+    if constexpr (LINES) {
+      float4_t first = __builtin_bit_cast(float4_t, w_next[t][u]), second = __builtin_bit_cast(float4_t, w_next[t][u + 1]);
+      rows_from_lines(first, second);
+      wv[t][u] = __builtin_bit_cast(gm_bf16x8_t, first);
+      wv[t][u + 1] = __builtin_bit_cast(gm_bf16x8_t, second);
+    } else {
+      wv[t][u] = w_next[t][u];
+      wv[t][u + 1] = w_next[t][u + 1];
+    }
   };
   ask(k_begin);
   const bf16_t* a_row[MT];
@@ -228,8 +252,10 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
     gm_bf16x8_t av[MT][4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
+      if (u % 2 == 0) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) wv[t][u] = w_next[t][u];
+        for (int t = 0; t < 2; ++t) take(t, u);
+      }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) av[mt][u] = gm_load(a_row[mt] + k0 + 32 * u, k0 + 32 * u + 8 * g4 < k_end);
     }
@@ -289,7 +315,7 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
   }
 }
 
-template <int EPI, typename TO>
+template <int EPI, typename TO, bool LINES>
 __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const GroupedArgs args) {
   static_assert(EPI == GM_PLAIN || EPI == GM_GLU || EPI == GM_ACT, "no gate here");
   __shared__ float4_t partial[3][8][64];
@@ -302,9 +328,9 @@ __global__ void __launch_bounds__(256) grouped_mfma_few_rows_kernel(const Groupe
   const int group = tile_group[tile], row0 = tile_row[tile];
   const int rows = min(64, starts[group + 1] - row0);
   // (the same for the whole workgroup)
-  if (rows <= 16) few_rows_tile<EPI, TO, 1>(args, group, row0, rows, order, partial);
-  else if (rows <= 32) few_rows_tile<EPI, TO, 2>(args, group, row0, rows, order, partial);
-  else few_rows_tile<EPI, TO, 4>(args, group, row0, rows, order, partial);
+  if (rows <= 16) few_rows_tile<EPI, TO, 1, LINES>(args, group, row0, rows, order, partial);
+  else if (rows <= 32) few_rows_tile<EPI, TO, 2, LINES>(args, group, row0, rows, order, partial);
+  else few_rows_tile<EPI, TO, 4, LINES>(args, group, row0, rows, order, partial);
 }
 
 // Tiles of the plan, as far as the host can tell: an expert's rows taken to lie evenly between 0.65 and 1.35 of their mean (16 experts, 2,072
@@ -377,7 +403,9 @@ template <int EPI, typename TO>
 static int grouped_plan_launch(const GroupedArgs& args, int tile_rows, int most_tiles, hipStream_t stream) {
   if (tile_rows == 64) {
     constexpr int COLS = EPI == GM_GLU ? GM_FEW_COLS / 2 : GM_FEW_COLS;
-    grouped_mfma_few_rows_kernel<EPI, TO><<<dim3((args.n + COLS - 1) / COLS, most_tiles), 256, 0, stream>>>(args);
+    const dim3 grid((args.n + COLS - 1) / COLS, most_tiles);
+    if (args.k % 64 == 0) grouped_mfma_few_rows_kernel<EPI, TO, true><<<grid, 256, 0, stream>>>(args);
+    else grouped_mfma_few_rows_kernel<EPI, TO, false><<<grid, 256, 0, stream>>>(args);
     return (int)hipGetLastError();
   }
   TileArgs tiles = {};

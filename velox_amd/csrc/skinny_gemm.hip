@@ -44,6 +44,22 @@ __device__ __forceinline__ Run16 load_run_packed(const bf16_t* p) {
   return r;
 }
 
+// The two pieces that a lane asks for of a row-major W, and its run behind the exchange (see rows_from_lines).
+__device__ __forceinline__ Run16 load_run_lines(const bf16_t* first, const bf16_t* second) {
+  Run16 r;
+  r.lo = __builtin_bit_cast(bf16x8_t, __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(first)));
+  r.hi = __builtin_bit_cast(bf16x8_t, __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(second)));
+  return r;
+}
+__device__ __forceinline__ Run16 run_from_lines(const Run16& r) {
+  float4_t first = __builtin_bit_cast(float4_t, r.lo), second = __builtin_bit_cast(float4_t, r.hi);
+  rows_from_lines(first, second);
+  Run16 out;
+  out.lo = __builtin_bit_cast(bf16x8_t, first);
+  out.hi = __builtin_bit_cast(bf16x8_t, second);
+  return out;
+}
+
 // the two halves `half` elements apart (8: one run of 32 bytes; 512: the packed layout, read through the caches)
 __device__ __forceinline__ Run16 load_run_halves(const bf16_t* p, int half) {
   Run16 r;
@@ -108,6 +124,7 @@ __device__ __forceinline__ void skinny_partial_sums(const bf16_t* __restrict__ a
   if (kb_hi > blocks_total) kb_hi = blocks_total;
 
   const bf16_t* w_ptr[RT];
+  const bf16_t* w_far[PACKED ? 1 : RT];
   bool w_ok[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
@@ -119,9 +136,11 @@ __device__ __forceinline__ void skinny_partial_sums(const bf16_t* __restrict__ a
       w_ok[rt] = n0 + 16 * (rt % RTO) < n;  // padded rows are zeros in memory
       w_ptr[rt] = w + (w_ok[rt] ? tile : 0) * (size_t)(k / 64) * 1024 + lane * 8;
       w_ok[rt] = w_ok[rt] && (w_half < 0 || (i >> 3) == w_half);
-    } else {
-      const size_t row = (size_t)col + (rt >= RTO ? n : 0);  // its row in W
-      w_ptr[rt] = w + (w_ok[rt] ? row : 0) * k + 16 * g;
+    } else {  // (whole cache lines, see rows_from_lines: a row beyond W is its last one again, its sums are never stored)
+      const size_t before = rt >= RTO ? n : 0;
+      w_ptr[rt] = w + (before + min(n0 + 16 * (rt % RTO) + (i & 7), n - 1)) * k + 16 * g + 8 * (i >> 3);
+      w_far[rt] = w + (before + min(n0 + 16 * (rt % RTO) + 8 + (i & 7), n - 1)) * k + 16 * g + 8 * (i >> 3);
+      w_ok[rt] = true;
     }
   }
   const bf16_t* a_ptr[CT];
@@ -150,19 +169,21 @@ __device__ __forceinline__ void skinny_partial_sums(const bf16_t* __restrict__ a
       const size_t k0 = (size_t)(kb + u) * 64;
       const size_t w0 = PACKED ? (size_t)(kb + u) * 1024 : k0;
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) wr[u][rt] = (in_range && w_ok[rt]) ? (PACKED ? load_run_packed(w_ptr[rt] + w0) : load_run(w_ptr[rt] + w0)) : zero_run();
+      for (int rt = 0; rt < RT; ++rt) wr[u][rt] = (in_range && w_ok[rt]) ? (PACKED ? load_run_packed(w_ptr[rt] + w0) : load_run_lines(w_ptr[rt] + w0, w_far[PACKED ? 0 : rt] + w0)) : zero_run();
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) ar[u][ct] = (in_range && a_ok[ct]) ? load_run_halves(a_ptr[ct] + (size_t)(kb + u) * a_block, a_half) : zero_run();
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
+      for (int rt = 0; rt < RT; ++rt) {
+        if constexpr (!PACKED) wr[u][rt] = run_from_lines(wr[u][rt]);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
           acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u][rt].lo, ar[u][ct].lo, acc[rt][ct], 0, 0, 0);
           acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u][rt].hi, ar[u][ct].hi, acc[rt][ct], 0, 0, 0);
         }
+      }
     if (kb == kb_lo) hooks.after_first();
   }
 
