@@ -823,6 +823,17 @@ def test_decoded_tokens_whose_keys_are_shared_out(ops, ref, dtype, nh, nkv, d, p
     assert torch.equal(run(moved), got[order])
 
 
+@pytest.mark.parametrize("m,n,k", [(17, 16384, 64), (32, 16388, 448), (33, 20004, 256), (64, 16400, 192)])
+def test_a_head_of_some_rows_streams_its_packed_copy(ops, m, n, k):
+    """Float32 results of 17 to 64 rows of a registered weight: products of bfloat16 numbers, exact in float32, and k additions."""
+    x, w = rand((m, k), torch.bfloat16, 63), rand((n, k), torch.bfloat16, 64)
+    got = ops.linear(x, ops.prepare_weight(w), None, torch.float32)
+    assert got.shape == (m, n) and got.dtype == torch.float32 and got.is_contiguous()
+    want = x.double() @ w.double().T
+    assert torch.all((got.double() - want).abs() <= k * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T) + 1e-30)
+    assert torch.equal(got, ops.skinny_gemm_splitk(x, w, splits=1, packed=ops.pack_rows(w))[0])
+
+
 @pytest.mark.parametrize("n,k", [(7, 260), (4094, 36), (4099, 512), (120001, 8), (30002, 300)])
 def test_gemm_fma_of_few_rows_in_every_shape(ops, n, k):
     """Two, four and eight rows of W a wave, numbers of rows of A between those that are built: a product's bits are those of each of its rows

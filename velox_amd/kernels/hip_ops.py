@@ -834,6 +834,12 @@ class HipOps:
         if (partials_ok and bias is None and self.use_skinny_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
                 and 16 < m <= 64 and k % 64 == 0 and n <= 8192 and n % 4 == 0):
             return self.skinny_gemm_splitk(x, weight, packed=packed)
+        if (out_dtype == torch.float32 and bias is None and packed is not None and self.use_skinny_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+                and 16 < m <= 64 and k % 64 == 0 and n % 4 == 0 and n >= 64 * self.num_cus and (m <= 32 or n <= 65536)):
+            # The head over more rows than the skinny kernel takes: the kernel that stages the activations of 64 rows of W streams the packed copy.
+            # Measured on MI355X (us, the library / this): 152,064 x 3,584, 17 rows 253 / 192, 25 257 / 203, 33 207 / 220, 57 221 / 243; 151,936 x 1,536,
+            # 25 109 / 98, 57 119 / 120; 32,000 x 4,096, 17 61 / 49, 33 62 / 52, 57 64 / 55.
+            return self.skinny_gemm_splitk(x, weight, splits=1, packed=packed)[0]
         if out_dtype == torch.bfloat16 and self.use_library_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
             parts = self.own_tile_parts(m, n, k, partials_ok and bias is None)
             if parts > 0 and not self._library_has_timed(m, n, k):
