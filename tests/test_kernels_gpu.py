@@ -870,6 +870,36 @@ def test_a_few_rows_into_the_residual(ops, ref, m, n, k):
     torch.testing.assert_close(residual, other, rtol=1e-5, atol=1e-5 * float(want.abs().max()))
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+@pytest.mark.parametrize("nh,nkv,d,k,page", [(4, 2, 64, 128, 4), (12, 2, 128, 1536, 16), (5, 2, 96, 192, 1), (28, 2, 128, 1088, 8), (16, 4, 32, 64, 16)])
+@pytest.mark.parametrize("use_bias", [True, False])
+def test_qkv_projection_of_a_few_rows_in_halves_of_its_tiles(ops, m, nh, nkv, d, k, page, use_bias):
+    """Against the kernel for up to 16 rows (``waves=8`` asks for it), with plain rows and with rows whose norm is still to be taken: the same
+    sums of exact products in another order of additions, rounded to bfloat16 once."""
+    from velox_amd.parts.base import ResidualSink
+    from velox_amd.parts.norms import RMSNorm
+
+    width, half = (nh + 2 * nkv) * d, d // 2
+    assert 512 <= width <= 16 * ops.num_cus and (ops._few_rows_pieces(m, k) <= 2 or m > 2)  # (three and four rows of the longer sums stay)
+    w, bias = ops.prepare_weight(rand((width, k), torch.bfloat16, 71, 0.05), rotary_heads=(nh, nkv, d)), rand((width,), torch.float32, 72) if use_bias else None
+    angles = torch.outer(torch.arange(64, dtype=torch.float32), 1.0 / (10000.0 ** (torch.arange(half, dtype=torch.float32) / half)))
+    cos, sin = angles.cos().cuda(), angles.sin().cuda()
+    positions, slots = torch.tensor([9, 0, 63, 5][:m], dtype=torch.int32).cuda(), torch.tensor([page, 3 * page - 1, 4 * page, 2 * page][:m], dtype=torch.int32).cuda()
+    norm = RMSNorm("", k, 1e-6)
+    norm.weight = 1.0 + rand((k,), torch.float32, 73, 0.1)
+    rows = rand((m, k), torch.bfloat16, 74)
+    deferred = ops.linear(rand((m, 256), torch.bfloat16, 75), ops.prepare_weight(rand((k, 256), torch.bfloat16, 76, 0.1)), None, torch.bfloat16,
+                          residual_norm=ResidualSink(rand((m, k), torch.float32, 77), norm))
+    for x in (rows, deferred):
+        results = []
+        for more in ({}, {"waves": 8}):
+            k_cache, v_cache = torch.full((5, nkv, page, d), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((5, nkv, d, page), 7.0, dtype=torch.bfloat16, device="cuda")
+            results.append((ops.qkv_rope_write(x, w, bias, nh, nkv, d, positions, cos, sin, slots, k_cache, v_cache, page, **more), k_cache, v_cache))
+        for got, want in zip(*results):
+            scale = float(want.float().abs().max())
+            torch.testing.assert_close(got.float(), want.float(), rtol=2.0 ** -7, atol=k * 2.0 ** -22 * scale)
+
+
 @pytest.mark.parametrize("nh,nkv,d,n,lens", [(12, 2, 128, 1536, [391]), (12, 2, 128, 1536, [1000, 3]), (28, 4, 128, 3584, [2048]), (14, 2, 64, 896, [100, 70, 128, 1]), (12, 2, 48, 512, [65])])
 def test_parts_of_an_attention_that_the_output_product_merges(ops, ref, nh, nkv, d, n, lens):
     from velox_amd.engine.batch import Workspace

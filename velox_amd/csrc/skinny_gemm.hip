@@ -609,30 +609,24 @@ struct AttentionParts {
   int splits, heads, dim;
 };
 constexpr int FEW_WAVES = 4, FEW_PAIRS = 4;
-template <int STAGED, int PARTS>
-__global__ void __launch_bounds__(FEW_WAVES * 64) skinny_few_rows_residual_kernel(const bf16_t* __restrict__ a, const AttentionParts parts, const bf16_t* __restrict__ w,
-                                                                                  float* __restrict__ residual, const float* __restrict__ norm_weight,
-                                                                                  bf16_t* __restrict__ next, float* __restrict__ sums, int m, int n, int k) {
-  __shared__ float4_t partial[FEW_WAVES][64];
+
+// The sums of half `half` (eight rows) of TILES row tiles of a packed W, left in partial[wave][tile][lane] with a barrier behind: lane (g, i) of the
+// first 32 holds rows 4 g .. + 3 of the half for row i of A as far as even blocks go, the lane 32 on the same of odd ones.  `after` runs
+// behind the first loads of W.
+template <int STAGED, int PARTS, int TILES, typename After, typename Before>
+__device__ __forceinline__ void few_rows_sums(const bf16_t* __restrict__ a, const AttentionParts& parts, const bf16_t* __restrict__ w, int first_tile, int half, int m, int k,
+                                              float4_t (&partial)[FEW_WAVES][TILES][64], After after, Before before_barrier) {
   __shared__ __attribute__((aligned(16))) bf16_t staged[FEW_WAVES][STAGED * 512];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, i = lane & 15;
-  const int tile = blockIdx.x >> 1, half = blockIdx.x & 1;
-  const int col = tile * 16 + 8 * half + 4 * g;  // (epilogue, lanes 0 .. 31 of the first wave: row i's columns col .. + 3)
-  const bool finishes = threadIdx.x < 32 && i < m;
-  float old_residual[4], weight[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const bool inside = finishes && col + j < n;
-    old_residual[j] = inside ? residual[(size_t)i * n + col + j] : 0.f;
-    weight[j] = inside ? norm_weight[col + j] : 0.f;
-  }
   // this wave's share of K, in pairs of blocks of 64 (the last pair's second block may not be there)
   const int blocks = k / 64, pairs = (blocks + 1) / 2, per_wave = (pairs + FEW_WAVES - 1) / FEW_WAVES;
   const int lo = min(wave * per_wave, pairs), hi = min(lo + per_wave, pairs);
   const int slice = 64 * (min(2 * hi, blocks) - min(2 * lo, blocks));
-  const bf16_t* w_lane = w + (size_t)tile * blocks * 1024 + (16 * g + 8 * half + (i & 7)) * 8;
-  float4_t even = {0.f, 0.f, 0.f, 0.f}, odd = {0.f, 0.f, 0.f, 0.f};
+  const bf16_t* w_lane = w + (size_t)first_tile * blocks * 1024 + (16 * g + 8 * half + (i & 7)) * 8;
+  float4_t even[TILES], odd[TILES];
+#pragma unroll
+  for (int tile = 0; tile < TILES; ++tile) even[tile] = odd[tile] = float4_t{0.f, 0.f, 0.f, 0.f};
   if (lo < hi) {
     float4_t piece[STAGED], merged[PARTS ? STAGED : 1][PARTS ? 2 * PARTS : 1];
     float logs[PARTS ? STAGED : 1][PARTS ? PARTS : 1];
@@ -654,15 +648,17 @@ __global__ void __launch_bounds__(FEW_WAVES * 64) skinny_few_rows_residual_kerne
         piece[t] = *reinterpret_cast<const float4_t*>(a + (size_t)row * k + c);
       }
     }
-    struct Group { Run16 w[FEW_PAIRS]; } x, y;
+    struct Group { Run16 w[FEW_PAIRS][TILES]; } x, y;
     auto load = [&](Group& q, int p0) {
 #pragma unroll
       for (int u = 0; u < FEW_PAIRS; ++u) {
         const int p = min(p0 + u, hi - 1);
-        q.w[u] = load_run_packed(w_lane + (size_t)(i < 8 ? 2 * p : min(2 * p + 1, blocks - 1)) * 1024);
+#pragma unroll
+        for (int tile = 0; tile < TILES; ++tile) q.w[u][tile] = load_run_packed(w_lane + ((size_t)tile * blocks + (i < 8 ? 2 * p : min(2 * p + 1, blocks - 1))) * 1024);
       }
     };
     load(x, lo);
+    after();
 #pragma unroll
     for (int t = 0; t < STAGED; ++t) {
       if constexpr (PARTS > 0) {
@@ -697,11 +693,17 @@ __global__ void __launch_bounds__(FEW_WAVES * 64) skinny_few_rows_residual_kerne
       for (int u = 0; u < FEW_PAIRS; ++u) {
         if (p0 + u >= hi) break;  // (uniform over the wave)
         const bf16x8_t* first = reinterpret_cast<const bf16x8_t*>(row + (p0 + u - lo) * 128);
-        even = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u].lo, first[0], even, 0, 0, 0);
-        even = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u].hi, first[1], even, 0, 0, 0);
+#pragma unroll
+        for (int tile = 0; tile < TILES; ++tile) {
+          even[tile] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u][tile].lo, first[0], even[tile], 0, 0, 0);
+          even[tile] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u][tile].hi, first[1], even[tile], 0, 0, 0);
+        }
         if (2 * (p0 + u) + 1 < blocks) {
-          odd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u].lo, first[8], odd, 0, 0, 0);
-          odd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u].hi, first[9], odd, 0, 0, 0);
+#pragma unroll
+          for (int tile = 0; tile < TILES; ++tile) {
+            odd[tile] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u][tile].lo, first[8], odd[tile], 0, 0, 0);
+            odd[tile] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[u][tile].hi, first[9], odd[tile], 0, 0, 0);
+          }
         }
       }
     };
@@ -718,14 +720,44 @@ __global__ void __launch_bounds__(FEW_WAVES * 64) skinny_few_rows_residual_kerne
       p += FEW_PAIRS;
     }
   }
-  partial[wave][lane] = lane < 32 ? even : odd;  // (rows 0 .. 7 of the one, 8 .. 15 of the other)
+  else {
+    after();
+  }
+#pragma unroll
+  for (int tile = 0; tile < TILES; ++tile) partial[wave][tile][lane] = lane < 32 ? even[tile] : odd[tile];  // (rows 0 .. 7 of the one, 8 .. 15 of the other)
+  before_barrier();
   __syncthreads();
+}
+// lane 0 .. 31's four sums of a tile
+template <int TILES>
+__device__ __forceinline__ float4_t few_rows_sum(const float4_t (&partial)[FEW_WAVES][TILES][64], int tile, int lane) {
+  float4_t sum = partial[0][tile][lane] + partial[0][tile][lane + 32];
+#pragma unroll
+  for (int wv = 1; wv < FEW_WAVES; ++wv) sum += partial[wv][tile][lane] + partial[wv][tile][lane + 32];
+  return sum;
+}
+
+template <int STAGED, int PARTS>
+__global__ void __launch_bounds__(FEW_WAVES * 64) skinny_few_rows_residual_kernel(const bf16_t* __restrict__ a, const AttentionParts parts, const bf16_t* __restrict__ w,
+                                                                                  float* __restrict__ residual, const float* __restrict__ norm_weight,
+                                                                                  bf16_t* __restrict__ next, float* __restrict__ sums, int m, int n, int k) {
+  __shared__ float4_t partial[FEW_WAVES][1][64];
+  const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
+  const int tile = blockIdx.x >> 1, half = blockIdx.x & 1;
+  const int col = tile * 16 + 8 * half + 4 * g;  // (epilogue, lanes 0 .. 31 of the first wave: row i's columns col .. + 3)
+  const bool finishes = threadIdx.x < 32 && i < m;
+  float old_residual[4], weight[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const bool inside = finishes && col + j < n;
+    old_residual[j] = inside ? residual[(size_t)i * n + col + j] : 0.f;
+    weight[j] = inside ? norm_weight[col + j] : 0.f;
+  }
+  few_rows_sums<STAGED, PARTS, 1>(a, parts, w, tile, half, m, k, partial, Nothing(), Nothing());
   if (threadIdx.x >= 64) return;
   float squares = 0.f;
   if (finishes) {
-    float4_t sum = partial[0][lane] + partial[0][lane + 32];
-#pragma unroll
-    for (int wv = 1; wv < FEW_WAVES; ++wv) sum += partial[wv][lane] + partial[wv][lane + 32];
+    const float4_t sum = few_rows_sum<1>(partial, 0, lane);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if (col + j >= n) break;
@@ -766,6 +798,76 @@ extern "C" int velox_skinny_few_rows_residual_bf16(const void* a, const void* w,
     else return -1;
   }
 #undef FEW_ROWS
+  return (int)hipGetLastError();
+}
+
+// The query/key/value product of up to four rows (skinny_qkv_rotary_kernel in halves of its two row tiles, with the loads of the kernel above): a narrow
+// W then has twice as many workgroups.  Measured on MI355X, us, whole tiles / halves: 1,536 -> 2,048, 1 and 2 rows 5.6 / 5.1,
+// 5.7 / 5.4; 2,048 -> 3,072, 1 and 2 rows 6.9 / 5.9, 6.5 / 6.1; 896 -> 1,152 4.8 / 4.5; with more halves than compute units 3,584 -> 4,608 9.6 / 11.2.
+template <int STAGED>
+__global__ void __launch_bounds__(FEW_WAVES * 64) skinny_few_rows_qkv_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const RotaryWrite args, int m, int k,
+                                                                             const RowScale rs) {
+  __shared__ float4_t partial[FEW_WAVES][2][64];
+  __shared__ float scale_part[FEW_WAVES][16];
+  __shared__ float scale_stage[FEW_WAVES][ROW_SCALE_ROUNDS][64];
+  const int lane = threadIdx.x & 63, g = lane >> 4, row = lane & 15, row_in = row < m ? row : 0;
+  const int pair = blockIdx.x >> 1, half = blockIdx.x & 1;  // of row tiles; rows 8 half .. + 7 of either
+  const int d = args.d, angles = d / 2, head = pair / (d / 32), j = pair % (d / 32);
+  const bool rotated = head < args.heads + args.kv_heads;
+  // (lanes 0 .. 31 of the first wave finish; the others ask for the same)
+  const int c = (rotated ? 16 : 32) * j + 8 * half + 4 * (g & 1), partner = rotated ? angles : 16;
+  const int slot = args.slots[row_in], position = args.positions[row_in];
+  const float* bias_at = args.bias ? args.bias + (size_t)head * d + c : args.cos_table;
+  float4_t bias_first = *reinterpret_cast<const float4_t*>(bias_at), bias_second = *reinterpret_cast<const float4_t*>(bias_at + (args.bias ? partner : 0));
+  float4_t cs = float4_t{1.f, 1.f, 1.f, 1.f}, sn = float4_t{0.f, 0.f, 0.f, 0.f};
+  auto fetch_angles = [&] {
+    const size_t angle = (size_t)position * angles + (rotated ? c : 0);
+    cs = *reinterpret_cast<const float4_t*>(args.cos_table + angle);
+    sn = *reinterpret_cast<const float4_t*>(args.sin_table + angle);
+  };
+  RowScaleLoads<FEW_WAVES>::issue(rs, m, scale_stage);
+  few_rows_sums<STAGED, 0, 2>(a, AttentionParts{}, w, 2 * pair, half, m, k, partial, fetch_angles, [&] { RowScaleLoads<FEW_WAVES>::leave(rs, scale_stage, scale_part); });
+  if (threadIdx.x >= 32 || row >= m) return;
+  const float row_scale = row_scale_of<FEW_WAVES>(rs, scale_part, row);
+  if (!args.bias) bias_first = bias_second = float4_t{0.f, 0.f, 0.f, 0.f};
+  const float4_t first = few_rows_sum<2>(partial, 0, lane) * row_scale + bias_first, second = few_rows_sum<2>(partial, 1, lane) * row_scale + bias_second;
+  const size_t page = (size_t)(slot / args.page_size);
+  const int offset = slot % args.page_size;
+  if (rotated) {
+    __attribute__((aligned(8))) bf16_t low[4];
+    __attribute__((aligned(8))) bf16_t high[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      low[e] = from_f32<bf16_t>(first[e] * cs[e] - second[e] * sn[e]);
+      high[e] = from_f32<bf16_t>(first[e] * sn[e] + second[e] * cs[e]);
+    }
+    bf16_t* dst = head < args.heads ? args.q_out + ((size_t)row * args.heads + head) * d + c
+                                    : args.k_cache + (((page * args.kv_heads + (head - args.heads)) * args.page_size) + offset) * d + c;
+    typedef float float2_t __attribute__((ext_vector_type(2)));
+    *reinterpret_cast<float2_t*>(dst) = *reinterpret_cast<const float2_t*>(low);
+    *reinterpret_cast<float2_t*>(dst + angles) = *reinterpret_cast<const float2_t*>(high);
+  } else {
+    bf16_t* dst = args.v_cache + ((page * args.kv_heads + (head - args.heads - args.kv_heads)) * d + c) * args.page_size + offset;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      dst[(size_t)e * args.page_size] = from_f32<bf16_t>(first[e]);
+      dst[(size_t)(16 + e) * args.page_size] = from_f32<bf16_t>(second[e]);
+    }
+  }
+}
+
+// As velox_skinny_qkv_rotary_bf16, for rows whose activations fit two pieces and at most 256 sums of squares a row; -1 otherwise.
+extern "C" int velox_skinny_few_rows_qkv_bf16(const void* a, const void* w, const float* bias, const int* positions, const float* cos_table, const float* sin_table,
+                                              const int* slots, void* q_out, void* k_cache, void* v_cache, int m, int k, int heads, int kv_heads, int d, int page_size,
+                                              const float* scale_partial, int scale_blocks, float inv_width, float eps, hipStream_t stream) {
+  if (m <= 0) return 0;
+  const int pairs = (k / 64 + 1) / 2, pieces = (m * ((pairs + FEW_WAVES - 1) / FEW_WAVES) * 128 + 511) / 512;
+  if (m > 16 || k % 64 != 0 || d % 32 != 0 || heads < 1 || kv_heads < 1 || page_size < 1 || pieces > 2 || (scale_partial != nullptr && scale_blocks > ROW_SCALE_BLOCKS / 2)) return -1;
+  const RotaryWrite args{bias, positions, cos_table, sin_table, slots, (bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, heads, kv_heads, d, page_size};
+  const RowScale rs{scale_partial, scale_blocks, inv_width, eps};
+  const int grid = (heads + 2 * kv_heads) * d / 16;
+  if (pieces <= 1) skinny_few_rows_qkv_kernel<1><<<grid, FEW_WAVES * 64, 0, stream>>>((const bf16_t*)a, (const bf16_t*)w, args, m, k, rs);
+  else skinny_few_rows_qkv_kernel<2><<<grid, FEW_WAVES * 64, 0, stream>>>((const bf16_t*)a, (const bf16_t*)w, args, m, k, rs);
   return (int)hipGetLastError();
 }
 

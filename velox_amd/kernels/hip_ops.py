@@ -135,6 +135,8 @@ class HipOps:
         c.velox_skinny_residual_norm_bf16.restype = _I
         c.velox_skinny_few_rows_residual_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P, _P, _I, _I, _I, _P]
         c.velox_skinny_few_rows_residual_bf16.restype = _I
+        c.velox_skinny_few_rows_qkv_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _F, _F, _P]
+        c.velox_skinny_few_rows_qkv_bf16.restype = _I
         c.velox_row_scale_apply.argtypes = [_P, _P, _I, _F, _F, _P, _I, _I, _P]
         c.velox_skinny_gemm_bf16.restype = _I
         c.velox_skinny_gemm_glu_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _F, _F, _I, _P, _P]
@@ -1811,6 +1813,14 @@ class HipOps:
         self._check("v_cache", v_cache, torch.bfloat16, (pages, num_kv_heads, head_dim, block_size), align=16)
         q = torch.empty((m, num_heads * head_dim), dtype=torch.bfloat16, device=self.device)
         x_packed = self._packed_rows_of(x, k)
+        # a few rows of a narrow weight: halves of its tiles, which are then at most a workgroup per compute unit (see the kernel)
+        if (waves is None and x_packed is None and m <= 4 and 512 <= width <= 16 * self.num_cus and self._few_rows_pieces(m, k) <= 2
+                and (deferred is None or deferred.sums.shape[1] <= 256)):
+            status = self._core.velox_skinny_few_rows_qkv_bf16(
+                _ptr(x), _ptr(packed), _ptr(bias), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(slot_mapping), _ptr(q), _ptr(k_cache), _ptr(v_cache),
+                m, k, num_heads, num_kv_heads, head_dim, block_size, *self._scale_args(deferred), self._stream())
+            self._launched(status, "skinny_few_rows_qkv")
+            return q
         status = self._core.velox_skinny_qkv_rotary_bf16(
             _ptr(x if x_packed is None else x_packed), _ptr(packed), _ptr(bias), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(slot_mapping), _ptr(q), _ptr(k_cache),
             _ptr(v_cache), m, k, num_heads, num_kv_heads, head_dim, block_size, int(waves or 8), *self._scale_args(deferred),
