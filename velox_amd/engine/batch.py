@@ -43,14 +43,15 @@ class WorkspaceError(RuntimeError):
 
 
 class Workspace:
-    """Scratch tensors by name, kept across steps so their addresses are stable.  A buffer begins as zeros (counters that their kernels
-    leave at zero need it).
+    """Scratch tensors by name, kept across steps so their addresses are stable.
 
     A captured step holds the addresses of the buffers it was captured with, so a buffer must never be replaced once a
     capture may exist.  The runner therefore asks every part what it can need at most (``Part.workspace_needs``),
     reserves that before anything runs and calls :meth:`fix`; from then on a request for more than is there is an
     error, not a new allocation.  A workspace that was never fixed (a test's own) grows on demand.
     """
+
+    counters = ("attention_arrivals",)  # buffers that begin as zeros, as their kernels leave them
 
     def __init__(self, device) -> None:
         self.device = device
@@ -66,7 +67,8 @@ class Workspace:
             have = "nothing" if buf is None else f"{buf.numel()} x {buf.dtype}"
             raise WorkspaceError(f"workspace buffer {name!r} holds {have} but {numel} x {dtype} are asked for; captured steps hold its "
                                  "address, so it cannot be replaced (the part that uses it must state this size in workspace_needs)")
-        self._buffers[name] = torch.zeros(max(int(numel), 1), dtype=dtype, device=self.device)
+        make = torch.zeros if name in self.counters else torch.empty
+        self._buffers[name] = make(max(int(numel), 1), dtype=dtype, device=self.device)
 
     def fix(self) -> None:
         self.fixed = True

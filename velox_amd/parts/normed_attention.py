@@ -209,7 +209,7 @@ class NormedAttentionMixer(Mixer):
         sizes = getattr(ops, "attention_scratch_elems", None)
         if sizes is None:
             return {}
-        partial_out, partial_lse = sizes(self.num_heads, self.num_kv_heads, self.cached_dim, limits.max_num_tokens, limits.max_num_seqs, limits.max_model_len)
+        partial_out, partial_lse = sizes(self.num_heads, self.num_kv_heads, self.cached_dim, limits.max_num_tokens, limits.max_num_seqs, limits.max_model_len, plain=False)
         return {"attention_partial_out": partial_out, "attention_partial_lse": partial_lse}
 
     def forward(self, x, ctx, cache, owns_cache: bool = True):
