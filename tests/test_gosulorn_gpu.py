@@ -255,6 +255,23 @@ def test_short_convolution_with_its_last_inputs(ops, ref, dtype, taps):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("channels", [68, 70])  # in pieces of four (chunks of four tokens) and one by one (chunks of sixteen)
+@pytest.mark.parametrize("taps", [2, 4, 5, 6, 8])  # up to five the first chunk of four writes the last inputs, beyond a kernel of its own
+def test_last_inputs_of_portions_around_a_chunk(ops, dtype, channels, taps):
+    g, dt = torch.Generator().manual_seed(taps), DTYPES[dtype]
+    lengths = [1, 3, 4, 5, 0, 7, 8, 9, 2, 16, 17, 40]
+    cu = torch.tensor([0] + torch.tensor(lengths).cumsum(0).tolist(), dtype=torch.int32)
+    slots = torch.arange(len(lengths), dtype=torch.int32).flip(0)
+    x, w = rnd(g, sum(lengths), channels, dtype=dt), rnd(g, channels, taps)
+    tail = rnd(g, len(lengths), taps - 1, channels, dtype=dt)
+    want = tail.clone()
+    for i, n in enumerate(lengths):
+        want[slots[i]] = torch.cat([tail[slots[i]], x[cu[i]:cu[i] + n]])[n:]
+    ops.short_conv(x, channels, w, tail, slots.cuda(), cu.cuda(), max(lengths), activation="silu")
+    assert torch.equal(tail, want)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,padded,half", [(4, 2, 24, 40, 48, 4), (3, 1, 16, 16, 16, 8), (8, 4, 64, 128, 128, 8), (2, 2, 10, 6, 16, 5)])
 def test_partial_rotation_and_padded_cache_write(ops, ref, dtype, heads, kv_heads, dim, vdim, padded, half):
     g, dt, page = torch.Generator().manual_seed(dim), DTYPES[dtype], 16
