@@ -121,3 +121,36 @@ def test_without_a_gpu_the_engine_refuses_loudly(tmp_path, monkeypatch):
     monkeypatch.setattr(build.os.path, "isfile", lambda path: False if str(path).endswith("hipcc") else real_isfile(path))
     with pytest.raises(build.BuildError, match="hipcc not found"):
         build.find_hipcc()
+
+
+def rules_of_the_kernels(num_cus: int = 256):
+    """The rules by which calls take one kernel or another, without a GPU."""
+    from velox_amd.kernels.hip_ops import HipOps
+
+    ops = HipOps.__new__(HipOps)
+    ops.num_cus, ops.use_skinny_gemm, ops.fuse_residual_norm = num_cus, True, True
+    return ops
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,width,page,taken", [
+    (12, 2, 128, 1536, 16, True), (12, 2, 128, 1536, 4, True), (16, 1, 64, 1024, 4, True),
+    (12, 2, 128, 1536, 2, False), (12, 2, 128, 1536, 1, False),  # fewer than four keys a page
+    (32, 1, 64, 2048, 16, False), (20, 1, 128, 2560, 16, False), (40, 2, 64, 2560, 16, False),  # more heads per KV head than a tile has rows
+])
+def test_an_attention_is_left_in_parts_only_by_the_kernel_that_leaves_them(heads, kv_heads, dim, width, page, taken):
+    """Captured bounds and steps alike: what the streaming kernel does not take is merged by the attention itself."""
+    from velox_amd.kernels.hip_ops import PreparedWeight
+    from velox_amd.parts.attention import AttentionMixer
+    from velox_amd.parts.base import ResidualSink
+    from velox_amd.parts.norms import RMSNorm
+
+    ops = rules_of_the_kernels()
+    mixer = AttentionMixer("", width, heads, kv_heads, dim)
+    mixer.o_weight = torch.zeros((width, heads * dim), dtype=torch.bfloat16)
+    weight = mixer._prepared["o_weight"] = PreparedWeight(mixer.o_weight)
+    weight.copies[1] = torch.zeros(0)
+    norm = RMSNorm("", width, 1e-5)
+    norm.weight = torch.ones(width)
+    sink = ResidualSink(torch.zeros(1, width), norm)
+    assert (ops.attention_parts(1, heads, kv_heads, dim, weight, sink, 391, page) > 0) == taken
+    assert (ops.attention_parts_keys in mixer.capture_key_bounds_of_pages(ops, 1, 32768, page)) == taken

@@ -4,6 +4,7 @@ import torch
 
 from helpers import CONFIGS, PAGE_SIZE, Harness, make_folder, random_tokens
 from plain_qwen2 import qwen2_logits, read_model_folder
+from velox_amd.engine.batch import StepEntry
 
 pytestmark = pytest.mark.gpu
 
@@ -130,3 +131,33 @@ def test_workspace_addresses_never_change_once_the_runner_exists(tmp_path, ops):
     assert h.runner.workspace.addresses() == before
     with pytest.raises(RuntimeError, match="cannot be replaced"):
         h.runner.workspace.get("attention_partial_out", 1 << 30)
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,page", [(4, 2, 128, 16), (4, 2, 128, 2), (4, 2, 128, 1), (32, 1, 16, 16), (32, 1, 16, 2), (16, 1, 32, 4)])
+def test_a_few_decoded_tokens_at_every_page_size_and_number_of_heads(tmp_path, ops, heads, kv_heads, dim, page):
+    """One and two decoded tokens behind some hundred keys, eagerly and through captured steps: with pages of fewer than four tokens or more
+    than 16 heads per KV head the attention is another kernel's, which merges the splits of its keys itself."""
+    from velox_amd.weights import write_random_model
+
+    config = {**CONFIGS["A"], "hidden_size": 512, "num_attention_heads": heads, "num_key_value_heads": kv_heads, "head_dim": dim, "max_position_embeddings": 4096}
+    folder = write_random_model(config, str(tmp_path / "wide"), 5, dtype="bfloat16")
+    config, weights = read_model_folder(folder)
+    tokens = {rid: random_tokens(config["vocab_size"], n, seed=n) for rid, n in (("a", 203), ("b", 98))}
+    h = Harness(folder, ops, torch.bfloat16, "cuda", page, num_pages=4096 // page, max_num_seqs=2, enable_graphs=True)
+    h.runner.capture_decode_graphs()
+    h.feed([(rid, sequence[:-4], []) for rid, sequence in tokens.items()])
+    for live in (["a"], ["b", "a"], ["b"], ["a", "b"]):
+        entries = []
+        for rid in live:
+            seq, computed = h.live[rid]
+            assert h.cache.append(seq, computed, 1)
+            entries.append(StepEntry(seq, [tokens[rid][computed]], computed, [0]))
+        eager = h.runner._forward(h.runner.builder.build(entries, ops, torch.bfloat16, h.runner.workspace)).float().cpu()
+        replays = h.runner.num_graph_replays
+        captured = h.runner.step(entries).float().cpu()
+        assert h.runner.num_graph_replays == replays + 1
+        for row, rid in enumerate(live):
+            h.live[rid][1] += 1
+            want = qwen2_logits(config, weights, tokens[rid][:h.live[rid][1]])[-1]
+            torch.testing.assert_close(captured[row], want, **TOL[torch.bfloat16])
+            torch.testing.assert_close(eager[row], want, **TOL[torch.bfloat16])

@@ -14,7 +14,7 @@ graphs are captured per batch-size bucket 1, 2, 4, ... (reference
 rows that read and write the reserved null page, and the step's tensors live at fixed
 addresses that the host refreshes before each replay.  A capture fixes how its kernels are
 launched; a part whose kernels would be launched differently behind short contexts says so
-(``Part.capture_key_bounds``) and gets further captures of the same bucket, each for steps whose
+(``Part.capture_key_bounds_of_pages``) and gets further captures of the same bucket, each for steps whose
 sequences all stay within a bound on their length; a step replays the tightest capture that
 covers it.  The captured activations live in the pool of the framework's graph allocator
 (``torch.cuda.graph_pool_handle``), shared by all captures; the step's inputs and the parts'
@@ -161,7 +161,7 @@ class ModelRunner:
             capacity = self.builder.section_total(bucket, bucket, bucket, self.builder.width)
             self._graph_buffers[bucket] = torch.zeros(capacity, dtype=torch.int32, device=self.device)
             self._graphs[bucket] = self._capture(self._graph_context(bucket, longest), warmup_iters)
-            bounds = sorted({int(b) for part in parts for b in part.capture_key_bounds(self.ops, bucket, longest) if 0 < int(b) < longest})
+            bounds = sorted({int(b) for part in parts for b in part.capture_key_bounds_of_pages(self.ops, bucket, longest, self.cache.page_size) if 0 < int(b) < longest})
             if bounds:
                 self._bounded_graphs[bucket] = [(bound, self._capture(self._graph_context(bucket, bound), warmup_iters)) for bound in bounds]
         torch.cuda.synchronize()

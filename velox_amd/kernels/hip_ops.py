@@ -898,25 +898,26 @@ class HipOps:
     # take more splits than are worth reading in each of its workgroups.
     attention_parts_keys = 2048
 
-    def attention_parts(self, tokens: int, num_heads: int, num_kv_heads: int, head_dim: int, weight, sink: Optional[ResidualSink], max_kv_len: int) -> int:
+    def attention_parts(self, tokens: int, num_heads: int, num_kv_heads: int, head_dim: int, weight, sink: Optional[ResidualSink], max_kv_len: int, block_size: int = 16) -> int:
         """In how many splits of the keys the attention of ``tokens`` single tokens may leave its output (``paged_attention(parts=)``) for the
         product with ``weight`` that adds it to ``sink`` to merge; 0: it merges them itself.  What this saves is the merge's kernel (3.3 us, and
         about as long when the last workgroup merges), what it costs is that each of the product's workgroups reads all parts: 0.2 us at up
         to four of them and one piece, 1.2 beyond.  Measured on MI355X, attention and product of a token (us, one pass / splits and
         merge / parts): 12 heads over 2, 1,536 wide, 60 keys 8.6 / - / 8.8, 391 13.3 / 12.7 / 9.2, 1,000 20 / 12.8 / 10.6, 4,000 53 / 14.8 /
         15.1; 28 over 4, 3,584 wide, 391 keys 16.6 / 15.5 / 14.3."""
-        if sink is None or sink.norm.deferred_form() is None or not 64 < max_kv_len <= self.attention_parts_keys or not self.merges_attention_parts(tokens, num_heads, num_kv_heads, head_dim, weight):
+        if sink is None or sink.norm.deferred_form() is None or not 64 < max_kv_len <= self.attention_parts_keys or not self.merges_attention_parts(tokens, num_heads, num_kv_heads, head_dim, weight, block_size):
             return 0
         return 2 if max_kv_len <= 128 else 4 if max_kv_len <= 1024 else 8
 
-    def merges_attention_parts(self, tokens: int, num_heads: int, num_kv_heads: int, head_dim: int, weight) -> bool:
-        """Whether the product of so many rows with ``weight`` can merge an attention's splits, for some number of keys."""
+    def merges_attention_parts(self, tokens: int, num_heads: int, num_kv_heads: int, head_dim: int, weight, block_size: int = 16) -> bool:
+        """Whether the product of so many rows with ``weight`` can merge an attention's splits, for some number of keys, in a cache whose pages
+        hold ``block_size`` tokens: only the streaming kernel leaves its splits."""
         weight, prepared = _weight_of(weight)
         packed = prepared.copy(1) if prepared is not None else None
         n, k = weight.shape
         return (packed is not None and weight.dtype == torch.bfloat16 and k == num_heads * head_dim and head_dim % 8 == 0 and k % 64 == 0 and 512 <= n <= 16 * self.num_cus
-                and self.use_skinny_gemm and self.fuse_residual_norm and head_dim <= self.MAX_TILED_HEAD_DIM and tokens <= 4 and self._few_rows_pieces(tokens, k) <= 2
-                and not self.shares_keys(tokens, num_kv_heads))
+                and self.use_skinny_gemm and self.fuse_residual_norm and tokens <= 4 and self._few_rows_pieces(tokens, k) <= 2
+                and self.streams_decoded_tokens(num_heads, num_kv_heads, head_dim, 2, block_size) and not self.shares_keys(tokens, num_kv_heads))
 
     def _linear_into_residual(self, x, weight: torch.Tensor, sink: ResidualSink, waves: Optional[int] = None, row_tiles: Optional[int] = None,
                               packed: Optional[torch.Tensor] = None) -> Optional[DeferredNorm]:
@@ -2082,6 +2083,12 @@ class HipOps:
                 rows = max(rows, self._shared_items(count, num_kv_heads, max_model_len, 4))
         return rows * num_heads * head_dim, rows * num_heads
 
+    def streams_decoded_tokens(self, num_heads: int, num_kv_heads: int, head_dim: int, element_size: int, block_size: int) -> bool:
+        """Whether the attention of single tokens can be the streaming kernel's, which alone leaves its splits to another kernel and shares keys
+        out: the query heads of a KV head are rows of one 16-row tile, four of a lane's keys lie in one page, and a wave's registers hold what it
+        has under way of a head."""
+        return num_heads // num_kv_heads <= 16 and block_size >= 4 and head_dim <= self.MAX_TILED_HEAD_DIM and element_size * head_dim <= 512
+
     def shares_keys(self, num_seqs: int, num_kv_heads: int) -> bool:
         """Whether a decode step's keys are shared out over the workgroups by how many each sequence has (``uneven``), and not each
         sequence's in equally many splits.  Measured on MI355X (us, equal splits / shared out): 57 sequences of 65 to 1,500 keys, 28 heads over
@@ -2155,8 +2162,9 @@ class HipOps:
             raise KernelError(f"max_q_len={max_q_len} outside [1, {tokens}]")
         if not 0 <= decode_prefix <= num_seqs or num_seqs > tokens:
             raise KernelError(f"decode_prefix={decode_prefix} does not fit {num_seqs} sequences with {tokens} tokens")
-        if parts and (not all_decode or tokens != num_seqs or sinks is not None or gate is not None or splits is not None or workspace is None or head_dim > self.MAX_TILED_HEAD_DIM):
-            raise KernelError("paged_attention: only an all-decode step's plain attention with a workspace is left in parts")
+        if parts and (not all_decode or tokens != num_seqs or sinks is not None or gate is not None or splits is not None or workspace is None
+                      or not self.streams_decoded_tokens(num_heads, num_kv_heads, head_dim, qkv.element_size(), block_size)):
+            raise KernelError("paged_attention: only an all-decode step's plain attention with a workspace, of the streaming kernel, is left in parts")
         out = torch.empty((0 if parts else tokens, num_heads * head_dim), dtype=qkv.dtype, device=self.device)
         bias_len = 0
         if distance_bias is not None:
@@ -2185,7 +2193,8 @@ class HipOps:
             part_o = part_lse = arrivals = None
             share = 0
             if (uneven and splits is None and decode_only and workspace is not None and distance_bias is None and softcap is None and gate is None
-                    and not keep_first and block_size >= 4 and group <= 16 and qkv.element_size() * head_dim <= 512 and self.shares_keys(count, num_kv_heads)):
+                    and not keep_first and self.streams_decoded_tokens(num_heads, num_kv_heads, head_dim, qkv.element_size(), block_size)
+                    and self.shares_keys(count, num_kv_heads)):
                 share, splits = max(1, self.num_cus // num_kv_heads), 1
                 items = self._shared_items(count, num_kv_heads, int(max_kv_len), block_size)
                 if items > 65535:

@@ -105,9 +105,12 @@ class AttentionMixer(Mixer):
         if choose is None or max_model_len <= SHORT_CONTEXT_KEYS:
             return ()
         differs = choose(batch, self.num_kv_heads, 1, max_model_len, True) != choose(batch, self.num_kv_heads, 1, SHORT_CONTEXT_KEYS, True)
-        bounds = (SHORT_CONTEXT_KEYS,) if differs else ()
+        return (SHORT_CONTEXT_KEYS,) if differs else ()
+
+    def capture_key_bounds_of_pages(self, ops, batch: int, max_model_len: int, block_size: int):
+        bounds = tuple(self.capture_key_bounds(ops, batch, max_model_len))
         merges = getattr(ops, "merges_attention_parts", None)  # (a few tokens' output product merges the splits behind up to so many keys)
-        if merges is not None and merges(batch, self.num_heads, self.num_kv_heads, self.head_dim, self.operand("o_weight")):
+        if merges is not None and max_model_len > SHORT_CONTEXT_KEYS and merges(batch, self.num_heads, self.num_kv_heads, self.head_dim, self.operand("o_weight"), block_size):
             bounds += (ops.attention_parts_keys,)
         return bounds
 
@@ -136,7 +139,7 @@ class AttentionMixer(Mixer):
         )
         # a few decoded tokens: the output product may merge the splits of their keys
         announced = getattr(ops, "attention_parts", None) if ctx.all_decode and sink is not None else None
-        parts = announced(q.shape[0], self.num_heads, self.num_kv_heads, self.head_dim, self.operand("o_weight"), sink, meta.max_kv_len) if announced is not None else 0
+        parts = announced(q.shape[0], self.num_heads, self.num_kv_heads, self.head_dim, self.operand("o_weight"), sink, meta.max_kv_len, cache.block_size) if announced is not None else 0
         attn = ops.paged_attention(
             q, self.num_heads, self.num_kv_heads, self.head_dim,
             cache.tensors["k"], cache.tensors["v"], cache.block_size,

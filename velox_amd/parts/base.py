@@ -138,6 +138,11 @@ class Part:
         step).  Default: none."""
         return ()
 
+    def capture_key_bounds_of_pages(self, ops, batch: int, max_model_len: int, block_size: int):
+        """The same in a cache whose pages hold ``block_size`` tokens, which some kernels' launches depend on as well: what the
+        step function asks.  Default: ``capture_key_bounds``."""
+        return self.capture_key_bounds(ops, batch, max_model_len)
+
     def workspace_needs(self, ops, limits) -> Dict[str, int]:
         """Scratch this part may ask ``ctx.workspace`` for: buffer name -> the most float32 elements, for any step within
         ``limits`` (``max_num_tokens``, ``max_num_seqs``, ``max_model_len``).  The step function reserves these before it
