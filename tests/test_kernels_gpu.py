@@ -823,6 +823,23 @@ def test_decoded_tokens_whose_keys_are_shared_out(ops, ref, dtype, nh, nkv, d, p
     assert torch.equal(run(moved), got[order])
 
 
+@pytest.mark.parametrize("count", [65279, 65280, 65535])
+def test_more_decoded_tokens_than_a_grid_has_room_for_when_keys_are_shared_out(ops, count):
+    """Their keys are then split equally: 65,535 single tokens were always taken."""
+    from velox_amd.engine.batch import Workspace
+
+    d, page = 16, 16
+    k_cache, v_cache = rand((2, 1, page, d), torch.float32, 81), rand((2, 1, d, page), torch.float32, 82)
+    q = rand((count, d), torch.float32, 83)
+    kv = torch.arange(count, dtype=torch.int32).remainder(page).add(1).cuda()
+    tables = torch.ones((count, 1), dtype=torch.int32, device="cuda")
+    assert (ops._shared_items(count, 1, page, page) <= 65535) == (count <= 65279)
+    got = ops.paged_attention(q, 1, 1, d, k_cache, v_cache, page, tables, torch.arange(count + 1, dtype=torch.int32, device="cuda"), kv, 1, page, 0.25, None, True,
+                              Workspace(torch.device("cuda")), uneven=True)
+    scores = (0.25 * q @ k_cache[1, 0].T).masked_fill(torch.arange(page, device="cuda") >= kv[:, None], float("-inf"))
+    torch.testing.assert_close(got, scores.softmax(-1) @ v_cache[1, 0].T, rtol=1e-4, atol=1e-5)
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 16384, 64), (32, 16388, 448), (33, 20004, 256), (64, 16400, 192)])
 def test_a_head_of_some_rows_streams_its_packed_copy(ops, m, n, k):
     """Float32 results of 17 to 64 rows of a registered weight: products of bfloat16 numbers, exact in float32, and k additions."""

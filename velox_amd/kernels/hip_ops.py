@@ -2098,7 +2098,8 @@ class HipOps:
         return 16 * num_seqs * num_kv_heads >= self.num_cus
 
     def _shared_items(self, num_seqs: int, num_kv_heads: int, max_kv_len: int, block_size: int) -> int:
-        """The most workgroups per KV head among which such a step's keys are shared out (a split's page ids fit the kernel's 2,046)."""
+        """The most workgroups per KV head among which such a step's keys are shared out (a split's page ids fit the kernel's 2,046).  They lie
+        along the grid's second dimension: beyond 65,535 a step's keys are split equally."""
         most = -(-(-(-max_kv_len // 16)) // (2046 * block_size // 16))
         return num_seqs * most + max(1, self.num_cus // num_kv_heads)
 
@@ -2194,11 +2195,9 @@ class HipOps:
             share = 0
             if (uneven and splits is None and decode_only and workspace is not None and distance_bias is None and softcap is None and gate is None
                     and not keep_first and self.streams_decoded_tokens(num_heads, num_kv_heads, head_dim, qkv.element_size(), block_size)
-                    and self.shares_keys(count, num_kv_heads)):
+                    and self.shares_keys(count, num_kv_heads) and self._shared_items(count, num_kv_heads, int(max_kv_len), block_size) <= 65535):
                 share, splits = max(1, self.num_cus // num_kv_heads), 1
                 items = self._shared_items(count, num_kv_heads, int(max_kv_len), block_size)
-                if items > 65535:
-                    raise KernelError(f"{count} sequences exceed the launch grid")
                 part_o = workspace.get("attention_partial_out", items * num_heads * head_dim)
                 part_lse = workspace.get("attention_partial_lse", items * num_heads)
                 arrivals = workspace.get("attention_arrivals", count * num_kv_heads)
