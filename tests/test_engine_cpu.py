@@ -154,3 +154,8 @@ def test_an_attention_is_left_in_parts_only_by_the_kernel_that_leaves_them(heads
     sink = ResidualSink(torch.zeros(1, width), norm)
     assert (ops.attention_parts(1, heads, kv_heads, dim, weight, sink, 391, page) > 0) == taken
     assert (ops.attention_parts_keys in mixer.capture_key_bounds_of_pages(ops, 1, 32768, page)) == taken
+
+
+@pytest.mark.parametrize("sequences,kv_heads,shared", [(64, 4, True), (128, 8, True), (129, 8, False), (1024, 4, False), (1024, 1, False)])
+def test_keys_are_shared_out_only_among_sequences_that_are_soon_looked_through(sequences, kv_heads, shared):
+    assert rules_of_the_kernels().shares_keys(sequences, kv_heads) == shared

@@ -2092,10 +2092,11 @@ class HipOps:
     def shares_keys(self, num_seqs: int, num_kv_heads: int) -> bool:
         """Whether a decode step's keys are shared out over the workgroups by how many each sequence has (``uneven``), and not each
         sequence's in equally many splits.  Measured on MI355X (us, equal splits / shared out): 57 sequences of 65 to 1,500 keys, 28 heads over
-        4 24.2 / 19.1, 23 of 100 to 2,000 20.0 / 12.7, one of 30,000 beside 63 of 200 337 / 29, 64 of 4,096 91.7 / 88.5, 64 of 512 16.1 / 16.0;
-        a few sequences have nothing to share and are slowed down by the merge at the kernel's end: 12 heads over 2, one of 60 keys 5.1 /
-        5.4, of 4,096 10.9 / 12.2."""
-        return 16 * num_seqs * num_kv_heads >= self.num_cus
+        4 24.2 / 19.1, 23 of 100 to 2,000 20.0 / 12.7, one of 30,000 beside 63 of 200 337 / 29, 64 of 4,096 91.7 / 88.5, 64 of 512 16.1 / 16.0.
+        Every workgroup looks for its share among all sequences, which many of them make dear (as many sequences of 60 keys and of 50 to 2,000, over 4
+        KV heads: 64 6.5 / 6.9 and 29.3 / 22.5, 128 9.3 / 10.4 and 54.9 / 36.5, 256 15.9 / 22.1 and 75.5 / 63.7, 512 29.9 / 52.2 and
+        131 / 142, 1,024 56 / 135 and 222 / 271): up to 128."""
+        return num_seqs <= 128 and 16 * num_seqs * num_kv_heads >= self.num_cus
 
     def _shared_items(self, num_seqs: int, num_kv_heads: int, max_kv_len: int, block_size: int) -> int:
         """The most workgroups per KV head among which such a step's keys are shared out (a split's page ids fit the kernel's 2,046).  They lie
