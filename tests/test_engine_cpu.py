@@ -156,6 +156,7 @@ def test_an_attention_is_left_in_parts_only_by_the_kernel_that_leaves_them(heads
     assert (ops.attention_parts_keys in mixer.capture_key_bounds_of_pages(ops, 1, 32768, page)) == taken
 
 
-@pytest.mark.parametrize("sequences,kv_heads,shared", [(64, 4, True), (128, 8, True), (129, 8, False), (1024, 4, False), (1024, 1, False)])
-def test_keys_are_shared_out_only_among_sequences_that_are_soon_looked_through(sequences, kv_heads, shared):
+@pytest.mark.parametrize("sequences,kv_heads,shared", [(64, 4, True), (128, 8, True), (129, 8, False), (1024, 4, False), (1024, 1, False),
+                                                       (1, 16, False), (2, 8, False), (4, 4, False), (16, 1, False), (1, 32, True), (8, 4, True), (32, 1, True)])
+def test_keys_are_shared_out_among_enough_sequences_that_are_soon_looked_through(sequences, kv_heads, shared):
     assert rules_of_the_kernels().shares_keys(sequences, kv_heads) == shared

@@ -793,10 +793,10 @@ def test_decode_behind_more_pages_than_the_streaming_kernel_keeps_ids_of(ops, re
 @pytest.mark.parametrize("nh,nkv,d,page,lens,window", [
     (28, 4, 128, 16, [1500, 65, 130, 300, 1, 700, 16, 17], None),  # some in several parts, some in one
     (28, 4, 128, 16, [3000] + [20] * 70, None),  # more sequences than a wave has lanes, one far longer
-    (6, 2, 64, 4, [9000, 77, 8300, 5, 500, 31, 32, 33], None),  # more page ids than a part has room for
-    (4, 2, 16, 4, [900, 1, 1, 1, 250, 128, 129, 127], 200),  # a window bounds what a sequence's share is
+    (6, 2, 64, 4, [9000, 77, 8300, 5, 500, 31, 32, 33] * 2, None),  # more page ids than a part has room for
+    (4, 2, 16, 4, [900, 1, 1, 1, 250, 128, 129, 127] * 2, 200),  # a window bounds what a sequence's share is
     (32, 8, 64, 64, [640] * 9, None),  # all alike
-    (3, 1, 256, 8, [2000 - 120 * b for b in range(16)], None),
+    (3, 1, 256, 8, [2000 - 60 * b for b in range(32)], None),
 ])
 def test_decoded_tokens_whose_keys_are_shared_out(ops, ref, dtype, nh, nkv, d, page, lens, window):
     """Single tokens behind unequal contexts, their keys shared out over the workgroups by how many each sequence has: the

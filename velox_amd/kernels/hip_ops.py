@@ -2095,8 +2095,11 @@ class HipOps:
         4 24.2 / 19.1, 23 of 100 to 2,000 20.0 / 12.7, one of 30,000 beside 63 of 200 337 / 29, 64 of 4,096 91.7 / 88.5, 64 of 512 16.1 / 16.0.
         Every workgroup looks for its share among all sequences, which many of them make dear (as many sequences of 60 keys and of 50 to 2,000, over 4
         KV heads: 64 6.5 / 6.9 and 29.3 / 22.5, 128 9.3 / 10.4 and 54.9 / 36.5, 256 15.9 / 22.1 and 75.5 / 63.7, 512 29.9 / 52.2 and
-        131 / 142, 1,024 56 / 135 and 222 / 271): up to 128."""
-        return num_seqs <= 128 and 16 * num_seqs * num_kv_heads >= self.num_cus
+        131 / 142, 1,024 56 / 135 and 222 / 271): up to 128.  A few sequences have nothing to share, as many splits as fill the compute units either
+        way, and wait for the merge at the kernel's end (1,000 keys, 4,000 and 50 to 4,000 among them: one over 16 KV heads 10.8 / 10.2 and 13.8 / 14.6, two over
+        8 10.4 / 10.3, 13.7 / 14.9 and 11.9 / 14.9, four over 4 10.5 / 10.6, 13.8 / 15.3 and 11.8 / 14.0; one over 32 11.3 / 10.9 and 18.9 / 17.8, four
+        over 8 11.1 / 11.0, 19.0 / 17.9 and 14.4 / 13.6, eight over 4 11.0 / 11.2, 18.9 / 18.3 and 14.2 / 14.5)."""
+        return num_seqs <= 128 and 8 * num_seqs * num_kv_heads >= self.num_cus
 
     def _shared_items(self, num_seqs: int, num_kv_heads: int, max_kv_len: int, block_size: int) -> int:
         """The most workgroups per KV head among which such a step's keys are shared out (a split's page ids fit the kernel's 2,046).  They lie
