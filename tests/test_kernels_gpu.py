@@ -1505,6 +1505,16 @@ def test_grouped_products_in_tiles_of_192_and_256_columns(ops, monkeypatch, hidd
     assert torch.equal(experts_against_float64(ops, rows, hidden, inter, 1, scale_input, unit), first)
 
 
+@pytest.mark.parametrize("rows", [(0, 700, 0, 0, 1, 0), (0, 0, 0, 0, 0, 129), (400, 1, 193, 0, 2, 64), (1, 1, 1, 1, 1, 60)])
+@pytest.mark.parametrize("hidden, inter, scale_input, unit", [(64, 2432, False, "glu"), (192, 128, True, "glu"), (4864, 64, True, "relu2")])
+def test_grouped_products_of_experts_that_get_very_unlike_numbers_of_rows(ops, monkeypatch, rows, hidden, inter, scale_input, unit):
+    """The width of the tiles is chosen by the rows that the experts were given, not by those that they could expect."""
+    monkeypatch.setattr(ops._core, "velox_routed_tile_rows", lambda *sizes: 128)
+    first = experts_against_float64(ops, rows, hidden, inter, 1, scale_input, unit)
+    monkeypatch.setattr(ops._core, "velox_routed_tile_rows", lambda *sizes: 192)
+    assert torch.equal(experts_against_float64(ops, rows, hidden, inter, 1, scale_input, unit), first)
+
+
 def experts_against_float64(ops, rows, hidden, inter, top, scale_input, unit):
     """Against float64.  Two roundings to bfloat16 (8 bits), each off by at most 2^-8 of its value: the units' middles, which the second
     product adds up (at most 2^-8 sum |W_down| |middle|), and the result.  Float32 sums of a few hundred terms add less than

@@ -342,20 +342,9 @@ static inline float plan_tiles_expected(int pairs, int experts, int tile_rows) {
   return experts * tiles;
 }
 
-// Columns of a tile, in 64: the fewest whose tiles take no more rounds over the compute units than those of 256 do.  A tile's order of additions is the
-// same at any width; a step of a narrower one is shorter, and where 256 columns leave compute units without a tile, W comes through more of
-// them (each gets some 40 GB/s of it).  Measured on MI355X, us of the two products with 256 columns / with these: 2,072 pairs over 16 experts of 2,048
-// -> 1,408 88.5 / 78.6, 4,000 pairs 119.9 / 110.1, 600 76.4 / 67.8; 32 experts of 4,096 -> 1,408, 1,340 pairs 251.7 / 233.7, 4,000
-// 322.5 / 297.6, 10,000 (more rounds in both: 256 columns stay) 457.6.
-static inline int plan_tile_cols(float row_tiles, int w_rows) {
-  auto rounds = [&](int ct) { return ceilf(row_tiles * ((w_rows + 64 * ct - 1) / (64 * ct)) / TL_WORKGROUPS); };
-  int ct = 4;
-  while (ct > 2 && rounds(ct - 1) <= rounds(4)) --ct;
-  return ct;
-}
-
 // The rows of a tile of the plan's products: 64 up to 64 pairs, above 128 or 192 (tiles_mfma.h's kernel), whichever is likely to cost less with as many
-// tiles as are expected, as wide as they are then taken (us of the two products in tiles of 128 and 192 rows: 16 experts of 2,048 -> 1,408, 600
+// tiles as are expected, as wide as they are then taken.  (Where a router sends all tokens to as few experts as it can the other one may be the
+// quicker: 8,192 pairs on 8 of 64 experts 118 and 129 us.)  (us of the two products in tiles of 128 and 192 rows: 16 experts of 2,048 -> 1,408, 600
 // pairs 70.2 and 75.6, 2,072 96 and 82, 3,000 99 and 112, 4,000 117 and 113, 6,000 153 and 139; 32 of 4,096 -> 1,408, 1,340 pairs 230 and 242, 4,000 316 and
 // 288, 10,000 517 and 466).  k % 64 != 0 is built for 128.  Experts with 2 GiB or more from a gate row to its up row, which the large tiles' loads do not
 // reach, stay with 64 rows at any number of pairs.  (Tiles of 64 rows were no quicker at any number of pairs above 64: 12 rows per expert
@@ -367,7 +356,7 @@ static inline int grouped_tile_rows(int pairs, int experts, int inter, int hidde
   for (int rt = 2; rt <= 3; ++rt) {
     const float tiles = plan_tiles_expected(pairs, experts, 64 * rt);
     auto product = [&](int w_rows, int k) {
-      const int ct = plan_tile_cols(tiles, w_rows), least = ct < rt ? ct : rt, most = ct < rt ? rt : ct;  // (3 x 2 costs what 2 x 3 does)
+      const int ct = plan_tile_cols((int)(tiles + 0.5f), w_rows), least = ct < rt ? ct : rt, most = ct < rt ? rt : ct;  // (3 x 2 costs what 2 x 3 does)
       const TileCost* t = TILE_COSTS;
       while (t->rt != least || t->ct != most) ++t;
       return tiles_cost_of(*t, tiles * ((w_rows + 64 * ct - 1) / (64 * ct)), k, 1);
@@ -378,16 +367,11 @@ static inline int grouped_tile_rows(int pairs, int experts, int inter, int hidde
 }
 
 template <int EPI, typename TO>
-static void grouped_tiles_launch(const TileArgs& tiles, int tile_rows, int ct, int workgroups, hipStream_t stream) {
-#define TILES(RT, CT, S, GATHER, TAIL) tiles_kernel<RT, CT, S, EPI, TO, true, GATHER, TAIL><<<workgroups, 256, 0, stream>>>(tiles)
-#define SHAPES(GATHER)                                       \
-  if (tiles.k % 64 != 0) TILES(2, 4, 3, GATHER, true);       \
-  else if (tile_rows == 192 && ct == 4) TILES(3, 4, 2, GATHER, false); \
-  else if (tile_rows == 192 && ct == 3) TILES(3, 3, 3, GATHER, false); \
-  else if (tile_rows == 192) TILES(3, 2, 3, GATHER, false);  \
-  else if (ct == 4) TILES(2, 4, 3, GATHER, false);           \
-  else if (ct == 3) TILES(2, 3, 3, GATHER, false);           \
-  else TILES(2, 2, 3, GATHER, false);
+static void grouped_tiles_launch(const TileArgs& tiles, int tile_rows, int workgroups, hipStream_t stream) {
+#define SHAPES(GATHER)                                                                                                                 \
+  if (tiles.k % 64 != 0) tiles_kernel<2, 4, 3, EPI, TO, true, GATHER, true><<<workgroups, 256, 0, stream>>>(tiles);                  \
+  else if (tile_rows == 192) plan_tiles_kernel<3, EPI, TO, GATHER><<<workgroups, 256, 0, stream>>>(tiles);                           \
+  else plan_tiles_kernel<2, EPI, TO, GATHER><<<workgroups, 256, 0, stream>>>(tiles);
   if constexpr (EPI != TL_PLAIN) {
     if (tiles.gather_top > 0) {
       SHAPES(true)
@@ -396,7 +380,6 @@ static void grouped_tiles_launch(const TileArgs& tiles, int tile_rows, int ct, i
   }
   SHAPES(false)
 #undef SHAPES
-#undef TILES
 }
 
 template <int EPI, typename TO>
@@ -425,14 +408,13 @@ static int grouped_plan_launch(const GroupedArgs& args, int tile_rows, int most_
   tiles.act = args.act;
   tiles.unit = args.unit;
   if (!tiles_fit(args.gather_top > 0 ? args.plan_pairs / args.gather_top : 256, args.a_ld, EPI == GM_GLU ? args.n + 256LL : 256, args.k)) return -1;
-  const int w_rows = (EPI == GM_GLU ? 2 : 1) * args.n, ct = tiles.k % 64 != 0 ? 4 : plan_tile_cols(plan_tiles_expected(args.plan_pairs, args.plan_groups, tile_rows), w_rows);
-  const long long most = (long long)most_tiles * ((w_rows + 64 * ct - 1) / (64 * ct));
+  const long long most = (long long)most_tiles * (((EPI == GM_GLU ? 2LL : 1LL) * args.n + 127) / 128);  // (of the narrowest)
   const int workgroups = (int)(most < TL_WORKGROUPS ? (most + TL_XCDS - 1) / TL_XCDS * TL_XCDS : TL_WORKGROUPS);
   if constexpr (EPI == GM_GLU) {
-    if (args.unit.alpha == 1.f && args.unit.limit == INFINITY && args.unit.shift == 0.f) grouped_tiles_launch<TL_SILU_UNIT, TO>(tiles, tile_rows, ct, workgroups, stream);
-    else grouped_tiles_launch<TL_UNIT, TO>(tiles, tile_rows, ct, workgroups, stream);
+    if (args.unit.alpha == 1.f && args.unit.limit == INFINITY && args.unit.shift == 0.f) grouped_tiles_launch<TL_SILU_UNIT, TO>(tiles, tile_rows, workgroups, stream);
+    else grouped_tiles_launch<TL_UNIT, TO>(tiles, tile_rows, workgroups, stream);
   } else {
-    grouped_tiles_launch<EPI == GM_ACT ? TL_ACT : TL_PLAIN, TO>(tiles, tile_rows, ct, workgroups, stream);
+    grouped_tiles_launch<EPI == GM_ACT ? TL_ACT : TL_PLAIN, TO>(tiles, tile_rows, workgroups, stream);
   }
   return (int)hipGetLastError();
 }

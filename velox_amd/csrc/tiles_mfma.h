@@ -121,16 +121,14 @@ __device__ __forceinline__ float tl_middle(float gate, float up, const TileArgs&
 
 // RT, CT: tiles of 32 rows and 32 columns per wave; S: buffers.  GATHER: rows through the plan's order.  TAIL: k % 64 != 0.
 template <int RT, int CT, int S, int EPI, typename TO, bool PLAN, bool GATHER, bool TAIL>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) tiles_kernel(const TileArgs args) {
+__device__ __forceinline__ void tiles_work(const TileArgs& args, char* smem) {
   static_assert(PLAN || !GATHER, "only a plan has an order");
   constexpr int WAVES = 4, TM = 64 * RT, TN = 64 * CT, STAGE = (TM + TN) * 128;
-  static_assert(S * STAGE <= 160 * 1024, "LDS of a compute unit");
   constexpr int RH0 = (RT + 1) / 2, RH1 = RT - RH0, CH0 = (CT + 1) / 2, CH1 = CT - CH0;  // halves of a wave's tiles
   constexpr int LA0 = 2 * RH0, LC0 = 2 * CH0, LC1 = 2 * CH1, LA1 = 2 * RH1, LOADS = LA0 + LC0 + LC1 + LA1;  // loads of a wave in a step, in this order
   constexpr bool GLU = EPI == TL_SILU || EPI == TL_RELU || EPI == TL_SILU_UNIT || EPI == TL_UNIT;
   constexpr int OUT_COLS = GLU ? TN / 2 : TN;  // output columns of the tile
   constexpr int BLOCK_ROWS = 1024 / TM;        // row tiles of a block
-  __shared__ __attribute__((aligned(1024))) char smem[S * STAGE];
 
   const int n = args.n, k = args.k;
   const int cols = (n + OUT_COLS - 1) / OUT_COLS;
@@ -174,11 +172,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
       const int* tile_row = tile_group + args.plan_max_tiles;
       // (a group's tiles follow one another, so at / cols lies among the tiles of the right one)
       const int near = at / cols;
-      group = tile_group[near];
-      begin = starts[group];
-      end = starts[group + 1];
+      group = __builtin_amdgcn_readfirstlane(tile_group[near]);
+      begin = __builtin_amdgcn_readfirstlane(starts[group]);
+      end = __builtin_amdgcn_readfirstlane(starts[group + 1]);
       tiles = (end - begin + TM - 1) / TM;
-      at -= (near - (tile_row[near] - begin) / TM) * cols;
+      at -= (near - (__builtin_amdgcn_readfirstlane(tile_row[near]) - begin) / TM) * cols;
     } else {
       t.split = at / (row_tiles * cols);
       at -= t.split * row_tiles * cols;
@@ -433,6 +431,43 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #undef TL_QUADRANT
 #undef TL_COLS
 #undef TL_ROWS
+}
+
+constexpr int tiles_lds(int rt, int ct, int s) { return s * (rt + ct) * 64 * 128; }
+
+template <int RT, int CT, int S, int EPI, typename TO, bool PLAN, bool GATHER, bool TAIL>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) tiles_kernel(const TileArgs args) {
+  static_assert(tiles_lds(RT, CT, S) <= 160 * 1024, "LDS of a compute unit");
+  __shared__ __attribute__((aligned(1024))) char smem[tiles_lds(RT, CT, S)];
+  tiles_work<RT, CT, S, EPI, TO, PLAN, GATHER, TAIL>(args, smem);
+}
+
+// Columns of a plan's tiles, in 64: the fewest whose tiles take no more rounds over the compute units than those of 256 do.  A tile's order of
+// additions is the same at any width; a step of a narrower one is shorter, and where 256 columns leave compute units without a tile, W
+// comes through more of them (each gets some 40 GB/s of it).
+__host__ __device__ inline int plan_tile_cols(int row_tiles, int w_rows) {
+  auto rounds = [&](int ct) { return (row_tiles * ((w_rows + 64 * ct - 1) / (64 * ct)) + TL_WORKGROUPS - 1) / TL_WORKGROUPS; };
+  int ct = 4;
+  while (ct > 2 && rounds(ct - 1) <= rounds(4)) --ct;
+  return ct;
+}
+
+// The plan's products in tiles as wide as its number of row tiles asks for, which only the device knows: the host can expect it, but a tile more
+// than makes whole rounds is a round more, and routers do not spread tokens evenly.  Measured on MI355X, us of a layer's routed experts with
+// 256 columns / with the widths that evenly spread rows would ask for / like this: 2,072 pairs over 16 experts of 2,048 -> 1,408, evenly
+// spread 96.9 / 89.1 / 89.8, by Zipf's law 97.8 / 125.7 / 95.4, all on two 78.1 / 64.7 / 67.8; 600 pairs, a quarter of the experts with nearly all
+// 86.0 / 100.7 / 82.1; 32 of 4,096 -> 1,408, 1,340 pairs 253 / 235 / 235, by the law's square 263 / 278 / 262, 10,000 pairs 439 / 429 /
+// 435; 64 of 2,048 -> 768, 8,192 pairs over experts that differ by a factor of four 216 / 234 / 207.
+template <int RT, int EPI, typename TO, bool GATHER>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) plan_tiles_kernel(const TileArgs args) {
+  constexpr int S4 = RT == 3 ? 2 : 3;
+  constexpr int LDS = tiles_lds(RT, 4, S4) > tiles_lds(RT, 3, 3) ? tiles_lds(RT, 4, S4) : tiles_lds(RT, 3, 3);
+  static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
+  __shared__ __attribute__((aligned(1024))) char smem[LDS];
+  const int ct = plan_tile_cols(args.plan[0], (EPI == TL_UNIT || EPI == TL_SILU_UNIT ? 2 : 1) * args.n);  // (uniform over the grid)
+  if (ct == 4) tiles_work<RT, 4, S4, EPI, TO, true, GATHER, false>(args, smem);
+  else if (ct == 3) tiles_work<RT, 3, 3, EPI, TO, true, GATHER, false>(args, smem);
+  else tiles_work<RT, 2, 3, EPI, TO, true, GATHER, false>(args, smem);
 }
 
 // Whether a tile's operands lie within the reach of its resources.
