@@ -179,9 +179,10 @@ __global__ void __launch_bounds__(256) grouped_mfma_kernel(const GroupedArgs arg
 // their up columns) of one tile; its four waves split K into quarters, each wave asks for four steps' operands at once, W's a
 // round ahead, and the waves' sums are added through LDS in the order of the waves (no atomics: the same result on every
 // run).  A tile works as many 16-row tiles as it has rows, whatever the step's number of pairs would allow.  With `row_scale` the
-// rows are scaled in registers, behind the wait for them and before that for W: the same bits as a scaled copy.  Measured on MI355X: 64
-// pairs over 32 experts of 4,096 -> 1,408 -> 4,096 193 us both products, 180 with W in whole lines past the caches (W: 650 + 325 MB), in a step 121 +
-// 66 and 107 + 67; 24 pairs over 16 experts of 2,048 -> 1,408 -> 2,048 61.6 and 56.5.
+// rows are scaled in registers, behind the wait for them and before that for W: the same bits as a scaled copy.  Measured on MI355X, us of a
+// layer's routed experts with W in pieces of 64 bytes through the caches / in lines past them / with every wave's quarter of K beginning on a
+// line (1,408 indices: 384, 384, 384 and 256 instead of four times 352, which begins two of them in the middle of a line): 64 pairs over 32 experts of
+// 4,096 -> 1,408 -> 4,096 (W: 650 + 325 MB) 202 / 190 / 181, 24 pairs over 16 of 2,048 -> 1,408 -> 2,048 61.0 / 56.5 / 53.9.
 template <int EPI, typename TO, int MT, bool LINES>
 __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int group, const int row0, const int rows, const int* order,
                                               float4_t (*partial)[8][64]) {
@@ -202,7 +203,7 @@ __device__ __forceinline__ void few_rows_tile(const GroupedArgs& args, const int
       const int col = min(col0[t] + (LINES ? 8 * half + (i & 7) : i), n - 1);
       w_row[t][half] = w_base + (size_t)(EPI == GM_GLU && t == 1 ? n + col : col) * k + piece;
     }
-  const int quarter = ((k + 127) / 128) * 32;  // indices per wave: a multiple of 32
+  const int quarter = LINES ? (k + 255) / 256 * 64 : (k + 127) / 128 * 32;  // indices per wave: whole steps, with LINES whole lines of W
   const int k_begin = wave * quarter, k_end = min(k, k_begin + quarter);
   // W is what there is to read: its next step is asked for before the current one is multiplied, and its first before the rows of
   // `a` have been looked up
