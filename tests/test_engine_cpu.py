@@ -132,6 +132,22 @@ def rules_of_the_kernels(num_cus: int = 256):
     return ops
 
 
+def an_output_product(heads, kv_heads, dim, width):
+    """A mixer whose output weight is prepared, the handle of that weight, and a sink for its product."""
+    from velox_amd.kernels.hip_ops import PreparedWeight
+    from velox_amd.parts.attention import AttentionMixer
+    from velox_amd.parts.base import ResidualSink
+    from velox_amd.parts.norms import RMSNorm
+
+    mixer = AttentionMixer("", width, heads, kv_heads, dim)
+    mixer.o_weight = torch.zeros((width, heads * dim), dtype=torch.bfloat16)
+    weight = mixer._prepared["o_weight"] = PreparedWeight(mixer.o_weight)
+    weight.copies[1] = torch.zeros(0)
+    norm = RMSNorm("", width, 1e-5)
+    norm.weight = torch.ones(width)
+    return mixer, weight, ResidualSink(torch.zeros(1, width), norm)
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,width,page,taken", [
     (12, 2, 128, 1536, 16, True), (12, 2, 128, 1536, 4, True), (16, 1, 64, 1024, 4, True),
     (12, 2, 128, 1536, 2, False), (12, 2, 128, 1536, 1, False),  # fewer than four keys a page
@@ -139,19 +155,8 @@ def rules_of_the_kernels(num_cus: int = 256):
 ])
 def test_an_attention_is_left_in_parts_only_by_the_kernel_that_leaves_them(heads, kv_heads, dim, width, page, taken):
     """Captured bounds and steps alike: what the streaming kernel does not take is merged by the attention itself."""
-    from velox_amd.kernels.hip_ops import PreparedWeight
-    from velox_amd.parts.attention import AttentionMixer
-    from velox_amd.parts.base import ResidualSink
-    from velox_amd.parts.norms import RMSNorm
-
     ops = rules_of_the_kernels()
-    mixer = AttentionMixer("", width, heads, kv_heads, dim)
-    mixer.o_weight = torch.zeros((width, heads * dim), dtype=torch.bfloat16)
-    weight = mixer._prepared["o_weight"] = PreparedWeight(mixer.o_weight)
-    weight.copies[1] = torch.zeros(0)
-    norm = RMSNorm("", width, 1e-5)
-    norm.weight = torch.ones(width)
-    sink = ResidualSink(torch.zeros(1, width), norm)
+    mixer, weight, sink = an_output_product(heads, kv_heads, dim, width)
     assert (ops.attention_parts(1, heads, kv_heads, dim, weight, sink, 391, page) > 0) == taken
     assert (ops.attention_parts_keys in mixer.capture_key_bounds_of_pages(ops, 1, 32768, page)) == taken
 
@@ -160,3 +165,15 @@ def test_an_attention_is_left_in_parts_only_by_the_kernel_that_leaves_them(heads
                                                        (1, 16, False), (2, 8, False), (4, 4, False), (16, 1, False), (1, 32, True), (8, 4, True), (32, 1, True)])
 def test_keys_are_shared_out_among_enough_sequences_that_are_soon_looked_through(sequences, kv_heads, shared):
     assert rules_of_the_kernels().shares_keys(sequences, kv_heads) == shared
+
+
+@pytest.mark.parametrize("tokens,heads,kv_heads,width,parts", [
+    (1, 12, 2, 1536, (0, 2, 4, 4, 8, 0)), (1, 16, 4, 3584, (0, 2, 4, 4, 8, 0)),  # a piece of activations a lane
+    (2, 12, 2, 1536, (0, 2, 4, 4, 8, 0)), (1, 24, 4, 2048, (0, 2, 4, 4, 8, 0)),  # two
+    (1, 28, 4, 3584, (0,) * 6), (1, 20, 4, 2560, (0,) * 6),  # two in more workgroups than there are compute units
+    (4, 12, 2, 1536, (0,) * 6), (5, 12, 2, 1536, (0,) * 6),
+])
+def test_in_how_many_parts_an_attention_is_left(tokens, heads, kv_heads, width, parts):
+    _, weight, sink = an_output_product(heads, kv_heads, 128, width)
+    ops = rules_of_the_kernels()
+    assert tuple(ops.attention_parts(tokens, heads, kv_heads, 128, weight, sink, keys) for keys in (64, 128, 384, 385, 1025, 2049)) == parts

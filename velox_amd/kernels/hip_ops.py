@@ -903,8 +903,12 @@ class HipOps:
         product with ``weight`` that adds it to ``sink`` to merge; 0: it merges them itself.  What this saves is the merge's kernel (3.3 us, and
         about as long when the last workgroup merges), what it costs is that each of the product's workgroups reads all parts: 0.2 us at up
         to four of them and one piece, 1.2 beyond.  Measured on MI355X, attention and product of a token (us, one pass / splits and
-        merge / parts): 12 heads over 2, 1,536 wide, 60 keys 8.6 / - / 8.8, 391 13.3 / 12.7 / 9.2, 1,000 20 / 12.8 / 10.6, 4,000 53 / 14.8 /
-        15.1; 28 over 4, 3,584 wide, 391 keys 16.6 / 15.5 / 14.3."""
+        merge / parts): 12 heads over 2, 1,536 wide, 60 keys 8.6 / - / 8.8, 391 13.3 / 12.7 / 9.2, 1,000 20 / 12.8 / 10.6, 4,000 53 / 14.8 / 15.1.
+        Captured steps have their bound's splits: with those of 384 keys, one pass / 4 parts, and of 2,048, splits of the longest context and
+        merge / 8 parts, 60, 384, 400, 1,000 and 2,000 keys 8.8 / 8.3, 12.5 / 10.0, 12.3 / 10.9, 12.8 / 11.3, 13.4 / 12.8.
+        Two pieces: two rows of that model 8.9 / 9.6, 12.5 / 11.3, 12.4 / 11.3, 13.0 / 12.1, 14.0 / 13.9, but not where the product has more workgroups
+        than there are compute units (28 heads over 4, 3,584 wide, a token 11.8 / 13.2, 15.2 / 15.1, 15.9 / 15.7, 16.0 / 16.8, 17.0 / 18.0; in
+        one piece, 16 heads over 4, 10.7 / 10.3, 14.2 / 12.1, 14.1 / 12.9, 14.8 / 13.7, 15.9 / 15.3)."""
         if sink is None or sink.norm.deferred_form() is None or not 64 < max_kv_len <= self.attention_parts_keys or not self.merges_attention_parts(tokens, num_heads, num_kv_heads, head_dim, weight, block_size):
             return 0
         return 2 if max_kv_len <= 128 else 4 if max_kv_len <= 1024 else 8
@@ -915,8 +919,9 @@ class HipOps:
         weight, prepared = _weight_of(weight)
         packed = prepared.copy(1) if prepared is not None else None
         n, k = weight.shape
+        pieces = self._few_rows_pieces(tokens, k)
         return (packed is not None and weight.dtype == torch.bfloat16 and k == num_heads * head_dim and head_dim % 8 == 0 and k % 64 == 0 and 512 <= n <= 16 * self.num_cus
-                and self.use_skinny_gemm and self.fuse_residual_norm and tokens <= 4 and self._few_rows_pieces(tokens, k) <= 2
+                and self.use_skinny_gemm and self.fuse_residual_norm and tokens <= 4 and (pieces == 1 or (pieces == 2 and n <= 8 * self.num_cus))
                 and self.streams_decoded_tokens(num_heads, num_kv_heads, head_dim, 2, block_size) and not self.shares_keys(tokens, num_kv_heads))
 
     def _linear_into_residual(self, x, weight: torch.Tensor, sink: ResidualSink, waves: Optional[int] = None, row_tiles: Optional[int] = None,
