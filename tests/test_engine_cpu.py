@@ -177,3 +177,10 @@ def test_in_how_many_parts_an_attention_is_left(tokens, heads, kv_heads, width, 
     _, weight, sink = an_output_product(heads, kv_heads, 128, width)
     ops = rules_of_the_kernels()
     assert tuple(ops.attention_parts(tokens, heads, kv_heads, 128, weight, sink, keys) for keys in (64, 128, 384, 385, 1025, 2049)) == parts
+
+
+@pytest.mark.parametrize("page,keys,rows", [(16, 1 << 20, 3364), (4, 1 << 20, 12964), (2, 1 << 20, 12964), (64, 1 << 20, 1600), (16, 1 << 17, 1600)])
+def test_scratch_for_shares_of_keys_is_that_of_the_caches_pages(page, keys, rows):
+    """100 single tokens of 28 heads over 4: workgroups per KV head that share out the step's keys, as many as hold the page ids of so many keys, or
+    what the splits of portions take."""
+    assert rules_of_the_kernels().attention_scratch_elems(28, 4, 128, 100, 100, keys, block_size=page) == (rows * 28 * 128, rows * 28)

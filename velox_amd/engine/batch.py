@@ -88,6 +88,7 @@ class StepLimits:
     max_num_tokens: int
     max_num_seqs: int
     max_model_len: int
+    block_size: int = 1  # tokens of a cache page (the fewest there can be where it is not said)
 
 
 @dataclass

@@ -75,7 +75,7 @@ class ModelRunner:
         self.last_prepare_ms = 0.0  # host time of the last step's batch layout (block tables, positions, ids)
         # every part's scratch at its largest, before anything runs: captured steps hold these addresses
         self.workspace = Workspace(self.device)
-        limits = StepLimits(self.max_num_tokens, self.max_num_seqs, cache.max_model_len)
+        limits = StepLimits(self.max_num_tokens, self.max_num_seqs, cache.max_model_len, cache.page_size)
         for part in model.all_parts():
             for name, numel in part.workspace_needs(ops, limits).items():
                 self.workspace.reserve(name, numel)

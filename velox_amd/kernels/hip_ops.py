@@ -2064,13 +2064,15 @@ class HipOps:
         return max(1, min(-(-self.num_cus // blocks), max_kv_len // 1024, 16))
 
     def attention_scratch_elems(self, num_heads: int, num_kv_heads: int, head_dim: int, max_num_tokens: int, max_num_seqs: int, max_model_len: int,
-                               plain: bool = True) -> Tuple[int, int]:
+                               plain: bool = True, block_size: int = 1) -> Tuple[int, int]:
         """The most float32 elements ``paged_attention`` asks its workspace for (partial outputs, partial log-sums) in
         any step of at most ``max_num_tokens`` tokens and ``max_num_seqs`` sequences behind at most ``max_model_len`` keys,
         with the splits that ``choose_splits`` and ``choose_portion_splits`` pick.  The bound counts TOKENS, not sequences:
         the sequence on the null page that pads a step up to a timed number of rows (one more than ``max_num_seqs``) brings
         tokens within ``max_num_tokens`` like any other and is covered.  ``plain``: the caller may share keys out (``uneven``) or leave
-        its splits to the next product (``parts``)."""
+        its splits to the next product (``parts``), where the streaming kernel works them; ``block_size``: tokens of a page, or the fewest that
+        it may have (the fewer, the more shares hold a sequence's page ids: 100 sequences of a million keys over 4 KV heads 12,964 rows with pages
+        of 4, 3,364 with 16)."""
         if head_dim > self.MAX_TILED_HEAD_DIM:
             return 0, 0  # (the plain kernel splits nothing)
         group = num_heads // num_kv_heads
@@ -2080,12 +2082,14 @@ class HipOps:
         for portion in range(1, max_num_tokens + 1):  # portions of prompts, behind up to max_num_seqs - 1 single tokens
             whole = min(max_num_tokens, portion + max_num_seqs - 1)
             rows = max(rows, whole * self.choose_portion_splits(portion, group, num_kv_heads, max_model_len))
-        if not plain:
+        block_size = max(block_size, 4)  # (a kernel that takes pages of fewer asks for no more than the above)
+        if not plain or not self.streams_decoded_tokens(num_heads, num_kv_heads, head_dim, 2, block_size):
             return rows * num_heads * head_dim, rows * num_heads
         rows = max(rows, 8 * min(4, max_num_seqs))  # a few single tokens whose output product merges up to eight splits
         for count in range(1, max_num_seqs + 1):  # single tokens whose keys are shared out by their number
-            if self.shares_keys(count, num_kv_heads):
-                rows = max(rows, self._shared_items(count, num_kv_heads, max_model_len, 4))
+            items = self._shared_items(count, num_kv_heads, max_model_len, block_size)
+            if self.shares_keys(count, num_kv_heads) and items <= 65535:
+                rows = max(rows, items)
         return rows * num_heads * head_dim, rows * num_heads
 
     def streams_decoded_tokens(self, num_heads: int, num_kv_heads: int, head_dim: int, element_size: int, block_size: int) -> bool:

@@ -118,7 +118,8 @@ class AttentionMixer(Mixer):
         sizes = getattr(ops, "attention_scratch_elems", None)
         if sizes is None:
             return {}
-        partial_out, partial_lse = sizes(self.num_heads, self.num_kv_heads, self.head_dim, limits.max_num_tokens, limits.max_num_seqs, limits.max_model_len)
+        partial_out, partial_lse = sizes(self.num_heads, self.num_kv_heads, self.head_dim, limits.max_num_tokens, limits.max_num_seqs, limits.max_model_len,
+                                         block_size=limits.block_size)
         return {"attention_partial_out": partial_out, "attention_partial_lse": partial_lse, "attention_arrivals": limits.max_num_seqs * self.num_kv_heads}
 
     products_in_parts = ("o_weight",)

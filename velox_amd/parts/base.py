@@ -145,7 +145,7 @@ class Part:
 
     def workspace_needs(self, ops, limits) -> Dict[str, int]:
         """Scratch this part may ask ``ctx.workspace`` for: buffer name -> the most float32 elements, for any step within
-        ``limits`` (``max_num_tokens``, ``max_num_seqs``, ``max_model_len``).  The step function reserves these before it
+        ``limits`` (``max_num_tokens``, ``max_num_seqs``, ``max_model_len``, ``block_size``).  The step function reserves these before it
         runs or captures anything and refuses to grow them later, because captured steps hold their addresses."""
         return {}
 
