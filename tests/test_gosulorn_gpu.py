@@ -828,3 +828,26 @@ def test_lengths_say_which_kernels_the_shorter_portions_need(ops, lengths):
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
     want = 0 if all(n == 0 or n >= ops.LINEAR_CHUNK_TOKENS for n in lengths) else 1 if all(n <= 2 or n >= ops.LINEAR_CHUNK_TOKENS for n in lengths) else 2
     assert ops.shorter_portions(tokens, len(lengths), max(lengths), ops.LINEAR_CHUNK_TOKENS, lengths) == want
+
+
+@pytest.mark.parametrize("rule, heads, dim, vdim", [("delta", 2, 64, 20), ("delta", 24, 128, 64), ("additive", 24, 64, 80)])
+@pytest.mark.parametrize("lengths", [[33, 1, 70, 2, 32, 100], [33] * 12 + [1, 50], [40] + [1] * 40 + [60, 1], [1] * 66 + [40, 2, 100, 1], [48] + [1] * 70 + [33], [35] * 70])
+def test_long_portions_in_every_order_that_workgroups_take_them_in(ops, rule, heads, dim, vdim, lengths):
+    """Few workgroups look for the longest sequence first, many, or those of more than 64 sequences, go from the back, and with the lengths at hand
+    there are none for the short ones in front: the same bits as without the lengths and as each sequence alone has, which may have a
+    compute unit to itself."""
+    run = scan_case(lengths, rule, rule == "additive", heads, heads, dim, vdim, torch.bfloat16)
+    everything = list(range(len(lengths)))
+    guessed, states = run(ops, everything)
+    known, after = run(ops, everything, q_lens=lengths)
+    assert all(torch.equal(a, b) for a, b in zip(guessed + states, known + after))
+    for i in sorted({0, len(lengths) // 2, len(lengths) - 1}):
+        (alone,), (end,) = run(ops, [i], q_lens=[lengths[i]])
+        assert torch.equal(known[i], alone) and torch.equal(after[i], end), lengths[i]
+
+
+def test_which_sequences_the_long_portions_are_among(ops):
+    assert ops.long_portions(5, 32) == (5, 5)
+    assert ops.long_portions(5, 32, [1, 40, 2, 32, 31]) == (2, 4)
+    assert ops.long_portions(3, 32, [40, 1, 1]) == (1, 3)
+    assert ops.long_portions(3, 32, [1, 1, 90]) == (1, 1)

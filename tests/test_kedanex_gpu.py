@@ -194,6 +194,29 @@ def test_pieces_and_chunks_among_many_sequences(ops, lengths):
     torch.testing.assert_close(states[0], states[1], rtol=2e-5, atol=2e-6)
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 64), (32, 64, 64), (32, 128, 64), (3, 16, 20)])
+@pytest.mark.parametrize("lengths", [(1, 1, 40, 1, 16, 17, 2, 100, 1, 33), (1,) * 12 + (70,), (48,) + (1,) * 66 + (32, 1)])
+def test_a_sequences_bits_are_those_it_has_alone_in_every_order_of_workgroups(ops, heads, dim, vdim, lengths):
+    """Few workgroups look for the longest sequence first and have a compute unit to themselves, many, or those of more than 64 sequences, go from
+    the back; sequences of one chunk read less ahead."""
+    count, rank, ks, vs = len(lengths), 8, heads * dim, heads * vdim
+    at = (0, ks, 2 * ks, 2 * ks + vs, 3 * ks + 2 * vs)
+    main = torch.randn(sum(lengths), 3 * ks + 2 * vs + rank).bfloat16().cuda()
+    w2, a_bias, w0 = torch.randn(ks, rank).bfloat16().cuda(), torch.randn(ks).cuda(), torch.randn(ks).cuda()
+    start, cu = torch.randn(count, heads, dim, vdim).cuda() * 0.3, [0] + list(np.cumsum(lengths))
+
+    def run(which):
+        state, rows = start.clone(), torch.cat([main[cu[i]:cu[i + 1]] for i in which])
+        out = ops.removal_scan(rows, *at, rank, heads, dim, vdim, a_bias, w2, w0, math.exp(-0.5), state, ints(which), ints([0] + list(np.cumsum([lengths[i] for i in which]))),
+                               max(lengths[i] for i in which), chunked=True)
+        return out, state
+
+    out, state = run(range(count))
+    for i in sorted({0, 2, count // 2, count - 1}):
+        alone, after = run([i])
+        assert torch.equal(alone, out[cu[i]:cu[i + 1]]) and torch.equal(after[i], state[i]), lengths[i]
+
+
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 64), (1, 128, 128), (3, 32, 48), (2, 12, 12), (1, 256, 16), (1, 72, 40)])
 def test_a_long_portion_equals_its_pieces_and_its_first_token_is_kept(ops, heads, dim, vdim):
     """600 tokens in one step, in pieces (one of a single token, one of two) and against the plain loop; with decays close

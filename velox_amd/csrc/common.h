@@ -107,20 +107,38 @@ __device__ __forceinline__ void rows_from_lines(float4_t& first, float4_t& secon
   }
 }
 
-// The sequence with the `rank`-th most tokens, ties in their order (beyond 64 sequences: from the back, since a step's single tokens come before
-// its portions of prompts).  The whole wave takes part.  For grids of a workgroup per sequence whose time is the longest chain's: it
-// has to begin with the first workgroups.
-__device__ __forceinline__ int sequence_by_length(const int* cu_q, int num_seqs, int rank) {
-  if (num_seqs > VELOX_WAVE) return num_seqs - 1 - rank;
+// Grids of a workgroup per sequence, head and tile whose time is the longest chain's: it has to begin with the first workgroups.  With up to
+// ORDERED_WORKGROUPS of them each looks for the sequence with the `rank`-th most tokens (ties in their order); with more, where that would cost more than
+// it gives, or beyond 64 sequences, it goes from the back, since a step's single tokens come before its portions of prompts.  (Chunks' read-outs of
+// 32 heads of 64 x 64, us, searched / from the back: 60 single tokens beside 1,024 119 / 109, 64 portions of 64 282 / 269.)  The whole wave takes
+// part; the lengths are gone through from their highest bit down, a few scalar instructions each.
+constexpr long long ORDERED_WORKGROUPS = 1024;
+static inline bool orders_sequences(long long workgroups, int num_seqs) { return num_seqs <= VELOX_WAVE && workgroups <= ORDERED_WORKGROUPS; }
+
+__device__ __forceinline__ int sequence_by_length(const int* cu_q, int num_seqs, int rank, bool ordered) {
+  if (!ordered) return num_seqs - 1 - rank;
   const int lane = threadIdx.x & (VELOX_WAVE - 1), at = lane < num_seqs ? lane : 0;
-  const int mine = lane < num_seqs ? cu_q[at + 1] - cu_q[at] : -1;
-  int before = 0;
-  for (int b = 0; b < num_seqs; ++b) {
-    const int other = __builtin_amdgcn_readlane(mine, b);
-    before += other > mine || (other == mine && b < lane) ? 1 : 0;
+  const int begin = cu_q[at], mine = cu_q[at + 1] - begin;
+  const int total = __builtin_amdgcn_readlane(begin + mine, num_seqs - 1);
+  uint64_t among = __ballot(lane < num_seqs);
+  for (int bit = 31 - __builtin_clz(total | 1); bit >= 0; --bit) {
+    const uint64_t more = among & __ballot((mine >> bit) & 1);
+    const int count = __popcll((unsigned long long)more);
+    if (rank < count) {
+      among = more;
+    } else {
+      rank -= count;
+      among &= ~more;
+    }
   }
-  return __ffsll((unsigned long long)__ballot(lane < num_seqs && before == rank)) - 1;
+  const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(among >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)among, 0));  // of the lanes before this one
+  return __ffsll((unsigned long long)__ballot(before == rank && ((among >> lane) & 1))) - 1;
 }
+
+// Grids of chains of up to ALONE_WORKGROUPS workgroups have a compute unit each to themselves: with ALONE_LDS bytes of LDS more no second one fits.  (Two
+// chains on a compute unit slow each other down, many short ones hide each other's waits.  Three portions of 400 to 1,300 tokens, 32 heads of 64 x 64,
+// 384 workgroups, us, up to two a compute unit / one: 134 / 124; eight of 300, 16 heads of 64 x 64, 512: 48 / 52; 32 heads, 1,024: 84 / 90.)
+constexpr size_t ALONE_WORKGROUPS = 384, ALONE_LDS = 80 * 1024;
 
 // Four consecutive elements of a row, widened to float32: one 8- or 16-byte access when `vec_ok` (the row starts on such a
 // boundary and k is a multiple of 4) and all four lie below k_limit, else element by element with zeros beyond k_limit.

@@ -49,6 +49,7 @@ struct LinearChunkArgs {
   int heads, kv_heads, dim, vdim;
   int num_seqs, long_from;      // sequences of at least long_from tokens are worked
   int first_head, head_count;   // the heads that this launch works; their records lie side by side in `scratch`
+  bool ordered;                 // the scan's sequences by their length, see sequence_by_length
 };
 
 // A chunk and head in `scratch`, in floats: -U' | R' | K' (each 16 * dim), P_16 (dim), Dv | Ov (each 16 * columns).  U' and R' as
@@ -270,14 +271,16 @@ struct ChunkReads {
 // read-outs a chunk later; buffer loads and stores leave the vector unit no addresses to add up.  One barrier a chunk: a buffer of `removed`
 // or `states` is written again behind the next chunk's barrier, one of `reads` behind the one that follows its readers'.  Measured on MI355X,
 // 82 chunks of the longest of three sequences, us, with everything in one chain / this: 8 heads of 128 x 128 72 / 55, 16 heads 77 / 58, additive, 8
-// heads of 128 x 256, 46 / 41.
+// heads of 128 x 256, 46 / 41.  Many short chains, prepared and scanned (with one workgroup a compute unit): 32 heads of 64 x 64, 64 portions of 64
+// 189 / 184 (288), of 200 488 / 477 (592); 32 heads of 128 x 128 613 / 530 (710), additive, 8 heads of 128 x 256, 202 / 183 (282): there is no bound from
+// above on a SIMD's waves, and the additive rule's fit the registers of eight.
 template <int WAVES, bool DELTA>
-__global__ void __launch_bounds__(128 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES / 2, WAVES / 2))) linear_chunk_scan_kernel(const LinearChunkArgs a) {
+__global__ void __launch_bounds__(128 * WAVES) __attribute__((amdgpu_waves_per_eu(DELTA ? WAVES / 2 : 8))) linear_chunk_scan_kernel(const LinearChunkArgs a) {
   static_assert(WAVES == 4 || WAVES == 8, "a chunk's 256 read-outs are finished by 256 lanes of the readers");
   __shared__ float4_t removed[2][DELTA ? WAVES : 1][64], reads[2][WAVES][64], states[2][WAVES][64];  // [buffer][wave][lane]
   // (heads lie along the grid's first dimension in both kernels: with a multiple of 8 heads the workgroups that read a record run
   // on the XCD that wrote it and share it in that XCD's L2)
-  const int h = a.first_head + blockIdx.x, tile = blockIdx.y, b = __builtin_amdgcn_readfirstlane(sequence_by_length(a.cu_q, a.num_seqs, blockIdx.z));
+  const int h = a.first_head + blockIdx.x, tile = blockIdx.y, b = __builtin_amdgcn_readfirstlane(sequence_by_length(a.cu_q, a.num_seqs, blockIdx.z, a.ordered));
   const int lo = __builtin_amdgcn_readfirstlane(a.cu_q[b]), hi = __builtin_amdgcn_readfirstlane(a.cu_q[b + 1]);
   if (hi - lo < a.long_from || hi <= lo) return;  // (the whole workgroup)
   const int lane = threadIdx.x & 63, any_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -414,12 +417,15 @@ extern "C" long long velox_linear_chunk_scratch_elems(int tokens, int num_seqs, 
 }
 
 template <bool DELTA>
-static void linear_chunk_launch(const LinearChunkArgs& a, int tokens, hipStream_t stream) {
+static void linear_chunk_launch(LinearChunkArgs a, int tokens, int long_seqs, int long_span, hipStream_t stream) {
   const size_t lds = (size_t)CHUNK * (3 * (a.dim + 4) + 4 * CHUNK_STRIDE) * sizeof(float);
   linear_chunk_prepare_kernel<DELTA><<<(unsigned)records_of_step(tokens, a.num_seqs) * (unsigned)a.head_count, 256, lds, stream>>>(a);
-  const dim3 grid(a.head_count, chunk_columns(a.vdim) / 16, a.num_seqs);
-  if (a.dim == 64) linear_chunk_scan_kernel<4, DELTA><<<grid, 512, 0, stream>>>(a);
-  else linear_chunk_scan_kernel<8, DELTA><<<grid, 1024, 0, stream>>>(a);
+  const int tiles = chunk_columns(a.vdim) / 16;
+  a.ordered = orders_sequences((long long)a.head_count * tiles * long_seqs, a.num_seqs);
+  const dim3 grid(a.head_count, tiles, a.ordered ? long_seqs : long_span);
+  const size_t alone = (long long)grid.x * grid.y * grid.z <= ALONE_WORKGROUPS ? ALONE_LDS : 0;
+  if (a.dim == 64) linear_chunk_scan_kernel<4, DELTA><<<grid, 512, alone, stream>>>(a);
+  else linear_chunk_scan_kernel<8, DELTA><<<grid, 1024, alone, stream>>>(a);
 }
 
 extern "C" int velox_linear_scan(const float* qk, const void* v, int v_dtype, int v_ld, int v_at, const float* decay, int decay_per_channel, const float* beta,
@@ -428,22 +434,24 @@ extern "C" int velox_linear_scan(const float* qk, const void* v, int v_dtype, in
 
 // The sequences of at least `long_from` tokens, then the shorter ones token by token: `shorter` says which kernels they may need (0: there
 // are none, 1: single tokens and pairs, 2: longer ones too).  Launched from here, since a call costs the host more than a launch.
+// There are at most `long_seqs` of the former, all among the last `long_span` sequences: a scan's workgroup of another sequence finds nothing to do,
+// but 60 single tokens beside a portion of 1,024 have 15,360 of them with 32 heads of 128 x 128 (319 us with them, 224 without).
 // beta: nullptr for the additive rule.  `scratch` holds the records of `heads_at_once`
 // heads (velox_linear_chunk_scratch_elems each), which are worked one such group after the other.  qk and a decay per channel are
 // read in 16-byte pieces (dim is a multiple of 16; the caller checks that the bases are aligned).
 extern "C" int velox_linear_chunk_scan(const float* qk, const void* v, int v_dtype, int v_ld, int v_at, const float* decay, int decay_per_channel,
                                        const float* beta, float* scratch, float* state, const int* slots, const int* cu_q, float* out, int num_seqs,
-                                       int tokens, int long_from, int shorter, int heads_at_once, int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
+                                       int tokens, int long_from, int long_seqs, int long_span, int shorter, int heads_at_once, int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
   if (num_seqs <= 0 || tokens <= 0) return 0;
   if (velox_linear_chunk_scratch_elems(tokens, num_seqs, dim, vdim) == 0 || heads < 1 || heads > 65535 || num_seqs > 65535 || heads_at_once < 1 ||
-      (long long)records_of_step(tokens, num_seqs) * (heads_at_once < heads ? heads_at_once : heads) > (1 << 23) || vdim > 65535 * 16 || kv_heads < 1 ||
+      (long long)records_of_step(tokens, num_seqs) * (heads_at_once < heads ? heads_at_once : heads) > (1 << 23) || vdim > 65535 * 16 || kv_heads < 1 || long_seqs < 1 || long_seqs > long_span || long_span > num_seqs ||
       heads % kv_heads != 0 || !scratch)
     return (int)hipErrorInvalidValue;
   for (int first = 0; first < heads; first += heads_at_once) {
     LinearChunkArgs a{qk, v, v_dtype == VELOX_BF16, v_ld, v_at, decay, decay_per_channel, beta, scratch, state, slots, cu_q, out, heads, kv_heads, dim, vdim,
-                      num_seqs, long_from, first, heads - first < heads_at_once ? heads - first : heads_at_once};
-    if (beta) linear_chunk_launch<true>(a, tokens, stream);
-    else linear_chunk_launch<false>(a, tokens, stream);
+                      num_seqs, long_from, first, heads - first < heads_at_once ? heads - first : heads_at_once, false};
+    if (beta) linear_chunk_launch<true>(a, tokens, long_seqs, long_span, stream);
+    else linear_chunk_launch<false>(a, tokens, long_seqs, long_span, stream);
   }
   const int status = (int)hipGetLastError();
   if (status != 0 || shorter == 0) return status;

@@ -37,6 +37,7 @@ struct RemovalChunkArgs {
   const int* slots;
   const int* cu_q;
   float* out;  // [T, heads * vdim]
+  bool ordered;  // the scan's sequences by their length, see sequence_by_length
 };
 
 // A chunk and head in `scratch`, in floats: U' | R' | -B | K (each 16 * dim), P_16 (dim), Dv | Ov | V (each 16 * columns).  U' and R' as
@@ -279,15 +280,19 @@ struct RemovalReads {
 // to add up.  One barrier a chunk: a buffer of `removed` or `states` is written again behind the next chunk's barrier, one of `reads` behind the
 // one that follows its readers'.  Measured on MI355X, 64 chunks, 32 heads of 64 x 64: 41.0 us with everything in one chain, 35.8 with the read-outs
 // a chunk later and buffer operations, 31.0 with waves of their own for them.
-// (At most 256 registers a wave: the matrix instructions then keep the state in ordinary registers.)
+// (At most 256 registers a wave: the matrix instructions then keep the state in ordinary registers.  There is no bound from above on a SIMD's waves: for
+// one the compiler asks for registers that nothing uses, and many short chains wait.)  Prepared and scanned, with everything in one chain / like this (with
+// one workgroup a compute unit and loads ahead for single tokens), us: 32 heads of 64 x 64, 64 portions of 64 276 / 269 (390), 60 single tokens beside
+// 1,024 150 / 109 (242), 200 beside 300 309 / 249 (409); 16 heads of 128 x 128 456 / 453 (549), 259 / 185 (333), 589 / 435 (649).
 template <int WAVES>
-__global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1)) __attribute__((amdgpu_waves_per_eu(2, 2))) removal_chunk_scan_kernel(const RemovalChunkArgs a) {
+__global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1)) __attribute__((amdgpu_waves_per_eu(2))) removal_chunk_scan_kernel(const RemovalChunkArgs a) {
   constexpr bool READERS = removal_readers(WAVES);
   __shared__ float4_t removed[2][WAVES][64], reads[2][WAVES][64], states[READERS ? 2 : 1][READERS ? WAVES : 1][64];  // the waves' parts of D and O, [buffer][wave][lane]
   // (heads lie along the grid fastest in both kernels: with a multiple of 8 heads the workgroups that read a record run
   // on the XCD that wrote it and share it in that XCD's L2)
-  // (the long chains begin first, not when the single tokens in front of them are done: 12 beside 1,024, 32 heads of 64 x 64, 49 -> 38 us)
-  const int h = blockIdx.x, tile = blockIdx.y, b = __builtin_amdgcn_readfirstlane(sequence_by_length(a.cu_q, gridDim.z, blockIdx.z));
+  // (the long chains begin first, not when the single tokens in front of them are done: 12 beside 1,024, 32 heads of 64 x 64, 49 -> 38 us;
+  // prepared and scanned 94 -> 83, and 76 since those read nothing ahead)
+  const int h = blockIdx.x, tile = blockIdx.y, b = __builtin_amdgcn_readfirstlane(sequence_by_length(a.cu_q, gridDim.z, blockIdx.z, a.ordered));
   const int lo = __builtin_amdgcn_readfirstlane(a.cu_q[b]), hi = __builtin_amdgcn_readfirstlane(a.cu_q[b + 1]);
   if (hi <= lo) return;  // (the whole workgroup)
   const int lane = threadIdx.x & 63, any_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -418,19 +423,24 @@ __global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1))
     // between a chunk's loads and its work on every path, so that waiting for the one does not wait for the others.
     RemovalOperands ops[SCAN_AHEAD];
     RemovalReads<WAVES> of_reads[SCAN_AHEAD];
+    if (chunks == 1) {  // (single tokens beside a long portion: a quarter of the loads)
+      load(ops[0], of_reads[0]);
+      work(0, ops[0], of_reads[0]);
+    } else {
 #pragma unroll
-    for (int j = 0; j < SCAN_AHEAD; ++j) load(ops[j], of_reads[j]);
-    int c = 0;
-    for (; c + SCAN_AHEAD <= chunks; c += SCAN_AHEAD) {
+      for (int j = 0; j < SCAN_AHEAD; ++j) load(ops[j], of_reads[j]);
+      int c = 0;
+      for (; c + SCAN_AHEAD <= chunks; c += SCAN_AHEAD) {
 #pragma unroll
-      for (int j = 0; j < SCAN_AHEAD; ++j) {
-        work(j & 1, ops[j], of_reads[j]);
-        load(ops[j], of_reads[j]);
+        for (int j = 0; j < SCAN_AHEAD; ++j) {
+          work(j & 1, ops[j], of_reads[j]);
+          load(ops[j], of_reads[j]);
+        }
       }
-    }
 #pragma unroll
-    for (int j = 0; j < SCAN_AHEAD - 1; ++j)
-      if (c + j < chunks) work(j & 1, ops[j], of_reads[j]);  // (the same for the whole workgroup)
+      for (int j = 0; j < SCAN_AHEAD - 1; ++j)
+        if (c + j < chunks) work(j & 1, ops[j], of_reads[j]);  // (the same for the whole workgroup)
+    }
     meet();
     if constexpr (READS) read_out((chunks - 1) & 1, last_reads);
     if constexpr (CHAINS) {
@@ -459,20 +469,23 @@ extern "C" long long velox_removal_chunk_scratch_elems(int tokens, int num_seqs,
 }
 
 template <typename T>
-static void removal_chunk_launch(const RemovalChunkArgs& a, int tokens, int num_seqs, hipStream_t stream) {
+static void removal_chunk_launch(RemovalChunkArgs a, int tokens, int num_seqs, hipStream_t stream) {
   // (1,024 tokens beside 12 single ones, 32 heads of 64 x 64, us: with the longest portion's chunks for every sequence 55.4, so 51.0, and six workgroups per
   // compute unit 44.4)
-  removal_chunk_prepare_kernel<T><<<(unsigned)(a.heads * step_items(tokens, num_seqs, CHUNK)), 256, removal_prepare_lds(a.dim, a.rank), stream>>>(a, num_seqs);
   const dim3 grid(a.heads, removal_columns(a.vdim) / 16, num_seqs);
+  const long long workgroups = (long long)grid.x * grid.y * grid.z;
+  a.ordered = orders_sequences(workgroups, num_seqs);
+  const size_t alone = workgroups <= ALONE_WORKGROUPS ? ALONE_LDS : 0;
+  removal_chunk_prepare_kernel<T><<<(unsigned)(a.heads * step_items(tokens, num_seqs, CHUNK)), 256, removal_prepare_lds(a.dim, a.rank), stream>>>(a, num_seqs);
   switch (a.dim / 16) {
-    case 1: removal_chunk_scan_kernel<1><<<grid, 128, 0, stream>>>(a); break;
-    case 2: removal_chunk_scan_kernel<2><<<grid, 256, 0, stream>>>(a); break;
-    case 3: removal_chunk_scan_kernel<3><<<grid, 384, 0, stream>>>(a); break;
-    case 4: removal_chunk_scan_kernel<4><<<grid, 512, 0, stream>>>(a); break;
-    case 5: removal_chunk_scan_kernel<5><<<grid, 320, 0, stream>>>(a); break;
-    case 6: removal_chunk_scan_kernel<6><<<grid, 384, 0, stream>>>(a); break;
-    case 7: removal_chunk_scan_kernel<7><<<grid, 448, 0, stream>>>(a); break;
-    default: removal_chunk_scan_kernel<8><<<grid, 512, 0, stream>>>(a); break;
+    case 1: removal_chunk_scan_kernel<1><<<grid, 128, alone, stream>>>(a); break;
+    case 2: removal_chunk_scan_kernel<2><<<grid, 256, alone, stream>>>(a); break;
+    case 3: removal_chunk_scan_kernel<3><<<grid, 384, alone, stream>>>(a); break;
+    case 4: removal_chunk_scan_kernel<4><<<grid, 512, alone, stream>>>(a); break;
+    case 5: removal_chunk_scan_kernel<5><<<grid, 320, alone, stream>>>(a); break;
+    case 6: removal_chunk_scan_kernel<6><<<grid, 384, alone, stream>>>(a); break;
+    case 7: removal_chunk_scan_kernel<7><<<grid, 448, alone, stream>>>(a); break;
+    default: removal_chunk_scan_kernel<8><<<grid, 512, alone, stream>>>(a); break;
   }
 }
 
@@ -483,7 +496,7 @@ extern "C" int velox_removal_chunk_scan(const void* main, int dtype, int ld, int
   if (velox_removal_chunk_scratch_elems(tokens, num_seqs, heads, dim, vdim, rank) == 0 || heads < 1 || heads > 65535 || num_seqs > 65535 ||
       heads * step_items(tokens, num_seqs, CHUNK) > 0x7fffffff || !scratch || !(scale * CHUNK < 13.f))
     return (int)hipErrorInvalidValue;
-  RemovalChunkArgs a{main, ld, r_at, k_at, v_at, a_at, low_at, rank, heads, dim, vdim, a_bias, w2, w0, scale, scratch, state, slots, cu_q, out};
+  RemovalChunkArgs a{main, ld, r_at, k_at, v_at, a_at, low_at, rank, heads, dim, vdim, a_bias, w2, w0, scale, scratch, state, slots, cu_q, out, false};
   if (dtype == VELOX_BF16) removal_chunk_launch<bf16_t>(a, tokens, num_seqs, stream);
   else removal_chunk_launch<float>(a, tokens, num_seqs, stream);
   VELOX_RETURN_LAUNCH_STATUS();

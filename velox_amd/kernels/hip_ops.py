@@ -217,7 +217,7 @@ class HipOps:
         c.velox_tiles_splits.argtypes = [_I, _I, _I, _I]
         for fn in (c.velox_tiles_bf16, c.velox_tiles_glu_bf16, c.velox_tiles_splits):
             fn.restype = _I
-        c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]
+        c.velox_linear_chunk_scan.argtypes = [_P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         c.velox_linear_chunk_scan.restype = _I
         c.velox_linear_chunk_scratch_elems.argtypes = [_I, _I, _I, _I]
         c.velox_linear_chunk_scratch_elems.restype = ctypes.c_longlong
@@ -1585,6 +1585,12 @@ class HipOps:
         most = max((n for n in q_lens if n < long_from), default=0)
         return 0 if most == 0 else 1 if most <= 2 else 2
 
+    @staticmethod
+    def long_portions(sequences: int, long_from: int, q_lens: Optional[Sequence[int]] = None) -> Tuple[int, int]:
+        """How many sequences have at least ``long_from`` tokens, at most, and among how many last ones they all are."""
+        at = None if q_lens is None else [i for i, n in enumerate(q_lens) if n >= long_from]
+        return (len(at), sequences - at[0]) if at else (sequences, sequences)
+
     def linear_scan(self, qk, v_source, v_at, decay, beta, state, slots, cu_q, max_q_len, heads, kv_heads, dim, vdim, rule, chunked: Optional[bool] = None,
                     q_lens: Optional[Sequence[int]] = None):
         """Per sequence and head, token by token from ``state[slot, head]`` ([dim, vdim] float32), which is written back:
@@ -1635,7 +1641,7 @@ class HipOps:
         scratch = torch.empty(per_head * heads_at_once, dtype=torch.float32, device=self.device)
         self._launched(self._core.velox_linear_chunk_scan(_ptr(qk), _ptr(v_source), _code(v_source.dtype), v_source.shape[1], int(v_at), _ptr(decay), int(per_channel),
                                                           _ptr(beta) if delta else _P(0), _ptr(scratch), _ptr(state), _ptr(slots), _ptr(cu_q), _ptr(out), sequences, tokens,
-                                                          long_from, shorter, heads_at_once, int(heads), int(kv_heads), int(dim), int(vdim), self._stream()), "linear_chunk_scan")
+                                                          long_from, *self.long_portions(sequences, long_from, q_lens), shorter, heads_at_once, int(heads), int(kv_heads), int(dim), int(vdim), self._stream()), "linear_chunk_scan")
         return out
 
     def gated_head_norm(self, read, weight, eps, gate_source, gate_at, gate_kind, heads, vdim, out_dtype):
