@@ -184,3 +184,9 @@ def test_scratch_for_shares_of_keys_is_that_of_the_caches_pages(page, keys, rows
     """100 single tokens of 28 heads over 4: workgroups per KV head that share out the step's keys, as many as hold the page ids of so many keys, or
     what the splits of portions take."""
     assert rules_of_the_kernels().attention_scratch_elems(28, 4, 128, 100, 100, keys, block_size=page) == (rows * 28 * 128, rows * 28)
+
+
+@pytest.mark.parametrize("rows,outputs,streamed", [(17, 16384, True), (17, 16383, False), (32, 18000, True), (32, 152064, True), (33, 16384, True), (33, 18000, False),
+                                                   (64, 22000, False), (64, 24576, True), (64, 32000, True), (33, 34000, False), (48, 65536, True), (33, 152064, False)])
+def test_heads_of_some_rows_that_fill_whole_rounds_of_workgroups_are_streamed(rows, outputs, streamed):
+    assert rules_of_the_kernels().streams_head(rows, outputs) == streamed

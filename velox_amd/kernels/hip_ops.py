@@ -837,10 +837,7 @@ class HipOps:
                 and 16 < m <= 64 and k % 64 == 0 and n <= 8192 and n % 4 == 0):
             return self.skinny_gemm_splitk(x, weight, packed=packed)
         if (out_dtype == torch.float32 and bias is None and packed is not None and self.use_skinny_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
-                and 16 < m <= 64 and k % 64 == 0 and n % 4 == 0 and n >= 64 * self.num_cus and (m <= 32 or n <= 65536)):
-            # The head over more rows than the skinny kernel takes: the kernel that stages the activations of 64 rows of W streams the packed copy.
-            # Measured on MI355X (us, the library / this): 152,064 x 3,584, 17 rows 253 / 192, 25 257 / 203, 33 207 / 220, 57 221 / 243; 151,936 x 1,536,
-            # 25 109 / 98, 57 119 / 120; 32,000 x 4,096, 17 61 / 49, 33 62 / 52, 57 64 / 55.
+                and 16 < m <= 64 and k % 64 == 0 and n % 4 == 0 and self.streams_head(m, n)):
             return self.skinny_gemm_splitk(x, weight, splits=1, packed=packed)[0]
         if out_dtype == torch.bfloat16 and self.use_library_gemm and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
             parts = self.own_tile_parts(m, n, k, partials_ok and bias is None)
@@ -864,6 +861,16 @@ class HipOps:
             if splits > 0:
                 return self.split_f32(x, weight, bias, splits)
         return self.gemm_fma(x, weight, bias, out_dtype)
+
+    def streams_head(self, m: int, n: int) -> bool:
+        """Whether the head over more rows than the skinny kernel takes is the product of the kernel that stages the activations of 64 rows of W
+        and streams the packed copy.  Measured on MI355X (us, the library / this): 152,064 x 3,584, 17 rows 253 / 192, 25 257 / 203, 33 207 / 220, 57
+        221 / 243; 151,936 x 1,536, 25 109 / 98, 57 119 / 120; 32,000 x 4,096, 17 61 / 49, 33 62 / 52, 57 64 / 55; 33 and 64 rows of 49,152 x 4,096
+        94 / 79, 93 / 85, 65,536 x 4,096 129 / 104, 131 / 115, 128,256 x 2,048 129 / 107, 134 / 120, x 4,096 213 / 207, 220 / 224.  Beyond 32 rows not where
+        the last round of workgroups is nearly empty, either: 18,000 x 4,096 40.2 / 42.0, 43.3 / 46.9, 22,000 x 2,048 25.5 / 24.6, 27.2 / 28.3, 24,576 x
+        4,096 51.1 / 47.5, 51.5 / 51.1."""
+        whole = 64 * self.num_cus  # rows of W in a round
+        return n >= whole and (m <= 32 or (n <= 4 * whole and 10 * n >= 7 * -(-n // whole) * whole))
 
     def _bias_in_bfloat16(self, bias: torch.Tensor) -> torch.Tensor:
         """A bfloat16 copy of a float32 bias vector, made once per vector (keyed by its storage; the float32 vector is kept
@@ -945,6 +952,7 @@ class HipOps:
         blocks = (n + 15) // 16
         # up to four rows of a narrow weight have a kernel of their own (see there); measured on MI355X, us, that one / half tiles below: 1,536 x
         # 8,960 with 1, 2 rows 7.6 / 9.6, 8.1 / 9.8, 1,536 x 1,536 with 1, 2, 4, 8 3.4 / 3.9, 3.5 / 3.9, 3.9 / 4.1, 4.2 / 4.1, 2,048 x 5,632 6.6 / 7.1
+        # (three and four rows of sums of 4,096 into 2,048 are the ones that lose: 6.5 / 6.0, 6.6 / 6.1; of 2,048 4.4 / 4.6, three of 5,632 7.1 / 7.3)
         few = parts is not None or (row_tiles is None and waves is None and m <= 4 and n >= 512 and 2 * blocks <= self.num_cus and self._few_rows_pieces(m, k) <= 10)
         if row_tiles is None:
             # one 16-row tile of the weight per workgroup while that is at most one workgroup per compute unit; a wider
