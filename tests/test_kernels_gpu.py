@@ -823,9 +823,72 @@ def test_decoded_tokens_whose_keys_are_shared_out(ops, ref, dtype, nh, nkv, d, p
     assert torch.equal(run(moved), got[order])
 
 
-@pytest.mark.parametrize("count", [65279, 65280, 65535])
-def test_more_decoded_tokens_than_a_grid_has_room_for_when_keys_are_shared_out(ops, count):
-    """Their keys are then split equally: 65,535 single tokens were always taken."""
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("sinks", [False, True])
+@pytest.mark.parametrize("nh,nkv,d,page", [(28, 4, 128, 16), (4, 4, 64, 4)])
+def test_a_captured_step_shares_its_keys_out_by_the_lengths_of_each_replay(ops, ref, dtype, sinks, nh, nkv, d, page):
+    """One launch captured for up to 4,096 keys (9,000 with pages of four tokens, more page ids than a share has room for) and a workspace that is as
+    large as was asked for: its replays cut the sequences by their lengths, and leave the counters of arrivals at zero."""
+    from velox_amd.engine.batch import Workspace
+
+    most = 4096 if page == 16 else 9000
+    case = _attention_case(dtype, nh, nkv, d, page, [(1, most - 7 * b) for b in range(16)], seed=7)
+    out_elems, lse_elems = ops.attention_scratch_elems(nh, nkv, d, 16, 16, most, block_size=page)
+    workspace = Workspace(torch.device("cuda"))
+    for name, elems in (("attention_partial_out", out_elems), ("attention_partial_lse", lse_elems), ("attention_arrivals", 16 * nkv)):
+        workspace.reserve(name, elems)
+    workspace.fix()
+    sink = rand((nh,), torch.float32, 8, 2.0) if sinks else None
+
+    def run():
+        return ops.paged_attention(case["qkv"], nh, nkv, d, case["k_cache"], case["v_cache"], page, case["tables"], case["cu"], case["kv"], 1, most, 1.0 / math.sqrt(d),
+                                   None, True, workspace, uneven=True, sinks=sink)
+
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = run()
+    full = case["kv"].tolist()
+    for lens in ([30 + b for b in range(16)], full, [1] * 15 + [full[15]], full[:1] + [17] * 15, [500, 1, 2000, 64, 65, 300, 1500, 16] * 2, [1] * 16):
+        case["kv"].copy_(torch.tensor(lens, dtype=torch.int32))
+        for _ in range(2):
+            graph.replay()
+            got = captured.clone()
+            torch.cuda.synchronize()
+            assert not workspace.get("attention_arrivals", 16 * nkv).any()
+            assert torch.equal(got, run())
+        want = ref.paged_attention(case["qkv"], nh, nkv, d, case["k_cache"], case["v_cache"], page, case["tables"], case["cu"], case["kv"], 1, max(lens), 1.0 / math.sqrt(d),
+                                   None, True, None, sinks=sink).float()
+        torch.testing.assert_close(got.float(), want, **(dict(rtol=1e-4, atol=1e-5) if dtype == torch.float32 else dict(rtol=2e-2, atol=2e-2)))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_keys_shared_out_in_front_of_portions(ops, ref, dtype):
+    """A mixed step: its single tokens' shares and its portions' splits use the same scratch, one after the other."""
+    from velox_amd.engine.batch import Workspace
+
+    nh, nkv, d, page = 16, 4, 64, 16
+    lens = [900, 3, 250, 64, 1, 2000, 128, 129, 17, 16]
+    case = _attention_case(dtype, nh, nkv, d, page, [(1, n) for n in lens] + [(70, 4500), (3, 3)], seed=9)
+    workspace = Workspace(torch.device("cuda"))
+    assert ops.shares_keys(len(lens), nkv)
+
+    def run(**more):
+        return ops.paged_attention(case["qkv"], nh, nkv, d, case["k_cache"], case["v_cache"], page, case["tables"], case["cu"], case["kv"], 70, 4500, 1.0 / math.sqrt(d), None,
+                                   False, workspace, decode_prefix=len(lens), portions_max_kv_len=4500, **more).float()
+
+    got = run(uneven=True)
+    want = _run_attention(ref, case, nh, nkv, d, page)
+    torch.testing.assert_close(got, want, **(dict(rtol=1e-4, atol=1e-5) if dtype == torch.float32 else dict(rtol=2e-2, atol=2e-2)))
+    assert not workspace.get("attention_arrivals", len(lens) * nkv).any()
+    assert torch.equal(run(uneven=True), got) and torch.equal(run()[len(lens):], got[len(lens):])
+
+
+@pytest.mark.parametrize("count,items", [(65280, None), (65535, None), (100, 65536), (100, 65535)])
+def test_more_decoded_tokens_or_shares_than_a_grid_has_room_for(ops, monkeypatch, count, items):
+    """Single tokens up to 65,535 were always taken, and so are a hundred whose contexts may be so long that there could be more shares of keys
+    than the grid's second dimension has room for: their keys are then split equally."""
     from velox_amd.engine.batch import Workspace
 
     d, page = 16, 16
@@ -833,9 +896,12 @@ def test_more_decoded_tokens_than_a_grid_has_room_for_when_keys_are_shared_out(o
     q = rand((count, d), torch.float32, 83)
     kv = torch.arange(count, dtype=torch.int32).remainder(page).add(1).cuda()
     tables = torch.ones((count, 1), dtype=torch.int32, device="cuda")
-    assert (ops._shared_items(count, 1, page, page) <= 65535) == (count <= 65279)
-    got = ops.paged_attention(q, 1, 1, d, k_cache, v_cache, page, tables, torch.arange(count + 1, dtype=torch.int32, device="cuda"), kv, 1, page, 0.25, None, True,
-                              Workspace(torch.device("cuda")), uneven=True)
+    if items is not None:
+        monkeypatch.setattr(ops, "_shared_items", lambda *sizes: items)
+    workspace = Workspace(torch.device("cuda"))
+    got = ops.paged_attention(q, 1, 1, d, k_cache, v_cache, page, tables, torch.arange(count + 1, dtype=torch.int32, device="cuda"), kv, 1, page, 0.25, None, True, workspace,
+                              uneven=True)
+    assert ("attention_arrivals" in workspace.addresses()) == (items == 65535)
     scores = (0.25 * q @ k_cache[1, 0].T).masked_fill(torch.arange(page, device="cuda") >= kv[:, None], float("-inf"))
     torch.testing.assert_close(got, scores.softmax(-1) @ v_cache[1, 0].T, rtol=1e-4, atol=1e-5)
 

@@ -1370,8 +1370,9 @@ __device__ __forceinline__ float4_t load_shared_four(const float* p) {
   return __builtin_bit_cast(float4_t, bits);
 }
 
-// UNEVEN: see shared_item; the grid is (items, kv heads), `splits` is the share, part_o and part_lse have a row per item, and the last
-// workgroup of a (sequence, KV head) to arrive merges them (arrivals: [sequence][kv head], zero before and after the launch).
+// UNEVEN: see shared_item; the grid is (KV heads, items), at most 65,535 items, since they lie along its second dimension; `splits` is the share,
+// part_o and part_lse have a row per item, a sequence's side by side, and the last workgroup of a (sequence, KV head) to arrive merges
+// them (arrivals: [sequence][KV head], zero before and after the launch).
 template <typename T, int DEPTH, int WAVES, bool UNEVEN = false>
 __global__ void __launch_bounds__(64 * WAVES) decode_attention_kernel(
     const T* __restrict__ qkv, int qkv_stride, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
