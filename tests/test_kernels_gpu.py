@@ -864,6 +864,39 @@ def test_a_captured_step_shares_its_keys_out_by_the_lengths_of_each_replay(ops, 
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_an_infinite_value_stays_infinite_whatever_merges_the_splits(ops, dtype):
+    """A value of infinity behind a key that counts makes its channel infinite, not a number that is none, also where a merge asks for more parts
+    than there are."""
+    from velox_amd.engine.batch import Workspace
+    from velox_amd.parts.base import ResidualSink
+    from velox_amd.parts.norms import RMSNorm
+
+    nh, nkv, d, page = 8, 4, 64, 16
+    case = _attention_case(dtype, nh, nkv, d, page, [(1, 700 + b) for b in range(8)], seed=12)
+    for b in range(8):  # the last key of every sequence, in the last split
+        case["v_cache"][case["tables"][b, (699 + b) // page].long(), 0, 5 + b, (699 + b) % page] = float("inf")
+    workspace = Workspace(torch.device("cuda"))
+    assert ops.shares_keys(8, nkv)
+    want = _run_attention(ops, case, nh, nkv, d, page, all_decode=True, splits=1, workspace=workspace)
+    assert int(want.isinf().sum()) == 8 * nh // nkv and not want.isnan().any()
+    for more in ({"uneven": True}, {"splits": 3}):
+        got = ops.paged_attention(case["qkv"], nh, nkv, d, case["k_cache"], case["v_cache"], page, case["tables"], case["cu"], case["kv"], 1, case["max_kv"], 1.0 / math.sqrt(d), None,
+                                  True, workspace, **more).float()
+        torch.testing.assert_close(got, want, **(dict(rtol=1e-4, atol=1e-5) if dtype == torch.float32 else dict(rtol=2e-2, atol=2e-2)))
+    if dtype == torch.bfloat16:
+        weight, norm, results = ops.prepare_weight(rand((512, nh * d), dtype, 13, 0.05)), RMSNorm("", 512, 1e-5), []
+        norm.weight = torch.ones(512, device="cuda")
+        for more in ({"splits": 1}, {"parts": 2}, {"parts": 3}, {"parts": 8}):
+            residual = torch.zeros((2, 512), device="cuda")
+            attention = ops.paged_attention(case["qkv"][:2], nh, nkv, d, case["k_cache"], case["v_cache"], page, case["tables"][:2], case["cu"][:3], case["kv"][:2], 1, case["max_kv"],
+                                            1.0 / math.sqrt(d), None, True, workspace, **more)
+            ops.linear(attention, weight, None, dtype, residual_norm=ResidualSink(residual, norm))
+            results.append(residual)
+        for got in results[1:]:
+            assert results[0].isinf().any() and torch.equal(got.isnan(), results[0].isnan()) and torch.equal(got.isinf(), results[0].isinf())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_keys_shared_out_in_front_of_portions(ops, ref, dtype):
     """A mixed step: its single tokens' shares and its portions' splits use the same scratch, one after the other."""
     from velox_amd.engine.batch import Workspace

@@ -1662,7 +1662,7 @@ __global__ void __launch_bounds__(64 * WAVES) decode_attention_kernel(
         for (int j = 0; j < MERGE_ROUND; ++j) {
           const float weight = s0 + j < splits && logs[j] != -INFINITY ? expf(logs[j] - safe) : 0.f;
           denom += weight;
-          acc += o[j] * weight;
+          acc += (s0 + j < splits ? o[j] : float4_t{0.f, 0.f, 0.f, 0.f}) * weight;  // (the last one, asked for again, may be infinite)
         }
       }
       if (sinks != nullptr && mx != -INFINITY) denom += expf(sinks[h] - mx);

@@ -671,8 +671,9 @@ __device__ __forceinline__ void few_rows_sums(const bf16_t* __restrict__ a, cons
         for (int s = 0; s < PARTS; ++s) {
           const float share = s < parts.splits && logs[t][s] != -INFINITY ? expf(logs[t][s] - safe) : 0.f;
           total += share;
-          low += merged[t][2 * s] * share;
-          high += merged[t][2 * s + 1] * share;
+          const float4_t none = {0.f, 0.f, 0.f, 0.f};  // (the last part, asked for again, may be infinite)
+          low += (s < parts.splits ? merged[t][2 * s] : none) * share;
+          high += (s < parts.splits ? merged[t][2 * s + 1] : none) * share;
         }
         const float over = total > 0.f ? total : 1.f;
         bf16x8_t eight;
