@@ -404,7 +404,7 @@ static void launch_skinny_fma(const void* a, const void* w, const float* bias, v
   {                                                                             \
     if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4 && sizeof(TO) == 4) {      \
       if (MT >= 3 && (long long)n * m >= 360000) SKINNY_ROWS(MT, (MT >= 3 ? 8 : 4)); \
-      else if (n < 16 * 256) SKINNY_ROWS(MT, 2);                                \
+      else if (n < 16 * TL_WORKGROUPS) SKINNY_ROWS(MT, 2);                      \
       else SKINNY_ROWS(MT, 4);                                                  \
     } else {                                                                    \
       SKINNY_ROWS(MT, 4);                                                       \
