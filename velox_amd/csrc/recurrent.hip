@@ -583,9 +583,14 @@ __global__ void __launch_bounds__(64) short_conv_vec_kernel(const T* __restrict_
     for (int j = 0; j < TAPS; ++j) u[j] = j == taps - 2 ? now[t] : (j + 1 < TAPS ? u[j + 1] : float4_t{0.f, 0.f, 0.f, 0.f});
   }
   if (update_here && blockIdx.y == 0 && my_tail && taps > 1) {
+    if (TOKENS > 1 && update_here != 1 && first + count != hi) {
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j)
+        if (j < taps - 1) u[j] = load4_as_f32(x, is_bf16, (size_t)(hi - (taps - 1) + j) * ld + c);
+    }
 #pragma unroll
     for (int j = 0; j < TAPS; ++j)
-      if (j < taps - 1) store4_from_f32(my_tail, is_bf16, (size_t)j * C, update_here == 1 || first + count == hi ? u[j] : load4_as_f32(x, is_bf16, (size_t)(hi - (taps - 1) + j) * ld + c));
+      if (j < taps - 1) store4_from_f32(my_tail, is_bf16, (size_t)j * C, u[j]);
   }
 }
 
