@@ -1298,8 +1298,9 @@ template <> struct KeyOps<bf16_t, true> {
 
 // How a decode step's keys are shared out by their number (UNEVEN below).  A workgroup gets some 40 GB/s from memory and no more, so a step
 // whose sequences are of unequal length is as long as its longest workgroup's walk.  A sequence therefore takes as many workgroups per KV head
-// as its part of the step's key tiles is of `share` (the compute units over the KV heads), with at least SHARE_TILES tiles each: what a
-// workgroup costs before its first tile is in is as long as eight tiles take.  From SHARE_UP on it is one more: with more than one workgroup on
+// as its part of the step's key tiles is of `share` (the compute units over the KV heads), with at least share_tiles() tiles each: what a
+// workgroup costs before its first tile is in, and the merge, are as long as eight tiles of 256-byte keys take, or sixteen of shorter ones (16 sequences of
+// 391 keys, 32 heads over 8 of 64 and of 32 channels, in one pass 8.4 and 7.5 us, in parts of at least eight tiles 9.3 and 8.9, of sixteen 8.7 and 7.8).  From SHARE_UP on it is one more: with more than one workgroup on
 // some compute units those decide (57 sequences of 65 to 1,500 keys, 28 heads over 4: in equal numbers of splits 24.2 us, shared out with
 // 0.75 to 2 workgroups per compute unit 20.7, 19.1, 21.6, 20.4, 19.1; 23 of 100 to 2,000: 20.0 and 13.2, 12.7, 17.3, 16.3, 16.3; 8 of 4,096
 // 19.0 and 18.1, 18.4, 24.4, 22.8, 21.9).  Sequences of less than half a share come last, beside the workgroups that are there
@@ -1308,7 +1309,8 @@ template <> struct KeyOps<bf16_t, true> {
 // b < 0: there are not that many.  There are at most num_seqs * most + share items, `most` being what the room for page ids asks of the
 // longest sequence.
 constexpr bool SHARES_KEYS = !BIASED && !KEEPS && !CAPPED && !GATED;
-constexpr int SHARE_TILES = 8, SHARE_MOST = 32;
+constexpr int SHARE_MOST = 32;
+template <typename T> constexpr int share_tiles() { return sizeof(T) * D >= 256 ? 8 : 16; }
 constexpr float SHARE_UP = 0.75f, SHARE_SMALL = 0.5f;
 struct SharedItem { int b, split, used, kv_len; };
 
@@ -1325,7 +1327,7 @@ __device__ __forceinline__ int sum_up_to_lane(int v) {
   return v;
 }
 
-template <typename TilesOf>
+template <int LEAST, typename TilesOf>
 __device__ __forceinline__ SharedItem shared_item(const int* kv_lens, int num_seqs, int share, int tiles_room, int item, TilesOf tiles_of) {
   const int lane = threadIdx.x & 63;
   auto len_at = [&](int b) { return kv_lens[min(b, num_seqs - 1)]; };
@@ -1340,7 +1342,7 @@ __device__ __forceinline__ SharedItem shared_item(const int* kv_lens, int num_se
     for (int base = 0; base < num_seqs; base += 64) {
       const int len = base == 0 ? len0 : len_at(base + lane), tiles = base == 0 ? tiles0 : tiles_at(base + lane, len);
       const float part = (float)tiles * per_tile;
-      const int fair = min(min((int)(part + (1.f - SHARE_UP)), tiles / SHARE_TILES), SHARE_MOST);
+      const int fair = min(min((int)(part + (1.f - SHARE_UP)), tiles / LEAST), SHARE_MOST);
       const int used = tiles == 0 || (part < SHARE_SMALL) != (small != 0) ? 0 : max(max(1, fair), (int)((float)(tiles - 1) * per_room) + 1);
       const int upto = sum_up_to_lane(used);
       const uint64_t holds = __ballot(before + upto > item);
@@ -1396,7 +1398,7 @@ __global__ void __launch_bounds__(64 * WAVES) decode_attention_kernel(
   int split = blockIdx.x, b = blockIdx.z, kv_len;
   const int page_size = 1 << page_shift;
   if constexpr (UNEVEN) {
-    const SharedItem found = shared_item(kv_lens, total_tokens, splits, ((DECODE_PAGE_IDS - 2) << page_shift) / 16, blockIdx.y, [&](int len) {
+    const SharedItem found = shared_item<share_tiles<T>()>(kv_lens, total_tokens, splits, ((DECODE_PAGE_IDS - 2) << page_shift) / 16, blockIdx.y, [&](int len) {
       return (len - KeyTiles::of<16>(len - window, window, 0, page_shift).n_begin + 15) / 16;
     });
     if (found.b < 0) return;  // (uniform over the workgroup)
