@@ -190,3 +190,53 @@ def test_scratch_for_shares_of_keys_is_that_of_the_caches_pages(page, keys, rows
                                                    (64, 22000, False), (64, 24576, True), (64, 32000, True), (33, 34000, False), (48, 65536, True), (33, 152064, False)])
 def test_heads_of_some_rows_that_fill_whole_rounds_of_workgroups_are_streamed(rows, outputs, streamed):
     assert rules_of_the_kernels().streams_head(rows, outputs) == streamed
+
+
+def test_no_garbage_is_collected_while_a_step_is_captured(monkeypatch):
+    """A collector that runs in the middle of a capture may give back what an engine that is gone had captured, which ends the process.  (Stand-ins
+    for the GPU's calls: what is asked is only when the collector is held.)"""
+    import contextlib
+    import gc
+    import threading
+
+    from velox_amd.engine import runner as module
+
+    class Anything:
+        def __getattr__(self, name):
+            return lambda *args, **more: None
+
+    for name in ("Stream", "CUDAGraph"):
+        monkeypatch.setattr(torch.cuda, name, lambda **more: Anything())
+    for name in ("stream", "graph"):
+        monkeypatch.setattr(torch.cuda, name, lambda *args, **more: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "current_stream", Anything)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
+    seen, runner = [], module.ModelRunner.__new__(module.ModelRunner)
+    runner.ops, runner.device, runner._graph_pool = object(), torch.device("cpu"), None
+    runner._forward = lambda ctx: seen.append(gc.isenabled())
+    assert gc.isenabled()
+    runner._capture(None, 2)
+    assert seen == [True, True, False] and gc.isenabled()
+    inside, leave = threading.Event(), threading.Event()
+
+    def other():
+        with module.collection_held():
+            inside.set()
+            leave.wait(10)
+
+    thread = threading.Thread(target=other)
+    with pytest.raises(ValueError), module.collection_held():
+        thread.start()
+        assert inside.wait(10) and not gc.isenabled()
+        raise ValueError
+    assert not gc.isenabled()  # (the other thread is still capturing)
+    leave.set()
+    thread.join()
+    assert gc.isenabled()
+    gc.disable()
+    try:
+        with module.collection_held():
+            pass
+        assert not gc.isenabled()  # (a program that holds it itself goes on doing so)
+    finally:
+        gc.enable()

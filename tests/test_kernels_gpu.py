@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from torch_ops import TorchOps, exponential_noise
+from velox_amd.engine.runner import collection_held
 
 pytestmark = pytest.mark.gpu
 
@@ -847,7 +848,7 @@ def test_a_captured_step_shares_its_keys_out_by_the_lengths_of_each_replay(ops, 
     run()
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
+    with collection_held(), torch.cuda.graph(graph):
         captured = run()
     full = case["kv"].tolist()
     for lens in ([30 + b for b in range(16)], full, [1] * 15 + [full[15]], full[:1] + [17] * 15, [500, 1, 2000, 64, 65, 300, 1500, 16] * 2, [1] * 16):
@@ -1881,7 +1882,7 @@ def test_products_of_recorded_steps(ops, monkeypatch, m, n, k, own):
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
+        with collection_held(), torch.cuda.graph(graph):
             out = ops.linear(x, w, None, torch.bfloat16)
     assert elsewhere == [True] and len(calls) == 2 * int(own)
     for seed in range(4):

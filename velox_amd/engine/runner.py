@@ -23,6 +23,8 @@ scratch are the runner's own buffers.
 from __future__ import annotations
 
 import contextlib
+import gc
+import threading
 import time
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -31,6 +33,35 @@ import torch
 from ..cache.manager import CacheManager
 from ..parts.model import DecoderModel
 from .batch import BatchBuilder, StepContext, StepEntry, StepLimits, Workspace
+
+
+class _CollectionHeld:
+    """While a step is captured no cyclic garbage is collected: it may hold the captured steps of an engine that is gone, and giving one back waits
+    for the device, which a capture forbids, so that the process ends.  Captures of several threads may overlap: the last one out lets the
+    collector go on, if the first found it on."""
+
+    def __init__(self) -> None:
+        self._lock = threading.Lock()
+        self._inside = 0
+        self._was_on = False
+
+    @contextlib.contextmanager
+    def __call__(self):
+        with self._lock:
+            if self._inside == 0:
+                self._was_on = gc.isenabled()
+                gc.disable()
+            self._inside += 1
+        try:
+            yield
+        finally:
+            with self._lock:
+                self._inside -= 1
+                if self._inside == 0 and self._was_on:
+                    gc.enable()
+
+
+collection_held = _CollectionHeld()
 
 
 def decode_buckets(max_num_seqs: int) -> List[int]:
@@ -176,7 +207,7 @@ class ModelRunner:
             torch.cuda.current_stream().wait_stream(stream)
             torch.cuda.synchronize()
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph, pool=self._graph_pool):
+            with collection_held(), torch.cuda.graph(graph, pool=self._graph_pool):
                 logits = self._forward(ctx)
         return graph, logits, ctx
 
