@@ -283,7 +283,8 @@ struct RemovalReads {
 // (At most 256 registers a wave: the matrix instructions then keep the state in ordinary registers.  There is no bound from above on a SIMD's waves: for
 // one the compiler asks for registers that nothing uses, and many short chains wait.)  Prepared and scanned, with everything in one chain / like this (with
 // one workgroup a compute unit and loads ahead for single tokens), us: 32 heads of 64 x 64, 64 portions of 64 276 / 269 (390), 60 single tokens beside
-// 1,024 150 / 109 (242), 200 beside 300 309 / 249 (409); 16 heads of 128 x 128 456 / 453 (549), 259 / 185 (333), 589 / 435 (649).
+// 1,024 150 / 109 (242), 200 beside 300 309 / 249 (409); 16 heads of 128 x 128 456 / 453 (549), 259 / 185 (333), 589 / 435 (649), 100 portions
+// of 40 tokens 530 / 520 (560, and 561 where they asked for loads ahead and finished read-outs of no chunk).
 template <int WAVES>
 __global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1)) __attribute__((amdgpu_waves_per_eu(2))) removal_chunk_scan_kernel(const RemovalChunkArgs a) {
   constexpr bool READERS = removal_readers(WAVES);
@@ -381,7 +382,16 @@ __global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1))
 #pragma unroll
       for (int i = 0; i < 4; ++i) z[i] = S[(size_t)i * vdim];
     }
-    auto work = [&](int buffer, const RemovalOperands& o, const RemovalReads<WAVES>& r) {
+    // `first`: no read-outs of a chunk before it are finished beside it
+    auto work = [&](auto first, int buffer, const RemovalOperands& o, const RemovalReads<WAVES>& r) {
+      auto finish_before = [&] {
+        if constexpr (decltype(first)::value) {
+          pending = left < CHUNK ? left : CHUNK;
+          left -= pending;
+        } else {
+          read_out(1 - buffer, r.before);
+        }
+      };
       float4_t d = {0.f, 0.f, 0.f, 0.f}, read = d, kept = z;
       if constexpr (CHAINS) {
         if constexpr (!READS) states[buffer][wave][lane] = z;
@@ -409,13 +419,13 @@ __global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1))
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) kept = mfma4(o.nb[e], d[e], kept);
-        if constexpr (READS) read_out(1 - buffer, r.before);
+        if constexpr (READS) finish_before();
         z = kept * o.p;
       } else {
         const float4_t state = states[buffer][wave][lane];
 #pragma unroll
         for (int e = 0; e < 4; ++e) read = mfma4(r.rp[e], state[e], read);
-        read_out(1 - buffer, r.before);
+        finish_before();
         reads[buffer][wave][lane] = read;
       }
     };
@@ -423,9 +433,14 @@ __global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1))
     // between a chunk's loads and its work on every path, so that waiting for the one does not wait for the others.
     RemovalOperands ops[SCAN_AHEAD];
     RemovalReads<WAVES> of_reads[SCAN_AHEAD];
-    if (chunks == 1) {  // (single tokens beside a long portion: a quarter of the loads)
-      load(ops[0], of_reads[0]);
-      work(0, ops[0], of_reads[0]);
+    if (chunks < SCAN_AHEAD) {  // (single tokens and short portions ask for their own chunks alone)
+#pragma unroll
+      for (int j = 0; j < SCAN_AHEAD - 1; ++j)
+        if (j < chunks) load(ops[j], of_reads[j]);
+      work(std::true_type{}, 0, ops[0], of_reads[0]);
+#pragma unroll
+      for (int j = 1; j < SCAN_AHEAD - 1; ++j)
+        if (j < chunks) work(std::false_type{}, j & 1, ops[j], of_reads[j]);
     } else {
 #pragma unroll
       for (int j = 0; j < SCAN_AHEAD; ++j) load(ops[j], of_reads[j]);
@@ -433,13 +448,13 @@ __global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1))
       for (; c + SCAN_AHEAD <= chunks; c += SCAN_AHEAD) {
 #pragma unroll
         for (int j = 0; j < SCAN_AHEAD; ++j) {
-          work(j & 1, ops[j], of_reads[j]);
+          work(std::false_type{}, j & 1, ops[j], of_reads[j]);
           load(ops[j], of_reads[j]);
         }
       }
 #pragma unroll
       for (int j = 0; j < SCAN_AHEAD - 1; ++j)
-        if (c + j < chunks) work(j & 1, ops[j], of_reads[j]);  // (the same for the whole workgroup)
+        if (c + j < chunks) work(std::false_type{}, j & 1, ops[j], of_reads[j]);  // (the same for the whole workgroup)
     }
     meet();
     if constexpr (READS) read_out((chunks - 1) & 1, last_reads);
