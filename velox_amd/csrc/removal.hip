@@ -292,7 +292,7 @@ __global__ void __launch_bounds__(64 * WAVES * (removal_readers(WAVES) ? 2 : 1))
   // (heads lie along the grid fastest in both kernels: with a multiple of 8 heads the workgroups that read a record run
   // on the XCD that wrote it and share it in that XCD's L2)
   // (the long chains begin first, not when the single tokens in front of them are done: 12 beside 1,024, 32 heads of 64 x 64, 49 -> 38 us;
-  // prepared and scanned 94 -> 83, and 76 since those read nothing ahead)
+  // prepared and scanned 94 -> 83, and 76 since those ask for their own chunk alone)
   const int h = blockIdx.x, tile = blockIdx.y, b = __builtin_amdgcn_readfirstlane(sequence_by_length(a.cu_q, gridDim.z, blockIdx.z, a.ordered));
   const int lo = __builtin_amdgcn_readfirstlane(a.cu_q[b]), hi = __builtin_amdgcn_readfirstlane(a.cu_q[b + 1]);
   if (hi <= lo) return;  // (the whole workgroup)
